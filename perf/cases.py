@@ -48,15 +48,15 @@ def _case(model, layers, rows=0, context=0, ragged=False, prompt=0, past=0, dtyp
 def listed():
     named = [
         # one user at the start of a chat with the smallest model: the shortest step there is, latency and launches
-        ("decode 1 row, 40 tokens", _case("llama-3.2-1b", 8, rows=1, context=40)),
+        ("decode 1 row of 40", _case("llama-3.2-1b", 8, rows=1, context=40)),
         # the headline: eight users with 2,048-token contexts
-        ("decode 8 rows, 2048", _case("llama-3.2-3b", 8, rows=8, context=2048)),
+        ("decode 8 rows of 2048", _case("llama-3.2-3b", 8, rows=8, context=2048)),
         # a full server: 64 users whose contexts differ, sampled as chat programs sample
-        ("decode 64 rows, ragged", _case("llama-3.2-3b", 4, rows=64, context=2048, ragged=True, sampling="filtered")),
+        ("decode 64 ragged rows", _case("llama-3.2-3b", 4, rows=64, context=2048, ragged=True, sampling="filtered")),
         # a server in the middle of its day: an odd number of users, between the few-row products and the full batch
-        ("decode 27 rows, ragged", _case("llama-3.2-1b", 8, rows=27, context=700, ragged=True, sampling="filtered")),
+        ("decode 27 ragged rows", _case("llama-3.2-1b", 8, rows=27, context=700, ragged=True, sampling="filtered")),
         # a few users with long documents: the cache is most of what a step reads
-        ("decode 3 rows, 12000", _case("llama-3.1-8b", 4, rows=3, context=12000, ragged=True)),
+        ("decode 3 rows of 12000", _case("llama-3.1-8b", 4, rows=3, context=12000, ragged=True)),
         # the headline's prompt: 2,048 tokens in one step
         ("prompt 2048", _case("llama-3.2-3b", 8, prompt=2048)),
         # a long document run as one step, of a size that divides nothing
@@ -66,10 +66,10 @@ def listed():
         # continuous batching: a portion of 449 tokens over 1,024 beside 63 decoding users (512 tokens a step)
         ("63 rows beside 449 of a prompt", _case("llama-3.2-1b", 8, rows=63, context=700, ragged=True, prompt=449, past=1024)),
         # trace replay in the 32-bit path: logits at every place, decoded tokens beside a portion
-        ("float32, 3 rows beside 300", _case("llama-3.2-1b", 4, rows=3, context=200, ragged=True, prompt=300, dtype="float32", want="all")),
+        ("float32 3 rows beside 300", _case("llama-3.2-1b", 4, rows=3, context=200, ragged=True, prompt=300, dtype="float32", want="all")),
         # linear attention with a state: a prompt, and eight users decoding
-        ("linear, prompt 2048", _case("mogisun-linear", 4, prompt=2048)),
-        ("linear, decode 8 rows", _case("mogisun-linear", 4, rows=8, context=500, ragged=True)),
+        ("linear prompt 2048", _case("mogisun-linear", 4, prompt=2048)),
+        ("linear decode 8 rows", _case("mogisun-linear", 4, rows=8, context=500, ragged=True)),
     ]
     return [dict(c, name=name) for name, c in named]
 
