@@ -1,13 +1,12 @@
-// Y[M, N] = X[M, K] * W[N, K]^T with float accumulation: the plain matrix product.
-//
-// This is the product of the 32-bit path (float operands, float fused multiply-adds, no
-// reduced-precision matrix mode) and the fallback for shapes the fast bfloat16 kernels
-// refuse.  Each output element is accumulated over k = 0 .. K-1 in that order, whatever
-// M is, so a row's result does not depend on the other rows of a batch.
+// Y[M, N] = X[M, K] * W[N, K]^T with float accumulation: the plain matrix product of bfloat16 operands, for shapes
+// that the fast kernels refuse.  (Float operands go to gemm_f32.hip.)  Each output element is accumulated over
+// k = 0 .. K-1 in that order, whatever M is, so a row's result does not depend on the other rows of a batch.
 //
 // 64 x 64 output tile per workgroup of 256 threads, 4 x 4 outputs per thread, K in steps
 // of 16 staged through LDS.  Any M, N, K (edges are guarded).
 #include "common.h"
+
+extern "C" int sia_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, hipStream_t stream);
 
 #define GT 64   // tile edge
 #define GK 16   // K step
@@ -70,10 +69,8 @@ SIA_EXPORT int sia_gemm_generic(const void* X, const void* W, void* Y, int M, in
     if (K <= 0) return SIA_BAD_ARGUMENT;
     dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT), block(256);
     if (grid.y > 65535) return SIA_BAD_ARGUMENT;
-    if (in_dtype == SIA_F32)
-        hipLaunchKernelGGL((gemm_generic_kernel<float, float>), grid, block, 0, stream, (const float*)X,
-                           (const float*)W, (float*)Y, M, N, K);
-    else if (in_dtype == SIA_BF16 && out_float)
+    if (in_dtype == SIA_F32) return sia_gemm_f32((const float*)X, (const float*)W, (float*)Y, M, N, K, stream);
+    if (in_dtype == SIA_BF16 && out_float)
         hipLaunchKernelGGL((gemm_generic_kernel<bf16_t, float>), grid, block, 0, stream, (const bf16_t*)X,
                            (const bf16_t*)W, (float*)Y, M, N, K);
     else if (in_dtype == SIA_BF16)

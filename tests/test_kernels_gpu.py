@@ -208,6 +208,25 @@ def test_float32_product_has_no_reduced_precision(hip):
     assert y[0, 1].item() - 8.0 == 2.0 ** -12
 
 
+# edges of the tiles (16, 32, 64, 128 columns; 16, 32, 64 rows), of a step of 64 k and of a piece of 16; the last is misaligned
+@pytest.mark.parametrize("shape", [(1, 1, 1), (16, 17, 4), (17, 16, 60), (33, 33, 64), (64, 63, 68), (65, 130, 130), (40, 4100, 80),
+                                   (129, 8320, 192), (300, 16500, 76), (50, 257, 128)])
+def test_float32_product(hip, shape):
+    """Against float64: a result is the sum of four chains of about K / 4 float products, each rounded once or twice, so
+    it errs by at most (K / 4 + 8) times 2^-24 of the sum of the products' sizes; and whichever kernel a number of
+    rows goes to, a row's bits are the same."""
+    M, N, K = shape
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    if shape[0] == 50:
+        x = rnd(M * K + 1, seed=1)[1:].view(M, K)
+    y = hip.linear(x, w)
+    wide = x.double().abs() @ w.double().abs().T
+    assert ((y.double() - x.double() @ w.double().T).abs() <= 2.0 ** -24 * (K / 4 + 8) * wide).all()
+    for rows in (1, 16, 17, 48):
+        if rows < M:
+            assert torch.equal(hip.linear(x[:rows].contiguous(), w), y[:rows]), rows
+
+
 def test_linear_rows_do_not_depend_on_the_batch(hip):
     x, w = rnd(67, 300, seed=1), rnd(130, 300, seed=2)
     whole = hip.linear(x, w)
