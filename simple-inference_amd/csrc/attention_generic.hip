@@ -1,6 +1,6 @@
 // Attention over the paged cache for any mix of prompt portions and decoded tokens:
 // the plain kernel.  It takes every head size up to 256, any number of heads and groups,
-// any page size and both element types, and is the kernel of the 32-bit path.
+// any page size and both element types.  (Float rows of up to 128 go to attention_f32.hip, which computes the same.)
 //
 // One wavefront per (token, query head).  Keys are visited in chunks of 64 absolute
 // positions (chunk c covers positions 64c .. 64c+63), so a token's result depends on its

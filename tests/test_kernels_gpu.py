@@ -420,6 +420,45 @@ def test_norm_shared_out_between_the_products_around_it(hip, shape):
 
 
 @pytest.mark.parametrize("geom", [
+    # heads, kv heads, head size, value size, page size, window, block, sinks, cap, kept first
+    (32, 8, 64, 64, 16, 0, 0, False, 0.0, 0), (24, 8, 128, 128, 16, 0, 0, False, 0.0, 0), (5, 5, 36, 20, 4, 0, 0, True, 0.0, 0),
+    (10, 2, 16, 16, 64, 70, 0, False, 5.0, 3), (6, 2, 100, 128, 128, 0, 96, True, 0.0, 0), (4, 2, 64, 65, 8, 1, 0, False, 0.0, 130),
+    (8, 1, 4, 1, 32, 200, 0, True, 2.0, 65),
+])
+def test_float32_attention_is_the_plain_kernels(hip, geom):
+    """The kernel whose workgroups share keys and values computes what the plain kernel does, with its order of sums:
+    the same bits, in every form, for runs that cross the eights of tokens and the chunks of keys.  Values that a row
+    does not see do not reach it, whatever they are."""
+    n_heads, n_kv, D, Dv, ps, window, block, with_sinks, cap, keep = geom
+    q_lens, kv_lens = [1, 1, 1, 13, 2, 150, 9], [1, 64, 500, 13, 129, 150, 300]
+    ctx = Ctx(q_lens, kv_lens)
+    pages = sum(-(-kv // ps) for kv in kv_lens) + 2
+    cache = Cache(pages, n_kv, ps, D, torch.float32, kv_lens, seed=3)
+    cache.k_pages.copy_(rnd(*cache.k_pages.shape, seed=4))
+    cache.v_pages = rnd(pages, n_kv, Dv, ps, seed=5)
+    qkv = rnd(ctx.n_tokens, (n_heads + n_kv) * D, seed=6)
+    sinks = rnd(n_heads, seed=7) if with_sinks else None
+    whole = hip.paged_attention(qkv, n_heads, n_kv, D, 0.3, window or None, ctx, cache, value_dim=Dv, chunk=block or None, sinks=sinks,
+                                softcap=cap or None, keep_first=keep)
+    plain = torch.empty_like(whole)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    for v in (False, True):
+        if v:      # the last token of the long prompt: no other row may see its value
+            at = sum(q_lens[:6]) - 1
+            page = cache.block_table[5, 149 // ps]
+            cache.v_pages[page, :, :, 149 % ps] = float("inf")
+        got = hip.paged_attention(qkv, n_heads, n_kv, D, 0.3, window or None, ctx, cache, value_dim=Dv, chunk=block or None, sinks=sinks,
+                                  softcap=cap or None, keep_first=keep)
+        rc = hip.core.sia_attention_generic(
+            ptr(qkv), qkv.shape[1], ptr(cache.k_pages), ptr(cache.v_pages), ptr(cache.block_table), cache.block_table.shape[1],
+            ptr(ctx.seq_of_token), ptr(ctx.positions), ptr(plain), ctx.n_tokens, n_heads, n_kv, D, Dv, ps, 0.3, window, block,
+            ptr(sinks), cap, keep, 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and torch.equal(got.isnan(), plain.isnan()) and torch.equal(got.nan_to_num(7.0), plain.nan_to_num(7.0)), v
+        if v:
+            assert torch.equal(got[:at], whole[:at]) and torch.equal(got[at + 1:], whole[at + 1:])
+
+
+@pytest.mark.parametrize("geom", [
     # heads, kv heads, head_dim, page_size, window
     (24, 8, 128, 16, None), (32, 8, 64, 64, None), (16, 1, 32, 8, None), (6, 2, 48, 16, 100), (5, 5, 112, 32, 700),
     (34, 2, 16, 16, None),
