@@ -24,7 +24,14 @@
 // the walk along a sequence cannot be shortened.  Such a step gives every pair several workgroups, each with a
 // slice of the state's columns (they are independent of one another), more lanes per column and fewer rows per
 // lane; the outputs go to a float workspace and a second kernel norms and gates them, since a norm spans a head.
+// A long prompt in bfloat16 is cut into segments that are walked at the same time, each from zero: what the state S
+// in front of a segment adds to its outputs is (q_t * P_t)^T S with P_t the products of the decays since the segment began,
+// and S itself follows from segment to segment by S <- diag(P_last) S + (the segment's own).  Only products of decays,
+// which lie in (0, 1), are taken ahead: nothing is divided by them.  (There the last bits of float depend on where the
+// step's portion began; the rows' products of a step of many rows do so anyway.)
 #include "common.h"
+
+#include <type_traits>
 
 __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
@@ -133,34 +140,68 @@ __device__ __forceinline__ float row16_sum(float v) {
     return v;
 }
 
+// The sums over the 16 lanes of a row of four values, lane r getting that of value r % 4: neighbours, then pairs, swap the
+// values that the other is to add up, so that five additions serve the four.
+__device__ __forceinline__ float row16_sum_of_four(const float (&v)[4], int r) {
+    auto moved = [](float x, auto ctrl) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    using neighbour = std::integral_constant<int, 0xB1>;     // quad_perm [1,0,3,2]
+    using pair = std::integral_constant<int, 0x4E>;          // quad_perm [2,3,0,1]
+    using by4 = std::integral_constant<int, 0x124>;          // row_ror:4
+    using by8 = std::integral_constant<int, 0x128>;          // row_ror:8
+    const bool odd = r & 1, high = r & 2;
+    const float a = (odd ? v[1] : v[0]) + moved(odd ? v[0] : v[1], neighbour());
+    const float b = (odd ? v[3] : v[2]) + moved(odd ? v[2] : v[3], neighbour());
+    float c = (high ? b : a) + moved(high ? a : b, pair());
+    c += moved(c, by4());
+    return c + moved(c, by8());
+}
+
+// Where a segment's state lies among those of the step: segments of seg_len tokens, which do not overlap, begin in different
+// multiples of it; the last ones of their sequences, which may be shorter, have the odd places (two of them lie at
+// least a whole segment apart).
+__device__ __forceinline__ int segment_place(int first, bool last_of_sequence, int seg_len) {
+    return 2 * (first / seg_len) + (last_of_sequence ? 1 : 0);
+}
+
 // The walk alone, for a prompt's step in bfloat16 whose heads' columns are shared out (D a multiple of 8, rows and
-// columns aligned to 16 bytes).  The 16 lanes of one row of a wave share two or four columns of the state, lane r
+// columns aligned to 16 bytes).  What bounds it: one prompt alone, a wave's chain of tokens (0.36 us each); cut into
+// segments, the vector units (three instructions an element of the state and token, 78 us at 2,048 tokens of 24 heads of 128).  The 16 lanes of one row of a wave share two or four columns of the state, lane r
 // keeping rows r * ROWS .. r * ROWS + ROWS - 1 of each (what a lane reads of q, k and the decays serves all its
 // columns: LDS bandwidth, which every lane's reads of the same numbers would exhaust, is spent once per
 // those columns); a token's outputs are sums over the row.  q, k and the decays lie in LDS so that the 16
 // lanes' 16-byte pieces of a read are one contiguous run (no bank meets twice).  Blocks of 32 tokens: their q, k
 // (16-byte pieces), decays (float4) and values are requested into registers while the block before is walked, so
-// that the walk never waits for memory.  Outputs go to the float workspace; the norm is the finishing kernel's.
-#define GLA_WALK_TOKENS 32
+// that the walk never waits for memory (16 tokens where four columns are shared, so that four workgroups fit a unit).
+// Outputs go to the float workspace; the norm is the finishing kernel's.
 #define GLA_WALK_THREADS 256
+constexpr int gla_walk_tokens(int columns) { return columns == 4 ? 16 : 32; }
 // KF: what is written (k) comes as floats [tokens, heads, D] from ``k_f32``, as the decays do, not as columns of the
 // rows.  ``q_share`` neighbouring heads read the same q columns; a sequence's matrices begin ``state_stride`` floats
 // after the sequence before it.
 // BEFORE: the query reads the state before this token's write.
+//
+// Segments (seg_len > 0): a sequence of more than seg_len tokens is cut into segments of that many, walked by workgroups of
+// their own at the same time: the first from the request's state, the others from zero.  Every segment leaves its last
+// state in ``seg_state``; the kernels behind this one add what the states in front of the segments contribute.
 template <int ROWS, int GLA_WALK_COLS, bool KF, bool BEFORE>
 __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
     const bf16_t* __restrict__ proj, int row_stride, int q_col, int k_col, int v_col, const float* __restrict__ alpha,
     const float* __restrict__ k_f32, int q_share, float* __restrict__ state, long long state_stride,
     const int* __restrict__ cu_q, const int* __restrict__ slots, int n_heads, int D, int Dv, float q_scale,
-    float* __restrict__ raw_out) {
+    float* __restrict__ raw_out, int seg_len, float* __restrict__ seg_state) {
     extern __shared__ float lds[];
-    constexpr int TB = GLA_WALK_TOKENS, C = GLA_WALK_COLS, threads = GLA_WALK_THREADS;
+    constexpr int C = GLA_WALK_COLS, TB = gla_walk_tokens(C), threads = GLA_WALK_THREADS;
     constexpr int slice = threads / 16 * C;      // columns a workgroup
     constexpr int Dp = 16 * ROWS;                // D filled up to the rows the lanes hold: what lies beyond D is zero
     const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
-    const int j0 = blockIdx.z * slice;
-    const int first = cu_q[seq], last = cu_q[seq + 1];
-    if (first >= last) return;
+    const int n_slices = (Dv + slice - 1) / slice;
+    const int j0 = blockIdx.z % n_slices * slice, seg = blockIdx.z / n_slices;
+    const int first = cu_q[seq] + seg * seg_len, end = cu_q[seq + 1];
+    if (first >= end) return;
+    const bool cut = seg_len > 0 && end - cu_q[seq] > seg_len;
+    const int last = cut ? min(first + seg_len, end) : end;
     float* q_s = lds;               // [TB][Dp], row d = r * ROWS + i at (i / 4) * 64 + r * 4 + i % 4
     float* k_s = q_s + TB * Dp;
     float* al_s = k_s + TB * Dp;
@@ -176,30 +217,33 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
             const int d = r * ROWS + i, j = j0 + jl + c;
-            S[c][i] = (j < Dv && d < D) ? S_mem[(size_t)d * Dv + j] : 0.f;
+            S[c][i] = (seg == 0 && j < Dv && d < D) ? S_mem[(size_t)d * Dv + j] : 0.f;
         }
+    if (cut) S_mem = seg_state + ((size_t)segment_place(first, last == end, seg_len) * n_heads + head) * D * Dv;
     const int d8 = D / 8, d4 = D / 4;
     const int q_at = q_col + (head / q_share) * D, k_at = k_col + (head / q_share) * D;
     // What is on its way from memory is held in named registers, and the two steps below are written out piece by
     // piece: arrays indexed in loops ended up in scratch memory here, and a wave then waited for every piece twice.
     static_assert(TB * slice / threads == 4, "four values a thread and block");
+    constexpr int NQ = (TB * Dp / 8 + threads - 1) / threads, NA = 2 * NQ;      // pieces of 16 bytes a thread and block
+    static_assert(NQ <= 4, "pieces in named registers");
     uint4 rq0, rq1, rq2, rq3, rk0, rk1, rk2, rk3;
     float4 ra0, ra1, ra2, ra3, ra4, ra5, ra6, ra7;
     float4 rf0, rf1, rf2, rf3, rf4, rf5, rf6, rf7;
     float rv0, rv1, rv2, rv3;
     // pieces beyond the block's end repeat its last piece (every load is issued, none is conditional)
 #define GLA_REQ_QK(i, Q, K)                                                                          \
-    do {                                                                                             \
+    if constexpr ((i) < NQ) {                                                                        \
         const int idx = min(tid + (i) * threads, rnt * d8 - 1);                                       \
         const bf16_t* row = proj + (size_t)(rt0 + idx / d8) * row_stride + (idx % d8) * 8;            \
         Q = *reinterpret_cast<const uint4*>(row + q_at);                                             \
         if constexpr (!KF) K = *reinterpret_cast<const uint4*>(row + k_at);                          \
-    } while (0)
+    }
 #define GLA_REQ_F(i, A, SRC)                                                                         \
-    do {                                                                                             \
+    if constexpr ((i) < NA) {                                                                        \
         const int idx = min(tid + (i) * threads, rnt * d4 - 1);                                       \
         A = *reinterpret_cast<const float4*>(SRC + ((size_t)(rt0 + idx / d4) * n_heads + head) * D + (idx % d4) * 4); \
-    } while (0)
+    }
 #define GLA_REQ_A(i, A) GLA_REQ_F(i, A, alpha)
 #define GLA_REQ_V(i, V)                                                                              \
     do {                                                                                             \
@@ -231,7 +275,7 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
         }                                                                                            \
     } while (0)
 #define GLA_DEP_QK(i, Q, K)                                                                          \
-    do {                                                                                             \
+    if constexpr ((i) < NQ) {                                                                        \
         const int idx = tid + (i) * threads;                                                         \
         if (idx < dnt * d8) {                                                                         \
             const int base = (idx / d8) * Dp, d0 = (idx % d8) * 8;                                   \
@@ -240,12 +284,12 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
             GLA_PUT(Q.z, K.z, d0 + 4);                                                               \
             GLA_PUT(Q.w, K.w, d0 + 6);                                                               \
         }                                                                                            \
-    } while (0)
+    }
 #define GLA_DEP_F(i, A, DST)                                                                         \
-    do {   /* four rows of one lane (ROWS is a multiple of 4) */                                     \
+    if constexpr ((i) < NA) {   /* four rows of one lane (ROWS is a multiple of 4) */                 \
         const int idx = tid + (i) * threads;                                                         \
         if (idx < dnt * d4) *reinterpret_cast<float4*>(DST + (idx / d4) * Dp + place((idx % d4) * 4)) = A; \
-    } while (0)
+    }
 #define GLA_DEP_A(i, A) GLA_DEP_F(i, A, al_s)
 #define GLA_DEP_V(i, V)                                                                              \
     do {                                                                                             \
@@ -289,9 +333,15 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
             float vv[C];
 #pragma unroll
             for (int i = 0; i < ROWS / 4; ++i) { qv[i] = qn[i]; kv[i] = kn[i]; av[i] = an[i]; }
+            if constexpr (C == 4) {
+                const float4 v4 = *reinterpret_cast<const float4*>(v_s + t * slice + jl);
+                vv[0] = v4.x; vv[1] = v4.y; vv[2] = v4.z; vv[3] = v4.w;
+            } else {
 #pragma unroll
-            for (int c = 0; c < C; ++c) vv[c] = v_s[t * slice + jl + c];
+                for (int c = 0; c < C; ++c) vv[c] = v_s[t * slice + jl + c];
+            }
             fetch(min(t + 1, TB - 1));
+            float sums[C];
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 const float v = vv[c];
@@ -315,8 +365,17 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
                         acc += qv[i].w * S[c][4 * i + 3];
                     }
                 }
-                acc = row16_sum(acc);
-                if (r == 0) o_s[t * slice + jl + c] = acc;
+                sums[c] = acc;
+            }
+            if constexpr (C == 4) {
+                const float sum = row16_sum_of_four(sums, r);
+                if (r < 4) o_s[t * slice + jl + r] = sum;
+            } else {
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    const float sum = row16_sum(sums[c]);
+                    if (r == 0) o_s[t * slice + jl + c] = sum;
+                }
             }
         }
         __syncthreads();
@@ -344,6 +403,137 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
 #undef GLA_DEP_A
 #undef GLA_DEP_V
 #undef GLA_DEPOSIT
+
+// The products of the decays from a segment's beginning on, in place of the decays (segments behind a sequence's first).
+// A thread a channel.
+__global__ __launch_bounds__(256) void segment_decays_kernel(float* __restrict__ alpha, const int* __restrict__ cu_q,
+                                                             int channels, int seg_len) {
+    const int seq = blockIdx.z, c = blockIdx.y * 256 + threadIdx.x;
+    const int first = cu_q[seq] + (blockIdx.x + 1) * seg_len, end = cu_q[seq + 1];
+    if (first >= end || c >= channels) return;
+    const int n = min(seg_len, end - first);
+    float* a = alpha + (size_t)first * channels + c;
+    float p = 1.f;
+    constexpr int AHEAD = 16;
+    float next[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) next[i] = a[(size_t)min(i, n - 1) * channels];
+    for (int t = 0; t < n; t += AHEAD) {
+        float now[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) now[i] = next[i];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) next[i] = a[(size_t)min(t + AHEAD + i, n - 1) * channels];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            p *= now[i];
+            if (t + i < n) a[(size_t)(t + i) * channels] = p;
+        }
+    }
+}
+
+// The state in front of every segment, in place of the segment's own last state; the state behind the last goes to the
+// request's slot.  A thread four neighbouring elements of a matrix.
+__global__ __launch_bounds__(256) void segment_states_kernel(const float* __restrict__ decays, float* __restrict__ seg_state,
+                                                             float* __restrict__ state, long long state_stride,
+                                                             const int* __restrict__ cu_q, const int* __restrict__ slots,
+                                                             int n_heads, int D, int Dv, int seg_len) {
+    const int seq = blockIdx.z, head = blockIdx.y, at = (blockIdx.x * 256 + threadIdx.x) * 4;
+    const int begin = cu_q[seq], end = cu_q[seq + 1];
+    if (end - begin <= seg_len || at >= D * Dv) return;
+    const int d = at / Dv;
+    auto matrix = [&](int first) {
+        return reinterpret_cast<float4*>(seg_state + ((size_t)segment_place(first, first + seg_len >= end, seg_len) * n_heads + head) * D * Dv + at);
+    };
+    auto decay = [&](int first) { return decays[((size_t)(min(first + seg_len, end) - 1) * n_heads + head) * D + d]; };
+    float4 S = *matrix(begin), local = *matrix(begin + seg_len);
+    float a = decay(begin + seg_len);
+    for (int first = begin + seg_len; first < end; first += seg_len) {
+        const int next = first + seg_len < end ? first + seg_len : first;
+        float4* here = matrix(first);
+        const float4 now = local;
+        const float now_a = a;
+        if (next != first) {      // before the store below, which the compiler must not assume to lie elsewhere
+            local = *matrix(next);
+            a = decay(next);
+        }
+        *here = S;
+        S = make_float4(now_a * S.x + now.x, now_a * S.y + now.y, now_a * S.z + now.z, now_a * S.w + now.w);
+    }
+    *reinterpret_cast<float4*>(state + (size_t)slots[seq] * state_stride + (size_t)head * D * Dv + at) = S;
+}
+
+// o_t += (q_t * P_t)^T S for the tokens of a segment, with the state S in front of it and the products P of the decays up
+// to the token: a product [tokens, D] x [D, Dv] in float on the matrix cores (v_mfma_f32_16x16x4_f32).  A wave has 32
+// tokens and 64 columns, a lane four neighbouring columns (one of each of four tiles), so that S and o move 16 bytes a
+// lane; instruction i of a step of 16 channels takes the channels 4 * (lane / 16) + i.
+typedef float segf32x4 __attribute__((ext_vector_type(4)));
+template <bool BEFORE>
+__global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __restrict__ proj, int row_stride, int q_col, int q_share,
+                                                              const float* __restrict__ decays, const float* __restrict__ seg_state,
+                                                              const int* __restrict__ cu_q, int n_heads, int D, int Dv, float q_scale,
+                                                              float* __restrict__ raw, int seg_len) {
+    const int seq = blockIdx.z, head = blockIdx.y % n_heads, j0 = blockIdx.y / n_heads * 64;
+    const int first = cu_q[seq] + (blockIdx.x + 1) * seg_len, end = cu_q[seq + 1];
+    const int t0 = first + threadIdx.x / SIA_WAVE * 32;
+    if (t0 >= end) return;      // a wave leaves as a whole; no barriers below
+    const int last = min(first + seg_len, end);
+    const int lane = threadIdx.x % SIA_WAVE, r = lane % 16, g = lane / 16;
+    const int j = j0 + 4 * r;
+    const bool has_j = j < Dv;      // Dv is a multiple of four
+    const float* S = seg_state + ((size_t)segment_place(first, first + seg_len >= end, seg_len) * n_heads + head) * D * Dv + (has_j ? j : 0);
+    const int q_at = q_col + head / q_share * D;
+
+    segf32x4 acc[2][4];      // [tile of 16 tokens][column of the four] = tokens 4 g .. 4 g + 3
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = t0 + 16 * m + 4 * g + i;
+            float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (t < last && has_j) o = *reinterpret_cast<const float4*>(raw + ((size_t)t * n_heads + head) * Dv + j);
+            acc[m][0][i] = o.x; acc[m][1][i] = o.y; acc[m][2][i] = o.z; acc[m][3][i] = o.w;
+        }
+    for (int d0 = 0; d0 < D; d0 += 16) {
+        const int d = d0 + 4 * g;
+        const bool has_d = d < D;      // D is a multiple of eight
+        float a[2][4];
+        float4 b[4];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const int t = min(t0 + 16 * m + r, last - 1);      // rows past the end repeat the last and are not stored
+            const uint2 q = *reinterpret_cast<const uint2*>(proj + (size_t)t * row_stride + q_at + (has_d ? d : 0));
+            float4 p = make_float4(1.f, 1.f, 1.f, 1.f);
+            if (!BEFORE || t > first)
+                p = *reinterpret_cast<const float4*>(decays + ((size_t)(BEFORE ? t - 1 : t) * n_heads + head) * D + (has_d ? d : 0));
+            const float z = has_d ? q_scale : 0.f;
+            a[m][0] = __uint_as_float(q.x << 16) * z * p.x;
+            a[m][1] = __uint_as_float(q.x & 0xffff0000u) * z * p.y;
+            a[m][2] = __uint_as_float(q.y << 16) * z * p.z;
+            a[m][3] = __uint_as_float(q.y & 0xffff0000u) * z * p.w;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] = *reinterpret_cast<const float4*>(S + (size_t)(has_d ? d + i : 0) * Dv);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][i], b[i].x, acc[m][0], 0, 0, 0);
+                acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][i], b[i].y, acc[m][1], 0, 0, 0);
+                acc[m][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][i], b[i].z, acc[m][2], 0, 0, 0);
+                acc[m][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[m][i], b[i].w, acc[m][3], 0, 0, 0);
+            }
+    }
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = t0 + 16 * m + 4 * g + i;
+            if (t < last && has_j)
+                *reinterpret_cast<float4*>(raw + ((size_t)t * n_heads + head) * Dv + j) =
+                    make_float4(acc[m][0][i], acc[m][1][i], acc[m][2][i], acc[m][3][i]);
+        }
+}
 
 // alpha[n, c] = exp(logsigmoid(a2_bias[c] + sum_m a[n, m] * A2[c, m]) / tau) for every token n and key channel c of all
 // heads: a thread a channel, eight tokens a workgroup (their low-rank inputs staged in LDS, a channel's row of A2
@@ -376,23 +566,128 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(const T* __restrict__ pr
         if (t < nt) alpha[(size_t)(n0 + t) * channels + c] = expf(log_sigmoid(z[t]) * tau_inv);
 }
 
-// y = o * rsqrt(mean(o^2) + eps) * w * silu(g) for outputs left in a float workspace: a wave a (token, head).
-template <typename T>
-__global__ __launch_bounds__(SIA_WAVE) void gla_finish_kernel(const float* __restrict__ raw, const T* __restrict__ proj,
-                                                              int row_stride, int g_col,
-                                                              const float* __restrict__ norm_w, T* __restrict__ out,
-                                                              int n_heads, int Dv, float eps) {
-    const int n = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
-    const float* o = raw + ((size_t)n * n_heads + head) * Dv;
-    float ss = 0.f;
-    for (int c = lane; c < Dv; c += SIA_WAVE) ss += o[c] * o[c];
-    const float inv = rsqrtf(wave_sum(ss) / (float)Dv + eps);
-    const T* g_row = proj + (size_t)n * row_stride + (g_col >= 0 ? g_col : 0) + head * Dv;
-    T* dst = out + ((size_t)n * n_heads + head) * Dv;
-    for (int c = lane; c < Dv; c += SIA_WAVE) {
-        const float g = g_col >= 0 ? to_float(g_row[c]) : 0.f;
-        dst[c] = from_float<T>(o[c] * inv * norm_w[c] * (g_col >= 0 ? g / (1.f + expf(-g)) : 1.f));
+// The same on the matrix cores (v_mfma_f32_16x16x32_bf16, float sums) where the rank is a multiple of 32 and rows lie on 16
+// bytes: a wave has 64 channels of 32 tokens, A2's rows as the left operand, so that a lane holds four neighbouring
+// channels of a token.  A thread a channel reads A2 two bytes a lane and a token's inputs from LDS once per channel.
+// 2,048 tokens, 3,072 channels, rank 64: 65 -> 30 us (the decays are 25 MB).
+typedef __bf16 recbf16x8 __attribute__((ext_vector_type(8)));
+__global__ __launch_bounds__(256) void gla_decay_mfma_kernel(const bf16_t* __restrict__ proj, int row_stride, int a_col,
+                                                             const bf16_t* __restrict__ a2, const float* __restrict__ a2_bias,
+                                                             float* __restrict__ alpha, int n_tokens, int channels, int rank,
+                                                             float tau_inv) {
+    const int lane = threadIdx.x % SIA_WAVE, r = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.x * 32, c0 = (blockIdx.y * 4 + threadIdx.x / SIA_WAVE) * 64;
+    if (c0 >= channels) return;      // a wave leaves as a whole; no barriers below
+    // rows that do not exist are read as the last one and not stored
+    const bf16_t *w[4], *a[2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = a2 + (size_t)min(c0 + 16 * i + r, channels - 1) * rank + 8 * g;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) a[t] = proj + (size_t)min(n0 + 16 * t + r, n_tokens - 1) * row_stride + a_col + 8 * g;
+    segf32x4 z[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[t][i] = segf32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < rank; k += 32) {
+        recbf16x8 wk[4], ak[2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wk[i] = __builtin_bit_cast(recbf16x8, *reinterpret_cast<const uint4*>(w[i] + k));
+#pragma unroll
+        for (int t = 0; t < 2; ++t) ak[t] = __builtin_bit_cast(recbf16x8, *reinterpret_cast<const uint4*>(a[t] + k));
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) z[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wk[i], ak[t], z[t][i], 0, 0, 0);
     }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int n = n0 + 16 * t + r;
+        if (n >= n_tokens) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int c = c0 + 16 * i + 4 * g;
+            if (c >= channels) continue;      // channels are a multiple of four
+            float4 b = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (a2_bias) b = *reinterpret_cast<const float4*>(a2_bias + c);
+            *reinterpret_cast<float4*>(alpha + (size_t)n * channels + c) =
+                make_float4(expf(log_sigmoid(z[t][i][0] + b.x) * tau_inv), expf(log_sigmoid(z[t][i][1] + b.y) * tau_inv),
+                            expf(log_sigmoid(z[t][i][2] + b.z) * tau_inv), expf(log_sigmoid(z[t][i][3] + b.w) * tau_inv));
+        }
+    }
+}
+
+// y = o * rsqrt(mean(o^2) + eps) * w * silu(g) for outputs left in a float workspace: a wave four (token, head) pairs, whose
+// loads are under way together (a workgroup of one wave a pair was bound by the dispatch of workgroups: 2,048 tokens of
+// 24 heads of 128 25 -> 20 us).
+#define GLA_FINISH_WAVES 4
+#define GLA_FINISH_PAIRS 4
+template <typename T>
+__global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_kernel(
+    const float* __restrict__ raw, const T* __restrict__ proj, int row_stride, int g_col, const float* __restrict__ norm_w,
+    T* __restrict__ out, int n_pairs, int n_heads, int Dv, float eps) {
+    const int lane = threadIdx.x % SIA_WAVE;
+    const int first = ((int)blockIdx.x * GLA_FINISH_WAVES + (int)threadIdx.x / SIA_WAVE) * GLA_FINISH_PAIRS;
+    if (first >= n_pairs) return;      // a wave leaves as a whole
+    // a lane has every 64th pair of neighbouring elements (the last one alone where Dv is odd); Dv is at most 512
+    constexpr int TURNS = 4;
+    float2 o[TURNS][GLA_FINISH_PAIRS];
+    float ss[GLA_FINISH_PAIRS] = {};
+    int at[GLA_FINISH_PAIRS], g_at[GLA_FINISH_PAIRS];
+#pragma unroll
+    for (int i = 0; i < GLA_FINISH_PAIRS; ++i) {
+        const int pair = min(first + i, n_pairs - 1), n = pair / n_heads;
+        at[i] = pair;
+        g_at[i] = n;
+    }
+#pragma unroll
+    for (int k = 0; k < TURNS; ++k) {
+        const int c = 2 * (lane + k * SIA_WAVE);
+#pragma unroll
+        for (int i = 0; i < GLA_FINISH_PAIRS; ++i) {
+            const float* p = raw + (size_t)at[i] * Dv + c;
+            o[k][i] = make_float2(0.f, 0.f);
+            if (c + 1 < Dv) o[k][i] = make_float2(p[0], p[1]);
+            else if (c < Dv) o[k][i].x = p[0];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < TURNS; ++k)
+#pragma unroll
+        for (int i = 0; i < GLA_FINISH_PAIRS; ++i) ss[i] += o[k][i].x * o[k][i].x + o[k][i].y * o[k][i].y;
+    float inv[GLA_FINISH_PAIRS];
+#pragma unroll
+    for (int i = 0; i < GLA_FINISH_PAIRS; ++i) inv[i] = rsqrtf(wave_sum(ss[i]) / (float)Dv + eps);
+#pragma unroll
+    for (int k = 0; k < TURNS; ++k) {
+        const int c = 2 * (lane + k * SIA_WAVE);
+        if (c >= Dv) break;
+        const bool two = c + 1 < Dv;
+        const float w0 = norm_w[c], w1 = two ? norm_w[c + 1] : 0.f;
+#pragma unroll
+        for (int i = 0; i < GLA_FINISH_PAIRS; ++i) {
+            float f0 = 1.f, f1 = 1.f;
+            if (g_col >= 0) {
+                const T* g_row = proj + (size_t)g_at[i] * row_stride + g_col + (at[i] - g_at[i] * n_heads) * Dv + c;
+                const float g0 = to_float(g_row[0]), g1 = two ? to_float(g_row[1]) : 0.f;
+                f0 = g0 / (1.f + expf(-g0));
+                f1 = g1 / (1.f + expf(-g1));
+            }
+            if (first + i >= n_pairs) continue;
+            T* y = out + (size_t)at[i] * Dv + c;
+            y[0] = from_float<T>(o[k][i].x * inv[i] * w0 * f0);
+            if (two) y[1] = from_float<T>(o[k][i].y * inv[i] * w1 * f1);
+        }
+    }
+}
+
+template <typename T>
+static void launch_finish(const float* raw, const void* proj, int row_stride, int g_col, const float* norm_w, void* out, int n_tokens,
+                          int n_heads, int Dv, float eps, hipStream_t stream) {
+    constexpr int pairs = GLA_FINISH_WAVES * GLA_FINISH_PAIRS;
+    const int n_pairs = n_tokens * n_heads;
+    hipLaunchKernelGGL(gla_finish_kernel<T>, dim3((n_pairs + pairs - 1) / pairs), dim3(GLA_FINISH_WAVES * SIA_WAVE), 0, stream,
+                       raw, (const T*)proj, row_stride, g_col, norm_w, (T*)out, n_pairs, n_heads, Dv, eps);
 }
 
 SIA_EXPORT int sia_gla_max_dims() { return 512; }
@@ -403,11 +698,21 @@ static bool gla_slices(int n_seqs, int max_q_len, int n_heads) {
     return max_q_len > 1;
 }
 
-// Floats of workspace a step of n_tokens needs: the decays [tokens, heads, D], and room for the raw outputs
-// [tokens, heads, Dv] of a step whose heads' columns are shared out.
+// The shortest segment that a prompt is cut into, and the shortest prompt that is cut (a cut costs three small kernels,
+// some 12 us; a token of the walk 0.36).
+#define SEG_MIN 64
+#define SEG_MIN_PROMPT 128
+
+// The raw outputs [tokens, heads, Dv] as floats, and behind them the states of the step's segments.
+static long long recurrence_space(int n_tokens, int n_heads, int D, int Dv) {
+    const long long states = n_tokens >= SEG_MIN_PROMPT ? 2 * (n_tokens / SEG_MIN + 1) : 0;
+    return (long long)n_tokens * n_heads * Dv + states * n_heads * D * Dv;
+}
+
+// Floats of workspace a step of n_tokens needs: the decays [tokens, heads, D], and the space above.
 SIA_EXPORT long long sia_gla_workspace(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv) {
     (void)n_seqs; (void)max_q_len;
-    return (long long)n_tokens * n_heads * D + (long long)n_tokens * n_heads * Dv;
+    return (long long)n_tokens * n_heads * D + recurrence_space(n_tokens, n_heads, D, Dv);
 }
 
 // The recurrence itself for a step's runs of tokens, whoever prepared its inputs: S <- diag(alpha) S + k v^T, o = S^T q.
@@ -417,10 +722,11 @@ SIA_EXPORT long long sia_gla_workspace(int n_tokens, int n_seqs, int max_q_len, 
 // head's columns are shared out between workgroups; otherwise they are normed over the head (norm_w, eps), gated by
 // silu of the columns at g_col (none if negative) and written to ``out``.  Returns through ``raw_used`` whether ``raw``
 // holds the outputs.  With ``bonus`` [heads, D] the query reads the state before the token's write and, unless the outputs are
-// raw, that write weighed by it; the norm's weights are then [heads, Dv].
+// raw, that write weighed by it; the norm's weights are then [heads, Dv].  ``alpha`` is working space: it may hold other
+// numbers afterwards.
 static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_col, int v_col, int g_col,
-                             const float* k_f32, int q_share, const float* alpha, const float* norm_w, float* state,
-                             long long state_stride, const int* cu_q, const int* slots, void* out, int n_seqs,
+                             const float* k_f32, int q_share, float* alpha, const float* norm_w, float* state,
+                             long long state_stride, const int* cu_q, const int* slots, void* out, int n_tokens, int n_seqs,
                              int max_q_len, int n_heads, int D, int Dv, float q_scale, float eps, int dtype,
                              float* raw_space, bool want_raw, bool* raw_used, hipStream_t stream,
                              const float* bonus = nullptr) {
@@ -450,34 +756,64 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
     // the walk with requests a block ahead, where its pieces are aligned and fit its registers.  (Its workgroups take
     // as many columns as their threads hold whatever the step: the waves of a workgroup share the staged tokens, and
     // what bounds the walk is a wave's own chain of tokens, not the number of workgroups.)
-    const int w_cols = 2;
+    const bool long_runs = max_q_len >= SEG_MIN_PROMPT && Dv % 4 == 0 && n_seqs <= 65535 && n_heads * ((Dv + 63) / 64) <= 65535 &&
+                           ((uintptr_t)raw_space % 16) == 0 && ((uintptr_t)state % 16) == 0 && state_stride % 4 == 0;
+    const int w_cols = long_runs ? 4 : 2;
     const int w_slice = GLA_WALK_THREADS / 16 * w_cols;
     const int w_rows = (D + 15) / 16;
     const int w_rows_t = w_rows <= 4 ? 4 : w_rows <= 8 ? 8 : w_rows <= 16 ? 16 : 32;
-    const size_t w_lds = (size_t)GLA_WALK_TOKENS * (3 * 16 * w_rows_t + 2 * w_slice) * sizeof(float);
+    const size_t w_lds = (size_t)gla_walk_tokens(w_cols) * (3 * 16 * w_rows_t + 2 * w_slice) * sizeof(float);
     const bool ahead = prompt && dtype == SIA_BF16 && D % 8 == 0 && row_stride % 8 == 0 && q_col % 8 == 0 &&
                        (k_f32 ? ((uintptr_t)k_f32 % 16) == 0 : k_col % 8 == 0) && ((uintptr_t)alpha % 16) == 0 &&
                        ((uintptr_t)proj % 16) == 0 &&
-                       GLA_WALK_TOKENS * (D / 8) <= 4 * GLA_WALK_THREADS && w_lds <= 60 * 1024 && w_rows_t <= 16;
+                       w_lds <= 60 * 1024 && w_rows_t <= 16;
     float* raw = (sliced || ahead || want_raw) ? raw_space : nullptr;
     if (raw_used) *raw_used = raw != nullptr;
     if (ahead) {
-        dim3 wgrid(n_seqs, n_heads, (Dv + w_slice - 1) / w_slice), wblock(GLA_WALK_THREADS);
+        // A step of few and long sequences leaves most of the chip idle behind the walk's chain of tokens: it is cut into
+        // segments, long ones where there are enough of them.  (Workgroups the step keeps busy without: the tokens
+        // over the longest run, times heads and slices.)  2,048 tokens of 24 heads of 128: one walk of 96 workgroups 740 us; 16
+        // segments 177 with two columns a lane group, 121 with four (LDS serves twice the columns, 140 registers), and 53 for
+        // the decays' products, the states and the outputs behind it (100 MB of states and outputs).
+        const int w_slices = (Dv + w_slice - 1) / w_slice;
+        const long long busy = (long long)(n_tokens / max_q_len) * n_heads * w_slices;
+        const bool segments = long_runs && busy < 768;
+        const int seg_len = !segments ? 0 : (long long)n_tokens * n_heads * w_slices / (2 * SEG_MIN) >= 768 ? 2 * SEG_MIN : SEG_MIN;
+        const int n_segs = segments ? (max_q_len + seg_len - 1) / seg_len : 1;
+        float* seg_state = raw_space + (size_t)n_tokens * n_heads * Dv;
+        dim3 wgrid(n_seqs, n_heads, w_slices * n_segs), wblock(GLA_WALK_THREADS);
 #define WALK_AS(ROWS, COLS, KF, BEFORE)                                                                                      \
     hipLaunchKernelGGL((gla_walk_kernel<ROWS, COLS, KF, BEFORE>), wgrid, wblock, w_lds, stream, (const bf16_t*)proj,         \
                        row_stride, q_col, k_col, v_col, alpha, k_f32, q_share, state, state_stride, cu_q, slots,     \
-                       n_heads, D, Dv, q_scale, raw)
+                       n_heads, D, Dv, q_scale, raw, seg_len, seg_state)
 #define WALK(ROWS, COLS)                                                                                             \
     do {                                                                                                             \
         if (bonus) WALK_AS(ROWS, COLS, false, true);                                                                 \
         else if (k_f32) WALK_AS(ROWS, COLS, true, false);                                                            \
         else WALK_AS(ROWS, COLS, false, false);                                                                      \
     } while (0)
-        if (w_rows_t == 4) WALK(4, 2);
-        else if (w_rows_t == 8) WALK(8, 2);
-        else WALK(16, 2);
+        if (w_cols == 4) {
+            if (w_rows_t == 4) WALK(4, 4);
+            else if (w_rows_t == 8) WALK(8, 4);
+            else WALK(16, 4);
+        } else if (w_rows_t == 4) WALK(4, 2);
+        else WALK(8, 2);      // a state of more than 128 rows would need more LDS for 32 tokens than is asked for
 #undef WALK
 #undef WALK_AS
+        if (n_segs > 1) {
+            const int channels = n_heads * D;
+            hipLaunchKernelGGL(segment_decays_kernel, dim3(n_segs - 1, (channels + 255) / 256, n_seqs), dim3(256), 0, stream, alpha,
+                               cu_q, channels, seg_len);
+            hipLaunchKernelGGL(segment_states_kernel, dim3((D * Dv / 4 + 255) / 256, n_heads, n_seqs), dim3(256), 0, stream, alpha,
+                               seg_state, state, state_stride, cu_q, slots, n_heads, D, Dv, seg_len);
+            const dim3 ogrid(n_segs - 1, n_heads * ((Dv + 63) / 64), n_seqs), oblock(seg_len / 32 * SIA_WAVE);
+            if (bonus)
+                hipLaunchKernelGGL(segment_outputs_kernel<true>, ogrid, oblock, 0, stream, (const bf16_t*)proj, row_stride, q_col,
+                                   q_share, alpha, seg_state, cu_q, n_heads, D, Dv, q_scale, raw, seg_len);
+            else
+                hipLaunchKernelGGL(segment_outputs_kernel<false>, ogrid, oblock, 0, stream, (const bf16_t*)proj, row_stride, q_col,
+                                   q_share, alpha, seg_state, cu_q, n_heads, D, Dv, q_scale, raw, seg_len);
+        }
     } else {
 #define LAUNCH_AS(T, ROWS, BONUS)                                                                                    \
     hipLaunchKernelGGL((gla_recurrent_kernel<T, ROWS, BONUS>), grid, block, bytes(TB), stream, (const T*)proj,       \
@@ -537,14 +873,14 @@ __global__ __launch_bounds__(4 * SIA_WAVE) void bonus_finish_kernel(const float*
     }
 }
 
-// floats of workspace behind the decays: the raw outputs [tokens, heads, D]
+// floats of workspace behind the decays
 SIA_EXPORT long long sia_bonus_recurrence_workspace(int n_tokens, int n_heads, int D) {
-    return (long long)n_tokens * n_heads * D;
+    return recurrence_space(n_tokens, n_heads, D, D);
 }
 
 // The recurrence with a bonus for the current token: rkvg is four matrices [tokens, heads * D] one behind the other (r, k, v
-// and the output gate), decays [tokens, heads, D] float, bonus and norm_w [heads, D].
-SIA_EXPORT int sia_bonus_recurrence(const void* rkvg, const float* decays, const float* bonus, const float* norm_w,
+// and the output gate), decays [tokens, heads, D] float (working space from here on), bonus and norm_w [heads, D].
+SIA_EXPORT int sia_bonus_recurrence(const void* rkvg, float* decays, const float* bonus, const float* norm_w,
                                     float* state, long long state_stride, const int* cu_q, const int* slots, void* out,
                                     int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, float eps, int dtype,
                                     float* workspace, hipStream_t stream) {
@@ -556,7 +892,7 @@ SIA_EXPORT int sia_bonus_recurrence(const void* rkvg, const float* decays, const
     const int width = n_heads * D, k_col = (int)plane, v_col = (int)(2 * plane), g_col = (int)(3 * plane);
     bool raw = false;
     const int code = launch_recurrence(rkvg, width, 0, k_col, v_col, g_col, nullptr, 1, decays, norm_w, state, state_stride,
-                                       cu_q, slots, out, n_seqs, max_q_len, n_heads, D, D, 1.f, eps, dtype, workspace,
+                                       cu_q, slots, out, n_tokens, n_seqs, max_q_len, n_heads, D, D, 1.f, eps, dtype, workspace,
                                        false, &raw, stream, bonus);
     if (code) return code;
     if (raw) {
@@ -586,7 +922,12 @@ SIA_EXPORT int sia_gla_recurrent(const void* proj, int row_stride, int q_col, in
         const int channels = n_heads * D;
         dim3 dgrid((n_tokens + GLA_DECAY_TOKENS - 1) / GLA_DECAY_TOKENS, (channels + 255) / 256), dblock(256);
         const size_t lds = (size_t)GLA_DECAY_TOKENS * rank * sizeof(float);
-        if (dtype == SIA_F32)
+        if (dtype == SIA_BF16 && rank % 32 == 0 && channels % 4 == 0 && row_stride % 8 == 0 && a_col % 8 == 0 &&
+            ((uintptr_t)proj | (uintptr_t)a2 | (uintptr_t)a2_bias | (uintptr_t)alpha) % 16 == 0)
+            hipLaunchKernelGGL(gla_decay_mfma_kernel, dim3((n_tokens + 31) / 32, (channels + 255) / 256), dblock, 0, stream,
+                               (const bf16_t*)proj, row_stride, a_col, (const bf16_t*)a2, a2_bias, alpha, n_tokens, channels,
+                               rank, 1.f / tau);
+        else if (dtype == SIA_F32)
             hipLaunchKernelGGL(gla_decay_kernel<float>, dgrid, dblock, lds, stream, (const float*)proj, row_stride, a_col,
                                (const float*)a2, a2_bias, alpha, n_tokens, channels, rank, 1.f / tau);
         else if (dtype == SIA_BF16)
@@ -597,17 +938,12 @@ SIA_EXPORT int sia_gla_recurrent(const void* proj, int row_stride, int q_col, in
     }
     bool raw = false;
     const int code = launch_recurrence(proj, row_stride, q_col, k_col, v_col, g_col, nullptr, 1, alpha, norm_w, state,
-                                       (long long)n_heads * D * Dv, cu_q, slots, out, n_seqs, max_q_len, n_heads, D, Dv,
+                                       (long long)n_heads * D * Dv, cu_q, slots, out, n_tokens, n_seqs, max_q_len, n_heads, D, Dv,
                                        q_scale, eps, dtype, raw_space, false, &raw, stream);
     if (code) return code;
     if (raw) {
-        dim3 fgrid(n_tokens, n_heads), fblock(SIA_WAVE);
-        if (dtype == SIA_F32)
-            hipLaunchKernelGGL(gla_finish_kernel<float>, fgrid, fblock, 0, stream, raw_space, (const float*)proj,
-                               row_stride, g_col, norm_w, (float*)out, n_heads, Dv, eps);
-        else
-            hipLaunchKernelGGL(gla_finish_kernel<bf16_t>, fgrid, fblock, 0, stream, raw_space, (const bf16_t*)proj,
-                               row_stride, g_col, norm_w, (bf16_t*)out, n_heads, Dv, eps);
+        if (dtype == SIA_F32) launch_finish<float>(raw_space, proj, row_stride, g_col, norm_w, out, n_tokens, n_heads, Dv, eps, stream);
+        else launch_finish<bf16_t>(raw_space, proj, row_stride, g_col, norm_w, out, n_tokens, n_heads, Dv, eps, stream);
     }
     return SIA_LAUNCH_CHECK();
 }
@@ -634,9 +970,9 @@ __global__ __launch_bounds__(256) void hgrn2_prepare_kernel(T* __restrict__ proj
     k_f32[(size_t)n * channels + c] = 1.f - f;
 }
 
-// floats of workspace: the gates and their complements [tokens, heads, D] each, the raw outputs [tokens, heads, Dv]
+// floats of workspace: the gates and their complements [tokens, heads, D] each, the recurrence's own
 SIA_EXPORT long long sia_hgrn2_workspace(int n_tokens, int n_heads, int D, int Dv) {
-    return 2LL * n_tokens * n_heads * D + (long long)n_tokens * n_heads * Dv;
+    return 2LL * n_tokens * n_heads * D + recurrence_space(n_tokens, n_heads, D, Dv);
 }
 
 SIA_EXPORT int sia_hgrn2_scan(void* proj, int row_stride, const float* f_bias, const float* lower, const float* norm_w,
@@ -662,17 +998,12 @@ SIA_EXPORT int sia_hgrn2_scan(void* proj, int row_stride, const float* f_bias, c
         return SIA_BAD_ARGUMENT;
     bool raw = false;
     const int code = launch_recurrence(proj, row_stride, 0, 0, 2 * channels, -1, kf, 1, alpha, norm_w, state,
-                                       (long long)n_heads * D * Dv, cu_q, slots, out, n_seqs, max_q_len, n_heads, D, Dv,
+                                       (long long)n_heads * D * Dv, cu_q, slots, out, n_tokens, n_seqs, max_q_len, n_heads, D, Dv,
                                        1.f, eps, dtype, raw_space, false, &raw, stream);
     if (code) return code;
     if (raw) {
-        dim3 fgrid(n_tokens, n_heads), fblock(SIA_WAVE);
-        if (dtype == SIA_F32)
-            hipLaunchKernelGGL(gla_finish_kernel<float>, fgrid, fblock, 0, stream, raw_space, (const float*)proj,
-                               row_stride, -1, norm_w, (float*)out, n_heads, Dv, eps);
-        else
-            hipLaunchKernelGGL(gla_finish_kernel<bf16_t>, fgrid, fblock, 0, stream, raw_space, (const bf16_t*)proj,
-                               row_stride, -1, norm_w, (bf16_t*)out, n_heads, Dv, eps);
+        if (dtype == SIA_F32) launch_finish<float>(raw_space, proj, row_stride, -1, norm_w, out, n_tokens, n_heads, Dv, eps, stream);
+        else launch_finish<bf16_t>(raw_space, proj, row_stride, -1, norm_w, out, n_tokens, n_heads, Dv, eps, stream);
     }
     return SIA_LAUNCH_CHECK();
 }
@@ -726,7 +1057,7 @@ __global__ __launch_bounds__(256) void ssd_finish_kernel(const float* __restrict
 }
 
 SIA_EXPORT long long sia_ssd_workspace(int n_tokens, int n_heads, int N, int P) {
-    return 2LL * n_tokens * n_heads * N + (long long)n_tokens * n_heads * P;
+    return 2LL * n_tokens * n_heads * N + recurrence_space(n_tokens, n_heads, N, P);
 }
 
 SIA_EXPORT int sia_ssd_scan(const void* proj, int row_stride, const void* xbc, int xbc_stride, const float* dt_bias,
@@ -753,7 +1084,7 @@ SIA_EXPORT int sia_ssd_scan(const void* proj, int row_stride, const void* xbc, i
         hipLaunchKernelGGL(ssd_prepare_kernel<T>, pgrid, pblock, 0, stream, (const T*)proj, row_stride, dt_col,         \
                            (const T*)xbc, xbc_stride, b_col, dt_bias, a_log, alpha, kf, n_heads, N, share);             \
         const int code = launch_recurrence(xbc, xbc_stride, c_col, 0, 0, -1, kf, share, alpha, norm_w, state,           \
-                                           state_stride, cu_q, slots, nullptr, n_seqs, max_q_len, n_heads, N, P, 1.f,   \
+                                           state_stride, cu_q, slots, nullptr, n_tokens, n_seqs, max_q_len, n_heads, N, P, 1.f, \
                                            eps, dtype, raw_space, true, &raw, stream);                                  \
         if (code) return code;                                                                                          \
         hipLaunchKernelGGL(ssd_finish_kernel<T>, fgrid, fblock, 0, stream, raw_space, (const T*)proj, row_stride,       \
@@ -822,7 +1153,7 @@ SIA_EXPORT int sia_decay_attention(void* proj, int row_stride, const float* deca
         hipLaunchKernelGGL(decay_prepare_kernel<T>, pgrid, pblock, 0, stream, (T*)proj, row_stride, decays, alpha,      \
                            n_heads, D, active);                                                                         \
         const int code = launch_recurrence(proj, row_stride, 0, qk, 2 * qk, -1, nullptr, 1, alpha, norm_w, state,       \
-                                           (long long)n_heads * D * Dv, cu_q, slots, nullptr, n_seqs, max_q_len,        \
+                                           (long long)n_heads * D * Dv, cu_q, slots, nullptr, n_tokens, n_seqs, max_q_len, \
                                            n_heads, D, Dv, 1.f, eps, dtype, raw_space, true, &raw, stream);             \
         if (code) return code;                                                                                          \
         hipLaunchKernelGGL(decay_finish_kernel<T>, fgrid, fblock, 0, stream, raw_space, (const T*)proj, row_stride,     \
@@ -1214,8 +1545,7 @@ static int launch_delta_rule(const void* qkv, int qkv_stride, const void* proj, 
             hipLaunchKernelGGL(delta_finish_kernel<bf16_t>, fgrid, fblock, 0, stream, workspace, gates, norm_w, (bf16_t*)out,
                                n_heads, Dv, eps);
         else
-            hipLaunchKernelGGL(gla_finish_kernel<bf16_t>, fgrid, fblock, 0, stream, workspace, (const bf16_t*)proj,
-                               proj_stride, g_col, norm_w, (bf16_t*)out, n_heads, Dv, eps);
+            launch_finish<bf16_t>(workspace, proj, proj_stride, g_col, norm_w, out, n_tokens, n_heads, Dv, eps, stream);
         return SIA_LAUNCH_CHECK();
     }
 #define LAUNCH(T, ROWS)                                                                                              \
@@ -1234,8 +1564,7 @@ static int launch_delta_rule(const void* qkv, int qkv_stride, const void* proj, 
             hipLaunchKernelGGL(delta_finish_kernel<T>, fgrid, fblock, 0, stream, workspace, gates, norm_w, (T*)out,  \
                                n_heads, Dv, eps);                                                                    \
         else if (raw)                                                                                                \
-            hipLaunchKernelGGL(gla_finish_kernel<T>, fgrid, fblock, 0, stream, workspace, (const T*)proj,            \
-                               proj_stride, g_col, norm_w, (T*)out, n_heads, Dv, eps);                               \
+            launch_finish<T>(workspace, proj, proj_stride, g_col, norm_w, out, n_tokens, n_heads, Dv, eps, stream);  \
     } while (0)
     if (dtype == SIA_F32) RUN(float);
     else if (dtype == SIA_BF16) RUN(bf16_t);

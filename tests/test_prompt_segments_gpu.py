@@ -1,0 +1,71 @@
+"""The recurrences with a matrix state over prompts that are cut into segments: a prompt taken whole and in portions that
+are too short to be cut leave the same states and the same outputs, for every mixer on that recurrence."""
+
+import pytest
+import torch
+
+from test_mogisun_mechanisms import context, lowered, rnd
+from simple_inference_amd.parts.context import LayerCache
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def run(op, k, rows, H, D, Dv, lengths, portion):
+    """Outputs and states of the sequences, every step bringing each of them up to ``portion`` more tokens."""
+    g = torch.Generator().manual_seed(5)
+    f32 = lambda t: t.float().to(DEV)
+    bf16 = lambda t: t.to(torch.bfloat16).to(DEV)
+    state = torch.zeros(len(lengths) + 2, H * D * Dv, device=DEV)
+    state[0].fill_(0.25)                     # the first sequence goes on from a state
+    norm, bias, lower = f32(1 + rnd(g, Dv, std=0.2)), f32(rnd(g, H * D)), f32(torch.rand(H * D, generator=g) * 0.9)
+    per_head, decays = f32(1 + rnd(g, H * Dv, std=0.2)), f32(0.9 + 0.0999 * torch.rand(H, generator=g))
+    a2, out = bf16(rnd(g, H * D, 32, std=0.3)), torch.empty(sum(lengths), H * Dv)
+    offsets, at = [sum(lengths[:s]) for s in range(len(lengths))], [0] * len(lengths)
+    while any(a < n for a, n in zip(at, lengths)):
+        who = [s for s, n in enumerate(lengths) if at[s] < n]
+        lens = [min(portion, lengths[s] - at[s]) for s in who]
+        idx = torch.cat([torch.arange(offsets[s] + at[s], offsets[s] + at[s] + n) for s, n in zip(who, lens)])
+        ctx, x = context(DEV, lens, who), rows[idx.to(DEV)].contiguous()
+        qk, v = H * D, H * Dv
+        if op == "gla":
+            y = k.gla_recurrent(x, (0, qk, 2 * qk, 2 * qk + v, 2 * qk + 2 * v), a2, bias, norm, H, D, Dv, 8.0, D ** -0.5, 1e-5, ctx,
+                                LayerCache(state=state.view(-1, H, D, Dv)))
+        elif op == "hgrn":
+            y = k.hgrn2_scan(x[:, :2 * qk + v].contiguous(), bias, lower, norm, H, D, Dv, 1e-5, ctx, state.view(-1, H, D, Dv))
+        elif op == "ssd":        # one group: keys and queries are shared by the heads
+            proj = x[:, :v + H].contiguous()
+            y = k.ssd_scan(proj, x[:, v + H:2 * v + H + 2 * D].contiguous(), f32(decays), f32(-decays), f32(decays), per_head, H, Dv, D,
+                           1, 1, 1e-5, ctx, state)
+        elif op == "decay":
+            y = k.decay_attention(x[:, :2 * qk + 2 * v].contiguous(), decays, per_head, H, D, Dv, 1e-5, ctx, state.view(-1, H, D, Dv))
+        else:
+            rkvg = torch.stack([x[:, i * qk:(i + 1) * qk] for i in range(4)]).contiguous()
+            y = k.bonus_recurrence(rkvg, x[:, -32:].contiguous(), a2, bias - 2.0, bias, per_head, H, D, 1e-5, ctx, state)
+        out[idx] = y.float().cpu()
+        for s, n in zip(who, lens):
+            at[s] += n
+    return out, state
+
+
+# the shortest prompt that is cut and ones just beside it, remainders of a segment from one token on, one token beside
+# them; states of more than 128 rows; value widths the cut does not take; enough heads for the long segments
+@pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
+@pytest.mark.parametrize("H,D,Dv,lengths", [
+    (2, 128, 128, [300, 1, 129, 64, 127]), (3, 40, 20, [128, 257]), (1, 200, 100, [191, 130]), (2, 64, 30, [200, 3]),
+    (80, 16, 16, [1300, 128, 2, 385])])
+def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, lengths):
+    """States are sums in float whose order differs by a product of decays taken first (relative 2^-23 a token); outputs
+    are rounded to bfloat16 once, so they are equal or neighbours (2^-7 relative)."""
+    from simple_inference_amd.kernels import HipKernels
+
+    if op == "bonus":
+        Dv = D
+    k = HipKernels()
+    g = torch.Generator().manual_seed(H * D)
+    rows, _ = lowered(rnd(g, sum(lengths), 2 * H * D + 2 * H * Dv + 2 * D + H + 32), torch.bfloat16, DEV)
+    whole, state = run(op, k, rows, H, D, Dv, lengths, 10 ** 6)
+    cut, want = run(op, k, rows, H, D, Dv, lengths, 100)
+    assert float((state - want).abs().max()) <= 2e-5 * float(want.abs().max())
+    assert bool(((whole - cut).abs() <= 2.0 ** -7 * cut.abs() + 1e-3 * float(cut.std())).all()), float((whole - cut).abs().max())
+    assert float(state[len(lengths):].abs().max()) == 0.0        # nobody else's slot was touched
