@@ -26,6 +26,16 @@
 // the digit that the histogram of the launch before it decides, and leaves what has been decided so far in the
 // row's workspace for the next (every workgroup of a row computes the same bits and writes them to the same
 // place).  Launches whose filter no row asks for are skipped by the caller's hint.
+//
+// Where every row that is sampled keeps few tokens by its top-k (the caller's hint too), two launches do, with the same
+// integers and so the same token:
+//   1. a chunk's workgroup holds the chunk in registers and leaves, in index order, every token that may be among the
+//      row's k largest: those not below the chunk's own k-th largest, or a little more where the digits found so far
+//      tell few enough apart;
+//   2. a workgroup a row takes top-k, top-p and the draw among those alone, its histograms in LDS; a row of so many equal
+//      values that a chunk's would not fit their places is read whole instead.
+// What bounds the series above is the launches: each waits for the digit of the one before.  top-k 50 and top-p 0.9 over
+// 128,256 entries: 47 -> 22 us for one row, 76 -> 26 for 27, 136 -> 38 for 64.
 #include "common.h"
 #include "no_alloc.h"
 
@@ -67,6 +77,11 @@ struct SampleRow {
 __device__ __forceinline__ uint32_t ordered_key(float f) {
     const uint32_t u = __float_as_uint(f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// The float with a given key.
+__device__ __forceinline__ float key_value(uint32_t key) {
+    return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
 }
 
 __device__ __forceinline__ u64 fixed_mass(float x, float mx, float one) { return (u64)(expf(x - mx) * one); }
@@ -498,6 +513,454 @@ __global__ __launch_bounds__(SIA_WAVE) void sample_pick_kernel(const float* __re
     }
 }
 
+// ---- few tokens kept by top-k ---------------------------------------------------------------------------------
+#define SP_MAX_K 256          // the largest k of this way
+#define SP_PLACES 512         // for a chunk's candidates
+#define SP_FEW 512            // tokens kept by top-k that one wave takes alone
+#define SP_CHUNK_TOKENS (SP_AT_ONCE * SP_THREADS)      // that a workgroup holds in registers
+
+// The candidates of a row, in place of its histograms.
+struct Candidates {
+    float logit[SP_CHUNKS][SP_PLACES];
+    int index[SP_CHUNKS][SP_PLACES];
+    int number[SP_CHUNKS];      // of a chunk's candidates; more than SP_PLACES: they are not there
+};
+static_assert(sizeof(Candidates) <= SP_CLEAR_BYTES, "in the histograms' place");
+
+// 1. maximum of each chunk, and its candidates
+// How many of the workgroup's threads a wave's `mine` counts together: the waves' counts meet in one of two rows of LDS in
+// turn, so that one barrier a call is enough.
+__device__ __forceinline__ int counted_together(int mine, int (&counts)[2][SP_WAVES], int turn) {
+    if (threadIdx.x % SIA_WAVE == 0) counts[turn & 1][threadIdx.x / SIA_WAVE] = mine;
+    __syncthreads();
+    int sum = 0;
+#pragma unroll
+    for (int w = 0; w < SP_WAVES; ++w) sum += counts[turn & 1][w];
+    return sum;
+}
+
+// The q-th largest of the lanes' keys (0 if a wave has not that many above 0); no barrier.
+__device__ __forceinline__ uint32_t largest_of_lanes(uint32_t key, int q) {
+    uint32_t found = 0;
+#pragma unroll 1
+    for (int bit = 31; bit >= 0; --bit) {
+        const uint32_t t = found | (1u << bit);
+        if (__popcll(__ballot(key >= t)) >= q) found = t;
+    }
+    return found;
+}
+
+__global__ __launch_bounds__(SP_THREADS, 8) void sample_candidates_kernel(const float* __restrict__ logits,
+                                                                          const float* __restrict__ temperature,
+                                                                          const int* __restrict__ top_k, int vocab,
+                                                                          SampleRow* __restrict__ ws) {
+    __shared__ float vals[SP_WAVES];
+    __shared__ int idxs[SP_WAVES];
+    __shared__ int found[SP_AT_ONCE * SP_WAVES];
+    __shared__ int counts[2][SP_WAVES];
+    __shared__ int total;
+    const int chunk = blockIdx.x, r = blockIdx.y, lane = threadIdx.x % SIA_WAVE, wave = threadIdx.x / SIA_WAVE;
+    const float* row = logits + (size_t)r * vocab;
+    const float T = temperature[r];
+    const int k = top_k[r];
+    int begin, end;
+    chunk_range(chunk, vocab, begin, end);
+    const int i0 = begin + threadIdx.x;
+    float v[SP_AT_ONCE];
+    load_together(row, i0, SP_THREADS, end, v);
+    float bv = -INFINITY;
+    int bi = vocab;
+#pragma unroll
+    for (int u = 0; u < SP_AT_ONCE; ++u)
+        if (i0 + u * SP_THREADS < end) take_better(bv, bi, v[u], i0 + u * SP_THREADS);
+#pragma unroll
+    for (int off = SIA_WAVE / 2; off > 0; off >>= 1) {
+        const float ov = __shfl_xor(bv, off, SIA_WAVE);
+        const int oi = __shfl_xor(bi, off, SIA_WAVE);
+        take_better(bv, bi, ov, oi);
+    }
+    if (lane == 0) { vals[wave] = bv; idxs[wave] = bi; }
+    __syncthreads();
+    bv = vals[0];
+    bi = idxs[0];
+    for (int w = 1; w < SP_WAVES; ++w) take_better(bv, bi, vals[w], idxs[w]);
+    if (threadIdx.x == 0) {
+        ws[r].chunk_max[chunk] = bv;
+        ws[r].chunk_arg[chunk] = bi;
+    }
+    if (!(T > 0.f)) return;  // the whole workgroup: a greedy row
+
+    uint32_t key[SP_AT_ONCE], top = 0;
+#pragma unroll
+    for (int u = 0; u < SP_AT_ONCE; ++u) {
+        key[u] = i0 + u * SP_THREADS < end ? ordered_key(v[u]) : 0;
+        top = max(top, key[u]);
+    }
+    // A bound that at least k tokens are not below: each wave's share of k of its lanes' largest keys, and of those the waves'
+    // smallest.  Hardly more tokens than that are not below it either.  Where the tokens are laid out so that too many are,
+    // the k-th largest of the threads' largest keys, bit by bit, which takes a barrier a bit.  (Logits as they are: to divide
+    // all of them by T costs more than the rest, and keeps their order but for values that become equal; a little
+    // room below the bound takes those in.  A very large T could make many equal: then nothing is left out here.)
+    uint32_t cut = 0;
+    if (end - begin > SP_PLACES && T < 1e6f) {
+        const uint32_t bound = largest_of_lanes(top, (k + SP_WAVES - 1) / SP_WAVES);
+        if (lane == 0) found[wave] = (int)bound;
+        __syncthreads();
+        cut = (uint32_t)found[0];
+        for (int w = 1; w < SP_WAVES; ++w) cut = min(cut, (uint32_t)found[w]);
+        int mine = 0, turn = 0;
+#pragma unroll
+        for (int u = 0; u < SP_AT_ONCE; ++u) mine += __popcll(__ballot(key[u] >= cut));
+        if (counted_together(mine, counts, turn++) > SP_PLACES) {
+            cut = 0;
+#pragma unroll 1
+            for (int bit = 31; bit >= 0; --bit, ++turn) {
+                const uint32_t t = cut | (1u << bit);
+                if (counted_together(__popcll(__ballot(top >= t)), counts, turn) >= k) cut = t;
+            }
+        }
+    }
+    // in index order: the loads of a thread are SP_THREADS apart.  A token without mass below the chunk's own maximum (more
+    // than 32 T below it; 45 to be safe) has none below the row's: it is never drawn, and whether it counts among the k
+    // changes nothing for those that are (only for tokens below it, which have no mass either).  A value that is no number
+    // is not below anything: it counts, as it does above.
+    const float least = cut ? key_value(cut) : -INFINITY;
+    const float low = fmaxf(least - fabsf(least) * 2e-6f, bv - 45.f * T);
+    uint32_t mine = 0;
+#pragma unroll
+    for (int u = 0; u < SP_AT_ONCE; ++u) {
+        const bool is = i0 + u * SP_THREADS < end && !(v[u] < low);
+        if (is) mine |= 1u << u;
+        const u64 all = __ballot(is);
+        if (lane == 0) found[u * SP_WAVES + wave] = __popcll(all);
+    }
+    __syncthreads();
+    if (wave == 0) {      // how many come before each wave's
+        constexpr int each = SP_AT_ONCE * SP_WAVES / SIA_WAVE;
+        int n[each], sum = 0;
+#pragma unroll
+        for (int i = 0; i < each; ++i) {
+            n[i] = found[lane * each + i];
+            sum += n[i];
+        }
+        int before = (int)lanes_up_to_sum((u64)sum) - sum;
+        if (lane == SIA_WAVE - 1) total = before + sum;
+#pragma unroll
+        for (int i = 0; i < each; ++i) {
+            found[lane * each + i] = before;
+            before += n[i];
+        }
+    }
+    __syncthreads();
+    Candidates* list = (Candidates*)(ws + r);
+    const int number = total;
+    if (threadIdx.x == 0) list->number[chunk] = number;
+    if (number > SP_PLACES) return;      // the whole workgroup
+#pragma unroll
+    for (int u = 0; u < SP_AT_ONCE; ++u) {
+        const u64 all = __ballot((mine >> u) & 1);
+        if ((mine >> u) & 1) {
+            const int at = found[u * SP_WAVES + wave] + __popcll(all & ((1ull << lane) - 1ull));
+            list->logit[chunk][at] = v[u];
+            list->index[chunk][at] = i0 + u * SP_THREADS;
+        }
+    }
+}
+
+// 2. the token of a row from its candidates: wave w has those of chunk w.
+__global__ __launch_bounds__(SP_THREADS) void sample_few_kernel(const float* __restrict__ logits, const float* __restrict__ temperature,
+                                                                const int* __restrict__ top_k, const float* __restrict__ top_p,
+                                                                const float* __restrict__ uniform, int* __restrict__ out, int vocab,
+                                                                SampleRow* __restrict__ ws, int filters, float one) {
+    constexpr int PER_LANE = SP_PLACES / SIA_WAVE;
+    __shared__ __align__(16) LocalHistogram<u64, 1> hist;
+    __shared__ float value[SP_CHUNKS][SP_PLACES];
+    __shared__ u64 few_mass[SP_THREADS];
+    __shared__ uint32_t few_key[SP_THREADS];
+    __shared__ int few_index[SP_THREADS];
+    __shared__ int counts[2][SP_WAVES];
+    __shared__ int n_few;
+    __shared__ Decided decided;
+    __shared__ u64 wave_mass[SP_WAVES];
+    static_assert(SP_WAVES == SP_CHUNKS, "a wave a chunk");
+    const int r = blockIdx.x, lane = threadIdx.x % SIA_WAVE, wave = threadIdx.x / SIA_WAVE;
+    const float T = temperature[r], p = top_p[r], u_row = uniform[r];
+    const int k = top_k[r];
+    SampleRow* mine = ws + r;
+    const Candidates* list = (const Candidates*)mine;
+    // everything is asked for at once, the places that hold no candidate too: each round trip to memory is 1.5 us
+    float listed_logit[PER_LANE];
+    int listed_index[PER_LANE];
+#pragma unroll
+    for (int j = 0; j < PER_LANE; ++j) {
+        listed_logit[j] = list->logit[wave][j * SIA_WAVE + lane];
+        listed_index[j] = list->index[wave][j * SIA_WAVE + lane];
+    }
+    const int my_chunk = lane % SP_CHUNKS;
+    float bv = mine->chunk_max[my_chunk];
+    int bi = mine->chunk_arg[my_chunk], number = list->number[my_chunk];
+#pragma unroll
+    for (int off = SP_CHUNKS / 2; off > 0; off >>= 1) {
+        const float ov = __shfl_xor(bv, off, SIA_WAVE);
+        const int oi = __shfl_xor(bi, off, SIA_WAVE);
+        take_better(bv, bi, ov, oi);
+    }
+    if (!(T > 0.f)) {  // the whole workgroup: a greedy row
+        if (threadIdx.x == 0) out[r] = bi < vocab ? bi : 0;
+        return;
+    }
+    const bool listed = __ballot(number > SP_PLACES) == 0;
+    const int here = __shfl(number, wave, SIA_WAVE);
+    int candidates = number;
+#pragma unroll
+    for (int off = SP_CHUNKS / 2; off > 0; off >>= 1) candidates += __shfl_xor(candidates, off, SIA_WAVE);
+    const float* row = logits + (size_t)r * vocab;
+    int begin, end;
+    chunk_range(wave, vocab, begin, end);
+    const int n = listed ? here : end - begin;      // tokens of this wave
+    if (listed) {
+#pragma unroll
+        for (int j = 0; j < PER_LANE; ++j) value[wave][j * SIA_WAVE + lane] = listed_logit[j];
+    } else {
+        candidates = vocab;
+    }
+    auto logit = [&](int i) { return i >= n ? -INFINITY : listed ? value[wave][i] : row[begin + i]; };
+
+    const float mx = bv / T;
+    uint32_t cut = 0;
+    const bool wants_k = (filters & 1) && k > 0 && k < vocab && k <= candidates;
+    if (listed) {
+        uint32_t key[PER_LANE], top = 0;
+#pragma unroll
+        for (int j = 0; j < PER_LANE; ++j) {
+            key[j] = j * SIA_WAVE + lane < n ? ordered_key(listed_logit[j] / T) : 0;
+            top = max(top, key[j]);
+        }
+        // a bound below the k-th largest, as in the launch before, if the candidates would not fit otherwise
+        if (wants_k && candidates > SP_THREADS) {
+            const uint32_t bound = largest_of_lanes(top, (k + SP_WAVES - 1) / SP_WAVES);
+            if (lane == 0) few_index[wave] = (int)bound;
+            __syncthreads();
+            cut = (uint32_t)few_index[0];
+            for (int w = 1; w < SP_WAVES; ++w) cut = min(cut, (uint32_t)few_index[w]);
+        }
+        int mine = 0, at = 0;
+#pragma unroll
+        for (int j = 0; j < PER_LANE; ++j)
+            if (j * SIA_WAVE < n) mine += __popcll(__ballot(j * SIA_WAVE + lane < n && key[j] >= cut));
+        int kept = counted_together(mine, counts, 0);
+        if (kept <= SP_THREADS) {      // they meet in LDS, in index order
+            for (int w = 0; w < wave; ++w) at += counts[0][w];
+#pragma unroll
+            for (int j = 0; j < PER_LANE; ++j) {
+                const bool is = j * SIA_WAVE + lane < n && key[j] >= cut;
+                const u64 all = __ballot(is);
+                if (is) {
+                    const int to = at + __popcll(all & ((1ull << lane) - 1ull));
+                    few_key[to] = key[j];
+                    few_mass[to] = fixed_mass(listed_logit[j] / T, mx, one);
+                    few_index[to] = listed_index[j];
+                }
+                at += __popcll(all);
+            }
+            __syncthreads();
+            if (wave == 0) {      // a wave alone needs no barriers: the k-th largest, bit by bit, and what is not below it
+                const int groups = (kept + SIA_WAVE - 1) / SIA_WAVE;
+                cut = 0;
+                if (wants_k) {
+                    // from the first bit in which the keys differ on, until the keys that are not below are k, or the last bit
+                    uint32_t high = 0, low = 0xffffffffu, own[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int e = j * SIA_WAVE + lane;
+                        own[j] = e < kept ? few_key[e] : 0;
+                        if (e < kept) { high = max(high, own[j]); low = min(low, own[j]); }
+                    }
+                    for (int e = 4 * SIA_WAVE + lane; e < kept; e += SIA_WAVE) {
+                        high = max(high, few_key[e]);
+                        low = min(low, few_key[e]);
+                    }
+#pragma unroll
+                    for (int off = SIA_WAVE / 2; off > 0; off >>= 1) {
+                        high = max(high, (uint32_t)__shfl_xor((int)high, off, SIA_WAVE));
+                        low = min(low, (uint32_t)__shfl_xor((int)low, off, SIA_WAVE));
+                    }
+                    const int same = high == low ? 32 : __clz((int)(high ^ low));
+                    cut = same == 32 ? high : same == 0 ? 0 : high & ~(0xffffffffu >> same);
+#pragma unroll 1
+                    for (int bit = 31 - same; bit >= 0; --bit) {
+                        const uint32_t t = cut | (1u << bit);
+                        int not_below = 0;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) not_below += __popcll(__ballot(own[j] >= t));
+                        for (int j = 4; j < groups; ++j) {
+                            const int e = j * SIA_WAVE + lane;
+                            not_below += __popcll(__ballot(e < kept && few_key[e] >= t));
+                        }
+                        if (not_below >= k) cut = t;
+                        if (not_below == k) break;
+                    }
+                }
+                if (p <= 0.f) cut = max(cut, ordered_key(mx));  // the top value only
+                int to = 0;
+#pragma unroll 1
+                for (int j = 0; j < groups; ++j) {
+                    const int e = j * SIA_WAVE + lane;
+                    const bool is = e < kept && few_key[e] >= cut;
+                    const u64 all = __ballot(is);
+                    if (is) {      // to places that this wave has read already
+                        const uint32_t moved_key = few_key[e];
+                        const u64 moved_mass = few_mass[e];
+                        const int moved_index = few_index[e], place = to + __popcll(all & ((1ull << lane) - 1ull));
+                        __builtin_amdgcn_wave_barrier();
+                        few_key[place] = moved_key;
+                        few_mass[place] = moved_mass;
+                        few_index[place] = moved_index;
+                    }
+                    to += __popcll(all);
+                }
+                if (lane == 0) n_few = to;
+            }
+            __syncthreads();
+            kept = n_few;
+            if (kept <= SP_FEW) {
+                if (wave > 0) return;      // what follows is one wave's, without barriers
+                uint32_t lowest = 0;
+                if ((filters & 2) && p > 0.f && p < 1.f) {
+                    u64 all = 0;
+                    for (int e = lane; e < kept; e += SIA_WAVE) all += few_mass[e];
+                    all = __shfl(lanes_up_to_sum(all), SIA_WAVE - 1, SIA_WAVE);
+                    const u64 limit = (u64)((double)p * (double)all);
+                    // the smallest key that top-p keeps: what is above it does not exceed the limit
+                    lowest = 0xffffffffu;
+                    for (int i0 = 0; i0 < kept; i0 += SIA_WAVE) {
+                        const int e = i0 + lane;
+                        const uint32_t own = e < kept ? few_key[e] : 0;
+                        u64 above = 0;
+#pragma unroll 4
+                        for (int j = 0; j < kept; ++j) above += few_key[j] > own ? few_mass[j] : 0;
+                        if (e < kept && few_mass[e] > 0 && above <= limit) lowest = min(lowest, own);
+                    }
+#pragma unroll
+                    for (int off = SIA_WAVE / 2; off > 0; off >>= 1) lowest = min(lowest, (uint32_t)__shfl_xor((int)lowest, off, SIA_WAVE));
+                }
+                auto drawn = [&](int e) { return e < kept && few_key[e] >= lowest ? few_mass[e] : 0; };
+                u64 total = 0, before = 0;
+                for (int e = lane; e < kept; e += SIA_WAVE) total += drawn(e);
+                total = __shfl(lanes_up_to_sum(total), SIA_WAVE - 1, SIA_WAVE);
+                u64 target = (u64)((double)u_row * (double)total);
+                if (total > 0 && target >= total) target = total - 1;
+                int pick = bi < vocab ? bi : 0;      // nothing has mass in fixed point but, perhaps, the maximum itself: that one
+                for (int i0 = 0; total > 0 && i0 < kept; i0 += SIA_WAVE) {
+                    const u64 up_to = before + lanes_up_to_sum(drawn(i0 + lane));
+                    const u64 passes = __ballot(up_to > target);
+                    if (passes) {
+                        pick = few_index[i0 + __ffsll((long long)passes) - 1];
+                        break;
+                    }
+                    before = __shfl(up_to, SIA_WAVE - 1, SIA_WAVE);
+                }
+                if (lane == 0) out[r] = pick;
+                return;
+            }
+        }
+        cut = 0;      // many equal values: the long way, from the list
+    }
+    if (wants_k) {
+        int* count = (int*)hist.bins[0];
+        Decided d;
+        d.prefix = 0;
+        d.k_rem = k;
+        d.carried = d.limit = 0;
+        for (int pass = 0; pass < SP_PASSES; ++pass) {
+            const int bins = sp_bins(pass), shift = sp_shift(pass);
+            const uint32_t high_mask = pass == 0 ? 0u : ~((1u << (shift + (pass == 1 ? 11 : 10))) - 1u);
+            for (int b = threadIdx.x; b < bins; b += SP_THREADS) count[b] = 0;
+            __syncthreads();
+            for (int i = lane; i < n; i += SIA_WAVE) {
+                const uint32_t key = ordered_key(logit(i) / T);
+                if ((key & high_mask) == cut) atomicAdd(&count[(key >> shift) & (bins - 1)], 1);
+            }
+            __syncthreads();
+            if (wave == 0) {
+                if (pass == 2) refine_top_k<sp_bins(2) / SIA_WAVE>(count, shift, d);
+                else refine_top_k<sp_bins(0) / SIA_WAVE>(count, shift, d);
+                if (lane == 0) decided = d;
+            }
+            __syncthreads();
+            cut = decided.prefix;
+        }
+    }
+    if (p <= 0.f) {
+        cut = max(cut, ordered_key(mx));  // the top value only
+    } else if ((filters & 2) && p < 1.f) {
+        const uint32_t cut_k = cut;
+        uint32_t prefix = 0;
+        Decided d;
+        d.prefix = 0;
+        d.k_rem = 0;
+        d.carried = d.limit = 0;
+        for (int pass = 0; pass < SP_PASSES; ++pass) {
+            const int bins = sp_bins(pass), shift = sp_shift(pass);
+            const uint32_t high_mask = pass == 0 ? 0u : ~((1u << (shift + (pass == 1 ? 11 : 10))) - 1u);
+            __syncthreads();
+            for (int b = threadIdx.x; b < bins; b += SP_THREADS) hist.bins[0][b] = 0;
+            __syncthreads();
+            for (int i = lane; i < n; i += SIA_WAVE) {
+                const float x = logit(i) / T;
+                const uint32_t key = ordered_key(x);
+                if (key >= cut_k && (key & high_mask) == prefix) {
+                    const u64 q = fixed_mass(x, mx, one);
+                    if (q) atomicAdd(&hist.bins[0][(key >> shift) & (bins - 1)], q);
+                }
+            }
+            __syncthreads();
+            if (wave == 0) {
+                if (pass == 2) refine_top_p<sp_bins(2) / SIA_WAVE>(hist.bins[0], shift, d, p, false);
+                else refine_top_p<sp_bins(0) / SIA_WAVE>(hist.bins[0], shift, d, p, pass == 0);
+                if (lane == 0) decided = d;
+            }
+            __syncthreads();
+            prefix = decided.prefix;
+        }
+        cut = max(cut, prefix);
+    }
+    // the first token, in index order, at which the cumulative mass of what is kept exceeds u * total
+    auto kept = [&](int i) {
+        const float x = logit(i) / T;
+        return ordered_key(x) >= cut ? fixed_mass(x, mx, one) : 0;
+    };
+    u64 sum = 0;
+    for (int i = lane; i < n; i += SIA_WAVE) sum += kept(i);
+    sum += lanes_above_sum(sum);
+    if (lane == 0) wave_mass[wave] = sum;
+    __syncthreads();
+    u64 total = 0, before = 0;
+    for (int w = 0; w < SP_WAVES; ++w) {
+        if (w == wave) before = total;
+        total += wave_mass[w];
+    }
+    if (total == 0) {  // nothing has mass in fixed point but, perhaps, the maximum itself: that one
+        if (threadIdx.x == 0) out[r] = bi < vocab ? bi : 0;
+        return;
+    }
+    u64 target = (u64)((double)u_row * (double)total);
+    if (target >= total) target = total - 1;
+    if (target < before || target >= before + wave_mass[wave]) return;  // another wave's
+    for (int i0 = 0; i0 < n; i0 += SIA_WAVE) {
+        const u64 up_to = before + lanes_up_to_sum(kept(i0 + lane));
+        const u64 passes = __ballot(up_to > target);
+        if (passes) {
+            const int i = i0 + __ffsll((long long)passes) - 1;
+            if (lane == 0) out[r] = listed ? list->index[wave][i] : begin + i;
+            return;
+        }
+        before = __shfl(up_to, SIA_WAVE - 1, SIA_WAVE);
+    }
+}
+
+SIA_EXPORT int sia_sample_few_max_k(void) { return SP_MAX_K; }
+
 SIA_EXPORT long long sia_sample_workspace_bytes(int rows) { return (long long)rows * (long long)sizeof(SampleRow); }
 
 // The launches of one call.
@@ -509,6 +972,13 @@ static int launch_sampling(const float* logits, const float* temperature, const 
     while (bits > 0 && ((long long)vocab << bits) >> bits != (long long)vocab) --bits;
     while (bits > 0 && (double)vocab * (double)(1ull << bits) >= 9.2e18) --bits;
     const float one = (float)(1ull << bits);
+    if ((filters & 8) && (filters & 1) && vocab <= SP_CHUNKS * SP_CHUNK_TOKENS) {
+        hipLaunchKernelGGL(sample_candidates_kernel, grid, block, 0, stream, logits, temperature, top_k, vocab, ws);
+        hipLaunchKernelGGL(sample_few_kernel, dim3(rows), block, 0, stream, logits, temperature, top_k, top_p, uniform, out, vocab,
+                           ws, filters, one);
+        return SIA_LAUNCH_CHECK();
+    }
+    filters &= 7;
     hipLaunchKernelGGL(sample_max_kernel, grid, block, 0, stream, logits, vocab, ws, (filters & 3) != 0);
     if (filters & 1)
         for (int pass = 0; pass < SP_PASSES; ++pass)
@@ -529,7 +999,8 @@ static int launch_sampling(const float* logits, const float* temperature, const 
 // One token per row.  workspace: sia_sample_workspace_bytes(rows) bytes, aligned to 16, which may hold anything
 // (what has to start at zero is set to zero by the first launch); calls that share a workspace must not overlap.
 // filters: bit 0 set if some row may have a top-k filter, bit 1 if some row may have a top-p filter in (0, 1),
-// bit 2 if some row has a temperature above 0; launches for filters that no row has are skipped, and a filter
+// bit 2 if some row has a temperature above 0, bit 3 only if every row with a temperature above 0 has a top_k of 1 to
+// sia_sample_few_max_k(); launches for filters that no row has are skipped, and a filter
 // whose bit is not set is not applied (rows decide for themselves inside the launches that run).  With
 // filters == 0 the parameter pointers may be null: every row takes its argmax.
 SIA_EXPORT int sia_sample(const float* logits, const float* temperature, const int* top_k, const float* top_p,

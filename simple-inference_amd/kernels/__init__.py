@@ -112,6 +112,7 @@ _SIGNATURES = {
     "sia_prenorm_block": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_sample": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_sample_workspace_bytes": [_c_int],
+    "sia_sample_few_max_k": [],
     "sia_sample_static": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_sample_static_max_rows": [],
     "sia_sample_static_init": [],
@@ -2051,17 +2052,22 @@ class HipKernels:
         return True
 
     # -- sampling ------------------------------------------------------------------
-    def sample(self, logits, temperature, top_k, top_p, uniform, all_greedy=False, filters=None):
+    def few_max_k(self) -> int:
+        """The largest top-k that ``sample`` counts as few."""
+        return int(self.core.sia_sample_few_max_k())
+
+    def sample(self, logits, temperature, top_k, top_p, uniform, all_greedy=False, filters=None, few=False):
         """One token per row.  What the caller knows on the host spares launches: ``all_greedy`` (every
         temperature is 0; the parameter tensors may then be None), or ``filters``, the sum of 1 if some row
-        may have a top-k filter and 2 if some row may have a top-p filter below 1 (None: both)."""
+        may have a top-k filter and 2 if some row may have a top-p filter below 1 (None: both); ``few``: every row with a
+        temperature has a top-k of 1 to ``few_max_k()`` (two launches then do, with the same tokens)."""
         rows, vocab = logits.shape
         self._want(logits, "logits", torch.float32)
         if all_greedy:
             filters = 0
             temperature = top_k = top_p = uniform = None
         else:
-            filters = 4 | (3 if filters is None else int(filters) & 3)
+            filters = 4 | (3 if filters is None else int(filters) & 3) | (8 if few else 0)
             self._want(temperature, "temperature", torch.float32, (rows,))
             self._want(top_k, "top_k", torch.int32, (rows,))
             self._want(top_p, "top_p", torch.float32, (rows,))

@@ -30,6 +30,8 @@ class Sampler:
         self.device = torch.device(device)
         self._mirrors: List[_Mirror] = []     # two, used in turn: a step may be prepared while the last one's copy waits
         self._turn = 0
+        # kernels that sample from few tokens faster say up to which top-k
+        self._few_max_k = kernels.few_max_k() if hasattr(kernels, "few_max_k") else 0
 
     def sample(self, logits: torch.Tensor, params: Sequence[SamplingParams], draw_indices: Sequence[int]) -> List[int]:
         """One token per row of float32 ``logits``; row i uses ``params[i]`` and its ``draw_indices[i]``-th draw."""
@@ -70,4 +72,6 @@ class Sampler:
             mirror.copied.record()
         mirror.in_use = True
         filters = (1 if any(k > 0 for k in top_k) else 0) | (2 if any(0.0 < p < 1.0 for p in top_p) else 0)
-        return self.kernels.sample(logits, dev[0], dev[3].view(torch.int32), dev[1], dev[2], filters=filters)
+        few = self._few_max_k > 0 and all(0 < k <= self._few_max_k for k, p in zip(top_k, params) if not p.greedy)
+        return self.kernels.sample(logits, dev[0], dev[3].view(torch.int32), dev[1], dev[2], filters=filters,
+                                   **({"few": True} if few else {}))

@@ -869,3 +869,29 @@ def test_sample_greedy_is_argmax_with_lowest_index_on_ties(hip):
     z = lambda dt, v: torch.full((3,), v, dtype=dt, device=DEV)
     got = hip.sample(logits, z(torch.float32, 0.0), z(torch.int32, 0), z(torch.float32, 1.0), z(torch.float32, 0.5))
     assert got.tolist() == [4321, 17, 0]
+
+
+@pytest.mark.parametrize("vocab", [1, 40, 511, 8192, 8193, 16 * 513, 128256, 131072, 131073])
+def test_sampling_among_few_tokens_is_the_series_of_launches(hip, vocab):
+    """The two launches for rows that all keep few tokens by top-k give the token of the series of launches, bit for bit:
+    over random rows, rows of equal values (more than fit a chunk's places), rows with few finite values, infinities and
+    values that are no numbers; any temperature, top-p and number; greedy rows beside them."""
+    g = torch.Generator().manual_seed(vocab)
+    rows = [torch.randn(vocab, generator=g) * s for s in (1.0, 4.0, 0.01, 30.0)]
+    rows += [torch.zeros(vocab), torch.randint(0, 3, (vocab,), generator=g).float(), torch.full((vocab,), -float("inf"))]
+    few = torch.full((vocab,), -float("inf"))
+    few[torch.randint(0, vocab, (7,), generator=g)] = torch.randn(7, generator=g)
+    high = torch.randn(vocab, generator=g)
+    high[: vocab // 3] += 80.0
+    odd = torch.randn(vocab, generator=g)
+    odd[torch.randint(0, vocab, (3,), generator=g)] = float("nan")
+    endless = torch.randn(vocab, generator=g)
+    endless[vocab // 2] = float("inf")
+    rows += [few, high, odd, endless]
+    cases = [(t, k, p, u) for t in (1.0, 0.7, 1e-3, 0.0, 5.0) for k, p, u in ((1, 1.0, 0.3), (50, 0.9, 0.77), (256, 0.5, 0.999),
+                                                                              (50, 0.0, 0.2), (7, 1.0, 0.0), (255, 0.99, 0.5))]
+    logits = torch.stack(rows).repeat_interleave(len(cases), 0).to(DEV)
+    column = lambda i, dtype: torch.tensor([c[i] for c in cases] * len(rows), dtype=dtype, device=DEV)
+    args = (logits, column(0, torch.float32), column(1, torch.int32), column(2, torch.float32), column(3, torch.float32))
+    for filters in (3, 1):
+        assert torch.equal(hip.sample(*args, filters=filters, few=True), hip.sample(*args, filters=filters)), filters
