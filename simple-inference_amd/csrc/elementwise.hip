@@ -698,3 +698,60 @@ SIA_EXPORT int sia_place_tokens(int* dst, const int* dst_rows, const int* src, c
                        n);
     return SIA_LAUNCH_CHECK();
 }
+
+// dst[i] = src[rows[i]] for rows of `words` pieces of T: what only some rows of a step are read for is taken on alone.
+template <typename T>
+__global__ __launch_bounds__(256) void take_rows_kernel(const T* __restrict__ src, const int* __restrict__ rows,
+                                                        T* __restrict__ dst, int words) {
+    const T* from = src + (size_t)rows[blockIdx.x] * words;
+    T* to = dst + (size_t)blockIdx.x * words;
+    for (int i = blockIdx.y * 256 + threadIdx.x; i < words; i += gridDim.y * 256) to[i] = from[i];
+}
+
+// bytes: of a row.  rows: n places below the number of rows of src.
+SIA_EXPORT int sia_take_rows(const void* src, const int* rows, void* dst, int n, long long bytes, hipStream_t stream) {
+    if (n <= 0 || bytes <= 0) return 0;
+    if (!src || !rows || !dst || bytes > 0x7fffffffLL) return SIA_BAD_ARGUMENT;
+    const uintptr_t at = (uintptr_t)src | (uintptr_t)dst | (uintptr_t)bytes;
+#define TAKE(T)                                                                                                     \
+    do {                                                                                                            \
+        const int words = (int)(bytes / sizeof(T));                                                                 \
+        const int parts = words < 64 * 256 ? (words + 255) / 256 : 64;                                              \
+        hipLaunchKernelGGL(take_rows_kernel<T>, dim3(n, parts), dim3(256), 0, stream, (const T*)src, rows, (T*)dst, words); \
+    } while (0)
+    if (at % sizeof(uint4) == 0) TAKE(uint4);
+    else if (at % sizeof(uint32_t) == 0) TAKE(uint32_t);
+    else TAKE(uint8_t);
+#undef TAKE
+    return SIA_LAUNCH_CHECK();
+}
+
+// Tokens of a step as sequences of one token each: token rows[i] becomes sequence i, whose last position is the token's
+// and whose pages are those of the sequence that the token belongs to.
+__global__ __launch_bounds__(256) void rows_alone_kernel(const int* __restrict__ rows, const int* __restrict__ positions,
+                                                         const int* __restrict__ seq_of_token, const int* __restrict__ table,
+                                                         int width, int* __restrict__ positions_out, int* __restrict__ kv_len,
+                                                         int* __restrict__ seq_out, int* __restrict__ cu_q,
+                                                         int* __restrict__ table_out) {
+    const int i = blockIdx.x, token = rows[i], seq = seq_of_token[token];
+    if (threadIdx.x == 0) {
+        const int pos = positions[token];
+        positions_out[i] = pos;
+        kv_len[i] = pos + 1;
+        seq_out[i] = i;
+        cu_q[i] = i;
+        if (i + 1 == (int)gridDim.x) cu_q[i + 1] = i + 1;
+    }
+    for (int c = threadIdx.x; c < width; c += 256) table_out[(size_t)i * width + c] = table[(size_t)seq * width + c];
+}
+
+SIA_EXPORT int sia_rows_alone(const int* rows, const int* positions, const int* seq_of_token, const int* table, int width,
+                              int* positions_out, int* kv_len, int* seq_out, int* cu_q, int* table_out, int n,
+                              hipStream_t stream) {
+    if (n <= 0) return 0;
+    if (!rows || !positions || !seq_of_token || !table || width <= 0 || !positions_out || !kv_len || !seq_out || !cu_q || !table_out)
+        return SIA_BAD_ARGUMENT;
+    hipLaunchKernelGGL(rows_alone_kernel, dim3(n), dim3(256), 0, stream, rows, positions, seq_of_token, table, width,
+                       positions_out, kv_len, seq_out, cu_q, table_out);
+    return SIA_LAUNCH_CHECK();
+}

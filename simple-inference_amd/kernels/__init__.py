@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import dataclasses
 from typing import Dict, Optional
 
 import torch
@@ -126,6 +127,8 @@ _SIGNATURES = {
     "sia_gemm_skinny_residual_tiled": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "sia_gemm_skinny_tile_height": [_c_int],
     "sia_gemm_skinny_tiled": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
+    "sia_take_rows": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ll, _c_ptr],
+    "sia_rows_alone": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_place_tokens": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_scale_rows": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_float, _c_ptr],
     "sia_stream_read": [_c_ptr, _c_ll, _c_ptr, _c_ptr],
@@ -409,6 +412,31 @@ class HipKernels:
             raise KernelError(f"{dst_rows.numel()} destination rows for {src_rows.numel()} source rows")
         self._check(self.core.sia_place_tokens(_ptr(token_ids), _ptr(dst_rows), _ptr(src_tokens), _ptr(src_rows),
                                                dst_rows.numel(), self._stream()), "place_tokens")
+
+    def take_rows(self, x, rows):
+        """``x[rows]`` for a matrix and int32 places on the device (which must lie inside it)."""
+        self._want(x, "matrix")
+        self._want(rows, "rows", torch.int32)
+        n = rows.numel()
+        out = torch.empty((n, *x.shape[1:]), dtype=x.dtype, device=x.device)
+        if n:
+            self._check(self.core.sia_take_rows(_ptr(x), _ptr(rows), _ptr(out), n, x.stride(0) * x.element_size(), self._stream()),
+                        "take_rows")
+        return out
+
+    def rows_alone(self, rows, ctx, cache):
+        """The context and the cache of a step in which the tokens at ``rows`` are sequences of one token each, for
+        attention over pages that hold everything they see."""
+        n, table = rows.numel(), cache.block_table
+        self._want(table, "block table", torch.int32)
+        new = lambda *shape: torch.empty(shape, dtype=torch.int32, device=table.device)
+        positions, kv_len, seq, cu_q, own = new(n), new(n), new(n), new(n + 1), new(n, table.shape[1])
+        self._check(self.core.sia_rows_alone(_ptr(rows), _ptr(ctx.positions), _ptr(ctx.seq_of_token), _ptr(table), table.shape[1],
+                                             _ptr(positions), _ptr(kv_len), _ptr(seq), _ptr(cu_q), _ptr(own), n, self._stream()),
+                    "rows_alone")
+        alone = dataclasses.replace(ctx, n_tokens=n, n_seqs=n, positions=positions, seq_of_token=seq, cu_q=cu_q, kv_len=kv_len,
+                                    max_q_len=1, n_decode_seqs=n, q_lens=[1] * n, max_run_kv_len=0, only_rows=None)
+        return alone, dataclasses.replace(cache, block_table=own)
 
     def embed(self, token_ids, table, scale=1.0):
         self._want(token_ids, "token_ids", torch.int32)

@@ -268,6 +268,10 @@ class Attention:
                 "rotary_dim": self.position.rotary_dim, "cos": cos, "sin": sin, "scale": self.scale,
                 "window": self.window}
 
+    def gives_only_rows(self) -> bool:
+        """Whether ``forward`` gives the rows ``ctx.only_rows`` alone where it is set."""
+        return type(self).forward is Attention.forward and not self.row_form
+
     def _options(self) -> bool:
         """Whether any of the further forms is switched on (the kernels then get them as keyword arguments)."""
         return (self.bias or self.qk_norm_eps is not None or self.sink or self.chunk is not None
@@ -353,11 +357,21 @@ class Attention:
         if self.out_gate:
             qkv, further = qkv
             gate_logits = further[:, :self.gates]
+        rows = getattr(ctx, "only_rows", None)      # keys and values are in the pages: of the rest, only these rows are read
+        if rows is not None and rows.numel() == 0:
+            return None
+        if rows is not None and gate_logits is None and rows.numel() <= ctx.n_seqs and ctx.n_tokens >= ctx.n_decode_seqs + 128:
+            # about a token a sequence: its attention alone is a decoded token's, not a prompt's
+            qkv = k.take_rows(qkv, rows)
+            ctx, cache = k.rows_alone(rows, ctx, cache)
+            rows = None
         out = k.paged_attention(
             qkv, self.num_heads, self.num_kv_heads, self.page_dim or self.head_dim, self.scale, self.window, ctx, cache,
             **attend)
         if gate_logits is not None:
             out = (k.element_gate(out, gate_logits, self.num_heads) if self.element_gate
                    else k.head_gate(out, gate_logits, self.num_heads))
+        if rows is not None:
+            out = k.take_rows(out, rows)
         y = k.pending_linear(out, self.w_o)   # the norm after it may have it added into the residual
         return BiasedDelta(y, self.b_o, k) if self.o_bias else y

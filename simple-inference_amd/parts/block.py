@@ -71,6 +71,46 @@ class PreNormBlock:
             stream.delta = self.token_input.forward(x, ctx)
             stream.post = self.token_input_norm
 
+    def forward_rows(self, stream, ctx, cache, rows):
+        """``forward`` for a model's last layer, of whose results only ``rows`` are read: the mixer sees all tokens, what
+        follows it those alone, and the stream is left with them.  False, with nothing done, for a block it does not fit."""
+        if (type(self).forward is not PreNormBlock.forward or self.feed_forward is None or self.token_input is not None
+                or not _by_row(self.feed_forward)):
+            return False
+        h = _normed(self.mixer_norm, self.mixer, stream)
+        delta = _mixed_rows(self.mixer, h, ctx, cache, rows)
+        if delta is None:
+            return True
+        stream.keep_rows(rows, ctx.kernels)
+        stream.delta = delta
+        stream.scale = self.residual_scale
+        stream.delta = self.feed_forward.forward(_normed(self.feed_forward_norm, self.feed_forward, stream), ctx)
+        stream.scale = self.residual_scale
+        return True
+
+
+def _by_row(*parts):
+    """Whether each of the parts says that a row of its result depends on that row of its input alone.  The class that
+    says so must be the one that computes it: a subclass with a computation of its own is no longer what was said."""
+    for part in parts:
+        owner = next((c for c in type(part).__mro__ if "forward" in c.__dict__ or "logits" in c.__dict__), object)
+        if not owner.__dict__.get("by_row", False):
+            return False
+    return True
+
+
+def _mixed_rows(mixer, h, ctx, cache, rows):
+    """The mixer's result at ``rows`` alone (None if there are none): from a mixer that gives only those, or taken out of
+    all of it."""
+    if not getattr(mixer, "gives_only_rows", lambda: False)():
+        y = mixer.forward(h, ctx, cache)
+        return ctx.kernels.take_rows(y.compute() if hasattr(y, "compute") else y, rows) if rows.numel() else None
+    ctx.only_rows = rows
+    try:
+        return mixer.forward(h, ctx, cache)
+    finally:
+        ctx.only_rows = None
+
 
 def _normed(norm, consumer, stream):
     """The norm's rows for ``consumer``.  A norm that ``gives_scaled_rows`` may leave the division by the root mean
@@ -121,6 +161,25 @@ class GatedPreNormBlock:
             logits = self.feed_forward_gate.logits(h)
             stream.delta = self.feed_forward.forward(h, ctx)
             stream.gate = (logits, self.feed_forward_gate.bias)
+
+    def forward_rows(self, stream, ctx, cache, rows):
+        """As ``PreNormBlock.forward_rows``."""
+        if type(self).forward is not GatedPreNormBlock.forward or self.feed_forward is None or not _by_row(
+                self.feed_forward, self.mixer_gate, self.feed_forward_gate):
+            return False
+        h = self.mixer_norm.forward(stream)
+        delta = _mixed_rows(self.mixer, h, ctx, cache, rows)
+        if delta is None:
+            return True
+        logits = self.mixer_gate.logits(ctx.kernels.take_rows(h, rows))
+        stream.keep_rows(rows, ctx.kernels)
+        stream.delta = delta
+        stream.gate = (logits, self.mixer_gate.bias)
+        h = self.feed_forward_norm.forward(stream)
+        logits = self.feed_forward_gate.logits(h)
+        stream.delta = self.feed_forward.forward(h, ctx)
+        stream.gate = (logits, self.feed_forward_gate.bias)
+        return True
 
 
 @register_block("sandwich")

@@ -50,6 +50,7 @@ class StepContext:
     max_run_kv_len: int = 0  # the longest kv_len among the sequences that bring more than one token (0: not known)
     extra: dict = field(default_factory=dict)  # name -> int32 [n_tokens]: what the step's entries brought beside tokens
     shared: dict = field(default_factory=dict)  # name -> what a layer of this step leaves for later layers of the step
+    only_rows: Optional[torch.Tensor] = None  # set for a mixer that ``gives_only_rows``: the only rows of its result that are read
 
 
 @dataclass
@@ -115,6 +116,11 @@ class ResidualStream:
         self.scale = None
         if value is not None:
             self.lowered = None
+
+    def keep_rows(self, rows, kernels) -> None:
+        """Goes on with the given rows alone.  A pending delta has them alone already (and nothing else is pending)."""
+        self.residual = kernels.take_rows(self.residual, rows)
+        self.lowered = None
 
     def scaled_terms(self):
         """The pending delta as ``[(tensor, factor)]`` with the stream's own factor multiplied in."""

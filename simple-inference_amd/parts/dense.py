@@ -17,6 +17,8 @@ ACTIVATIONS = ("relu2", "gelu_tanh", "gelu")
 class DenseFeedForward:
     """params: hidden_size, intermediate_size, activation."""
 
+    by_row = True     # a row of the result depends on that row of the input alone
+
     def __init__(self, params, env):
         self.hidden = int(params["hidden_size"])
         self.inter = int(params["intermediate_size"])

@@ -15,6 +15,8 @@ from .registry import register_gate
 class SigmoidLinearGate:
     """params: hidden_size, and optionally bias (default True)."""
 
+    by_row = True     # a row of the result depends on that row of the input alone
+
     def __init__(self, params, env):
         self.hidden = int(params["hidden_size"])
         self.has_bias = bool(params.get("bias", True))

@@ -92,4 +92,13 @@ class GatedLinearAttention:
         proj = k.linear(h, self.w_in)
         out = k.gla_recurrent(proj, self.columns, self.w_a2, self.b_a2, self.norm, self.num_heads, self.key_dim,
                               self.value_dim, self.tau, self.key_dim ** -0.5, self.eps, ctx, cache)
+        rows = getattr(ctx, "only_rows", None)      # the states hold all tokens: of the rest, only these rows are read
+        if rows is not None:
+            if rows.numel() == 0:
+                return None
+            out = k.take_rows(out, rows)
         return k.pending_linear(out, self.w_o)
+
+    def gives_only_rows(self) -> bool:
+        """Whether ``forward`` gives the rows ``ctx.only_rows`` alone where it is set."""
+        return type(self).forward is GatedLinearAttention.forward

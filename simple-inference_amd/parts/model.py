@@ -158,8 +158,21 @@ class DecoderModel:
         for e, li in enumerate(self.order):
             if e in self.entries:
                 self.stream_ops[self.entries[e]].forward(stream, ctx, first)
-            self.layers[li].block.forward(stream, ctx, caches[e])
+            block = self.layers[li].block
+            if e + 1 == len(self.order) and self._few_rows_read(ctx) and getattr(block, "forward_rows", None) is not None:
+                rows = ctx.logit_rows if ctx.n_logit_rows else ctx.positions[:0]
+                if block.forward_rows(stream, ctx, caches[e], rows):
+                    return self.head.forward(self.final_norm.forward(stream)) if ctx.n_logit_rows else None
+            block.forward(stream, ctx, caches[e])
         if ctx.n_logit_rows == 0:
             return None
         h = self.final_norm.forward(stream, rows=ctx.logit_rows)
         return self.head.forward(h)
+
+    @staticmethod
+    def _few_rows_read(ctx: StepContext) -> bool:
+        """Whether the last layer's results are read at so few of the step's rows that going on with those alone pays
+        (what a layer writes for later steps, keys, values and states, it writes for all): a prompt's portion needs its
+        last row, or none.  Steps of up to 16 rows are bound by reading the weights, whatever their rows.  (A prompt's last
+        layer at the 3B widths, 2,048 tokens: 0.48 -> 0.16 ms; at the 8B widths, 7,001 tokens: 3.0 -> 0.5 ms.)"""
+        return ctx.n_tokens > 16 and 2 * ctx.n_logit_rows <= ctx.n_tokens and hasattr(ctx.kernels, "take_rows")

@@ -40,6 +40,8 @@ class MixtureOfExperts:
     correction, identity_experts, activation ("swiglu", the default, "clamped" or "gelu"), limit, shared_limit and
     router_bias (with softmax scores)."""
 
+    by_row = True     # a row of the result depends on that row of the input alone
+
     def __init__(self, params, env):
         self.hidden = int(params["hidden_size"])
         self.experts = int(params["experts"])

@@ -24,6 +24,8 @@ class SwiGLU:
 
     takes_scaled_rows = True   # the input goes to ``gated_linear`` only
 
+    by_row = True     # a row of the result depends on that row of the input alone
+
     def __init__(self, params, env):
         self.hidden = int(params["hidden_size"])
         self.inter = int(params["intermediate_size"])
