@@ -130,6 +130,118 @@ __global__ __launch_bounds__(512) void gla_recurrent_kernel(
     }
 }
 
+// A step of one token a sequence in bfloat16: a workgroup a (sequence, head), whose state of D x Dv floats is read and
+// written once, 16 bytes a lane in rows of the matrix, all of it under way at once.  Bound by those bytes and the way to
+// memory and back; what the kernel above does for such a step reads 4 bytes a lane, four rows an instruction.
+// Thread (group, quad) has four columns of rows group, group + G, ...; the groups' shares of the outputs are added by lane
+// exchanges and through LDS.  Dv a power of two from 16 to 256, D up to ROWS * G.
+// LOW_RANK: the decays exp(logsigmoid(a2 a + bias) / tau) are taken here, four lanes a channel, while the state is on
+// its way; else they come as floats.
+// 8 sequences of 24 heads of 128 x 128 (25 MB), rank 64: 15.5 us and 9.4 for the decays -> 10.9 for both.
+struct LowRank {
+    const bf16_t* a2;
+    const float* bias;
+    int a_col, rank;
+    float tau_inv;
+};
+template <int ROWS, bool BONUS, bool LOW_RANK>
+__global__ __launch_bounds__(512) void state_decode_kernel(
+    const bf16_t* __restrict__ proj, int row_stride, int q_col, int k_col, int v_col, int g_col,
+    const float* __restrict__ alpha, const LowRank low, const float* __restrict__ norm_w, float* __restrict__ state,
+    long long state_stride, const int* __restrict__ cu_q, const int* __restrict__ slots, bf16_t* __restrict__ out, int n_heads,
+    int D, int Dv, float q_scale, float eps, float* __restrict__ raw_out, const float* __restrict__ k_f32, int q_share,
+    const float* __restrict__ bonus) {
+    constexpr int WAVES = 8;
+    __shared__ float part[WAVES][256];
+    __shared__ float decay[LOW_RANK ? 512 : 1];
+    __shared__ float squares[WAVES];
+    const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
+    const int n = cu_q[seq];
+    if (cu_q[seq + 1] <= n) return;
+    const int quads = Dv / 4, G = 512 / quads, quad = tid % quads, group = tid / quads;
+    float* S_mem = state + (size_t)slots[seq] * state_stride + (size_t)head * D * Dv + 4 * quad;
+    float4 S[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) S[i] = *reinterpret_cast<const float4*>(S_mem + (size_t)min(group + i * G, D - 1) * Dv);
+    const bf16_t* row = proj + (size_t)n * row_stride;
+    const size_t at = ((size_t)n * n_heads + head) * D;
+    const bf16_t *q_row = row + q_col + head / q_share * D, *k_row = row + k_col + head / q_share * D;
+    float q[ROWS], k[ROWS], a[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        const int d = min(group + i * G, D - 1);
+        q[i] = bf16_to_float(q_row[d]) * q_scale;
+        k[i] = k_f32 ? k_f32[at + d] : bf16_to_float(k_row[d]);
+        if (!LOW_RANK) a[i] = alpha[at + d];
+    }
+    const uint2 v2 = *reinterpret_cast<const uint2*>(row + v_col + head * Dv + 4 * quad);
+    const float v[4] = {__uint_as_float(v2.x << 16), __uint_as_float(v2.x & 0xffff0000u), __uint_as_float(v2.y << 16),
+                        __uint_as_float(v2.y & 0xffff0000u)};
+    if (LOW_RANK) {
+        const uint4* in = reinterpret_cast<const uint4*>(row + low.a_col);
+        for (int c = tid / 4; c < D; c += 512 / 4) {      // four lanes a channel, pieces of eight in turn
+            const uint4* w = reinterpret_cast<const uint4*>(low.a2 + (size_t)(head * D + c) * low.rank);
+            float z = 0.f;
+            for (int m = tid % 4; m < low.rank / 8; m += 4) {
+                Vec8<bf16_t> x, y;
+                x.u = in[m];
+                y.u = w[m];
+                float xs[8], ys[8];
+                x.get(xs);
+                y.get(ys);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) z += xs[e] * ys[e];
+            }
+            z += __shfl_xor(z, 1, SIA_WAVE);
+            z += __shfl_xor(z, 2, SIA_WAVE);
+            if (tid % 4 == 0) decay[c] = expf(log_sigmoid(z + (low.bias ? low.bias[head * D + c] : 0.f)) * low.tau_inv);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) a[i] = decay[min(group + i * G, D - 1)];
+    }
+    float o[4] = {};
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        const int d = group + i * G;
+        if (d >= D) continue;
+        const float u = BONUS && !raw_out ? bonus[(size_t)head * D + d] : 0.f;
+        float s[4] = {S[i].x, S[i].y, S[i].z, S[i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float write = k[i] * v[e];
+            if (BONUS) o[e] += q[i] * (s[e] + u * write);
+            s[e] = a[i] * s[e] + write;
+            if (!BONUS) o[e] += q[i] * s[e];
+        }
+        *reinterpret_cast<float4*>(S_mem + (size_t)d * Dv) = make_float4(s[0], s[1], s[2], s[3]);
+    }
+    for (int off = quads; off < SIA_WAVE; off <<= 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] += __shfl_xor(o[e], off, SIA_WAVE);
+    const int wave = tid / SIA_WAVE, lane = tid % SIA_WAVE;
+    if (lane < quads) *reinterpret_cast<float4*>(&part[wave][4 * quad]) = make_float4(o[0], o[1], o[2], o[3]);
+    __syncthreads();
+    float y = 0.f;
+    if (tid < Dv)
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) y += part[w][tid];
+    if (raw_out) {
+        if (tid < Dv) raw_out[((size_t)n * n_heads + head) * Dv + tid] = y;
+        return;
+    }
+    const float ss = wave_sum(y * y);
+    if (lane == 0) squares[wave] = ss;
+    __syncthreads();
+    if (tid >= Dv) return;
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) total += squares[w];      // of threads beyond the columns: zeros
+    const float g = g_col >= 0 ? bf16_to_float(row[g_col + head * Dv + tid]) : 0.f;
+    out[((size_t)n * n_heads + head) * Dv + tid] =
+        float_to_bf16(y * rsqrtf(total / (float)Dv + eps) * norm_w[(BONUS ? head * Dv : 0) + tid] * (g_col >= 0 ? g / (1.f + expf(-g)) : 1.f));
+}
+
 // Sum over the 16 lanes of a row of a wave by lane exchanges inside the vector unit (no trip through LDS's crossbar):
 // neighbours, pairs of a quad, the mirrored half, the mirrored row.  Every lane of the row gets the sum.
 __device__ __forceinline__ float row16_sum(float v) {
@@ -715,6 +827,38 @@ SIA_EXPORT long long sia_gla_workspace(int n_tokens, int n_seqs, int max_q_len, 
     return (long long)n_tokens * n_heads * D + recurrence_space(n_tokens, n_heads, D, Dv);
 }
 
+// A step of one token a sequence, if the kernel for it takes these sizes and addresses; false with nothing done if not.
+static bool launch_state_decode(const void* proj, int row_stride, int q_col, int k_col, int v_col, int g_col, const float* k_f32,
+                                int q_share, const float* alpha, const LowRank* low, const float* norm_w, float* state,
+                                long long state_stride, const int* cu_q, const int* slots, void* out, int n_seqs, int max_q_len,
+                                int n_heads, int D, int Dv, float q_scale, float eps, int dtype, float* raw, hipStream_t stream,
+                                const float* bonus) {
+    const int rows = (D * (Dv / 4) + 511) / 512;      // of the state a thread has
+    if (max_q_len != 1 || dtype != SIA_BF16 || Dv < 16 || Dv > 256 || (Dv & (Dv - 1)) || rows > 16 || D > 512 || row_stride % 4 ||
+        v_col % 4 || state_stride % 4 || ((uintptr_t)proj % 8) || ((uintptr_t)state % 16) || n_heads > 65535)
+        return false;
+    if (low && (low->rank % 8 || low->a_col % 8 || row_stride % 8 || ((uintptr_t)proj % 16) || ((uintptr_t)low->a2 % 16))) return false;
+    const dim3 grid(n_seqs, n_heads), block(512);
+    const LowRank none{};
+#define DECODE_AS(ROWS, BONUS, LOW)                                                                                      \
+    hipLaunchKernelGGL((state_decode_kernel<ROWS, BONUS, LOW>), grid, block, 0, stream, (const bf16_t*)proj, row_stride, q_col, \
+                       k_col, v_col, g_col, alpha, low ? *low : none, norm_w, state, state_stride, cu_q, slots, (bf16_t*)out,   \
+                       n_heads, D, Dv, q_scale, eps, raw, k_f32, q_share, bonus)
+#define DECODE(ROWS)                                                                                                     \
+    do {                                                                                                                 \
+        if (bonus) DECODE_AS(ROWS, true, false);                                                                         \
+        else if (low) DECODE_AS(ROWS, false, true);                                                                      \
+        else DECODE_AS(ROWS, false, false);                                                                              \
+    } while (0)
+    if (rows <= 2) DECODE(2);
+    else if (rows <= 4) DECODE(4);
+    else if (rows <= 8) DECODE(8);
+    else DECODE(16);
+#undef DECODE
+#undef DECODE_AS
+    return true;
+}
+
 // The recurrence itself for a step's runs of tokens, whoever prepared its inputs: S <- diag(alpha) S + k v^T, o = S^T q.
 // q and v (and k, unless k_f32 gives it as floats [tokens, heads, D]) are columns of rows of the compute type; head h
 // reads the q (and such a k) of head h / q_share.  A sequence's matrices lie state_stride floats apart from the next
@@ -730,6 +874,12 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
                              int max_q_len, int n_heads, int D, int Dv, float q_scale, float eps, int dtype,
                              float* raw_space, bool want_raw, bool* raw_used, hipStream_t stream,
                              const float* bonus = nullptr) {
+    if (launch_state_decode(proj, row_stride, q_col, k_col, v_col, g_col, k_f32, q_share, alpha, nullptr, norm_w, state, state_stride,
+                            cu_q, slots, out, n_seqs, max_q_len, n_heads, D, Dv, q_scale, eps, dtype, want_raw ? raw_space : nullptr,
+                            stream, bonus)) {
+        if (raw_used) *raw_used = want_raw;
+        return 0;
+    }
     // columns a workgroup: all of a head's, or with a workspace a slice of them, as narrow as it takes to fill the chip
     int slice = Dv;
     const bool prompt = gla_slices(n_seqs, max_q_len, n_heads);
@@ -918,6 +1068,11 @@ SIA_EXPORT int sia_gla_recurrent(const void* proj, int row_stride, int q_col, in
         return SIA_BAD_ARGUMENT;
     float* alpha = workspace;
     float* raw_space = workspace + (size_t)n_tokens * n_heads * D;
+    const LowRank low{(const bf16_t*)a2, a2_bias, a_col, rank, 1.f / tau};
+    if (launch_state_decode(proj, row_stride, q_col, k_col, v_col, g_col, nullptr, 1, nullptr, &low, norm_w, state,
+                            (long long)n_heads * D * Dv, cu_q, slots, out, n_seqs, max_q_len, n_heads, D, Dv, q_scale, eps, dtype,
+                            nullptr, stream, nullptr))
+        return SIA_LAUNCH_CHECK();
     {
         const int channels = n_heads * D;
         dim3 dgrid((n_tokens + GLA_DECAY_TOKENS - 1) / GLA_DECAY_TOKENS, (channels + 255) / 256), dblock(256);

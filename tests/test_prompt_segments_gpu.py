@@ -69,3 +69,25 @@ def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, len
     assert float((state - want).abs().max()) <= 2e-5 * float(want.abs().max())
     assert bool(((whole - cut).abs() <= 2.0 ** -7 * cut.abs() + 1e-3 * float(cut.std())).all()), float((whole - cut).abs().max())
     assert float(state[len(lengths):].abs().max()) == 0.0        # nobody else's slot was touched
+
+
+# narrow and wide values, rows that do not divide by the groups of threads, the most rows a thread takes; value widths that
+# are no power of two go the general way
+@pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
+@pytest.mark.parametrize("H,D,Dv", [(3, 7, 16), (2, 128, 256), (1, 512, 16), (2, 100, 32), (3, 128, 128), (2, 33, 64), (2, 40, 20)])
+def test_steps_of_one_token_are_the_portion_walked_along(op, H, D, Dv):
+    """As above, with the sums over a column in another order: relative 2^-23 a term."""
+    from simple_inference_amd.kernels import HipKernels
+
+    if op == "bonus":
+        D = Dv if Dv & (Dv - 1) == 0 else D
+        Dv = D
+    k = HipKernels()
+    g = torch.Generator().manual_seed(H * D)
+    lengths = [9, 1, 6]
+    rows, _ = lowered(rnd(g, sum(lengths), 2 * H * D + 2 * H * Dv + 2 * D + H + 32 + (-(2 * H * D + 2 * H * Dv + 2 * D + H)) % 8),
+                      torch.bfloat16, DEV)
+    one, state = run(op, k, rows, H, D, Dv, lengths, 1)
+    whole, want = run(op, k, rows, H, D, Dv, lengths, 10 ** 6)
+    assert float((state - want).abs().max()) <= 2e-6 * float(want.abs().max())
+    assert bool(((one - whole).abs() <= 2.0 ** -7 * whole.abs() + 1e-3 * float(whole.std())).all()), float((one - whole).abs().max())
