@@ -173,6 +173,7 @@ class DecoderModel:
     def _few_rows_read(ctx: StepContext) -> bool:
         """Whether the last layer's results are read at so few of the step's rows that going on with those alone pays
         (what a layer writes for later steps, keys, values and states, it writes for all): a prompt's portion needs its
-        last row, or none.  Steps of up to 16 rows are bound by reading the weights, whatever their rows.  (A prompt's last
-        layer at the 3B widths, 2,048 tokens: 0.48 -> 0.16 ms; at the 8B widths, 7,001 tokens: 3.0 -> 0.5 ms.)"""
-        return ctx.n_tokens > 16 and 2 * ctx.n_logit_rows <= ctx.n_tokens and hasattr(ctx.kernels, "take_rows")
+        last row, or none.  (A prompt's last layer at the 3B widths, 2,048 tokens: 0.48 -> 0.16 ms; at the 8B widths, 7,001
+        tokens: 3.0 -> 0.5 ms.)  Steps of fewer rows are bound by reading the weights, and keep the one call a layer: eight
+        layers at 33 rows 918 -> 896 us (3B widths) and 731 -> 731 (1B), at 24 rows 827 -> 814 and 722 -> 727."""
+        return ctx.n_tokens >= 32 and 2 * ctx.n_logit_rows <= ctx.n_tokens and hasattr(ctx.kernels, "take_rows")
