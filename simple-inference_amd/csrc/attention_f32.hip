@@ -167,10 +167,12 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
                     p_w[h * CHUNK + lane] = p;
                 }
                 __builtin_amdgcn_wave_barrier();      // the wave's LDS accesses run in order: no more than that is needed
-                // values of keys that the row does not see may be anything: they are left out, not weighted with 0
+                // values of keys that the row does not see may be anything: they are left out, not weighted with 0.  In a
+                // chunk with kept positions that are those from `gap` to the window too.
                 const int j_first = c0 < keep ? 0 : max(lo, c0) - c0, j_last = min(pos, c0 + CHUNK - 1) - c0;
+                const int gap = c0 < keep ? keep - c0 : j_first, gap_end = c0 < keep ? lo - c0 : j_first;
                 for (int jj = j_first & ~3; jj <= j_last; jj += 4) {
-                    const bool whole = jj >= j_first && jj + 3 <= j_last;
+                    const bool whole = jj >= j_first && jj + 3 <= j_last && (jj + 3 < gap || jj >= gap_end);
                     f32x4 pp[HB];
 #pragma unroll
                     for (int h = 0; h < HB; ++h) pp[h] = *(const f32x4*)(p_w + h * CHUNK + jj);
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
                         if (!whole)
 #pragma unroll
                             for (int e = 0; e < 4; ++e)
-                                if (jj + e < j_first || jj + e > j_last) vv[e] = 0.f;
+                                if (jj + e < j_first || jj + e > j_last || (jj + e >= gap && jj + e < gap_end)) vv[e] = 0.f;
 #pragma unroll
                         for (int h = 0; h < HB; ++h)
 #pragma unroll

@@ -458,6 +458,26 @@ def test_float32_attention_is_the_plain_kernels(hip, geom):
             assert torch.equal(got[:at], whole[:at]) and torch.equal(got[at + 1:], whole[at + 1:])
 
 
+# kept positions that end inside a four, at its end, and in the second and third chunk of keys
+@pytest.mark.parametrize("keep", [3, 4, 61, 64, 130])
+def test_float32_attention_leaves_out_values_between_the_kept_positions_and_the_window(hip, keep):
+    """What lies in the pages between the kept first positions and a row's window does not reach the row: with infinities
+    and values that are no numbers there, every result has the bits that it has without."""
+    n_heads, n_kv, D, ps, window = 8, 2, 64, 16, 50
+    q_lens, kv_lens = [1, 1, 40], [300, 500, 260]
+    ctx = Ctx(q_lens, kv_lens)
+    cache = Cache(sum(-(-kv // ps) for kv in kv_lens), n_kv, ps, D, torch.float32, kv_lens, seed=3)
+    cache.k_pages.copy_(rnd(*cache.k_pages.shape, seed=4))
+    cache.v_pages.copy_(rnd(*cache.v_pages.shape, seed=5))
+    qkv = rnd(ctx.n_tokens, (n_heads + n_kv) * D, seed=6)
+    attend = lambda: hip.paged_attention(qkv, n_heads, n_kv, D, 0.3, window, ctx, cache, keep_first=keep)
+    want = attend()
+    for s, (q, kv) in enumerate(zip(q_lens, kv_lens)):
+        for j in range(keep, kv - q - window + 1):      # what no row of the sequence sees
+            cache.v_pages[cache.block_table[s, j // ps], :, :, j % ps] = float("inf") if j % 2 else float("nan")
+    assert want.isfinite().all() and torch.equal(attend(), want)
+
+
 @pytest.mark.parametrize("geom", [
     # heads, kv heads, head_dim, page_size, window
     (24, 8, 128, 16, None), (32, 8, 64, 64, None), (16, 1, 32, 8, None), (6, 2, 48, 16, 100), (5, 5, 112, 32, 700),
