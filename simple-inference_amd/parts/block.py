@@ -22,6 +22,7 @@ kernel of the norm that follows.
 
 from __future__ import annotations
 
+from .context import BiasedDelta, NormedSum, ScaledSum
 from .registry import register_block
 
 
@@ -104,12 +105,23 @@ def _mixed_rows(mixer, h, ctx, cache, rows):
     all of it."""
     if not getattr(mixer, "gives_only_rows", lambda: False)():
         y = mixer.forward(h, ctx, cache)
-        return ctx.kernels.take_rows(y.compute() if hasattr(y, "compute") else y, rows) if rows.numel() else None
+        return _rows_of(y, rows, ctx.kernels) if rows.numel() else None
     ctx.only_rows = rows
     try:
         return mixer.forward(h, ctx, cache)
     finally:
         ctx.only_rows = None
+
+
+def _rows_of(y, rows, kernels):
+    """A sublayer's result at ``rows`` alone, in the form in which it was left: a sum or a bias that whoever adds it into
+    the residual takes in float32 is not rounded to the compute dtype on the way."""
+    take = lambda t: kernels.take_rows(t, rows)
+    if isinstance(y, (ScaledSum, NormedSum)):
+        return type(y)([(take(t), *rest) for t, *rest in y.values()], kernels)
+    if isinstance(y, BiasedDelta):
+        return BiasedDelta(take(y.value()), y.bias, kernels)
+    return take(y.compute() if hasattr(y, "compute") else y)
 
 
 def _normed(norm, consumer, stream):
