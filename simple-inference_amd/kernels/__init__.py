@@ -419,9 +419,9 @@ class HipKernels:
         self._want(rows, "rows", torch.int32)
         n = rows.numel()
         out = torch.empty((n, *x.shape[1:]), dtype=x.dtype, device=x.device)
-        if n:
-            self._check(self.core.sia_take_rows(_ptr(x), _ptr(rows), _ptr(out), n, x.stride(0) * x.element_size(), self._stream()),
-                        "take_rows")
+        if out.numel():      # (a single row's stride says nothing: it may be one of a wider matrix)
+            self._check(self.core.sia_take_rows(_ptr(x), _ptr(rows), _ptr(out), n, out.numel() // n * out.element_size(),
+                                                self._stream()), "take_rows")
         return out
 
     def rows_alone(self, rows, ctx, cache):

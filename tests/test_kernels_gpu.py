@@ -72,6 +72,19 @@ def test_embed(hip, dtype, hidden):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [1, 33, 4096, 70000])
+def test_take_rows(hip, dtype, width):
+    """Rows of every width and alignment; a matrix of one row, whose stride is that of the wider matrix it comes from."""
+    x = rnd(9, width, dtype=dtype, seed=1)
+    rows = torch.tensor([8, 0, 3, 3], dtype=torch.int32, device=DEV)
+    assert torch.equal(hip.take_rows(x, rows), x[rows.long()])
+    assert hip.take_rows(x, rows[:0]).shape == (0, width)
+    one = rnd(1, 3 * width, dtype=dtype, seed=2)[:, :width]
+    assert one.is_contiguous() and one.stride(0) == 3 * width
+    assert torch.equal(hip.take_rows(one, rows[1:2].repeat(2)), one.repeat(2, 1))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hidden", [40, 1000, 3072, 5000])
 def test_add_rmsnorm(hip, dtype, hidden):
     res = rnd(7, hidden, seed=1, scale=3.0)
