@@ -270,11 +270,19 @@ __device__ __forceinline__ float row16_sum_of_four(const float (&v)[4], int r) {
     return c + moved(c, by8());
 }
 
-// Where a segment's state lies among those of the step: segments of seg_len tokens, which do not overlap, begin in different
-// multiples of it; the last ones of their sequences, which may be shorter, have the odd places (two of them lie at
-// least a whole segment apart).
-__device__ __forceinline__ int segment_place(int first, bool last_of_sequence, int seg_len) {
-    return 2 * (first / seg_len) + (last_of_sequence ? 1 : 0);
+// How a step's runs of tokens are cut into segments: of ``len`` tokens (0: not at all), the last of a sequence perhaps shorter.
+struct Segments {
+    int len;
+    bool by_sequence;      // of the two ways to place their states below, whichever needs fewer places
+};
+
+// Where a segment's state lies among those of the step.  By sequence: from one segment to the next either its first
+// token moves on by a whole length or the sequence is the next one.  Else: segments of full length, which do not overlap,
+// begin in different multiples of it; the last ones of their sequences have the odd places (two of them lie at least a
+// whole segment apart).
+__device__ __forceinline__ int segment_place(int first, int end, int seq, Segments cut) {
+    const int multiple = first / cut.len;
+    return cut.by_sequence ? multiple + seq : 2 * multiple + (first + cut.len >= end ? 1 : 0);
 }
 
 // The walk alone, for a prompt's step in bfloat16 whose heads' columns are shared out (D a multiple of 8, rows and
@@ -294,7 +302,7 @@ constexpr int gla_walk_tokens(int columns) { return columns == 4 ? 16 : 32; }
 // after the sequence before it.
 // BEFORE: the query reads the state before this token's write.
 //
-// Segments (seg_len > 0): a sequence of more than seg_len tokens is cut into segments of that many, walked by workgroups of
+// Segments (cut.len > 0): a sequence of more than so many tokens is cut into segments of that length, walked by workgroups of
 // their own at the same time: the first from the request's state, the others from zero.  Every segment leaves its last
 // state in ``seg_state``; the kernels behind this one add what the states in front of the segments contribute.
 template <int ROWS, int GLA_WALK_COLS, bool KF, bool BEFORE>
@@ -302,7 +310,7 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
     const bf16_t* __restrict__ proj, int row_stride, int q_col, int k_col, int v_col, const float* __restrict__ alpha,
     const float* __restrict__ k_f32, int q_share, float* __restrict__ state, long long state_stride,
     const int* __restrict__ cu_q, const int* __restrict__ slots, int n_heads, int D, int Dv, float q_scale,
-    float* __restrict__ raw_out, int seg_len, float* __restrict__ seg_state) {
+    float* __restrict__ raw_out, Segments cut, float* __restrict__ seg_state) {
     extern __shared__ float lds[];
     constexpr int C = GLA_WALK_COLS, TB = gla_walk_tokens(C), threads = GLA_WALK_THREADS;
     constexpr int slice = threads / 16 * C;      // columns a workgroup
@@ -310,10 +318,10 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
     const int seq = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
     const int n_slices = (Dv + slice - 1) / slice;
     const int j0 = blockIdx.z % n_slices * slice, seg = blockIdx.z / n_slices;
-    const int first = cu_q[seq] + seg * seg_len, end = cu_q[seq + 1];
+    const int first = cu_q[seq] + seg * cut.len, end = cu_q[seq + 1];
     if (first >= end) return;
-    const bool cut = seg_len > 0 && end - cu_q[seq] > seg_len;
-    const int last = cut ? min(first + seg_len, end) : end;
+    const bool is_cut = cut.len > 0 && end - cu_q[seq] > cut.len;
+    const int last = is_cut ? min(first + cut.len, end) : end;
     float* q_s = lds;               // [TB][Dp], row d = r * ROWS + i at (i / 4) * 64 + r * 4 + i % 4
     float* k_s = q_s + TB * Dp;
     float* al_s = k_s + TB * Dp;
@@ -331,7 +339,7 @@ __global__ __launch_bounds__(GLA_WALK_THREADS) void gla_walk_kernel(
             const int d = r * ROWS + i, j = j0 + jl + c;
             S[c][i] = (seg == 0 && j < Dv && d < D) ? S_mem[(size_t)d * Dv + j] : 0.f;
         }
-    if (cut) S_mem = seg_state + ((size_t)segment_place(first, last == end, seg_len) * n_heads + head) * D * Dv;
+    if (is_cut) S_mem = seg_state + ((size_t)segment_place(first, end, seq, cut) * n_heads + head) * D * Dv;
     const int d8 = D / 8, d4 = D / 4;
     const int q_at = q_col + (head / q_share) * D, k_at = k_col + (head / q_share) * D;
     // What is on its way from memory is held in named registers, and the two steps below are written out piece by
@@ -549,13 +557,13 @@ __global__ __launch_bounds__(256) void segment_decays_kernel(float* __restrict__
 __global__ __launch_bounds__(256) void segment_states_kernel(const float* __restrict__ decays, float* __restrict__ seg_state,
                                                              float* __restrict__ state, long long state_stride,
                                                              const int* __restrict__ cu_q, const int* __restrict__ slots,
-                                                             int n_heads, int D, int Dv, int seg_len) {
+                                                             int n_heads, int D, int Dv, Segments cut) {
     const int seq = blockIdx.z, head = blockIdx.y, at = (blockIdx.x * 256 + threadIdx.x) * 4;
-    const int begin = cu_q[seq], end = cu_q[seq + 1];
+    const int begin = cu_q[seq], end = cu_q[seq + 1], seg_len = cut.len;
     if (end - begin <= seg_len || at >= D * Dv) return;
     const int d = at / Dv;
     auto matrix = [&](int first) {
-        return reinterpret_cast<float4*>(seg_state + ((size_t)segment_place(first, first + seg_len >= end, seg_len) * n_heads + head) * D * Dv + at);
+        return reinterpret_cast<float4*>(seg_state + ((size_t)segment_place(first, end, seq, cut) * n_heads + head) * D * Dv + at);
     };
     auto decay = [&](int first) { return decays[((size_t)(min(first + seg_len, end) - 1) * n_heads + head) * D + d]; };
     float4 S = *matrix(begin), local = *matrix(begin + seg_len);
@@ -584,8 +592,8 @@ template <bool BEFORE>
 __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __restrict__ proj, int row_stride, int q_col, int q_share,
                                                               const float* __restrict__ decays, const float* __restrict__ seg_state,
                                                               const int* __restrict__ cu_q, int n_heads, int D, int Dv, float q_scale,
-                                                              float* __restrict__ raw, int seg_len) {
-    const int seq = blockIdx.z, head = blockIdx.y % n_heads, j0 = blockIdx.y / n_heads * 64;
+                                                              float* __restrict__ raw, Segments cut) {
+    const int seq = blockIdx.z, head = blockIdx.y % n_heads, j0 = blockIdx.y / n_heads * 64, seg_len = cut.len;
     const int first = cu_q[seq] + (blockIdx.x + 1) * seg_len, end = cu_q[seq + 1];
     const int t0 = first + threadIdx.x / SIA_WAVE * 32;
     if (t0 >= end) return;      // a wave leaves as a whole; no barriers below
@@ -593,7 +601,7 @@ __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __re
     const int lane = threadIdx.x % SIA_WAVE, r = lane % 16, g = lane / 16;
     const int j = j0 + 4 * r;
     const bool has_j = j < Dv;      // Dv is a multiple of four
-    const float* S = seg_state + ((size_t)segment_place(first, first + seg_len >= end, seg_len) * n_heads + head) * D * Dv + (has_j ? j : 0);
+    const float* S = seg_state + ((size_t)segment_place(first, end, seq, cut) * n_heads + head) * D * Dv + (has_j ? j : 0);
     const int q_at = q_col + head / q_share * D;
 
     segf32x4 acc[2][4];      // [tile of 16 tokens][column of the four] = tokens 4 g .. 4 g + 3
@@ -815,16 +823,40 @@ static bool gla_slices(int n_seqs, int max_q_len, int n_heads) {
 #define SEG_MIN 64
 #define SEG_MIN_PROMPT 128
 
+static long long segment_places(int n_tokens, int n_seqs, Segments cut) {
+    if (cut.len == 0) return 0;
+    const long long multiples = (n_tokens - 1) / cut.len + 1;
+    return cut.by_sequence ? multiples + n_seqs - 1 : 2 * multiples;
+}
+
+// How a step is cut, from its sizes alone, so that whoever makes the workspace and whoever launches agree.
+// A step of few and long sequences leaves most of the chip idle behind the walk's chain of tokens: it is cut into
+// segments, long ones where there are enough of them.  (Workgroups the step keeps busy without: the tokens
+// over the longest run, times heads and slices.)  2,048 tokens of 24 heads of 128: one walk of 96 workgroups 740 us; 16
+// segments 177 with two columns a lane group, 121 with four (LDS serves twice the columns, 140 registers), and 53 for
+// the decays' products, the states and the outputs behind it (100 MB of states and outputs).
+static Segments segments_of(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv, int dtype) {
+    const Segments none{0, false};
+    const int slices = (Dv + 63) / 64;
+    if (dtype != SIA_BF16 || max_q_len < SEG_MIN_PROMPT || D % 8 || D > 256 || Dv % 4 || n_seqs > 65535 ||
+        (long long)n_heads * slices > 65535)
+        return none;
+    if ((long long)(n_tokens / max_q_len) * n_heads * slices >= 768) return none;
+    const int len = (long long)n_tokens * n_heads * slices / (2 * SEG_MIN) >= 768 ? 2 * SEG_MIN : SEG_MIN;
+    if ((long long)slices * ((max_q_len + len - 1) / len) > 65535) return none;      // a grid's third number
+    const Segments by_sequence{len, true}, apart{len, false};
+    return segment_places(n_tokens, n_seqs, by_sequence) <= segment_places(n_tokens, n_seqs, apart) ? by_sequence : apart;
+}
+
 // The raw outputs [tokens, heads, Dv] as floats, and behind them the states of the step's segments.
-static long long recurrence_space(int n_tokens, int n_heads, int D, int Dv) {
-    const long long states = n_tokens >= SEG_MIN_PROMPT ? 2 * (n_tokens / SEG_MIN + 1) : 0;
+static long long recurrence_space(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv, int dtype) {
+    const long long states = segment_places(n_tokens, n_seqs, segments_of(n_tokens, n_seqs, max_q_len, n_heads, D, Dv, dtype));
     return (long long)n_tokens * n_heads * Dv + states * n_heads * D * Dv;
 }
 
 // Floats of workspace a step of n_tokens needs: the decays [tokens, heads, D], and the space above.
-SIA_EXPORT long long sia_gla_workspace(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv) {
-    (void)n_seqs; (void)max_q_len;
-    return (long long)n_tokens * n_heads * D + recurrence_space(n_tokens, n_heads, D, Dv);
+SIA_EXPORT long long sia_gla_workspace(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv, int dtype) {
+    return (long long)n_tokens * n_heads * D + recurrence_space(n_tokens, n_seqs, max_q_len, n_heads, D, Dv, dtype);
 }
 
 // A step of one token a sequence, if the kernel for it takes these sizes and addresses; false with nothing done if not.
@@ -920,22 +952,16 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
     float* raw = (sliced || ahead || want_raw) ? raw_space : nullptr;
     if (raw_used) *raw_used = raw != nullptr;
     if (ahead) {
-        // A step of few and long sequences leaves most of the chip idle behind the walk's chain of tokens: it is cut into
-        // segments, long ones where there are enough of them.  (Workgroups the step keeps busy without: the tokens
-        // over the longest run, times heads and slices.)  2,048 tokens of 24 heads of 128: one walk of 96 workgroups 740 us; 16
-        // segments 177 with two columns a lane group, 121 with four (LDS serves twice the columns, 140 registers), and 53 for
-        // the decays' products, the states and the outputs behind it (100 MB of states and outputs).
         const int w_slices = (Dv + w_slice - 1) / w_slice;
-        const long long busy = (long long)(n_tokens / max_q_len) * n_heads * w_slices;
-        const bool segments = long_runs && busy < 768;
-        const int seg_len = !segments ? 0 : (long long)n_tokens * n_heads * w_slices / (2 * SEG_MIN) >= 768 ? 2 * SEG_MIN : SEG_MIN;
-        const int n_segs = segments ? (max_q_len + seg_len - 1) / seg_len : 1;
+        Segments cut{0, false};
+        if (long_runs) cut = segments_of(n_tokens, n_seqs, max_q_len, n_heads, D, Dv, dtype);
+        const int seg_len = cut.len, n_segs = seg_len ? (max_q_len + seg_len - 1) / seg_len : 1;
         float* seg_state = raw_space + (size_t)n_tokens * n_heads * Dv;
         dim3 wgrid(n_seqs, n_heads, w_slices * n_segs), wblock(GLA_WALK_THREADS);
 #define WALK_AS(ROWS, COLS, KF, BEFORE)                                                                                      \
     hipLaunchKernelGGL((gla_walk_kernel<ROWS, COLS, KF, BEFORE>), wgrid, wblock, w_lds, stream, (const bf16_t*)proj,         \
                        row_stride, q_col, k_col, v_col, alpha, k_f32, q_share, state, state_stride, cu_q, slots,     \
-                       n_heads, D, Dv, q_scale, raw, seg_len, seg_state)
+                       n_heads, D, Dv, q_scale, raw, cut, seg_state)
 #define WALK(ROWS, COLS)                                                                                             \
     do {                                                                                                             \
         if (bonus) WALK_AS(ROWS, COLS, false, true);                                                                 \
@@ -955,14 +981,14 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
             hipLaunchKernelGGL(segment_decays_kernel, dim3(n_segs - 1, (channels + 255) / 256, n_seqs), dim3(256), 0, stream, alpha,
                                cu_q, channels, seg_len);
             hipLaunchKernelGGL(segment_states_kernel, dim3((D * Dv / 4 + 255) / 256, n_heads, n_seqs), dim3(256), 0, stream, alpha,
-                               seg_state, state, state_stride, cu_q, slots, n_heads, D, Dv, seg_len);
+                               seg_state, state, state_stride, cu_q, slots, n_heads, D, Dv, cut);
             const dim3 ogrid(n_segs - 1, n_heads * ((Dv + 63) / 64), n_seqs), oblock(seg_len / 32 * SIA_WAVE);
             if (bonus)
                 hipLaunchKernelGGL(segment_outputs_kernel<true>, ogrid, oblock, 0, stream, (const bf16_t*)proj, row_stride, q_col,
-                                   q_share, alpha, seg_state, cu_q, n_heads, D, Dv, q_scale, raw, seg_len);
+                                   q_share, alpha, seg_state, cu_q, n_heads, D, Dv, q_scale, raw, cut);
             else
                 hipLaunchKernelGGL(segment_outputs_kernel<false>, ogrid, oblock, 0, stream, (const bf16_t*)proj, row_stride, q_col,
-                                   q_share, alpha, seg_state, cu_q, n_heads, D, Dv, q_scale, raw, seg_len);
+                                   q_share, alpha, seg_state, cu_q, n_heads, D, Dv, q_scale, raw, cut);
         }
     } else {
 #define LAUNCH_AS(T, ROWS, BONUS)                                                                                    \
@@ -1024,8 +1050,8 @@ __global__ __launch_bounds__(4 * SIA_WAVE) void bonus_finish_kernel(const float*
 }
 
 // floats of workspace behind the decays
-SIA_EXPORT long long sia_bonus_recurrence_workspace(int n_tokens, int n_heads, int D) {
-    return recurrence_space(n_tokens, n_heads, D, D);
+SIA_EXPORT long long sia_bonus_recurrence_workspace(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int dtype) {
+    return recurrence_space(n_tokens, n_seqs, max_q_len, n_heads, D, D, dtype);
 }
 
 // The recurrence with a bonus for the current token: rkvg is four matrices [tokens, heads * D] one behind the other (r, k, v
@@ -1126,8 +1152,8 @@ __global__ __launch_bounds__(256) void hgrn2_prepare_kernel(T* __restrict__ proj
 }
 
 // floats of workspace: the gates and their complements [tokens, heads, D] each, the recurrence's own
-SIA_EXPORT long long sia_hgrn2_workspace(int n_tokens, int n_heads, int D, int Dv) {
-    return 2LL * n_tokens * n_heads * D + recurrence_space(n_tokens, n_heads, D, Dv);
+SIA_EXPORT long long sia_hgrn2_workspace(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv, int dtype) {
+    return 2LL * n_tokens * n_heads * D + recurrence_space(n_tokens, n_seqs, max_q_len, n_heads, D, Dv, dtype);
 }
 
 SIA_EXPORT int sia_hgrn2_scan(void* proj, int row_stride, const float* f_bias, const float* lower, const float* norm_w,
@@ -1211,8 +1237,8 @@ __global__ __launch_bounds__(256) void ssd_finish_kernel(const float* __restrict
     }
 }
 
-SIA_EXPORT long long sia_ssd_workspace(int n_tokens, int n_heads, int N, int P) {
-    return 2LL * n_tokens * n_heads * N + recurrence_space(n_tokens, n_heads, N, P);
+SIA_EXPORT long long sia_ssd_workspace(int n_tokens, int n_seqs, int max_q_len, int n_heads, int N, int P, int dtype) {
+    return 2LL * n_tokens * n_heads * N + recurrence_space(n_tokens, n_seqs, max_q_len, n_heads, N, P, dtype);
 }
 
 SIA_EXPORT int sia_ssd_scan(const void* proj, int row_stride, const void* xbc, int xbc_stride, const float* dt_bias,

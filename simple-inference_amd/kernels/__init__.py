@@ -50,7 +50,7 @@ _SIGNATURES = {
                         _c_int, _c_ptr],
     "sia_gemm_skinny_grouped": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "sia_low_rank_decay": [_c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_ptr],
-    "sia_bonus_recurrence_workspace": [_c_int, _c_int, _c_int],
+    "sia_bonus_recurrence_workspace": [_c_int] * 6,
     "sia_bonus_recurrence": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
                              _c_int, _c_int, _c_float, _c_int, _c_ptr, _c_ptr],
     "sia_moe_route_biased": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
@@ -69,7 +69,7 @@ _SIGNATURES = {
     "sia_gla_recurrent": [_c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                           _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float,
                           _c_int, _c_ptr, _c_int, _c_ptr],
-    "sia_gla_workspace": [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int],
+    "sia_gla_workspace": [_c_int] * 7,
     "sia_moe_route": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "sia_moe_route_ex": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                          _c_float, _c_ptr],
@@ -77,10 +77,10 @@ _SIGNATURES = {
                      _c_int, _c_int, _c_int, _c_ptr],
     "sia_causal_conv": [_c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
-    "sia_hgrn2_workspace": [_c_int, _c_int, _c_int, _c_int],
+    "sia_hgrn2_workspace": [_c_int] * 7,
     "sia_hgrn2_scan": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int,
                        _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr, _c_ptr],
-    "sia_ssd_workspace": [_c_int, _c_int, _c_int, _c_int],
+    "sia_ssd_workspace": [_c_int] * 7,
     "sia_ssd_scan": [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_ptr, _c_ptr,
                      _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr,
                      _c_ptr],
@@ -794,7 +794,7 @@ class HipKernels:
         out = torch.empty((n, n_heads * value_dim), dtype=proj.dtype, device=proj.device)
         # float scratch for the decays and, where a prompt's step shares a head's columns out between workgroups, for
         # their raw outputs (kept with the step: its layers run in turn)
-        floats = self.core.sia_gla_workspace(n, ctx.n_seqs, ctx.max_q_len, n_heads, key_dim, value_dim)
+        floats = self.core.sia_gla_workspace(n, ctx.n_seqs, ctx.max_q_len, n_heads, key_dim, value_dim, _DT[proj.dtype])
         workspace = getattr(ctx, "recurrent_workspace", None)
         if workspace is None or workspace.numel() < floats:
             workspace = torch.empty((floats,), dtype=torch.float32, device=proj.device)
@@ -1010,7 +1010,8 @@ class HipKernels:
         stride = self._state_rows(state, ctx, inner * head_dim)
         out = torch.empty((n, inner), dtype=rkvg.dtype, device=rkvg.device)
         decays = n * inner + (-n * inner) % 4
-        workspace = self._float_workspace(ctx, decays + self.core.sia_bonus_recurrence_workspace(n, n_heads, head_dim), rkvg.device)
+        floats = self.core.sia_bonus_recurrence_workspace(n, ctx.n_seqs, ctx.max_q_len, n_heads, head_dim, _DT[rkvg.dtype])
+        workspace = self._float_workspace(ctx, decays + floats, rkvg.device)
         raw = workspace[decays:]
         self._check(self.core.sia_low_rank_decay(_ptr(low), rank, rank, _ptr(w2), _ptr(w0), inner, _ptr(workspace), n,
                                                  _DT[rkvg.dtype], self._stream()), "low_rank_decay")
@@ -1080,7 +1081,8 @@ class HipKernels:
             raise KernelError(f"{n_heads} heads of {head_dim} do not split into {groups} groups and {norm_groups} parts")
         stride = self._state_rows(state, ctx, n_heads * state_size * head_dim)
         out = torch.empty((n, inner), dtype=proj.dtype, device=proj.device)
-        workspace = self._float_workspace(ctx, self.core.sia_ssd_workspace(n, n_heads, state_size, head_dim), proj.device)
+        workspace = self._float_workspace(ctx, self.core.sia_ssd_workspace(n, ctx.n_seqs, ctx.max_q_len, n_heads, state_size, head_dim,
+                                                                           _DT[proj.dtype]), proj.device)
         self._check(self.core.sia_ssd_scan(
             _ptr(proj), width, _ptr(xbc), xbc.shape[1], _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(norm_weight),
             _ptr(state), stride, _ptr(ctx.cu_q), _ptr(ctx.state_slots), _ptr(out), n, ctx.n_seqs, ctx.max_q_len, n_heads,
@@ -1108,7 +1110,8 @@ class HipKernels:
             raise KernelError(f"state rows are not [{n_heads}, {key_dim}, {value_dim}]")
         self._state_rows(state, ctx, qk * value_dim)
         out = torch.empty((n, n_heads * value_dim), dtype=proj.dtype, device=proj.device)
-        workspace = self._float_workspace(ctx, self.core.sia_hgrn2_workspace(n, n_heads, key_dim, value_dim), proj.device)
+        workspace = self._float_workspace(ctx, self.core.sia_hgrn2_workspace(n, ctx.n_seqs, ctx.max_q_len, n_heads, key_dim, value_dim,
+                                                                             _DT[proj.dtype]), proj.device)
         self._check(self.core.sia_hgrn2_scan(
             _ptr(proj), width, _ptr(f_bias), _ptr(lower), _ptr(norm_weight), _ptr(state), _ptr(ctx.cu_q),
             _ptr(ctx.state_slots), _ptr(out), n, ctx.n_seqs, ctx.max_q_len, n_heads, key_dim, value_dim, float(eps),
@@ -1212,7 +1215,7 @@ class HipKernels:
         self._state_rows(state, ctx, qk * value_dim)
         out = torch.empty((n, inner), dtype=proj.dtype, device=proj.device)
         workspace = self._float_workspace(
-            ctx, self.core.sia_gla_workspace(n, ctx.n_seqs, ctx.max_q_len, n_heads, key_dim, value_dim), proj.device)
+            ctx, self.core.sia_gla_workspace(n, ctx.n_seqs, ctx.max_q_len, n_heads, key_dim, value_dim, _DT[proj.dtype]), proj.device)
         self._check(self.core.sia_decay_attention(
             _ptr(proj), width, _ptr(decays), _ptr(norm_weight), _ptr(state), _ptr(ctx.cu_q), _ptr(ctx.state_slots),
             _ptr(out), n, ctx.n_seqs, ctx.max_q_len, n_heads, key_dim, value_dim, float(eps), _DT[proj.dtype],

@@ -12,7 +12,8 @@ DEV = "cuda:0"
 
 
 def run(op, k, rows, H, D, Dv, lengths, portion):
-    """Outputs and states of the sequences, every step bringing each of them up to ``portion`` more tokens."""
+    """Outputs and states of the sequences, every step bringing each of them up to ``portion`` more tokens, and whether any
+    step was cut: whether it wrote into its workspace behind the decays and the raw outputs."""
     g = torch.Generator().manual_seed(5)
     f32 = lambda t: t.float().to(DEV)
     bf16 = lambda t: t.to(torch.bfloat16).to(DEV)
@@ -22,12 +23,14 @@ def run(op, k, rows, H, D, Dv, lengths, portion):
     per_head, decays = f32(1 + rnd(g, H * Dv, std=0.2)), f32(0.9 + 0.0999 * torch.rand(H, generator=g))
     a2, out = bf16(rnd(g, H * D, 32, std=0.3)), torch.empty(sum(lengths), H * Dv)
     offsets, at = [sum(lengths[:s]) for s in range(len(lengths))], [0] * len(lengths)
+    was_cut = False
     while any(a < n for a, n in zip(at, lengths)):
         who = [s for s, n in enumerate(lengths) if at[s] < n]
         lens = [min(portion, lengths[s] - at[s]) for s in who]
         idx = torch.cat([torch.arange(offsets[s] + at[s], offsets[s] + at[s] + n) for s, n in zip(who, lens)])
         ctx, x = context(DEV, lens, who), rows[idx.to(DEV)].contiguous()
         qk, v = H * D, H * Dv
+        space = ctx.recurrent_workspace = torch.full((sum(lens) * (2 * qk + v) + 2 * (sum(lens) // 64 + 1) * qk * Dv + 4,), float("nan"), device=DEV)
         if op == "gla":
             y = k.gla_recurrent(x, (0, qk, 2 * qk, 2 * qk + v, 2 * qk + 2 * v), a2, bias, norm, H, D, Dv, 8.0, D ** -0.5, 1e-5, ctx,
                                 LayerCache(state=state.view(-1, H, D, Dv)))
@@ -43,17 +46,26 @@ def run(op, k, rows, H, D, Dv, lengths, portion):
             rkvg = torch.stack([x[:, i * qk:(i + 1) * qk] for i in range(4)]).contiguous()
             y = k.bonus_recurrence(rkvg, x[:, -32:].contiguous(), a2, bias - 2.0, bias, per_head, H, D, 1e-5, ctx, state)
         out[idx] = y.float().cpu()
+        assert ctx.recurrent_workspace is space
+        was_cut |= not space[sum(lens) * ((2 if op in ("hgrn", "ssd") else 1) * qk + v) + (-sum(lens) * qk) % 4:].isnan().all()
         for s, n in zip(who, lens):
             at[s] += n
-    return out, state
+    return out, state, was_cut
+
+
+def projected(g, n, H, D, Dv):
+    """Rows wide enough for every mixer's columns, a multiple of eight."""
+    width = 2 * H * D + 2 * H * Dv + 2 * D + H + 32
+    return lowered(rnd(g, n, width + -width % 8), torch.bfloat16, DEV)[0]
 
 
 # the shortest prompt that is cut and ones just beside it, remainders of a segment from one token on, one token beside
-# them; states of more than 128 rows; value widths the cut does not take; enough heads for the long segments
+# them; states of more than 128 rows; enough heads for the long segments; sequences enough for the sparse places of
+# segments; value widths that the cut does not take
 @pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
 @pytest.mark.parametrize("H,D,Dv,lengths", [
-    (2, 128, 128, [300, 1, 129, 64, 127]), (3, 40, 20, [128, 257]), (1, 200, 100, [191, 130]), (2, 64, 30, [200, 3]),
-    (80, 16, 16, [1300, 128, 2, 385])])
+    (2, 128, 128, [300, 1, 129, 64, 127]), (3, 40, 24, [128, 257]), (1, 200, 104, [191, 130]), (2, 64, 30, [200, 3]),
+    (80, 16, 16, [1300, 128, 2, 385]), (2, 64, 64, [200, 1, 1, 1, 1, 1, 1, 1, 65])])
 def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, lengths):
     """States are sums in float whose order differs by a product of decays taken first (relative 2^-23 a token); outputs
     are rounded to bfloat16 once, so they are equal or neighbours (2^-7 relative)."""
@@ -63,9 +75,10 @@ def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, len
         Dv = D
     k = HipKernels()
     g = torch.Generator().manual_seed(H * D)
-    rows, _ = lowered(rnd(g, sum(lengths), 2 * H * D + 2 * H * Dv + 2 * D + H + 32), torch.bfloat16, DEV)
-    whole, state = run(op, k, rows, H, D, Dv, lengths, 10 ** 6)
-    cut, want = run(op, k, rows, H, D, Dv, lengths, 100)
+    rows = projected(g, sum(lengths), H, D, Dv)
+    whole, state, was_cut = run(op, k, rows, H, D, Dv, lengths, 10 ** 6)
+    cut, want, portions_were_cut = run(op, k, rows, H, D, Dv, lengths, 100)
+    assert was_cut == (Dv % 4 == 0) and not portions_were_cut
     assert float((state - want).abs().max()) <= 2e-5 * float(want.abs().max())
     assert bool(((whole - cut).abs() <= 2.0 ** -7 * cut.abs() + 1e-3 * float(cut.std())).all()), float((whole - cut).abs().max())
     assert float(state[len(lengths):].abs().max()) == 0.0        # nobody else's slot was touched
@@ -85,9 +98,31 @@ def test_steps_of_one_token_are_the_portion_walked_along(op, H, D, Dv):
     k = HipKernels()
     g = torch.Generator().manual_seed(H * D)
     lengths = [9, 1, 6]
-    rows, _ = lowered(rnd(g, sum(lengths), 2 * H * D + 2 * H * Dv + 2 * D + H + 32 + (-(2 * H * D + 2 * H * Dv + 2 * D + H)) % 8),
-                      torch.bfloat16, DEV)
-    one, state = run(op, k, rows, H, D, Dv, lengths, 1)
-    whole, want = run(op, k, rows, H, D, Dv, lengths, 10 ** 6)
+    rows = projected(g, sum(lengths), H, D, Dv)
+    one, state, _ = run(op, k, rows, H, D, Dv, lengths, 1)
+    whole, want, _ = run(op, k, rows, H, D, Dv, lengths, 10 ** 6)
     assert float((state - want).abs().max()) <= 2e-6 * float(want.abs().max())
     assert bool(((one - whole).abs() <= 2.0 ** -7 * whole.abs() + 1e-3 * float(whole.std())).all()), float((one - whole).abs().max())
+
+
+@pytest.mark.parametrize("dtype,lengths,H,D,Dv", [
+    ("float32", [1000], 24, 128, 128), ("bfloat16", [1] * 200, 24, 128, 128), ("bfloat16", [300] * 40, 24, 128, 128),
+    ("bfloat16", [1000], 4, 264, 64), ("bfloat16", [1000], 4, 64, 30), ("bfloat16", [100, 100], 4, 64, 64),
+    ("bfloat16", [2 ** 20], 1, 8, 512), ("bfloat16", [2048], 24, 128, 128), ("bfloat16", [16384], 24, 128, 128),
+    ("bfloat16", [449] + [1] * 63, 24, 128, 128)])
+def test_a_step_that_is_not_cut_asks_for_no_room_for_segments(dtype, lengths, H, D, Dv):
+    """The workspace is the decays and the raw outputs alone where the step is not cut: float32, one token a sequence,
+    enough sequences to fill the chip, states and widths the walk does not take, portions, more segments than a grid has
+    places; and a state a segment (of 64 tokens, or 128 in a long step), with no more than one further a sequence or a
+    segment, where it is."""
+    from simple_inference_amd.kernels import HipKernels, _DT
+
+    core = HipKernels().core
+    n, kind, cut = sum(lengths), _DT[getattr(torch, dtype)], lengths in ([2048], [16384], [449] + [1] * 63)
+    facts = (n, len(lengths), max(lengths), H, D)
+    segment = 128 if n * H * 2 // 128 >= 768 else 64
+    room = (-(-n // segment) + min(len(lengths) - 1, -(-n // segment))) * H * D * Dv if cut else 0
+    assert core.sia_gla_workspace(*facts, Dv, kind) == n * H * (D + Dv) + room
+    assert core.sia_hgrn2_workspace(*facts, Dv, kind) == core.sia_ssd_workspace(*facts, Dv, kind) == n * H * (2 * D + Dv) + room
+    if D == Dv:
+        assert core.sia_bonus_recurrence_workspace(*facts, kind) == n * H * D + room
