@@ -818,15 +818,24 @@ static bool gla_slices(int n_seqs, int max_q_len, int n_heads) {
     return max_q_len > 1;
 }
 
-// The shortest segment that a prompt is cut into, and the shortest prompt that is cut (a cut costs three small kernels,
-// some 12 us; a token of the walk 0.36).
+// The shortest segment that a prompt is cut into, and the shortest run of tokens that the walk with four columns a lane
+// group is taken for.
 #define SEG_MIN 64
-#define SEG_MIN_PROMPT 128
+#define WALK_MIN_RUN 128
 
 static long long segment_places(int n_tokens, int n_seqs, Segments cut) {
     if (cut.len == 0) return 0;
     const long long multiples = (n_tokens - 1) / cut.len + 1;
     return cut.by_sequence ? multiples + n_seqs - 1 : 2 * multiples;
+}
+
+// Whether runs that are not cut are walked with four columns a lane group (a longer chain a token, but LDS serves twice
+// the columns) or two: where the workgroups are many, and where two would not fit into LDS.  Four against two, us:
+//   24 heads of 128 x 128, 128 tokens:  one run 83 against 62, 4 runs 96 against 88, 8 runs 118 against 133; one run beside 63
+//   single tokens 268 against 405;   24 of 64 x 64, 16 runs 82 against 80, one beside 63 104 against 120;   80 of 64 x 128, 4
+//   runs 120 against 135;   16 of 256 x 256, one run of 128 133 against 205 by the kernel that takes every size.
+static bool four_columns(int n_seqs, int n_heads, int D, int Dv) {
+    return D > 128 || (long long)n_seqs * n_heads * ((Dv + 63) / 64) * D >= 256 * 128;
 }
 
 // How a step is cut, from its sizes alone, so that whoever makes the workspace and whoever launches agree.
@@ -835,13 +844,20 @@ static long long segment_places(int n_tokens, int n_seqs, Segments cut) {
 // over the longest run, times heads and slices.)  2,048 tokens of 24 heads of 128: one walk of 96 workgroups 740 us; 16
 // segments 177 with two columns a lane group, 121 with four (LDS serves twice the columns, 140 registers), and 53 for
 // the decays' products, the states and the outputs behind it (100 MB of states and outputs).
+// A cut costs three kernels and the more traffic the more heads and rows; a run saves its chain: `shortest` follows where
+// both are even, in tokens of the longest run (measured with one run, 4, 8 and 16):  24 heads of 128 x 128 at 190, 210, -, -;  4 of them at
+// 172, 175, 192, 200;  24 of 64 x 64 at 165, 180, 200, 300;  8 of 128 x 64 at 172, 185, 190, 210;  32 of 16 x 64 at 148, 160,
+// 150, -.  States of more than 128 rows (no walk with two columns):  16 of 256 x 256 one run of 128 122 us against 133, 4
+// runs of 128 152 against 148 and of 256 257 against 257, 8 runs of 192 323 against 261;  4 of 256 x 128 are cut from 128 on with up to 16.
 static Segments segments_of(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv, int dtype) {
     const Segments none{0, false};
     const int slices = (Dv + 63) / 64;
-    if (dtype != SIA_BF16 || max_q_len < SEG_MIN_PROMPT || D % 8 || D > 256 || Dv % 4 || n_seqs > 65535 ||
+    if (dtype != SIA_BF16 || max_q_len < WALK_MIN_RUN || D % 8 || D > 256 || Dv % 4 || n_seqs > 65535 ||
         (long long)n_heads * slices > 65535)
         return none;
-    if ((long long)(n_tokens / max_q_len) * n_heads * slices >= 768) return none;
+    const long long busy = (long long)(n_tokens / max_q_len) * n_heads * slices;
+    const int shortest = D <= 128 ? 136 + 5 * D / 16 + (int)(busy / 4) : (long long)n_seqs * n_heads * slices * D <= 256 * 128 ? 128 : 512;
+    if (busy >= 768 || max_q_len < shortest) return none;
     const int len = (long long)n_tokens * n_heads * slices / (2 * SEG_MIN) >= 768 ? 2 * SEG_MIN : SEG_MIN;
     if ((long long)slices * ((max_q_len + len - 1) / len) > 65535) return none;      // a grid's third number
     const Segments by_sequence{len, true}, apart{len, false};
@@ -938,9 +954,11 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
     // the walk with requests a block ahead, where its pieces are aligned and fit its registers.  (Its workgroups take
     // as many columns as their threads hold whatever the step: the waves of a workgroup share the staged tokens, and
     // what bounds the walk is a wave's own chain of tokens, not the number of workgroups.)
-    const bool long_runs = max_q_len >= SEG_MIN_PROMPT && Dv % 4 == 0 && n_seqs <= 65535 && n_heads * ((Dv + 63) / 64) <= 65535 &&
+    const bool long_runs = max_q_len >= WALK_MIN_RUN && Dv % 4 == 0 && n_seqs <= 65535 && n_heads * ((Dv + 63) / 64) <= 65535 &&
                            ((uintptr_t)raw_space % 16) == 0 && ((uintptr_t)state % 16) == 0 && state_stride % 4 == 0;
-    const int w_cols = long_runs ? 4 : 2;
+    Segments cut{0, false};
+    if (long_runs) cut = segments_of(n_tokens, n_seqs, max_q_len, n_heads, D, Dv, dtype);
+    const int w_cols = long_runs && (cut.len || four_columns(n_seqs, n_heads, D, Dv)) ? 4 : 2;
     const int w_slice = GLA_WALK_THREADS / 16 * w_cols;
     const int w_rows = (D + 15) / 16;
     const int w_rows_t = w_rows <= 4 ? 4 : w_rows <= 8 ? 8 : w_rows <= 16 ? 16 : 32;
@@ -953,8 +971,6 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
     if (raw_used) *raw_used = raw != nullptr;
     if (ahead) {
         const int w_slices = (Dv + w_slice - 1) / w_slice;
-        Segments cut{0, false};
-        if (long_runs) cut = segments_of(n_tokens, n_seqs, max_q_len, n_heads, D, Dv, dtype);
         const int seg_len = cut.len, n_segs = seg_len ? (max_q_len + seg_len - 1) / seg_len : 1;
         float* seg_state = raw_space + (size_t)n_tokens * n_heads * Dv;
         dim3 wgrid(n_seqs, n_heads, w_slices * n_segs), wblock(GLA_WALK_THREADS);
