@@ -1119,7 +1119,12 @@ SIA_EXPORT int sia_gla_recurrent(const void* proj, int row_stride, int q_col, in
         const int channels = n_heads * D;
         dim3 dgrid((n_tokens + GLA_DECAY_TOKENS - 1) / GLA_DECAY_TOKENS, (channels + 255) / 256), dblock(256);
         const size_t lds = (size_t)GLA_DECAY_TOKENS * rank * sizeof(float);
-        if (dtype == SIA_BF16 && rank % 32 == 0 && channels % 4 == 0 && row_stride % 8 == 0 && a_col % 8 == 0 &&
+        // The matrix cores where there is work for them: a wave has 64 channels of 32 tokens to itself, and few waves take
+        // longer than a thread a channel does.  A layer's whole recurrence, us, without and with:  rank 64, 3,072 channels, 32
+        // tokens 31 / 37, 128: 63 / 67, 256: 89 / 91, 384: 102 / 98, 2,048: 232 / 202;  512 channels, 512: 80 / 85, 2,048: 106 / 105;
+        // rank 32, 3,072 channels, 512: 98 / 101, 1,024: 128 / 129;  rank 128, 128: 66 / 69, 256: 95 / 92.
+        const bool many = (long long)n_tokens * channels * rank >= 1LL << 26;
+        if (many && dtype == SIA_BF16 && rank % 32 == 0 && channels % 4 == 0 && row_stride % 8 == 0 && a_col % 8 == 0 &&
             ((uintptr_t)proj | (uintptr_t)a2 | (uintptr_t)a2_bias | (uintptr_t)alpha) % 16 == 0)
             hipLaunchKernelGGL(gla_decay_mfma_kernel, dim3((n_tokens + 31) / 32, (channels + 255) / 256), dblock, 0, stream,
                                (const bf16_t*)proj, row_stride, a_col, (const bf16_t*)a2, a2_bias, alpha, n_tokens, channels,

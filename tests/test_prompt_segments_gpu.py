@@ -61,13 +61,14 @@ def projected(g, n, H, D, Dv):
 
 # the shortest prompt that is cut and the one just beside it, remainders of a segment from one token on, one token beside
 # them; states of more than 128 rows; enough heads for the long segments; sequences enough for the sparse places of
-# segments; runs that are walked whole with four columns a lane group; value widths that the cut does not take
+# segments; runs that are walked whole with four columns a lane group; tokens enough for decays on the matrix cores (its
+# portions are below that); value widths that the cut does not take
 @pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
 @pytest.mark.parametrize("H,D,Dv,lengths,cut", [
     (2, 128, 128, [300, 1, 129, 64, 127], True), (2, 128, 128, [177], True), (2, 128, 128, [176], False),
     (3, 40, 24, [128, 257], True), (1, 200, 104, [191, 130], True), (1, 200, 104, [128], True), (2, 64, 30, [300, 3], False),
     (80, 16, 16, [1300, 128, 2, 385], True), (2, 64, 64, [200, 1, 1, 1, 1, 1, 1, 1, 65], True),
-    (8, 128, 128, [130] * 15 + [140], False), (12, 256, 256, [130] * 3, False)])
+    (8, 128, 128, [130] * 15 + [140], False), (12, 256, 256, [130] * 3, False), (24, 128, 128, [1100], True)])
 def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, lengths, cut):
     """States are sums in float whose order differs by a product of decays taken first (relative 2^-23 a token); outputs
     are rounded to bfloat16 once, so they are equal or neighbours (2^-7 relative)."""
