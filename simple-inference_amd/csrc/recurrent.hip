@@ -737,25 +737,24 @@ __global__ __launch_bounds__(256) void gla_decay_mfma_kernel(const bf16_t* __res
     }
 }
 
-// y = o * rsqrt(mean(o^2) + eps) * w * silu(g) for outputs left in a float workspace: a wave four (token, head) pairs, whose
-// loads are under way together (a workgroup of one wave a pair was bound by the dispatch of workgroups: 2,048 tokens of
+// y = o * rsqrt(mean(o^2) + eps) * w * silu(g) for outputs left in a float workspace: a wave one (token, head) pair or four,
+// whose loads are under way together (a workgroup of one wave a pair was bound by the dispatch of workgroups: 2,048 tokens of
 // 24 heads of 128 25 -> 20 us).
 #define GLA_FINISH_WAVES 4
-#define GLA_FINISH_PAIRS 4
-template <typename T>
+template <typename T, int PAIRS>
 __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_kernel(
     const float* __restrict__ raw, const T* __restrict__ proj, int row_stride, int g_col, const float* __restrict__ norm_w,
     T* __restrict__ out, int n_pairs, int n_heads, int Dv, float eps) {
     const int lane = threadIdx.x % SIA_WAVE;
-    const int first = ((int)blockIdx.x * GLA_FINISH_WAVES + (int)threadIdx.x / SIA_WAVE) * GLA_FINISH_PAIRS;
+    const int first = ((int)blockIdx.x * GLA_FINISH_WAVES + (int)threadIdx.x / SIA_WAVE) * PAIRS;
     if (first >= n_pairs) return;      // a wave leaves as a whole
     // a lane has every 64th pair of neighbouring elements (the last one alone where Dv is odd); Dv is at most 512
     constexpr int TURNS = 4;
-    float2 o[TURNS][GLA_FINISH_PAIRS];
-    float ss[GLA_FINISH_PAIRS] = {};
-    int at[GLA_FINISH_PAIRS], g_at[GLA_FINISH_PAIRS];
+    float2 o[TURNS][PAIRS];
+    float ss[PAIRS] = {};
+    int at[PAIRS], g_at[PAIRS];
 #pragma unroll
-    for (int i = 0; i < GLA_FINISH_PAIRS; ++i) {
+    for (int i = 0; i < PAIRS; ++i) {
         const int pair = min(first + i, n_pairs - 1), n = pair / n_heads;
         at[i] = pair;
         g_at[i] = n;
@@ -764,7 +763,7 @@ __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_kernel
     for (int k = 0; k < TURNS; ++k) {
         const int c = 2 * (lane + k * SIA_WAVE);
 #pragma unroll
-        for (int i = 0; i < GLA_FINISH_PAIRS; ++i) {
+        for (int i = 0; i < PAIRS; ++i) {
             const float* p = raw + (size_t)at[i] * Dv + c;
             o[k][i] = make_float2(0.f, 0.f);
             if (c + 1 < Dv) o[k][i] = make_float2(p[0], p[1]);
@@ -774,10 +773,10 @@ __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_kernel
 #pragma unroll
     for (int k = 0; k < TURNS; ++k)
 #pragma unroll
-        for (int i = 0; i < GLA_FINISH_PAIRS; ++i) ss[i] += o[k][i].x * o[k][i].x + o[k][i].y * o[k][i].y;
-    float inv[GLA_FINISH_PAIRS];
+        for (int i = 0; i < PAIRS; ++i) ss[i] += o[k][i].x * o[k][i].x + o[k][i].y * o[k][i].y;
+    float inv[PAIRS];
 #pragma unroll
-    for (int i = 0; i < GLA_FINISH_PAIRS; ++i) inv[i] = rsqrtf(wave_sum(ss[i]) / (float)Dv + eps);
+    for (int i = 0; i < PAIRS; ++i) inv[i] = rsqrtf(wave_sum(ss[i]) / (float)Dv + eps);
 #pragma unroll
     for (int k = 0; k < TURNS; ++k) {
         const int c = 2 * (lane + k * SIA_WAVE);
@@ -785,7 +784,7 @@ __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_kernel
         const bool two = c + 1 < Dv;
         const float w0 = norm_w[c], w1 = two ? norm_w[c + 1] : 0.f;
 #pragma unroll
-        for (int i = 0; i < GLA_FINISH_PAIRS; ++i) {
+        for (int i = 0; i < PAIRS; ++i) {
             float f0 = 1.f, f1 = 1.f;
             if (g_col >= 0) {
                 const T* g_row = proj + (size_t)g_at[i] * row_stride + g_col + (at[i] - g_at[i] * n_heads) * Dv + c;
@@ -801,13 +800,19 @@ __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_kernel
     }
 }
 
+// Four pairs a wave where there are many narrow ones; a layer's recurrence, one and four, us:  24 heads of 128, 32 tokens 23.7 and
+// 25.8, 512: 75.1 and 75.9, 1,024: 91.5 and 91.2, 2,048: 138.9 and 137.7;  16 of 256, 32 tokens 24.9 and 27.7, 2,048: 149.0 and 151.6.
 template <typename T>
 static void launch_finish(const float* raw, const void* proj, int row_stride, int g_col, const float* norm_w, void* out, int n_tokens,
                           int n_heads, int Dv, float eps, hipStream_t stream) {
-    constexpr int pairs = GLA_FINISH_WAVES * GLA_FINISH_PAIRS;
     const int n_pairs = n_tokens * n_heads;
-    hipLaunchKernelGGL(gla_finish_kernel<T>, dim3((n_pairs + pairs - 1) / pairs), dim3(GLA_FINISH_WAVES * SIA_WAVE), 0, stream,
-                       raw, (const T*)proj, row_stride, g_col, norm_w, (T*)out, n_pairs, n_heads, Dv, eps);
+    auto launch = [&](auto kernel, int pairs) {
+        const int each = GLA_FINISH_WAVES * pairs;
+        hipLaunchKernelGGL(kernel, dim3((n_pairs + each - 1) / each), dim3(GLA_FINISH_WAVES * SIA_WAVE), 0, stream, raw, (const T*)proj,
+                           row_stride, g_col, norm_w, (T*)out, n_pairs, n_heads, Dv, eps);
+    };
+    if (n_pairs >= 20000 && Dv <= 128) launch(gla_finish_kernel<T, 4>, 4);
+    else launch(gla_finish_kernel<T, 1>, 1);
 }
 
 SIA_EXPORT int sia_gla_max_dims() { return 512; }

@@ -61,8 +61,8 @@ def projected(g, n, H, D, Dv):
 
 # the shortest prompt that is cut and the one just beside it, remainders of a segment from one token on, one token beside
 # them; states of more than 128 rows; enough heads for the long segments; sequences enough for the sparse places of
-# segments; runs that are walked whole with four columns a lane group; tokens enough for decays on the matrix cores (its
-# portions are below that); value widths that the cut does not take
+# segments; runs that are walked whole with four columns a lane group; tokens enough for decays on the matrix cores and for
+# the finishing kernel's four pairs a wave (its portions are below both); value widths that the cut does not take
 @pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
 @pytest.mark.parametrize("H,D,Dv,lengths,cut", [
     (2, 128, 128, [300, 1, 129, 64, 127], True), (2, 128, 128, [177], True), (2, 128, 128, [176], False),
