@@ -438,12 +438,15 @@ def test_norm_shared_out_between_the_products_around_it(hip, shape):
     (10, 2, 16, 16, 64, 70, 0, False, 5.0, 3), (6, 2, 100, 128, 128, 0, 96, True, 0.0, 0), (4, 2, 64, 65, 8, 1, 0, False, 0.0, 130),
     (8, 1, 4, 1, 32, 200, 0, True, 2.0, 65),
 ])
-def test_float32_attention_is_the_plain_kernels(hip, geom):
+@pytest.mark.parametrize("more", [0, 700, 1500])
+def test_float32_attention_is_the_plain_kernels(hip, geom, more):
     """The kernel whose workgroups share keys and values computes what the plain kernel does, with its order of sums:
-    the same bits, in every form, for runs that cross the eights of tokens and the chunks of keys.  Values that a row
-    does not see do not reach it, whatever they are."""
+    the same bits, in every form, for runs that cross the eights of tokens and the chunks of keys, in steps of few tokens
+    (a workgroup each) and of many.  Values that a row does not see do not reach it, whatever they are."""
     n_heads, n_kv, D, Dv, ps, window, block, with_sinks, cap, keep = geom
     q_lens, kv_lens = [1, 1, 1, 13, 2, 150, 9], [1, 64, 500, 13, 129, 150, 300]
+    if more:
+        q_lens, kv_lens = q_lens + [more], kv_lens + [more]
     ctx = Ctx(q_lens, kv_lens)
     pages = sum(-(-kv // ps) for kv in kv_lens) + 2
     cache = Cache(pages, n_kv, ps, D, torch.float32, kv_lens, seed=3)
@@ -469,6 +472,26 @@ def test_float32_attention_is_the_plain_kernels(hip, geom):
         assert rc == 0 and torch.equal(got.isnan(), plain.isnan()) and torch.equal(got.nan_to_num(7.0), plain.nan_to_num(7.0)), v
         if v:
             assert torch.equal(got[:at], whole[:at]) and torch.equal(got[at + 1:], whole[at + 1:])
+
+
+@pytest.mark.parametrize("n_heads,n_kv,D", [(32, 8, 64), (24, 8, 128), (6, 6, 32)])
+@pytest.mark.parametrize("q_lens,kv_lens", [([16], [16]), ([17], [17]), ([1, 1, 3], [16, 2, 16]), ([3] * 16, [300] * 16), ([2] * 70, [40] * 70),
+                                            ([1, 40], [70, 40]), ([64], [264]), ([65], [265])])
+def test_float32_attention_has_the_same_bits_whichever_way_it_goes(hip, n_heads, n_kv, D, q_lens, kv_lens):
+    """Few keys (the plain kernel), few tokens or short runs (a workgroup a token), more (eight tokens a workgroup): each
+    sequence's rows are those that it has alone."""
+    ctx, ps = Ctx(q_lens, kv_lens), 16
+    cache = Cache(sum(-(-kv // ps) for kv in kv_lens), n_kv, ps, D, torch.float32, kv_lens, seed=3)
+    cache.k_pages.copy_(rnd(*cache.k_pages.shape, seed=4))
+    cache.v_pages.copy_(rnd(*cache.v_pages.shape, seed=5))
+    qkv = rnd(ctx.n_tokens, (n_heads + n_kv) * D, seed=6)
+    out = hip.paged_attention(qkv, n_heads, n_kv, D, 0.3, None, ctx, cache)
+    plain = torch.empty_like(out)
+    rc = hip.core.sia_attention_generic(
+        qkv.data_ptr(), qkv.shape[1], cache.k_pages.data_ptr(), cache.v_pages.data_ptr(), cache.block_table.data_ptr(),
+        cache.block_table.shape[1], ctx.seq_of_token.data_ptr(), ctx.positions.data_ptr(), plain.data_ptr(), ctx.n_tokens, n_heads,
+        n_kv, D, D, ps, 0.3, 0, 0, None, 0.0, 0, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(out, plain)
 
 
 # kept positions that end inside a four, at its end, and in the second and third chunk of keys
