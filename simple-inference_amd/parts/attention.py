@@ -259,8 +259,8 @@ class Attention:
 
     def plain_form(self):
         """What this mixer is, as plain data, for kernels that can run a whole block in one call; None for the forms
-        that only ``forward`` covers (reading another layer's keys and values)."""
-        if not self.writes_kv or type(self).forward is not Attention.forward or self._options():
+        that only ``forward`` covers (reading another layer's keys and values, a bias behind the output projection)."""
+        if not self.writes_kv or type(self).forward is not Attention.forward or self._options() or self.o_bias:
             return None     # a subclass with a forward of its own is no longer what this form describes
         cos, sin = self.position.tables()
         return {"kind": "paged_attention", "w_qkv": self.w_qkv, "w_o": self.w_o, "hidden": self.hidden,

@@ -228,3 +228,5 @@ def test_a_part_with_a_forward_of_its_own_no_longer_says_it_is_the_plain_one():
     assert built(Attention, OtherNorm, SwiGLU, PreNormBlock).plain_form()["mixer_norm"] is None
     assert built(Attention, RMSNorm, OtherFeedForward, PreNormBlock).plain_form()["feed_forward"] is None
     assert built(Attention, RMSNorm, SwiGLU, OtherBlock).plain_form() is None
+    attn_params["o_bias"] = True      # the one call adds no bias behind the output projection
+    assert built(Attention, RMSNorm, SwiGLU, PreNormBlock).plain_form()["mixer"] is None
