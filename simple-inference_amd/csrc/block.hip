@@ -69,12 +69,14 @@ struct SiaBlockStep {
         if (rc_ != 0) return rc_;  \
     } while (0)
 
-// residual += delta (where there is one); then the block.  Leaves the block's last product in S->fed, not yet added.
+// residual += delta (where there is one); then the block up to its attention, whose results are left in S->attended, or
+// without ``attend`` up to its projected rows, which are left in S->qkv with keys and values in the pages: what a caller that
+// goes on with some rows alone needs of all of them.
 // block_table [n_seqs, table_width], k_pages, v_pages: the block's cache in this step.  0, or the first launch's error.
-SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, const int* block_table,
-                                 int table_width, void* k_pages, void* v_pages, int page_size, hipStream_t stream) {
+SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, const int* block_table,
+                                 int table_width, void* k_pages, void* v_pages, int page_size, int attend, hipStream_t stream) {
     if (!B || !S || !S->product || !S->attend_runs || S->n_tokens <= 0 || S->n_tokens > 65535) return SIA_BAD_ARGUMENT;
-    const int M = S->n_tokens, H = B->hidden, Q = B->n_heads * B->head_dim;
+    const int M = S->n_tokens, H = B->hidden;
     const int qkv_width = (B->n_heads + 2 * B->n_kv) * B->head_dim;
     SIA_STEP(sia_add_rmsnorm(S->residual, delta, B->mixer_norm_gain, S->normed, nullptr, M, H, B->mixer_norm_eps,
                              SIA_BF16, stream));
@@ -82,6 +84,7 @@ SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, co
     SIA_STEP(sia_rope_kv_write(S->qkv, qkv_width, B->cos_table, B->sin_table, S->positions, S->seq_of_token,
                                block_table, table_width, k_pages, v_pages, M, B->n_heads, B->n_kv, B->head_dim,
                                B->rotary_dim, page_size, SIA_BF16, stream));
+    if (!attend) return 0;
     if (S->n_single > 0) {
         if (!S->attend_single) return SIA_BAD_ARGUMENT;
         SIA_STEP(S->attend_single(S->qkv, qkv_width, k_pages, v_pages, block_table, table_width, S->cu_q, S->kv_len,
@@ -92,6 +95,14 @@ SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, co
         SIA_STEP(S->attend_runs(S->qkv, qkv_width, k_pages, v_pages, block_table, table_width, S->cu_q, S->kv_len,
                                 S->attended, S->n_single, S->n_seqs, S->n_tiles, S->n_tiles_split, S->n_tiles_long,
                                 S->q_bound, S->kv_bound, B->n_heads, B->n_kv, page_size, B->scale, B->window, stream));
+    return 0;
+}
+
+// The whole block.  Leaves its last product in S->fed, not yet added.
+SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, const int* block_table,
+                                 int table_width, void* k_pages, void* v_pages, int page_size, hipStream_t stream) {
+    SIA_STEP(sia_prenorm_mixer(B, S, delta, block_table, table_width, k_pages, v_pages, page_size, 1, stream));
+    const int M = S->n_tokens, H = B->hidden, Q = B->n_heads * B->head_dim;
     SIA_STEP(S->product(S->attended, B->w_o, S->mixed, M, H, Q, 0, stream));
     SIA_STEP(sia_add_rmsnorm(S->residual, S->mixed, B->feed_forward_norm_gain, S->normed, nullptr, M, H,
                              B->feed_forward_norm_eps, SIA_BF16, stream));

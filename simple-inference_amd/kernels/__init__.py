@@ -111,6 +111,7 @@ _SIGNATURES = {
     "sia_attention_generic_max_head_dim": [],
     "sia_gemm_generic": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "sia_prenorm_block": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
+    "sia_prenorm_mixer": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
     "sia_sample": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_sample_workspace_bytes": [_c_int],
     "sia_sample_few_max_k": [],
@@ -2046,41 +2047,58 @@ class HipKernels:
         steps[key] = (step, buffers)
         return steps[key]
 
-    def prenorm_block(self, block, stream, ctx, cache) -> bool:
-        """Runs a pre-norm block of RMS norms, paged attention and SwiGLU on a step of many rows with one call into
-        the library (the same launches, in the same order, as the parts' own calls make); False, with nothing done,
-        where that form does not apply: the caller then goes part by part."""
+    def _block_call(self, block, stream, ctx, cache):
+        """The first arguments of the one-call forms of a block in this step, and the step's buffers; None where they do not
+        apply."""
         if not self.whole_blocks or self.blas is None or not self.use_mfma_attention:
-            return False
+            return None
         residual = stream.residual
         M = ctx.n_tokens
         if (M <= self._skinny_rows or M > 65535 or getattr(ctx, "extra", None)
                 or residual.dtype != torch.float32 or cache.k_pages is None or cache.page_size < 8):
-            return False
+            return None
         made = self._block_own(block)
         if not made:
-            return False
+            return None
         own, _, positions_covered = made
         if (tuple(residual.shape) != (M, own.hidden) or not residual.is_contiguous() or cache.k_pages.dtype != torch.bfloat16
                 or (positions_covered is not None and positions_covered <= ctx.max_kv_len - 1)):
-            return False
+            return None
         step = self._block_step(own, ctx, residual.device)
         if step is None:
-            return False
+            return None
         delta = stream.delta    # computes it if it is a product not yet computed
         if delta is not None and (delta.dtype != torch.bfloat16 or tuple(delta.shape) != (M, own.hidden)
                                   or not delta.is_contiguous()):
-            return False
+            return None
         self._check_pages(cache.k_pages, cache.v_pages, cache.block_table, cache.page_size, own.n_kv, own.head_dim,
                           torch.bfloat16, ctx)
         step_struct, buffers = step
         step_struct.residual = _ptr(residual)
-        self._check(self.core.sia_prenorm_block(
-            ctypes.addressof(own), ctypes.addressof(step_struct), _ptr(delta), _ptr(cache.block_table),
-            cache.block_table.shape[1], _ptr(cache.k_pages), _ptr(cache.v_pages), cache.page_size, self._stream()),
-            "prenorm_block")
-        stream.delta = buffers[-1]
+        return (ctypes.addressof(own), ctypes.addressof(step_struct), _ptr(delta), _ptr(cache.block_table),
+                cache.block_table.shape[1], _ptr(cache.k_pages), _ptr(cache.v_pages), cache.page_size), buffers
+
+    def prenorm_block(self, block, stream, ctx, cache) -> bool:
+        """Runs a pre-norm block of RMS norms, paged attention and SwiGLU on a step of many rows with one call into
+        the library (the same launches, in the same order, as the parts' own calls make); False, with nothing done,
+        where that form does not apply: the caller then goes part by part."""
+        call = self._block_call(block, stream, ctx, cache)
+        if call is None:
+            return False
+        self._check(self.core.sia_prenorm_block(*call[0], self._stream()), "prenorm_block")
+        stream.delta = call[1][-1]
         return True
+
+    def prenorm_mixer(self, block, stream, ctx, cache, attend):
+        """Such a block up to its attention with one call: what is pending is added into the residual, keys and values are
+        written, and the attention's rows are returned, or without ``attend`` the projected ones.  None, with nothing done,
+        where that form does not apply.  (The rows are the step's: the next block of the step writes over them.)"""
+        call = self._block_call(block, stream, ctx, cache)
+        if call is None:
+            return None
+        self._check(self.core.sia_prenorm_mixer(*call[0], int(attend), self._stream()), "prenorm_mixer")
+        stream.delta = None
+        return call[1][2 if attend else 1]
 
     # -- sampling ------------------------------------------------------------------
     def few_max_k(self) -> int:

@@ -272,6 +272,28 @@ class Attention:
         """Whether ``forward`` gives the rows ``ctx.only_rows`` alone where it is set."""
         return type(self).forward is Attention.forward and not self.row_form
 
+    def rows_alone(self, rows, ctx) -> bool:
+        """Whether attention of the rows that are read is taken as that of decoded tokens, not with the whole step's: about
+        a token a sequence, of a step with enough others."""
+        return rows.numel() <= ctx.n_seqs and ctx.n_tokens >= ctx.n_decode_seqs + 128
+
+    def forward_rows(self, prepare, ctx, cache, rows):
+        """The rows ``rows`` of the mixer's result (None if there are none) from what ``prepare(attend)`` gives: all rows of
+        the attention, or without ``attend`` the projected ones, with keys and values in the pages; None, with nothing done,
+        for "not in this way", and then this is False."""
+        alone = rows.numel() == 0 or self.rows_alone(rows, ctx)
+        y = prepare(not alone)
+        if y is None:
+            return False
+        if rows.numel() == 0:
+            return None
+        k = self.env.kernels
+        y = k.take_rows(y, rows)
+        if alone:
+            ctx, cache = k.rows_alone(rows, ctx, cache)
+            y = k.paged_attention(y, self.num_heads, self.num_kv_heads, self.head_dim, self.scale, self.window, ctx, cache)
+        return k.pending_linear(y, self.w_o)
+
     def _options(self) -> bool:
         """Whether any of the further forms is switched on (the kernels then get them as keyword arguments)."""
         return (self.bias or self.qk_norm_eps is not None or self.sink or self.chunk is not None
@@ -360,8 +382,7 @@ class Attention:
         rows = getattr(ctx, "only_rows", None)      # keys and values are in the pages: of the rest, only these rows are read
         if rows is not None and rows.numel() == 0:
             return None
-        if rows is not None and gate_logits is None and rows.numel() <= ctx.n_seqs and ctx.n_tokens >= ctx.n_decode_seqs + 128:
-            # about a token a sequence: its attention alone is a decoded token's, not a prompt's
+        if rows is not None and gate_logits is None and self.rows_alone(rows, ctx):
             qkv = k.take_rows(qkv, rows)
             ctx, cache = k.rows_alone(rows, ctx, cache)
             rows = None

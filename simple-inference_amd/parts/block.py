@@ -78,8 +78,14 @@ class PreNormBlock:
         if (type(self).forward is not PreNormBlock.forward or self.feed_forward is None or self.token_input is not None
                 or not _by_row(self.feed_forward)):
             return False
-        h = _normed(self.mixer_norm, self.mixer, stream)
-        delta = _mixed_rows(self.mixer, h, ctx, cache, rows)
+        # Kernels that make all of a block's launches in one call make those up to the attention in one, too (and take the
+        # block or leave it by what it and its parts say they are).
+        prepare, delta = getattr(ctx.kernels, "prenorm_mixer", None), False
+        if prepare is not None and hasattr(self.mixer, "forward_rows"):
+            delta = self.mixer.forward_rows(lambda attend: prepare(self, stream, ctx, cache, attend), ctx, cache, rows)
+        if delta is False:
+            h = _normed(self.mixer_norm, self.mixer, stream)
+            delta = _mixed_rows(self.mixer, h, ctx, cache, rows)
         if delta is None:
             return True
         stream.keep_rows(rows, ctx.kernels)

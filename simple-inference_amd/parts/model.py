@@ -175,5 +175,8 @@ class DecoderModel:
         (what a layer writes for later steps, keys, values and states, it writes for all): a prompt's portion needs its
         last row, or none.  (A prompt's last layer at the 3B widths, 2,048 tokens: 0.48 -> 0.16 ms; at the 8B widths, 7,001
         tokens: 3.0 -> 0.5 ms.)  Steps of fewer rows are bound by reading the weights, and keep the one call a layer: eight
-        layers at 33 rows 918 -> 896 us (3B widths) and 731 -> 731 (1B), at 24 rows 827 -> 814 and 722 -> 727."""
+        layers at 33 rows 918 -> 896 us (3B widths) and 731 -> 731 (1B), at 24 rows 827 -> 814 and 722 -> 727.  A single pass on
+        an idle device, which the host may bound (it takes 20 to 50 us more here), whole -> rows:  1B 32 tokens 905 -> 902, 45: 919
+        -> 912, 128: 1,043 -> 1,023, 300: 1,268 -> 1,234;  3B 1,001 -> 991, 1,108 -> 1,099, 1,440 -> 1,397, 1,550 -> 1,498;  four layers at
+        the 8B widths 903 -> 886 at 32, 972 -> 951 at 64, 1,219 -> 1,145 at 128."""
         return ctx.n_tokens >= 32 and 2 * ctx.n_logit_rows <= ctx.n_tokens and hasattr(ctx.kernels, "take_rows")
