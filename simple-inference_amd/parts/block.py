@@ -75,7 +75,7 @@ class PreNormBlock:
     def forward_rows(self, stream, ctx, cache, rows):
         """``forward`` for a model's last layer, of whose results only ``rows`` are read: the mixer sees all tokens, what
         follows it those alone, and the stream is left with them.  False, with nothing done, for a block it does not fit."""
-        if (type(self).forward is not PreNormBlock.forward or self.feed_forward is None or self.token_input is not None
+        if (_has_another_forward(self, PreNormBlock) or self.feed_forward is None or self.token_input is not None
                 or not _by_row(self.feed_forward)):
             return False
         # Kernels that make all of a block's launches in one call make those up to the attention in one, too (and take the
@@ -94,6 +94,11 @@ class PreNormBlock:
         stream.delta = self.feed_forward.forward(_normed(self.feed_forward_norm, self.feed_forward, stream), ctx)
         stream.scale = self.residual_scale
         return True
+
+
+def _has_another_forward(block, kind):
+    """Whether a block's class, or somebody who wraps this one block, has a forward in place of the kind's own."""
+    return type(block).forward is not kind.forward or "forward" in vars(block)
 
 
 def _by_row(*parts):
@@ -182,7 +187,7 @@ class GatedPreNormBlock:
 
     def forward_rows(self, stream, ctx, cache, rows):
         """As ``PreNormBlock.forward_rows``."""
-        if type(self).forward is not GatedPreNormBlock.forward or self.feed_forward is None or not _by_row(
+        if _has_another_forward(self, GatedPreNormBlock) or self.feed_forward is None or not _by_row(
                 self.feed_forward, self.mixer_gate, self.feed_forward_gate):
             return False
         h = self.mixer_norm.forward(stream)

@@ -82,3 +82,20 @@ def test_what_a_mixer_leaves_to_the_residual_is_taken_there_by_rows_too(block, r
     want = last.forward(whole, rows=rows)
     assert made.forward_rows(alone, ctx, None, rows)
     assert torch.equal(last.forward(alone), want)
+
+
+@pytest.mark.parametrize("kind", [PreNormBlock, GatedPreNormBlock])
+def test_a_block_whose_forward_is_wrapped_is_run_by_it(kind):
+    """Somebody who put a forward of their own in place of a block's, by a class or on the block, sees every step."""
+    k = RowTwins()
+    env = BuildEnv(k, torch.device("cpu"), torch.bfloat16, 64)
+    parts = dict(mixer=Mixer(lambda: rnd(TOKENS, HIDDEN, seed=1)), mixer_norm=norm(env), feed_forward=Half(), feed_forward_norm=norm(env))
+    if kind is GatedPreNormBlock:
+        parts.update(mixer_gate=Gate(), feed_forward_gate=Gate())
+    rows, ctx = torch.tensor([3], dtype=torch.int32), SimpleNamespace(kernels=k)
+    by_rows = lambda block: block.forward_rows(ResidualStream(rnd(TOKENS, HIDDEN, seed=5, dtype=torch.float32)), ctx, None, rows)
+    assert by_rows(kind(**parts))
+    wrapped = kind(**parts)
+    wrapped.forward = lambda *args: kind.forward(wrapped, *args)
+    assert not by_rows(wrapped)
+    assert not by_rows(type("Other", (kind,), {"forward": lambda self, *args: kind.forward(self, *args)})(**parts))
