@@ -221,9 +221,11 @@ def test_float32_product_has_no_reduced_precision(hip):
     assert y[0, 1].item() - 8.0 == 2.0 ** -12
 
 
-# edges of the tiles (16, 32, 64, 128 columns; 16, 32, 64 rows), of a step of 64 k and of a piece of 16; the last is misaligned
+# edges of the tiles (16, 32, 64, 128 columns; 16, 32, 64 rows), of a step of 64 k and of a piece of 16; the one of 50 rows is
+# misaligned.  By the rule's rounds: 16 rows and fewer stream, 17 to 50 and (64, 63) take 32 x 16, (300, 16500) and (129, 8320)
+# 64 x 128, (303, 3070) and (64, 16383) 64 x 64, (40, 4100) 32 x 32
 @pytest.mark.parametrize("shape", [(1, 1, 1), (16, 17, 4), (17, 16, 60), (33, 33, 64), (64, 63, 68), (65, 130, 130), (40, 4100, 80),
-                                   (129, 8320, 192), (300, 16500, 76), (50, 257, 128)])
+                                   (129, 8320, 192), (300, 16500, 76), (50, 257, 128), (303, 3070, 76), (64, 16383, 66)])
 def test_float32_product(hip, shape):
     """Against float64: a result is the sum of four chains of about K / 4 float products, each rounded once or twice, so
     it errs by at most (K / 4 + 8) times 2^-24 of the sum of the products' sizes; and whichever kernel a number of
