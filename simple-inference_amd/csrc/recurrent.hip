@@ -14,8 +14,8 @@
 //
 // The decays of all tokens and channels are computed first, by a kernel of their own (they do not depend on the
 // state, and a step's tokens are thousands of independent little products), into a float workspace.
-// A workgroup owns one (sequence, head) and walks the sequence's tokens of this step in order, so a request's
-// numbers depend on its own tokens only: not on how its prompt was cut, nor on what else the step holds.
+// A workgroup owns one (sequence, head) and walks the sequence's tokens of this step in order; an entry of the state
+// is written by the request's own tokens in their order.
 // Thread (j, r) keeps rows r, r + R, r + 2R, ... of column j of S in registers (R a power of two: the lanes of a
 // column are neighbours and add their shares of o by lane exchanges).  Blocks of a few tokens are staged through
 // LDS (q, k, alpha, v, g as floats), walked, and their outputs normed and gated a token a wave.
@@ -27,8 +27,12 @@
 // A long prompt in bfloat16 is cut into segments that are walked at the same time, each from zero: what the state S
 // in front of a segment adds to its outputs is (q_t * P_t)^T S with P_t the products of the decays since the segment began,
 // and S itself follows from segment to segment by S <- diag(P_last) S + (the segment's own).  Only products of decays,
-// which lie in (0, 1), are taken ahead: nothing is divided by them.  (There the last bits of float depend on where the
-// step's portion began; the rows' products of a step of many rows do so anyway.)
+// which lie in (0, 1), are taken ahead: nothing is divided by them.
+//
+// What a request's numbers depend on beside its own tokens: the number of sequences and the longest run choose how many lanes
+// share a column, and with it the order of an output's sum over the state's rows, in float32 too (states keep their bits
+// there).  In bfloat16 the step's tokens, sequences and longest run also say whether and how prompts are cut, and with a cut the last
+// bits of float of a state depend on where its segments began.
 #include "common.h"
 
 #include <type_traits>

@@ -527,7 +527,6 @@ struct Candidates {
 };
 static_assert(sizeof(Candidates) <= SP_CLEAR_BYTES, "in the histograms' place");
 
-// 1. maximum of each chunk, and its candidates
 // How many of the workgroup's threads a wave's `mine` counts together: the waves' counts meet in one of two rows of LDS in
 // turn, so that one barrier a call is enough.
 __device__ __forceinline__ int counted_together(int mine, int (&counts)[2][SP_WAVES], int turn) {
@@ -550,6 +549,7 @@ __device__ __forceinline__ uint32_t largest_of_lanes(uint32_t key, int q) {
     return found;
 }
 
+// 1. maximum of each chunk, and its candidates
 __global__ __launch_bounds__(SP_THREADS, 8) void sample_candidates_kernel(const float* __restrict__ logits,
                                                                           const float* __restrict__ temperature,
                                                                           const int* __restrict__ top_k, int vocab,

@@ -1896,8 +1896,9 @@ class HipKernels:
             self._check(self.core.sia_attention_f32(
                 _ptr(qkv), width, _ptr(cache.k_pages), _ptr(cache.v_pages), _ptr(cache.block_table),
                 cache.block_table.shape[1], _ptr(ctx.seq_of_token), _ptr(ctx.positions), _ptr(out), n, ctx.n_decode_seqs,
-                ctx.n_seqs, int(ctx.kv_bound or ctx.max_kv_len), n_heads, n_kv_heads, head_dim, value_dim, page, float(scale), int(window or 0), int(chunk or 0), _ptr(sinks),
-                float(softcap or 0.0), int(keep_first), self._stream()), "attention_f32")
+                ctx.n_seqs, int(ctx.kv_bound or ctx.max_kv_len), n_heads, n_kv_heads, head_dim, value_dim, page, float(scale),
+                int(window or 0), int(chunk or 0), _ptr(sinks), float(softcap or 0.0), int(keep_first), self._stream()),
+                "attention_f32")
             return out
         self._check(self.core.sia_attention_generic(
             _ptr(qkv), width, _ptr(cache.k_pages), _ptr(cache.v_pages), _ptr(cache.block_table),
