@@ -76,7 +76,7 @@ class PreNormBlock:
         """``forward`` for a model's last layer, of whose results only ``rows`` are read: the mixer sees all tokens, what
         follows it those alone, and the stream is left with them.  False, with nothing done, for a block it does not fit."""
         if (_has_another_forward(self, PreNormBlock) or self.feed_forward is None or self.token_input is not None
-                or not _by_row(self.feed_forward)):
+                or _wrapped(self.feed_forward_norm) or not _by_row(self.feed_forward)):
             return False
         # Kernels that make all of a block's launches in one call make those up to the attention in one, too (and take the
         # block or leave it by what it and its parts say they are).
@@ -96,14 +96,22 @@ class PreNormBlock:
         return True
 
 
+def _wrapped(*parts):
+    """Whether somebody has put a computation of their own in place of one of these parts', on the part."""
+    return any("forward" in own or "logits" in own for own in (getattr(part, "__dict__", {}) for part in parts))
+
+
 def _has_another_forward(block, kind):
     """Whether a block's class, or somebody who wraps this one block, has a forward in place of the kind's own."""
-    return type(block).forward is not kind.forward or "forward" in vars(block)
+    return type(block).forward is not kind.forward or _wrapped(block)
 
 
 def _by_row(*parts):
     """Whether each of the parts says that a row of its result depends on that row of its input alone.  The class that
-    says so must be the one that computes it: a subclass with a computation of its own is no longer what was said."""
+    says so must be the one that computes it: a subclass with a computation of its own, or a part that somebody wraps (and
+    who is to see every token), is no longer what was said."""
+    if _wrapped(*parts):
+        return False
     for part in parts:
         owner = next((c for c in type(part).__mro__ if "forward" in c.__dict__ or "logits" in c.__dict__), object)
         if not owner.__dict__.get("by_row", False):
@@ -114,7 +122,7 @@ def _by_row(*parts):
 def _mixed_rows(mixer, h, ctx, cache, rows):
     """The mixer's result at ``rows`` alone (None if there are none): from a mixer that gives only those, or taken out of
     all of it."""
-    if not getattr(mixer, "gives_only_rows", lambda: False)():
+    if _wrapped(mixer) or not getattr(mixer, "gives_only_rows", lambda: False)():
         y = mixer.forward(h, ctx, cache)
         return _rows_of(y, rows, ctx.kernels) if rows.numel() else None
     ctx.only_rows = rows
@@ -187,8 +195,8 @@ class GatedPreNormBlock:
 
     def forward_rows(self, stream, ctx, cache, rows):
         """As ``PreNormBlock.forward_rows``."""
-        if _has_another_forward(self, GatedPreNormBlock) or self.feed_forward is None or not _by_row(
-                self.feed_forward, self.mixer_gate, self.feed_forward_gate):
+        if (_has_another_forward(self, GatedPreNormBlock) or self.feed_forward is None or _wrapped(self.feed_forward_norm)
+                or not _by_row(self.feed_forward, self.mixer_gate, self.feed_forward_gate)):
             return False
         h = self.mixer_norm.forward(stream)
         delta = _mixed_rows(self.mixer, h, ctx, cache, rows)

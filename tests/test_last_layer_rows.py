@@ -99,3 +99,32 @@ def test_a_block_whose_forward_is_wrapped_is_run_by_it(kind):
     wrapped.forward = lambda *args: kind.forward(wrapped, *args)
     assert not by_rows(wrapped)
     assert not by_rows(type("Other", (kind,), {"forward": lambda self, *args: kind.forward(self, *args)})(**parts))
+
+
+class RowsMixer(Mixer):
+    def forward(self, h, ctx, cache):
+        rows = getattr(ctx, "only_rows", None)
+        return self.result() if rows is None else ctx.kernels.take_rows(self.result(), rows)
+
+    def gives_only_rows(self):
+        return True
+
+
+@pytest.mark.parametrize("kind,name", [(PreNormBlock, n) for n in ("mixer", "feed_forward", "feed_forward_norm")]
+                         + [(GatedPreNormBlock, n) for n in ("mixer", "feed_forward", "feed_forward_norm", "mixer_gate", "feed_forward_gate")])
+def test_a_part_that_somebody_wraps_is_still_run_for_all_tokens(kind, name):
+    """Somebody who put a computation of their own in front of a part's, on the part, is handed every token's rows."""
+    k = RowTwins()
+    env = BuildEnv(k, torch.device("cpu"), torch.bfloat16, 64)
+    parts = dict(mixer=RowsMixer(lambda: rnd(TOKENS, HIDDEN, seed=1)), mixer_norm=norm(env), feed_forward=Half(),
+                 feed_forward_norm=norm(env))
+    if kind is GatedPreNormBlock:
+        parts.update(mixer_gate=Gate(), feed_forward_gate=Gate())
+    made, ctx, seen = kind(**parts), SimpleNamespace(kernels=k), []
+    method = "logits" if name.endswith("gate") else "forward"
+    own = getattr(parts[name], method)
+    setattr(parts[name], method, lambda *args, **more: seen.append(own(*args, **more)) or seen[-1])
+    stream = ResidualStream(rnd(TOKENS, HIDDEN, seed=5, dtype=torch.float32))
+    if not made.forward_rows(stream, ctx, None, torch.tensor([3], dtype=torch.int32)):
+        made.forward(stream, ctx, None)
+    assert [len(t) for t in seen] == [TOKENS]
