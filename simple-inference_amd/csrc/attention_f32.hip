@@ -20,7 +20,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define TURNS (TOKENS / WAVES)
 
 // DP: 64 or 128, the head sizes' upper bound.  HB: heads a wave takes together.
-template <int DP, int HB>
+// KEEP: with kept first positions; what tells them from the window costs the others 3 to 5 % (one token over 550 keys beside seven
+// more, 32 heads of 64 on 8: 64.8 us with, 61.1 without;  600 tokens 138.7 and 131.0).
+template <int DP, int HB, bool KEEP>
 __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
     const float* __restrict__ q, int q_row_stride, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ seq_of_token,
@@ -71,8 +73,8 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
             return chunk > 0 ? max(lo, pos - pos % chunk) : lo;
         };
         // chunks that some row of the run may see, in order: those of the kept positions, then from the window's on
-        const int lo0 = oldest(first), keep0 = min(keep_first, oldest(last)), c_lo = lo0 / CHUNK * CHUNK;
-        auto next_chunk = [&](int c0) { return c0 + CHUNK < keep0 ? c0 + CHUNK : max(c0 + CHUNK, c_lo); };
+        const int lo0 = oldest(first), keep0 = KEEP ? min(keep_first, oldest(last)) : 0, c_lo = lo0 / CHUNK * CHUNK;
+        auto next_chunk = [&](int c0) { return KEEP && c0 + CHUNK < keep0 ? c0 + CHUNK : max(c0 + CHUNK, c_lo); };
         auto page_of = [&](int c0) {
             const int j = c0 + lane;
             return j <= last && (j >> page_log2) < table_width ? table[j >> page_log2] : -1;
@@ -121,7 +123,7 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
                 for (int a = 0; a < DP / SIA_WAVE; ++a) acc[t][h][a] = 0.f;
             }
 
-        int c0 = keep0 > 0 ? 0 : c_lo;
+        int c0 = KEEP && keep0 > 0 ? 0 : c_lo;
         int page = page_of(c0), page_next = page_of(next_chunk(c0));
         fetch(c0, page);
         while (c0 <= last) {
@@ -137,10 +139,10 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
             for (int t = 0; t < TURNS; ++t) {
                 const int i = wave + t * WAVES;
                 if (i >= n) continue;
-                const int pos = positions[t0 + i], lo = oldest(pos), keep = min(keep_first, lo);
-                if (c0 > pos || (c0 + CHUNK <= lo && c0 >= keep)) continue;      // no visible key in this chunk
+                const int pos = positions[t0 + i], lo = oldest(pos), keep = KEEP ? min(keep_first, lo) : 0;
+                if (c0 > pos || (c0 + CHUNK <= lo && !(KEEP && c0 < keep))) continue;      // no visible key in this chunk
                 const int j = c0 + lane;
-                const bool visible = (j >= lo || j < keep) && j <= pos && has_page;
+                const bool visible = (j >= lo || (KEEP && j < keep)) && j <= pos && has_page;
                 float s[HB];
 #pragma unroll
                 for (int h = 0; h < HB; ++h) s[h] = 0.f;
@@ -169,12 +171,12 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
                     p_w[h * CHUNK + lane] = p;
                 }
                 __builtin_amdgcn_wave_barrier();      // the wave's LDS accesses run in order: no more than that is needed
-                // values of keys that the row does not see may be anything: they are left out, not weighted with 0.  (In a
-                // chunk with kept positions the loop is run for those, and again for what the window holds of the chunk: a test for
-                // the gap between them inside the loop cost every chunk; four layers of 303 tokens at the 1B widths 3,581 us, so 3,565.)
+                // values of keys that the row does not see may be anything: they are left out, not weighted with 0.  In a
+                // chunk with kept positions the loop is run for those, and again for what the window holds of the chunk.
                 const int j_last = min(pos, c0 + CHUNK - 1) - c0;
-                int j_from = c0 < keep ? 0 : max(lo, c0) - c0, j_to = c0 < keep ? min(keep, c0 + CHUNK) - 1 - c0 : j_last;
-                while (j_from <= j_to) {
+                const bool kept = KEEP && c0 < keep;
+                int j_from = kept ? 0 : max(lo, c0) - c0, j_to = kept ? min(keep, c0 + CHUNK) - 1 - c0 : j_last;
+                for (;;) {
                     for (int jj = j_from & ~3; jj <= j_to; jj += 4) {
                         const bool whole = jj >= j_from && jj + 3 <= j_to;
                         f32x4 pp[HB];
@@ -193,6 +195,7 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
                                 for (int e = 0; e < 4; ++e) acc[t][h][a] += pp[h][e] * vv[e];
                         }
                     }
+                    if (!KEEP || j_to >= j_last) break;
                     j_from = max(lo - c0, j_to + 1);
                     j_to = j_last;
                 }
@@ -233,14 +236,15 @@ static int launch(const float* q, int q_row_stride, const float* k_pages, const 
     const long long at_once = 256 * min(2, 160 * 1024 / bytes), many = n_tokens - n_single, runs = n_seqs - n_single;
     if (many > 0 && 4 * many * n_tokens * (n_heads / HB) <= at_once * max(4 * many, 3 * TOKENS * runs)) n_single = n_tokens;
     const dim3 grid(n_single + (n_tokens - n_single + TOKENS - 1) / TOKENS, n_heads / HB);
-    auto kernel = attention_f32_kernel<DP, HB>;
-    static bool set[64] = {};      // more LDS than a kernel gets unasked, allowed once per device
+    const bool keeps = keep_first > 0;
+    auto kernel = keeps ? attention_f32_kernel<DP, HB, true> : attention_f32_kernel<DP, HB, false>;
+    static bool set[64][2] = {};      // more LDS than a kernel gets unasked, allowed once per device
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return (int)hipGetLastError();
-    if (device < 0 || device >= 64 || !set[device]) {
+    if (device < 0 || device >= 64 || !set[device][keeps]) {
         const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e != hipSuccess) return (int)e;
-        if (device >= 0 && device < 64) set[device] = true;
+        if (device >= 0 && device < 64) set[device][keeps] = true;
     }
     hipLaunchKernelGGL(kernel, grid, dim3(WAVES * SIA_WAVE), bytes, stream, q, q_row_stride, k_pages, v_pages, block_table,
                        table_width, seq_of_token, positions, out, n_tokens, n_single, n_heads, n_kv, head_dim, value_dim,
