@@ -8,7 +8,7 @@
 // earlier.  A token that is its sequence's only one (decode) has a workgroup of its own, and so has every token of a step
 // that leaves the chip room for that.  Everything a row's result is made of (chunks, order of sums, exponentials) is as in the
 // plain kernel, so it depends on the row's own keys only, not on which of the forms it goes through.
-//   303 tokens (three decoded over 200 keys, a prompt of 300), 32 heads of 64 on 8: 240 -> 59 us;  one token over 16,000 keys 3,895 ->
+//   303 tokens (three decoded over 200 keys, a prompt of 300), 32 heads of 64 on 8: 240 -> 58 us;  one token over 16,000 keys 3,895 ->
 //   1,365, 64 over 2,048 810 -> 215.
 #include "common.h"
 
@@ -225,15 +225,18 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
 template <int DP, int HB>
 static int launch(const float* q, int q_row_stride, const float* k_pages, const float* v_pages, const int* block_table,
                   int table_width, const int* seq_of_token, const int* positions, float* out, int n_tokens, int n_single,
-                  int n_seqs, int n_heads, int n_kv, int head_dim, int value_dim, int page_size, float scale, int window, int chunk,
-                  const float* sinks, float cap, int keep_first, hipStream_t stream) {
+                  int n_seqs, int max_kv, int max_run_kv, int n_heads, int n_kv, int head_dim, int value_dim, int page_size, float scale,
+                  int window, int chunk, const float* sinks, float cap, int keep_first, hipStream_t stream) {
     constexpr int bytes = (CHUNK * (DP + 4) + DP * (CHUNK + 4) + TOKENS * HB * DP + WAVES * HB * CHUNK) * (int)sizeof(float);
     // Eight tokens a workgroup share what is loaded, but follow one another in a wave, and their sequences one another in the
     // workgroup: a token each where one round of two workgroups a unit (one, if LDS holds no more) takes them all, or, if an eight
     // holds several sequences, three rounds for four of them.  32 heads of 64 on 8, us, the plain kernel, eight, one:  8 tokens over 72 keys
     // 20, 25, 14.5;  16 over 216 53, 49, 27;  64 over 264 87, 59, 36;  128 over 328 182, 71, 80 (two rounds);  24 heads of
-    // 128 on 8, 16 sequences of 3 over 300 (two rounds) 164, 170, 90.
-    const long long at_once = 256 * min(2, 160 * 1024 / bytes), many = n_tokens - n_single, runs = n_seqs - n_single;
+    // 128 on 8, 16 sequences of 3 over 300 (two rounds) 164, 170, 90.  Where single tokens see more keys than the others do, the step
+    // takes as long as theirs, which a second workgroup on the unit makes longer: 45 tokens beside six over up to 145 keys 19.0 eight, 20.3 one;
+    // 60 beside three over up to 234 24.9 and 25.5;  with the others' keys more, 45 beside one over 30 15.2 and 9.6.
+    const long long many = n_tokens - n_single, runs = n_seqs - n_single;
+    const long long at_once = 256 * (n_single > 0 && max_run_kv < max_kv ? 1 : min(2, 160 * 1024 / bytes));
     if (many > 0 && 4 * many * n_tokens * (n_heads / HB) <= at_once * max(4 * many, 3 * TOKENS * runs)) n_single = n_tokens;
     const dim3 grid(n_single + (n_tokens - n_single + TOKENS - 1) / TOKENS, n_heads / HB);
     const bool keeps = keep_first > 0;
@@ -256,13 +259,13 @@ extern "C" int sia_attention_generic(const void*, int, const void*, const void*,
                                      int, int, int, int, int, int, float, int, int, const float*, float, int, int, hipStream_t);
 
 // The arguments of the plain kernel, and n_single: that many tokens, the first ones, are their sequences' only ones; n_seqs;
-// max_kv: no sequence holds more keys.  Rows of other sizes, and rows and pages that do not lie in sixteens of bytes, go to the plain
-// kernel; so do steps whose sequences hold so few keys that bringing them into LDS first takes longer than a wave a row and head
+// max_kv: no sequence holds more keys, max_run_kv: nor does one of more than a token (max_kv if that is not known).
+// Rows of other sizes, and rows and pages that do not lie in sixteens of bytes, go to the plain kernel; so do steps whose sequences hold so few keys that bringing them into LDS first takes longer than a wave a row and head
 // does, as long as those waves find room:  32 heads of 64 on 8, plain against this, us:  one token over 4 keys 6.1 / 8.2, 16: 7.4 / 8.6, 40:
 // 12.1 / 9.4, 16 tokens over 16 7.4 / 14.5;  24 heads of 128 on 8:  4: 6.6 / 10.4, 16: 11.3 / 10.9, 64 sequences over 16 13.4 / 20.8.
 SIA_EXPORT int sia_attention_f32(const float* q, int q_row_stride, const float* k_pages, const float* v_pages,
                                  const int* block_table, int table_width, const int* seq_of_token, const int* positions,
-                                 float* out, int n_tokens, int n_single, int n_seqs, int max_kv, int n_heads, int n_kv,
+                                 float* out, int n_tokens, int n_single, int n_seqs, int max_kv, int max_run_kv, int n_heads, int n_kv,
                                  int head_dim, int value_dim, int page_size, float scale, int window, int chunk, const float* sinks, float cap,
                                  int keep_first, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
@@ -280,7 +283,8 @@ SIA_EXPORT int sia_attention_f32(const float* q, int q_row_stride, const float* 
     auto run = [&](auto narrow, auto wide) {
         return (head_dim <= 64 && value_dim <= 64 ? narrow : wide)(
             q, q_row_stride, k_pages, v_pages, block_table, table_width, seq_of_token, positions, out, n_tokens, n_single,
-            n_seqs, n_heads, n_kv, head_dim, value_dim, page_size, scale, window, chunk, sinks, cap, keep_first, stream);
+            n_seqs, max_kv, max_run_kv, n_heads, n_kv, head_dim, value_dim, page_size, scale, window, chunk, sinks, cap, keep_first,
+            stream);
     };
     if (group % 4 == 0) return run(launch<64, 4>, launch<128, 4>);
     if (group % 3 == 0) return run(launch<64, 3>, launch<128, 3>);

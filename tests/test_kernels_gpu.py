@@ -478,11 +478,12 @@ def test_float32_attention_is_the_plain_kernels(hip, geom, more):
 
 @pytest.mark.parametrize("n_heads,n_kv,D", [(32, 8, 64), (24, 8, 128), (6, 6, 32)])
 @pytest.mark.parametrize("q_lens,kv_lens", [([16], [16]), ([17], [17]), ([1, 1, 3], [16, 2, 16]), ([3] * 16, [300] * 16), ([2] * 70, [40] * 70),
-                                            ([1, 40], [70, 40]), ([64], [264]), ([65], [265])])
+                                            ([1, 40], [70, 40]), ([1, 40], [30, 40]), ([64], [264]), ([65], [265])])
 def test_float32_attention_has_the_same_bits_whichever_way_it_goes(hip, n_heads, n_kv, D, q_lens, kv_lens):
     """Few keys (the plain kernel), few tokens or short runs (a workgroup a token), more (eight tokens a workgroup): each
     sequence's rows are those that it has alone."""
     ctx, ps = Ctx(q_lens, kv_lens), 16
+    ctx.max_run_kv_len = max([kv for q, kv in zip(q_lens, kv_lens) if q > 1], default=0)
     cache = Cache(sum(-(-kv // ps) for kv in kv_lens), n_kv, ps, D, torch.float32, kv_lens, seed=3)
     cache.k_pages.copy_(rnd(*cache.k_pages.shape, seed=4))
     cache.v_pages.copy_(rnd(*cache.v_pages.shape, seed=5))
