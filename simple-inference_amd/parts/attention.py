@@ -272,16 +272,22 @@ class Attention:
         """Whether ``forward`` gives the rows ``ctx.only_rows`` alone where it is set."""
         return type(self).forward is Attention.forward and not self.row_form
 
-    ALONE_FROM = 768     # keys
+    ALONE_FROM = 768         # keys
+    ALONE_BESIDE = 128       # tokens beside the single ones
 
     def rows_alone(self, rows, ctx) -> bool:
         """Whether attention of the rows that are read is taken as that of decoded tokens, not with the whole step's: about
-        a token a sequence, over keys enough to be worth the metadata made for it.  (Eight layers at the 1B and 3B widths and
-        four at 8B, whole -> alone:  a prompt of 128 840 -> 843 us, 1,197 -> 1,200, 971 -> 974, of 512 1,140 -> 1,141, 1,582 -> 1,583,
-        1,270 -> 1,274, of 1,024 1,696 -> 1,689, 2,260 -> 2,248, 1,873 -> 1,859;  17 tokens over 8,000 1,891 -> 1,753, 1,888 -> 1,769, 1,252 ->
-        1,133, 128 over 1,024 978 -> 969, 1,321 -> 1,313, 1,020 -> 1,014;  160 beside 63 rows of 700 1,216 -> 1,211, 1,672 -> 1,667, 1,264 -> 1,260.)"""
+        a token a sequence, over keys enough to be worth the metadata made for it; or with tokens enough beside decoded ones,
+        whose attention is then one launch instead of two; or in float32, whose attention takes longer.  (Eight layers at the 1B
+        and 3B widths and four at 8B, whole -> alone:  a prompt of 128 840 -> 843 us, 1,197 -> 1,200, 971 -> 974, of 512
+        1,140 -> 1,141, 1,582 -> 1,583, 1,270 -> 1,274, of 1,024 1,696 -> 1,689, 2,260 -> 2,248, 1,873 -> 1,859;  17 tokens over
+        8,000 1,891 -> 1,753, 1,888 -> 1,769, 1,252 -> 1,133, 128 over 1,024 978 -> 969, 1,321 -> 1,313, 1,020 -> 1,014;  160 beside
+        63 rows of 700 1,216 -> 1,211, 1,672 -> 1,667, 1,264 -> 1,260.  Four layers at 3B:  128 beside 8 rows of 100 652 -> 647,
+        300 beside 8 of 300 755 -> 745, beside 40 894 -> 885, 600 beside 40 of 500 1,083 -> 1,066.)"""
         span = min(n for n in (ctx.max_kv_len, self.window, self.chunk) if n is not None)
-        return rows.numel() <= ctx.n_seqs and span >= self.ALONE_FROM
+        beside = ((ctx.n_decode_seqs > 0 or self.env.dtype == torch.float32)
+                  and ctx.n_tokens >= ctx.n_decode_seqs + self.ALONE_BESIDE)
+        return rows.numel() <= ctx.n_seqs and (span >= self.ALONE_FROM or beside)
 
     def forward_rows(self, prepare, ctx, cache, rows):
         """The rows ``rows`` of the mixer's result (None if there are none) from what ``prepare(attend)`` gives: all rows of

@@ -74,6 +74,7 @@ def test_the_rows_that_are_read_alone_give_the_same_logits(folders, name, dtype,
     (the tolerance of the engine's tests).  Pre-norm blocks with a feed-forward and nothing behind it go by rows in the five
     steps of 32 tokens and more; others say that they do not, or are not asked (sandwich blocks)."""
     monkeypatch.setattr(Attention, "ALONE_FROM", alone_from)
+    monkeypatch.setattr(Attention, "ALONE_BESIDE", alone_from)
     got, got_kept, block, said, alone = steps(folders[name], dtype)
     monkeypatch.setattr(DecoderModel, "_few_rows_read", staticmethod(lambda ctx: False))
     want, want_kept, _, none, _ = steps(folders[name], dtype)
