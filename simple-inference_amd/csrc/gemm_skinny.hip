@@ -1,24 +1,31 @@
-// Y[M, N] = X[M, K] * W[N, K]^T in bfloat16 with float accumulation, for few rows (M <= 16):
-// the matrix products of a decode step, where every weight is read once and the time is the time
-// to stream W from HBM.
+// Y[M, N] = X[M, K] * W[N, K]^T in bfloat16 with float accumulation, for few rows (M <= 64): the matrix products of a
+// decode step and of a short prompt, where every weight is read once and the time is the time to stream W from HBM.
 //
-// One workgroup of 8 or 16 waves per RB blocks of up to 16 rows of W.  K is cut into chunks of 128, and chunk c
+// One workgroup of 4 or 8 waves per RB blocks of up to 16 rows of W.  K is cut into chunks of 128, and chunk c
 // belongs to *share* c % 16: a share's chunks are summed front to back into one accumulator, and the 16 shares'
-// sums are added as (s0 + s8) + (s1 + s9) + ... + (s7 + s15), left to right.  With 16 waves every wave has one
-// share and the sums meet in LDS; with 8, wave w has shares w and w + 8 (chunks w, w + 8, w + 16, ... alternate
-// between its two accumulators) and adds the two itself, so the workgroup still walks its rows front to back
-// and needs half the LDS.  A wave's step covers 64 k of RB blocks of rows with 2*RB MFMAs 16x16x32:
-//   A = W[row of lane r in block rb][k0 + 16g .. + 15]   two 16-byte loads a lane, 128 contiguous bytes per row
-//   B = X[r][same k]                                     loaded once for all RB blocks
+// sums are added as (s0 + s8) + (s1 + s9) + ... + (s7 + s15), left to right.  Wave w has the shares w, w + WAVES, ...,
+// one accumulator each, and the workgroup walks its rows front to back.  A wave's step covers 64 k of its blocks with
+// MFMAs 16x16x32:
+//   A = W[row of lane r in block rb][k0 + 16g .. + 15],   B = X[r of block mb][same k]
 // (an MFMA's k index only has to mean the same element in A and B, so lane group g may take the 16
-// consecutive k that start at 16g and feed them to two MFMAs.)  X is small and comes from the caches, once per
-// workgroup.
+// consecutive k that start at 16g and feed them to two MFMAs.)
 //
-// A compute unit streams its rows at a rate of its own, well below its share of what the memory delivers, so a
-// product is as fast as the busiest compute unit: a block holds `bh` <= 16 rows, chosen on the host so that
+// A step's rows of W and X come to LDS directly (global_load_lds), into a ring of SLOTS steps that the wave has for
+// itself: nobody waits at a barrier before the sums meet, and what is on its way takes no registers.  A load
+// instruction brings the 128 bytes of 8 rows, whole cache lines in lane order.  (Loaded straight into the MFMAs' registers,
+// neighbouring lanes hold different rows, so an instruction touches 16 lines in pieces of 16 bytes, and the address unit,
+// not the memory, sets the pace.  us a launch, everything from memory, before -> now:  gate/up with SwiGLU of 8,192 x 2,048
+// 17.7 -> 14.4, x 3,072 21.0 -> 19.8, 14,336 x 4,096 50 -> 42.5;  2,048 x 8,192 11.1 -> 8.2, 3,072 x 8,192 12.3 -> 10.7;  a read of
+// the same bytes that does nothing else takes 12.1, 19.2, 42; 7.6, 10.2.  A second copy of W in the order of the loads gains nothing
+// over this.)
+//   Inside a 1 KiB tile of 8 rows the 16-byte pieces of a row are permuted by the row's number (the lane that writes place p
+// of row r fetches piece p ^ turn(r)), so that the 16 lanes that a 128-bit LDS read serves at a time meet no bank twice.
+//
+// X is fetched once per workgroup (L2 serves it); a workgroup whose rows are few against X's takes more of them at once.
+// A product is as fast as the busiest compute unit: a block holds `bh` <= 16 rows, chosen on the host so that
 // the workgroups come out as a whole number of rounds over the compute units (3,072 rows on 256 units: 256
-// blocks of 12, not 192 of 16).  Lanes r >= bh load the block's last row again (the same cache lines, no further
-// traffic) and rows m >= M of X the last live one; what the MFMAs make of them is never stored.
+// blocks of 12, not 192 of 16).  Rows beyond the block, and rows m >= M of X, are the last live one again (the same cache
+// lines, no further traffic), or not fetched where a whole tile of 8 is beyond; what the MFMAs make of them is never stored.
 //
 // The result element (m, n) is summed over k in an order that depends on K only, not on M, the other rows,
 // the number of waves, the row blocks of a workgroup or their height: whichever shape a launch takes, a row's
@@ -30,12 +37,41 @@
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-constexpr int SK_STEP = 64;    // k per step of one wave
-constexpr int SK_CHUNK = 128;  // k per chunk: two steps
-constexpr int SK_SHARES = 16;  // chunk c is summed into share c % 16
+constexpr int SK_STEP = 64;      // k per step of one wave: 128 bytes of a row
+constexpr int SK_CHUNK = 128;    // k per chunk: two steps
+constexpr int SK_SHARES = 16;    // chunk c is summed into share c % 16
+constexpr int SK_MAX_ROWS = 64;
+constexpr int SK_TILE = 1024;    // bytes of a load instruction: 8 rows of a step
+constexpr int SK_LDS = 160 * 1024;
 
-__device__ __forceinline__ bf16x8 ld8(const bf16_t* p) {
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
+// 16 bytes a lane from `src` into LDS at dst + 16 * lane; counts in vmcnt.
+__device__ __forceinline__ void load_to_lds(const void* src, void* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// Until at most `AT_MOST` of the wave's loads are on their way (they end in the order in which they were made).
+template <int AT_MOST> __device__ __forceinline__ void wait_loads() {
+    static_assert(AT_MOST >= 0 && AT_MOST < 64, "vmcnt has 6 bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AT_MOST) : "memory");
+}
+
+// The same for `steps` <= SLOTS - 1 steps behind the one that is waited for.
+template <int LOADS, int SLOTS> __device__ __forceinline__ void wait_step(int steps) {
+    if constexpr (SLOTS == 1)
+        wait_loads<0>();
+    else if (steps >= SLOTS - 1)
+        wait_loads<(SLOTS - 1) * LOADS>();
+    else
+        wait_step<LOADS, SLOTS - 1>(steps);
+}
+
+// Place p of row r (of 16) holds piece p ^ turn(r).  A 128-bit LDS read is served 16 lanes at a time, lanes 0-3, 12-15, 20-23
+// and 24-27 first: rows 0-3 and 12-15 of one lane group, 4-11 of the next, whose pieces differ by 2.  Rows 2j and 2j + 1 lie in
+// the two halves of the 64 banks; this order of j keeps the eight places of a half apart for every such set.
+__device__ __forceinline__ int turn(int r) {
+    const int j = r >> 1;
+    return (j & 1) | ((j >> 2) & 1) << 1 | (((j >> 1) ^ (j >> 2)) & 1) << 2;
 }
 
 enum SkinnyEpilogue { EPI_STORE = 0, EPI_SWIGLU = 1, EPI_ROPE = 2, EPI_RESIDUAL = 3, EPI_ACT = 4, EPI_GROUPED = 5 };
@@ -57,10 +93,10 @@ struct ResidualOut {
     float* residual;      // [M][N], updated in place
     const float* gain;    // [N], the norm's weight
     bf16_t* scaled;       // [M][N] = residual * gain, not yet divided by the row's root mean square
-    float* partials;      // [column blocks][16]: sum over a block's columns of residual^2, by row
+    float* partials;      // [column blocks][16]: sum over a block's columns of residual^2, by row (M <= 16)
 };
 
-// X is such a `scaled` matrix: row m of the result is to be multiplied by rsqrt(sum_p partials[p][m] / K + eps).
+// X is such a `scaled` matrix (M <= 16): row m of the result is to be multiplied by rsqrt(sum_p partials[p][m] / K + eps).
 struct RowScale {
     const float* partials;
     int n_partials;
@@ -81,7 +117,8 @@ struct Epilogue {
     int groups, group_rows, last_rows, group_blocks;   // EPI_GROUPED: see below
 };
 
-// RB: blocks of bh rows of W per workgroup; WAVES: 8 or 16 waves that split K.
+// RB: blocks of bh rows of W per workgroup; MB: blocks of 16 rows of X; WAVES: 4 or 8 waves that split K; SLOTS: steps in
+// a wave's ring; WI: tiles of 8 rows that a block of W has (1 where bh <= 8); XI: tiles of X (1 where M <= 8, else 2 MB).
 //   EPI_STORE:   row block rb holds bh rows of W and gives as many columns of Y (TOut)
 //   EPI_ACT:     as EPI_STORE, with an activation without a gate applied to the float sums, rounded once
 //   EPI_SWIGLU:  W = [gate; up] of N rows each; the first RB / 2 row blocks are gate rows, the others the up rows of
@@ -98,25 +135,36 @@ struct Epilogue {
 //                [groups][M][K], group g has group_rows rows of W (the last one last_rows) and gives the matrix
 //                Y + g * M * group_rows, [M][its rows]; a workgroup's blocks lie in one group (group_blocks workgroups
 //                each).
+// With MB > 1 (more than 16 rows) the epilogues that change the sums, EPI_SWIGLU and EPI_ROPE, round them to bfloat16 first, as
+// EPI_STORE does: steps of that many rows give the bits of the product and the kernel behind it.
 // Output columns come in *units*: a column of Y (EPI_STORE, EPI_RESIDUAL, EPI_SWIGLU, where unit u needs row u of
 // the gate half and row u of the up half of W), or a pair of columns that the rotation mixes (EPI_ROPE: unit u is
 // column u % (head_dim / 2) of head u / (head_dim / 2) together with the column head_dim / 2 further).  A workgroup
 // owns UNIT_BLOCKS blocks of bh consecutive units from blockIdx.x * UNIT_BLOCKS * bh on.
-// TILED: W is not [N][K] but a copy laid out for this cut, so that every load instruction of a wave reads one
-// run of memory: [block of bh rows][step of 64 k][half of a lane's 16 k][row][lane group][8 k] (see
-// sia_gemm_skinny_tiled_weights).  The same elements meet in the same products, so no bit changes.
-template <typename TOut, int RB, int WAVES, int EPI, bool SCALED, bool TILED = false>
+template <typename TOut, int EPI, bool SCALED, int RB, int MB, int WAVES, int SLOTS, int WI, int XI>
 __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16_t* __restrict__ X,
                                                                      const bf16_t* __restrict__ W,
                                                                      TOut* __restrict__ Y, int M, int N, int K,
                                                                      int bh, const Epilogue ep) {
-    static_assert(WAVES == 8 || WAVES == 16, "8 or 16 waves share the 16 shares of K");
+    static_assert(WAVES == 4 || WAVES == 8, "4 or 8 waves share the 16 shares of K");
     static_assert(EPI != EPI_ROPE || RB == 2, "the rotation pairs two row blocks");
     static_assert(EPI != EPI_SWIGLU || RB % 2 == 0, "gate and up rows come in equal numbers");
+    static_assert((WI == 1 || WI == 2) && (XI == 2 * MB || (MB == 1 && XI == 1)), "tiles of 8 rows");
+    static_assert(MB == 1 || (!SCALED && EPI != EPI_RESIDUAL && EPI != EPI_ACT), "forms of up to 16 rows");
+    constexpr bool ROUND_FIRST = MB > 1;
+    constexpr int THREADS = WAVES * SIA_WAVE;
     constexpr int SPW = SK_SHARES / WAVES;  // shares per wave
     constexpr int UNIT_BLOCKS = EPI == EPI_SWIGLU ? RB / 2 : EPI == EPI_ROPE ? 1 : RB;
-    __shared__ float part[WAVES][RB][16][17];
-    __shared__ float squares[SK_SHARES][16];
+    constexpr int LOADS = RB * WI + XI;     // of a step
+    constexpr int ROWS = MB * 16;
+    // the ring, and when the weights have been read the sums of pairs of shares and a row's sums of squares in its place
+    constexpr int RING = WAVES * SLOTS * LOADS * SK_TILE;
+    constexpr int PART = 8 * RB * ROWS * 17 * 4, SQUARES = SCALED ? SK_SHARES * 16 * 4 : 0;
+    constexpr int LDS = RING > PART + SQUARES ? RING : PART + SQUARES;
+    static_assert(LDS <= SK_LDS, "a workgroup's LDS");
+    __shared__ __attribute__((aligned(1024))) char lds[LDS];
+    float(*part)[RB][ROWS][17] = reinterpret_cast<float(*)[RB][ROWS][17]>(lds);
+    float(*squares)[16] = reinterpret_cast<float(*)[16]>(lds + PART);
     const RopeOut& rope = ep.rope;
     int bx = blockIdx.x;
     if (EPI == EPI_GROUPED) {
@@ -135,22 +183,25 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     // the unit of place n of unit block jb; places beyond the block or beyond the last unit repeat a unit before
     auto unit_at = [&](int jb, int n) { return min(u0 + jb * bh + min(n, bh - 1), units - 1); };
     auto is_live = [&](int jb, int n) { return n < bh && u0 + jb * bh + n < units; };
-    const bf16_t* x_row = X + (size_t)min(r, M - 1) * K + g * 16;
-    const bf16_t* w_row[RB];
+    auto row_of = [&](int rb, int n) {
+        const int u = unit_at(rb % UNIT_BLOCKS, n);
+        if (EPI == EPI_ROPE)  // the second row block holds the rotation's partners
+            return (u / rope_half) * rope.head_dim + u % rope_half + rb * rope_half;
+        return u + (rb / UNIT_BLOCKS) * N;  // rb / UNIT_BLOCKS: 0 gate (or all), 1 up
+    };
+    // load l of a step: its first row, the same in all lanes, and this lane's 16 bytes from there at k = 0.  Lane p of a row's
+    // eight fetches the piece that belongs at place p.  (Units ascend with n and rows with units: the offset is not negative.)
+    const bf16_t* base[LOADS];
+    unsigned offset[LOADS];
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-        int row;
-        if (EPI == EPI_ROPE) {  // the second row block holds the rotation's partners
-            const int u = unit_at(0, r);
-            row = (u / rope_half) * rope.head_dim + u % rope_half + rb * rope_half;
-        } else {  // rb / UNIT_BLOCKS: 0 gate (or all), 1 up
-            row = unit_at(rb % UNIT_BLOCKS, r) + (rb / UNIT_BLOCKS) * N;
-        }
-        w_row[rb] = W + (size_t)row * K + g * 16;
-        if (TILED)  // the block's tiles: (step, half) apart by bh * 32 elements, this lane's piece inside a tile
-            w_row[rb] = W + (size_t)(blockIdx.x * RB + rb) * (K / SK_STEP) * 2 * bh * 32 + (min(r, bh - 1) * 4 + g) * 8;
+    for (int l = 0; l < LOADS; ++l) {
+        const bool of_w = l < RB * WI;
+        const int n = 8 * (of_w ? l % WI : l - RB * WI) + lane / 8;
+        const int first = of_w ? __builtin_amdgcn_readfirstlane(row_of(l / WI, 0)) : 0;
+        const int row = of_w ? row_of(l / WI, n) : min(n, M - 1);
+        base[l] = (of_w ? W : X) + (size_t)first * K;
+        offset[l] = ((unsigned)(row - first) * (unsigned)K + ((lane & 7) ^ turn(n & 15)) * 8) * 2;
     }
-    static_assert(!TILED || EPI == EPI_STORE || EPI == EPI_RESIDUAL, "tiled weights: a row block is a block of columns");
 
     // requested before the weights, used after them.  The sums of squares of a row are added up the way the
     // products are: 64 runners (16 shares of 4 lane groups), runner l taking partials l, l + 64, ...
@@ -166,77 +217,119 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
                 sq[j][i] = p < ep.scale.n_partials ? ep.scale.partials[p * 16 + sq_m] : 0.f;
             }
     }
-    constexpr int RES_ITER = (RB * 256 + WAVES * SIA_WAVE - 1) / (WAVES * SIA_WAVE);
+    constexpr int RES_ITER = EPI == EPI_RESIDUAL ? (RB * 256 + THREADS - 1) / THREADS : 1;
     float res_old[RES_ITER], res_gain[RES_ITER];
     if (EPI == EPI_RESIDUAL) {
 #pragma unroll
         for (int it = 0; it < RES_ITER; ++it) {
-            const int idx = threadIdx.x + it * WAVES * SIA_WAVE;
+            const int idx = threadIdx.x + it * THREADS;
             const int j = idx / 256, m = (idx / 16) % 16, n = idx % 16;
             const bool live = idx < RB * 256 && m < M && is_live(j, n);
             res_old[it] = live ? ep.res.residual[(size_t)m * N + u0 + j * bh + n] : 0.f;
             res_gain[it] = live ? ep.res.gain[u0 + j * bh + n] : 0.f;
         }
     }
+    constexpr int ROPE_ITER = EPI == EPI_ROPE ? (ROWS * 16 + THREADS - 1) / THREADS : 1;
+    int position[ROPE_ITER], sequence[ROPE_ITER];
+    if (EPI == EPI_ROPE) {
+#pragma unroll
+        for (int it = 0; it < ROPE_ITER; ++it) {
+            const int m = min((int)(threadIdx.x + it * THREADS) / 16, M - 1);
+            position[it] = rope.positions[m];
+            sequence[it] = rope.seq_of_token[m];
+        }
+    }
 
-    // acc[j] belongs to share wave + j * WAVES.  This wave's t-th chunk is chunk wave + t * WAVES, of share
-    // (wave + t * WAVES) % 16 = wave + (t % SPW) * WAVES, so it goes into accumulator t % SPW; the chunks are
-    // taken in order of t, which is each share's own order.  (Loading a second group of chunks into registers of
-    // their own while the first is multiplied was measured and changes nothing: enough waves are in flight.)
-    floatx4 acc[SPW][RB];
+    // Step s of the wave: half s % 2 of its chunk s / 2, chunk wave + (s / 2) * WAVES of the row, whose share has the
+    // accumulator (s / 2) % SPW.  Only the row's last chunk may be half a chunk (K is a multiple of 64).
+    const int row_steps = K / SK_STEP;
+    const int turns = row_steps / (2 * WAVES), rest = row_steps % (2 * WAVES) - 2 * wave;
+    const int steps = 2 * turns + min(max(rest, 0), 2);
+    char* ring = lds + wave * (SLOTS * LOADS * SK_TILE);
+    auto request = [&](int s, int slot) {
+        const size_t k = (size_t)(wave + (s >> 1) * WAVES) * SK_CHUNK + (s & 1) * SK_STEP;
+        char* to = ring + slot * (LOADS * SK_TILE);
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) load_to_lds((const char*)(base[l] + k) + offset[l], to + l * SK_TILE);
+    };
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s)
+        if (s < steps) request(s, s);
+
+    // what the rotation and the cache write need is on its way beside the weights
+    float rope_cos[ROPE_ITER], rope_sin[ROPE_ITER];
+    int rope_page[ROPE_ITER];
+    if (EPI == EPI_ROPE) {
+        const int u = unit_at(0, threadIdx.x % 16), head = u / rope_half, j = u % rope_half;
+#pragma unroll
+        for (int it = 0; it < ROPE_ITER; ++it) {
+            const bool rotates = head < rope.n_heads + rope.n_kv, cached = head >= rope.n_heads;
+            const size_t at = (size_t)position[it] * rope_half + j;
+            rope_cos[it] = rotates ? rope.cos_table[at] : 1.f;
+            rope_sin[it] = rotates ? rope.sin_table[at] : 0.f;
+            rope_page[it] = cached ? rope.block_table[(size_t)sequence[it] * rope.table_width + position[it] / rope.page_size] : 0;
+        }
+    }
+
+    const int wr = WI == 1 ? r & 7 : r, xr = XI == 1 ? r & 7 : r;
+    const int w_at[2] = {wr * 128 + ((2 * g) ^ turn(wr)) * 16, wr * 128 + ((2 * g + 1) ^ turn(wr)) * 16};
+    const int x_at[2] = {xr * 128 + ((2 * g) ^ turn(xr)) * 16, xr * 128 + ((2 * g + 1) ^ turn(xr)) * 16};
+    floatx4 acc[SPW][RB][MB];
 #pragma unroll
     for (int j = 0; j < SPW; ++j)
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) acc[j][rb] = floatx4{0.f, 0.f, 0.f, 0.f};
-    constexpr int HOP = WAVES * SK_CHUNK;  // from one chunk of the wave to its next
-    for (int k0 = wave * SK_CHUNK; k0 < K; k0 += SPW * HOP) {
+        for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int j = 0; j < SPW; ++j) {
-            // k is the same in all lanes of the wave (a scalar): a step outside K is skipped by a branch of the
-            // wave, not by a mask of lanes.  K is a multiple of 64, so a step is inside or outside as a whole.
-            const int k = k0 + j * HOP;
-            bf16x8 a[2][RB][2], b[2][2];
+            for (int mb = 0; mb < MB; ++mb) acc[j][rb][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+    int slot = 0;
+    for (int s0 = 0; s0 < steps; s0 += 2 * SPW) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-                if (k + u * SK_STEP < K) {
+        for (int t = 0; t < 2 * SPW; ++t) {
+            const int s = s0 + t, j = t / 2;
+            // s is the same in all lanes of the wave (a scalar): a step beyond the last is skipped by a branch
+            if (s < steps) {
+                wait_step<LOADS, SLOTS>(steps - 1 - s);
+                const char* from = ring + slot * (LOADS * SK_TILE);
+                bf16x8 a[RB][2], b[MB][2];
 #pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) {
-                        if (TILED) {
-                            const size_t tile = (size_t)((k / SK_STEP + u) * 2) * bh * 32;
-                            a[u][rb][0] = ld8(w_row[rb] + tile);
-                            a[u][rb][1] = ld8(w_row[rb] + tile + bh * 32);
-                        } else {
-                            a[u][rb][0] = ld8(w_row[rb] + k + u * SK_STEP);
-                            a[u][rb][1] = ld8(w_row[rb] + k + u * SK_STEP + 8);
-                        }
-                    }
-                    b[u][0] = ld8(x_row + k + u * SK_STEP);
-                    b[u][1] = ld8(x_row + k + u * SK_STEP + 8);
+                for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) b[mb][h] = *(const bf16x8*)(from + (RB * WI + 2 * mb) * SK_TILE + x_at[h]);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) a[rb][h] = *(const bf16x8*)(from + rb * WI * SK_TILE + w_at[h]);
                 }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot has been read: it may be filled again
+                if (s + SLOTS < steps) request(s + SLOTS, slot);
+                slot = slot + 1 < SLOTS ? slot + 1 : 0;
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-                if (k + u * SK_STEP < K) {
+                for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) {
-                        acc[j][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][rb][0], b[u][0], acc[j][rb], 0, 0, 0);
-                        acc[j][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][rb][1], b[u][1], acc[j][rb], 0, 0, 0);
+                    for (int mb = 0; mb < MB; ++mb) {
+                        acc[j][rb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb][0], b[mb][0], acc[j][rb][mb], 0, 0, 0);
+                        acc[j][rb][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb][1], b[mb][1], acc[j][rb][mb], 0, 0, 0);
                     }
-                }
+            }
         }
     }
-    // acc[j][rb][i] = share wave + j * WAVES of row m = r, column 4g + i of row block rb
+    __syncthreads();  // every wave has read its ring
+    // acc[j][rb][mb][i] = share wave + j * WAVES of row m = 16 mb + r, column 4g + i of row block rb; part[w]: shares w and w + 8
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            part[wave][rb][r][g * 4 + i] = SPW == 2 ? acc[0][rb][i] + acc[SPW - 1][rb][i] : acc[0][rb][i];
-    // the sum over all of k of element (j, m, n): pairs of shares s and s + 8, then the pairs left to right
+        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < SPW / 2; ++j)
+                    part[wave + j * WAVES][rb][mb * 16 + r][g * 4 + i] = acc[j][rb][mb][i] + acc[j + SPW / 2][rb][mb][i];
+    // the sum over all of k of element (j, m, n)
     auto total = [&](int j, int m, int n) -> float {
         float s = 0.f;
 #pragma unroll
-        for (int w = 0; w < 8; ++w) s += WAVES == 16 ? part[w][j][m][n] + part[w + 8][j][m][n] : part[w][j][m][n];
+        for (int w = 0; w < 8; ++w) s += part[w][j][m][n];
         return s;
     };
+    auto rounded = [](float x) { return ROUND_FIRST ? bf16_to_float(float_to_bf16(x)) : x; };
     if (SCALED) {
 #pragma unroll
         for (int j = 0; j < SPW; ++j) {
@@ -258,46 +351,51 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
         return rsqrtf(ss / (float)K + ep.scale.eps);
     };
     if (EPI == EPI_ROPE) {
-        const int m = threadIdx.x / 16, n = threadIdx.x % 16;
-        if (threadIdx.x >= 256 || m >= M || !is_live(0, n)) return;
-        float a = total(0, m, n), b = total(1, m, n);  // columns j and j + half of the head
-        const float rs = row_scale(m);
-        a *= rs;
-        b *= rs;
-        const int u = u0 + n, head = u / rope_half, j = u % rope_half, pos = rope.positions[m];
+        const int n = threadIdx.x % 16;
+        if (!is_live(0, n)) return;
+        const int u = u0 + n, head = u / rope_half, j = u % rope_half;
         const bool is_v = head >= rope.n_heads + rope.n_kv;
-        if (!is_v) {
-            const float c = rope.cos_table[(size_t)pos * rope_half + j], sn = rope.sin_table[(size_t)pos * rope_half + j];
-            const float ra = a * c - b * sn, rb_ = b * c + a * sn;
-            a = ra;
-            b = rb_;
-        }
-        if (head < rope.n_heads) {
-            TOut* y = Y + (size_t)m * N + head * rope.head_dim;
-            y[j] = from_float<TOut>(a);
-            y[j + rope_half] = from_float<TOut>(b);
-            return;
-        }
-        const int page = rope.block_table[(size_t)rope.seq_of_token[m] * rope.table_width + pos / rope.page_size];
-        if (page < 0) return;  // never for a token the step owns
-        const int off = pos % rope.page_size, D = rope.head_dim, ps = rope.page_size;
-        if (!is_v) {
-            const int hk = head - rope.n_heads;
-            bf16_t* dst = rope.k_pages + (((size_t)page * rope.n_kv + hk) * ps + off) * D;
-            dst[j] = float_to_bf16(a);
-            dst[j + rope_half] = float_to_bf16(b);
-        } else {
-            const int hk = head - rope.n_heads - rope.n_kv;
-            bf16_t* dst = rope.v_pages + ((size_t)page * rope.n_kv + hk) * D * ps + off;
-            dst[(size_t)j * ps] = float_to_bf16(a);
-            dst[(size_t)(j + rope_half) * ps] = float_to_bf16(b);
+#pragma unroll
+        for (int it = 0; it < ROPE_ITER; ++it) {
+            const int m = (threadIdx.x + it * THREADS) / 16;
+            if (m >= M) return;
+            float a = total(0, m, n), b = total(1, m, n);  // columns j and j + half of the head
+            const float rs = row_scale(m);
+            a = rounded(a * rs);
+            b = rounded(b * rs);
+            if (!is_v) {
+                const float c = rope_cos[it], sn = rope_sin[it];
+                const float ra = a * c - b * sn, rb_ = b * c + a * sn;
+                a = ra;
+                b = rb_;
+            }
+            if (head < rope.n_heads) {
+                TOut* y = Y + (size_t)m * N + head * rope.head_dim;
+                y[j] = from_float<TOut>(a);
+                y[j + rope_half] = from_float<TOut>(b);
+                continue;
+            }
+            const int page = rope_page[it];
+            if (page < 0) continue;  // never for a token the step owns
+            const int off = position[it] % rope.page_size, D = rope.head_dim, ps = rope.page_size;
+            if (!is_v) {
+                const int hk = head - rope.n_heads;
+                bf16_t* dst = rope.k_pages + (((size_t)page * rope.n_kv + hk) * ps + off) * D;
+                dst[j] = float_to_bf16(a);
+                dst[j + rope_half] = float_to_bf16(b);
+            } else {
+                const int hk = head - rope.n_heads - rope.n_kv;
+                bf16_t* dst = rope.v_pages + ((size_t)page * rope.n_kv + hk) * D * ps + off;
+                dst[(size_t)j * ps] = float_to_bf16(a);
+                dst[(size_t)(j + rope_half) * ps] = float_to_bf16(b);
+            }
         }
         return;
     }
     if (EPI == EPI_RESIDUAL) {
 #pragma unroll
         for (int it = 0; it < RES_ITER; ++it) {
-            const int idx = threadIdx.x + it * WAVES * SIA_WAVE;
+            const int idx = threadIdx.x + it * THREADS;
             const int j = idx / 256, m = (idx / 16) % 16, n = idx % 16;
             if (idx >= RB * 256 || m >= M) continue;  // a whole 16-lane group leaves or stays
             const bool live = is_live(j, n);
@@ -317,15 +415,13 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
         }
         return;
     }
-    for (int idx = threadIdx.x; idx < UNIT_BLOCKS * 256; idx += WAVES * SIA_WAVE) {
-        const int j = idx / 256, m = (idx / 16) % 16, n = idx % 16;
+    for (int idx = threadIdx.x; idx < UNIT_BLOCKS * ROWS * 16; idx += THREADS) {
+        const int j = idx / (ROWS * 16), m = (idx / 16) % ROWS, n = idx % 16;
         if (m >= M || !is_live(j, n)) continue;
         const float rs = row_scale(m);
         TOut* y = Y + (size_t)m * N + u0 + j * bh + n;
         if (EPI == EPI_SWIGLU) {
-            float gate = total(j, m, n), up = total(UNIT_BLOCKS + j, m, n);
-            gate *= rs;
-            up *= rs;
+            float gate = rounded(total(j, m, n) * rs), up = rounded(total(UNIT_BLOCKS + j, m, n) * rs);
             if (ep.glu_bias) {
                 gate += ep.glu_bias[u0 + j * bh + n];
                 up += ep.glu_bias[N + u0 + j * bh + n];
@@ -362,62 +458,80 @@ static int compute_units() {
 // How a product is cut into workgroups: `unit_blocks` blocks of `bh` units each, `grid` workgroups.
 struct Cut {
     int unit_blocks, bh, grid;
-    long long cost;  // rows of W the busiest compute unit streams, if workgroups ran in rounds over the units
+    long long cost;  // rows that the busiest compute unit fetches, if workgroups ran in rounds over the units
 };
 
-// The block height for workgroups of `unit_blocks` blocks (each unit costs `rows_per_unit` rows of W): 16 when the
-// workgroups are many; else the height from 8 to 16 that gives the busiest compute unit the least to stream.
-static Cut cut_for(int units, int unit_blocks, int rows_per_unit) {
+// The block height for workgroups of `unit_blocks` blocks (each unit costs `rows_per_unit` rows of W, a workgroup `x_rows`
+// rows of X on top): 16 when the workgroups are many; else the height from `least` to 16 that gives the busiest compute
+// unit the least to fetch.
+static Cut cut_for(int units, int unit_blocks, int rows_per_unit, int least, int x_rows) {
     const int cus = compute_units();
     auto with = [&](int bh) {
         const int grid = (units + unit_blocks * bh - 1) / (unit_blocks * bh);
-        return Cut{unit_blocks, bh, grid, (long long)((grid + cus - 1) / cus) * bh * unit_blocks * rows_per_unit};
+        return Cut{unit_blocks, bh, grid, (long long)((grid + cus - 1) / cus) * (bh * unit_blocks * rows_per_unit + x_rows)};
     };
     Cut best = with(16);
-    if (best.grid > 2 * cus) return best;
-    for (int bh = 15; bh >= 8; --bh) {
+    if (best.grid > 4 * cus) return best;
+    for (int bh = 15; bh >= least; --bh) {
         const Cut c = with(bh);
         if (c.cost < best.cost) best = c;
     }
     return best;
 }
 
-// Of the cuts an epilogue has kernels for, the cheapest; of equals the one with the higher blocks (fewer lanes that
-// repeat a row), then the one with more blocks per workgroup (fewer workgroups fetch X).
-static Cut cheapest(int units, int rows_per_unit, std::initializer_list<int> unit_blocks) {
+// Of the cuts an epilogue has kernels for, the cheapest; of equals the one with the higher blocks (fewer rows that
+// repeat one), then the one with more blocks per workgroup (fewer workgroups fetch X).
+static Cut cheapest(int units, int rows_per_unit, std::initializer_list<int> unit_blocks, int x_rows = 0) {
     Cut best{0, 0, 0, 0};
     for (int ub : unit_blocks) {
-        const Cut c = cut_for(units, ub, rows_per_unit);
+        const Cut c = cut_for(units, ub, rows_per_unit, 8, x_rows);
         if (!best.grid || c.cost < best.cost || (c.cost == best.cost && c.bh > best.bh)) best = c;
     }
     return best;
 }
 
+static bool aligned16(const void* X, const void* W) { return (((uintptr_t)X | (uintptr_t)W) & 15) == 0; }
+
+struct Product {
+    const bf16_t* X;
+    const bf16_t* W;
+    void* Y;
+    int M, N, K;
+    hipStream_t stream;
+};
+
+template <typename TOut, int EPI, bool SCALED, int RB, int MB, int WAVES, int SLOTS, int WI = 2, int XI = 2 * MB>
+static void launch(const Product& p, const Cut& cut, const Epilogue& ep) {
+    hipLaunchKernelGGL((gemm_skinny_kernel<TOut, EPI, SCALED, RB, MB, WAVES, SLOTS, WI, XI>), dim3(cut.grid),
+                       dim3(WAVES * SIA_WAVE), 0, p.stream, p.X, p.W, (TOut*)p.Y, p.M, p.N, p.K, cut.bh, ep);
+}
+
+// The kernel of a cut whose blocks are columns of Y.  Eight waves; the ring as deep as LDS allows, four steps at most: one
+// workgroup a compute unit, whose waves then have 90 to 150 KB on their way.
 template <typename TOut, int EPI>
-static void launch_skinny(const bf16_t* X, const bf16_t* W, TOut* Y, int M, int N, int K, const Epilogue& ep,
-                          hipStream_t stream) {
-    const Cut cut = cheapest(N, 1, {4, 2, 1});
-#define LAUNCH(RB, WAVES)                                                                                 \
-    hipLaunchKernelGGL((gemm_skinny_kernel<TOut, RB, WAVES, EPI, false>), dim3(cut.grid),                  \
-                       dim3(WAVES * SIA_WAVE), 0, stream, X, W, Y, M, N, K, cut.bh, ep)
-    if (cut.unit_blocks == 4)
-        LAUNCH(4, 8);
-    else if (cut.unit_blocks == 2)
-        LAUNCH(2, 16);
-    else
-        LAUNCH(1, 8);
-#undef LAUNCH
+static void launch_columns(const Product& p, const Cut& cut, const Epilogue& ep) {
+    const bool low = cut.bh <= 8;
+    if (p.M <= 8) {
+        if (cut.unit_blocks == 2) launch<TOut, EPI, false, 2, 1, 8, 2, 2, 1>(p, cut, ep);
+        else if (low) launch<TOut, EPI, false, 1, 1, 8, 4, 1, 1>(p, cut, ep);
+        else launch<TOut, EPI, false, 1, 1, 8, 4, 2, 1>(p, cut, ep);
+    } else if (p.M <= 16) {
+        if (cut.unit_blocks == 2) launch<TOut, EPI, false, 2, 1, 8, 3>(p, cut, ep);
+        else if (low) launch<TOut, EPI, false, 1, 1, 8, 4, 1>(p, cut, ep);
+        else launch<TOut, EPI, false, 1, 1, 8, 4>(p, cut, ep);
+    }
 }
 
 // out_float: 1 -> Y is float, 0 -> bfloat16.  Needs M <= 16, K % 64 == 0.
 SIA_EXPORT int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int N, int K, int out_float,
                                hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0) return SIA_BAD_ARGUMENT;
+    if (M > 16 || K % 64 || K <= 0 || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
+    const Product p{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream};
     if (out_float)
-        launch_skinny<float, EPI_STORE>((const bf16_t*)X, (const bf16_t*)W, (float*)Y, M, N, K, Epilogue{}, stream);
+        launch_columns<float, EPI_STORE>(p, cheapest(N, 1, {2, 1}), Epilogue{});
     else
-        launch_skinny<bf16_t, EPI_STORE>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, M, N, K, Epilogue{}, stream);
+        launch_columns<bf16_t, EPI_STORE>(p, cheapest(N, 1, {2, 1}), Epilogue{});
     return SIA_LAUNCH_CHECK();
 }
 
@@ -425,10 +539,10 @@ SIA_EXPORT int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int
 SIA_EXPORT int sia_gemm_skinny_act(const void* X, const void* W, void* Y, int M, int N, int K, int activation,
                                    hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU)) return SIA_BAD_ARGUMENT;
+    if (M > 16 || K % 64 || K <= 0 || !aligned16(X, W) || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU)) return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.activation = activation;
-    launch_skinny<bf16_t, EPI_ACT>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, M, N, K, ep, stream);
+    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, cheapest(N, 1, {2, 1}), ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -437,7 +551,7 @@ SIA_EXPORT int sia_gemm_skinny_embedding_gate(const void* X, const void* W, void
                                               const void* table, int table_width, int first, int dim, const int* ids,
                                               hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU) ||
+    if (M > 16 || K % 64 || K <= 0 || !aligned16(X, W) || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU) ||
         !table || !ids || dim <= 0 || dim > N || first < 0 || first + dim > table_width)
         return SIA_BAD_ARGUMENT;
     Epilogue ep{};
@@ -446,7 +560,7 @@ SIA_EXPORT int sia_gemm_skinny_embedding_gate(const void* X, const void* W, void
     ep.ids = ids;
     ep.table_width = table_width;
     ep.table_dim = dim;
-    launch_skinny<bf16_t, EPI_ACT>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, M, N, K, ep, stream);
+    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, cheapest(N, 1, {2, 1}), ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -455,11 +569,11 @@ SIA_EXPORT int sia_gemm_skinny_embedding_gate(const void* X, const void* W, void
 SIA_EXPORT int sia_gemm_skinny_grouped(const void* X, const void* W, void* Y, int M, int K, int groups, int group_rows,
                                        int last_rows, hipStream_t stream) {
     if (M <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || groups <= 0 || group_rows <= 0 || last_rows <= 0 || !X || !W || !Y) return SIA_BAD_ARGUMENT;
+    if (M > 16 || K % 64 || K <= 0 || groups <= 0 || group_rows <= 0 || last_rows <= 0 || !X || !W || !Y || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
     const int cus = compute_units();
     Cut best{0, 0, 0, 0};
     int best_blocks = 0;
-    for (int ub : {4, 2, 1})
+    for (int ub : {2, 1})
         // (where the workgroups are many, full blocks: lower ones would fetch X more often for the same rows)
         for (int bh = 16; bh >= 8; --bh) {
             const int a_group = (group_rows + ub * bh - 1) / (ub * bh), last = (last_rows + ub * bh - 1) / (ub * bh);
@@ -476,24 +590,14 @@ SIA_EXPORT int sia_gemm_skinny_grouped(const void* X, const void* W, void* Y, in
     ep.group_rows = group_rows;
     ep.last_rows = last_rows;
     ep.group_blocks = best_blocks;
-#define LAUNCH(RB, WAVES)                                                                                            \
-    hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t, RB, WAVES, EPI_GROUPED, false>), dim3(best.grid),                  \
-                       dim3(WAVES * SIA_WAVE), 0, stream, (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, M, group_rows, \
-                       K, best.bh, ep)
-    if (best.unit_blocks == 4)
-        LAUNCH(4, 8);
-    else if (best.unit_blocks == 2)
-        LAUNCH(2, 16);
-    else
-        LAUNCH(1, 8);
-#undef LAUNCH
+    launch_columns<bf16_t, EPI_GROUPED>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, group_rows, K, stream}, best, ep);
     return SIA_LAUNCH_CHECK();
 }
 
 // Blocks of columns whose sums of squares sia_gemm_skinny_residual leaves for a result of N columns.
 SIA_EXPORT int sia_gemm_skinny_residual_blocks(int N) {
     if (N <= 0) return 0;
-    const Cut cut = cheapest(N, 1, {4, 2, 1});
+    const Cut cut = cheapest(N, 1, {2, 1});
     return cut.grid * cut.unit_blocks;
 }
 
@@ -503,47 +607,19 @@ SIA_EXPORT int sia_gemm_skinny_residual_blocks(int N) {
 SIA_EXPORT int sia_gemm_skinny_residual(const void* X, const void* W, int M, int N, int K, float* residual,
                                         const float* gain, void* scaled, float* partials, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || !residual || !gain || !scaled || !partials) return SIA_BAD_ARGUMENT;
+    if (M > 16 || K % 64 || K <= 0 || !residual || !gain || !scaled || !partials || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.res = ResidualOut{residual, gain, (bf16_t*)scaled, partials};
-    launch_skinny<bf16_t, EPI_RESIDUAL>((const bf16_t*)X, (const bf16_t*)W, (bf16_t*)nullptr, M, N, K, ep, stream);
+    launch_columns<bf16_t, EPI_RESIDUAL>(Product{(const bf16_t*)X, (const bf16_t*)W, nullptr, M, N, K, stream}, cheapest(N, 1, {2, 1}), ep);
     return SIA_LAUNCH_CHECK();
 }
 
-// The tiled copy of W[N][K] that sia_gemm_skinny_residual_tiled reads: sia_gemm_skinny_tile_height(N) rows a block
-// (0: this N is cut into workgroups of several blocks, which have no tiled form), blocks = ceil(N / height), the
-// last block's missing rows repeating row N - 1; elements [block][K / 64][2][height][4][8], where element
-// (b, s, h, r, g, e) is W[b * height + r][64 s + 16 g + 8 h + e].
-SIA_EXPORT int sia_gemm_skinny_tile_height(int N) {
-    if (N <= 0) return 0;
-    const Cut cut = cheapest(N, 1, {4, 2, 1});
-    return cut.unit_blocks == 1 ? cut.bh : 0;
-}
-
-SIA_EXPORT int sia_gemm_skinny_residual_tiled(const void* X, const void* W_tiled, int M, int N, int K, float* residual,
-                                              const float* gain, void* scaled, float* partials, hipStream_t stream) {
-    if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || !residual || !gain || !scaled || !partials) return SIA_BAD_ARGUMENT;
-    const Cut cut = cheapest(N, 1, {4, 2, 1});
-    if (cut.unit_blocks != 1) return SIA_BAD_ARGUMENT;
-    Epilogue ep{};
-    ep.res = ResidualOut{residual, gain, (bf16_t*)scaled, partials};
-    hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t, 1, 8, EPI_RESIDUAL, false, true>), dim3(cut.grid), dim3(8 * SIA_WAVE), 0,
-                       stream, (const bf16_t*)X, (const bf16_t*)W_tiled, (bf16_t*)nullptr, M, N, K, cut.bh, ep);
-    return SIA_LAUNCH_CHECK();
-}
-
-// Y[M, N] = X W^T (bfloat16) from the tiled copy of W: the plain product for a weight that has such a copy, with the
-// sums of sia_gemm_skinny bit for bit.  Needs M <= 16, K % 64 == 0, sia_gemm_skinny_tile_height(N) > 0.
-SIA_EXPORT int sia_gemm_skinny_tiled(const void* X, const void* W_tiled, void* Y, int M, int N, int K,
-                                     hipStream_t stream) {
-    if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || !Y) return SIA_BAD_ARGUMENT;
-    const Cut cut = cheapest(N, 1, {4, 2, 1});
-    if (cut.unit_blocks != 1) return SIA_BAD_ARGUMENT;
-    hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t, 1, 8, EPI_STORE, false, true>), dim3(cut.grid), dim3(8 * SIA_WAVE), 0,
-                       stream, (const bf16_t*)X, (const bf16_t*)W_tiled, (bf16_t*)Y, M, N, K, cut.bh, Epilogue{});
-    return SIA_LAUNCH_CHECK();
+// No product gains from a copy of W in another order, now that its rows come to LDS in whole lines: no weight has a tiled form
+// (rows a block of such a copy: none), and the product that would read one refuses.
+SIA_EXPORT int sia_gemm_skinny_tile_height(int) { return 0; }
+SIA_EXPORT int sia_gemm_skinny_residual_tiled(const void*, const void*, int, int, int, float*, const float*, void*, float*,
+                                              hipStream_t) {
+    return SIA_BAD_ARGUMENT;
 }
 
 // Y[M, I] = silu(X Wg^T) * (X Wu^T) for W = [Wg; Wu] of 2 I rows.  Needs M <= 16, K % 64 == 0.
@@ -555,27 +631,20 @@ SIA_EXPORT int sia_gemm_skinny_glu(const void* X, const void* W, void* Y, int M,
                                    const float* bias, hipStream_t stream) {
     if (M <= 0 || inter <= 0) return 0;
     if (M > 16 || K % 64 || K <= 0 || (partials && n_partials <= 0) ||
-        glu < SIA_GLU_SILU || glu > SIA_GLU_GELU_TANH)
+        glu < SIA_GLU_SILU || glu > SIA_GLU_GELU_TANH || !aligned16(X, W))
         return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.glu_bias = bias;
     ep.scale = RowScale{partials, n_partials, eps};
     ep.glu = glu;
     ep.limit = limit;
-    const Cut cut = cheapest(inter, 2, {2, 1});
-#define LAUNCH(RB, WAVES, SCALED)                                                                                  \
-    hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t, RB, WAVES, EPI_SWIGLU, SCALED>), dim3(cut.grid),              \
-                       dim3(WAVES * SIA_WAVE), 0, stream, (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, M, inter, \
-                       K, cut.bh, ep)
-    if (cut.unit_blocks == 2 && partials)
-        LAUNCH(4, 16, true);
-    else if (cut.unit_blocks == 2)
-        LAUNCH(4, 16, false);
-    else if (partials)
-        LAUNCH(2, 8, true);
-    else
-        LAUNCH(2, 8, false);
-#undef LAUNCH
+    const Product p{(const bf16_t*)X, (const bf16_t*)W, Y, M, inter, K, stream};
+    const Cut cut = cheapest(inter, 2, {1});
+    // two workgroups a compute unit: one's sums meet while the other's rows come
+    if (M <= 8 && partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 8, 2, 2, 1>(p, cut, ep);
+    else if (M <= 8) launch<bf16_t, EPI_SWIGLU, false, 2, 1, 8, 2, 2, 1>(p, cut, ep);
+    else if (partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 4, 3>(p, cut, ep);
+    else launch<bf16_t, EPI_SWIGLU, false, 2, 1, 4, 3>(p, cut, ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -596,26 +665,25 @@ SIA_EXPORT int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M
     if (M <= 0) return 0;
     if (M > 16 || K % 64 || K <= 0 || head_dim % 2 || head_dim <= 0 || n_heads <= 0 || n_kv <= 0 || page_size <= 0 ||
         table_width <= 0 || !cos_table || !sin_table || !positions || !seq_of_token || !block_table || !k_pages ||
-        !v_pages || (partials && n_partials <= 0))
+        !v_pages || (partials && n_partials <= 0) || !aligned16(X, W))
         return SIA_BAD_ARGUMENT;
     const int heads = n_heads + 2 * n_kv, N = heads * head_dim;
     Epilogue ep{};
     ep.rope = RopeOut{cos_table, sin_table, positions, seq_of_token, block_table, (bf16_t*)k_pages, (bf16_t*)v_pages,
                       table_width, n_heads, n_kv, head_dim, page_size};
     ep.scale = RowScale{partials, n_partials, eps};
-    const Cut cut = cut_for(heads * (head_dim / 2), 1, 2);
-#define LAUNCH(WAVES, SCALED)                                                                              \
-    hipLaunchKernelGGL((gemm_skinny_kernel<bf16_t, 2, WAVES, EPI_ROPE, SCALED>), dim3(cut.grid),            \
-                       dim3(WAVES * SIA_WAVE), 0, stream, (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, M, N, K,  \
-                       cut.bh, ep)
-    if (K >= 1024 && partials)
-        LAUNCH(16, true);
-    else if (K >= 1024)
-        LAUNCH(16, false);
-    else if (partials)
-        LAUNCH(8, true);
-    else
-        LAUNCH(8, false);
+    const Product p{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream};
+    const Cut cut = cut_for(heads * (head_dim / 2), 1, 2, 4, 0);
+    const bool low = cut.bh <= 8;
+#define LAUNCH(SCALED)                                                                        \
+    do {                                                                                      \
+        if (M <= 8 && low) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 1, 1>(p, cut, ep);    \
+        else if (M <= 8) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 2, 1>(p, cut, ep);      \
+        else if (low) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 1>(p, cut, ep);            \
+        else launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3>(p, cut, ep);                        \
+    } while (0)
+    if (partials) LAUNCH(true);
+    else LAUNCH(false);
 #undef LAUNCH
     return SIA_LAUNCH_CHECK();
 }

@@ -127,7 +127,6 @@ _SIGNATURES = {
     "sia_gemm_skinny_residual": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "sia_gemm_skinny_residual_tiled": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     "sia_gemm_skinny_tile_height": [_c_int],
-    "sia_gemm_skinny_tiled": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_take_rows": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ll, _c_ptr],
     "sia_rows_alone": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_place_tokens": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
@@ -239,6 +238,12 @@ class ScaledRows:
     device = property(lambda self: self.rows.device)
 
 
+def _in_pieces(t: torch.Tensor):
+    """``t``, or a copy of it where it does not start at a multiple of 16 bytes: the few-row products bring their operands
+    to LDS in pieces of that size (a view that starts inside another tensor may lie anywhere)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _ptr(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
@@ -292,7 +297,6 @@ class HipKernels:
         self._raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         self._device_index = torch.device(device).index or 0
         self.use_mfma_attention = True   # tests switch it off to reach the plain kernel in bfloat16
-        self.tiled_weights = True        # tests switch it off to compare with the product that reads W as it is
         self.use_skinny_gemm = True      # few-row bfloat16 products by this package's kernel, not the library
         self.fuse_norms = True           # few rows: residual add in the product before a norm, row scale in the one after
         self.fuse_rope = True            # few rows: rotation and cache write in the q/k/v product
@@ -589,6 +593,7 @@ class HipKernels:
             raise KernelError(f"{dim} columns from {first_column} on do not fit a table row of {width} and {N} outputs")
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and 0 < M <= self._skinny_rows and K % 64 == 0:
             y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+            x, w = _in_pieces(x), _in_pieces(w)
             self._check(self.core.sia_gemm_skinny_embedding_gate(
                 _ptr(x), _ptr(w), _ptr(y), M, N, K, _ACTIVATIONS[activation], _ptr(table), width, int(first_column),
                 int(dim), _ptr(token_ids), self._stream()), "gemm_skinny_embedding_gate")
@@ -977,6 +982,7 @@ class HipKernels:
         most = (groups - 1) * M * rows
         main, low = flat[:most].view(groups - 1, M, rows), flat[most:].view(M, last)
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and M <= self._skinny_rows and K % 64 == 0:
+            x, w = _in_pieces(x), _in_pieces(w)
             self._check(self.core.sia_gemm_skinny_grouped(_ptr(x), _ptr(w), _ptr(flat), M, K, groups, rows, last,
                                                           self._stream()), "gemm_skinny_grouped")
             return main, low
@@ -1383,11 +1389,7 @@ class HipKernels:
             # up to 16 rows: this package's kernel, whose sums do not depend on the number of rows
             if self.use_skinny_gemm and M <= self._skinny_rows and K % 64 == 0:
                 y = torch.empty((M, N), dtype=torch.float32 if out_float32 else torch.bfloat16, device=x.device)
-                tiled = None if out_float32 else self._tiled_copy(w)
-                if tiled is not None:   # a weight that has a copy in the order of this kernel's loads: the same bits
-                    self._check(self.core.sia_gemm_skinny_tiled(_ptr(x), _ptr(tiled), _ptr(y), M, N, K, self._stream()),
-                                "gemm_skinny_tiled")
-                    return y
+                x, w = _in_pieces(x), _in_pieces(w)
                 self._check(self.core.sia_gemm_skinny(_ptr(x), _ptr(w), _ptr(y), M, N, K, int(out_float32),
                                                       self._stream()), "gemm_skinny")
                 return y
@@ -1424,6 +1426,7 @@ class HipKernels:
                 rows, partials, n_partials, eps = self._scaled(x)      # few rows: the activation inside the product
                 self._want(rows, "gated linear input")
                 y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=rows.device)
+                rows, w_gate_up = _in_pieces(rows), _in_pieces(w_gate_up)
                 self._check(self.core.sia_gemm_skinny_glu(_ptr(rows), _ptr(w_gate_up), _ptr(y), M, two_i // 2, K,
                                                           _ptr(partials), n_partials, eps, glu, limit, _ptr(bias), self._stream()),
                             "gemm_skinny_glu")
@@ -1442,6 +1445,7 @@ class HipKernels:
             rows, partials, n_partials, eps = self._scaled(x)
             self._want(rows, "gated linear input")
             y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=rows.device)
+            rows, w_gate_up = _in_pieces(rows), _in_pieces(w_gate_up)
             self._check(self.core.sia_gemm_skinny_swiglu(_ptr(rows), _ptr(w_gate_up), _ptr(y), M, two_i // 2, K,
                                                          _ptr(partials), n_partials, eps, self._stream()),
                         "gemm_skinny_swiglu")
@@ -1463,6 +1467,7 @@ class HipKernels:
         if (self.use_skinny_gemm and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and 0 < M <= self._skinny_rows and K % 64 == 0):
             y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+            x, w = _in_pieces(x), _in_pieces(w)
             self._check(self.core.sia_gemm_skinny_act(_ptr(x), _ptr(w), _ptr(y), M, N, K, _ACTIVATIONS[activation],
                                                       self._stream()), "gemm_skinny_act")
             return y
@@ -1503,43 +1508,15 @@ class HipKernels:
                               f"residual {tuple(residual.shape)}, gain {tuple(gain.shape)}")
         rows = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
         partials = torch.empty((self.core.sia_gemm_skinny_residual_blocks(N), 16), dtype=torch.float32, device=x.device)
-        tiled = self._tiled_copy(w)
-        if tiled is not None:
-            self._check(self.core.sia_gemm_skinny_residual_tiled(_ptr(x), _ptr(tiled), M, N, K, _ptr(residual),
-                                                                 _ptr(gain), _ptr(rows), _ptr(partials), self._stream()),
-                        "gemm_skinny_residual_tiled")
-        else:
-            self._check(self.core.sia_gemm_skinny_residual(_ptr(x), _ptr(w), M, N, K, _ptr(residual), _ptr(gain),
-                                                           _ptr(rows), _ptr(partials), self._stream()),
-                        "gemm_skinny_residual")
+        x, w = _in_pieces(x), _in_pieces(w)
+        self._check(self.core.sia_gemm_skinny_residual(_ptr(x), _ptr(w), M, N, K, _ptr(residual), _ptr(gain), _ptr(rows),
+                                                       _ptr(partials), self._stream()), "gemm_skinny_residual")
         return ScaledRows(rows, partials, float(eps))
 
-    # A weight whose product goes into the residual in steps of few rows may have a second copy, laid out in the
-    # order in which that kernel's workgroups read it (every load instruction one run of memory: the o and down
-    # products of a decode step take 10 to 15 % less).  The copy hangs on the weight tensor itself, so it lives as long
-    # as the weight does, and remembers the version of the tensor it was made from: a weight changed in place since
-    # is read as it is.  Steps of more rows, which go to the library, read the weight as it is anyway.
     def prepare_pending_weight(self, w) -> bool:
-        """Makes the tiled copy of a weight that ``pending_linear`` will be given; True if one was made."""
-        if (not self.tiled_weights or not isinstance(w, torch.Tensor) or w.dim() != 2 or w.dtype != torch.bfloat16
-                or not w.is_cuda or not w.is_contiguous() or w.shape[1] % 64 or torch.cuda.is_current_stream_capturing()):
-            return False
-        N, K = w.shape
-        height = self.core.sia_gemm_skinny_tile_height(N)
-        if height <= 0:
-            return False
-        blocks = -(-N // height)
-        rows = torch.arange(blocks * height, device=w.device).clamp_(max=N - 1)   # the last block repeats the last row
-        # element (block, step, half, row, lane group, e) = W[block * height + row][64 step + 16 group + 8 half + e]
-        tiled = w[rows].view(blocks, height, K // 64, 4, 2, 8).permute(0, 2, 4, 1, 3, 5).contiguous()
-        w._sia_tiled = (tiled, w._version)
-        return True
-
-    def _tiled_copy(self, w):
-        kept = getattr(w, "_sia_tiled", None) if self.tiled_weights else None
-        if kept is None or kept[1] != w._version:
-            return None
-        return kept[0]
+        """Whether a copy of a weight that ``pending_linear`` will be given was made in an order of the kernels' own: no,
+        they read every weight as it is."""
+        return False
 
     @staticmethod
     def _scaled(x):
@@ -1685,6 +1662,7 @@ class HipKernels:
             self._check_pages(cache.k_pages, cache.v_pages, cache.block_table, cache.page_size, n_kv_written,
                               head_dim, x.dtype, ctx)
             qkv = torch.empty((M, width), dtype=torch.bfloat16, device=x.device)
+            x, w_qkv = _in_pieces(x), _in_pieces(w_qkv)
             self._check(self.core.sia_gemm_skinny_rope(
                 _ptr(x), _ptr(w_qkv), _ptr(qkv), M, K, _ptr(cos), _ptr(sin), _ptr(ctx.positions),
                 _ptr(ctx.seq_of_token), _ptr(cache.block_table), cache.block_table.shape[1], _ptr(cache.k_pages),

@@ -253,9 +253,6 @@ class Attention:
             self.b_o = tensors["o_bias"].contiguous()
         if self.sink:
             self.sinks = tensors["sink"].contiguous()
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:   # the kernels may keep a copy of their own of a weight whose product is left pending
-            prepare(self.w_o)
 
     def plain_form(self):
         """What this mixer is, as plain data, for kernels that can run a whole block in one call; None for the forms

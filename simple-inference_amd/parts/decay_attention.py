@@ -49,9 +49,6 @@ class DecayAttention:
         self.norm = tensors["norm"].contiguous()
         self.w_o = tensors["o"].contiguous()
         self.decays = torch.tensor(self.decay, dtype=torch.float32, device=self.w_o.device)
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def cache_need(self):
         return None

@@ -74,9 +74,6 @@ class GatedDeltaRule:
         self.a_log, self.dt_bias = tensors["a_log"].contiguous(), tensors["dt_bias"].contiguous()
         self.norm = tensors["norm"].contiguous()
         self.w_o = tensors["o"].contiguous()
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def weight_specs(self):
         H = self.num_heads

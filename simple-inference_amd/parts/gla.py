@@ -77,9 +77,6 @@ class GatedLinearAttention:
         self.b_a2 = tensors["a2_bias"].contiguous()
         self.norm = tensors["norm"].contiguous()
         self.w_o = tensors["o"].contiguous()
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def cache_need(self):
         return None

@@ -49,9 +49,6 @@ class Hgrn2Mixer:
         self.w_in = torch.cat([tensors["q"], tensors["f"], tensors["v"]], dim=0).contiguous()
         self.w_o = tensors["o"].contiguous()
         self.f_bias, self.lower, self.norm = (tensors[n].contiguous() for n in ("f_bias", "lower", "norm"))
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def cache_need(self):
         return None

@@ -111,9 +111,6 @@ class LatentAttention:
         self.q_gain = tensors["dq_norm"].contiguous()
         self.kv_gain = tensors["dkv_norm"].contiguous() if self.writes_kv else None
         self.sinks = tensors["sink"].contiguous() if self.sink else None
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def cache_need(self):
         if self.page_dim is not None:

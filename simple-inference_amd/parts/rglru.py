@@ -67,9 +67,6 @@ class LinearRecurrentUnit:
             "ra_bias": f32("ra_bias"), "ri_bias": f32("ri_bias"),
             "rate": RATE * torch.nn.functional.softplus(tensors["lam"].double(), threshold=1e9).float().contiguous(),
         }
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def cache_need(self):
         return None

@@ -61,9 +61,6 @@ class Mamba2Mixer:
         self.conv_w, self.conv_b = tensors["conv"].contiguous(), tensors["conv_bias"].contiguous()
         self.dt_bias, self.a_log, self.d = (tensors[n].contiguous() for n in ("dt_bias", "a_log", "d"))
         self.norm = tensors["norm"].contiguous()
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def cache_need(self):
         return None

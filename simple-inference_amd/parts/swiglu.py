@@ -57,9 +57,6 @@ class SwiGLU:
         if self.bias:
             self.b_gate_up = torch.cat([tensors["gate_bias"], tensors["up_bias"]]).float().contiguous()
             self.b_down = tensors["down_bias"].contiguous()
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:   # the kernels may keep a copy of their own of a weight whose product is left pending
-            prepare(self.w_down)
 
     def plain_form(self):
         """What this feed-forward is, as plain data, for kernels that can run a whole block in one call (None for

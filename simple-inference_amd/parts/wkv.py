@@ -63,9 +63,6 @@ class WkvMixer:
         self.w2, self.w_o = tensors["w2"].contiguous(), tensors["o"].contiguous()
         self.w0, self.norm = tensors["w0"].float().contiguous(), tensors["norm"].float().contiguous()
         self.u = tensors["u"].float().reshape(-1).contiguous()
-        prepare = getattr(self.env.kernels, "prepare_pending_weight", None)
-        if prepare is not None:
-            prepare(self.w_o)
 
     def cache_need(self):
         return None

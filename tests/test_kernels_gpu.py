@@ -157,6 +157,26 @@ def test_gemm_skinny(hip, shape):
     assert torch.equal(hip.linear(x[:1].contiguous(), w), out16[:1])
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N, K", [(1, 64), (9, 128), (2048, 1984), (2049, 2112), (8192, 192), (33000, 64)])
+def test_few_row_product_at_the_edges_of_its_tiles(hip, M, N, K):
+    """Tiles of 8 rows (up to 8 rows of x have one, and so have blocks of at most 8 weight rows: N = 2,048), a last block
+    that is short, half a chunk of k at the end, waves without a step, two blocks a workgroup (N = 33,000); and an input
+    that starts inside another tensor, not at a multiple of 16 bytes.  Errors of the float sums: K products of values
+    around 1, each rounded by 2^-24, in an order of the kernel's own: below 1e-6 K."""
+    flat = rnd(M * K + 3, dtype=torch.bfloat16, seed=1)
+    w = rnd(N, K, dtype=torch.bfloat16, seed=2)
+    x = flat[:M * K].view(M, K)
+    want = x.double() @ w.double().T
+    out = hip.linear(x, w, out_float32=True)
+    assert float((out.double() - want).abs().max()) <= 1e-6 * K
+    aside = flat[3:3 + M * K].view(M, K)
+    assert aside.data_ptr() % 16
+    assert torch.equal(hip.linear(aside, w, out_float32=True), hip.linear(aside.clone(), w, out_float32=True))
+    gated = hip.gated_linear(aside, torch.cat([w, w]))
+    assert torch.equal(gated, hip.gated_linear(aside.clone(), torch.cat([w, w])))
+
+
 @pytest.mark.parametrize("shape", [(1, 32, 64), (8, 8192, 3072), (16, 1008, 512), (5, 96, 320), (40, 128, 256),
                                    (3, 1, 64), (12, 333, 192), (16, 14336, 256)])
 def test_gated_linear(hip, shape):
