@@ -1,6 +1,7 @@
 // One pre-norm block (attention with rotation over the paged cache, SwiGLU feed-forward, RMS norms) of a step of
 // many rows, as one call: the launches that the parts' own calls would make one by one, in the same order, on the
-// same buffers.  Nothing is computed here; it spares the host the way through the interpreter between the launches,
+// same buffers.  In steps of up to 64 rows the rotation with the cache write and the activation are epilogues of this package's
+// products, which round first and give the bits of the kernels that they replace.  Nothing is computed here; it spares the host the way through the interpreter between the launches,
 // which in a step of a few hundred tokens of a small model takes longer than the GPU needs for them.  The matrix
 // products and the matrix-core attention live in other libraries: the caller hands their entry points in.
 #include "common.h"
@@ -13,6 +14,14 @@ int sia_rope_kv_write(void* qkv, int row_stride, const float* cos_table, const f
                       const int* seq_of_token, const int* block_table, int table_width, void* k_pages, void* v_pages,
                       int n_tokens, int n_heads, int n_kv, int head_dim, int rotary_dim, int page_size, int dtype,
                       hipStream_t stream);
+int sia_gemm_skinny_takes(int M, int N, int K);
+int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int N, int K, int out_float, hipStream_t stream);
+int sia_gemm_skinny_swiglu(const void* X, const void* W, void* Y, int M, int inter, int K, const float* partials,
+                           int n_partials, float eps, hipStream_t stream);
+int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M, int K, const float* cos_table, const float* sin_table,
+                         const int* positions, const int* seq_of_token, const int* block_table, int table_width,
+                         void* k_pages, void* v_pages, int n_heads, int n_kv, int head_dim, int page_size,
+                         const float* partials, int n_partials, float eps, hipStream_t stream);
 }
 
 typedef int (*ProductFn)(const void* X, const void* W, void* Y, int M, int N, int K, int out_float, hipStream_t stream);
@@ -61,7 +70,14 @@ struct SiaBlockStep {
     float* ws_acc;
     float* ws_ml;
     int n_tokens, n_seqs, n_single, max_splits, n_tiles, n_tiles_split, n_tiles_long, q_bound, kv_bound;
+    int own_products;         // whether products that this package's kernels take go to them, not all to `product`
 };
+
+// Y = X W^T by whoever takes a product of this size.
+static int block_product(const SiaBlockStep* S, const void* X, const void* W, void* Y, int N, int K, hipStream_t stream) {
+    if (S->own_products && sia_gemm_skinny_takes(S->n_tokens, N, K)) return sia_gemm_skinny(X, W, Y, S->n_tokens, N, K, 0, stream);
+    return S->product(X, W, Y, S->n_tokens, N, K, 0, stream);
+}
 
 #define SIA_STEP(call)             \
     do {                           \
@@ -80,10 +96,16 @@ SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, co
     const int qkv_width = (B->n_heads + 2 * B->n_kv) * B->head_dim;
     SIA_STEP(sia_add_rmsnorm(S->residual, delta, B->mixer_norm_gain, S->normed, nullptr, M, H, B->mixer_norm_eps,
                              SIA_BF16, stream));
-    SIA_STEP(S->product(S->normed, B->w_qkv, S->qkv, M, qkv_width, H, 0, stream));
-    SIA_STEP(sia_rope_kv_write(S->qkv, qkv_width, B->cos_table, B->sin_table, S->positions, S->seq_of_token,
-                               block_table, table_width, k_pages, v_pages, M, B->n_heads, B->n_kv, B->head_dim,
-                               B->rotary_dim, page_size, SIA_BF16, stream));
+    if (S->own_products && B->rotary_dim == B->head_dim && B->head_dim % 2 == 0 && sia_gemm_skinny_takes(M, qkv_width, H)) {
+        SIA_STEP(sia_gemm_skinny_rope(S->normed, B->w_qkv, S->qkv, M, H, B->cos_table, B->sin_table, S->positions,
+                                      S->seq_of_token, block_table, table_width, k_pages, v_pages, B->n_heads, B->n_kv,
+                                      B->head_dim, page_size, nullptr, 0, 0.f, stream));
+    } else {
+        SIA_STEP(block_product(S, S->normed, B->w_qkv, S->qkv, qkv_width, H, stream));
+        SIA_STEP(sia_rope_kv_write(S->qkv, qkv_width, B->cos_table, B->sin_table, S->positions, S->seq_of_token,
+                                   block_table, table_width, k_pages, v_pages, M, B->n_heads, B->n_kv, B->head_dim,
+                                   B->rotary_dim, page_size, SIA_BF16, stream));
+    }
     if (!attend) return 0;
     if (S->n_single > 0) {
         if (!S->attend_single) return SIA_BAD_ARGUMENT;
@@ -103,11 +125,15 @@ SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, co
                                  int table_width, void* k_pages, void* v_pages, int page_size, hipStream_t stream) {
     SIA_STEP(sia_prenorm_mixer(B, S, delta, block_table, table_width, k_pages, v_pages, page_size, 1, stream));
     const int M = S->n_tokens, H = B->hidden, Q = B->n_heads * B->head_dim;
-    SIA_STEP(S->product(S->attended, B->w_o, S->mixed, M, H, Q, 0, stream));
+    SIA_STEP(block_product(S, S->attended, B->w_o, S->mixed, H, Q, stream));
     SIA_STEP(sia_add_rmsnorm(S->residual, S->mixed, B->feed_forward_norm_gain, S->normed, nullptr, M, H,
                              B->feed_forward_norm_eps, SIA_BF16, stream));
-    SIA_STEP(S->product(S->normed, B->w_gate_up, S->gate_up, M, 2 * B->inter, H, 0, stream));
-    SIA_STEP(sia_swiglu(S->gate_up, S->activated, M, B->inter, SIA_BF16, stream));
-    SIA_STEP(S->product(S->activated, B->w_down, S->fed, M, H, B->inter, 0, stream));
+    if (S->own_products && M <= 64 && H % 64 == 0) {
+        SIA_STEP(sia_gemm_skinny_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, nullptr, 0, 0.f, stream));
+    } else {
+        SIA_STEP(S->product(S->normed, B->w_gate_up, S->gate_up, M, 2 * B->inter, H, 0, stream));
+        SIA_STEP(sia_swiglu(S->gate_up, S->activated, M, B->inter, SIA_BF16, stream));
+    }
+    SIA_STEP(block_product(S, S->activated, B->w_down, S->fed, H, B->inter, stream));
     return 0;
 }

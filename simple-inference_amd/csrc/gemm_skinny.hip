@@ -365,7 +365,8 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
             b = rounded(b * rs);
             if (!is_v) {
                 const float c = rope_cos[it], sn = rope_sin[it];
-                const float ra = a * c - b * sn, rb_ = b * c + a * sn;
+                float ra = a * c - b * sn, rb_ = b * c + a * sn;
+                if (ROUND_FIRST) rotate_pair(a, b, c, sn, ra, rb_);
                 a = ra;
                 b = rb_;
             }
@@ -441,7 +442,20 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     }
 }
 
+// The rows up to which every epilogue has a kernel; EPI_STORE, EPI_SWIGLU and EPI_ROPE go up to SK_MAX_ROWS.
 SIA_EXPORT int sia_gemm_skinny_max_rows() { return 16; }
+SIA_EXPORT int sia_gemm_skinny_most_rows() { return SK_MAX_ROWS; }
+
+// Whether a product goes to this file's kernels rather than to the BLAS library.  Up to 32 rows all do; beyond, X's rows weigh
+// as much as W's in what a workgroup fetches, and the library is ahead where the columns are many or k is long.  us, own
+// against the library's best candidate:  27 rows 2,048 x 2,048 4.5 / 8.4, 5,120 x 3,072 11.1 / 12.4, 3,072 x 8,192 16.8 / 16.8,
+// 4,096 x 14,336 33 / 30, 12,288 x 3,072 17.8 / 18.1, 128,256 x 3,072 160 / 165;  45 rows 2,048 x 2,048 5.8 / 8.7, 2,048 x 8,192 16.3 / 15.2,
+// 3,072 x 8,192 19.1 / 22.0, 9,216 x 3,072 18.5 / 20.6, 12,288 x 3,072 21.0 / 20.4;  64 rows 3,072 x 3,072 11.4 / 16.2, 3,072 x 8,192 22.4 / 23.7,
+// 8,192 x 2,048 13.6 / 14.0, 4,096 x 14,336 43 / 40, 16,384 x 3,072 26.7 / 23.9, 128,256 x 3,072 195 / 186.
+SIA_EXPORT int sia_gemm_skinny_takes(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 64 || M > SK_MAX_ROWS) return 0;
+    return M <= 32 || (N <= 10240 && (M <= 48 || K <= 8192));
+}
 
 // Compute units of the current device (asked once per device).
 static int compute_units() {
@@ -507,7 +521,7 @@ static void launch(const Product& p, const Cut& cut, const Epilogue& ep) {
 }
 
 // The kernel of a cut whose blocks are columns of Y.  Eight waves; the ring as deep as LDS allows, four steps at most: one
-// workgroup a compute unit, whose waves then have 90 to 150 KB on their way.
+// workgroup a compute unit, whose waves then have 90 to 160 KB on their way.
 template <typename TOut, int EPI>
 static void launch_columns(const Product& p, const Cut& cut, const Epilogue& ep) {
     const bool low = cut.bh <= 8;
@@ -522,16 +536,36 @@ static void launch_columns(const Product& p, const Cut& cut, const Epilogue& ep)
     }
 }
 
-// out_float: 1 -> Y is float, 0 -> bfloat16.  Needs M <= 16, K % 64 == 0.
+// 17 to 64 rows: the same, and four blocks a workgroup where the columns are many.
+template <typename TOut, int MB>
+static void launch_more_rows(const Product& p, const Cut& cut) {
+    constexpr int TWO = MB == 4 ? 1 : 2, ONE = MB == 2 ? 3 : 2;   // steps in the ring of two blocks, and of one
+    const Epilogue ep{};
+    if (cut.unit_blocks == 4) launch<TOut, EPI_STORE, false, 4, MB, 8, 1>(p, cut, ep);
+    else if (cut.unit_blocks == 2) launch<TOut, EPI_STORE, false, 2, MB, 8, TWO>(p, cut, ep);
+    else if (cut.bh <= 8) launch<TOut, EPI_STORE, false, 1, MB, 8, ONE, 1>(p, cut, ep);
+    else launch<TOut, EPI_STORE, false, 1, MB, 8, ONE>(p, cut, ep);
+}
+
+template <typename TOut> static void launch_store(const Product& p) {
+    if (p.M <= 16) return launch_columns<TOut, EPI_STORE>(p, cheapest(p.N, 1, {2, 1}), Epilogue{});
+    const int mb = (p.M + 15) / 16;
+    const Cut cut = cheapest(p.N, 1, {4, 2, 1}, mb * 16);
+    if (mb == 2) launch_more_rows<TOut, 2>(p, cut);
+    else if (mb == 3) launch_more_rows<TOut, 3>(p, cut);
+    else launch_more_rows<TOut, 4>(p, cut);
+}
+
+// out_float: 1 -> Y is float, 0 -> bfloat16.  Needs M <= 64, K % 64 == 0.
 SIA_EXPORT int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int N, int K, int out_float,
                                hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
+    if (M > SK_MAX_ROWS || K % 64 || K <= 0 || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
     const Product p{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream};
     if (out_float)
-        launch_columns<float, EPI_STORE>(p, cheapest(N, 1, {2, 1}), Epilogue{});
+        launch_store<float>(p);
     else
-        launch_columns<bf16_t, EPI_STORE>(p, cheapest(N, 1, {2, 1}), Epilogue{});
+        launch_store<bf16_t>(p);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -630,8 +664,8 @@ SIA_EXPORT int sia_gemm_skinny_glu(const void* X, const void* W, void* Y, int M,
                                    const float* partials, int n_partials, float eps, int glu, float limit,
                                    const float* bias, hipStream_t stream) {
     if (M <= 0 || inter <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || (partials && n_partials <= 0) ||
-        glu < SIA_GLU_SILU || glu > SIA_GLU_GELU_TANH || !aligned16(X, W))
+    if (M > SK_MAX_ROWS || (M > 16 && (partials || glu != SIA_GLU_SILU || bias)) || K % 64 || K <= 0 ||
+        (partials && n_partials <= 0) || glu < SIA_GLU_SILU || glu > SIA_GLU_GELU_TANH || !aligned16(X, W))
         return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.glu_bias = bias;
@@ -639,12 +673,26 @@ SIA_EXPORT int sia_gemm_skinny_glu(const void* X, const void* W, void* Y, int M,
     ep.glu = glu;
     ep.limit = limit;
     const Product p{(const bf16_t*)X, (const bf16_t*)W, Y, M, inter, K, stream};
-    const Cut cut = cheapest(inter, 2, {1});
-    // two workgroups a compute unit: one's sums meet while the other's rows come
-    if (M <= 8 && partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 8, 2, 2, 1>(p, cut, ep);
-    else if (M <= 8) launch<bf16_t, EPI_SWIGLU, false, 2, 1, 8, 2, 2, 1>(p, cut, ep);
-    else if (partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 4, 3>(p, cut, ep);
-    else launch<bf16_t, EPI_SWIGLU, false, 2, 1, 4, 3>(p, cut, ep);
+    if (M <= 16) {
+        // two workgroups a compute unit: one's sums meet while the other's rows come
+        const Cut cut = cheapest(inter, 2, {1});
+        if (M <= 8 && partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 8, 2, 2, 1>(p, cut, ep);
+        else if (M <= 8) launch<bf16_t, EPI_SWIGLU, false, 2, 1, 8, 2, 2, 1>(p, cut, ep);
+        else if (partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 4, 3>(p, cut, ep);
+        else launch<bf16_t, EPI_SWIGLU, false, 2, 1, 4, 3>(p, cut, ep);
+        return SIA_LAUNCH_CHECK();
+    }
+    // More rows: 64 rows of W a workgroup, against which X's weigh less; two workgroups of 32 where the rows are short and
+    // one's few steps would stand alone (8,192 x 2,048, 27 rows 18.0 -> 15.7 us, 45 18.2 -> 17.7, 64 19.4 -> 20.8; x 3,072 20.9 -> 21.6,
+    // 23.5 -> 25.0, 24.9 -> 29.4)
+    const int mb = (M + 15) / 16;
+    const bool wide = mb == 4 || K > 2048;
+    const Cut cut = cheapest(inter, 2, {wide ? 2 : 1}, mb * 16);
+    if (mb == 4) launch<bf16_t, EPI_SWIGLU, false, 4, 4, 8, 1>(p, cut, ep);
+    else if (mb == 3 && wide) launch<bf16_t, EPI_SWIGLU, false, 4, 3, 8, 1>(p, cut, ep);
+    else if (mb == 3) launch<bf16_t, EPI_SWIGLU, false, 2, 3, 4, 2>(p, cut, ep);
+    else if (wide) launch<bf16_t, EPI_SWIGLU, false, 4, 2, 8, 1>(p, cut, ep);
+    else launch<bf16_t, EPI_SWIGLU, false, 2, 2, 4, 2>(p, cut, ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -663,7 +711,7 @@ SIA_EXPORT int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M
                                     int n_heads, int n_kv, int head_dim, int page_size, const float* partials,
                                     int n_partials, float eps, hipStream_t stream) {
     if (M <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || head_dim % 2 || head_dim <= 0 || n_heads <= 0 || n_kv <= 0 || page_size <= 0 ||
+    if (M > SK_MAX_ROWS || (M > 16 && partials) || K % 64 || K <= 0 || head_dim % 2 || head_dim <= 0 || n_heads <= 0 || n_kv <= 0 || page_size <= 0 ||
         table_width <= 0 || !cos_table || !sin_table || !positions || !seq_of_token || !block_table || !k_pages ||
         !v_pages || (partials && n_partials <= 0) || !aligned16(X, W))
         return SIA_BAD_ARGUMENT;
@@ -675,6 +723,16 @@ SIA_EXPORT int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M
     const Product p{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream};
     const Cut cut = cut_for(heads * (head_dim / 2), 1, 2, 4, 0);
     const bool low = cut.bh <= 8;
+    if (M > 16) {
+        const int mb = (M + 15) / 16;
+        if (mb == 2 && low) launch<bf16_t, EPI_ROPE, false, 2, 2, 8, 2, 1>(p, cut, ep);
+        else if (mb == 2) launch<bf16_t, EPI_ROPE, false, 2, 2, 8, 2>(p, cut, ep);
+        else if (mb == 3 && low) launch<bf16_t, EPI_ROPE, false, 2, 3, 8, 2, 1>(p, cut, ep);
+        else if (mb == 3) launch<bf16_t, EPI_ROPE, false, 2, 3, 8, 2>(p, cut, ep);
+        else if (low) launch<bf16_t, EPI_ROPE, false, 2, 4, 8, 2, 1>(p, cut, ep);
+        else launch<bf16_t, EPI_ROPE, false, 2, 4, 8, 1>(p, cut, ep);
+        return SIA_LAUNCH_CHECK();
+    }
 #define LAUNCH(SCALED)                                                                        \
     do {                                                                                      \
         if (M <= 8 && low) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 1, 1>(p, cut, ep);    \

@@ -33,8 +33,10 @@ __global__ void rope_kv_write_kernel(T* __restrict__ qkv, int row_stride,
         T* x = row + h * head_dim;
         const float a = to_float(x[j]), b = to_float(x[j + half]);
         const float c = cs[j], s = sn[j];
-        x[j] = from_float<T>(a * c - b * s);
-        x[j + half] = from_float<T>(b * c + a * s);
+        float ra, rb;
+        rotate_pair(a, b, c, s, ra, rb);
+        x[j] = from_float<T>(ra);
+        x[j + half] = from_float<T>(rb);
     }
     if (n_kv == 0) return;
 
@@ -50,9 +52,11 @@ __global__ void rope_kv_write_kernel(T* __restrict__ qkv, int row_stride,
         const T* x = k_row + h * head_dim;
         float val;
         if (d < half) {
-            val = to_float(x[d]) * cs[d] - to_float(x[d + half]) * sn[d];
+            float other;
+            rotate_pair(to_float(x[d]), to_float(x[d + half]), cs[d], sn[d], val, other);
         } else if (d < rotary_dim) {
-            val = to_float(x[d]) * cs[d - half] + to_float(x[d - half]) * sn[d - half];
+            float other;
+            rotate_pair(to_float(x[d - half]), to_float(x[d]), cs[d - half], sn[d - half], other, val);
         } else {
             val = to_float(x[d]);
         }
@@ -103,10 +107,7 @@ __global__ void rope_kv_write_vec_kernel(T* __restrict__ qkv, int row_stride, co
             float a[8], b[8], c[8], s[8], ra[8], rb[8];
             va.get(a); vb.get(b); vc.get(c); vs.get(s);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                ra[i] = a[i] * c[i] - b[i] * s[i];
-                rb[i] = b[i] * c[i] + a[i] * s[i];
-            }
+            for (int i = 0; i < 8; ++i) rotate_pair(a[i], b[i], c[i], s[i], ra[i], rb[i]);
             va.set(ra);
             vb.set(rb);
             if (is_q) {

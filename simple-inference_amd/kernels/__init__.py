@@ -120,6 +120,8 @@ _SIGNATURES = {
     "sia_sample_static_init": [],
     "sia_gemm_skinny": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_skinny_max_rows": [],
+    "sia_gemm_skinny_most_rows": [],
+    "sia_gemm_skinny_takes": [_c_int, _c_int, _c_int],
     "sia_gemm_skinny_residual_blocks": [_c_int],
     "sia_gemm_skinny_swiglu": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_float, _c_ptr],
     "sia_gemm_skinny_rope": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int,
@@ -262,7 +264,7 @@ class _BlockStep(ctypes.Structure):
                                                "attended", "mixed", "gate_up", "activated", "fed", "positions",
                                                "seq_of_token", "cu_q", "kv_len", "ws_acc", "ws_ml")]
                 + [(n, ctypes.c_int) for n in ("n_tokens", "n_seqs", "n_single", "max_splits", "n_tiles", "n_tiles_split",
-                                               "n_tiles_long", "q_bound", "kv_bound")])
+                                               "n_tiles_long", "q_bound", "kv_bound", "own_products")])
 
 
 def _bind(lib, signatures):
@@ -302,7 +304,9 @@ class HipKernels:
         self.fuse_rope = True            # few rows: rotation and cache write in the q/k/v product
         self.whole_blocks = True         # many rows: a block's launches in one call (``prenorm_block``)
         self._products_known: Dict[tuple, bool] = {}
-        self._skinny_rows = self.core.sia_gemm_skinny_max_rows()
+        self._skinny_rows = self.core.sia_gemm_skinny_max_rows()      # all forms of the few-row products
+        self._skinny_most = self.core.sia_gemm_skinny_most_rows()     # the plain and the gated one
+        self._own_known: Dict[tuple, bool] = {}
         self.blas = self._load_blas()    # the BLAS library called directly; None: its products go through torch
 
     def _load_blas(self):
@@ -1386,8 +1390,8 @@ class HipKernels:
         M, K = x.shape
         N = w.shape[0]
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
-            # up to 16 rows: this package's kernel, whose sums do not depend on the number of rows
-            if self.use_skinny_gemm and M <= self._skinny_rows and K % 64 == 0:
+            # few rows: this package's kernel, whose sums do not depend on the number of rows
+            if self.use_skinny_gemm and (M <= self._skinny_rows and K % 64 == 0 or self._own_product(M, N, K)):
                 y = torch.empty((M, N), dtype=torch.float32 if out_float32 else torch.bfloat16, device=x.device)
                 x, w = _in_pieces(x), _in_pieces(w)
                 self._check(self.core.sia_gemm_skinny(_ptr(x), _ptr(w), _ptr(y), M, N, K, int(out_float32),
@@ -1441,7 +1445,7 @@ class HipKernels:
                                               _ptr(bias), _DT[gu.dtype], self._stream()), "glu")
             return out
         if (self.use_skinny_gemm and x.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16
-                and M <= self._skinny_rows and two_i % 2 == 0 and K % 64 == 0 and w_gate_up.shape[1] == K):
+                and M <= self._skinny_most and two_i % 2 == 0 and K % 64 == 0 and w_gate_up.shape[1] == K):
             rows, partials, n_partials, eps = self._scaled(x)
             self._want(rows, "gated linear input")
             y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=rows.device)
@@ -1951,6 +1955,16 @@ class HipKernels:
                 softcap, keep_first, self._stream()), "attn_prefill")
 
     # -- a whole block in one call -------------------------------------------------
+    def _own_product(self, M, N, K) -> bool:
+        """Whether a plain bfloat16 product of this size goes to this package's kernels (``sia_gemm_skinny_takes``)."""
+        if M > self._skinny_most:
+            return False
+        key = (M, N, K)
+        known = self._own_known.get(key)
+        if known is None:
+            known = self._own_known[key] = bool(self.core.sia_gemm_skinny_takes(M, N, K))
+        return known
+
     def _library_can(self, M, N, K) -> bool:
         key = (M, N, K)
         known = self._products_known.get(key)
@@ -1984,7 +1998,7 @@ class HipKernels:
             wanted += ((at["cos"], f32, None), (at["sin"], f32, None))
         for t, dtype, shape in wanted:
             if (not isinstance(t, torch.Tensor) or t.device.type != "cuda" or t.dtype != dtype or not t.is_contiguous()
-                    or (shape is not None and tuple(t.shape) != shape)):
+                    or (shape is not None and tuple(t.shape) != shape) or t.data_ptr() % 16):
                 return False
         if (ff["hidden"] != H or n1["size"] != H or n2["size"] != H or D % 16 or D > 256 or not at["scale"] > 0
                 or (rd and (at["cos"].shape[1] != rd // 2 or at["sin"].shape != at["cos"].shape))):
@@ -2023,7 +2037,8 @@ class HipKernels:
         fn = lambda f: ctypes.cast(f, ctypes.c_void_p).value
         step = _BlockStep(fn(self.blas.sia_blas_mm), fn(lib.sia_attn_decode), fn(lib.sia_attn_prefill), None,
                           *[_ptr(b) for b in buffers], _ptr(ctx.positions), _ptr(ctx.seq_of_token), _ptr(ctx.cu_q),
-                          _ptr(ctx.kv_len), _ptr(ws_acc), _ptr(ws_ml), M, ctx.n_seqs, n_dec, max_splits, *tiles)
+                          _ptr(ctx.kv_len), _ptr(ws_acc), _ptr(ws_ml), M, ctx.n_seqs, n_dec, max_splits, *tiles,
+                          int(self.use_skinny_gemm))
         steps[key] = (step, buffers)
         return steps[key]
 

@@ -191,6 +191,49 @@ def test_gated_linear(hip, shape):
     torch.testing.assert_close(out.double(), ref, rtol=2e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("heads, kv, D, K", [(3, 1, 32, 192), (24, 8, 128, 320), (32, 8, 64, 2048), (5, 5, 96, 3072)])
+def test_products_of_17_to_64_rows(hip, M, heads, kv, D, K):
+    """This package's products of more than 16 rows: a row's sums are those of a product of up to 16 rows, bit for bit, and
+    the forms with an activation or with rotation and cache write give the bits of the plain product and the kernel behind
+    it (runs of several tokens, pages that a run shares with the next).  The widths take one, two and four blocks of weight
+    rows a workgroup and blocks of up to 8 and up to 16 rows, the lengths of k half a chunk at the end."""
+    dtype, ps = torch.bfloat16, 16
+    width = (heads + 2 * kv) * D
+    x = rnd(M, K, dtype=dtype, seed=1)
+    w = rnd(width, K, dtype=dtype, seed=2, scale=K ** -0.5)
+
+    def own(w, out_float32=False):
+        y = torch.empty((M, w.shape[0]), dtype=torch.float32 if out_float32 else dtype, device=DEV)
+        assert hip.core.sia_gemm_skinny(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, w.shape[0], K, int(out_float32),
+                                        hip._stream()) == 0
+        return y
+
+    few = [x[i:i + 16].contiguous() for i in range(0, M, 16)]
+    for tall in (w, rnd(16390, K, dtype=dtype, seed=3, scale=K ** -0.5)):
+        assert torch.equal(own(tall), torch.cat([hip.linear(a, tall) for a in few]))
+        assert torch.equal(own(tall, True), torch.cat([hip.linear(a, tall, out_float32=True) for a in few]))
+    for inter in (width // 2, 8200):
+        gate_up = rnd(2 * inter, K, dtype=dtype, seed=4, scale=K ** -0.5)
+        assert torch.equal(hip.gated_linear(x, gate_up), hip.swiglu(own(gate_up)))
+
+    lens = [M // 2, 1, M - M // 2 - 1]
+    ctx = Ctx(lens, [n + past for n, past in zip(lens, (0, 37, 9))])
+    pages = sum(-(-int(n) // ps) for n in ctx.kv_len.tolist()) + 2
+    caches = [Cache(pages, kv, ps, D, dtype, ctx.kv_len.tolist(), seed=5) for _ in range(2)]
+    ang = torch.outer(torch.arange(128, dtype=torch.float32), 1.0 / (10000.0 ** (torch.arange(0, D, 2, dtype=torch.float32) / D)))
+    cos, sin = ang.cos().to(DEV), ang.sin().to(DEV)
+    apart = own(w)
+    hip.rope_kv_write(apart, heads, kv, D, D, cos, sin, ctx, caches[0])
+    at_once, c = torch.empty_like(apart), caches[1]
+    assert hip.core.sia_gemm_skinny_rope(
+        x.data_ptr(), w.data_ptr(), at_once.data_ptr(), M, K, cos.data_ptr(), sin.data_ptr(), ctx.positions.data_ptr(),
+        ctx.seq_of_token.data_ptr(), c.block_table.data_ptr(), c.block_table.shape[1], c.k_pages.data_ptr(),
+        c.v_pages.data_ptr(), heads, kv, D, ps, None, 0, 0.0, hip._stream()) == 0
+    assert torch.equal(apart[:, :heads * D], at_once[:, :heads * D])
+    assert torch.equal(caches[0].k_pages, c.k_pages) and torch.equal(caches[0].v_pages, c.v_pages)
+
+
 @pytest.mark.parametrize("shape", [(17, 3072, 3072), (512, 5120, 3072), (2048, 16384, 3072), (130, 3072, 8192),
                                    (33, 1008, 200), (64, 320, 96)])
 def test_library_product_called_directly(hip, shape):
