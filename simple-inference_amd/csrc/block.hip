@@ -14,6 +14,14 @@ int sia_rope_kv_write(void* qkv, int row_stride, const float* cos_table, const f
                       const int* seq_of_token, const int* block_table, int table_width, void* k_pages, void* v_pages,
                       int n_tokens, int n_heads, int n_kv, int head_dim, int rotary_dim, int page_size, int dtype,
                       hipStream_t stream);
+int sia_add_rmsnorm_slices(float* residual, const float* slices, int splits, const float* weight, void* out, int n, int hidden,
+                           float eps, hipStream_t stream);
+int sia_gemm_tiles_takes(int M, int N, int K);
+int sia_gemm_tiles_takes_swiglu(int M, int inter, int K);
+int sia_gemm_tiles_splits(int M, int N, int K);
+int sia_gemm_tiles(const void* X, const void* W, void* Y, float* slices, int M, int N, int K, hipStream_t stream);
+int sia_gemm_tiles_swiglu(const void* X, const void* W, void* Y, int M, int inter, int K, hipStream_t stream);
+int sia_sum_slices(const float* slices, void* Y, int splits, long long n, hipStream_t stream);
 int sia_gemm_skinny_takes(int M, int N, int K);
 int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int N, int K, int out_float, hipStream_t stream);
 int sia_gemm_skinny_swiglu(const void* X, const void* W, void* Y, int M, int inter, int K, const float* partials,
@@ -71,13 +79,9 @@ struct SiaBlockStep {
     float* ws_ml;
     int n_tokens, n_seqs, n_single, max_splits, n_tiles, n_tiles_split, n_tiles_long, q_bound, kv_bound;
     int own_products;         // whether products that this package's kernels take go to them, not all to `product`
+    float* slices;            // room for the largest product that they leave in slices (null if none does)
+    int fed_splits;           // more than 1: the block's last product stays in that many slices, for the next norm to add
 };
-
-// Y = X W^T by whoever takes a product of this size.
-static int block_product(const SiaBlockStep* S, const void* X, const void* W, void* Y, int N, int K, hipStream_t stream) {
-    if (S->own_products && sia_gemm_skinny_takes(S->n_tokens, N, K)) return sia_gemm_skinny(X, W, Y, S->n_tokens, N, K, 0, stream);
-    return S->product(X, W, Y, S->n_tokens, N, K, 0, stream);
-}
 
 #define SIA_STEP(call)             \
     do {                           \
@@ -85,17 +89,33 @@ static int block_product(const SiaBlockStep* S, const void* X, const void* W, vo
         if (rc_ != 0) return rc_;  \
     } while (0)
 
-// residual += delta (where there is one); then the block up to its attention, whose results are left in S->attended, or
+// Y = X W^T by whoever takes a product of this size.
+static int block_product(const SiaBlockStep* S, const void* X, const void* W, void* Y, int N, int K, hipStream_t stream) {
+    const int M = S->n_tokens;
+    if (S->own_products && sia_gemm_skinny_takes(M, N, K)) return sia_gemm_skinny(X, W, Y, M, N, K, 0, stream);
+    if (S->own_products && sia_gemm_tiles_takes(M, N, K)) {
+        SIA_STEP(sia_gemm_tiles(X, W, Y, S->slices, M, N, K, stream));
+        const int splits = sia_gemm_tiles_splits(M, N, K);
+        return splits > 1 ? sia_sum_slices(S->slices, Y, splits, (long long)M * N, stream) : 0;
+    }
+    return S->product(X, W, Y, M, N, K, 0, stream);
+}
+
+// residual += delta (where there is one; with delta_splits > 1 it lies in that many slices in S->slices); then the block up to its attention, whose results are left in S->attended, or
 // without ``attend`` up to its projected rows, which are left in S->qkv with keys and values in the pages: what a caller that
 // goes on with some rows alone needs of all of them.
 // block_table [n_seqs, table_width], k_pages, v_pages: the block's cache in this step.  0, or the first launch's error.
-SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, const int* block_table,
+SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, int delta_splits, const int* block_table,
                                  int table_width, void* k_pages, void* v_pages, int page_size, int attend, hipStream_t stream) {
     if (!B || !S || !S->product || !S->attend_runs || S->n_tokens <= 0 || S->n_tokens > 65535) return SIA_BAD_ARGUMENT;
     const int M = S->n_tokens, H = B->hidden;
     const int qkv_width = (B->n_heads + 2 * B->n_kv) * B->head_dim;
-    SIA_STEP(sia_add_rmsnorm(S->residual, delta, B->mixer_norm_gain, S->normed, nullptr, M, H, B->mixer_norm_eps,
-                             SIA_BF16, stream));
+    if (delta_splits > 1)
+        SIA_STEP(sia_add_rmsnorm_slices(S->residual, S->slices, delta_splits, B->mixer_norm_gain, S->normed, M, H,
+                                        B->mixer_norm_eps, stream));
+    else
+        SIA_STEP(sia_add_rmsnorm(S->residual, delta, B->mixer_norm_gain, S->normed, nullptr, M, H, B->mixer_norm_eps,
+                                 SIA_BF16, stream));
     if (S->own_products && B->rotary_dim == B->head_dim && B->head_dim % 2 == 0 && sia_gemm_skinny_takes(M, qkv_width, H)) {
         SIA_STEP(sia_gemm_skinny_rope(S->normed, B->w_qkv, S->qkv, M, H, B->cos_table, B->sin_table, S->positions,
                                       S->seq_of_token, block_table, table_width, k_pages, v_pages, B->n_heads, B->n_kv,
@@ -120,20 +140,25 @@ SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, co
     return 0;
 }
 
-// The whole block.  Leaves its last product in S->fed, not yet added.
-SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, const int* block_table,
+// The whole block.  Leaves its last product in S->fed, not yet added (with S->fed_splits > 1 in slices in S->slices).
+SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, int delta_splits, const int* block_table,
                                  int table_width, void* k_pages, void* v_pages, int page_size, hipStream_t stream) {
-    SIA_STEP(sia_prenorm_mixer(B, S, delta, block_table, table_width, k_pages, v_pages, page_size, 1, stream));
+    SIA_STEP(sia_prenorm_mixer(B, S, delta, delta_splits, block_table, table_width, k_pages, v_pages, page_size, 1, stream));
     const int M = S->n_tokens, H = B->hidden, Q = B->n_heads * B->head_dim;
     SIA_STEP(block_product(S, S->attended, B->w_o, S->mixed, H, Q, stream));
     SIA_STEP(sia_add_rmsnorm(S->residual, S->mixed, B->feed_forward_norm_gain, S->normed, nullptr, M, H,
                              B->feed_forward_norm_eps, SIA_BF16, stream));
     if (S->own_products && M <= 64 && H % 64 == 0) {
         SIA_STEP(sia_gemm_skinny_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, nullptr, 0, 0.f, stream));
+    } else if (S->own_products && sia_gemm_tiles_takes_swiglu(M, B->inter, H)) {
+        SIA_STEP(sia_gemm_tiles_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, stream));
     } else {
         SIA_STEP(S->product(S->normed, B->w_gate_up, S->gate_up, M, 2 * B->inter, H, 0, stream));
         SIA_STEP(sia_swiglu(S->gate_up, S->activated, M, B->inter, SIA_BF16, stream));
     }
-    SIA_STEP(block_product(S, S->activated, B->w_down, S->fed, H, B->inter, stream));
+    if (S->fed_splits > 1)
+        SIA_STEP(sia_gemm_tiles(S->activated, B->w_down, S->fed, S->slices, M, H, B->inter, stream));
+    else
+        SIA_STEP(block_product(S, S->activated, B->w_down, S->fed, H, B->inter, stream));
     return 0;
 }

@@ -30,49 +30,15 @@
 // The result element (m, n) is summed over k in an order that depends on K only, not on M, the other rows,
 // the number of waves, the row blocks of a workgroup or their height: whichever shape a launch takes, a row's
 // result is the same bit for bit.
-#include "common.h"
+#include "lds_load.h"
 
 #include <initializer_list>
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
-
-constexpr int SK_STEP = 64;      // k per step of one wave: 128 bytes of a row
+constexpr int SK_STEP = LL_STEP;
 constexpr int SK_CHUNK = 128;    // k per chunk: two steps
 constexpr int SK_SHARES = 16;    // chunk c is summed into share c % 16
 constexpr int SK_MAX_ROWS = 64;
-constexpr int SK_TILE = 1024;    // bytes of a load instruction: 8 rows of a step
-constexpr int SK_LDS = 160 * 1024;
-
-// 16 bytes a lane from `src` into LDS at dst + 16 * lane; counts in vmcnt.
-__device__ __forceinline__ void load_to_lds(const void* src, void* dst) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-}
-
-// Until at most `AT_MOST` of the wave's loads are on their way (they end in the order in which they were made).
-template <int AT_MOST> __device__ __forceinline__ void wait_loads() {
-    static_assert(AT_MOST >= 0 && AT_MOST < 64, "vmcnt has 6 bits");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AT_MOST) : "memory");
-}
-
-// The same for `steps` <= SLOTS - 1 steps behind the one that is waited for.
-template <int LOADS, int SLOTS> __device__ __forceinline__ void wait_step(int steps) {
-    if constexpr (SLOTS == 1)
-        wait_loads<0>();
-    else if (steps >= SLOTS - 1)
-        wait_loads<(SLOTS - 1) * LOADS>();
-    else
-        wait_step<LOADS, SLOTS - 1>(steps);
-}
-
-// Place p of row r (of 16) holds piece p ^ turn(r).  A 128-bit LDS read is served 16 lanes at a time, lanes 0-3, 12-15, 20-23
-// and 24-27 first: rows 0-3 and 12-15 of one lane group, 4-11 of the next, whose pieces differ by 2.  Rows 2j and 2j + 1 lie in
-// the two halves of the 64 banks; this order of j keeps the eight places of a half apart for every such set.
-__device__ __forceinline__ int turn(int r) {
-    const int j = r >> 1;
-    return (j & 1) | ((j >> 2) & 1) << 1 | (((j >> 1) ^ (j >> 2)) & 1) << 2;
-}
+constexpr int SK_TILE = LL_TILE;
 
 enum SkinnyEpilogue { EPI_STORE = 0, EPI_SWIGLU = 1, EPI_ROPE = 2, EPI_RESIDUAL = 3, EPI_ACT = 4, EPI_GROUPED = 5 };
 
@@ -161,7 +127,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     constexpr int RING = WAVES * SLOTS * LOADS * SK_TILE;
     constexpr int PART = 8 * RB * ROWS * 17 * 4, SQUARES = SCALED ? SK_SHARES * 16 * 4 : 0;
     constexpr int LDS = RING > PART + SQUARES ? RING : PART + SQUARES;
-    static_assert(LDS <= SK_LDS, "a workgroup's LDS");
+    static_assert(LDS <= LL_LDS, "a workgroup's LDS");
     __shared__ __attribute__((aligned(1024))) char lds[LDS];
     float(*part)[RB][ROWS][17] = reinterpret_cast<float(*)[RB][ROWS][17]>(lds);
     float(*squares)[16] = reinterpret_cast<float(*)[16]>(lds + PART);
@@ -288,7 +254,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
             const int s = s0 + t, j = t / 2;
             // s is the same in all lanes of the wave (a scalar): a step beyond the last is skipped by a branch
             if (s < steps) {
-                wait_step<LOADS, SLOTS>(steps - 1 - s);
+                wait_step<LOADS, SLOTS - 1>(steps - 1 - s);
                 const char* from = ring + slot * (LOADS * SK_TILE);
                 bf16x8 a[RB][2], b[MB][2];
 #pragma unroll
@@ -446,7 +412,9 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
 SIA_EXPORT int sia_gemm_skinny_max_rows() { return 16; }
 SIA_EXPORT int sia_gemm_skinny_most_rows() { return SK_MAX_ROWS; }
 
-// Whether a product goes to this file's kernels rather than to the BLAS library.  Up to 32 rows all do; beyond, X's rows weigh
+extern "C" int sia_gemm_tiles_takes(int M, int N, int K);
+
+// Whether a product goes to this file's kernels rather than to the tiles of gemm_tiles.hip or to the BLAS library.  Up to 32 rows all do; beyond, X's rows weigh
 // as much as W's in what a workgroup fetches, and the library is ahead where the columns are many or k is long.  us, own
 // against the library's best candidate:  27 rows 2,048 x 2,048 4.5 / 8.4, 5,120 x 3,072 11.1 / 12.4, 3,072 x 8,192 16.8 / 16.8,
 // 4,096 x 14,336 33 / 30, 12,288 x 3,072 17.8 / 18.1, 128,256 x 3,072 160 / 165;  45 rows 2,048 x 2,048 5.8 / 8.7, 2,048 x 8,192 16.3 / 15.2,
@@ -454,19 +422,7 @@ SIA_EXPORT int sia_gemm_skinny_most_rows() { return SK_MAX_ROWS; }
 // 8,192 x 2,048 13.6 / 14.0, 4,096 x 14,336 43 / 40, 16,384 x 3,072 26.7 / 23.9, 128,256 x 3,072 195 / 186.
 SIA_EXPORT int sia_gemm_skinny_takes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 || M > SK_MAX_ROWS) return 0;
-    return M <= 32 || (N <= 10240 && (M <= 48 || K <= 8192));
-}
-
-// Compute units of the current device (asked once per device).
-static int compute_units() {
-    static int known[64];
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 256;
-    if (!known[device]) {
-        int n = 0;
-        known[device] = (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && n > 0) ? n : 256;
-    }
-    return known[device];
+    return M <= 32 || (!sia_gemm_tiles_takes(M, N, K) && N <= 10240 && (M <= 48 || K <= 8192));
 }
 
 // How a product is cut into workgroups: `unit_blocks` blocks of `bh` units each, `grid` workgroups.
@@ -503,8 +459,6 @@ static Cut cheapest(int units, int rows_per_unit, std::initializer_list<int> uni
     }
     return best;
 }
-
-static bool aligned16(const void* X, const void* W) { return (((uintptr_t)X | (uintptr_t)W) & 15) == 0; }
 
 struct Product {
     const bf16_t* X;

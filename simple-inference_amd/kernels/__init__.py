@@ -110,8 +110,8 @@ _SIGNATURES = {
     "sia_attention_max_head_dim": [],
     "sia_attention_generic_max_head_dim": [],
     "sia_gemm_generic": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
-    "sia_prenorm_block": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
-    "sia_prenorm_mixer": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
+    "sia_prenorm_block": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
+    "sia_prenorm_mixer": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
     "sia_sample": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_sample_workspace_bytes": [_c_int],
     "sia_sample_few_max_k": [],
@@ -120,6 +120,12 @@ _SIGNATURES = {
     "sia_sample_static_init": [],
     "sia_gemm_skinny": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_skinny_max_rows": [],
+    "sia_gemm_tiles_takes": [_c_int, _c_int, _c_int],
+    "sia_gemm_tiles_takes_swiglu": [_c_int, _c_int, _c_int],
+    "sia_gemm_tiles_splits": [_c_int, _c_int, _c_int],
+    "sia_gemm_tiles": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
+    "sia_sum_slices": [_c_ptr, _c_ptr, _c_int, _c_ll, _c_ptr],
+    "sia_gemm_tiles_swiglu": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_skinny_most_rows": [],
     "sia_gemm_skinny_takes": [_c_int, _c_int, _c_int],
     "sia_gemm_skinny_residual_blocks": [_c_int],
@@ -132,6 +138,7 @@ _SIGNATURES = {
     "sia_take_rows": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ll, _c_ptr],
     "sia_rows_alone": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_place_tokens": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
+    "sia_add_rmsnorm_slices": [_c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_float, _c_ptr],
     "sia_scale_rows": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_float, _c_ptr],
     "sia_stream_read": [_c_ptr, _c_ll, _c_ptr, _c_ptr],
     "sia_add_rmsnorm_scaled": [_c_ptr, _c_ptr, _c_float, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_float,
@@ -225,6 +232,19 @@ class PendingProduct:
         return self.kernels.linear(self.x, self.w)
 
 
+class SlicedProduct:
+    """A block's last product, left in slices of its k that nobody has added up yet.  The next block of the step adds them in
+    its norm; anybody else gets the tensor from ``compute()``."""
+
+    __slots__ = ("slices", "splits", "out", "kernels")
+
+    def __init__(self, slices, splits, out, kernels):
+        self.slices, self.splits, self.out, self.kernels = slices, splits, out, kernels
+
+    def compute(self):
+        return self.kernels.sum_slices(self.slices, self.splits, self.out)
+
+
 class ScaledRows:
     """Rows of an RMS norm that are multiplied by the gain but not yet divided by their root mean square:
     ``norm(x) = rows * rsqrt(sum_p partials[p, m] / width + eps)``.  ``linear``, ``gated_linear`` and ``qkv_to_cache``
@@ -264,7 +284,8 @@ class _BlockStep(ctypes.Structure):
                                                "attended", "mixed", "gate_up", "activated", "fed", "positions",
                                                "seq_of_token", "cu_q", "kv_len", "ws_acc", "ws_ml")]
                 + [(n, ctypes.c_int) for n in ("n_tokens", "n_seqs", "n_single", "max_splits", "n_tiles", "n_tiles_split",
-                                               "n_tiles_long", "q_bound", "kv_bound", "own_products")])
+                                               "n_tiles_long", "q_bound", "kv_bound", "own_products")]
+                + [("slices", ctypes.c_void_p), ("fed_splits", ctypes.c_int)])
 
 
 def _bind(lib, signatures):
@@ -1397,6 +1418,13 @@ class HipKernels:
                 self._check(self.core.sia_gemm_skinny(_ptr(x), _ptr(w), _ptr(y), M, N, K, int(out_float32),
                                                       self._stream()), "gemm_skinny")
                 return y
+            splits = 0 if out_float32 or not self.use_skinny_gemm else self._tile_splits(M, N, K)
+            if splits:
+                x, w = _in_pieces(x), _in_pieces(w)
+                y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+                slices = torch.empty((splits, M, N), dtype=torch.float32, device=x.device) if splits > 1 else None
+                self._check(self.core.sia_gemm_tiles(_ptr(x), _ptr(w), _ptr(y), _ptr(slices), M, N, K, self._stream()), "gemm_tiles")
+                return y if slices is None else self.sum_slices(slices, splits, y)
             return self._library_product(x, w, out_float32)
         # True 32-bit product.  A float32-stored matrix meeting bfloat16 activations widens them.
         back = None
@@ -1454,7 +1482,20 @@ class HipKernels:
                                                          _ptr(partials), n_partials, eps, self._stream()),
                         "gemm_skinny_swiglu")
             return y
+        if (self.use_skinny_gemm and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16
+                and two_i % 2 == 0 and w_gate_up.shape[1] == K and self._tiles_gate(M, two_i // 2, K)):
+            self._want(x, "gated linear input")
+            x, w_gate_up = _in_pieces(x), _in_pieces(w_gate_up)
+            y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=x.device)
+            self._check(self.core.sia_gemm_tiles_swiglu(_ptr(x), _ptr(w_gate_up), _ptr(y), M, two_i // 2, K, self._stream()),
+                        "gemm_tiles_swiglu")
+            return y
         return self.swiglu(self.linear(x, w_gate_up))
+
+    def sum_slices(self, slices, splits, out):
+        """``out`` = the sum of a product's slices, rounded."""
+        self._check(self.core.sia_sum_slices(_ptr(slices), _ptr(out), splits, out.numel(), self._stream()), "sum_slices")
+        return out
 
     def activated_linear(self, x, w, activation):
         """``act(x @ w^T)`` for an activation without a gate (``relu2``, ``gelu_tanh``): one kernel for few rows,
@@ -1965,6 +2006,27 @@ class HipKernels:
             known = self._own_known[key] = bool(self.core.sia_gemm_skinny_takes(M, N, K))
         return known
 
+    def _tile_splits(self, M, N, K) -> int:
+        """Slices in which this package's tiles leave a product of this size; 0 where it is the library's."""
+        if M <= 32 or M > 1024:
+            return 0
+        key = (M, N, K, "tiles")
+        known = self._own_known.get(key)
+        if known is None:
+            known = self._own_known[key] = (self.core.sia_gemm_tiles_splits(M, N, K)
+                                            if self.core.sia_gemm_tiles_takes(M, N, K) else 0)
+        return known
+
+    def _tiles_gate(self, M, inter, K) -> bool:
+        """Whether the gated product of this size goes to the tiles."""
+        if M <= self._skinny_most or M > 1024:
+            return False
+        key = (M, inter, K, "gate")
+        known = self._own_known.get(key)
+        if known is None:
+            known = self._own_known[key] = bool(self.core.sia_gemm_tiles_takes_swiglu(M, inter, K))
+        return known
+
     def _library_can(self, M, N, K) -> bool:
         key = (M, N, K)
         known = self._products_known.get(key)
@@ -2039,6 +2101,14 @@ class HipKernels:
                           *[_ptr(b) for b in buffers], _ptr(ctx.positions), _ptr(ctx.seq_of_token), _ptr(ctx.cu_q),
                           _ptr(ctx.kv_len), _ptr(ws_acc), _ptr(ws_ml), M, ctx.n_seqs, n_dec, max_splits, *tiles,
                           int(self.use_skinny_gemm))
+        if self.use_skinny_gemm:      # products that this package's tiles leave in slices
+            sizes = [(n, self._tile_splits(M, n, k)) for n, k in ((width, H), (H, Q), (H, I))]
+            room = max(s * M * n if s > 1 else 0 for n, s in sizes)
+            if room:
+                buffers.append(torch.empty(room, dtype=torch.float32, device=device))
+                step.slices = _ptr(buffers[-1])
+                if H % 8 == 0 and H <= 8192:
+                    step.fed_splits = sizes[-1][1]
         steps[key] = (step, buffers)
         return steps[key]
 
@@ -2062,7 +2132,11 @@ class HipKernels:
         step = self._block_step(own, ctx, residual.device)
         if step is None:
             return None
-        delta = stream.delta    # computes it if it is a product not yet computed
+        raw, splits = stream.raw_delta, 1
+        if isinstance(raw, SlicedProduct) and _ptr(raw.slices) == step[0].slices:     # this step's block before this one
+            delta, splits = raw.out, raw.splits
+        else:
+            delta = stream.delta    # computes it if it is a product not yet computed
         if delta is not None and (delta.dtype != torch.bfloat16 or tuple(delta.shape) != (M, own.hidden)
                                   or not delta.is_contiguous()):
             return None
@@ -2070,8 +2144,8 @@ class HipKernels:
                           torch.bfloat16, ctx)
         step_struct, buffers = step
         step_struct.residual = _ptr(residual)
-        return (ctypes.addressof(own), ctypes.addressof(step_struct), _ptr(delta), _ptr(cache.block_table),
-                cache.block_table.shape[1], _ptr(cache.k_pages), _ptr(cache.v_pages), cache.page_size), buffers
+        return (ctypes.addressof(own), ctypes.addressof(step_struct), _ptr(delta), splits, _ptr(cache.block_table),
+                cache.block_table.shape[1], _ptr(cache.k_pages), _ptr(cache.v_pages), cache.page_size), buffers, step_struct
 
     def prenorm_block(self, block, stream, ctx, cache) -> bool:
         """Runs a pre-norm block of RMS norms, paged attention and SwiGLU on a step of many rows with one call into
@@ -2081,7 +2155,8 @@ class HipKernels:
         if call is None:
             return False
         self._check(self.core.sia_prenorm_block(*call[0], self._stream()), "prenorm_block")
-        stream.delta = call[1][-1]
+        fed, splits = call[1][6], call[2].fed_splits
+        stream.delta = SlicedProduct(call[1][7], splits, fed, self) if splits > 1 else fed
         return True
 
     def prenorm_mixer(self, block, stream, ctx, cache, attend):

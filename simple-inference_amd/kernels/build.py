@@ -40,7 +40,7 @@ HIPCC_FLAGS = [
 # name -> sources.  "core" is everything a model needs in either dtype; further libraries
 # are specialisations compiled for the sizes a model has (see ``specialised``).
 LIBRARIES: Dict[str, Sequence[str]] = {
-    "core": ("elementwise.hip", "rope_cache.hip", "qk_prepare.hip", "attention_generic.hip", "attention_f32.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_skinny.hip",
+    "core": ("elementwise.hip", "rope_cache.hip", "qk_prepare.hip", "attention_generic.hip", "attention_f32.hip", "gemm_generic.hip", "gemm_f32.hip", "gemm_skinny.hip", "gemm_tiles.hip",
              "sampling.hip", "bandwidth.hip", "block.hip", "gated.hip", "recurrent.hip", "moe.hip", "dyt.hip", "conv.hip", "latent.hip",
              "layernorm.hip", "lowrank.hip", "token_input.hip", "row_prepare.hip", "rglru.hip", "token_shift.hip"),
     # the vendor's BLAS library called directly (the products of steps of many tokens); optional: without it those

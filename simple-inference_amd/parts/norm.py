@@ -90,7 +90,8 @@ class RMSNorm:
             if rows is None:
                 stream.delta = None
             return out
-        if scaled_ok and rows is None and hasattr(stream.raw_delta, "compute") and hasattr(k, "linear_into_residual"):
+        if (scaled_ok and rows is None and hasattr(stream.raw_delta, "compute") and not hasattr(stream.raw_delta, "slices")
+                and hasattr(k, "linear_into_residual")):
             out = k.linear_into_residual(stream.raw_delta, stream.residual, self.weight, self.eps)
             stream.delta = None
             return out

@@ -234,6 +234,44 @@ def test_products_of_17_to_64_rows(hip, M, heads, kv, D, K):
     assert torch.equal(caches[0].k_pages, c.k_pages) and torch.equal(caches[0].v_pages, c.v_pages)
 
 
+@pytest.mark.parametrize("M", [65, 96, 97, 128, 129, 200, 257, 300, 513])
+@pytest.mark.parametrize("N, K", [(64, 64), (136, 320), (1032, 1088), (2048, 8192), (5120, 3072), (16384, 192)])
+def test_tiles_of_a_product_of_many_rows(hip, M, N, K):
+    """The tiles of products between the few-row kernels and the library: row blocks and column blocks that are short at
+    the end, one slice of k and several, slices of unequal length, the gated form.  Errors of the float sums: K products
+    of values around 1, below 1e-6 K, and a rounding to bfloat16 of the result (2^-8 of it at most)."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2)
+    want = x.double() @ w.double().T
+    splits = hip.core.sia_gemm_tiles_splits(M, N, K)
+    assert splits >= 1
+    y = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    slices = torch.full((splits, M, N), float("nan"), device=DEV)
+    assert hip.core.sia_gemm_tiles(x.data_ptr(), w.data_ptr(), y.data_ptr(), slices.data_ptr(), M, N, K, hip._stream()) == 0
+    if splits > 1:
+        assert float((slices.double().sum(0) - want).abs().max()) <= 1e-6 * K
+        hip.sum_slices(slices, splits, y)
+    assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6 * K).all())
+    gated = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert hip.core.sia_gemm_tiles_swiglu(x.data_ptr(), w.data_ptr(), gated.data_ptr(), M, N // 2, K, hip._stream()) == 0
+    ref = torch.nn.functional.silu(want[:, :N // 2]) * want[:, N // 2:]
+    scale = K ** 0.5        # of a gate or an up value; three roundings of 2^-9 each, the activation's slope below 1.1
+    assert bool(((gated.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -8 * scale * (want[:, N // 2:].abs() + scale)).all())
+
+
+@pytest.mark.parametrize("M, hidden, splits", [(1, 8, 2), (65, 64, 1), (70, 2048, 3), (128, 3080, 16), (300, 8192, 5)])
+def test_the_norm_that_adds_a_product_s_slices(hip, M, hidden, splits):
+    """The same bits as the slices' sum and the norm behind it in launches of their own."""
+    slices = rnd(splits, M, hidden, seed=1)
+    res, gain = rnd(M, hidden, seed=2, scale=3.0), rnd(hidden, seed=3) + 1.0
+    delta = hip.sum_slices(slices, splits, torch.empty((M, hidden), dtype=torch.bfloat16, device=DEV))
+    a, b = res.clone(), res.clone()
+    want = hip.add_rmsnorm(a, delta, gain, 1e-5, torch.bfloat16)
+    got = torch.empty_like(want)
+    assert hip.core.sia_add_rmsnorm_slices(b.data_ptr(), slices.data_ptr(), splits, gain.data_ptr(), got.data_ptr(), M, hidden,
+                                           1e-5, hip._stream()) == 0
+    assert torch.equal(a, b) and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("shape", [(17, 3072, 3072), (512, 5120, 3072), (2048, 16384, 3072), (130, 3072, 8192),
                                    (33, 1008, 200), (64, 320, 96)])
 def test_library_product_called_directly(hip, shape):

@@ -185,6 +185,29 @@ def test_the_four_cuts_at_real_widths(models, name, dtype):
         print(f"\n{name} bfloat16, 2 layers: worst {worst:.3e}, same best token at {top1:.1%} of 495 places")
 
 
+@pytest.mark.parametrize("name, lengths", [("1b", (65, 130, 200)), ("3b", (45, 96, 256)), ("8b", (33, 300, 500))])
+def test_prompts_of_every_kind_of_product_in_one_call_a_block_and_part_by_part(models, name, lengths):
+    """Prompts whose products are this package's few-row kernels, its tiles in one slice and in several, and the library's:
+    a block's launches in one call, where a product's slices are added in the next norm, and part by part give the same
+    bits, and both agree with the plain implementation."""
+    _, cfg, _ = models(name)
+    prompts = {i: random_tokens(cfg["vocab_size"], n, seed=500 + n) for i, n in enumerate(lengths)}
+    outs = []
+    for whole in (True, False):
+        runner, cache, kernels = runner_for(models, name, "bfloat16", num_pages=sum(-(-n // PAGE) for n in lengths) + 1)
+        kernels.whole_blocks = whole
+        schedule = [([(i, t, [0, len(t) - 1] if i == 0 else list(range(len(t) - 40, len(t))))], []) for i, t in prompts.items()]
+        schedule[0] = ([(0, prompts[0], list(range(len(prompts[0]))))], [])
+        outs.append(run_schedule(runner, cache, schedule))
+        kernels.whole_blocks = True
+    for i in prompts:
+        assert outs[0][i].keys() == outs[1][i].keys()
+        for place in outs[0][i]:
+            assert torch.equal(outs[0][i][place], outs[1][i][place]), (i, place)
+    worst, _ = worst_error(models, name, outs[0], prompts, allowed=TOLERANCE["hip-bf16"])
+    assert worst <= TOLERANCE["hip-bf16"], f"{worst:.3e}"
+
+
 @pytest.mark.parametrize("mode", ["float32", "bfloat16", "bfloat16-unfused"])
 def test_steps_of_1_8_16_17_and_64_single_tokens_at_3b_widths(models, mode):
     """64 requests with prompts of 3 to 34 tokens decode together, then 17, 16, 8 and one of them: a step of up to
