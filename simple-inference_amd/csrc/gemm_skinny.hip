@@ -211,9 +211,16 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     const int row_steps = K / SK_STEP;
     const int turns = row_steps / (2 * WAVES), rest = row_steps % (2 * WAVES) - 2 * wave;
     const int steps = 2 * turns + min(max(rest, 0), 2);
+    // Rows a multiple of 4 KiB apart lie alike in the memory's channels: workgroups that walk them in step would all be in the
+    // same half of the channels.  Every other workgroup (of a die) takes the chunks of shares s and s + 8 in the other order:
+    // each share's own order stays, and the two are added to each other.  (us: 128,256 x 2,048 91.5 -> 87.6 for one row, 121 -> 108 for
+    // 27, 14,336 x 4,096 gated 43.4 -> 41.7 and 49.7 -> 45.5, 6,144 x 4,096 11.4 -> 10.7; gated rows of one turn lose, 8,192 x 2,048 13.5 -> 14.7
+    // for one row, 20.5 -> 23.1 for 64: not these.)
+    const bool alike = K % (SK_SHARES * SK_CHUNK) == 0 && (EPI != EPI_SWIGLU || K > SK_SHARES * SK_CHUNK);
+    const int swap = alike && (blockIdx.x >> 3 & 1) ? SPW / 2 : 0;
     char* ring = lds + wave * (SLOTS * LOADS * SK_TILE);
     auto request = [&](int s, int slot) {
-        const size_t k = (size_t)(wave + (s >> 1) * WAVES) * SK_CHUNK + (s & 1) * SK_STEP;
+        const size_t k = (size_t)(wave + ((s >> 1) ^ swap) * WAVES) * SK_CHUNK + (s & 1) * SK_STEP;
         char* to = ring + slot * (LOADS * SK_TILE);
 #pragma unroll
         for (int l = 0; l < LOADS; ++l) load_to_lds((const char*)(base[l] + k) + offset[l], to + l * SK_TILE);
