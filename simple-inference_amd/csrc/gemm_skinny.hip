@@ -213,21 +213,23 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     const int steps = 2 * turns + min(max(rest, 0), 2);
     // Rows a multiple of 4 KiB apart lie alike in the memory's channels: workgroups that walk them in step would all be in the
     // same half of the channels.  Every other workgroup (of a die) takes the chunks of shares s and s + 8 in the other order:
-    // each share's own order stays, and the two are added to each other.  (us: 128,256 x 2,048 91.5 -> 87.6 for one row, 121 -> 108 for
-    // 27, 14,336 x 4,096 gated 43.4 -> 41.7 and 49.7 -> 45.5, 6,144 x 4,096 11.4 -> 10.7; gated rows of one turn lose, 8,192 x 2,048 13.5 -> 14.7
-    // for one row, 20.5 -> 23.1 for 64: not these.)
-    const bool alike = K % (SK_SHARES * SK_CHUNK) == 0 && (EPI != EPI_SWIGLU || K > SK_SHARES * SK_CHUNK);
-    const int swap = alike && (blockIdx.x >> 3 & 1) ? SPW / 2 : 0;
+    // each share's own order stays, and the two are added to each other.  (us: 128,256 x 2,048 91.5 -> 87.0 for one row, 120 -> 108 for
+    // 27, 14,336 x 4,096 gated 43.0 -> 42.2 for 16 and 48.7 -> 45.4 for 27, 6,144 x 4,096 11.3 -> 10.6, 8,192 x 2,048 gated 20.6 -> 18.4 for 64;
+    // but 13.7 -> 14.6 for one row, whose two turns are all on their way at once: not that.)
+    const bool alike = K % (SK_SHARES * SK_CHUNK) == 0 && (EPI != EPI_SWIGLU || XI > 1 || K > SK_SHARES * SK_CHUNK);
+    constexpr int HOP = WAVES * SK_CHUNK;  // from one chunk of the wave to its next
+    const int swap = alike && (blockIdx.x >> 3 & 1) ? SPW / 2 * HOP : 0;
     char* ring = lds + wave * (SLOTS * LOADS * SK_TILE);
-    auto request = [&](int s, int slot) {
-        const size_t k = (size_t)(wave + ((s >> 1) ^ swap) * WAVES) * SK_CHUNK + (s & 1) * SK_STEP;
+    // step s0 + u, s0 a multiple of 2 SPW and u known to the compiler
+    auto request = [&](int s0, int u, int slot) {
+        const size_t k = (size_t)(wave * SK_CHUNK + (s0 / 2 + u / 2) * HOP + u % 2 * SK_STEP + (u / 2 % SPW < SPW / 2 ? swap : -swap));
         char* to = ring + slot * (LOADS * SK_TILE);
 #pragma unroll
         for (int l = 0; l < LOADS; ++l) load_to_lds((const char*)(base[l] + k) + offset[l], to + l * SK_TILE);
     };
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s)
-        if (s < steps) request(s, s);
+        if (s < steps) request(0, s, s);
 
     // what the rotation and the cache write need is on its way beside the weights
     float rope_cos[ROPE_ITER], rope_sin[ROPE_ITER];
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
                     for (int rb = 0; rb < RB; ++rb) a[rb][h] = *(const bf16x8*)(from + rb * WI * SK_TILE + w_at[h]);
                 }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot has been read: it may be filled again
-                if (s + SLOTS < steps) request(s + SLOTS, slot);
+                if (s + SLOTS < steps) request(s0, t + SLOTS, slot);
                 slot = slot + 1 < SLOTS ? slot + 1 : 0;
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb)
@@ -429,7 +431,7 @@ extern "C" int sia_gemm_tiles_takes(int M, int N, int K);
 // 8,192 x 2,048 13.6 / 14.0, 4,096 x 14,336 43 / 40, 16,384 x 3,072 26.7 / 23.9, 128,256 x 3,072 195 / 186.
 SIA_EXPORT int sia_gemm_skinny_takes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 || M > SK_MAX_ROWS) return 0;
-    return M <= 32 || (!sia_gemm_tiles_takes(M, N, K) && N <= 10240 && (M <= 48 || K <= 8192));
+    return M <= 32 || (!sia_gemm_tiles_takes(M, N, K) && N <= 10 * 1024 && (M <= 48 || K <= 8 * 1024));
 }
 
 // How a product is cut into workgroups: `unit_blocks` blocks of `bh` units each, `grid` workgroups.

@@ -22,9 +22,9 @@
 
 // GLU: W = [gate; up] of N rows each, Y = silu(gate) * up of the sums rounded to bfloat16 (the bits of the product and the
 // activation kernel behind it); a wave's columns are half gate, half up, of the same columns of Y, so that a lane holds both.
-template <int BM, int BN, int WM, int WN, int DX, int DW, bool GLU>
+template <typename TOut, int BM, int BN, int WM, int WN, int DX, int DW, bool GLU>
 __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_tiles_kernel(const bf16_t* __restrict__ X,
-                                                                     const bf16_t* __restrict__ W, bf16_t* __restrict__ Y,
+                                                                     const bf16_t* __restrict__ W, TOut* __restrict__ Y,
                                                                      float* __restrict__ slices, int M, int N, int K,
                                                                      int splits, int row_blocks, int pairs) {
     constexpr int WAVES = WM * WN, LOADERS = WAVES / 2;
@@ -142,6 +142,10 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_tiles_kernel(const bf16
         for (int i = 0; i < (GLU ? TN / 2 : TN); ++i) {
             const int n = n0 + wn * (BNO / WN) + i * 16 + g * 4;
             if (n >= N) continue;
+            if constexpr (sizeof(TOut) == 4) {   // whole k in one slice
+                *(floatx4*)(Y + (size_t)m * N + n) = acc[i][j];
+                continue;
+            }
             if (!GLU && splits > 1) {
                 *(floatx4*)(slices + ((size_t)slice * M + m) * N + n) = acc[i][j];
                 continue;
@@ -208,12 +212,12 @@ static TilePlan tile_plan(int M, int N, int K, bool glu) {
     return best;
 }
 
-template <int BM, int BN, int WM, int WN, int DX, int DW, bool GLU>
+template <typename TOut, int BM, int BN, int WM, int WN, int DX, int DW, bool GLU>
 static void launch_shape(const void* X, const void* W, void* Y, float* slices, int M, int N, int K, int splits, hipStream_t stream) {
     constexpr int COLUMNS = GLU ? BN / 2 : BN;
     const int row_blocks = (M + BM - 1) / BM, pairs = ((N + COLUMNS - 1) / COLUMNS) * splits;
-    hipLaunchKernelGGL((gemm_tiles_kernel<BM, BN, WM, WN, DX, DW, GLU>), dim3((pairs + 7) / 8 * 8 * row_blocks),
-                       dim3(WM * WN * SIA_WAVE), 0, stream, (const bf16_t*)X, (const bf16_t*)W, (bf16_t*)Y, slices, M, N, K,
+    hipLaunchKernelGGL((gemm_tiles_kernel<TOut, BM, BN, WM, WN, DX, DW, GLU>), dim3((pairs + 7) / 8 * 8 * row_blocks),
+                       dim3(WM * WN * SIA_WAVE), 0, stream, (const bf16_t*)X, (const bf16_t*)W, (TOut*)Y, slices, M, N, K,
                        splits, row_blocks, pairs);
 }
 
@@ -222,7 +226,7 @@ static int launch_tiles(const void* X, const void* W, void* Y, float* slices, in
     const TilePlan plan = tile_plan(M, N, K, GLU);
     if (plan.splits > 1 && !slices) return SIA_BAD_ARGUMENT;
 #define SHAPE(I, ...) \
-    if (plan.shape == I) launch_shape<__VA_ARGS__, GLU>(X, W, Y, slices, M, N, K, plan.splits, stream)
+    if (plan.shape == I) launch_shape<bf16_t, __VA_ARGS__, GLU>(X, W, Y, slices, M, N, K, plan.splits, stream)
     SHAPE(0, 64, 64, 2, 2, 2, 4);
     SHAPE(1, 96, 64, 2, 2, 2, 4);
     SHAPE(2, 128, 64, 2, 2, 2, 3);
@@ -246,7 +250,7 @@ static bool tiles_can(int M, int N, int K) {
 // 9.0 / 10.7, 3,072 x 3,072 at 112 12.7 / 17, 12,288 x 3,072 at 128 25.9 / 29: these stay.)
 SIA_EXPORT int sia_gemm_tiles_takes(int M, int N, int K) {
     if (M <= 32 || M > 1024 || !tiles_can(M, N, K)) return 0;
-    return K >= 2 * N ? (long long)N * K >= 1 << 22 : M > 64 && M <= 256 && N <= 8192 && (long long)N * K >= 15 << 20;
+    return K >= 2 * N ? (long long)N * K >= 1 << 22 : M > 64 && M <= 256 && N <= 8 * 1024 && (long long)N * K >= 15 << 20;
 }
 
 // The same for the gated product: where its tiles come out in one round that fills at least 9/10 of the compute units with
@@ -269,6 +273,28 @@ SIA_EXPORT int sia_gemm_tiles(const void* X, const void* W, void* Y, float* slic
     if (M <= 0 || N <= 0) return 0;
     if (!tiles_can(M, N, K) || !aligned16(X, W) || ((uintptr_t)Y & 7) || ((uintptr_t)slices & 15)) return SIA_BAD_ARGUMENT;
     return launch_tiles<false>(X, W, Y, slices, M, N, K, stream);
+}
+
+// An output head of more than 16 rows in float: W's rows are so many that whole tiles fill the chip many times over, and the
+// workgroups' rings ask for W the deepest.  Rows of W a multiple of 4 KiB apart lie alike in the memory's channels, which tiles of
+// one step's width feel the most: not those.  (us, the better of few-row kernels and library / tiles, of 128,256 x 3,072: 17 rows
+// 150 / 141, 27 154 / 145, 33 166 / 148, 64 182 / 159, 65 188 / 158, 128 200 / 177;  x 2,048: 27 rows 108 / 116, 64 127 / 127, 128 142 / 149;
+// x 4,096: 201 / 231, 218 / 243, 245 / 257.)
+SIA_EXPORT int sia_gemm_tiles_takes_head(int M, int N, int K) {
+    return M > 16 && M <= 128 && N >= 32 * 1024 && K % 2048 != 0 && tiles_can(M, N, K);
+}
+
+// Y[M, N] = X W^T in float.  Needs M <= 128.
+SIA_EXPORT int sia_gemm_tiles_head(const void* X, const void* W, float* Y, int M, int N, int K, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (M > 128 || !tiles_can(M, N, K) || !aligned16(X, W) || ((uintptr_t)Y & 15)) return SIA_BAD_ARGUMENT;
+    if (M <= 32)
+        launch_shape<float, 32, 128, 1, 4, 2, 3, false>(X, W, Y, nullptr, M, N, K, 1, stream);
+    else if (M <= 64)
+        launch_shape<float, 64, 128, 2, 2, 1, 3, false>(X, W, Y, nullptr, M, N, K, 1, stream);
+    else
+        launch_shape<float, 128, 256, 2, 4, 2, 2, false>(X, W, Y, nullptr, M, N, K, 1, stream);
+    return SIA_LAUNCH_CHECK();
 }
 
 // Y = the sum of `splits` slices of n floats each (n a multiple of 4), rounded to bfloat16.

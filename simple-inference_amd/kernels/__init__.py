@@ -124,6 +124,8 @@ _SIGNATURES = {
     "sia_gemm_tiles_takes_swiglu": [_c_int, _c_int, _c_int],
     "sia_gemm_tiles_splits": [_c_int, _c_int, _c_int],
     "sia_gemm_tiles": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
+    "sia_gemm_tiles_takes_head": [_c_int, _c_int, _c_int],
+    "sia_gemm_tiles_head": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_sum_slices": [_c_ptr, _c_ptr, _c_int, _c_ll, _c_ptr],
     "sia_gemm_tiles_swiglu": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_skinny_most_rows": [],
@@ -1411,6 +1413,11 @@ class HipKernels:
         M, K = x.shape
         N = w.shape[0]
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
+            if out_float32 and self.use_skinny_gemm and self._tiled_head(M, N, K):
+                x, w = _in_pieces(x), _in_pieces(w)
+                y = torch.empty((M, N), dtype=torch.float32, device=x.device)
+                self._check(self.core.sia_gemm_tiles_head(_ptr(x), _ptr(w), _ptr(y), M, N, K, self._stream()), "gemm_tiles_head")
+                return y
             # few rows: this package's kernel, whose sums do not depend on the number of rows
             if self.use_skinny_gemm and (M <= self._skinny_rows and K % 64 == 0 or self._own_product(M, N, K)):
                 y = torch.empty((M, N), dtype=torch.float32 if out_float32 else torch.bfloat16, device=x.device)
@@ -2017,6 +2024,16 @@ class HipKernels:
                                             if self.core.sia_gemm_tiles_takes(M, N, K) else 0)
         return known
 
+    def _tiled_head(self, M, N, K) -> bool:
+        """Whether an output head of this size goes to the tiles."""
+        if M <= self._skinny_rows or M > 128:
+            return False
+        key = (M, N, K, "head")
+        known = self._own_known.get(key)
+        if known is None:
+            known = self._own_known[key] = bool(self.core.sia_gemm_tiles_takes_head(M, N, K))
+        return known
+
     def _tiles_gate(self, M, inter, K) -> bool:
         """Whether the gated product of this size goes to the tiles."""
         if M <= self._skinny_most or M > 1024:
@@ -2107,7 +2124,7 @@ class HipKernels:
             if room:
                 buffers.append(torch.empty(room, dtype=torch.float32, device=device))
                 step.slices = _ptr(buffers[-1])
-                if H % 8 == 0 and H <= 8192:
+                if H % 8 == 0 and H <= 8 * 1024:
                     step.fed_splits = sizes[-1][1]
         steps[key] = (step, buffers)
         return steps[key]

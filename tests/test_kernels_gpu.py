@@ -258,6 +258,17 @@ def test_tiles_of_a_product_of_many_rows(hip, M, N, K):
     assert bool(((gated.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -8 * scale * (want[:, N // 2:].abs() + scale)).all())
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("N, K", [(32768, 64), (32900, 192), (40004, 1088)])
+def test_tiles_of_an_output_head(hip, M, N, K):
+    """Float results of whole k in each of the three shapes, the last columns' tile short; errors as above."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2)
+    assert hip.core.sia_gemm_tiles_takes_head(M, N, K)
+    y = hip.linear(x, w, out_float32=True)
+    assert y.dtype == torch.float32
+    assert float((y.double() - x.double() @ w.double().T).abs().max()) <= 1e-6 * K
+
+
 @pytest.mark.parametrize("M, hidden, splits", [(1, 8, 2), (65, 64, 1), (70, 2048, 3), (128, 3080, 16), (300, 8192, 5)])
 def test_the_norm_that_adds_a_product_s_slices(hip, M, hidden, splits):
     """The same bits as the slices' sum and the norm behind it in launches of their own."""
