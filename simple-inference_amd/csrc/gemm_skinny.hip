@@ -32,6 +32,7 @@
 // result is the same bit for bit.
 #include "lds_load.h"
 
+#include <algorithm>
 #include <initializer_list>
 
 constexpr int SK_STEP = LL_STEP;
@@ -437,7 +438,7 @@ SIA_EXPORT int sia_gemm_skinny_takes(int M, int N, int K) {
 // How a product is cut into workgroups: `unit_blocks` blocks of `bh` units each, `grid` workgroups.
 struct Cut {
     int unit_blocks, bh, grid;
-    long long cost;  // rows that the busiest compute unit fetches, if workgroups ran in rounds over the units
+    double cost;
 };
 
 // The block height for workgroups of `unit_blocks` blocks (each unit costs `rows_per_unit` rows of W, a workgroup `x_rows`
@@ -447,7 +448,7 @@ static Cut cut_for(int units, int unit_blocks, int rows_per_unit, int least, int
     const int cus = compute_units();
     auto with = [&](int bh) {
         const int grid = (units + unit_blocks * bh - 1) / (unit_blocks * bh);
-        return Cut{unit_blocks, bh, grid, (long long)((grid + cus - 1) / cus) * (bh * unit_blocks * rows_per_unit + x_rows)};
+        return Cut{unit_blocks, bh, grid, (double)((grid + cus - 1) / cus) * (bh * unit_blocks * rows_per_unit + x_rows)};
     };
     Cut best = with(16);
     if (best.grid > 4 * cus) return best;
@@ -469,6 +470,74 @@ static Cut cheapest(int units, int rows_per_unit, std::initializer_list<int> uni
     return best;
 }
 
+// A kernel for up to 16 rows: blocks of columns a workgroup, waves, steps in a wave's ring, and whether it has a form with
+// half a tile for blocks of up to 8.
+struct Shape {
+    int blocks, waves, slots;
+    bool low;
+};
+
+// Workgroups of a shape that LDS has room for on a compute unit.
+static int room_for(const Shape& s, int bh, int M) {
+    const int tiles = s.blocks * (s.low && bh <= 8 ? 1 : 2) + (M <= 8 ? 1 : 2);
+    return std::max(1, LL_LDS / (s.waves * s.slots * tiles * SK_TILE));
+}
+
+// us that `grid` workgroups of blocks of `bh` rows of W take beside M <= 16 rows of X.  As many as have room in LDS run on a
+// compute unit at a time, and each such round costs a start and an end: the ring fills, the sums meet.  A unit fetches at a
+// rate that what it has on its way allows: 30 GB/s of its own and 1.5 us a trip.  Rows of X (L2 serves them) and repeated
+// rows of W (the same lines) cost half.
+static double few_rows_us(int M, int K, int grid, int bh, const Shape& s) {
+    const int cus = compute_units(), w_rows = s.blocks * (s.low && bh <= 8 ? 8 : 16), x_rows = M <= 8 ? 8 : 16;
+    const int ring = s.waves * s.slots * (w_rows + x_rows) / 8;   // KiB
+    const int room = room_for(s, bh, M), on_unit = (grid + cus - 1) / cus, at_a_time = std::min(on_unit, room);
+    const double rate = 30.0 / (1.0 + 1.5 * 30.0 / (at_a_time * ring));
+    const double rows = s.blocks * bh + 0.5 * (w_rows - s.blocks * bh) + 0.5 * x_rows;
+    return 3.0 * ((on_unit + room - 1) / room) + on_unit * rows * K * 2e-3 / rate;
+}
+
+// The shapes that launch_columns has: up to 8 rows, and up to 16.  (Four blocks a workgroup for 9 to 16 rows: LDS holds two such
+// workgroups of one step a wave, but only one of two blocks and three steps.  us of 16 rows without -> with them: 9,216 x 3,072
+// 17.0 -> 12.4, 12,352 x 3,072 24.5 -> 16.0, 28,672 x 4,096 49.6 -> 42.3, a head of 128,256 x 3,072 156 -> 147.5.  For up to 8 rows two
+// blocks leave room for two workgroups as well: a head of 128,256 x 2,048 89 us, with four blocks 95.)
+static const Shape FEW_ROWS_SHAPES[2][3] = {{{2, 8, 2, false}, {1, 8, 4, true}}, {{4, 8, 1, false}, {2, 8, 3, false}, {1, 8, 4, true}}};
+
+// Of those and the heights of their blocks, what takes the shortest; of equals the higher blocks, then more of them.
+// grid_of(columns): workgroups of that many columns that the result takes.  (By the rows alone, which cheapest goes by, 12,352
+// columns got five rounds of blocks of 10: 8 rows x 1,024 11.3 us, now 6.6, x 3,072 20.5, now 15.1.  From 120 rows of W a unit on the
+// rounds of up to 8 rows run into each other, and the rows do decide: 32,000 x 4,096, one row, 45 us, by rounds 51.)
+template <typename GridOf> static Cut few_rows_cut(int M, int K, GridOf grid_of) {
+    const int columns = grid_of(1);
+    if (M <= 8 && columns > 120 * compute_units()) {
+        Cut cut = cheapest(columns, 1, {2, 1});
+        cut.grid = grid_of(cut.unit_blocks * cut.bh);   // (groups end in workgroups of their own)
+        return cut;
+    }
+    Cut best{0, 0, 0, 0};
+    for (const Shape& s : FEW_ROWS_SHAPES[M > 8])
+        for (int bh = 16; s.blocks && bh >= (s.low ? 8 : 9); --bh) {
+            const int grid = grid_of(s.blocks * bh);
+            const double us = few_rows_us(M, K, grid, bh, s);
+            if (!best.grid || us < best.cost || (us == best.cost && bh > best.bh)) best = Cut{s.blocks, bh, grid, us};
+        }
+    return best;
+}
+
+static Cut few_rows_cut(int M, int K, int N) {
+    return few_rows_cut(M, K, [&](int columns) { return (N + columns - 1) / columns; });
+}
+
+// How a plain product of up to 16 rows is cut: cut[0] blocks of cut[1] columns a workgroup, cut[2] workgroups, cut[3] of them at a
+// time on a compute unit.  0, or SIA_BAD_ARGUMENT.
+SIA_EXPORT int sia_gemm_skinny_cut(int M, int N, int K, int* cut) {
+    if (M <= 0 || M > 16 || N <= 0 || K <= 0 || !cut) return SIA_BAD_ARGUMENT;
+    const Cut c = few_rows_cut(M, K, N);
+    cut[0] = c.unit_blocks, cut[1] = c.bh, cut[2] = c.grid, cut[3] = 1;
+    for (const Shape& s : FEW_ROWS_SHAPES[M > 8])
+        if (s.blocks == c.unit_blocks) cut[3] = room_for(s, c.bh, M);
+    return 0;
+}
+
 struct Product {
     const bf16_t* X;
     const bf16_t* W;
@@ -483,11 +552,13 @@ static void launch(const Product& p, const Cut& cut, const Epilogue& ep) {
                        dim3(WAVES * SIA_WAVE), 0, p.stream, p.X, p.W, (TOut*)p.Y, p.M, p.N, p.K, cut.bh, ep);
 }
 
-// The kernel of a cut whose blocks are columns of Y.  Eight waves; the ring as deep as LDS allows, four steps at most: one
-// workgroup a compute unit, whose waves then have 90 to 160 KB on their way.
+// The kernel of a cut whose blocks are columns of Y, up to 16 rows.  Eight waves; the ring as deep as leaves a compute unit one
+// or two workgroups, four steps at most: 64 to 160 KB are then on their way.
 template <typename TOut, int EPI>
 static void launch_columns(const Product& p, const Cut& cut, const Epilogue& ep) {
     const bool low = cut.bh <= 8;
+    if constexpr (EPI != EPI_RESIDUAL)   // (whose cut is by the columns alone, in one block or two)
+        if (cut.unit_blocks == 4) return launch<TOut, EPI, false, 4, 1, 8, 1>(p, cut, ep);
     if (p.M <= 8) {
         if (cut.unit_blocks == 2) launch<TOut, EPI, false, 2, 1, 8, 2, 2, 1>(p, cut, ep);
         else if (low) launch<TOut, EPI, false, 1, 1, 8, 4, 1, 1>(p, cut, ep);
@@ -511,7 +582,7 @@ static void launch_more_rows(const Product& p, const Cut& cut) {
 }
 
 template <typename TOut> static void launch_store(const Product& p) {
-    if (p.M <= 16) return launch_columns<TOut, EPI_STORE>(p, cheapest(p.N, 1, {2, 1}), Epilogue{});
+    if (p.M <= 16) return launch_columns<TOut, EPI_STORE>(p, few_rows_cut(p.M, p.K, p.N), Epilogue{});
     const int mb = (p.M + 15) / 16;
     const Cut cut = cheapest(p.N, 1, {4, 2, 1}, mb * 16);
     if (mb == 2) launch_more_rows<TOut, 2>(p, cut);
@@ -539,7 +610,7 @@ SIA_EXPORT int sia_gemm_skinny_act(const void* X, const void* W, void* Y, int M,
     if (M > 16 || K % 64 || K <= 0 || !aligned16(X, W) || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU)) return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.activation = activation;
-    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, cheapest(N, 1, {2, 1}), ep);
+    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, few_rows_cut(M, K, N), ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -557,7 +628,7 @@ SIA_EXPORT int sia_gemm_skinny_embedding_gate(const void* X, const void* W, void
     ep.ids = ids;
     ep.table_width = table_width;
     ep.table_dim = dim;
-    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, cheapest(N, 1, {2, 1}), ep);
+    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, few_rows_cut(M, K, N), ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -567,26 +638,15 @@ SIA_EXPORT int sia_gemm_skinny_grouped(const void* X, const void* W, void* Y, in
                                        int last_rows, hipStream_t stream) {
     if (M <= 0) return 0;
     if (M > 16 || K % 64 || K <= 0 || groups <= 0 || group_rows <= 0 || last_rows <= 0 || !X || !W || !Y || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
-    const int cus = compute_units();
-    Cut best{0, 0, 0, 0};
-    int best_blocks = 0;
-    for (int ub : {2, 1})
-        // (where the workgroups are many, full blocks: lower ones would fetch X more often for the same rows)
-        for (int bh = 16; bh >= 8; --bh) {
-            const int a_group = (group_rows + ub * bh - 1) / (ub * bh), last = (last_rows + ub * bh - 1) / (ub * bh);
-            const int grid = (groups - 1) * a_group + last;
-            const Cut c{ub, bh, grid, (long long)((grid + cus - 1) / cus) * bh * ub};
-            if (!best.grid || c.cost < best.cost || (c.cost == best.cost && c.bh > best.bh)) {
-                best = c;
-                best_blocks = a_group;
-            }
-            if (bh == 16 && grid > 2 * cus) break;
-        }
+    const Cut best = few_rows_cut(M, K, [&](int columns) {
+        return (groups - 1) * ((group_rows + columns - 1) / columns) + (last_rows + columns - 1) / columns;
+    });
+    const int columns = best.unit_blocks * best.bh;
     Epilogue ep{};
     ep.groups = groups;
     ep.group_rows = group_rows;
     ep.last_rows = last_rows;
-    ep.group_blocks = best_blocks;
+    ep.group_blocks = (group_rows + columns - 1) / columns;
     launch_columns<bf16_t, EPI_GROUPED>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, group_rows, K, stream}, best, ep);
     return SIA_LAUNCH_CHECK();
 }

@@ -129,6 +129,7 @@ _SIGNATURES = {
     "sia_sum_slices": [_c_ptr, _c_ptr, _c_int, _c_ll, _c_ptr],
     "sia_gemm_tiles_swiglu": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_skinny_most_rows": [],
+    "sia_gemm_skinny_cut": [_c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_skinny_takes": [_c_int, _c_int, _c_int],
     "sia_gemm_skinny_residual_blocks": [_c_int],
     "sia_gemm_skinny_swiglu": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_float, _c_ptr],

@@ -1,5 +1,6 @@
 """Each HIP kernel alone against its plain torch twin, at sizes other than the tiny models'."""
 
+import ctypes
 import math
 
 import pytest
@@ -175,6 +176,44 @@ def test_few_row_product_at_the_edges_of_its_tiles(hip, M, N, K):
     assert torch.equal(hip.linear(aside, w, out_float32=True), hip.linear(aside.clone(), w, out_float32=True))
     gated = hip.gated_linear(aside, torch.cat([w, w]))
     assert torch.equal(gated, hip.gated_linear(aside.clone(), torch.cat([w, w])))
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N", [9216, 11008, 12288, 12352, 14336, 18432])
+def test_few_row_products_of_many_columns_are_cut_by_whole_rounds(hip, M, N):
+    """A compute unit gets its share of the columns in at most two rounds of the workgroups that it holds at a time (by the
+    rows alone it was five rounds of one workgroup of 10 for 12,352 columns), and at most a quarter more of them than that."""
+    cut = (ctypes.c_int * 4)()
+    for K in (1024, 3072, 4096):
+        assert hip.core.sia_gemm_skinny_cut(M, N, K, cut) == 0
+        blocks, height, grid, at_a_time = cut
+        assert grid == -(-N // (blocks * height))
+        units = torch.cuda.get_device_properties(0).multi_processor_count
+        on_unit = -(-grid // units)
+        assert -(-on_unit // at_a_time) <= 2, (K, list(cut))
+        assert on_unit * blocks * height <= 1.25 * N / units, (K, list(cut))
+
+
+@pytest.mark.parametrize("N, K", [(9217, 64), (9216, 1984), (12352, 3072), (16390, 512), (70001, 192)])
+def test_few_row_products_of_four_blocks_a_workgroup(hip, N, K):
+    """9 to 16 rows beside many columns take four blocks a workgroup; up to 8 rows never do.  A row's sums are the same bit for
+    bit, in the plain product (short last workgroup and block, half a chunk of k at the end), with an activation and in groups."""
+    x, w = rnd(16, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2, scale=K ** -0.5)
+    cut = (ctypes.c_int * 4)()
+    halves = (x[:8].contiguous(), x[8:].contiguous())
+    for M in (9, 11, 16):
+        assert hip.core.sia_gemm_skinny_cut(M, N, K, cut) == 0 and cut[0] == 4
+        some = x[:M].contiguous()
+        for call in (lambda a: hip.linear(a, w, out_float32=True), lambda a: hip.linear(a, w),
+                     lambda a: hip.activated_linear(a, w, "relu2")):
+            assert torch.equal(call(some), torch.cat([call(h) for h in halves])[:M])
+        rows = N // 3 - 5
+        main, low = hip.grouped_linear(torch.stack([some, some.flip(0), 2 * some]), w, rows)
+        assert torch.equal(main[0], hip.linear(some, w[:rows]))
+        assert torch.equal(main[1], hip.linear(some.flip(0), w[rows:2 * rows]))
+        assert torch.equal(low, hip.linear(2 * some, w[2 * rows:]))
+    want = x.double() @ w.double().T    # K roundings of 2^-24 of a sum that stays below 8
+    assert float((hip.linear(x, w, out_float32=True).double() - want).abs().max()) <= 5e-7 * K
 
 
 @pytest.mark.parametrize("shape", [(1, 32, 64), (8, 8192, 3072), (16, 1008, 512), (5, 96, 320), (40, 128, 256),
