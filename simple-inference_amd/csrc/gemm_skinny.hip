@@ -201,9 +201,9 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     if (EPI == EPI_ROPE) {
 #pragma unroll
         for (int it = 0; it < ROPE_ITER; ++it) {
-            const int m = min((int)(threadIdx.x + it * THREADS) / 16, M - 1);
-            position[it] = rope.positions[m];
-            sequence[it] = rope.seq_of_token[m];
+            const int m = (threadIdx.x + it * THREADS) / 16;   // (waves beyond the rows wait for their weights alone)
+            position[it] = m < M ? rope.positions[m] : 0;
+            sequence[it] = m < M ? rope.seq_of_token[m] : 0;
         }
     }
 
@@ -239,6 +239,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
         const int u = unit_at(0, threadIdx.x % 16), head = u / rope_half, j = u % rope_half;
 #pragma unroll
         for (int it = 0; it < ROPE_ITER; ++it) {
+            if ((int)(threadIdx.x + it * THREADS) / 16 >= M) break;
             const bool rotates = head < rope.n_heads + rope.n_kv, cached = head >= rope.n_heads;
             const size_t at = (size_t)position[it] * rope_half + j;
             rope_cos[it] = rotates ? rope.cos_table[at] : 1.f;
@@ -760,6 +761,8 @@ SIA_EXPORT int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M
         else launch<bf16_t, EPI_ROPE, false, 2, 4, 8, 1>(p, cut, ep);
         return SIA_LAUNCH_CHECK();
     }
+    // up to 8 rows: two steps leave a compute unit room for two workgroups, three for one (us of 9,216 x 3,072, one row: 13.7 / 14.9)
+    const bool pairs = cut.grid > compute_units();
 #define LAUNCH(SCALED)                                                                        \
     do {                                                                                      \
         if (M <= 8 && low) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 1, 1>(p, cut, ep);    \

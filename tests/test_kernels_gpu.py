@@ -458,7 +458,7 @@ def test_rope_kv_write_of_a_long_step(hip, geom):
 @pytest.mark.parametrize("geom", [
     # heads, kv heads, head_dim, page_size, hidden, rows
     (24, 8, 128, 64, 3072, 8), (3, 1, 32, 8, 192, 16), (5, 5, 96, 16, 1088, 1), (2, 1, 256, 32, 64, 5),
-    (7, 7, 64, 4, 2048, 13), (5, 1, 48, 16, 320, 9), (32, 8, 64, 16, 2048, 4), (1, 1, 16, 2, 64, 3),
+    (7, 7, 64, 4, 2048, 13), (5, 1, 48, 16, 320, 9), (32, 8, 64, 16, 2048, 4), (1, 1, 16, 2, 64, 3), (24, 24, 128, 16, 320, 7),
 ])
 def test_qkv_product_that_rotates_and_writes_the_pages(hip, geom):
     """Few rows: one kernel multiplies, rotates q and k and writes k and v into the pages.  Compared with the
