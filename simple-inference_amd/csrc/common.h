@@ -61,11 +61,11 @@ __device__ __forceinline__ float gated_activation(float g, float u, int kind, fl
     return g / (1.f + expf(-g)) * u;
 }
 
-// Rotation of a pair by an angle's cosine and sine: a' = a c - b s, b' = b c + a s, rounded the same wherever it is done (left to
-// the compiler, which of the two products is fused into the sum differs from kernel to kernel).
+// Rotation of a pair by an angle's cosine and sine: a' = a c - b s, b' = b c + a s, rounded the same wherever it is done: b s and
+// a s are rounded, a c and b c are not (left to the compiler, which product is fused into the sum differs from kernel to kernel).
 __device__ __forceinline__ void rotate_pair(float a, float b, float c, float s, float& ra, float& rb) {
     ra = fmaf(a, c, -(b * s));
-    rb = fmaf(a, s, b * c);
+    rb = fmaf(b, c, a * s);
 }
 
 // Eight consecutive elements of a row as one register value: 32 bytes of float or 16 of bfloat16.

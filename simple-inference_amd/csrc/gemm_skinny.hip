@@ -342,8 +342,8 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
             b = rounded(b * rs);
             if (!is_v) {
                 const float c = rope_cos[it], sn = rope_sin[it];
-                float ra = a * c - b * sn, rb_ = b * c + a * sn;
-                if (ROUND_FIRST) rotate_pair(a, b, c, sn, ra, rb_);
+                float ra, rb_;
+                rotate_pair(a, b, c, sn, ra, rb_);
                 a = ra;
                 b = rb_;
             }

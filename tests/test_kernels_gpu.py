@@ -432,6 +432,34 @@ def test_rope_kv_write_and_attention(hip, dtype, geom):
         torch.testing.assert_close(out.float(), ref.float(), **tol(dtype))
 
 
+@pytest.mark.parametrize("geom", [(24, 8, 128, 128, 16), (5, 1, 48, 32, 8), (3, 3, 12, 8, 4), (4, 2, 64, 64, 16)])
+@pytest.mark.parametrize("tokens", [3, 130])
+def test_the_rotation_s_rounding(hip, geom, tokens):
+    """A rotated pair is fma(a, c, -(b s)) and fma(b, c, a s), bit for bit: what prompts and decoded tokens of any step get,
+    so that their outputs stay what they were.  Inputs of 8 bits make the fused products exact in 64 bits."""
+    n_heads, n_kv, D, rot, ps = geom
+    ctx = Ctx([tokens], [tokens + 100])
+    x = rnd(tokens, (n_heads + 2 * n_kv) * D, dtype=torch.bfloat16, seed=1).float()
+    ang = torch.outer(torch.arange(tokens + 100, dtype=torch.float32), 1.0 / (10000.0 ** (torch.arange(0, rot, 2, dtype=torch.float32) / rot)))
+    cos, sin = ang.cos().to(DEV), ang.sin().to(DEV)
+    cache = Cache(-(-(tokens + 100) // ps) + 1, n_kv, ps, D, torch.float32, [tokens + 100])
+    out = x.clone()
+    hip.rope_kv_write(out, n_heads, n_kv, D, rot, cos, sin, ctx, cache)
+    heads = x[:, :n_heads * D].view(tokens, n_heads, D)
+    a, b = heads[..., :rot // 2], heads[..., rot // 2:rot]
+    c, s = (t[ctx.positions.long()][:, None] for t in (cos, sin))
+    want = torch.cat([(a.double() * c.double() - (b * s).double()).float(), (b.double() * c.double() + (a * s).double()).float(),
+                      heads[..., rot:]], -1)
+    assert torch.equal(out[:, :n_heads * D].view(tokens, n_heads, D), want)
+    keys = x[:, n_heads * D:(n_heads + n_kv) * D].view(tokens, n_kv, D)
+    a, b = keys[..., :rot // 2], keys[..., rot // 2:rot]
+    want = torch.cat([(a.double() * c.double() - (b * s).double()).float(), (b.double() * c.double() + (a * s).double()).float(),
+                      keys[..., rot:]], -1)
+    for t, pos in enumerate(ctx.positions.tolist()):
+        page = int(cache.block_table[0, pos // ps])
+        assert torch.equal(cache.k_pages[page, :, pos % ps], want[t])
+
+
 @pytest.mark.parametrize("geom", [(24, 8, 128, 128, 16), (5, 1, 48, 32, 8), (3, 3, 64, 64, 4)])
 def test_rope_kv_write_of_a_long_step(hip, geom):
     """More than a thousand tokens in one step (the kernel then gives a thread several items): two prompt portions,
