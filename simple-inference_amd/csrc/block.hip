@@ -153,7 +153,7 @@ SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, co
     } else if (S->own_products && sia_gemm_tiles_takes_swiglu(M, B->inter, H)) {
         SIA_STEP(sia_gemm_tiles_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, stream));
     } else {
-        SIA_STEP(S->product(S->normed, B->w_gate_up, S->gate_up, M, 2 * B->inter, H, 0, stream));
+        SIA_STEP(block_product(S, S->normed, B->w_gate_up, S->gate_up, 2 * B->inter, H, stream));
         SIA_STEP(sia_swiglu(S->gate_up, S->activated, M, B->inter, SIA_BF16, stream));
     }
     if (S->fed_splits > 1)

@@ -2120,7 +2120,7 @@ class HipKernels:
                           _ptr(ctx.kv_len), _ptr(ws_acc), _ptr(ws_ml), M, ctx.n_seqs, n_dec, max_splits, *tiles,
                           int(self.use_skinny_gemm))
         if self.use_skinny_gemm:      # products that this package's tiles leave in slices
-            sizes = [(n, self._tile_splits(M, n, k)) for n, k in ((width, H), (H, Q), (H, I))]
+            sizes = [(n, self._tile_splits(M, n, k)) for n, k in ((width, H), (H, Q), (2 * I, H), (H, I))]
             room = max(s * M * n if s > 1 else 0 for n, s in sizes)
             if room:
                 buffers.append(torch.empty(room, dtype=torch.float32, device=device))

@@ -208,6 +208,32 @@ def test_prompts_of_every_kind_of_product_in_one_call_a_block_and_part_by_part(m
     assert worst <= TOLERANCE["hip-bf16"], f"{worst:.3e}"
 
 
+@pytest.mark.parametrize("hidden, inter", [(2048, 4096), (3072, 4096), (4096, 2048)])
+def test_a_block_in_one_call_at_widths_where_the_gated_tiles_refuse(tmp_path, hidden, inter):
+    """Feed-forwards no wider than the stream: the gated product has no kernel with the activation inside at most numbers of
+    rows, and both ways through a block take the same plain product (tiles, in slices or not, or the library's) and the
+    activation behind it: the same bits."""
+    from simple_inference_amd.config import EngineConfig
+    from simple_inference_amd.engine import build_model
+    from simple_inference_amd.weights import random_tensors, write_model_folder
+    cfg = dict(preset(SHAPES["3b"]), num_hidden_layers=LAYERS, hidden_size=hidden, intermediate_size=inter, vocab_size=512,
+               num_attention_heads=hidden // 128, num_key_value_heads=4, head_dim=128, max_position_embeddings=4096)
+    model, mcfg = build_model(cfg, EngineConfig(device="cpu", dtype="float32", max_seq_len=64), kernels=None)
+    tensors = random_tensors(model.expected_tensors(), seed=9, std=0.02, gain_std=0.1, device="cuda:0")
+    folder = write_model_folder(tmp_path, mcfg.to_dict(), tensors)
+    lengths = (40, 65, 97, 150, 204, 300, 600)
+    prompts = {i: random_tokens(512, n, seed=700 + n) for i, n in enumerate(lengths)}
+    outs = []
+    for whole in (True, False):
+        runner, cache, kernels = runner_for(lambda _: (folder,), None, "bfloat16", max_seq_len=1024,
+                                            num_pages=sum(-(-n // PAGE) for n in lengths) + 1, max_running=len(lengths))
+        kernels.whole_blocks = whole
+        outs.append(run_schedule(runner, cache, [([(i, t, list(range(len(t))))], []) for i, t in prompts.items()]))
+    for i in prompts:
+        for place in outs[0][i]:
+            assert torch.equal(outs[0][i][place], outs[1][i][place]), (lengths[i], place)
+
+
 @pytest.mark.parametrize("mode", ["float32", "bfloat16", "bfloat16-unfused"])
 def test_steps_of_1_8_16_17_and_64_single_tokens_at_3b_widths(models, mode):
     """64 requests with prompts of 3 to 34 tokens decode together, then 17, 16, 8 and one of them: a step of up to
