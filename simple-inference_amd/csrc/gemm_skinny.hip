@@ -425,15 +425,25 @@ SIA_EXPORT int sia_gemm_skinny_most_rows() { return SK_MAX_ROWS; }
 
 extern "C" int sia_gemm_tiles_takes(int M, int N, int K);
 
-// Whether a product goes to this file's kernels rather than to the tiles of gemm_tiles.hip or to the BLAS library.  Up to 32 rows all do; beyond, X's rows weigh
-// as much as W's in what a workgroup fetches, and the library is ahead where the columns are many or k is long.  us, own
-// against the library's best candidate:  27 rows 2,048 x 2,048 4.5 / 8.4, 5,120 x 3,072 11.1 / 12.4, 3,072 x 8,192 16.8 / 16.8,
-// 4,096 x 14,336 33 / 30, 12,288 x 3,072 17.8 / 18.1, 128,256 x 3,072 160 / 165;  45 rows 2,048 x 2,048 5.8 / 8.7, 2,048 x 8,192 16.3 / 15.2,
-// 3,072 x 8,192 19.1 / 22.0, 9,216 x 3,072 18.5 / 20.6, 12,288 x 3,072 21.0 / 20.4;  64 rows 3,072 x 3,072 11.4 / 16.2, 3,072 x 8,192 22.4 / 23.7,
-// 8,192 x 2,048 13.6 / 14.0, 4,096 x 14,336 43 / 40, 16,384 x 3,072 26.7 / 23.9, 128,256 x 3,072 195 / 186.
+// Whether a product goes to this file's kernels rather than to the tiles of gemm_tiles.hip or to the BLAS library.  Up to 16 rows all
+// do.  Beyond, X's rows weigh as much as W's in what a workgroup fetches, and k is in one piece: the tiles are ahead over long k,
+// the library where the columns are many, or few and k so long that few workgroups walk it for long (k of 5,120 to 10,240, which the tiles
+// do not take).  A multiple of 8,192 columns comes to a unit as 32 rows of W that start a large power of two apart, which the channels
+// of the memory feel; the library's shapes do not.  us, own / the library's best candidate:
+//   at 27 rows 2,048 x 2,048 4.5 / 8.4, 5,120 x 3,072 11.1 / 12.4;  at 32 8,192 x 5,120 21.7 / 20.8, 8,192 x 8,192 33.3 / 30.4 (stays), 28,672 x
+//   3,072 38.3 / 35.0 (stays), x 4,096 0.86 of the other, 18,432 x 1,024 0.95
+//   at 40 rows 2,048 x 4,096 0.78, 1,024 x 5,120 0.60, 512 x 6,144 1.08, 1,024 x 8,192 14.6 / 12.5, 2,560 x 8,192 17.5 / 16.5 (these three
+//   stay), 9,216 x 3,072 0.89, 12,288 x 3,072 1.02 (stays)
+//   at 57 rows 3,072 x 4,096 0.95, 5,120 x 5,120 0.99, 6,144 x 4,096 1.00, 6,144 x 5,120 1.08 (stays), 9,216 x 8,192 1.01 (stays), 8,192 x 3,072 0.95,
+//   8,192 x 4,096 21.4 / 19.1 (stays)
 SIA_EXPORT int sia_gemm_skinny_takes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 || M > SK_MAX_ROWS) return 0;
-    return M <= 32 || (!sia_gemm_tiles_takes(M, N, K) && N <= 10 * 1024 && (M <= 48 || K <= 8 * 1024));
+    if (M <= 16) return 1;
+    if (sia_gemm_tiles_takes(M, N, K)) return 0;
+    if (N % 8192 == 0 && (M > 48 ? K >= 4096 : M > 20 && K % 8192 == 0)) return 0;
+    if (M <= 32) return N <= 20 * 1024 || K % 2048 == 0;
+    if (N > 10 * 1024 || (K > 5 * 1024 && N < 1536) || (K > 6 * 1024 && N < 3072)) return 0;
+    return M <= 48 || (K <= 8 * 1024 && (N < 6 * 1024 || K < 5 * 1024));
 }
 
 // How a product is cut into workgroups: `unit_blocks` blocks of `bh` units each, `grid` workgroups.

@@ -243,14 +243,32 @@ static bool tiles_can(int M, int N, int K) {
            (long long)N * K < 1LL << 30 && (long long)M * K < 1LL << 30 && (long long)M * N < 1LL << 30;
 }
 
-// Whether a plain product goes to the tiles: long k over few columns from 33 to 1,024 rows, other products of some size from 65 to
-// 256 rows.  (us, few-row kernels or library / tiles with the sum in its own launch:  3,072 x 8,192 at 64 rows 22.4 / 20.6, of which
-// 4 are the sum, which the next norm makes for less, at 256 34.8 / 28.4, at 1,024 68 / 67;  4,096 x 14,336 40 / 30, 63 / 49, 139 / 115;
-// 5,120 x 3,072 at 96 18.7 / 17.2, at 192 27 / 20, at 288 21.2 / 24.5;  6,144 x 4,096 at 128 26 / 22, at 288 29.7 / 34.8;  2,048 x 2,048 at 128
-// 9.0 / 10.7, 3,072 x 3,072 at 112 12.7 / 17, 12,288 x 3,072 at 128 25.9 / 29: these stay.)
+// Whether a plain product of 21 to 1,024 rows goes to the tiles: long k over few columns (k at least twice the columns), where
+// slices of k fill the chip, and other products of some size from 65 to 256 rows.  How large it has to be follows what else there
+// is: up to 64 rows the few-row kernels are near for k up to 8,192; from 65 on the library is, and well ahead again at 8,192 columns
+// up to some 160 rows (k of 2,048 to 4,096 and 8,192).  us, the better of few-row kernel and library / tiles with the sum of the slices in
+// its own launch, of which the norm behind a block's last product saves 3:
+//   at 32 rows 4,096 x 14,336 35 / 32, 3,072 x 14,336 29.9 / 25.5, 512 x 14,336 21.0 / 14.6, 64 to 768 x 65,536 0.36 to 0.46 of the
+//   other;  4,096 x 9,216 23.6 / 22.4, at 24 22.0 / 24.4 (stays)
+//   at 40 rows 2,048 x 8,192 14.4 / 14.7, 2,048 x 5,120 12.4 / 12.5;  1,024 x 8,192 12.5 / 13.3 (stays);  at 57 1,536 x 6,144 16.1 / 13.4
+//   at 96 rows 3,072 x 8,192 36.7 / 21.9, 2,560 x 6,144 18.5 / 18.3, 1,024 x 9,216 17.3 / 16.3, 512 x 11,008 33 / 13.5;  512 x 9,216 at 80
+//   11.1 / 12.3, 1,536 x 6,144 at 65 to 128 0.84 to 1.15 of the other, 2,048 x 4,096 at 256 16.3 / 20.7 (stay)
+//   at 384 rows 1,024 x 8,192 24.8 / 19.4, 2,048 x 5,120 26.3 / 21.3;  1,024 x 5,120 at 512 0.99 to 1.16 of the other, 2,048 x 4,096 at 768
+//   24.6 / 28.1 (stay)
+//   others:  5,120 x 3,072 at 96 18.6 / 17.3, at 192 27.1 / 20.3;  8,192 x 14,336 at 128 87 / 61;  8,192 x 2,048 at 192 23.2 / 18.4, at 65
+//   14.4 / 16.1 (stays);  8,192 x 8,192 at 65 36 / 44, 2,048 x 2,048 at 128 9.0 / 10.7, 12,288 x 3,072 25.9 / 29 (stay)
 SIA_EXPORT int sia_gemm_tiles_takes(int M, int N, int K) {
-    if (M <= 32 || M > 1024 || !tiles_can(M, N, K)) return 0;
-    return K >= 2 * N ? (long long)N * K >= 1 << 22 : M > 64 && M <= 256 && N <= 8 * 1024 && (long long)N * K >= 15 << 20;
+    if (M <= 20 || M > 1024 || !tiles_can(M, N, K)) return 0;
+    const long long size = (long long)N * K, MI = 1 << 20;
+    if (K >= 2 * N) {
+        if (M <= 32) return K > 12 * 1024 && size >= MI / 2;
+        if (K > 10 * 1024 && size >= MI / 2) return 1;
+        if (M <= 64) return size >= (M > 48 ? 7 : 9) * MI;
+        if (M > 256) return K >= 5 * 1024 && size >= 6 * MI;
+        return (size >= 12 * MI && (M > 80 || N >= 2048)) || (K >= 9 * 1024 && N >= 1024);
+    }
+    if (M <= 64 || M > 256 || size < 15 * MI) return 0;
+    return N <= 6 * 1024 || (N <= 8 * 1024 && (M > 160 || K > 8 * 1024 || (M <= 128 && K > 4 * 1024 && K % 8192)));
 }
 
 // The same for the gated product: where its tiles come out in one round that fills at least 9/10 of the compute units with

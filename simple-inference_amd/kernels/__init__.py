@@ -2015,8 +2015,8 @@ class HipKernels:
         return known
 
     def _tile_splits(self, M, N, K) -> int:
-        """Slices in which this package's tiles leave a product of this size; 0 where it is the library's."""
-        if M <= 32 or M > 1024:
+        """Slices in which this package's tiles leave a product of this size; 0 where it is another's."""
+        if M <= self._skinny_rows or M > 1024:
             return 0
         key = (M, N, K, "tiles")
         known = self._own_known.get(key)

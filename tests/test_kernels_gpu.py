@@ -273,7 +273,38 @@ def test_products_of_17_to_64_rows(hip, M, heads, kv, D, K):
     assert torch.equal(caches[0].k_pages, c.k_pages) and torch.equal(caches[0].v_pages, c.v_pages)
 
 
-@pytest.mark.parametrize("M", [65, 96, 97, 128, 129, 200, 257, 300, 513])
+@pytest.mark.parametrize("M, N, K, route", [
+    (16, 8192, 8192, "own"), (20, 8192, 8192, "own"), (21, 8192, 8192, "library"), (48, 8192, 4096, "own"), (49, 8192, 4096, "library"),
+    (32, 20480, 1088, "own"), (32, 20484, 1088, "library"), (32, 20484, 2048, "own"), (33, 10240, 1088, "own"), (33, 10244, 1088, "library"),
+    (20, 4096, 14336, "own"), (21, 4096, 14336, "tiles"), (32, 4096, 12288, "own"), (33, 4096, 12288, "tiles"),
+    (33, 1024, 8192, "library"), (33, 1536, 6144, "tiles"), (33, 1532, 5184, "library"), (33, 1532, 5120, "own"), (33, 2560, 6208, "tiles"),
+    (48, 1024, 4096, "own"), (49, 1536, 5120, "tiles"), (49, 1532, 4096, "own"), (49, 6144, 4096, "own"), (49, 6144, 5120, "library"),
+    (64, 6140, 5120, "own"), (64, 5120, 8256, "library"), (64, 512, 11008, "tiles"), (64, 512, 9216, "library"),
+    (33, 64, 11008, "tiles"), (33, 64, 10240, "library"), (21, 40, 14336, "tiles"), (20, 40, 14336, "own"), (300, 64, 65536, "tiles"),
+    (80, 1536, 8192, "library"), (81, 1536, 8192, "tiles"), (80, 2048, 8192, "tiles"), (128, 1536, 6144, "library"), (256, 1024, 9216, "tiles"),
+    (256, 2048, 4096, "library"), (257, 2048, 5120, "tiles"), (1024, 1024, 6144, "tiles"), (1025, 2048, 8192, "library"),
+    (257, 2048, 4096, "library"), (65, 5120, 3072, "tiles"), (65, 5116, 3072, "library"), (160, 8192, 2048, "library"),
+    (161, 8192, 2048, "tiles"), (128, 8192, 5120, "tiles"), (128, 8192, 8192, "library"), (129, 8192, 5120, "library"), (65, 8192, 8256, "tiles"),
+    (256, 8196, 3072, "library"), (257, 5120, 3072, "library")])
+def test_products_go_where_they_are_made_fastest(hip, M, N, K, route):
+    """The borders of the rules by which a bfloat16 product goes to the few-row kernels, the tiles or the library, and its
+    result on either side: K products of values around 1, below 1e-6 K, and a rounding of 2^-8 at most."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2)
+    names = {"sia_gemm_skinny": "own", "sia_gemm_tiles": "tiles"}
+    real, went = {n: getattr(hip.core, n) for n in names}, []
+    for n in names:
+        setattr(hip.core, n, lambda *a, n=n: went.append(names[n]) or real[n](*a))
+    try:
+        out = hip.linear(x, w)
+    finally:
+        for n in names:
+            setattr(hip.core, n, real[n])
+    assert went == ([route] if route != "library" else [])
+    want = (x.float() @ w.float().T).double()   # (in float32: another rounding of 1e-6 K at most)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2e-6 * K).all())
+
+
+@pytest.mark.parametrize("M", [21, 32, 33, 48, 64, 65, 96, 97, 128, 129, 200, 257, 300, 513])
 @pytest.mark.parametrize("N, K", [(64, 64), (136, 320), (1032, 1088), (2048, 8192), (5120, 3072), (16384, 192)])
 def test_tiles_of_a_product_of_many_rows(hip, M, N, K):
     """The tiles of products between the few-row kernels and the library: row blocks and column blocks that are short at
