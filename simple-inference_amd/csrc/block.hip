@@ -23,6 +23,7 @@ int sia_gemm_tiles(const void* X, const void* W, void* Y, float* slices, int M, 
 int sia_gemm_tiles_swiglu(const void* X, const void* W, void* Y, int M, int inter, int K, hipStream_t stream);
 int sia_sum_slices(const float* slices, void* Y, int splits, long long n, hipStream_t stream);
 int sia_gemm_skinny_takes(int M, int N, int K);
+int sia_gemm_skinny_takes_swiglu(int M, int inter, int K);
 int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int N, int K, int out_float, hipStream_t stream);
 int sia_gemm_skinny_swiglu(const void* X, const void* W, void* Y, int M, int inter, int K, const float* partials,
                            int n_partials, float eps, hipStream_t stream);
@@ -148,7 +149,7 @@ SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, co
     SIA_STEP(block_product(S, S->attended, B->w_o, S->mixed, H, Q, stream));
     SIA_STEP(sia_add_rmsnorm(S->residual, S->mixed, B->feed_forward_norm_gain, S->normed, nullptr, M, H,
                              B->feed_forward_norm_eps, SIA_BF16, stream));
-    if (S->own_products && M <= 64 && H % 64 == 0) {
+    if (S->own_products && sia_gemm_skinny_takes_swiglu(M, B->inter, H)) {
         SIA_STEP(sia_gemm_skinny_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, nullptr, 0, 0.f, stream));
     } else if (S->own_products && sia_gemm_tiles_takes_swiglu(M, B->inter, H)) {
         SIA_STEP(sia_gemm_tiles_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, stream));

@@ -446,6 +446,21 @@ SIA_EXPORT int sia_gemm_skinny_takes(int M, int N, int K) {
     return M <= 48 || (K <= 8 * 1024 && (N < 6 * 1024 || K < 5 * 1024));
 }
 
+// Whether the product with SwiGLU inside goes to this file's kernel.  Up to 16 rows always.  More rows weigh in every workgroup,
+// and k is in one piece: where the columns are few and k long, too few workgroups walk too long; where the columns are many
+// and k short, the library's tiles fill the chip, unless the rows of W are a multiple of 4 KiB apart, where it loses.  us, library or
+// tiles and activation / this kernel:
+//   inter 1,024 x 3,072 at 27 rows 15.0 / 11.3, at 57 13.3 / 16.4;  x 5,120 at 27 20.7 / 17.3, at 48 17.5 / 22.0;  x 14,336 at 57 29.0 / 53.4
+//   inter 2,560 x 4,096 at 48 25.3 / 17.8, at 64 20.4 / 20.6;  x 8,192 at 64 32.2 / 35.6
+//   inter 4,096 x 3,072 at 64 23.0 / 20.2;  x 5,120 at 48 29.1 / 27.4;  x 8,192 at 32 34.1 / 35.7, at 64 37.6 / 41.7
+//   inter 5,120 x 8,192 at 64 46.5 / 44.6;  inter 8,192 x 3,072 at 64 28.5 / 27.0;  inter 9,216 x 3,072 at 57 37.4 / 38.6;  inter 14,336 at 57 x 3,072 41.3 / 47.2, x 4,096 57.7 / 55.4
+SIA_EXPORT int sia_gemm_skinny_takes_swiglu(int M, int inter, int K) {
+    if (M <= 0 || inter <= 0 || K <= 0 || K % 64 || M > SK_MAX_ROWS) return 0;
+    if (M <= 16) return 1;
+    if (K % 2048 && (M > 48 ? inter > 8704 && (K > 2048 || inter > 10 * 1024) : M > 32 && inter > 10 * 1024)) return 0;
+    return inter >= 4608 || K <= 2048 || (inter >= 2560 ? K <= 3072 || (K <= 5120 && M <= 48) : K <= 5120 && M <= 32);
+}
+
 // How a product is cut into workgroups: `unit_blocks` blocks of `bh` units each, `grid` workgroups.
 struct Cut {
     int unit_blocks, bh, grid;

@@ -131,6 +131,7 @@ _SIGNATURES = {
     "sia_gemm_skinny_most_rows": [],
     "sia_gemm_skinny_cut": [_c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_skinny_takes": [_c_int, _c_int, _c_int],
+    "sia_gemm_skinny_takes_swiglu": [_c_int, _c_int, _c_int],
     "sia_gemm_skinny_residual_blocks": [_c_int],
     "sia_gemm_skinny_swiglu": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_float, _c_ptr],
     "sia_gemm_skinny_rope": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int,
@@ -1481,7 +1482,8 @@ class HipKernels:
                                               _ptr(bias), _DT[gu.dtype], self._stream()), "glu")
             return out
         if (self.use_skinny_gemm and x.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16
-                and M <= self._skinny_most and two_i % 2 == 0 and K % 64 == 0 and w_gate_up.shape[1] == K):
+                and two_i % 2 == 0 and w_gate_up.shape[1] == K
+                and (M <= self._skinny_rows and K % 64 == 0 or self._own_gate(M, two_i // 2, K))):
             rows, partials, n_partials, eps = self._scaled(x)
             self._want(rows, "gated linear input")
             y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=rows.device)
@@ -2012,6 +2014,16 @@ class HipKernels:
         known = self._own_known.get(key)
         if known is None:
             known = self._own_known[key] = bool(self.core.sia_gemm_skinny_takes(M, N, K))
+        return known
+
+    def _own_gate(self, M, inter, K) -> bool:
+        """Whether the gated product of this size has the few-row kernel with the activation inside."""
+        if M > self._skinny_most:
+            return False
+        key = (M, inter, K, "few gate")
+        known = self._own_known.get(key)
+        if known is None:
+            known = self._own_known[key] = bool(self.core.sia_gemm_skinny_takes_swiglu(M, inter, K))
         return known
 
     def _tile_splits(self, M, N, K) -> int:

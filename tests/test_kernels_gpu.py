@@ -273,6 +273,29 @@ def test_products_of_17_to_64_rows(hip, M, heads, kv, D, K):
     assert torch.equal(caches[0].k_pages, c.k_pages) and torch.equal(caches[0].v_pages, c.v_pages)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("inter, K, takes", [(1024, 2048, (17, 64)), (1024, 2112, (17, 32)), (1024, 5184, ()), (2560, 3072, (17, 64)),
+                                             (2560, 5120, (17, 48)), (4607, 8192, ()), (4608, 8192, (17, 64)), (8704, 3072, (17, 64)),
+                                             (8705, 3072, (17, 48)), (10241, 1088, (17, 32)), (10241, 2048, (17, 64))])
+def test_gated_products_of_17_to_64_rows_go_where_they_are_made_faster(hip, M, inter, K, takes):
+    """The few-row kernel with the activation inside, or product and activation: the same rows either way (the product
+    rounds first in both; its sums' order may differ: a rounding of bfloat16 in gate and up and one of the result)."""
+    own = bool(takes) and takes[0] <= M <= takes[1]
+    assert bool(hip.core.sia_gemm_skinny_takes_swiglu(M, inter, K)) == own
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(2 * inter, K, dtype=torch.bfloat16, seed=2, scale=K ** -0.5)
+    launched, real = [], hip.core.sia_gemm_skinny_swiglu
+    hip.core.sia_gemm_skinny_swiglu = lambda *a: launched.append(1) or real(*a)
+    try:
+        out = hip.gated_linear(x, w)
+    finally:
+        hip.core.sia_gemm_skinny_swiglu = real
+    assert bool(launched) == own
+    gu = x.double() @ w.double().T
+    ref = torch.nn.functional.silu(gu[:, :inter]) * gu[:, inter:]
+    bound = 2.0 ** -8 * (ref.abs() + gu[:, inter:].abs() * (gu[:, :inter].abs() * 1.1 + 1e-3) + gu[:, :inter].abs() * gu[:, inter:].abs()) + 1e-5
+    assert bool(((out.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M, N, K, route", [
     (16, 8192, 8192, "own"), (20, 8192, 8192, "own"), (21, 8192, 8192, "library"), (48, 8192, 4096, "own"), (49, 8192, 4096, "library"),
     (32, 20480, 1088, "own"), (32, 20484, 1088, "library"), (32, 20484, 2048, "own"), (33, 10240, 1088, "own"), (33, 10244, 1088, "library"),
