@@ -272,14 +272,18 @@ SIA_EXPORT int sia_gemm_tiles_takes(int M, int N, int K) {
 }
 
 // The same for the gated product: where its tiles come out in one round that fills at least 9/10 of the compute units with
-// tiles at least 4/5 full, and the activation kernel is saved.  (us, library and activation / tiles, of 8,192 x 2,048: 96 rows
+// tiles at least 4/5 full, and the activation kernel is saved.  Their k is in one piece: a longer one pays from 129 to 256 rows
+// alone, where the library is at its weakest and the plain tiles, which cut k, do not take the product.  (us, library and activation / tiles, of 8,192 x 2,048: 96 rows
 // 22.7 / 21.8, 192 31.2 / 27.0, 256 34.4 / 28.6, 320 35.5 / 39.2 (three quarters of the units: stays), 1,024 72 / 67;  8,192 x 3,072: 256 46.6 / 39.3,
-// 512 61.8 / 57.5, 640 66 / 81 (two rounds: stays);  14,336 x 4,096, 224 tiles: 256 74.6 / 82.2 (stays).)
+// 512 61.8 / 57.5, 640 66 / 81 (two rounds: stays);  14,336 x 4,096, 224 tiles: 256 74.6 / 82.2 (stays).  x 4,096, the better of
+// library and tiles and the activation behind it / tiles with it inside: inter 5,120 at 256 0.79 of the other, 8,192 at 192 52.7 / 51.8;  2,560 at 192
+// 26.6 / 27.4, 8,192 at 512 74 / 80, 1,024 at 512 25.1 / 26.4, 1,536 x 14,336 at 320 52 / 83, 2,560 x 14,336 at 192 62 / 87 (stay).)
 SIA_EXPORT int sia_gemm_tiles_takes_swiglu(int M, int inter, int K) {
     if (M <= 64 || M > 1024 || !tiles_can(M, inter, K) || (long long)inter * K >= 1LL << 29) return 0;
     const TilePlan plan = tile_plan(M, inter, K, true);
     const long long cus = compute_units();
     const TileShape t = TILE_SHAPES[plan.shape];
+    if (K > 3072 && (M <= 128 || M > 256 || (sia_gemm_tiles_takes(M, 2 * inter, K) && (inter < 4096 || K > 4096)))) return 0;
     return plan.workgroups <= cus && 10 * plan.workgroups >= 9 * cus && 5LL * M * 2 * inter >= 4 * cus * t.bm * t.bn;
 }
 

@@ -296,6 +296,28 @@ def test_gated_products_of_17_to_64_rows_go_where_they_are_made_faster(hip, M, i
     assert bool(((out.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M, inter, K, inside", [
+    (65, 8192, 2048, False), (128, 8192, 2048, True), (512, 8192, 3072, True), (512, 8192, 3136, False), (128, 8192, 4096, False),
+    (192, 8192, 4096, True), (256, 8192, 4096, True), (257, 8192, 4096, False), (256, 5120, 8192, True), (192, 2560, 4096, False),
+    (512, 1024, 14336, False), (1024, 8192, 2048, True), (1025, 8192, 2048, False)])
+def test_gated_tiles_are_taken_where_their_undivided_k_pays(hip, M, inter, K, inside):
+    """The borders of the rule, and either way the same rows: three roundings of bfloat16 (gate, up, result) on top of sums of
+    K products in any order."""
+    assert bool(hip.core.sia_gemm_tiles_takes_swiglu(M, inter, K)) == inside
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(2 * inter, K, dtype=torch.bfloat16, seed=2, scale=K ** -0.5)
+    launched, real = [], hip.core.sia_gemm_tiles_swiglu
+    hip.core.sia_gemm_tiles_swiglu = lambda *a: launched.append(1) or real(*a)
+    try:
+        out = hip.gated_linear(x, w)
+    finally:
+        hip.core.sia_gemm_tiles_swiglu = real
+    assert bool(launched) == inside
+    gate, up = (x.float() @ w.float().T).double().split(inter, 1)
+    ref = torch.nn.functional.silu(gate) * up
+    bound = 2.0 ** -8 * (ref.abs() + up.abs() * (gate.abs() * 1.1 + 1e-3) + gate.abs() * up.abs()) + 1e-5
+    assert bool(((out.double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M, N, K, route", [
     (16, 8192, 8192, "own"), (20, 8192, 8192, "own"), (21, 8192, 8192, "library"), (48, 8192, 4096, "own"), (49, 8192, 4096, "library"),
     (32, 20480, 1088, "own"), (32, 20484, 1088, "library"), (32, 20484, 2048, "own"), (33, 10240, 1088, "own"), (33, 10244, 1088, "library"),
