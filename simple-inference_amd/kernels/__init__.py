@@ -595,6 +595,7 @@ class HipKernels:
                 if ones is None or ones.numel() != hidden or ones.device != residual.device:
                     ones = self._ones = torch.ones(hidden, dtype=torch.float32, device=residual.device)
                 return self.linear_into_residual(delta, residual, ones, 0.0).rows     # times a gain of one: x itself
+        if hasattr(delta, "compute"):      # a product not yet computed, or not yet added up
             delta = delta.compute()
         if out_dtype not in _DT:
             raise KernelError(f"output dtype {out_dtype} is not float32 or bfloat16")

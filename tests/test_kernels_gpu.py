@@ -398,6 +398,22 @@ def test_the_norm_that_adds_a_product_s_slices(hip, M, hidden, splits):
     assert torch.equal(a, b) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_a_residual_read_itself_takes_a_product_left_in_slices(hip, dtype):
+    """``ResidualStream.lower`` behind a block that left its last product in slices: as behind one that left the rows."""
+    from simple_inference_amd.kernels import SlicedProduct
+    from simple_inference_amd.parts.context import ResidualStream
+    slices, residual = rnd(3, 70, 64, seed=1), rnd(70, 64, seed=2)
+    out = torch.empty(70, 64, dtype=torch.bfloat16, device=DEV)
+    ways = []
+    for delta in (SlicedProduct(slices, 3, out, hip), hip.sum_slices(slices, 3, torch.empty_like(out))):
+        stream = ResidualStream(residual.clone(), delta)
+        if dtype == torch.float32:
+            stream.settle(hip)
+        ways.append((stream.lower(hip, dtype), stream.residual))
+    assert all(torch.equal(a, b) for a, b in zip(*ways))
+
+
 @pytest.mark.parametrize("shape", [(17, 3072, 3072), (512, 5120, 3072), (2048, 16384, 3072), (130, 3072, 8192),
                                    (33, 1008, 200), (64, 320, 96)])
 def test_library_product_called_directly(hip, shape):
