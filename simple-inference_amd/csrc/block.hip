@@ -90,11 +90,15 @@ struct SiaBlockStep {
         if (rc_ != 0) return rc_;  \
     } while (0)
 
+// Whether this package's products may be asked: a weight that does not begin at a multiple of 16 bytes is the library's.
+static bool may_own(const SiaBlockStep* S, const void* W) { return S->own_products && ((uintptr_t)W & 15) == 0; }
+
 // Y = X W^T by whoever takes a product of this size.
 static int block_product(const SiaBlockStep* S, const void* X, const void* W, void* Y, int N, int K, hipStream_t stream) {
     const int M = S->n_tokens;
-    if (S->own_products && sia_gemm_skinny_takes(M, N, K)) return sia_gemm_skinny(X, W, Y, M, N, K, 0, stream);
-    if (S->own_products && sia_gemm_tiles_takes(M, N, K)) {
+    const bool own = may_own(S, W);
+    if (own && sia_gemm_skinny_takes(M, N, K)) return sia_gemm_skinny(X, W, Y, M, N, K, 0, stream);
+    if (own && sia_gemm_tiles_takes(M, N, K)) {
         SIA_STEP(sia_gemm_tiles(X, W, Y, S->slices, M, N, K, stream));
         const int splits = sia_gemm_tiles_splits(M, N, K);
         return splits > 1 ? sia_sum_slices(S->slices, Y, splits, (long long)M * N, stream) : 0;
@@ -117,7 +121,7 @@ SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, co
     else
         SIA_STEP(sia_add_rmsnorm(S->residual, delta, B->mixer_norm_gain, S->normed, nullptr, M, H, B->mixer_norm_eps,
                                  SIA_BF16, stream));
-    if (S->own_products && B->rotary_dim == B->head_dim && B->head_dim % 2 == 0 && sia_gemm_skinny_takes(M, qkv_width, H)) {
+    if (may_own(S, B->w_qkv) && B->rotary_dim == B->head_dim && B->head_dim % 2 == 0 && sia_gemm_skinny_takes(M, qkv_width, H)) {
         SIA_STEP(sia_gemm_skinny_rope(S->normed, B->w_qkv, S->qkv, M, H, B->cos_table, B->sin_table, S->positions,
                                       S->seq_of_token, block_table, table_width, k_pages, v_pages, B->n_heads, B->n_kv,
                                       B->head_dim, page_size, nullptr, 0, 0.f, stream));
@@ -141,7 +145,8 @@ SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, co
     return 0;
 }
 
-// The whole block.  Leaves its last product in S->fed, not yet added (with S->fed_splits > 1 in slices in S->slices).
+// The whole block.  Leaves its last product in S->fed, not yet added (with S->fed_splits > 1, and a w_down that begins at a multiple
+// of 16 bytes, in slices in S->slices).
 SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, int delta_splits, const int* block_table,
                                  int table_width, void* k_pages, void* v_pages, int page_size, hipStream_t stream) {
     SIA_STEP(sia_prenorm_mixer(B, S, delta, delta_splits, block_table, table_width, k_pages, v_pages, page_size, 1, stream));
@@ -149,15 +154,15 @@ SIA_EXPORT int sia_prenorm_block(const SiaBlockOwn* B, const SiaBlockStep* S, co
     SIA_STEP(block_product(S, S->attended, B->w_o, S->mixed, H, Q, stream));
     SIA_STEP(sia_add_rmsnorm(S->residual, S->mixed, B->feed_forward_norm_gain, S->normed, nullptr, M, H,
                              B->feed_forward_norm_eps, SIA_BF16, stream));
-    if (S->own_products && sia_gemm_skinny_takes_swiglu(M, B->inter, H)) {
+    if (may_own(S, B->w_gate_up) && sia_gemm_skinny_takes_swiglu(M, B->inter, H)) {
         SIA_STEP(sia_gemm_skinny_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, nullptr, 0, 0.f, stream));
-    } else if (S->own_products && sia_gemm_tiles_takes_swiglu(M, B->inter, H)) {
+    } else if (may_own(S, B->w_gate_up) && sia_gemm_tiles_takes_swiglu(M, B->inter, H)) {
         SIA_STEP(sia_gemm_tiles_swiglu(S->normed, B->w_gate_up, S->activated, M, B->inter, H, stream));
     } else {
         SIA_STEP(block_product(S, S->normed, B->w_gate_up, S->gate_up, 2 * B->inter, H, stream));
         SIA_STEP(sia_swiglu(S->gate_up, S->activated, M, B->inter, SIA_BF16, stream));
     }
-    if (S->fed_splits > 1)
+    if (S->fed_splits > 1 && may_own(S, B->w_down))
         SIA_STEP(sia_gemm_tiles(S->activated, B->w_down, S->fed, S->slices, M, H, B->inter, stream));
     else
         SIA_STEP(block_product(S, S->activated, B->w_down, S->fed, H, B->inter, stream));

@@ -108,7 +108,10 @@ struct Epilogue {
 // the gate half and row u of the up half of W), or a pair of columns that the rotation mixes (EPI_ROPE: unit u is
 // column u % (head_dim / 2) of head u / (head_dim / 2) together with the column head_dim / 2 further).  A workgroup
 // owns UNIT_BLOCKS blocks of bh consecutive units from blockIdx.x * UNIT_BLOCKS * bh on.
-template <typename TOut, int EPI, bool SCALED, int RB, int MB, int WAVES, int SLOTS, int WI, int XI>
+// DIRECT: X and W begin at multiples of 16 bytes, as the way straight to LDS needs.  Else every lane loads its own operands, which
+// may begin at any element, into registers, a chunk at a time (the same sums, in one shape; us of 3,072 x 3,072, 8 rows, W 6 bytes
+// beside such a multiple: 13.4, by lines of 128 bytes through registers and LDS 18.3, with a copy of W first 15.4).
+template <typename TOut, int EPI, bool SCALED, int RB, int MB, int WAVES, int SLOTS, int WI, int XI, bool DIRECT>
 __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16_t* __restrict__ X,
                                                                      const bf16_t* __restrict__ W,
                                                                      TOut* __restrict__ Y, int M, int N, int K,
@@ -117,6 +120,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     static_assert(EPI != EPI_ROPE || RB == 2, "the rotation pairs two row blocks");
     static_assert(EPI != EPI_SWIGLU || RB % 2 == 0, "gate and up rows come in equal numbers");
     static_assert((WI == 1 || WI == 2) && (XI == 2 * MB || (MB == 1 && XI == 1)), "tiles of 8 rows");
+    static_assert(DIRECT || (SLOTS == 1 && MB == 1), "a form of up to 16 rows, without a ring");
     static_assert(MB == 1 || (!SCALED && EPI != EPI_RESIDUAL && EPI != EPI_ACT), "forms of up to 16 rows");
     constexpr bool ROUND_FIRST = MB > 1;
     constexpr int THREADS = WAVES * SIA_WAVE;
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     constexpr int LOADS = RB * WI + XI;     // of a step
     constexpr int ROWS = MB * 16;
     // the ring, and when the weights have been read the sums of pairs of shares and a row's sums of squares in its place
-    constexpr int RING = WAVES * SLOTS * LOADS * SK_TILE;
+    constexpr int RING = DIRECT ? WAVES * SLOTS * LOADS * SK_TILE : 0;
     constexpr int PART = 8 * RB * ROWS * 17 * 4, SQUARES = SCALED ? SK_SHARES * 16 * 4 : 0;
     constexpr int LDS = RING > PART + SQUARES ? RING : PART + SQUARES;
     static_assert(LDS <= LL_LDS, "a workgroup's LDS");
@@ -230,7 +234,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
     };
 #pragma unroll
     for (int s = 0; s < SLOTS; ++s)
-        if (s < steps) request(0, s, s);
+        if (DIRECT && s < steps) request(0, s, s);
 
     // what the rotation and the cache write need is on its way beside the weights
     float rope_cos[ROPE_ITER], rope_sin[ROPE_ITER];
@@ -258,8 +262,35 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_skinny_kernel(const bf16
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) acc[j][rb][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (!DIRECT) {
+        const bf16_t* own[RB + 1];   // the lane's rows of W, and of X
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) own[rb] = W + (size_t)row_of(rb, r) * K + g * 16;
+        own[RB] = X + (size_t)min(r, M - 1) * K + g * 16;
+        for (int s0 = 0; s0 < steps; s0 += 2 * SPW)
+#pragma unroll
+            for (int j = 0; j < SPW; ++j) {
+                bf16x8 held[2][RB + 1][2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    if (s0 + 2 * j + u < steps) {
+                        const int k = wave * SK_CHUNK + (s0 / 2 + j) * HOP + u * SK_STEP;
+#pragma unroll
+                        for (int l = 0; l <= RB; ++l) __builtin_memcpy(held[u][l], own[l] + k, 32);
+                    }
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    if (s0 + 2 * j + u < steps) {
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb) {
+                            acc[j][rb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(held[u][rb][0], held[u][RB][0], acc[j][rb][0], 0, 0, 0);
+                            acc[j][rb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(held[u][rb][1], held[u][RB][1], acc[j][rb][0], 0, 0, 0);
+                        }
+                    }
+            }
+    }
     int slot = 0;
-    for (int s0 = 0; s0 < steps; s0 += 2 * SPW) {
+    for (int s0 = 0; DIRECT && s0 < steps; s0 += 2 * SPW) {
 #pragma unroll
         for (int t = 0; t < 2 * SPW; ++t) {
             const int s = s0 + t, j = t / 2;
@@ -532,7 +563,13 @@ static const Shape FEW_ROWS_SHAPES[2][3] = {{{2, 8, 2, false}, {1, 8, 4, true}},
 // grid_of(columns): workgroups of that many columns that the result takes.  (By the rows alone, which cheapest goes by, 12,352
 // columns got five rounds of blocks of 10: 8 rows x 1,024 11.3 us, now 6.6, x 3,072 20.5, now 15.1.  From 120 rows of W a unit on the
 // rounds of up to 8 rows run into each other, and the rows do decide: 32,000 x 4,096, one row, 45 us, by rounds 51.)
-template <typename GridOf> static Cut few_rows_cut(int M, int K, GridOf grid_of) {
+// Without ``direct`` operands there is one shape, of one block.
+template <typename GridOf> static Cut few_rows_cut(int M, int K, bool direct, GridOf grid_of) {
+    if (!direct) {
+        Cut cut = cheapest(grid_of(1), 1, {1});
+        cut.grid = grid_of(cut.bh);
+        return cut;
+    }
     const int columns = grid_of(1);
     if (M <= 8 && columns > 120 * compute_units()) {
         Cut cut = cheapest(columns, 1, {2, 1});
@@ -549,8 +586,8 @@ template <typename GridOf> static Cut few_rows_cut(int M, int K, GridOf grid_of)
     return best;
 }
 
-static Cut few_rows_cut(int M, int K, int N) {
-    return few_rows_cut(M, K, [&](int columns) { return (N + columns - 1) / columns; });
+static Cut few_rows_cut(int M, int K, int N, bool direct = true) {
+    return few_rows_cut(M, K, direct, [&](int columns) { return (N + columns - 1) / columns; });
 }
 
 // How a plain product of up to 16 rows is cut: cut[0] blocks of cut[1] columns a workgroup, cut[2] workgroups, cut[3] of them at a
@@ -572,16 +609,26 @@ struct Product {
     hipStream_t stream;
 };
 
-template <typename TOut, int EPI, bool SCALED, int RB, int MB, int WAVES, int SLOTS, int WI = 2, int XI = 2 * MB>
+template <typename TOut, int EPI, bool SCALED, int RB, int MB, int WAVES, int SLOTS, int WI = 2, int XI = 2 * MB, bool DIRECT = true>
 static void launch(const Product& p, const Cut& cut, const Epilogue& ep) {
-    hipLaunchKernelGGL((gemm_skinny_kernel<TOut, EPI, SCALED, RB, MB, WAVES, SLOTS, WI, XI>), dim3(cut.grid),
+    hipLaunchKernelGGL((gemm_skinny_kernel<TOut, EPI, SCALED, RB, MB, WAVES, SLOTS, WI, XI, DIRECT>), dim3(cut.grid),
                        dim3(WAVES * SIA_WAVE), 0, p.stream, p.X, p.W, (TOut*)p.Y, p.M, p.N, p.K, cut.bh, ep);
+}
+
+// The one shape for up to 16 rows of operands that begin anywhere: RB blocks of weight rows a workgroup.
+template <typename TOut, int EPI, bool SCALED, int RB> static void launch_anywhere(const Product& p, const Cut& cut, const Epilogue& ep) {
+    launch<TOut, EPI, SCALED, RB, 1, 8, 1, 2, 2, false>(p, cut, ep);
 }
 
 // The kernel of a cut whose blocks are columns of Y, up to 16 rows.  Eight waves; the ring as deep as leaves a compute unit one
 // or two workgroups, four steps at most: 64 to 160 KB are then on their way.
 template <typename TOut, int EPI>
 static void launch_columns(const Product& p, const Cut& cut, const Epilogue& ep) {
+    if (!aligned16(p.X, p.W)) {
+        if constexpr (EPI == EPI_RESIDUAL)
+            if (cut.unit_blocks == 2) return launch_anywhere<TOut, EPI, false, 2>(p, cut, ep);
+        return launch_anywhere<TOut, EPI, false, 1>(p, cut, ep);
+    }
     const bool low = cut.bh <= 8;
     if constexpr (EPI != EPI_RESIDUAL)   // (whose cut is by the columns alone, in one block or two)
         if (cut.unit_blocks == 4) return launch<TOut, EPI, false, 4, 1, 8, 1>(p, cut, ep);
@@ -608,7 +655,7 @@ static void launch_more_rows(const Product& p, const Cut& cut) {
 }
 
 template <typename TOut> static void launch_store(const Product& p) {
-    if (p.M <= 16) return launch_columns<TOut, EPI_STORE>(p, few_rows_cut(p.M, p.K, p.N), Epilogue{});
+    if (p.M <= 16) return launch_columns<TOut, EPI_STORE>(p, few_rows_cut(p.M, p.K, p.N, aligned16(p.X, p.W)), Epilogue{});
     const int mb = (p.M + 15) / 16;
     const Cut cut = cheapest(p.N, 1, {4, 2, 1}, mb * 16);
     if (mb == 2) launch_more_rows<TOut, 2>(p, cut);
@@ -620,7 +667,7 @@ template <typename TOut> static void launch_store(const Product& p) {
 SIA_EXPORT int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int N, int K, int out_float,
                                hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > SK_MAX_ROWS || K % 64 || K <= 0 || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
+    if (M > SK_MAX_ROWS || K % 64 || K <= 0 || (M > 16 && !aligned16(X, W))) return SIA_BAD_ARGUMENT;
     const Product p{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream};
     if (out_float)
         launch_store<float>(p);
@@ -633,10 +680,10 @@ SIA_EXPORT int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int
 SIA_EXPORT int sia_gemm_skinny_act(const void* X, const void* W, void* Y, int M, int N, int K, int activation,
                                    hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || !aligned16(X, W) || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU)) return SIA_BAD_ARGUMENT;
+    if (M > 16 || K % 64 || K <= 0 || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU)) return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.activation = activation;
-    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, few_rows_cut(M, K, N), ep);
+    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, few_rows_cut(M, K, N, aligned16(X, W)), ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -645,7 +692,7 @@ SIA_EXPORT int sia_gemm_skinny_embedding_gate(const void* X, const void* W, void
                                               const void* table, int table_width, int first, int dim, const int* ids,
                                               hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || !aligned16(X, W) || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU) ||
+    if (M > 16 || K % 64 || K <= 0 || (activation != SIA_RELU2 && activation != SIA_GELU_TANH && activation != SIA_GELU) ||
         !table || !ids || dim <= 0 || dim > N || first < 0 || first + dim > table_width)
         return SIA_BAD_ARGUMENT;
     Epilogue ep{};
@@ -654,7 +701,7 @@ SIA_EXPORT int sia_gemm_skinny_embedding_gate(const void* X, const void* W, void
     ep.ids = ids;
     ep.table_width = table_width;
     ep.table_dim = dim;
-    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, few_rows_cut(M, K, N), ep);
+    launch_columns<bf16_t, EPI_ACT>(Product{(const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, stream}, few_rows_cut(M, K, N, aligned16(X, W)), ep);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -663,8 +710,8 @@ SIA_EXPORT int sia_gemm_skinny_embedding_gate(const void* X, const void* W, void
 SIA_EXPORT int sia_gemm_skinny_grouped(const void* X, const void* W, void* Y, int M, int K, int groups, int group_rows,
                                        int last_rows, hipStream_t stream) {
     if (M <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || groups <= 0 || group_rows <= 0 || last_rows <= 0 || !X || !W || !Y || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
-    const Cut best = few_rows_cut(M, K, [&](int columns) {
+    if (M > 16 || K % 64 || K <= 0 || groups <= 0 || group_rows <= 0 || last_rows <= 0 || !X || !W || !Y) return SIA_BAD_ARGUMENT;
+    const Cut best = few_rows_cut(M, K, aligned16(X, W), [&](int columns) {
         return (groups - 1) * ((group_rows + columns - 1) / columns) + (last_rows + columns - 1) / columns;
     });
     const int columns = best.unit_blocks * best.bh;
@@ -690,7 +737,7 @@ SIA_EXPORT int sia_gemm_skinny_residual_blocks(int N) {
 SIA_EXPORT int sia_gemm_skinny_residual(const void* X, const void* W, int M, int N, int K, float* residual,
                                         const float* gain, void* scaled, float* partials, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (M > 16 || K % 64 || K <= 0 || !residual || !gain || !scaled || !partials || !aligned16(X, W)) return SIA_BAD_ARGUMENT;
+    if (M > 16 || K % 64 || K <= 0 || !residual || !gain || !scaled || !partials) return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.res = ResidualOut{residual, gain, (bf16_t*)scaled, partials};
     launch_columns<bf16_t, EPI_RESIDUAL>(Product{(const bf16_t*)X, (const bf16_t*)W, nullptr, M, N, K, stream}, cheapest(N, 1, {2, 1}), ep);
@@ -713,8 +760,8 @@ SIA_EXPORT int sia_gemm_skinny_glu(const void* X, const void* W, void* Y, int M,
                                    const float* partials, int n_partials, float eps, int glu, float limit,
                                    const float* bias, hipStream_t stream) {
     if (M <= 0 || inter <= 0) return 0;
-    if (M > SK_MAX_ROWS || (M > 16 && (partials || glu != SIA_GLU_SILU || bias)) || K % 64 || K <= 0 ||
-        (partials && n_partials <= 0) || glu < SIA_GLU_SILU || glu > SIA_GLU_GELU_TANH || !aligned16(X, W))
+    if (M > SK_MAX_ROWS || (M > 16 && (partials || glu != SIA_GLU_SILU || bias || !aligned16(X, W))) || K % 64 || K <= 0 ||
+        (partials && n_partials <= 0) || glu < SIA_GLU_SILU || glu > SIA_GLU_GELU_TANH)
         return SIA_BAD_ARGUMENT;
     Epilogue ep{};
     ep.glu_bias = bias;
@@ -726,8 +773,10 @@ SIA_EXPORT int sia_gemm_skinny_glu(const void* X, const void* W, void* Y, int M,
         // two workgroups a compute unit: one's sums meet while the other's rows come.  Where there is one a unit, it has eight
         // waves (9 rows, four waves / eight: 4,096 x 2,048 7.5 / 6.4 us, 8,192 x 8,192 32 / 29).
         const Cut cut = cheapest(inter, 2, {1});
-        const bool alone = cut.grid <= compute_units();
-        if (M <= 8 && partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 8, 2, 2, 1>(p, cut, ep);
+        const bool alone = cut.grid <= compute_units(), direct = aligned16(X, W);
+        if (!direct && partials) launch_anywhere<bf16_t, EPI_SWIGLU, true, 2>(p, cut, ep);
+        else if (!direct) launch_anywhere<bf16_t, EPI_SWIGLU, false, 2>(p, cut, ep);
+        else if (M <= 8 && partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 8, 2, 2, 1>(p, cut, ep);
         else if (M <= 8) launch<bf16_t, EPI_SWIGLU, false, 2, 1, 8, 2, 2, 1>(p, cut, ep);
         else if (alone && partials) launch<bf16_t, EPI_SWIGLU, true, 2, 1, 8, 3>(p, cut, ep);
         else if (alone) launch<bf16_t, EPI_SWIGLU, false, 2, 1, 8, 3>(p, cut, ep);
@@ -764,9 +813,9 @@ SIA_EXPORT int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M
                                     int n_heads, int n_kv, int head_dim, int page_size, const float* partials,
                                     int n_partials, float eps, hipStream_t stream) {
     if (M <= 0) return 0;
-    if (M > SK_MAX_ROWS || (M > 16 && partials) || K % 64 || K <= 0 || head_dim % 2 || head_dim <= 0 || n_heads <= 0 || n_kv <= 0 || page_size <= 0 ||
+    if (M > SK_MAX_ROWS || (M > 16 && (partials || !aligned16(X, W))) || K % 64 || K <= 0 || head_dim % 2 || head_dim <= 0 || n_heads <= 0 || n_kv <= 0 || page_size <= 0 ||
         table_width <= 0 || !cos_table || !sin_table || !positions || !seq_of_token || !block_table || !k_pages ||
-        !v_pages || (partials && n_partials <= 0) || !aligned16(X, W))
+        !v_pages || (partials && n_partials <= 0))
         return SIA_BAD_ARGUMENT;
     const int heads = n_heads + 2 * n_kv, N = heads * head_dim;
     Epilogue ep{};
@@ -788,9 +837,11 @@ SIA_EXPORT int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M
     }
     // up to 8 rows: two steps leave a compute unit room for two workgroups, three for one (us of 9,216 x 3,072, one row: 13.7 / 14.9)
     const bool pairs = cut.grid > compute_units();
+    const bool direct = aligned16(X, W);
 #define LAUNCH(SCALED)                                                                        \
     do {                                                                                      \
-        if (M <= 8 && low) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 1, 1>(p, cut, ep);    \
+        if (!direct) launch_anywhere<bf16_t, EPI_ROPE, SCALED, 2>(p, cut, ep);                \
+        else if (M <= 8 && low) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 1, 1>(p, cut, ep);    \
         else if (M <= 8) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 2, 1>(p, cut, ep);      \
         else if (low) launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3, 1>(p, cut, ep);            \
         else launch<bf16_t, EPI_ROPE, SCALED, 2, 1, 8, 3>(p, cut, ep);                        \

@@ -264,10 +264,10 @@ class ScaledRows:
     device = property(lambda self: self.rows.device)
 
 
-def _in_pieces(t: torch.Tensor):
-    """``t``, or a copy of it where it does not start at a multiple of 16 bytes: the few-row products bring their operands
-    to LDS in pieces of that size (a view that starts inside another tensor may lie anywhere)."""
-    return t if t.data_ptr() % 16 == 0 else t.clone()
+def _in_pieces(*tensors) -> bool:
+    """Whether all begin at a multiple of 16 bytes: products bring their operands to LDS in pieces of that size.  (A view that
+    begins inside another tensor may lie anywhere; products of up to 16 rows have a form for it, others go to the library.)"""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -623,7 +623,6 @@ class HipKernels:
             raise KernelError(f"{dim} columns from {first_column} on do not fit a table row of {width} and {N} outputs")
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and 0 < M <= self._skinny_rows and K % 64 == 0:
             y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-            x, w = _in_pieces(x), _in_pieces(w)
             self._check(self.core.sia_gemm_skinny_embedding_gate(
                 _ptr(x), _ptr(w), _ptr(y), M, N, K, _ACTIVATIONS[activation], _ptr(table), width, int(first_column),
                 int(dim), _ptr(token_ids), self._stream()), "gemm_skinny_embedding_gate")
@@ -1012,7 +1011,6 @@ class HipKernels:
         most = (groups - 1) * M * rows
         main, low = flat[:most].view(groups - 1, M, rows), flat[most:].view(M, last)
         if self.use_skinny_gemm and x.dtype == torch.bfloat16 and M <= self._skinny_rows and K % 64 == 0:
-            x, w = _in_pieces(x), _in_pieces(w)
             self._check(self.core.sia_gemm_skinny_grouped(_ptr(x), _ptr(w), _ptr(flat), M, K, groups, rows, last,
                                                           self._stream()), "gemm_skinny_grouped")
             return main, low
@@ -1416,21 +1414,18 @@ class HipKernels:
         M, K = x.shape
         N = w.shape[0]
         if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16:
-            if out_float32 and self.use_skinny_gemm and self._tiled_head(M, N, K):
-                x, w = _in_pieces(x), _in_pieces(w)
+            if out_float32 and self.use_skinny_gemm and self._tiled_head(M, N, K) and _in_pieces(x, w):
                 y = torch.empty((M, N), dtype=torch.float32, device=x.device)
                 self._check(self.core.sia_gemm_tiles_head(_ptr(x), _ptr(w), _ptr(y), M, N, K, self._stream()), "gemm_tiles_head")
                 return y
             # few rows: this package's kernel, whose sums do not depend on the number of rows
-            if self.use_skinny_gemm and (M <= self._skinny_rows and K % 64 == 0 or self._own_product(M, N, K)):
+            if self.use_skinny_gemm and (M <= self._skinny_rows and K % 64 == 0 or self._own_product(M, N, K) and _in_pieces(x, w)):
                 y = torch.empty((M, N), dtype=torch.float32 if out_float32 else torch.bfloat16, device=x.device)
-                x, w = _in_pieces(x), _in_pieces(w)
                 self._check(self.core.sia_gemm_skinny(_ptr(x), _ptr(w), _ptr(y), M, N, K, int(out_float32),
                                                       self._stream()), "gemm_skinny")
                 return y
             splits = 0 if out_float32 or not self.use_skinny_gemm else self._tile_splits(M, N, K)
-            if splits:
-                x, w = _in_pieces(x), _in_pieces(w)
+            if splits and _in_pieces(x, w):
                 y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
                 slices = torch.empty((splits, M, N), dtype=torch.float32, device=x.device) if splits > 1 else None
                 self._check(self.core.sia_gemm_tiles(_ptr(x), _ptr(w), _ptr(y), _ptr(slices), M, N, K, self._stream()), "gemm_tiles")
@@ -1468,7 +1463,6 @@ class HipKernels:
                 rows, partials, n_partials, eps = self._scaled(x)      # few rows: the activation inside the product
                 self._want(rows, "gated linear input")
                 y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=rows.device)
-                rows, w_gate_up = _in_pieces(rows), _in_pieces(w_gate_up)
                 self._check(self.core.sia_gemm_skinny_glu(_ptr(rows), _ptr(w_gate_up), _ptr(y), M, two_i // 2, K,
                                                           _ptr(partials), n_partials, eps, glu, limit, _ptr(bias), self._stream()),
                             "gemm_skinny_glu")
@@ -1484,19 +1478,18 @@ class HipKernels:
             return out
         if (self.use_skinny_gemm and x.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16
                 and two_i % 2 == 0 and w_gate_up.shape[1] == K
-                and (M <= self._skinny_rows and K % 64 == 0 or self._own_gate(M, two_i // 2, K))):
+                and (M <= self._skinny_rows and K % 64 == 0 or self._own_gate(M, two_i // 2, K) and _in_pieces(x, w_gate_up))):
             rows, partials, n_partials, eps = self._scaled(x)
             self._want(rows, "gated linear input")
             y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=rows.device)
-            rows, w_gate_up = _in_pieces(rows), _in_pieces(w_gate_up)
             self._check(self.core.sia_gemm_skinny_swiglu(_ptr(rows), _ptr(w_gate_up), _ptr(y), M, two_i // 2, K,
                                                          _ptr(partials), n_partials, eps, self._stream()),
                         "gemm_skinny_swiglu")
             return y
         if (self.use_skinny_gemm and isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and w_gate_up.dtype == torch.bfloat16
-                and two_i % 2 == 0 and w_gate_up.shape[1] == K and self._tiles_gate(M, two_i // 2, K)):
+                and two_i % 2 == 0 and w_gate_up.shape[1] == K and self._tiles_gate(M, two_i // 2, K)
+                and _in_pieces(x, w_gate_up)):
             self._want(x, "gated linear input")
-            x, w_gate_up = _in_pieces(x), _in_pieces(w_gate_up)
             y = torch.empty((M, two_i // 2), dtype=torch.bfloat16, device=x.device)
             self._check(self.core.sia_gemm_tiles_swiglu(_ptr(x), _ptr(w_gate_up), _ptr(y), M, two_i // 2, K, self._stream()),
                         "gemm_tiles_swiglu")
@@ -1523,7 +1516,6 @@ class HipKernels:
         if (self.use_skinny_gemm and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and 0 < M <= self._skinny_rows and K % 64 == 0):
             y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-            x, w = _in_pieces(x), _in_pieces(w)
             self._check(self.core.sia_gemm_skinny_act(_ptr(x), _ptr(w), _ptr(y), M, N, K, _ACTIVATIONS[activation],
                                                       self._stream()), "gemm_skinny_act")
             return y
@@ -1564,7 +1556,6 @@ class HipKernels:
                               f"residual {tuple(residual.shape)}, gain {tuple(gain.shape)}")
         rows = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
         partials = torch.empty((self.core.sia_gemm_skinny_residual_blocks(N), 16), dtype=torch.float32, device=x.device)
-        x, w = _in_pieces(x), _in_pieces(w)
         self._check(self.core.sia_gemm_skinny_residual(_ptr(x), _ptr(w), M, N, K, _ptr(residual), _ptr(gain), _ptr(rows),
                                                        _ptr(partials), self._stream()), "gemm_skinny_residual")
         return ScaledRows(rows, partials, float(eps))
@@ -1718,7 +1709,6 @@ class HipKernels:
             self._check_pages(cache.k_pages, cache.v_pages, cache.block_table, cache.page_size, n_kv_written,
                               head_dim, x.dtype, ctx)
             qkv = torch.empty((M, width), dtype=torch.bfloat16, device=x.device)
-            x, w_qkv = _in_pieces(x), _in_pieces(w_qkv)
             self._check(self.core.sia_gemm_skinny_rope(
                 _ptr(x), _ptr(w_qkv), _ptr(qkv), M, K, _ptr(cos), _ptr(sin), _ptr(ctx.positions),
                 _ptr(ctx.seq_of_token), _ptr(cache.block_table), cache.block_table.shape[1], _ptr(cache.k_pages),
@@ -2091,7 +2081,7 @@ class HipKernels:
             wanted += ((at["cos"], f32, None), (at["sin"], f32, None))
         for t, dtype, shape in wanted:
             if (not isinstance(t, torch.Tensor) or t.device.type != "cuda" or t.dtype != dtype or not t.is_contiguous()
-                    or (shape is not None and tuple(t.shape) != shape) or t.data_ptr() % 16):
+                    or (shape is not None and tuple(t.shape) != shape)):
                 return False
         if (ff["hidden"] != H or n1["size"] != H or n2["size"] != H or D % 16 or D > 256 or not at["scale"] > 0
                 or (rd and (at["cos"].shape[1] != rd // 2 or at["sin"].shape != at["cos"].shape))):
@@ -2186,7 +2176,8 @@ class HipKernels:
         if call is None:
             return False
         self._check(self.core.sia_prenorm_block(*call[0], self._stream()), "prenorm_block")
-        fed, splits = call[1][6], call[2].fed_splits
+        made = block.plain_forms[0]
+        fed, splits = call[1][6], call[2].fed_splits if made.w_down % 16 == 0 else 1
         stream.delta = SlicedProduct(call[1][7], splits, fed, self) if splits > 1 else fed
         return True
 

@@ -398,6 +398,64 @@ def test_the_norm_that_adds_a_product_s_slices(hip, M, hidden, splits):
     assert torch.equal(a, b) and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("rows", [1, 8, 9, 16])
+@pytest.mark.parametrize("N, K", [(64, 64), (1000, 1984), (4100, 3136), (9216, 320)])
+def test_few_row_products_of_weights_that_begin_anywhere(hip, rows, N, K):
+    """A weight inside another tensor is read where it lies, with the bits of a copy that begins at a multiple of 16 bytes: in
+    the plain product, with an activation or a gate, in groups, into the residual, with rotation and cache write."""
+    from simple_inference_amd.kernels import PendingProduct
+    flat = rnd(N * K + 5, dtype=torch.bfloat16, seed=2, scale=K ** -0.5)
+    w = flat[5:].view(N, K)
+    assert w.data_ptr() % 16
+    copy, x = w.clone(), rnd(rows, K, dtype=torch.bfloat16, seed=1)
+    y = torch.empty(rows, N, dtype=torch.bfloat16, device=DEV)
+    assert hip.core.sia_gemm_skinny(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows, N, K, 0, hip._stream()) == 0
+    assert torch.equal(y, hip.linear(x, copy))
+    many = torch.stack([x, x.flip(0), -x])
+    gain, residual = (rnd(N, seed=3) + 1.0).contiguous(), rnd(rows, N, seed=4)
+
+    def into_residual(w):
+        r = residual.clone()
+        scaled = hip.linear_into_residual(PendingProduct(x, w, hip), r, gain, 1e-5)
+        return r, scaled.rows, scaled.partials[:, :rows]
+
+    for call in (lambda w: [hip.linear(x, w, out_float32=True)], lambda w: [hip.activated_linear(x, w, "gelu_tanh")],
+                 lambda w: [hip.gated_linear(x, w)],
+                 lambda w: hip.grouped_linear(many, w, N // 3), into_residual):
+        assert all(torch.equal(a, b) for a, b in zip(call(w), call(copy)))
+    if N in (64, 9216):
+        heads, kv, D = {64: (2, 1, 16), 9216: (24, 24, 128)}[N]
+        ctx = Ctx([1] * rows, [7 + i for i in range(rows)])
+        ang = torch.outer(torch.arange(64, dtype=torch.float32), 1.0 / (10000.0 ** (torch.arange(0, D, 2, dtype=torch.float32) / D)))
+        outs = []
+        for weight in (w, copy):
+            cache = Cache(2 * rows + 1, kv, 16, D, torch.bfloat16, ctx.kv_len.tolist(), seed=6)
+            outs.append((hip.qkv_to_cache(x, weight, heads, kv, D, D, ang.cos().to(DEV), ang.sin().to(DEV), ctx, cache)[:, :heads * D],
+                         cache.k_pages, cache.v_pages))
+        assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+@pytest.mark.parametrize("rows", [17, 40, 64, 100, 300])
+def test_products_of_more_rows_of_weights_that_begin_anywhere_are_the_library_s(hip, rows):
+    """Neither copied nor given to kernels that bring whole pieces to LDS: one product by the library, where it lies."""
+    N, K = 2048, 8192
+    flat = rnd(N * K + 5, dtype=torch.bfloat16, seed=2, scale=K ** -0.5)
+    w, x = flat[5:].view(N, K), rnd(rows, K, dtype=torch.bfloat16, seed=1)
+    went, real = [], {n: getattr(hip.core, n) for n in ("sia_gemm_skinny", "sia_gemm_tiles", "sia_gemm_skinny_swiglu", "sia_gemm_tiles_swiglu")}
+    for n in real:
+        setattr(hip.core, n, lambda *a, n=n: went.append(n) or real[n](*a))
+    try:
+        out, gated = hip.linear(x, w), hip.gated_linear(x, w)
+    finally:
+        for n in real:
+            setattr(hip.core, n, real[n])
+    assert not went
+    assert torch.equal(out, hip._library_product(x, w, False))
+    want = x.double() @ w.double().T    # K roundings of 2^-24 of a sum that stays below 8, and one to bfloat16
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 5e-7 * K).all())
+    assert torch.equal(gated, hip.swiglu(out))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_a_residual_read_itself_takes_a_product_left_in_slices(hip, dtype):
     """``ResidualStream.lower`` behind a block that left its last product in slices: as behind one that left the rows."""

@@ -208,11 +208,9 @@ def test_prompts_of_every_kind_of_product_in_one_call_a_block_and_part_by_part(m
     assert worst <= TOLERANCE["hip-bf16"], f"{worst:.3e}"
 
 
-@pytest.mark.parametrize("hidden, inter", [(2048, 4096), (3072, 4096), (4096, 2048)])
-def test_a_block_in_one_call_at_widths_where_the_gated_tiles_refuse(tmp_path, hidden, inter):
-    """Feed-forwards no wider than the stream: the gated product has no kernel with the activation inside at most numbers of
-    rows, and both ways through a block take the same plain product (tiles, in slices or not, or the library's) and the
-    activation behind it: the same bits."""
+def whole_and_part_by_part(tmp_path, hidden, inter, lengths, change=lambda model: None):
+    """Prompts of these lengths through a small-vocabulary model of these widths, each block in one call and part by part:
+    both ways' logits, and the calls that the first made."""
     from simple_inference_amd.config import EngineConfig
     from simple_inference_amd.engine import build_model
     from simple_inference_amd.weights import random_tensors, write_model_folder
@@ -221,17 +219,46 @@ def test_a_block_in_one_call_at_widths_where_the_gated_tiles_refuse(tmp_path, hi
     model, mcfg = build_model(cfg, EngineConfig(device="cpu", dtype="float32", max_seq_len=64), kernels=None)
     tensors = random_tensors(model.expected_tensors(), seed=9, std=0.02, gain_std=0.1, device="cuda:0")
     folder = write_model_folder(tmp_path, mcfg.to_dict(), tensors)
-    lengths = (40, 65, 97, 150, 204, 300, 600)
     prompts = {i: random_tokens(512, n, seed=700 + n) for i, n in enumerate(lengths)}
-    outs = []
+    outs, calls = [], []
     for whole in (True, False):
         runner, cache, kernels = runner_for(lambda _: (folder,), None, "bfloat16", max_seq_len=1024,
                                             num_pages=sum(-(-n // PAGE) for n in lengths) + 1, max_running=len(lengths))
+        change(runner.model)
         kernels.whole_blocks = whole
-        outs.append(run_schedule(runner, cache, [([(i, t, list(range(len(t))))], []) for i, t in prompts.items()]))
+        real = kernels.core.sia_prenorm_block
+        kernels.core.sia_prenorm_block = lambda *a: calls.append(1) or real(*a)
+        try:
+            outs.append(run_schedule(runner, cache, [([(i, t, list(range(len(t))))], []) for i, t in prompts.items()]))
+        finally:
+            kernels.core.sia_prenorm_block = real
     for i in prompts:
         for place in outs[0][i]:
             assert torch.equal(outs[0][i][place], outs[1][i][place]), (lengths[i], place)
+    return len(calls)
+
+
+@pytest.mark.parametrize("hidden, inter", [(2048, 4096), (3072, 4096), (4096, 2048)])
+def test_a_block_in_one_call_at_widths_where_the_gated_tiles_refuse(tmp_path, hidden, inter):
+    """Feed-forwards no wider than the stream: the gated product has no kernel with the activation inside at most numbers of
+    rows, and both ways through a block take the same plain product (tiles, in slices or not, or the library's) and the
+    activation behind it: the same bits."""
+    assert whole_and_part_by_part(tmp_path, hidden, inter, (40, 65, 97, 150, 204, 300, 600))
+
+
+@pytest.mark.parametrize("moved", [("w_qkv",), ("w_o", "w_down"), ("w_gate_up",)])
+def test_a_block_in_one_call_whose_weights_begin_anywhere(tmp_path, moved):
+    """A weight that lies inside another tensor, not at a multiple of 16 bytes, keeps its block in one call: the product with it
+    goes to the library, its neighbours and the next block (which may find slices, or not) to whom they went."""
+    def change(model):
+        for name in moved:
+            part = next(p for p, _ in model.layers[0].parts if hasattr(p, name))
+            w = getattr(part, name)
+            flat = torch.empty(w.numel() + 3, dtype=w.dtype, device=w.device)
+            flat[3:].copy_(w.flatten())
+            setattr(part, name, flat[3:].view(w.shape))
+    lengths = (20, 50, 97, 300)
+    assert whole_and_part_by_part(tmp_path, 2048, 8192, lengths, change) >= LAYERS * len(lengths)
 
 
 @pytest.mark.parametrize("mode", ["float32", "bfloat16", "bfloat16-unfused"])
