@@ -744,14 +744,6 @@ SIA_EXPORT int sia_gemm_skinny_residual(const void* X, const void* W, int M, int
     return SIA_LAUNCH_CHECK();
 }
 
-// No product gains from a copy of W in another order, now that its rows come to LDS in whole lines: no weight has a tiled form
-// (rows a block of such a copy: none), and the product that would read one refuses.
-SIA_EXPORT int sia_gemm_skinny_tile_height(int) { return 0; }
-SIA_EXPORT int sia_gemm_skinny_residual_tiled(const void*, const void*, int, int, int, float*, const float*, void*, float*,
-                                              hipStream_t) {
-    return SIA_BAD_ARGUMENT;
-}
-
 // Y[M, I] = silu(X Wg^T) * (X Wu^T) for W = [Wg; Wu] of 2 I rows.  Needs M <= 16, K % 64 == 0.
 // With `partials` (else null) X is a `scaled` matrix of sia_gemm_skinny_residual and the rows are divided by their
 // root mean square first.

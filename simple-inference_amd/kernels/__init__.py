@@ -137,8 +137,6 @@ _SIGNATURES = {
     "sia_gemm_skinny_rope": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int,
                              _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_int, _c_float, _c_ptr],
     "sia_gemm_skinny_residual": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
-    "sia_gemm_skinny_residual_tiled": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
-    "sia_gemm_skinny_tile_height": [_c_int],
     "sia_take_rows": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ll, _c_ptr],
     "sia_rows_alone": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_place_tokens": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr],
@@ -1559,11 +1557,6 @@ class HipKernels:
         self._check(self.core.sia_gemm_skinny_residual(_ptr(x), _ptr(w), M, N, K, _ptr(residual), _ptr(gain), _ptr(rows),
                                                        _ptr(partials), self._stream()), "gemm_skinny_residual")
         return ScaledRows(rows, partials, float(eps))
-
-    def prepare_pending_weight(self, w) -> bool:
-        """Whether a copy of a weight that ``pending_linear`` will be given was made in an order of the kernels' own: no,
-        they read every weight as it is."""
-        return False
 
     @staticmethod
     def _scaled(x):

@@ -373,6 +373,32 @@ def test_tiles_of_a_product_of_many_rows(hip, M, N, K):
     assert bool(((gated.double() - ref).abs() <= 2.0 ** -7 * ref.abs() + 2.0 ** -8 * scale * (want[:, N // 2:].abs() + scale)).all())
 
 
+@pytest.mark.parametrize("M, N, K, gated", [(511, 16384, 2048, True), (821, 16384, 2048, True), (1023, 16384, 3072, True),
+                                            (1024, 16384, 3072, True), (450, 3072, 8192, False), (769, 3072, 8192, False),
+                                            (1023, 4096, 14336, False), (600, 4096, 14336, False)])
+def test_the_largest_tiles_over_long_k(hip, M, N, K, gated):
+    """Tiles of 128 x 256 and 256 x 256 through many rounds of their shallow rings, the gated form in one slice and the plain
+    one in several, rows that are no multiple of a tile.  Bounds as below (values around 1 in K products)."""
+    x, w = rnd(M, K, dtype=torch.bfloat16, seed=1), rnd(N, K, dtype=torch.bfloat16, seed=2, scale=K ** -0.5)
+    want = x.double() @ w.double().T
+    if gated:
+        out = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert hip.core.sia_gemm_tiles_swiglu(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N // 2, K, hip._stream()) == 0
+        gate, up = want.split(N // 2, 1)
+        ref = torch.nn.functional.silu(gate) * up
+        bound = 2.0 ** -8 * (ref.abs() + up.abs() * (gate.abs() * 1.1 + 1e-3) + gate.abs() * up.abs()) + 1e-5
+        assert bool(((out.double() - ref).abs() <= bound).all())
+        return
+    splits = hip.core.sia_gemm_tiles_splits(M, N, K)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    slices = torch.full((splits, M, N), float("nan"), device=DEV)
+    assert hip.core.sia_gemm_tiles(x.data_ptr(), w.data_ptr(), out.data_ptr(), slices.data_ptr(), M, N, K, hip._stream()) == 0
+    if splits > 1:      # K roundings of 2^-24 of a sum that stays below 8
+        assert float((slices.double().sum(0) - want).abs().max()) <= 5e-7 * K
+        hip.sum_slices(slices, splits, out)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 5e-7 * K).all())
+
+
 @pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 128])
 @pytest.mark.parametrize("N, K", [(32768, 64), (32900, 192), (40004, 1088)])
 def test_tiles_of_an_output_head(hip, M, N, K):
@@ -960,38 +986,25 @@ def test_few_row_products_do_not_depend_on_the_number_of_rows(hip):
 
 
 @pytest.mark.parametrize("N, K", [(3072, 3072), (3070, 8192), (2048, 2048), (4099, 192)])
-def test_a_tiled_copy_of_a_weight_changes_no_bit_of_the_product_into_the_residual(hip, N, K):
-    """The product into the residual reads, where the kernels made one, a copy of the weight laid out in the order
-    of its loads.  The same elements meet in the same sums: residual, scaled rows and sums of squares are the same
-    bit for bit as from the weight as it is, for every number of rows, also where the last block of rows is short
-    (3,070 and 4,099 rows).  A weight changed in place after the copy was made is read as it is."""
+def test_the_product_into_the_residual_reads_the_weight_as_it_is(hip, N, K):
+    """Residual, scaled rows and sums of squares against the product in 64 bits, also where the last block of rows is short
+    (3,070 and 4,099 rows), and again when the weight has been changed in place: nothing of it is kept."""
     dtype = torch.bfloat16
     x = rnd(16, K, dtype=dtype, seed=1)
     w = rnd(N, K, dtype=dtype, seed=2, scale=K ** -0.5)
     res = rnd(16, N, seed=3, scale=2.0)
     gain = (rnd(N, seed=4, scale=0.3) + 1.0).contiguous()
-
-    def through(m):
-        r = res[:m].clone()
-        scaled = hip.linear_into_residual(hip.pending_linear(x[:m].contiguous(), w), r, gain, 1e-5)
-        return r, scaled.rows, scaled.partials[:, :m].clone()
-
-    plain = {m: through(m) for m in (1, 7, 16)}
-    made = hip.prepare_pending_weight(w)
-    assert made == (hip.core.sia_gemm_skinny_tile_height(N) > 0)
-    for m, want in plain.items():
-        for got, expected in zip(through(m), want):
-            assert torch.equal(got, expected), (N, K, m)
-    if made:
-        assert hip._tiled_copy(w) is not None
-        w.mul_(2.0)                                    # the copy no longer says what the weight holds
-        assert hip._tiled_copy(w) is None
-        r, rows, _ = through(5)
-        want = res[:5] + (x[:5].float() @ w.float().T).to(dtype).float()
-        torch.testing.assert_close(r, want, atol=2e-2, rtol=2e-2)
-        assert hip.prepare_pending_weight(w) and hip._tiled_copy(w) is not None
-        for got, expected in zip(through(5), (r, rows)):
-            assert torch.equal(got, expected)
+    for _ in range(2):
+        product = x.double() @ w.double().T
+        for m in (1, 7, 16):
+            r = res[:m].clone()
+            scaled = hip.linear_into_residual(hip.pending_linear(x[:m].contiguous(), w), r, gain, 1e-5)
+            # the product is rounded to bfloat16 (2^-9 of it, and what its float sums leave), the sum to 32 bits
+            want = res[:m].double() + product[:m]
+            assert bool(((r.double() - want).abs() <= 2.0 ** -8 * product[:m].abs() + 5e-7 * K).all())
+            assert torch.equal(scaled.rows, (r * gain).to(dtype))
+            torch.testing.assert_close(scaled.partials[:, :m].double().sum(0), r.double().square().sum(1), rtol=1e-5, atol=0)
+        w.mul_(2.0)
 
 
 @pytest.mark.parametrize("q_len, kv_len, window", [(130, 130, None), (900, 1000, None), (1900, 1900, None),

@@ -3,8 +3,8 @@
 Two layers of each of the three shapes the presets name (the widths, head counts, head sizes, vocabulary and
 frequency scaling of the 3B, 1B and 8B models; fewer layers, so that the plain implementation on the CPU takes
 seconds), with seeded random weights, in float32 and in bfloat16.  At these widths the engine takes the paths the
-tiny models never reach together: the few-row products with fused epilogues at K of 3,072 to 14,336 in their
-16-wave shapes, the BLAS library from 17 rows on, the matrix-core attention of head sizes 128 and 64 with groups
+tiny models never reach together: the few-row products with fused epilogues at K of 3,072 to 14,336, this package's
+products and the BLAS library's from 17 rows on, each where it is the faster, the matrix-core attention of head sizes 128 and 64 with groups
 of 3 and 4, key splits of 1 to 8 workgroups, a vocabulary of 128,256 (reference:
 ``benchmarks/bench_paged_cudagraph.py:236-264`` compares its fast path's logits at the real model the same way).
 """
@@ -246,7 +246,7 @@ def test_a_block_in_one_call_at_widths_where_the_gated_tiles_refuse(tmp_path, hi
     assert whole_and_part_by_part(tmp_path, hidden, inter, (40, 65, 97, 150, 204, 300, 600))
 
 
-@pytest.mark.parametrize("moved", [("w_qkv",), ("w_o", "w_down"), ("w_gate_up",)])
+@pytest.mark.parametrize("moved", [(), ("w_qkv",), ("w_o", "w_down"), ("w_gate_up",)])
 def test_a_block_in_one_call_whose_weights_begin_anywhere(tmp_path, moved):
     """A weight that lies inside another tensor, not at a multiple of 16 bytes, keeps its block in one call: the product with it
     goes to the library, its neighbours and the next block (which may find slices, or not) to whom they went."""
@@ -257,7 +257,7 @@ def test_a_block_in_one_call_whose_weights_begin_anywhere(tmp_path, moved):
             flat = torch.empty(w.numel() + 3, dtype=w.dtype, device=w.device)
             flat[3:].copy_(w.flatten())
             setattr(part, name, flat[3:].view(w.shape))
-    lengths = (20, 50, 97, 300)
+    lengths = (20, 50, 97, 300, 820)
     assert whole_and_part_by_part(tmp_path, 2048, 8192, lengths, change) >= LAYERS * len(lengths)
 
 
@@ -265,7 +265,7 @@ def test_a_block_in_one_call_whose_weights_begin_anywhere(tmp_path, moved):
 def test_steps_of_1_8_16_17_and_64_single_tokens_at_3b_widths(models, mode):
     """64 requests with prompts of 3 to 34 tokens decode together, then 17, 16, 8 and one of them: a step of up to
     16 rows takes this package's products (with the fused epilogues, or, in the third mode, without: product,
-    rotation and cache write, norm and activation as kernels of their own), from 17 rows on the BLAS library."""
+    rotation and cache write, norm and activation as kernels of their own), from 17 rows on this package's or the library's."""
     dtype = "float32" if mode == "float32" else "bfloat16"
     _, cfg, _ = models("3b")
     vocab = cfg["vocab_size"]
