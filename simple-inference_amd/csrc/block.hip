@@ -1,9 +1,10 @@
 // One pre-norm block (attention with rotation over the paged cache, SwiGLU feed-forward, RMS norms) of a step of
 // many rows, as one call: the launches that the parts' own calls would make one by one, in the same order, on the
-// same buffers.  In steps of up to 64 rows the rotation with the cache write and the activation are epilogues of this package's
-// products, which round first and give the bits of the kernels that they replace.  Nothing is computed here; it spares the host the way through the interpreter between the launches,
-// which in a step of a few hundred tokens of a small model takes longer than the GPU needs for them.  The matrix
-// products and the matrix-core attention live in other libraries: the caller hands their entry points in.
+// same buffers.  Where this package's products take a step's, the rotation with the cache write and the activation are their
+// epilogues, which round first and give the bits of the kernels that they replace.  Nothing is computed here; it spares
+// the host the way through the interpreter between the launches, which in a step of a few hundred tokens of a small model
+// takes longer than the GPU needs for them.  The BLAS library's products and the matrix-core attention live in other
+// libraries: the caller hands their entry points in.
 #include "common.h"
 
 extern "C" {
@@ -106,8 +107,8 @@ static int block_product(const SiaBlockStep* S, const void* X, const void* W, vo
     return S->product(X, W, Y, M, N, K, 0, stream);
 }
 
-// residual += delta (where there is one; with delta_splits > 1 it lies in that many slices in S->slices); then the block up to its attention, whose results are left in S->attended, or
-// without ``attend`` up to its projected rows, which are left in S->qkv with keys and values in the pages: what a caller that
+// residual += delta (where there is one; with delta_splits > 1 it lies in that many slices in S->slices); then the block up to
+// its attention, whose results are left in S->attended, or without ``attend`` up to its projected rows, which are left in S->qkv with keys and values in the pages: what a caller that
 // goes on with some rows alone needs of all of them.
 // block_table [n_seqs, table_width], k_pages, v_pages: the block's cache in this step.  0, or the first launch's error.
 SIA_EXPORT int sia_prenorm_mixer(const SiaBlockOwn* B, const SiaBlockStep* S, const void* delta, int delta_splits, const int* block_table,

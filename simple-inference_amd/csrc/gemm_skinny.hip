@@ -17,14 +17,14 @@
 // not the memory, sets the pace.  us a launch, everything from memory, before -> now:  gate/up with SwiGLU of 8,192 x 2,048
 // 17.7 -> 14.4, x 3,072 21.0 -> 19.8, 14,336 x 4,096 50 -> 42.5;  2,048 x 8,192 11.1 -> 8.2, 3,072 x 8,192 12.3 -> 10.7;  a read of
 // the same bytes that does nothing else takes 12.1, 19.2, 42; 7.6, 10.2.  A second copy of W in the order of the loads gains nothing
-// over this.)
+// over this at these widths; over k of 11,008 it took 18.5 for 4,096 columns where this takes 21.5, over 8,192 14.3 and 15.6.)
 //   Inside a 1 KiB tile of 8 rows the 16-byte pieces of a row are permuted by the row's number (the lane that writes place p
 // of row r fetches piece p ^ turn(r)), so that the 16 lanes that a 128-bit LDS read serves at a time meet no bank twice.
 //
 // X is fetched once per workgroup (L2 serves it); a workgroup whose rows are few against X's takes more of them at once.
 // A product is as fast as the busiest compute unit: a block holds `bh` <= 16 rows, chosen on the host so that
-// the workgroups come out as a whole number of rounds over the compute units (3,072 rows on 256 units: 256
-// blocks of 12, not 192 of 16).  Rows beyond the block, and rows m >= M of X, are the last live one again (the same cache
+// the workgroups come out as whole rounds over the compute units, of as many at a time as LDS holds (3,072 rows on
+// 256 units: 256 blocks of 12, not 192 of 16).  Rows beyond the block, and rows m >= M of X, are the last live one again (the same cache
 // lines, no further traffic), or not fetched where a whole tile of 8 is beyond; what the MFMAs make of them is never stored.
 //
 // The result element (m, n) is summed over k in an order that depends on K only, not on M, the other rows,
@@ -663,7 +663,8 @@ template <typename TOut> static void launch_store(const Product& p) {
     else launch_more_rows<TOut, 4>(p, cut);
 }
 
-// out_float: 1 -> Y is float, 0 -> bfloat16.  Needs M <= 64, K % 64 == 0.
+// out_float: 1 -> Y is float, 0 -> bfloat16.  Needs K % 64 == 0 and M <= 16, or M <= 64 for operands that begin at multiples of
+// 16 bytes.
 SIA_EXPORT int sia_gemm_skinny(const void* X, const void* W, void* Y, int M, int N, int K, int out_float,
                                hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
@@ -744,7 +745,9 @@ SIA_EXPORT int sia_gemm_skinny_residual(const void* X, const void* W, int M, int
     return SIA_LAUNCH_CHECK();
 }
 
-// Y[M, I] = silu(X Wg^T) * (X Wu^T) for W = [Wg; Wu] of 2 I rows.  Needs M <= 16, K % 64 == 0.
+// Y[M, I] = silu(X Wg^T) * (X Wu^T) for W = [Wg; Wu] of 2 I rows.  Needs K % 64 == 0 and M <= 16, or M <= 64 for operands that
+// begin at multiples of 16 bytes, without partials or bias and with silu.  Up to 16 rows the activation is of the float sums; with
+// more they are rounded to bfloat16 first (the bits of the product and the activation kernel).
 // With `partials` (else null) X is a `scaled` matrix of sia_gemm_skinny_residual and the rows are divided by their
 // root mean square first.
 // glu, limit: another gated activation than silu(gate) * up (SiaGlu of common.h); bias: [2 I] floats or null.
@@ -795,10 +798,12 @@ SIA_EXPORT int sia_gemm_skinny_swiglu(const void* X, const void* W, void* Y, int
     return sia_gemm_skinny_glu(X, W, Y, M, inter, K, partials, n_partials, eps, SIA_GLU_SILU, 0.f, nullptr, stream);
 }
 
-// The q/k/v product of single-token steps with the rotation and the cache write in its epilogue:
+// The q/k/v product of few tokens with the rotation and the cache write in its epilogue:
 // W = [q heads | k heads | v heads], head_dim even, every dim of a head rotates (tables of head_dim / 2 floats
 // a position).  Rotated q goes to Y[M][(n_heads + 2 n_kv) head_dim] (its k and v columns are not written); rotated
-// k and v go to the pages at each token's position.  Needs M <= 16, K % 64 == 0.  `partials` as above.
+// k and v go to the pages at each token's position.  Needs K % 64 == 0 and M <= 16, or M <= 64 for operands that begin at
+// multiples of 16 bytes and without partials.  Up to 16 rows the float sums are rotated; with more they are rounded to bfloat16
+// first (the bits of the product and the rotation kernel).  `partials` as above.
 SIA_EXPORT int sia_gemm_skinny_rope(const void* X, const void* W, void* Y, int M, int K, const float* cos_table,
                                     const float* sin_table, const int* positions, const int* seq_of_token,
                                     const int* block_table, int table_width, void* k_pages, void* v_pages,

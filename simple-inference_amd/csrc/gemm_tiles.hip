@@ -1,4 +1,4 @@
-// Y[M, N] = X[M, K] * W[N, K]^T in bfloat16 with float accumulation, for steps of some 33 to 1,024 rows: too many to walk along W
+// Y[M, N] = X[M, K] * W[N, K]^T in bfloat16 with float accumulation, for steps of some 21 to 1,024 rows: too many to walk along W
 // with all of X beside it (gemm_skinny.hip), too few for tiles of whole k to fill the chip, which is where the BLAS library loses
 // (3,072 x 8,192: 43 us at 128 rows and 59 at 192, where the weights' bytes take 8).
 //

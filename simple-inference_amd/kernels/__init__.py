@@ -328,7 +328,7 @@ class HipKernels:
         self.whole_blocks = True         # many rows: a block's launches in one call (``prenorm_block``)
         self._products_known: Dict[tuple, bool] = {}
         self._skinny_rows = self.core.sia_gemm_skinny_max_rows()      # all forms of the few-row products
-        self._skinny_most = self.core.sia_gemm_skinny_most_rows()     # the plain and the gated one
+        self._skinny_most = self.core.sia_gemm_skinny_most_rows()     # the plain one, SwiGLU and the rotation, within limits
         self._own_known: Dict[tuple, bool] = {}
         self.blas = self._load_blas()    # the BLAS library called directly; None: its products go through torch
 
