@@ -471,9 +471,9 @@ SIA_EXPORT int sia_gemm_skinny_takes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 || M > SK_MAX_ROWS) return 0;
     if (M <= 16) return 1;
     if (sia_gemm_tiles_takes(M, N, K)) return 0;
-    if (N % 8192 == 0 && (M > 48 ? K >= 4096 : M > 20 && K % 8192 == 0)) return 0;
+    if (N % (8 * 1024) == 0 && (M > 48 ? K >= 4 * 1024 : M > 20 && K % (8 * 1024) == 0)) return 0;
     if (M <= 32) return N <= 20 * 1024 || K % 2048 == 0;
-    if (N > 10 * 1024 || (K > 5 * 1024 && N < 1536) || (K > 6 * 1024 && N < 3072)) return 0;
+    if (N > 10 * 1024 || (K > 5 * 1024 && N < 1536) || (K > 6 * 1024 && N < 3 * 1024)) return 0;
     return M <= 48 || (K <= 8 * 1024 && (N < 6 * 1024 || K < 5 * 1024));
 }
 
@@ -489,7 +489,7 @@ SIA_EXPORT int sia_gemm_skinny_takes_swiglu(int M, int inter, int K) {
     if (M <= 0 || inter <= 0 || K <= 0 || K % 64 || M > SK_MAX_ROWS) return 0;
     if (M <= 16) return 1;
     if (K % 2048 && (M > 48 ? inter > 8704 && (K > 2048 || inter > 10 * 1024) : M > 32 && inter > 10 * 1024)) return 0;
-    return inter >= 4608 || K <= 2048 || (inter >= 2560 ? K <= 3072 || (K <= 5120 && M <= 48) : K <= 5120 && M <= 32);
+    return inter >= 4608 || K <= 2048 || (inter >= 2560 ? K <= 3 * 1024 || (K <= 5 * 1024 && M <= 48) : K <= 5 * 1024 && M <= 32);
 }
 
 // How a product is cut into workgroups: `unit_blocks` blocks of `bh` units each, `grid` workgroups.

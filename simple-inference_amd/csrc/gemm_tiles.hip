@@ -268,7 +268,7 @@ SIA_EXPORT int sia_gemm_tiles_takes(int M, int N, int K) {
         return (size >= 12 * MI && (M > 80 || N >= 2048)) || (K >= 9 * 1024 && N >= 1024);
     }
     if (M <= 64 || M > 256 || size < 15 * MI) return 0;
-    return N <= 6 * 1024 || (N <= 8 * 1024 && (M > 160 || K > 8 * 1024 || (M <= 128 && K > 4 * 1024 && K % 8192)));
+    return N <= 6 * 1024 || (N <= 8 * 1024 && (M > 160 || K > 8 * 1024 || (M <= 128 && K > 4 * 1024 && K % (8 * 1024))));
 }
 
 // The same for the gated product: where its tiles come out in one round that fills at least 9/10 of the compute units with
@@ -283,7 +283,7 @@ SIA_EXPORT int sia_gemm_tiles_takes_swiglu(int M, int inter, int K) {
     const TilePlan plan = tile_plan(M, inter, K, true);
     const long long cus = compute_units();
     const TileShape t = TILE_SHAPES[plan.shape];
-    if (K > 3072 && (M <= 128 || M > 256 || (sia_gemm_tiles_takes(M, 2 * inter, K) && (inter < 4096 || K > 4096)))) return 0;
+    if (K > 3 * 1024 && (M <= 128 || M > 256 || (sia_gemm_tiles_takes(M, 2 * inter, K) && (inter < 4 * 1024 || K > 4 * 1024)))) return 0;
     return plan.workgroups <= cus && 10 * plan.workgroups >= 9 * cus && 5LL * M * 2 * inter >= 4 * cus * t.bm * t.bn;
 }
 
