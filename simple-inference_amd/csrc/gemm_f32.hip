@@ -1,298 +1,732 @@
-// Y[M, N] = X[M, K] * W[N, K]^T in float on the matrix cores: the product of the 32-bit path.
+// Y[M, N] = X[M, K] * W[N, K]^T in float: the product of the 32-bit path, on the bfloat16 matrix cores.
 //
-// v_mfma_f32_16x16x4_f32 multiplies and adds floats as they are (no reduced-precision mode): 157 TFLOP/s where the
-// vector units give the plain kernel 24.
+// A float of 24 bits is the sum of three bfloat16 numbers, exactly: x0 = x rounded, x1 = (x - x0) rounded, x2 = x - x0 - x1.
+// (Parts below 2^-133 vanish: of numbers under 2^-110 the last bits.)  A product of two parts is exact in float, and of the nine
+// products of parts the six above 2^-24 of the whole are summed: x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0.  The matrix cores
+// multiply bfloat16 sixteen times as fast as float, so six products are 2.7 times as fast, and weights that are
+// bfloat16 numbers kept in 32 bits (a checkpoint's) have parts w1 = w2 = 0 and need three.
 //
-// One order of sums for every shape, whatever M is, so that a row's result does not depend on the other rows of a
-// batch or on which kernel below runs:  K is cut into steps of 64; a step's four pieces of 16 go to four sums
-// s0 .. s3, piece by piece in order; within a piece instruction i = 0 .. 3 adds the k = 4 q + i of q = 0 .. 3 at once.
-// The result is (s0 + s1) + (s2 + s3).  Shorter chains than k after k: the error against 64 bits is smaller.
+// The order of sums, the same for every shape, whatever M is, so that a row's result does not depend on the other rows of a
+// batch or on which kernel below runs:  a chunk of 32 k is summed from zero, its small products first (v_mfma_f32_16x16x32_bf16),
+// and the chunks' sums are added in order.  Where N is small, K is cut into slices that N and K alone decide
+// (slices_of), and the slices' sums are added in order.  Short chains and small terms first: the error against 64 bits is below
+// that of v_mfma_f32_16x16x4_f32 in four chains, which this replaces (2-norm, normal operands of 24 bits, k of 64, 512, 2,048, 8,192
+// and 14,336: 8.4e-8, 2.0e-7, 4.1e-7, 8.1e-7, 1.1e-6 -> 5e-8, 8e-8, 1.0e-7, 1.6e-7, 2.1e-7).  Leaving out the products of w1 and w2 where all
+// of them are zero changes no bit: they add zero.
 //
-// * Up to 16 rows: a workgroup owns 16 rows of W; its four waves take a sum each and stream W past the step's rows,
-//   eight to sixteen steps of loads in flight a wave.  Bound by reading W.
-// * More rows: tiles of Y.  A workgroup has the waves of a tile four times, once per sum; X and W are staged through
-//   LDS in steps of 64 k.  Bound by the matrix cores.
-#include "common.h"
+// Infinities and NaN, and finite numbers that round to an infinite part: some product of parts is then not finite, and neither is
+// the result.  A result that is not finite is made again, k after k with fused multiply-adds (plain_sum).
+//
+// * Few rows: a workgroup's waves stream W past the step's rows.  Bound by reading W, or by what the workgroups fetch from L2.
+// * More rows: X is split into its parts ahead, once, in the order in which the matrix cores read it; tiles of Y, X's parts and W as it
+//   is staged through LDS by loads that pass no registers, W split where it is read.  Neither loads alone (217 of 337 us at 303 rows,
+//   65,536 columns and k of 2,048) nor products and LDS reads alone (195 to 215) take the time: what is left is what the two do not share.
+// us, v_mfma_f32_16x16x4_f32 -> now, weights of 8 bits and of 24:  303 rows x 128,256 x 2,048 1,461 -> 640 and 1,040, x 16,384 x 2,048 206 -> 107
+// and 163, x 2,048 x 8,192 146 -> 68 and 96, x 3,072 x 2,048 42 -> 35 and 44;  one row x 2,048 x 2,048 9.2 -> 6.0 and 7.3, x 2,048 x 8,192 26.6 -> 19.5
+// and 22.5, x 28,672 x 4,096 105 -> 95 and 102;  64 rows x 2,048 x 2,048 11.7 -> 8.0 and 9.6.  Slower: weights of 24 bits at 17 to 32 rows
+// of 16,384 x 2,048 (34 -> 37), rows that begin anywhere at 200 to 600 rows of 1,000 x 333 (10.4 -> 13.6).
+#include "lds_load.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-#define SUMS 4            // sums a result is made of
-#define PIECE 16          // consecutive k of a sum
-#define STEP (SUMS * PIECE)
+constexpr int CHUNK = 32;      // k that are summed from zero
+constexpr int PARTS = 3;
+constexpr int PART_BLOCK = PARTS * SIA_WAVE;      // 16-byte pieces of the parts of 16 rows of X in a chunk
 
-__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
+// ---------------------------------------------------------------------------------------------------------
+// parts and products
+// ---------------------------------------------------------------------------------------------------------
 
-__device__ __forceinline__ f32x4 sum_of_piece(f32x4 w, f32x4 x, f32x4 c) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) c = mfma4(w[i], x[i], c);
-    return c;
-}
-
-// Four consecutive floats at p, a row's floats from k on (p points at float k).  ALIGNED: K is a multiple of four and the
-// rows start on 16 bytes, so that the four lie inside or outside the row together; outside, the row's last four are read,
-// without a branch, for in_row() to turn into zeros where they are used (not here: a use is a wait for the load).
-template <bool ALIGNED>
-__device__ __forceinline__ f32x4 load4(const float* __restrict__ p, int k, int K) {
-    if (ALIGNED) return *(const f32x4*)(p + min(0, K - 4 - k));
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (k + i < K) v[i] = p[i];
+// a and b as bfloat16, rounded to nearest, a in the low half
+__device__ __forceinline__ uint32_t round_pair(float a, float b) {
+    uint32_t v;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(v) : "v"(a), "v"(b));
     return v;
 }
 
-__device__ __forceinline__ f32x4 in_row(f32x4 v, int k, int K) { return k < K ? v : f32x4{0.f, 0.f, 0.f, 0.f}; }
-
-// The four results of a lane: row `m` of Y, columns n .. n + 3.
-__device__ __forceinline__ void store4(float* __restrict__ Y, int m, int n, int M, int N, bool whole, f32x4 v) {
-    if (m >= M) return;
-    float* at = Y + (size_t)m * N + n;
-    if (whole && n + 3 < N) {
-        *(f32x4*)at = v;
-        return;
-    }
+// The parts of eight consecutive floats, each eight bfloat16 in order.
+__device__ __forceinline__ void split8(u32x4 first, u32x4 second, u32x4 (&part)[PARTS]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (n + i < N) at[i] = v[i];
+    for (int e = 0; e < 4; ++e) {
+        const u32x4& v = e < 2 ? first : second;
+        float a = __uint_as_float(v[2 * (e & 1)]), b = __uint_as_float(v[2 * (e & 1) + 1]);
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+            const uint32_t r = round_pair(a, b);
+            part[p][e] = r;
+            a -= __uint_as_float(r << 16), b -= __uint_as_float(r & 0xffff0000u);
+        }
+    }
 }
+
+// The first part of eight floats that have no other.
+__device__ __forceinline__ u32x4 upper_halves(u32x4 a, u32x4 b) {
+    return u32x4{__builtin_amdgcn_perm(a[1], a[0], 0x07060302), __builtin_amdgcn_perm(a[3], a[2], 0x07060302),
+                 __builtin_amdgcn_perm(b[1], b[0], 0x07060302), __builtin_amdgcn_perm(b[3], b[2], 0x07060302)};
+}
+
+__device__ __forceinline__ uint32_t or_of(u32x4 a, u32x4 b) { return (a[0] | a[1] | a[2] | a[3]) | (b[0] | b[1] | b[2] | b[3]); }
+
+__device__ __forceinline__ f32x4 product(u32x4 w, u32x4 x, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), c, 0, 0, 0);
+}
+
+// The sum of a chunk's products of a block of 16 rows of X with TN blocks of 16 rows of W.  The blocks alternate: a product is done
+// when the next one that adds to it begins.
+template <int TN>
+__device__ __forceinline__ void chunk_one_part(const u32x4 (&w0)[TN], const u32x4 (&x)[PARTS], f32x4 (&t)[TN]) {
+#pragma unroll
+    for (int p = PARTS - 1; p >= 0; --p)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) t[j] = product(w0[j], x[p], p == PARTS - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : t[j]);
+}
+
+template <int TN>
+__device__ __forceinline__ void chunk_of_parts(const u32x4 (&w)[TN][PARTS], const u32x4 (&x)[PARTS], f32x4 (&t)[TN]) {
+    constexpr int ORDER[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};      // parts of W and X, small products first
+#pragma unroll
+    for (int o = 0; o < 6; ++o)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) t[j] = product(w[j][ORDER[o][0]], x[ORDER[o][1]], o == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : t[j]);
+}
+
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
+
+__device__ __forceinline__ float plain_sum(const float* __restrict__ x, const float* __restrict__ w, int K) {
+    float s = 0.f;
+    for (int k = 0; k < K; ++k) s = fmaf(x[k], w[k], s);
+    return s;
+}
+
+// Slices of K, in chunks: from N and K alone.  Few rows of W beside a long K are too little for the chip without; an output head
+// is enough, and its tiles then need no second sum.
+__host__ __device__ static inline int slices_of(int N, int K) { return N > 32 * 1024 || K <= 4 * CHUNK ? 1 : N > 12 * 1024 ? 2 : 8; }
+__device__ __forceinline__ int slice_begin(int chunks, int slice, int slices) { return (int)((long long)chunks * slice / slices); }
 
 // ---------------------------------------------------------------------------------------------------------
 // few rows
 // ---------------------------------------------------------------------------------------------------------
 
-#define FLIGHT 8   // steps of loads that a wave has issued before it multiplies the eight in front of them
+// A workgroup has MB blocks of 16 rows of X and WAVES / SLICES groups of NB blocks of 16 rows of W; a wave has a slice of K of one group.
+// A wave's step is U chunks, whose sums do not depend on one another.  W's and X's rows come to LDS directly as they are, 128 bytes of eight
+// rows an instruction, into a ring of SLOTS steps that the wave has for itself, and are split where they are read.  (Loaded into registers,
+// an instruction touches 16 lines in pieces of 16 bytes: see gemm_skinny.hip.)  XI: tiles of 8 rows of X, 2 MB or 1.
+// DIRECT: rows begin at multiples of 16 bytes and K is a multiple of 4.  Else operands are read float by float, into registers.
+template <int SLICES, int WAVES, int MB, int NB, int XI, int U, int SLOTS, bool DIRECT>
+__global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(const float* __restrict__ X, const float* __restrict__ W,
+                                                                            float* __restrict__ Y, int M, int N, int K) {
+    static_assert(WAVES % SLICES == 0, "a wave a slice");
+    constexpr int GROUPS = WAVES / SLICES;
+    static_assert(XI == 2 * MB || (MB == 1 && XI == 1), "tiles of 8 rows");
+    constexpr int CHUNK_LOADS = 2 * NB + XI, LOADS = U * CHUNK_LOADS;
+    constexpr int RING = DIRECT ? WAVES * SLOTS * LOADS * LL_TILE : 0, SUMS = SLICES > 1 ? WAVES * MB * NB * 256 * 4 : 0;
+    constexpr int LDS = RING > SUMS ? RING : SUMS > 0 ? SUMS : 16;
+    static_assert(LDS <= LL_LDS, "a workgroup's LDS");
+    __shared__ __attribute__((aligned(1024))) char lds[LDS];
+    const int lane = threadIdx.x % SIA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SIA_WAVE);
+    const int r = lane % 16, g = lane / 16;
+    const int m0 = blockIdx.y * MB * 16, slice = wave % SLICES, group = wave / SLICES;
+    const int n0 = (blockIdx.x * GROUPS + group) * NB * 16;
+    const int chunks = (K + CHUNK - 1) / CHUNK;
+    const int begin = slice_begin(chunks, slice, SLICES);
+    const int steps = n0 < N ? slice_begin(chunks, slice + 1, SLICES) - begin : 0;      // chunks of this wave
 
-template <bool ALIGNED>
-__global__ __launch_bounds__(256) void gemm_f32_few_rows_kernel(const float* __restrict__ X, const float* __restrict__ W,
-                                                                float* __restrict__ Y, int M, int N, int K, bool whole) {
-    __shared__ f32x4 part[SUMS / 2][SIA_WAVE];
-    const int lane = threadIdx.x % SIA_WAVE, sum = threadIdx.x / SIA_WAVE;
-    const int r = lane % 16, q = lane / 16;
-    const int n0 = blockIdx.x * 16;
-    const int steps = (K + STEP - 1) / STEP;
-    const int k0 = sum * PIECE + 4 * q;
-    // rows that do not exist are read as the last one and not stored
-    const float* w_row = W + (size_t)min(n0 + r, N - 1) * K + k0;
-    const float* x_row = X + (size_t)min(r, M - 1) * K + k0;
-
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f}, w[2][FLIGHT], x[2][FLIGHT];
-    auto fetch = [&](int set, int s0) {
+    f32x4 total[MB][NB];
 #pragma unroll
-        for (int s = 0; s < FLIGHT; ++s) {
-            const int at = (s0 + s) * STEP;
-            w[set][s] = load4<ALIGNED>(w_row + at, k0 + at, K);
-            x[set][s] = load4<ALIGNED>(x_row + at, k0 + at, K);
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) total[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // U chunks from s on; chunks behind the last are zeros, which change nothing
+    auto multiply = [&](int s, u32x4 (&wa)[U][NB], u32x4 (&wb)[U][NB], u32x4 (&xa)[U][MB], u32x4 (&xb)[U][MB]) {
+        const u32x4 none = {0, 0, 0, 0};
+        uint32_t bits = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = (begin + s + u) * CHUNK + 8 * g;
+            if (s + u >= steps)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) wa[u][j] = none, wb[u][j] = none;
+            if (s + u >= steps || (begin + s + u + 1) * CHUNK > K)
+#pragma unroll
+                for (int b = 0; b < MB; ++b) {      // behind the last k too (W has there what was read instead)
+                    if (s + u >= steps || k >= K) xa[u][b] = none;
+                    if (s + u >= steps || k + 4 >= K) xb[u][b] = none;
+                }
+#pragma unroll
+            for (int j = 0; j < NB; ++j) bits |= or_of(wa[u][j], wb[u][j]);
+        }
+        if (!__any((bits & 0xffffu) != 0)) {
+            f32x4 t[U][MB][NB];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                u32x4 w0[NB];
+#pragma unroll
+                for (int j = 0; j < NB; ++j) w0[j] = upper_halves(wa[u][j], wb[u][j]);
+#pragma unroll
+                for (int b = 0; b < MB; ++b) {
+                    u32x4 x[PARTS];
+                    split8(xa[u][b], xb[u][b], x);
+                    chunk_one_part(w0, x, t[u][b]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) total[b][j] += t[u][b][j];
+        } else {
+            f32x4 t[U][MB][NB];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                u32x4 w[NB][PARTS];
+#pragma unroll
+                for (int j = 0; j < NB; ++j) split8(wa[u][j], wb[u][j], w[j]);
+#pragma unroll
+                for (int b = 0; b < MB; ++b) {
+                    u32x4 x[PARTS];
+                    split8(xa[u][b], xb[u][b], x);
+                    chunk_of_parts(w, x, t[u][b]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) total[b][j] += t[u][b][j];
         }
     };
-    auto multiply = [&](int set, int s0) {
+    u32x4 wa[U][NB], wb[U][NB], xa[U][MB], xb[U][MB];
+    if constexpr (DIRECT) {
+        // rows that do not exist are read as the last one and not stored
+        const float* from[CHUNK_LOADS];
+        int piece[CHUNK_LOADS];
 #pragma unroll
-        for (int s = 0; s < FLIGHT; ++s) {
-            const int k = k0 + (s0 + s) * STEP;
-            acc = sum_of_piece(in_row(w[set][s], k, K), in_row(x[set][s], k, K), acc);
+        for (int l = 0; l < CHUNK_LOADS; ++l) {
+            const int row = (l < 2 * NB ? l : l - 2 * NB) * 8 + lane / 8;
+            from[l] = l < 2 * NB ? W + (size_t)min(n0 + row, N - 1) * K : X + (size_t)min(m0 + row, M - 1) * K;
+            piece[l] = begin * CHUNK + ((lane & 7) ^ turn(row & 15)) * 4;
         }
-    };
-    fetch(0, 0);
-    for (int s0 = 0; s0 < steps; s0 += 2 * FLIGHT) {     // steps past the end add zero times zero
-        fetch(1, s0 + FLIGHT);
-        multiply(0, s0);
-        if (s0 + 2 * FLIGHT < steps) fetch(0, s0 + 2 * FLIGHT);
-        multiply(1, s0 + FLIGHT);
+        char* const ring = lds + wave * (SLOTS * LOADS * LL_TILE);
+        // steps of U chunks; the last one's chunks behind the end are loaded again, so that the waits count the same
+        auto request = [&](int s, int slot) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int l = 0; l < CHUNK_LOADS; ++l)
+                    load_to_lds(from[l] + min(min(s + u, steps - 1) * CHUNK + piece[l], K - 4), ring + ((slot * U + u) * CHUNK_LOADS + l) * LL_TILE);
+        };
+#pragma unroll
+        for (int s = 0; s < SLOTS; ++s)
+            if (s * U < steps) request(s * U, s);
+        const int at[2] = {r * 128 + ((2 * g) ^ turn(r)) * 16, r * 128 + ((2 * g + 1) ^ turn(r)) * 16};
+        const int xr = XI == 1 ? r & 7 : r;
+        const int x_at[2] = {xr * 128 + ((2 * g) ^ turn(xr)) * 16, xr * 128 + ((2 * g + 1) ^ turn(xr)) * 16};
+        int slot = 0;
+        for (int s = 0; s < steps; s += U) {
+            wait_step<LOADS, SLOTS - 1>((steps - 1) / U - s / U);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const char* in = ring + (slot * U + u) * CHUNK_LOADS * LL_TILE;
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    wa[u][j] = *(const u32x4*)(in + 2 * j * LL_TILE + at[0]), wb[u][j] = *(const u32x4*)(in + 2 * j * LL_TILE + at[1]);
+#pragma unroll
+                for (int b = 0; b < MB; ++b) {
+                    const char* in_x = in + (2 * NB + 2 * b) * LL_TILE;
+                    xa[u][b] = *(const u32x4*)(in_x + x_at[0]), xb[u][b] = *(const u32x4*)(in_x + x_at[1]);
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the slot has been read: it may be filled again
+            if (s + SLOTS * U < steps) request(s + SLOTS * U, slot);
+            slot = slot + 1 < SLOTS ? slot + 1 : 0;
+            multiply(s, wa, wb, xa, xb);
+        }
+    } else {
+        const uint32_t *w_row[NB], *x_row[MB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) w_row[j] = (const uint32_t*)W + (size_t)min(n0 + j * 16 + r, N - 1) * K;
+#pragma unroll
+        for (int b = 0; b < MB; ++b) x_row[b] = (const uint32_t*)X + (size_t)min(m0 + b * 16 + r, M - 1) * K;
+        for (int s = 0; s < steps; s += U) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = (begin + min(s + u, steps - 1)) * CHUNK + 8 * g;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) wa[u][j][e] = w_row[j][min(k + e, K - 1)], wb[u][j][e] = w_row[j][min(k + 4 + e, K - 1)];
+#pragma unroll
+                    for (int b = 0; b < MB; ++b)
+                        xa[u][b][e] = k + e < K ? x_row[b][k + e] : 0, xb[u][b][e] = k + 4 + e < K ? x_row[b][k + 4 + e] : 0;
+                }
+            }
+            multiply(s, wa, wb, xa, xb);
+        }
     }
-    // (s0 + s1) + (s2 + s3)
-    if (sum & 1) part[sum / 2][lane] = acc;
+    // row m of Y and its four columns from n on
+    auto finish = [&](int m, int n, f32x4 v) {
+        if (m >= M) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < N) Y[(size_t)m * N + n + e] = finite(v[e]) ? v[e] : plain_sum(X + (size_t)m * K, W + (size_t)(n + e) * K, K);
+    };
+    if (SLICES == 1) {
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) finish(m0 + b * 16 + r, n0 + j * 16 + 4 * g, total[b][j]);
+        return;
+    }
+    f32x4* const part = (f32x4*)lds;
+    __syncthreads();      // every wave has read its ring
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) part[(((slice * GROUPS + group) * MB + b) * NB + j) * SIA_WAVE + lane] = total[b][j];
     __syncthreads();
-    if (!(sum & 1)) acc += part[sum / 2][lane];
-    if (sum == 2) part[1][lane] = acc;      // its own half of the memory, which it has just read
-    __syncthreads();
-    if (sum == 0) store4(Y, r, n0 + 4 * q, M, N, whole, acc + part[1][lane]);
+    constexpr int BLOCKS = GROUPS * MB * NB;
+#pragma unroll
+    for (int i = 0; i < (BLOCKS + WAVES - 1) / WAVES; ++i) {
+        const int block = wave + i * WAVES;
+        if (block >= BLOCKS) return;
+        f32x4 v = part[block * SIA_WAVE + lane];
+#pragma unroll
+        for (int s = 1; s < SLICES; ++s) v += part[(s * BLOCKS + block) * SIA_WAVE + lane];
+        finish(m0 + block / NB % MB * 16 + r, (blockIdx.x * GROUPS + block / (MB * NB)) * NB * 16 + block % NB * 16 + 4 * g, v);
+    }
+}
+
+// Small rings, and more workgroups on a unit, are faster than deep ones (us for one row and weights of 8 bits, 8 waves, the best two of
+// each:  2,048 x 2,048 6.4 with one step of two chunks, 6.8 with three;  28,672 x 4,096 78 and 86).
+template <int MB, int NB, int XI, bool DIRECT>
+static void launch_few_rows(const float* X, const float* W, float* Y, int M, int N, int K, hipStream_t stream) {
+    const int slices = slices_of(N, K), y = (M + MB * 16 - 1) / (MB * 16);
+    auto columns = [&](int groups) { return dim3((N + groups * NB * 16 - 1) / (groups * NB * 16), y); };
+    constexpr int EACH = 2 * NB + XI, U = MB * NB == 1 ? 2 : 1;
+    constexpr int SLOTS2 = EACH <= 3 ? 3 : EACH <= 8 ? 2 : 1, SLOTS = EACH <= 9 && MB * NB <= 4 ? 2 : 1;
+    if (slices == 8)
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<8, 8, MB, NB, XI, U, 1, DIRECT>), columns(1), dim3(512), 0, stream, X, W, Y, M, N, K);
+    else if (slices == 2)
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<2, 4, MB, NB, XI, U, SLOTS2, DIRECT>), columns(2), dim3(256), 0, stream, X, W, Y, M, N, K);
+    else if (N <= 32 * 1024)
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<1, 4, MB, NB, XI, U, 1, DIRECT>), columns(4), dim3(256), 0, stream, X, W, Y, M, N, K);
+    else
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<1, 8, MB, NB, XI, U, SLOTS, DIRECT>), columns(8), dim3(512), 0, stream, X, W, Y, M, N, K);
+}
+
+// The shape of the few-row kernel: blocks of X's and W's rows, and at what rate its workgroups fetch (MB a us).  More blocks share what is read
+// and split of the other operand, where enough workgroups are left.
+struct FewRows {
+    int mb, nb;
+    double rate;
+};
+static FewRows few_rows_shape(int M, int N, int K) {
+    if (M <= 8 && N > 32 * 1024 && K % CHUNK == 0) return {1, 4, 12};      // rows of whole cache lines
+    if (M <= 16 || K <= 4 * CHUNK) return {1, 1, 16};
+    if (N < 8 * 1024) return {2, 1, 16};
+    if (M > 32 && N > 12 * 1024) return {4, 2, 10};
+    if (N <= 32 * 1024) return {2, 2, 12};
+    return K % CHUNK == 0 ? FewRows{2, 4, 12} : FewRows{2, 2, 7};
+}
+
+static void few_rows(const float* X, const float* W, float* Y, int M, int N, int K, bool direct, hipStream_t stream) {
+    const FewRows few = few_rows_shape(M, N, K);
+    if (!direct && M <= 16)
+        launch_few_rows<1, 1, 2, false>(X, W, Y, M, N, K, stream);
+    else if (!direct)
+        launch_few_rows<2, 1, 4, false>(X, W, Y, M, N, K, stream);
+    else if (few.mb == 4)
+        launch_few_rows<4, 2, 8, true>(X, W, Y, M, N, K, stream);
+    else if (few.mb == 2 && few.nb == 4)
+        launch_few_rows<2, 4, 4, true>(X, W, Y, M, N, K, stream);
+    else if (few.mb == 2 && few.nb == 2)
+        launch_few_rows<2, 2, 4, true>(X, W, Y, M, N, K, stream);
+    else if (few.mb == 2)
+        launch_few_rows<2, 1, 4, true>(X, W, Y, M, N, K, stream);
+    else if (few.nb == 4)
+        launch_few_rows<1, 4, 1, true>(X, W, Y, M, N, K, stream);
+    else if (M <= 8)
+        launch_few_rows<1, 1, 1, true>(X, W, Y, M, N, K, stream);
+    else
+        launch_few_rows<1, 1, 2, true>(X, W, Y, M, N, K, stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // tiles
 // ---------------------------------------------------------------------------------------------------------
 
-#define STAGES 3
+// The parts of X as the matrix cores read them: [chunk][block of 16 rows][part][lane] of 16 bytes, zeros beyond X.
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ X, u32x4* __restrict__ parts, int M, int K, int blocks,
+                                                         int chunks, bool direct) {
+    const long long id = (long long)blockIdx.x * 4 + threadIdx.x / SIA_WAVE;
+    const int lane = threadIdx.x % SIA_WAVE, c = (int)(id % chunks);
+    const long long b = id / chunks;
+    if (b >= blocks) return;
+    const long long row = b * 16 + lane % 16;
+    const int k = c * CHUNK + lane / 16 * 8;
+    u32x4 v[2] = {u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}}, p[PARTS];
+    const uint32_t* from = (const uint32_t*)X + row * K + k;
+    if (direct) {      // K is a multiple of 4
+        if (row < M && k < K) v[0] = *(const u32x4*)from;
+        if (row < M && k + 4 < K) v[1] = *(const u32x4*)(from + 4);
+    } else
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (row < M && k + e < K) v[e / 4][e % 4] = from[e];
+    split8(v[0], v[1], p);
+    u32x4* at = parts + ((long long)c * blocks + b) * PART_BLOCK + lane;
+#pragma unroll
+    for (int e = 0; e < PARTS; ++e) at[e * SIA_WAVE] = p[e];
+}
 
-// A tile of BM rows of X by BN rows of W, taken by waves of WM by WN, four times over (once per sum).
-template <int BM, int BN, int WM, int WN, bool ALIGNED>
-__global__ __launch_bounds__(SUMS * (BM / WM) * (BN / WN) * SIA_WAVE) void gemm_f32_tile_kernel(
-    const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int tiles_m,
-    int n_tiles, int per_die, bool whole) {
-    constexpr int WAVES = (BM / WM) * (BN / WN), THREADS = SUMS * WAVES * SIA_WAVE;
-    constexpr int TM = WM / 16, TN = WN / 16;
-    constexpr int ROWS = BM + BN, PIECES = ROWS * (STEP / 4), LOADS = (PIECES + THREADS - 1) / THREADS;
-    constexpr int STAGE = ROWS * STEP;
-    static_assert(STAGES * STAGE >= 2 * BM * BN, "the partial sums are added in the stages' memory");
-    extern __shared__ float lds[];
+// Rows of K floats that begin anywhere, copied to rows of `stride` (K up to a multiple of 4, zeros behind).  Four elements a thread.
+__global__ __launch_bounds__(256) void align_rows_kernel(const float* __restrict__ W, f32x4* __restrict__ out, int K, int stride, size_t pieces) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= pieces) return;
+    const size_t row = i / (stride / 4);
+    const int k = (int)(i % (stride / 4)) * 4;
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? W[row * K + k + e] : 0.f;
+    out[i] = v;
+}
 
+// A tile of BM rows of W, taken by WM x WN waves.  A ring of D + 1 chunks of both in LDS, asked for D ahead; one
+// barrier a chunk: what is read next has come, what was read last may be overwritten.
+// apart: a workgroup has one slice of K, whose sums go to `slices` ([slice][M][Ns]) for sum_slices_f32_kernel.  Else it has all of K, and
+// adds up the slices, SLICED: in registers, else in Y.
+// Wt: W's rows as they are read, from multiples of 16 bytes, Kt floats apart (a multiple of 4).
+template <int BM, int BN, int WM, int WN, int D, bool SLICED>
+__global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
+    const u32x4* __restrict__ parts, const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ Wt,
+    float* __restrict__ Y, float* __restrict__ slices, int M, int N, int K, int Kt, int Ns, int n_slices, bool apart, bool four,
+    int tiles_m, int n_tiles, int per_die) {
+    constexpr int WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
+    constexpr int XT = BM / 16 * PARTS, WT = BN / 8;                 // KiB of a chunk
+    constexpr int LX = (XT + WAVES - 1) / WAVES, LW = WT / WAVES;    // loads of a wave
+    constexpr int STAGE = (XT + WT) * LL_TILE, LOADS = LX + LW;
+    static_assert(TM * WM * 16 == BM && TN * WN * 16 == BN && LW * WAVES == WT && (D + 1) * STAGE <= LL_LDS, "tiles");
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
     // Workgroups go to the dies in turn: a die gets consecutive tiles, row tiles of X innermost, so that the rows of W
     // that they share are read by one die.
     const int tile = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
     if (tile >= n_tiles) return;
-    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    const int slice = apart ? (tile / tiles_m) % n_slices : 0;
+    const int m0 = (tile % tiles_m) * BM, n0 = tile / tiles_m / (apart ? n_slices : 1) * BN;
+    const int chunks = (K + CHUNK - 1) / CHUNK, blocks = (M + 15) / 16;
+    const int lane = threadIdx.x % SIA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SIA_WAVE);
+    const int wm = wave % WM, wn = wave / WM, r = lane % 16, g = lane / 16;
 
-    const int tid = threadIdx.x, lane = tid % SIA_WAVE, wave = tid / SIA_WAVE;
-    const int sum = wave / WAVES, wm = (wave % WAVES) % (BM / WM), wn = (wave % WAVES) / (BM / WM);
-    const int r = lane % 16, q = lane / 16;
-    const int steps = (K + STEP - 1) / STEP;
-
-    // The loads of a step are issued two steps before they are put into LDS: a step is shorter than the way from memory.
-    const float* from[LOADS];
-    int k_of[LOADS];
-    f32x4 next[2][LOADS];
+    // X: KiB beyond the tile or the last block repeat the last one (into the same place: the same bytes)
+    int x_kib[LX], x_from[LX];
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {     // rows that do not exist are read as the last one and not stored
-        const int piece = tid + i * THREADS, row = min(piece / (STEP / 4), ROWS - 1);
-        k_of[i] = (piece % (STEP / 4)) * 4;
-        from[i] = (row < BM ? X + (size_t)min(m0 + row, M - 1) * K : W + (size_t)min(n0 + row - BM, N - 1) * K) + k_of[i];
+    for (int l = 0; l < LX; ++l) {
+        x_kib[l] = min(wave * LX + l, XT - 1);
+        x_from[l] = min(x_kib[l], (blocks - m0 / 16) * PARTS - 1) * SIA_WAVE + lane;
     }
-    auto fetch = [&](int set, int s) {
+    const float* w_from[LW];
+    int piece[LW];
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i) next[set][i] = load4<ALIGNED>(from[i] + s * STEP, k_of[i] + s * STEP, K);
-    };
-    // Sixteen pieces of four floats are a row of a stage; piece p of row r lies at place p ^ (r % 16).
-    auto put = [&](int set, int s, float* stage) {
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-            const int piece = tid + i * THREADS, row = piece / (STEP / 4), at = ((piece % (STEP / 4)) ^ (row % 16)) * 4;
-            if (PIECES % THREADS == 0 || row < ROWS)
-                *(f32x4*)(stage + row * STEP + at) = in_row(next[set][i], k_of[i] + s * STEP, K);
-        }
-    };
+    for (int l = 0; l < LW; ++l) {      // rows that do not exist are read as the last one and not stored
+        const int row = (wave * LW + l) * 8 + lane / 8;
+        w_from[l] = Wt + (size_t)min(n0 + row, N - 1) * Kt;
+        piece[l] = ((lane & 7) ^ turn(row & 15)) * 4;
+    }
+    const int x_at = wm * TM * PARTS * LL_TILE + lane * 16, w_at = XT * LL_TILE + (wn * (BN / WN) + r) * 128;
+    const int place[2] = {((2 * g) ^ turn(r)) * 16, ((2 * g + 1) ^ turn(r)) * 16};
 
-    f32x4 acc[TM][TN], x[2][TM], w[2][TN];
+    const int begin = apart ? slice_begin(chunks, slice, n_slices) : 0;
+    const int steps = (apart ? slice_begin(chunks, slice + 1, n_slices) : chunks) - begin;
+    const u32x4* x_first = parts + ((size_t)begin * blocks + m0 / 16) * PART_BLOCK;
+    auto request = [&](int s, int slot) {
+        char* to = lds + slot * STAGE;
+        const u32x4* from = x_first + (size_t)s * blocks * PART_BLOCK;
+#pragma unroll
+        for (int l = 0; l < LX; ++l) load_to_lds(from + x_from[l], to + x_kib[l] * LL_TILE);
+        to += XT * LL_TILE + wave * LW * LL_TILE;
+        // behind the last k: the row's last four (X's parts are zero there)
+#pragma unroll
+        for (int l = 0; l < LW; ++l) load_to_lds(w_from[l] + min((begin + s) * CHUNK + piece[l], Kt - 4), to + l * LL_TILE);
+    };
+    f32x4 total[TM][TN], sum[SLICED ? TM : 1][SLICED ? TN : 1];      // of the slice, of the slices before it
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    const int place = ((sum * 4 + q) ^ r) * 4;
-    const int x_at = (wm * WM + r) * STEP + place, w_at = (BM + wn * WN + r) * STEP + place;
-    auto read = [&](int set, const float* stage) {
+        for (int j = 0; j < TN; ++j) {
+            total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (SLICED) sum[i][j] = total[i][j];
+        }
+    // total[i][j]: row 16 i + r of the wave's tile, columns 16 j + 4 g .. + 3
+    const int m_first = m0 + wm * (BM / WM) + r, n_first = n0 + wn * (BN / WN) + 4 * g, stride = apart ? Ns : N;
+    float* const to = apart ? slices + (size_t)slice * M * Ns : Y;
+    bool odd = false;
+    auto store = [&](bool more) {      // more: Y has the slices before
 #pragma unroll
-        for (int i = 0; i < TM; ++i) x[set][i] = *(const f32x4*)(stage + x_at + i * 16 * STEP);
+        for (int i = 0; i < TM; ++i) {
+            const int m = m_first + i * 16;
+            if (m >= M) continue;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) w[set][j] = *(const f32x4*)(stage + w_at + j * 16 * STEP);
+            for (int j = 0; j < TN; ++j) {
+                const int n = n_first + j * 16;
+                float* at = to + (size_t)m * stride + n;
+                f32x4 v = total[i][j];
+                if constexpr (SLICED) v = sum[i][j] + v;
+                if (four || apart) {
+                    if (n >= N) continue;
+                    if (more) v = *(const f32x4*)at + v;
+                    *(f32x4*)at = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < N) {
+                            if (more) v[e] = at[e] + v[e];
+                            at[e] = v[e];
+                        }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) odd |= !finite(v[e]);
+            }
+        }
     };
-    // A step multiplies what lies in registers while the next step's operands are read from LDS, the step after it is
-    // written there and the one two further on is on its way from memory.  A wave issues in order, and the waves of a
-    // workgroup pass every barrier together: LDS and matrix cores work at the same time only if each wave's own
-    // instructions alternate, so the schedule is written down.  Steps past the end move zeros: no branches.
-    constexpr int OTHERS = TM + TN + 2 * LOADS, EACH = (4 * TM * TN) / OTHERS > 0 ? (4 * TM * TN) / OTHERS : 1;
-    int now = 0;      // s % STAGES
-    auto step = [&](int s, int parity) {      // parity: s % 2, known where the loop is unrolled
-        const int after = now + 1 == STAGES ? 0 : now + 1, third = after + 1 == STAGES ? 0 : after + 1;
-        read(parity ^ 1, lds + after * STAGE);
-        put(parity, s + 2, lds + third * STAGE);     // read last in the step before the one before
-        fetch(parity, s + 4);
+    int ended = 0, end = apart ? chunks : 0;      // slices behind, where this one ends
+    while (end == 0) end = slice_begin(chunks, ++ended, n_slices);      // (slices may be empty)
+    bool more = false;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+    for (int s = 0; s < D; ++s)
+        if (s < steps) request(s, s);
+    int slot = 0;
+    for (int s = 0; s < steps; ++s) {
+        wait_step<LOADS, D - 1>(steps - 1 - s);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + D < steps) request(s + D, slot == 0 ? D : slot - 1);
+        const char* stage = lds + slot * STAGE;
+        slot = slot == D ? 0 : slot + 1;
+        u32x4 a[TN], b[TN];
+        uint32_t bits = 0;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            a[j] = *(const u32x4*)(stage + w_at + j * 2 * LL_TILE + place[0]);
+            b[j] = *(const u32x4*)(stage + w_at + j * 2 * LL_TILE + place[1]);
+        }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bits |= or_of(a[j], b[j]);
+        auto read_x = [&](int i, u32x4 (&x)[PARTS]) {
+#pragma unroll
+            for (int e = 0; e < PARTS; ++e) x[e] = *(const u32x4*)(stage + x_at + (i * PARTS + e) * LL_TILE);
+        };
+        if (!__any((bits & 0xffffu) != 0)) {
+            u32x4 w0[TN];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) w0[j] = upper_halves(a[j], b[j]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                u32x4 x[PARTS];
+                f32x4 t[TN];
+                read_x(i, x);
+                chunk_one_part(w0, x, t);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) total[i][j] += t[j];
+            }
+        } else {
+            u32x4 w[TN][PARTS];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) split8(a[j], b[j], w[j]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                u32x4 x[PARTS];
+                f32x4 t[TN];
+                read_x(i, x);
+                chunk_of_parts(w, x, t);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) total[i][j] += t[j];
+            }
+        }
+        if (s + 1 == end && s + 1 < steps) {
+            if constexpr (SLICED) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) sum[i][j] += total[i][j];
+            } else {
+                store(more);
+                more = true;
+            }
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = mfma4(w[parity][j][e], x[parity][i][e], acc[i][j]);
-#pragma unroll
-        for (int i = 0; i < TM + TN; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);    // products
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);       // a read from LDS
+                for (int j = 0; j < TN; ++j) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            while (end == s + 1) end = slice_begin(chunks, ++ended, n_slices);
         }
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);
-            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);       // a write to LDS
-            __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);       // a load
-        }
-        __builtin_amdgcn_sched_barrier(0);      // the products stay in front of the barrier
-        __syncthreads();
-        now = after;
-    };
-    fetch(0, 0);
-    fetch(1, 1);
-    put(0, 0, lds);
-    fetch(0, 2);
-    put(1, 1, lds + STAGE);
-    fetch(1, 3);
-    __syncthreads();
-    read(0, lds);
-    for (int s = 0; s < steps; s += 2) {
-        step(s, 0);
-        step(s + 1, 1);
     }
-
-    // (s0 + s1) + (s2 + s3), through the memory of the stages
-    f32x4* part = (f32x4*)lds + (size_t)(sum / 2) * (BM * BN / 4) + (wm + wn * (BM / WM)) * (TM * TN * SIA_WAVE) + lane;
-    if (sum & 1)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) part[(i * TN + j) * SIA_WAVE] = acc[i][j];
-    __syncthreads();
-    if (!(sum & 1))
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] += part[(i * TN + j) * SIA_WAVE];
-    if (sum == 2)      // its own half of the memory, which it has just read
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) part[(i * TN + j) * SIA_WAVE] = acc[i][j];
-    __syncthreads();
-    if (sum == 0) {
-        const f32x4* other = part + BM * BN / 4;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                store4(Y, m0 + wm * WM + i * 16 + r, n0 + wn * WN + j * 16 + 4 * q, M, N, whole,
-                       acc[i][j] + other[(i * TN + j) * SIA_WAVE]);
+    store(more);
+    if (apart || !odd) return;
+#pragma clang loop unroll(disable)
+    for (int i = 0; i < TM * TN * 4; ++i) {
+        const int m = m_first + i / (TN * 4) * 16, n = n_first + i / 4 % TN * 16 + i % 4;
+        if (m >= M || n >= N) continue;
+        float* at = Y + (size_t)m * N + n;
+        if (!finite(*(volatile float*)at)) *at = plain_sum(X + (size_t)m * K, W + (size_t)n * K, K);
     }
 }
 
-template <int BM, int BN, int WM, int WN>
-static int launch_tiles(const float* X, const float* W, float* Y, int M, int N, int K, bool aligned, bool whole, hipStream_t stream) {
-    constexpr int threads = SUMS * (BM / WM) * (BN / WN) * SIA_WAVE, bytes = STAGES * (BM + BN) * STEP * (int)sizeof(float);
-    const int tiles_m = (M + BM - 1) / BM;
-    const long long tiles = (long long)tiles_m * ((N + BN - 1) / BN);
-    if (tiles > (1 << 30)) return SIA_BAD_ARGUMENT;
-    const int per_die = (int)((tiles + 7) / 8);
-    auto kernel = aligned ? gemm_f32_tile_kernel<BM, BN, WM, WN, true> : gemm_f32_tile_kernel<BM, BN, WM, WN, false>;
-    static bool set[64][2] = {};      // more LDS than a kernel gets unasked, allowed once per device
+// Y = the slices' sums added in order.  Four elements of a row a thread.
+__global__ __launch_bounds__(256) void sum_slices_f32_kernel(const float* __restrict__ slices, const float* __restrict__ X,
+                                                             const float* __restrict__ W, float* __restrict__ Y, int N, int K, int Ns, int n_slices,
+                                                             size_t elements, bool four) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;      // of M rows of Ns
+    if (i >= elements) return;
+    const size_t m = i / Ns;
+    const int n = (int)(i % Ns);
+    f32x4 v = *(const f32x4*)(slices + i);
+    for (int s = 1; s < n_slices; ++s) v += *(const f32x4*)(slices + s * elements + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (!finite(v[e]) && n + e < N) v[e] = plain_sum(X + m * K, W + (size_t)(n + e) * K, K);
+    float* at = Y + m * N + n;
+    if (four)
+        *(f32x4*)at = v;
+    else
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < N) at[e] = v[e];
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// which kernel
+// ---------------------------------------------------------------------------------------------------------
+
+// The shapes, how many workgroups of each a compute unit holds at a time, and what a product costs in microseconds, by least squares
+// over 1,100 timings (512 to 128,256 columns, k of 2,048 to 14,336, 17 to 1,024 rows; a shape's median error 3 %, the choice 2.7 % above
+// the best of eleven shapes on average): a launch, a round of workgroups over the device, a chunk of a round, slices apart, a MB of
+// their sums written and read, a MB of W.
+struct F32Shape {
+    int bm, bn, at_a_time;
+    double launch, round, step, apart, sums, weights;
+};
+static const F32Shape F32_SHAPES[] = {{128, 256, 1, 3.7, 6.8, 1.33, 1.5, 0.145, 0.030},
+                                      {96, 256, 1, 5.7, 2.6, 1.15, 2.4, 0.170, 0.015},
+                                      {64, 128, 2, 23.4, -9.0, 0.894, -8.7, 0.359, 0.087},
+                                      {64, 128, 2, 6.9, -1.4, 1.18, 2.4, 0.287, 0.026},
+                                      {32, 64, 3, 14.3, -3.8, 0.624, -2.8, 0.384, 0.066}};
+constexpr int N_F32_SHAPES = sizeof(F32_SHAPES) / sizeof(F32_SHAPES[0]);
+
+struct F32Plan {
+    int shape;      // -1: the few-row kernel
+    bool apart;
+    long long parts, copied, slices;      // bytes of the workspace
+};
+
+// direct: both operands' rows begin at multiples of 16 bytes.
+static F32Plan f32_plan(int M, int N, int K, bool direct) {
+    F32Plan best{-1, false, 0, 0, 0};
+    const int cus = compute_units(), n_slices = slices_of(N, K), chunks = (K + CHUNK - 1) / CHUNK, stride = (K + 3) / 4 * 4;
+    const long long copied = direct ? 0 : (long long)N * stride * 4;
+    if (M <= 16 || copied > 1LL << 28) return best;
+    // the few-row kernel: what its workgroups fetch (their rows of W and X, from L2 for the most part), or W from memory; float by float it
+    // takes twice as long
+    const FewRows few = few_rows_shape(M, N, K);
+    const int rows_w = few.nb * 16, rows_x = few.mb * 16;
+    const double fetched = (double)((M + rows_x - 1) / rows_x) * ((N + rows_w - 1) / rows_w) * (rows_w + rows_x) * K * 4e-6;
+    // the tiles take half as long again for weights of 24 bits, the few-row kernel a tenth: a line between the two
+    double least = (2.5 + fmax(fetched / few.rate, (double)N * K * 4e-6 / 5.4)) * (direct ? 1 : 3) / 1.15;
+    for (int i = 0; i < N_F32_SHAPES; ++i) {
+        const F32Shape t = F32_SHAPES[i];
+        const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        for (int apart = 0; apart <= (n_slices > 1); ++apart) {
+            const long long workgroups = tiles * (apart ? n_slices : 1), room = (long long)cus * t.at_a_time;
+            if (workgroups > 1 << 30 || (apart && (long long)n_slices * M * N > 1LL << 27)) continue;
+            const int steps = apart ? (chunks + n_slices - 1) / n_slices : chunks;
+            // workgroups that share a unit: a last round that fills a part of them is as much shorter
+            const double rounds = (double)(workgroups / room) + (double)((workgroups % room + cus - 1) / cus) / t.at_a_time;
+            double us = (direct ? 0 : 4) + t.launch + t.weights * N * K * 4e-6 + rounds * (t.round + t.step * steps);
+            if (apart) us += t.apart + t.sums * n_slices * M * N * 8e-6;
+            if (!apart && t.bn == 256) us += t.sums * (n_slices - 1) * M * N * 8e-6;      // in Y
+            if (us >= least) continue;
+            least = us;
+            best.shape = i, best.apart = apart;
+        }
+    }
+    if (best.shape < 0) return best;
+    best.parts = (long long)((M + 15) / 16) * chunks * PART_BLOCK * 16;
+    best.copied = copied;
+    best.slices = best.apart ? (long long)n_slices * M * ((N + 3) / 4 * 4) * 4 : 0;
+    return best;
+}
+
+template <int BM, int BN, int WM, int WN, int D, bool SLICED>
+static int launch_f32_shape(const float* X, const float* W, const float* Wt, float* Y, u32x4* parts, float* slices, int M, int N, int K, int Kt,
+                            bool apart, bool four, hipStream_t stream) {
+    constexpr int bytes = (D + 1) * (BM / 16 * PARTS + BN / 8) * LL_TILE;
+    const int n_slices = slices_of(N, K), tiles_m = (M + BM - 1) / BM;
+    const int n_tiles = tiles_m * ((N + BN - 1) / BN) * (apart ? n_slices : 1), per_die = (n_tiles + 7) / 8;
+    const auto kernel = gemm_f32_tile_kernel<BM, BN, WM, WN, D, SLICED>;
+    static bool set[64];      // more LDS than a kernel gets unasked, allowed once per device
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return (int)hipGetLastError();
-    if (device < 0 || device >= 64 || !set[device][aligned]) {
+    if (device < 0 || device >= 64 || !set[device]) {
         const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e != hipSuccess) return (int)e;
-        if (device >= 0 && device < 64) set[device][aligned] = true;
+        if (device >= 0 && device < 64) set[device] = true;
     }
-    hipLaunchKernelGGL(kernel, dim3(8 * per_die), dim3(threads), bytes, stream, X, W, Y, M, N, K, tiles_m, (int)tiles, per_die, whole);
+    hipLaunchKernelGGL(kernel, dim3(8 * per_die), dim3(WM * WN * SIA_WAVE), bytes, stream, parts, X, W, Wt, Y, slices, M, N, K, Kt, (N + 3) / 4 * 4,
+                       n_slices, apart, four, tiles_m, n_tiles, per_die);
     return SIA_LAUNCH_CHECK();
 }
 
-// Which kernel: the time of a step of 64 k in microseconds (measured on 256 compute units with operands that come from
-// memory; the matrix cores alone would take 0.23, 0.91 and 1.81 for the last three) times the rounds over the device.  The
-// two small tiles share a compute unit and need no whole rounds.
-//   303 rows x 16384 x 2048:  64x64 211 us (96 TFLOP/s), 64x128 221, 32x32 258;    x 2048 x 8192:  32x32 138, 64x64 153;
-//   303 x 128256 x 2048:  64x128 1467 us (109 TFLOP/s), 64x64 1620, 32x32 1808;   24 x 2048 x 8192:  32x16 47, 32x32 58
-// where one 4 by 4 block of outputs a thread on the vector units took 596, 904, 5088 and 800.
-// 16 rows and fewer: 2048 x 8192 27 us at one row (2.5 TB/s), 34 at 8; 16384 x 2048 30 (4.5 TB/s); 128256 x 2048 209 (5.0).
-extern "C" int sia_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, hipStream_t stream) {
-    const bool aligned = K % 4 == 0 && ((uintptr_t)X | (uintptr_t)W) % 16 == 0;
-    const bool whole = N % 4 == 0 && (uintptr_t)Y % 16 == 0;
-    if (M <= 16) {
-        auto kernel = aligned ? gemm_f32_few_rows_kernel<true> : gemm_f32_few_rows_kernel<false>;
-        hipLaunchKernelGGL(kernel, dim3((N + 15) / 16), dim3(256), 0, stream, X, W, Y, M, N, K, whole);
+template <int BM, int BN, int WM, int WN, int D>
+static int launch_f32_tiles(const float* X, const float* W, const float* Wt, float* Y, u32x4* parts, float* slices, int M, int N, int K, int Kt,
+                            bool apart, bool four, hipStream_t stream) {
+    if (apart || slices_of(N, K) == 1 || BN == 256)      // (registers of the large ones are full)
+        return launch_f32_shape<BM, BN, WM, WN, D, false>(X, W, Wt, Y, parts, slices, M, N, K, Kt, apart, four, stream);
+    return launch_f32_shape<BM, BN, WM, WN, D, BN != 256>(X, W, Wt, Y, parts, slices, M, N, K, Kt, false, four, stream);
+}
+
+// Bytes of workspace that a product of this size wants (0: none).  direct: K is a multiple of 4 and X and W are on 16 bytes.
+SIA_EXPORT long long sia_gemm_f32_workspace(int M, int N, int K, int direct) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const F32Plan plan = f32_plan(M, N, K, direct);
+    return plan.shape < 0 ? 0 : plan.parts + plan.copied + plan.slices;
+}
+
+// With `workspace` (of sia_gemm_f32_workspace bytes, on 16) the tiles where they are the faster way; without, the few-row kernel, whatever M
+// is, with the same bits.
+SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* workspace, int M, int N, int K, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (K <= 0 || ((uintptr_t)workspace & 15)) return SIA_BAD_ARGUMENT;
+    const bool direct = K % 4 == 0 && aligned16(X, W), four = N % 4 == 0 && ((uintptr_t)Y & 15) == 0;
+    const F32Plan plan = workspace ? f32_plan(M, N, K, direct) : F32Plan{-1, false, 0, 0, 0};
+    if (plan.shape < 0) {
+        constexpr int MOST = 65535 * 16;      // rows of a launch
+        for (; M > MOST; M -= MOST, X += (size_t)MOST * K, Y += (size_t)MOST * N) few_rows(X, W, Y, MOST, N, K, direct, stream);
+        few_rows(X, W, Y, M, N, K, direct, stream);
         return SIA_LAUNCH_CHECK();
     }
-    auto rounds = [&](int bm, int bn) { return (double)((M + bm - 1) / bm) * ((N + bn - 1) / bn) / 256; };
-    const double shared[2] = {0.37 * fmax(1.0, rounds(32, 16)), 0.44 * fmax(1.0, rounds(32, 32))};
-    const double alone[2] = {1.17 * ceil(rounds(64, 64)), 2.15 * ceil(rounds(64, 128))};
-    const double best = fmin(fmin(shared[0], shared[1]), fmin(alone[0], alone[1]));
-    if (best == alone[1]) return launch_tiles<64, 128, 64, 64>(X, W, Y, M, N, K, aligned, whole, stream);
-    if (best == alone[0]) return launch_tiles<64, 64, 32, 64>(X, W, Y, M, N, K, aligned, whole, stream);
-    if (best == shared[1]) return launch_tiles<32, 32, 32, 16>(X, W, Y, M, N, K, aligned, whole, stream);
-    return launch_tiles<32, 16, 32, 16>(X, W, Y, M, N, K, aligned, whole, stream);
+    u32x4* const parts = (u32x4*)workspace;
+    f32x4* const copy = (f32x4*)((char*)workspace + plan.parts);
+    float* const slices = (float*)((char*)workspace + plan.parts + plan.copied);
+    const int blocks = (M + 15) / 16, chunks = (K + CHUNK - 1) / CHUNK, Kt = (K + 3) / 4 * 4, Ns = (N + 3) / 4 * 4;
+    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)(((long long)blocks * chunks + 3) / 4)), dim3(256), 0, stream, X, parts, M, K, blocks, chunks,
+                       direct);
+    if (!direct) {
+        const size_t pieces = (size_t)N * (Kt / 4);
+        hipLaunchKernelGGL(align_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, W, copy, K, Kt, pieces);
+    }
+    const float* const Wt = direct ? W : (const float*)copy;
+    const bool apart = plan.apart;
+    int status = SIA_BAD_ARGUMENT;
+#define SHAPE(I, ...) \
+    if (plan.shape == I) status = launch_f32_tiles<__VA_ARGS__>(X, W, Wt, Y, parts, slices, M, N, K, Kt, apart, four, stream)
+    SHAPE(0, 128, 256, 2, 4, 1);
+    SHAPE(1, 96, 256, 2, 4, 2);
+    SHAPE(2, 64, 128, 2, 2, 1);
+    SHAPE(3, 64, 128, 2, 4, 2);
+    SHAPE(4, 32, 64, 2, 2, 2);
+#undef SHAPE
+    if (status == 0 && apart)
+        hipLaunchKernelGGL(sum_slices_f32_kernel, dim3((unsigned)(((size_t)M * Ns / 4 + 255) / 256)), dim3(256), 0, stream, slices, X, W, Y, N, K, Ns,
+                           slices_of(N, K), (size_t)M * Ns, four);
+    return status ? status : SIA_LAUNCH_CHECK();
 }

@@ -6,7 +6,7 @@
 // of 16 staged through LDS.  Any M, N, K (edges are guarded).
 #include "common.h"
 
-extern "C" int sia_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K, hipStream_t stream);
+extern "C" int sia_gemm_f32(const float* X, const float* W, float* Y, void* workspace, int M, int N, int K, hipStream_t stream);
 
 #define GT 64   // tile edge
 #define GK 16   // K step
@@ -69,7 +69,7 @@ SIA_EXPORT int sia_gemm_generic(const void* X, const void* W, void* Y, int M, in
     if (K <= 0) return SIA_BAD_ARGUMENT;
     dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT), block(256);
     if (grid.y > 65535) return SIA_BAD_ARGUMENT;
-    if (in_dtype == SIA_F32) return sia_gemm_f32((const float*)X, (const float*)W, (float*)Y, M, N, K, stream);
+    if (in_dtype == SIA_F32) return sia_gemm_f32((const float*)X, (const float*)W, (float*)Y, nullptr, M, N, K, stream);
     if (in_dtype == SIA_BF16 && out_float)
         hipLaunchKernelGGL((gemm_generic_kernel<bf16_t, float>), grid, block, 0, stream, (const bf16_t*)X,
                            (const bf16_t*)W, (float*)Y, M, N, K);

@@ -110,6 +110,8 @@ _SIGNATURES = {
     "sia_attention_max_head_dim": [],
     "sia_attention_generic_max_head_dim": [],
     "sia_gemm_generic": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "sia_gemm_f32": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
+    "sia_gemm_f32_workspace": [_c_int, _c_int, _c_int, _c_int],
     "sia_prenorm_block": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_prenorm_mixer": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
     "sia_sample": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
@@ -309,6 +311,7 @@ class HipKernels:
         self.core = build.load_library("core")
         _bind(self.core, _SIGNATURES)
         self.core.sia_sample_workspace_bytes.restype = ctypes.c_longlong
+        self.core.sia_gemm_f32_workspace.restype = ctypes.c_longlong
         self.core.sia_gla_workspace.restype = ctypes.c_longlong
         self.core.sia_moe_tiled_workspace.restype = ctypes.c_longlong
         self.core.sia_hgrn2_workspace.restype = ctypes.c_longlong
@@ -1017,11 +1020,19 @@ class HipKernels:
             self._product_into(x[g], wg, main[g] if g + 1 < groups else low)
         return main, low
 
+    def _float_product(self, x, w, y):
+        """``y = x @ w^T`` in float32 (csrc/gemm_f32.hip); the rows' parts and the slices of k lie in a workspace."""
+        M, K = x.shape
+        N = w.shape[0]
+        size = self.core.sia_gemm_f32_workspace(M, N, K, int(K % 4 == 0 and _in_pieces(x, w)))
+        workspace = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
+        self._check(self.core.sia_gemm_f32(_ptr(x), _ptr(w), _ptr(y), _ptr(workspace), M, N, K, self._stream()), "gemm_f32")
+
     def _product_into(self, x, w, y):
         M, K = x.shape
         N = w.shape[0]
         if x.dtype == torch.float32:
-            self._check(self.core.sia_gemm_generic(_ptr(x), _ptr(w), _ptr(y), M, N, K, 0, 1, self._stream()), "gemm_generic")
+            self._float_product(x, w, y)
         elif self.blas is None or self.blas.sia_blas_mm(_ptr(x), _ptr(w), _ptr(y), M, N, K, 0, self._stream()) != 0:
             torch.mm(x, w.t(), out=y)
 
@@ -1437,8 +1448,7 @@ class HipKernels:
         if w.dtype == torch.bfloat16:
             w = self.cast(w, torch.float32)
         y = torch.empty((M, N), dtype=torch.float32, device=x.device)
-        self._check(self.core.sia_gemm_generic(_ptr(x), _ptr(w), _ptr(y), M, N, K, 0, 1, self._stream()),
-                    "gemm_generic")
+        self._float_product(x, w, y)
         if back is not None and not out_float32:
             y = self.cast(y, back)
         return y

@@ -536,6 +536,52 @@ def test_library_product_with_candidates_tried_out(hip, shape):
     assert torch.equal(outs[1], outs[3])   # the kept algorithm is used from then on
 
 
+@pytest.mark.parametrize("bits", [8, 24])
+@pytest.mark.parametrize("N, K", [(1, 4), (15, 31), (97, 129), (1000, 333), (520, 1056), (3072, 260), (8200, 2048), (12290, 192), (33000, 40)])
+def test_float32_products_of_parts(hip, N, K, bits):
+    """Every way the product goes (few rows, tiles, whole k and slices, empty slices too, short last chunks, tiles and columns, rows on 16 bytes or
+    not) against 64 bits, weights of one part and of three, one row of three parts among others of one; a row has the same bits whatever
+    rows are beside it.  A chunk's sum is at most 192 roundings of 2^-24 of sums below sum |x w|, the chunks' and slices' sums
+    K / 32 + 8 more, and what is left out of the parts' products 2^-24 of each."""
+    w = rnd(N, K, seed=2)
+    if bits == 8:
+        w = w.bfloat16().float()
+        w[N // 2] = rnd(K, seed=3)
+    x = rnd(700, K, seed=1)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    all_rows = hip.linear(x, w)
+    assert bool(((all_rows.double() - want).abs() <= (201 + K / 32) * 2.0 ** -24 * size + 1e-30).all())
+    for M in (1, 8, 9, 16, 17, 32, 33, 64, 65, 130, 303):
+        assert torch.equal(hip.linear(x[700 - M:].contiguous(), w), all_rows[700 - M:]), M
+    few = torch.empty(33, N, device=DEV)      # without a workspace: the few-row kernel
+    assert hip.core.sia_gemm_f32(x.data_ptr(), w.data_ptr(), few.data_ptr(), None, 33, N, K, hip._stream()) == 0
+    assert torch.equal(few, all_rows[:33])
+    flat = torch.empty(N * K + 1, device=DEV)
+    flat[1:] = w.flatten()
+    for M in (5, 40, 303):
+        assert torch.equal(hip.linear(x[:M].contiguous(), flat[1:].view(N, K)), all_rows[:M]), M
+
+
+@pytest.mark.parametrize("M, N, K", [(3, 96, 64), (40, 520, 333), (100, 2048, 512), (70, 40000, 64), (40, 12800, 256)])
+def test_float32_products_that_are_not_finite(hip, M, N, K):
+    """Infinities, NaN, products of an infinity with zero and the largest finite numbers give what floats give."""
+    largest = torch.finfo(torch.float32).max
+    for where, value in (("x", float("inf")), ("x", float("nan")), ("w", float("-inf")), ("x", largest), ("w", largest)):
+        for bits in (8, 24):
+            x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+            if bits == 8:
+                w = w.bfloat16().float()
+            if abs(value) == largest:
+                x[:, 1:], w[:, 1:] = 0.0, 0.0
+                x[:, 0], w[:, 0] = 1.0, 1.0
+            (x if where == "x" else w)[1, 0] = value
+            w[2, 0] = 0.0
+            want, got = (x.double() @ w.double().T).float(), hip.linear(x, w)
+            assert torch.equal(torch.isnan(want), torch.isnan(got)) and torch.equal(torch.isinf(want), torch.isinf(got))
+            odd = ~torch.isfinite(want) & ~torch.isnan(want) | (want.abs() == largest)
+            assert torch.equal(want[odd], got[odd])
+
+
 def test_float32_product_has_no_reduced_precision(hip):
     """An operand bit below bfloat16 (8 bits) and tf32 (10 bits) resolution must reach the product."""
     K = 8
