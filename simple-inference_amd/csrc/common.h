@@ -25,6 +25,13 @@ __device__ __forceinline__ bf16_t float_to_bf16(float f) {
     return (bf16_t)(u >> 16);
 }
 
+// a and b rounded the same way, a in the low half: one instruction.
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+    uint32_t v;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(v) : "v"(a), "v"(b));
+    return v;
+}
+
 __device__ __forceinline__ float to_float(float x) { return x; }
 __device__ __forceinline__ float to_float(bf16_t x) { return bf16_to_float(x); }
 

@@ -38,13 +38,6 @@ constexpr int PART_BLOCK = PARTS * SIA_WAVE;      // 16-byte pieces of the parts
 // parts and products
 // ---------------------------------------------------------------------------------------------------------
 
-// a and b as bfloat16, rounded to nearest, a in the low half
-__device__ __forceinline__ uint32_t round_pair(float a, float b) {
-    uint32_t v;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(v) : "v"(a), "v"(b));
-    return v;
-}
-
 // The parts of eight consecutive floats, each eight bfloat16 in order.
 __device__ __forceinline__ void split8(u32x4 first, u32x4 second, u32x4 (&part)[PARTS]) {
 #pragma unroll
@@ -53,7 +46,7 @@ __device__ __forceinline__ void split8(u32x4 first, u32x4 second, u32x4 (&part)[
         float a = __uint_as_float(v[2 * (e & 1)]), b = __uint_as_float(v[2 * (e & 1) + 1]);
 #pragma unroll
         for (int p = 0; p < PARTS; ++p) {
-            const uint32_t r = round_pair(a, b);
+            const uint32_t r = bf16_pair(a, b);
             part[p][e] = r;
             a -= __uint_as_float(r << 16), b -= __uint_as_float(r & 0xffff0000u);
         }

@@ -289,7 +289,7 @@ __device__ __forceinline__ int segment_place(int first, int end, int seq, Segmen
     return cut.by_sequence ? multiple + seq : 2 * multiple + (first + cut.len >= end ? 1 : 0);
 }
 
-// The walk alone, for a prompt's step in bfloat16 whose heads' columns are shared out (D a multiple of 8, rows and
+// The walk alone, of sizes that do not go by blocks (below), for a prompt's step in bfloat16 whose heads' columns are shared out (D a multiple of 8, rows and
 // columns aligned to 16 bytes).  What bounds it: one prompt alone, a wave's chain of tokens (0.36 us each); cut into
 // segments, the vector units (three instructions an element of the state and token, 78 us at 2,048 tokens of 24 heads of 128).  The 16 lanes of one row of a wave share two or four columns of the state, lane r
 // keeping rows r * ROWS .. r * ROWS + ROWS - 1 of each (what a lane reads of q, k and the decays serves all its
@@ -659,6 +659,250 @@ __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __re
         }
 }
 
+// The recurrence by blocks of 16 tokens on the matrix cores, for runs of a prompt in bfloat16.
+// With P_t the products of a block's decays up to token t, R_s those behind token s and S the state in front of the block:
+//   o_t = (q_t * P_t)^T S + sum_(s <= t) A_ts v_s,   A_ts = sum_d q_td k_sd prod_(s < r <= t) alpha_rd,   S <- diag(P_15) S + sum_s (k_s * R_s) v_s^T
+// A = (q P) (k / P)^T where no channel of 64 has decayed to 2^-40 within the block; else its part of A is made pair by pair on the vector units,
+// from products of decays alone, lane (s, four channels) carrying k_s prod alpha from token to token.
+// A workgroup of BLOCK_D / 16 waves has a (segment, head) and BLOCK_D columns of its state, a wave 16 of them, D x 16 floats in the registers in which
+// the matrix cores leave them: lane (r, g) has S[16 b + 4 g + i][r], which is also how S^T is read as a left operand when instruction i of a
+// block of channels takes the channels 4 g + i.  S and A are multiplied as floats (v_mfma_f32_16x16x4_f32); k R goes into the state's
+// product as the three bfloat16 numbers that it is the sum of, values as they are (v_mfma_f32_16x16x16_bf16, float sums).
+// All but the values is staged in LDS a block at a time, requested a block ahead.
+// Segments behind one another: with OUT false only what a segment adds to the state (all but a sequence's last), and the product of its
+// decays; block_states_kernel makes the states in front of the segments; with OUT true the outputs, from there.
+// What bounds it: the barriers between staging, A and products, LDS (a wave reads 13 KiB a block) and the float products (36 of 32
+// cycles), about in equal parts; 124 registers leave two workgroups a unit.
+// us, a layer's recurrence with its decays and the finishing kernel, by the walk (with two or four columns a lane group) -> by blocks:  24 heads
+// of 128 x 128, one run of 33 tokens 29 -> 29, 64 39 -> 33, 128 60 -> 50, 200 85 -> 55, 512 104 -> 66, 2,048 214 -> 142 (the walk, its decays'
+// products, states and outputs 124 + 11 + 13 + 30 -> what segments add, states, outputs 29 + 13 + 64), 4,096 390 -> 244;  16 runs of 64 127 -> 66,
+// of 200 242 -> 157, one run of 449 beside 63 tokens 752 -> 449;  24 of 64 x 64, 2,048 115 -> 89;  8 of 128 x 64, 2,048 109 -> 72.
+// D up to BLOCK_D and a multiple of 16.  KF, q_share, state_stride, BEFORE and the segments as in the walk above.
+constexpr int BLOCK_TOKENS = 16, BLOCK_COLUMN = BLOCK_TOKENS + 4;
+constexpr float BLOCK_LEAST = 9.094947e-13f;      // 2^-40
+typedef short segshort4 __attribute__((ext_vector_type(4)));
+template <int BLOCK_D, bool OUT, bool KF, bool BEFORE>
+__global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
+    const bf16_t* __restrict__ proj, int row_stride, int q_col, int k_col, int v_col, const float* __restrict__ alpha,
+    const float* __restrict__ k_f32, int q_share, float* __restrict__ state, long long state_stride,
+    const int* __restrict__ cu_q, const int* __restrict__ slots, int n_heads, int D, int Dv, float q_scale,
+    float* __restrict__ raw_out, Segments cut, float* __restrict__ seg_state, float* __restrict__ seg_decay) {
+    constexpr int T = BLOCK_TOKENS, TILES = BLOCK_D / 16, BLOCK_WAVES = BLOCK_D / 16, BLOCK_ROW = BLOCK_D + 4, PARTS = 3;
+    __shared__ __attribute__((aligned(16))) float qp_s[OUT ? T * BLOCK_ROW : 4];      // q P, by token
+    __shared__ __attribute__((aligned(16))) float kx_s[OUT ? T * BLOCK_ROW : 4];      // k / P, or k
+    __shared__ __attribute__((aligned(16))) float q_s[OUT ? T * BLOCK_ROW : 4], al_s[OUT ? T * BLOCK_ROW : 4];
+    __shared__ __attribute__((aligned(16))) uint2 kr_s[PARTS][BLOCK_D][4 + 1];       // parts of k R, by channel: four tokens a piece
+    __shared__ __attribute__((aligned(16))) float end_s[BLOCK_D];                     // P of the block's last token
+    __shared__ __attribute__((aligned(16))) float a_s[OUT ? BLOCK_WAVES * T * BLOCK_COLUMN : 4];      // [wave's channels][t][s]
+    __shared__ int by_pairs[2];      // of 64 channels each
+    const int n_slices = (Dv + BLOCK_D - 1) / BLOCK_D;
+    const int seq = blockIdx.x, head = blockIdx.y, slice = blockIdx.z % n_slices, seg = blockIdx.z / n_slices;
+    const int begin = cu_q[seq], first = begin + seg * cut.len, end = cu_q[seq + 1];
+    if (first >= end) return;
+    const bool is_cut = cut.len > 0 && end - begin > cut.len;
+    const int last = is_cut ? min(first + cut.len, end) : end;
+    if (!is_cut && seg > 0) return;
+    if (!OUT && (!is_cut || last == end)) return;
+    const int tid = threadIdx.x, lane = tid % SIA_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / SIA_WAVE), r = lane % 16, g = lane / 16;
+    const int j = slice * BLOCK_D + wave * 16 + r;
+    const bool has_j = slice * BLOCK_D + wave * 16 < Dv;      // Dv is a multiple of 16: a wave has columns or has none
+    const int matrix = D * Dv, from = 4 * g * Dv + j;      // a tile's rows 4 g .. 4 g + 3 begin there
+    float* const own = state + (size_t)slots[seq] * state_stride + (size_t)head * matrix;
+    float* const segment = seg_state + ((size_t)(is_cut ? segment_place(first, end, seq, cut) : 0) * n_heads + head) * matrix;
+    segf32x4 S[TILES];
+#pragma unroll
+    for (int b = 0; b < TILES; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            S[b][i] = 0.f;
+            if (OUT && has_j && 16 * b < D) S[b][i] = (is_cut ? segment : own)[(16 * b + i) * Dv + from];
+        }
+    // Staging: a thread has a channel.  What it makes of the block:  0 q P;  1 k R;  2 k / P
+    const int role = __builtin_amdgcn_readfirstlane(tid / BLOCK_D), ch = tid % BLOCK_D;
+    const bool has_ch = ch < D, stages = OUT ? role < 3 : role == 1;
+    const int at = head / q_share * D + (has_ch ? ch : 0), at_f = head * D + (has_ch ? ch : 0);
+    float x[T], al[T];
+    uint16_t v_next[4];
+    const unsigned x_at = (unsigned)((role == 0 ? q_col : k_col) + at), f_at = (unsigned)at_f, v_at = (unsigned)(v_col + head * Dv + j);
+    auto request = [&](int t0) {      // tokens behind the last repeat it
+        if (stages) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const size_t n = __builtin_amdgcn_readfirstlane(min(t0 + t, last - 1));      // a row begins at a scalar
+                const float* floats = alpha + n * n_heads * D;
+                if (KF && role != 0)
+                    x[t] = (k_f32 + n * n_heads * D)[f_at];
+                else
+                    x[t] = bf16_to_float((proj + n * row_stride)[x_at]);
+                al[t] = floats[f_at];
+            }
+        }
+        if (has_j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v_next[i] = (proj + (size_t)min(t0 + 4 * g + i, last - 1) * row_stride)[v_at];
+    };
+    request(first);
+    float seg_product = 1.f;
+    for (int t0 = first; t0 < last; t0 += T) {
+        const int nt = min(T, last - t0);
+        if (nt < T || !has_ch)
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                if (!has_ch || t >= nt) x[t] = 0.f, al[t] = 1.f;
+        const segshort4 v = {(short)v_next[0], (short)v_next[1], (short)v_next[2], (short)v_next[3]};      // of no weight behind the last token: k is zero there
+        if (role == 1) {
+            float p = 1.f;
+#pragma unroll
+            for (int t = T - 1; t >= 0; --t) {
+                x[t] *= p;
+                p *= al[t];
+            }
+            end_s[ch] = p;
+            seg_product *= p;
+#pragma unroll
+            for (int e = 0; e < PARTS; ++e)
+#pragma unroll
+                for (int t = 0; t < T; t += 4) {
+                    uint2 u;
+                    u.x = bf16_pair(x[t], x[t + 1]), u.y = bf16_pair(x[t + 2], x[t + 3]);
+                    kr_s[e][ch][t / 4] = u;
+                    x[t] -= __uint_as_float(u.x << 16), x[t + 1] -= __uint_as_float(u.x & 0xffff0000u);
+                    x[t + 2] -= __uint_as_float(u.y << 16), x[t + 3] -= __uint_as_float(u.y & 0xffff0000u);
+                }
+        } else if (OUT && stages) {
+            float p = 1.f;
+#pragma unroll
+            for (int t = 0; t < T; ++t) p *= al[t];
+            const bool pairs = __any(!(p >= BLOCK_LEAST));
+            p = 1.f;
+            if (role == 0) {
+                if (lane == 0) by_pairs[wave % (BLOCK_D / 64)] = pairs;
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    if (!BEFORE) p *= al[t];
+                    qp_s[t * BLOCK_ROW + ch] = x[t] * q_scale * p;
+                    if (BEFORE) p *= al[t];
+                }
+                if (pairs)
+#pragma unroll
+                    for (int t = 0; t < T; ++t) q_s[t * BLOCK_ROW + ch] = x[t] * q_scale, al_s[t * BLOCK_ROW + ch] = al[t];
+            } else {
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    p *= al[t];
+                    kx_s[t * BLOCK_ROW + ch] = pairs ? x[t] : x[t] / p;
+                }
+            }
+        }
+        __syncthreads();
+        if (t0 + T < last) request(t0 + T);
+        if (OUT) {
+            const int c = wave * 16 + 4 * g;      // the lane's four of the wave's 16 channels
+            const float4 k4 = *reinterpret_cast<const float4*>(kx_s + r * BLOCK_ROW + c);
+            segf32x4 A = {0.f, 0.f, 0.f, 0.f};      // A_ts of t = 4 g + i, s = r
+            if (!by_pairs[wave / 4]) {
+                const float4 q4 = *reinterpret_cast<const float4*>(qp_s + r * BLOCK_ROW + c);
+                A = __builtin_amdgcn_mfma_f32_16x16x4f32(q4.x, k4.x, A, 0, 0, 0);
+                A = __builtin_amdgcn_mfma_f32_16x16x4f32(q4.y, k4.y, A, 0, 0, 0);
+                A = __builtin_amdgcn_mfma_f32_16x16x4f32(q4.z, k4.z, A, 0, 0, 0);
+                A = __builtin_amdgcn_mfma_f32_16x16x4f32(q4.w, k4.w, A, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (BEFORE ? 4 * g + i <= r : 4 * g + i < r) A[i] = 0.f;
+            } else {
+                // a token's sums of the four lane groups go to its row by a product with a row of ones
+                float4 ck = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 2
+                for (int t = 0; t < T; ++t) {
+                    const float4 q4 = *reinterpret_cast<const float4*>(q_s + t * BLOCK_ROW + c);
+                    const float4 a4 = *reinterpret_cast<const float4*>(al_s + t * BLOCK_ROW + c);
+                    if (!BEFORE) ck = t == r ? k4 : make_float4(ck.x * a4.x, ck.y * a4.y, ck.z * a4.z, ck.w * a4.w);
+                    const float sum = (q4.x * ck.x + q4.y * ck.y) + (q4.z * ck.z + q4.w * ck.w);
+                    A = __builtin_amdgcn_mfma_f32_16x16x4f32(t == r ? 1.f : 0.f, sum, A, 0, 0, 0);
+                    if (BEFORE) ck = t == r ? k4 : make_float4(ck.x * a4.x, ck.y * a4.y, ck.z * a4.z, ck.w * a4.w);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a_s[(wave * T + 4 * g + i) * BLOCK_COLUMN + r] = A[i];
+            __syncthreads();
+        }
+        if (has_j) {
+            if (OUT) {
+                segf32x4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                float4 a4 = make_float4(0.f, 0.f, 0.f, 0.f);      // A_ts of t = r, s = 4 g .. 4 g + 3
+#pragma unroll 2
+                for (int w = 0; w < BLOCK_WAVES; ++w) {
+                    const float4 part = *reinterpret_cast<const float4*>(a_s + (w * T + r) * BLOCK_COLUMN + 4 * g);
+                    a4.x += part.x, a4.y += part.y, a4.z += part.z, a4.w += part.w;
+                }
+#pragma unroll
+                for (int b = 0; b < TILES; ++b) {
+                    const float4 qp = *reinterpret_cast<const float4*>(qp_s + r * BLOCK_ROW + 16 * b + 4 * g);
+                    o[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[b][0], qp.x, o[b & 1], 0, 0, 0);
+                    o[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[b][1], qp.y, o[b & 1], 0, 0, 0);
+                    o[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[b][2], qp.z, o[b & 1], 0, 0, 0);
+                    o[b & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[b][3], qp.w, o[b & 1], 0, 0, 0);
+                    if (b % 2) __builtin_amdgcn_sched_barrier(0);      // operands of two steps in registers, not of all
+                }
+                segf32x4 av = {0.f, 0.f, 0.f, 0.f};
+                av = __builtin_amdgcn_mfma_f32_16x16x4f32(bf16_to_float((uint16_t)v[0]), a4.x, av, 0, 0, 0);
+                av = __builtin_amdgcn_mfma_f32_16x16x4f32(bf16_to_float((uint16_t)v[1]), a4.y, av, 0, 0, 0);
+                av = __builtin_amdgcn_mfma_f32_16x16x4f32(bf16_to_float((uint16_t)v[2]), a4.z, av, 0, 0, 0);
+                av = __builtin_amdgcn_mfma_f32_16x16x4f32(bf16_to_float((uint16_t)v[3]), a4.w, av, 0, 0, 0);
+                // columns 4 g .. 4 g + 3 of token r
+                const segf32x4 sum = (o[0] + o[1]) + av;
+                if (r < nt)
+                    *reinterpret_cast<segf32x4*>(raw_out + ((size_t)(t0 + r) * n_heads + head) * Dv + slice * BLOCK_D + wave * 16 + 4 * g) = sum;
+            }
+#pragma unroll
+            for (int b = 0; b < TILES; ++b) {
+                const float4 p = *reinterpret_cast<const float4*>(end_s + 16 * b + 4 * g);
+                segf32x4 added = {0.f, 0.f, 0.f, 0.f};      // small parts first
+#pragma unroll
+                for (int e = PARTS - 1; e >= 0; --e)
+                    added = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(segshort4, kr_s[e][16 * b + r][g]), v, added, 0, 0, 0);
+                S[b][0] = fmaf(S[b][0], p.x, added[0]), S[b][1] = fmaf(S[b][1], p.y, added[1]);
+                S[b][2] = fmaf(S[b][2], p.z, added[2]), S[b][3] = fmaf(S[b][3], p.w, added[3]);
+                if (b % 2) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __syncthreads();
+    }
+    if (!OUT && role == 1 && has_ch && slice == 0)
+        seg_decay[((size_t)segment_place(first, end, seq, cut) * n_heads + head) * D + ch] = seg_product;
+    if (has_j && (!OUT || last == end))
+#pragma unroll
+        for (int b = 0; b < TILES; ++b)
+            if (16 * b < D)      // a multiple of 16
+#pragma unroll
+                for (int i = 0; i < 4; ++i) (OUT ? own : segment)[(16 * b + i) * Dv + from] = S[b][i];
+}
+
+// The state in front of every segment of a sequence that is cut, in place of what the segment adds to it.  A thread four neighbouring
+// elements of a matrix.
+__global__ __launch_bounds__(256) void block_states_kernel(const float* __restrict__ seg_decay, float* __restrict__ seg_state,
+                                                           const float* __restrict__ state, long long state_stride,
+                                                           const int* __restrict__ cu_q, const int* __restrict__ slots, int n_heads,
+                                                           int D, int Dv, Segments cut) {
+    const int seq = blockIdx.z, head = blockIdx.y, at = (blockIdx.x * 256 + threadIdx.x) * 4;
+    const int begin = cu_q[seq], end = cu_q[seq + 1];
+    if (end - begin <= cut.len || at >= D * Dv) return;
+    const int d = at / Dv;
+    float4 S = *reinterpret_cast<const float4*>(state + (size_t)slots[seq] * state_stride + (size_t)head * D * Dv + at);
+    auto place = [&](int first) { return (size_t)segment_place(first, end, seq, cut) * n_heads + head; };
+    auto matrix = [&](int first) { return reinterpret_cast<float4*>(seg_state + place(first) * D * Dv + at); };
+    float4 added = *matrix(begin);
+    float a = seg_decay[place(begin) * D + d];
+    for (int first = begin; first < end; first += cut.len) {
+        const bool more = first + 2 * cut.len < end;      // the segment behind this one is not the last
+        const float4 now = added;
+        const float now_a = a;
+        if (more) added = *matrix(first + cut.len), a = seg_decay[place(first + cut.len) * D + d];
+        *matrix(first) = S;
+        if (first + cut.len < end) S = make_float4(now_a * S.x + now.x, now_a * S.y + now.y, now_a * S.z + now.z, now_a * S.w + now.w);
+    }
+}
+
 // alpha[n, c] = exp(logsigmoid(a2_bias[c] + sum_m a[n, m] * A2[c, m]) / tau) for every token n and key channel c of all
 // heads: a thread a channel, eight tokens a workgroup (their low-rank inputs staged in LDS, a channel's row of A2
 // read once for the eight).
@@ -832,6 +1076,11 @@ static bool gla_slices(int n_seqs, int max_q_len, int n_heads) {
 #define SEG_MIN 64
 #define WALK_MIN_RUN 128
 
+// Whether runs go by blocks on the matrix cores, from BLOCKS_MIN_RUN tokens on (two blocks: even with the walk, 29 us for 24 heads of
+// 128 x 128; one block of 20 tokens 25 / 24).  States that leave more than half of a workgroup's channels or columns empty are walked.
+#define BLOCKS_MIN_RUN 32
+static bool by_blocks(int D, int Dv) { return D % 16 == 0 && D >= 64 && D <= 128 && Dv % 16 == 0 && Dv >= 64; }
+
 static long long segment_places(int n_tokens, int n_seqs, Segments cut) {
     if (cut.len == 0) return 0;
     const long long multiples = (n_tokens - 1) / cut.len + 1;
@@ -963,7 +1212,8 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
     // the walk with requests a block ahead, where its pieces are aligned and fit its registers.  (Its workgroups take
     // as many columns as their threads hold whatever the step: the waves of a workgroup share the staged tokens, and
     // what bounds the walk is a wave's own chain of tokens, not the number of workgroups.)
-    const bool long_runs = max_q_len >= WALK_MIN_RUN && Dv % 4 == 0 && n_seqs <= 65535 && n_heads * ((Dv + 63) / 64) <= 65535 &&
+    const bool blocks = by_blocks(D, Dv) && max_q_len >= BLOCKS_MIN_RUN;
+    const bool long_runs = (max_q_len >= WALK_MIN_RUN || blocks) && Dv % 4 == 0 && n_seqs <= 65535 && n_heads * ((Dv + 63) / 64) <= 65535 &&
                            ((uintptr_t)raw_space % 16) == 0 && ((uintptr_t)state % 16) == 0 && state_stride % 4 == 0;
     Segments cut{0, false};
     if (long_runs) cut = segments_of(n_tokens, n_seqs, max_q_len, n_heads, D, Dv, dtype);
@@ -982,6 +1232,36 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
         const int w_slices = (Dv + w_slice - 1) / w_slice;
         const int seg_len = cut.len, n_segs = seg_len ? (max_q_len + seg_len - 1) / seg_len : 1;
         float* seg_state = raw_space + (size_t)n_tokens * n_heads * Dv;
+        if (blocks && long_runs) {
+            float* seg_decay = raw;      // behind the states nobody reads them, and the outputs come after
+            const int width = D <= 64 && Dv <= 64 ? 64 : 128;
+            const dim3 bgrid(n_seqs, n_heads, (Dv + width - 1) / width * n_segs), bblock(width / 16 * SIA_WAVE);
+#define BLOCKS_AS(WIDTH, OUT, KF, BEFORE)                                                                                    \
+    hipLaunchKernelGGL((gla_blocks_kernel<WIDTH, OUT, KF, BEFORE>), bgrid, bblock, 0, stream, (const bf16_t*)proj, row_stride,   \
+                       q_col, k_col, v_col, alpha, k_f32, q_share, state, state_stride, cu_q, slots, n_heads, D, Dv, q_scale,   \
+                       raw, cut, seg_state, seg_decay)
+#define BLOCKS_OF(WIDTH, OUT)                                                                                                \
+    do {                                                                                                                     \
+        if (bonus) BLOCKS_AS(WIDTH, OUT, false, true);                                                                       \
+        else if (k_f32) BLOCKS_AS(WIDTH, OUT, true, false);                                                                  \
+        else BLOCKS_AS(WIDTH, OUT, false, false);                                                                            \
+    } while (0)
+#define BLOCKS(OUT)                                                                                                          \
+    do {                                                                                                                     \
+        if (width == 64) BLOCKS_OF(64, OUT);                                                                                 \
+        else BLOCKS_OF(128, OUT);                                                                                            \
+    } while (0)
+            if (n_segs > 1) {
+                BLOCKS(false);
+                hipLaunchKernelGGL(block_states_kernel, dim3((D * Dv / 4 + 255) / 256, n_heads, n_seqs), dim3(256), 0, stream, seg_decay,
+                                   seg_state, state, state_stride, cu_q, slots, n_heads, D, Dv, cut);
+            }
+            BLOCKS(true);
+#undef BLOCKS
+#undef BLOCKS_OF
+#undef BLOCKS_AS
+            return 0;
+        }
         dim3 wgrid(n_seqs, n_heads, w_slices * n_segs), wblock(GLA_WALK_THREADS);
 #define WALK_AS(ROWS, COLS, KF, BEFORE)                                                                                      \
     hipLaunchKernelGGL((gla_walk_kernel<ROWS, COLS, KF, BEFORE>), wgrid, wblock, w_lds, stream, (const bf16_t*)proj,         \

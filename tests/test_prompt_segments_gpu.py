@@ -87,6 +87,46 @@ def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, len
     assert float(state[len(lengths):].abs().max()) == 0.0        # nobody else's slot was touched
 
 
+@pytest.mark.parametrize("decay", ["usual", "strong", "mixed"])
+@pytest.mark.parametrize("H,D,Dv,lengths", [
+    (2, 64, 64, [32, 1, 15, 16, 17]), (3, 128, 128, [33, 47, 2]), (2, 80, 192, [100, 31, 1]), (1, 112, 80, [48] * 5), (2, 64, 144, [200, 3]),
+    (2, 128, 64, [513]), (1, 128, 128, [177, 300])])
+def test_runs_by_blocks_against_64_bits(H, D, Dv, lengths, decay):
+    """Whole and cut runs, last blocks of one to 16 tokens, widths that leave waves or channels idle; decays as trained, decays that
+    leave nothing within a block (which go pair by pair), and those in some channels only.  A state's error is that of its decays
+    (four units in the last place a token) and of some 100 sums, of what the same recurrence gives with absolute values."""
+    from simple_inference_amd.kernels import HipKernels
+
+    k, rank, tau, n = HipKernels(), 32, 16.0, sum(lengths)
+    g = torch.Generator().manual_seed(D + Dv)
+    cols = (0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv))
+    rows = rnd(g, n, cols[4] + rank).to(torch.bfloat16).to(DEV)
+    a2, bias = rnd(g, H * D, rank, std=0.1).to(torch.bfloat16).to(DEV), rnd(g, H * D, std=0.1).to(DEV)
+    if decay != "usual":
+        bias -= 2000.0
+    if decay == "mixed":
+        bias.view(H, D)[:, :D // 2] += 2000.0
+    norm = (1 + rnd(g, Dv, std=0.2)).float().to(DEV)
+    state = rnd(g, len(lengths), H, D, Dv).float().to(DEV)
+    want, size = state.double(), state.double().abs()
+    x = rows.double()
+    q, key = (x[:, cols[i]:cols[i] + H * D].view(n, H, D, 1) for i in (0, 1))
+    v, gate = (x[:, cols[i]:cols[i] + H * Dv].view(n, H, 1, Dv) for i in (2, 3))
+    alpha = torch.exp(torch.nn.functional.logsigmoid(x[:, cols[4]:] @ a2.double().T + bias.double()) / tau).view(n, H, D, 1)
+    o, t = torch.empty(n, H, Dv, dtype=torch.float64, device=DEV), 0
+    for s, length in enumerate(lengths):
+        for _ in range(length):
+            want[s] = alpha[t] * want[s] + key[t] * v[t]
+            size[s] = alpha[t] * size[s] + (key[t] * v[t]).abs()
+            o[t] = (want[s] * q[t]).sum(1) * D ** -0.5
+            t += 1
+    y = k.gla_recurrent(rows, cols, a2, bias.float(), norm, H, D, Dv, tau, D ** -0.5, 1e-5, context(DEV, lengths, list(range(len(lengths)))),
+                        LayerCache(state=state)).double().view(n, H, Dv)
+    ref = o * torch.rsqrt((o * o).mean(-1, keepdim=True) + 1e-5) * norm.double() * torch.nn.functional.silu(gate.squeeze(2))
+    assert bool(((state.double() - want).abs() <= (4 * max(lengths) + 100) * 2.0 ** -24 * size + 1e-30).all())
+    assert bool(((y - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.std()).all()), float((y - ref).abs().max())
+
+
 # narrow and wide values, rows that do not divide by the groups of threads, the most rows a thread takes; value widths that
 # are no power of two go the general way
 @pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
