@@ -127,6 +127,33 @@ def test_runs_by_blocks_against_64_bits(H, D, Dv, lengths, decay):
     assert bool(((y - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.std()).all()), float((y - ref).abs().max())
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("H,Dv,n", [(1, 8, 3), (3, 24, 33), (5, 64, 51), (2, 136, 40), (3, 256, 7), (2, 512, 129), (3, 20, 33)])
+def test_norm_and_gate_behind_a_prompt_s_recurrence(H, Dv, n, shift):
+    """Groups of one to 64 lanes a (token, head), lanes without elements, a last workgroup in part, and rows that do not begin at 16
+    bytes (the general form).  With decays and keys that leave the outputs q k v of one channel, each is known to a few
+    roundings of float; the result is rounded once to bfloat16 (2^-9)."""
+    from simple_inference_amd.kernels import HipKernels
+
+    k, D, rank, eps = HipKernels(), 16, 8, 1e-5
+    g = torch.Generator().manual_seed(Dv + shift)
+    cols = (0, H * D, 2 * H * D, 2 * H * D + H * Dv + shift, 2 * H * (D + Dv) + 8)
+    rows = rnd(g, n, cols[4] + rank).to(torch.bfloat16)
+    a2, bias = torch.zeros(H * D, rank, dtype=torch.bfloat16), torch.full((H * D,), -1e6)      # a state forgets what was before
+    norm = (1 + rnd(g, Dv, std=0.2)).float()
+    state = torch.zeros(1, H, D, Dv, device=DEV)
+    x = rows.double()
+    q, key = (x[:, cols[i]:cols[i] + H * D].view(n, H, D) for i in (0, 1))
+    v, gate = (x[:, cols[i]:cols[i] + H * Dv].view(n, H, Dv) for i in (2, 3))
+    o = (q * key).sum(-1, keepdim=True) * D ** -0.5 * v
+    ref = o * torch.rsqrt((o * o).mean(-1, keepdim=True) + eps) * norm.double() * torch.nn.functional.silu(gate)
+    y = k.gla_recurrent(rows.to(DEV), cols, a2.to(DEV), bias.to(DEV), norm.to(DEV), H, D, Dv, 1.0, D ** -0.5, eps,
+                        context(DEV, [n], [0]), LayerCache(state=state)).double().cpu().view(n, H, Dv)
+    # the sum over D may cancel: 18 roundings of its terms' sizes beside it, which the norm passes on at most whole
+    spread = 18 * 2.0 ** -24 * (q * key).abs().sum(-1, keepdim=True) / (q * key).sum(-1, keepdim=True).abs()
+    assert bool(((y - ref).abs() <= (2.0 ** -8 + spread) * ref.abs() + 1e-30).all()), float((y - ref).abs().max())
+
+
 # narrow and wide values, rows that do not divide by the groups of threads, the most rows a thread takes; value widths that
 # are no power of two go the general way
 @pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
