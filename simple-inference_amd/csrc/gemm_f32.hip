@@ -15,7 +15,9 @@
 // of them are zero changes no bit: they add zero.
 //
 // Infinities and NaN, and finite numbers that round to an infinite part: some product of parts is then not finite, and neither is
-// the result.  A result that is not finite is made again, k after k with fused multiply-adds (plain_sum).
+// the result.  A result that is not finite is made again from the floats as they are, on the float matrix cores (float_sums), 16 x 16
+// results a wave at a time.  us, by a thread a result, k after k -> now (and without any):  a row of NaN among 303, x 128,256 x 2,048 8,450 -> 1,131
+// (726), x 2,048 x 2,048 1,208 -> 67 (32), all 303 of them 2,996 -> 124;  one row alone, x 128,256 x 2,048 4,400 -> 401 (194).
 //
 // * Few rows: a workgroup's waves stream W past the step's rows.  Bound by reading W, or by what the workgroups fetch from L2.
 // * More rows: X is split into its parts ahead, once, in the order in which the matrix cores read it; tiles of Y, X's parts and W as it
@@ -86,10 +88,45 @@ __device__ __forceinline__ void chunk_of_parts(const u32x4 (&w)[TN][PARTS], cons
 
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
 
-__device__ __forceinline__ float plain_sum(const float* __restrict__ x, const float* __restrict__ w, int K) {
-    float s = 0.f;
-    for (int k = 0; k < K; ++k) s = fmaf(x[k], w[k], s);
-    return s;
+// A block of 16 x 16 results by v_mfma_f32_16x16x4_f32, for those that the parts do not give:  x and w are the rows r = lane % 16 of either
+// operand, the lane gets row r and columns 4 g .. 4 g + 3, g = lane / 16.  All lanes take part.  Pieces of 16 k go to four sums in
+// turn, (s0 + s1) + (s2 + s3): a result depends on its row and column alone, whoever asks for it.
+__device__ __forceinline__ f32x4 float_sums(const float* __restrict__ x, const float* __restrict__ w, int K) {
+    const int g = (threadIdx.x % SIA_WAVE) / 16;
+    const bool wide = __all(K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0);
+    f32x4 sum[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) sum[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma clang loop unroll(disable)
+    for (int k0 = 0; k0 < K; k0 += 64) {      // pieces of 16 k, 4 g .. 4 g + 3 of each in this lane; zeros behind the last k
+        f32x4 a[4], b[4];
+        if (wide) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int at = min(k0 + 16 * s + 4 * g, K - 4);
+                a[s] = *(const f32x4*)(w + at), b[s] = *(const f32x4*)(x + at);
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int at = min(k0 + 16 * s + 4 * g + i, K - 1);
+                    a[s][i] = w[at], b[s][i] = x[at];
+                }
+        }
+        if (k0 + 64 > K)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (k0 + 16 * s + 4 * g + i >= K) a[s][i] = 0.f, b[s][i] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) sum[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][i], b[s][i], sum[s], 0, 0, 0);
+    }
+    return (sum[0] + sum[1]) + (sum[2] + sum[3]);
 }
 
 // Slices of K, in chunks: from N and K alone.  Few rows of W beside a long K are too little for the chip without; an output head
@@ -259,18 +296,26 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
             multiply(s, wa, wb, xa, xb);
         }
     }
-    // row m of Y and its four columns from n on
+    // a block of results from row m and column n on
     auto finish = [&](int m, int n, f32x4 v) {
-        if (m >= M) return;
+        bool odd = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) odd |= m + r < M && n + 4 * g + e < N && !finite(v[e]);
+        if (__any(odd)) {
+            const f32x4 again = float_sums(X + (size_t)min(m + r, M - 1) * K, W + (size_t)min(n + r, N - 1) * K, K);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = finite(v[e]) ? v[e] : again[e];
+        }
+        if (m + r >= M) return;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            if (n + e < N) Y[(size_t)m * N + n + e] = finite(v[e]) ? v[e] : plain_sum(X + (size_t)m * K, W + (size_t)(n + e) * K, K);
+            if (n + 4 * g + e < N) Y[(size_t)(m + r) * N + n + 4 * g + e] = v[e];
     };
     if (SLICES == 1) {
 #pragma unroll
         for (int b = 0; b < MB; ++b)
 #pragma unroll
-            for (int j = 0; j < NB; ++j) finish(m0 + b * 16 + r, n0 + j * 16 + 4 * g, total[b][j]);
+            for (int j = 0; j < NB; ++j) finish(m0 + b * 16, n0 + j * 16, total[b][j]);
         return;
     }
     f32x4* const part = (f32x4*)lds;
@@ -288,7 +333,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
         f32x4 v = part[block * SIA_WAVE + lane];
 #pragma unroll
         for (int s = 1; s < SLICES; ++s) v += part[(s * BLOCKS + block) * SIA_WAVE + lane];
-        finish(m0 + block / NB % MB * 16 + r, (blockIdx.x * GROUPS + block / (MB * NB)) * NB * 16 + block % NB * 16 + 4 * g, v);
+        finish(m0 + block / NB % MB * 16, (blockIdx.x * GROUPS + block / (MB * NB)) * NB * 16 + block % NB * 16, v);
     }
 }
 
@@ -555,30 +600,45 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
         }
     }
     store(more);
-    if (apart || !odd) return;
+    if (apart || !__any(odd)) return;
 #pragma clang loop unroll(disable)
-    for (int i = 0; i < TM * TN * 4; ++i) {
-        const int m = m_first + i / (TN * 4) * 16, n = n_first + i / 4 % TN * 16 + i % 4;
-        if (m >= M || n >= N) continue;
+    for (int i = 0; i < TM * TN; ++i) {      // a lane's results are what it has stored
+        const int m = m_first + i / TN * 16, n = n_first + i % TN * 16;
         float* at = Y + (size_t)m * N + n;
-        if (!finite(*(volatile float*)at)) *at = plain_sum(X + (size_t)m * K, W + (size_t)n * K, K);
+        unsigned again = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (m < M && n + e < N && !finite(*(volatile float*)(at + e))) again |= 1u << e;
+        if (!__any(again != 0)) continue;
+        const f32x4 v = float_sums(X + (size_t)min(m, M - 1) * K, W + (size_t)min(n - 4 * g + r, N - 1) * K, K);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (again >> e & 1) at[e] = v[e];
     }
 }
 
-// Y = the slices' sums added in order.  Four elements of a row a thread.
+// Y = the slices' sums added in order.  A wave has 16 rows and columns, as float_sums gives them, a workgroup 64 columns.
 __global__ __launch_bounds__(256) void sum_slices_f32_kernel(const float* __restrict__ slices, const float* __restrict__ X,
-                                                             const float* __restrict__ W, float* __restrict__ Y, int N, int K, int Ns, int n_slices,
-                                                             size_t elements, bool four) {
-    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;      // of M rows of Ns
-    if (i >= elements) return;
-    const size_t m = i / Ns;
-    const int n = (int)(i % Ns);
+                                                             const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K, int Ns,
+                                                             int n_slices, bool four) {
+    const int lane = threadIdx.x % SIA_WAVE, r = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.y * 64 + threadIdx.x / SIA_WAVE * 16, n = n0 + 4 * g;
+    const long long m = (long long)blockIdx.x * 16 + r;
+    if (n0 >= N) return;      // a wave leaves as a whole
+    const bool live = m < M && n < N;
+    const size_t elements = (size_t)M * Ns, i = live ? m * Ns + n : 0;
     f32x4 v = *(const f32x4*)(slices + i);
     for (int s = 1; s < n_slices; ++s) v += *(const f32x4*)(slices + s * elements + i);
+    bool odd = false;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (!finite(v[e]) && n + e < N) v[e] = plain_sum(X + m * K, W + (size_t)(n + e) * K, K);
-    float* at = Y + m * N + n;
+    for (int e = 0; e < 4; ++e) odd |= live && n + e < N && !finite(v[e]);
+    if (__any(odd)) {
+        const f32x4 again = float_sums(X + (size_t)(m < M ? m : M - 1) * K, W + (size_t)min(n0 + r, N - 1) * K, K);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = finite(v[e]) ? v[e] : again[e];
+    }
+    if (!live) return;
+    float* at = Y + (size_t)m * N + n;
     if (four)
         *(f32x4*)at = v;
     else
@@ -719,7 +779,7 @@ SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* work
     SHAPE(4, 32, 64, 2, 2, 2);
 #undef SHAPE
     if (status == 0 && apart)
-        hipLaunchKernelGGL(sum_slices_f32_kernel, dim3((unsigned)(((size_t)M * Ns / 4 + 255) / 256)), dim3(256), 0, stream, slices, X, W, Y, N, K, Ns,
-                           slices_of(N, K), (size_t)M * Ns, four);
+        hipLaunchKernelGGL(sum_slices_f32_kernel, dim3((M + 15) / 16, (N + 63) / 64), dim3(256), 0, stream, slices, X, W, Y, M, N, K, Ns,
+                           slices_of(N, K), four);
     return status ? status : SIA_LAUNCH_CHECK();
 }

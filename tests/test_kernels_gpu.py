@@ -582,6 +582,38 @@ def test_float32_products_that_are_not_finite(hip, M, N, K):
             assert torch.equal(want[odd], got[odd])
 
 
+@pytest.mark.parametrize("M, N, K", [(1, 33000, 2048), (40, 12800, 2048), (303, 16384, 2048), (303, 2048, 2048), (303, 33000, 1024)])
+def test_float32_products_that_are_not_finite_keep_a_step_s_pace(hip, M, N, K):
+    """A row of NaN is made again by whole blocks: eight times the product's own time is far from one thread after the other's walks (12 to
+    90 times) and from what it takes (under four).  What is made again has the same bits whoever makes it."""
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    huge = x.clone()
+    huge[M // 2, 5::7] = 3.3999e38      # rounds to an infinite part: the floats' product, finite
+    some = w * 1e-30
+    got = hip.linear(huge, some)
+    assert bool(torch.isfinite(got).all()) and torch.equal(got[M // 2:M // 2 + 1], hip.linear(huge[M // 2:M // 2 + 1], some))
+    want, size = huge.double() @ some.double().T, huge.double().abs() @ some.double().abs().T
+    assert bool(((got.double() - want).abs() <= (24 + K / 4) * 2.0 ** -24 * size).all())
+
+    def us(x):
+        times = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            a.record()
+            hip.linear(x, w)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) * 1e3)
+        return min(times)
+
+    plain = us(x)
+    x[M // 2, 3] = float("nan")
+    odd = us(x)
+    assert bool(torch.isnan(hip.linear(x, w)[M // 2]).all())
+    assert odd <= 8 * plain + 20, (odd, plain)
+
+
 def test_float32_product_has_no_reduced_precision(hip):
     """An operand bit below bfloat16 (8 bits) and tf32 (10 bits) resolution must reach the product."""
     K = 8
