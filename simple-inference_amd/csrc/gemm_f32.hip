@@ -1,7 +1,8 @@
 // Y[M, N] = X[M, K] * W[N, K]^T in float: the product of the 32-bit path, on the bfloat16 matrix cores.
 //
 // A float of 24 bits is the sum of three bfloat16 numbers, exactly: x0 = x rounded, x1 = (x - x0) rounded, x2 = x - x0 - x1.
-// (Parts below 2^-133 vanish: of numbers under 2^-110 the last bits.)  A product of two parts is exact in float, and of the nine
+// (A number under 2^-110 may have a rest below 2^-133, which no bfloat16 number holds: its results are made as those that are not finite,
+// below.)  A product of two parts is exact in float, and of the nine
 // products of parts the six above 2^-24 of the whole are summed: x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0.  The matrix cores
 // multiply bfloat16 sixteen times as fast as float, so six products are 2.7 times as fast, and weights that are
 // bfloat16 numbers kept in 32 bits (a checkpoint's) have parts w1 = w2 = 0 and need three.
@@ -40,18 +41,38 @@ constexpr int PART_BLOCK = PARTS * SIA_WAVE;      // 16-byte pieces of the parts
 // parts and products
 // ---------------------------------------------------------------------------------------------------------
 
-// The parts of eight consecutive floats, each eight bfloat16 in order.
-__device__ __forceinline__ void split8(u32x4 first, u32x4 second, u32x4 (&part)[PARTS]) {
+// The parts of eight consecutive floats, each eight bfloat16 in order.  Returned: bits of which the low 16 are zero if the parts are all there
+// is of them.  (What is left for the third part has eight bits; below 2^-126, of a number under 2^-110, they may reach lower than
+// bfloat16 does.  NaN, where some part is not finite, ends in zeros too.)
+__device__ __forceinline__ uint32_t split8(u32x4 first, u32x4 second, u32x4 (&part)[PARTS]) {
+    uint32_t rest = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const u32x4& v = e < 2 ? first : second;
         float a = __uint_as_float(v[2 * (e & 1)]), b = __uint_as_float(v[2 * (e & 1) + 1]);
 #pragma unroll
-        for (int p = 0; p < PARTS; ++p) {
+        for (int p = 0; p < PARTS - 1; ++p) {
             const uint32_t r = bf16_pair(a, b);
             part[p][e] = r;
             a -= __uint_as_float(r << 16), b -= __uint_as_float(r & 0xffff0000u);
         }
+        part[PARTS - 1][e] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302);
+        rest |= __float_as_uint(a) | __float_as_uint(b);
+    }
+    return rest;
+}
+
+// Whether any lane's parts leave something out.
+__device__ __forceinline__ bool any_rest(uint32_t rest) { return __any((rest & 0xffffu) != 0); }
+
+// NaN for the third part of those of the eight floats that have a rest: what they are multiplied with is then made again.
+__device__ __forceinline__ void mark_rests(u32x4 first, u32x4 second, u32x4& third) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float v = __uint_as_float((e < 4 ? first : second)[e % 4]);
+#pragma unroll
+        for (int p = 0; p < PARTS - 1; ++p) v -= __uint_as_float(bf16_pair(v, v) << 16);
+        if (__float_as_uint(v) & 0xffffu) third[e / 2] |= e % 2 ? 0x7fff0000u : 0x7fffu;
     }
 }
 
@@ -167,6 +188,11 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
     for (int b = 0; b < MB; ++b)
 #pragma unroll
         for (int j = 0; j < NB; ++j) total[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    uint32_t rest_x[MB], rest_w[NB];      // of the rows r (a branch at every split: 17 rows x 2,048 x 8,192 22.8 us, 22.0 so)
+#pragma unroll
+    for (int b = 0; b < MB; ++b) rest_x[b] = 0;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) rest_w[j] = 0;
     // U chunks from s on; chunks behind the last are zeros, which change nothing
     auto multiply = [&](int s, u32x4 (&wa)[U][NB], u32x4 (&wb)[U][NB], u32x4 (&xa)[U][MB], u32x4 (&xb)[U][MB]) {
         const u32x4 none = {0, 0, 0, 0};
@@ -196,7 +222,7 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
 #pragma unroll
                 for (int b = 0; b < MB; ++b) {
                     u32x4 x[PARTS];
-                    split8(xa[u][b], xb[u][b], x);
+                    rest_x[b] |= split8(xa[u][b], xb[u][b], x);
                     chunk_one_part(w0, x, t[u][b]);
                 }
             }
@@ -212,11 +238,11 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
             for (int u = 0; u < U; ++u) {
                 u32x4 w[NB][PARTS];
 #pragma unroll
-                for (int j = 0; j < NB; ++j) split8(wa[u][j], wb[u][j], w[j]);
+                for (int j = 0; j < NB; ++j) rest_w[j] |= split8(wa[u][j], wb[u][j], w[j]);
 #pragma unroll
                 for (int b = 0; b < MB; ++b) {
                     u32x4 x[PARTS];
-                    split8(xa[u][b], xb[u][b], x);
+                    rest_x[b] |= split8(xa[u][b], xb[u][b], x);
                     chunk_of_parts(w, x, t[u][b]);
                 }
             }
@@ -295,6 +321,31 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
             }
             multiply(s, wa, wb, xa, xb);
         }
+    }
+    uint32_t rest = 0;
+#pragma unroll
+    for (int b = 0; b < MB; ++b) rest |= rest_x[b];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) rest |= rest_w[j];
+    if (any_rest(rest)) {      // the results of these rows of X and W are made again
+        auto row_has = [&](uint32_t v) {
+            v |= __shfl_xor(v, 16, SIA_WAVE);
+            return ((v | __shfl_xor(v, 32, SIA_WAVE)) & 0xffffu) != 0;
+        };
+        bool has_x[MB], has_w[NB];
+#pragma unroll
+        for (int b = 0; b < MB; ++b) has_x[b] = row_has(rest_x[b]);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) has_w[j] = row_has(rest_w[j]);
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool column = __shfl(has_w[j], 4 * g + e, SIA_WAVE);
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+                    if (has_x[b] || column) total[b][j][e] = __builtin_nanf("");
+            }
     }
     // a block of results from row m and column n on
     auto finish = [&](int m, int n, f32x4 v) {
@@ -414,7 +465,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
 #pragma unroll
         for (int e = 0; e < 8; ++e)
             if (row < M && k + e < K) v[e / 4][e % 4] = from[e];
-    split8(v[0], v[1], p);
+    if (split8(v[0], v[1], p) & 0xffffu) mark_rests(v[0], v[1], p[PARTS - 1]);
     u32x4* at = parts + ((long long)c * blocks + b) * PART_BLOCK + lane;
 #pragma unroll
     for (int e = 0; e < PARTS; ++e) at[e * SIA_WAVE] = p[e];
@@ -570,8 +621,12 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
             }
         } else {
             u32x4 w[TN][PARTS];
+            uint32_t rest = 0;
 #pragma unroll
-            for (int j = 0; j < TN; ++j) split8(a[j], b[j], w[j]);
+            for (int j = 0; j < TN; ++j) rest |= split8(a[j], b[j], w[j]);
+            if (any_rest(rest))
+#pragma unroll
+                for (int j = 0; j < TN; ++j) mark_rests(a[j], b[j], w[j][PARTS - 1]);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
                 u32x4 x[PARTS];

@@ -614,6 +614,26 @@ def test_float32_products_that_are_not_finite_keep_a_step_s_pace(hip, M, N, K):
     assert odd <= 8 * plain + 20, (odd, plain)
 
 
+@pytest.mark.parametrize("M, N, K", [(3, 96, 64), (40, 520, 333), (100, 2048, 512), (303, 2050, 2048), (70, 40000, 64)])
+def test_float32_products_of_small_numbers(hip, M, N, K):
+    """Operands whose last bits lie below what bfloat16 holds, rows and columns of them among others, keep all their bits: a row's or column's
+    sums are then those of floats, at most K / 4 + 24 roundings, and others' as ever (tested above).  Results below 2^-126 are known to
+    a rounding of their own unit a term."""
+    for sx, sw, bits in ((-112, 0, 8), (-120, 0, 24), (-126, 30, 24), (0, -115, 24), (-60, -60, 24), (-137, 8, 8), (0, -130, 8), (-70, -70, 24)):
+        x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+        if bits == 8:
+            w = w.bfloat16().float()
+        x[::2] *= 2.0 ** sx
+        w[1::2] *= 2.0 ** sw
+        want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+        assert bool(((hip.linear(x, w).double() - want).abs() <= (24 + K / 4) * 2.0 ** -24 * size + K * 2.0 ** -149).all()), (sx, sw, bits)
+    # two operands whose only large product is of a small number
+    x, w = torch.zeros(M, K, device=DEV), torch.zeros(N, K, device=DEV)
+    x[:, 0], x[:, 1], w[:, 0], w[:, 1] = 1.0, rnd(M, seed=3) * 2.0 ** -120, rnd(N, seed=4) * 2.0 ** -120, 1.0
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    assert bool(((hip.linear(x, w).double() - want).abs() <= 4 * 2.0 ** -24 * size).all())
+
+
 def test_float32_product_has_no_reduced_precision(hip):
     """An operand bit below bfloat16 (8 bits) and tf32 (10 bits) resolution must reach the product."""
     K = 8
