@@ -2,18 +2,18 @@
 //
 // A float of 24 bits is the sum of three bfloat16 numbers, exactly: x0 = x rounded, x1 = (x - x0) rounded, x2 = x - x0 - x1.
 // (A number under 2^-110 may have a rest below 2^-133, which no bfloat16 number holds: its results are made as those that are not finite,
-// below.)  A product of two parts is exact in float, and of the nine
-// products of parts the six above 2^-24 of the whole are summed: x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0.  The matrix cores
-// multiply bfloat16 sixteen times as fast as float, so six products are 2.7 times as fast, and weights that are
-// bfloat16 numbers kept in 32 bits (a checkpoint's) have parts w1 = w2 = 0 and need three.
+// below.)  A product of two parts is exact in float, and all but x2 w2, under 2^-32 of the whole, are summed.  The matrix cores multiply
+// bfloat16 sixteen times as fast as float, so eight products are twice as fast, and weights that are bfloat16 numbers kept in 32
+// bits (a checkpoint's) have parts w1 = w2 = 0 and need three.
 //
 // The order of sums, the same for every shape, whatever M is, so that a row's result does not depend on the other rows of a
-// batch or on which kernel below runs:  a chunk of 32 k is summed from zero, its small products first (v_mfma_f32_16x16x32_bf16),
-// and the chunks' sums are added in order.  Where N is small, K is cut into slices that N and K alone decide
-// (slices_of), and the slices' sums are added in order.  Short chains and small terms first: the error against 64 bits is below
-// that of v_mfma_f32_16x16x4_f32 in four chains, which this replaces (2-norm, normal operands of 24 bits, k of 64, 512, 2,048, 8,192
-// and 14,336: 8.4e-8, 2.0e-7, 4.1e-7, 8.1e-7, 1.1e-6 -> 5e-8, 8e-8, 1.0e-7, 1.6e-7, 2.1e-7).  Leaving out the products of w1 and w2 where all
-// of them are zero changes no bit: they add zero.
+// batch or on which kernel below runs:  the products x0 w0 of a chunk of 32 k are summed from zero (v_mfma_f32_16x16x32_bf16), and the chunks'
+// sums added in order as floats; the small products have a sum of their own, on the matrix cores, which is added at the end.
+// Where N is small, K is cut into slices that N and K alone decide (slices_of), and the slices' sums are added in order.  Leaving
+// out the products of w1 and w2 where all of them are zero changes no bit: they add zero.  A result of one product is rounded as a float's
+// (5.97e-8 at most; the matrix cores alone, which cut: 1.3e-7), of many it is nearer to 64 bits than with v_mfma_f32_16x16x4_f32 in
+// four chains, which this replaces (2-norm, normal operands of 24 bits, k of 1, 2, 8, 64, 512, 2,048, 8,192: 2.54e-8, 3.1e-8, 5.3e-8, 8.3e-8,
+// 2.07e-7, 4.07e-7, 8.1e-7 -> 2.54e-8, 2.6e-8, 2.8e-8, 4.7e-8, 7.3e-8, 8.8e-8, 1.27e-7).
 //
 // Infinities and NaN, and finite numbers that round to an infinite part: some product of parts is then not finite, and neither is
 // the result.  A result that is not finite is made again from the floats as they are, on the float matrix cores (float_sums), 16 x 16
@@ -22,12 +22,13 @@
 //
 // * Few rows: a workgroup's waves stream W past the step's rows.  Bound by reading W, or by what the workgroups fetch from L2.
 // * More rows: X is split into its parts ahead, once, in the order in which the matrix cores read it; tiles of Y, X's parts and W as it
-//   is staged through LDS by loads that pass no registers, W split where it is read.  Neither loads alone (217 of 337 us at 303 rows,
-//   65,536 columns and k of 2,048) nor products and LDS reads alone (195 to 215) take the time: what is left is what the two do not share.
-// us, v_mfma_f32_16x16x4_f32 -> now, weights of 8 bits and of 24:  303 rows x 128,256 x 2,048 1,461 -> 640 and 1,040, x 16,384 x 2,048 206 -> 107
-// and 163, x 2,048 x 8,192 146 -> 68 and 96, x 3,072 x 2,048 42 -> 35 and 44;  one row x 2,048 x 2,048 9.2 -> 6.0 and 7.3, x 2,048 x 8,192 26.6 -> 19.5
-// and 22.5, x 28,672 x 4,096 105 -> 95 and 102;  64 rows x 2,048 x 2,048 11.7 -> 8.0 and 9.6.  Slower: weights of 24 bits at 17 to 32 rows
-// of 16,384 x 2,048 (34 -> 37), rows that begin anywhere at 200 to 600 rows of 1,000 x 333 (10.4 -> 13.6).
+//   is staged through LDS by loads that pass no registers, W split where it is read.  Two sums a result
+//   are what its registers hold: 128 x 256 outputs, which one sum allowed (303 x 128,256 x 2,048 664 us), would spill.
+// us, v_mfma_f32_16x16x4_f32 -> now, weights of 8 bits and of 24:  303 rows x 128,256 x 2,048 1,464 -> 710 and 1,352, x 16,384 x 2,048 204 -> 110
+// and 191, x 2,048 x 8,192 135 -> 70 and 102, x 3,072 x 2,048 42 -> 37 and 50;  one row x 2,048 x 2,048 8.7 -> 5.9 and 7.4, x 2,048 x 8,192 23.6 -> 14.4
+// and 19.2, x 14,336 x 4,096 51 -> 40 and 42;  64 rows x 2,048 x 2,048 11.9 -> 9 and 11.  Slower: 200 to 1,024 rows of 1,000 x 1,000 (512: 16.6 -> 19.5
+// and 20.6), and with weights of 24 bits 17 to 64 rows of 14,336 to 16,384 columns (17 x 16,384 x 2,048 29.1 -> 30.6, 32 x 14,336 x 4,096 50.7 -> 57.9) and
+// 130 to 1,024 rows of 2,048 to 3,072 (512 x 2,048 x 2,048 42.9 -> 54.5, 303 x 3,072 x 2,048 42.7 -> 49.7).
 #include "lds_load.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -88,23 +89,27 @@ __device__ __forceinline__ f32x4 product(u32x4 w, u32x4 x, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), c, 0, 0, 0);
 }
 
-// The sum of a chunk's products of a block of 16 rows of X with TN blocks of 16 rows of W.  The blocks alternate: a product is done
-// when the next one that adds to it begins.
+// A chunk's products of a block of 16 rows of X with TN blocks of 16 rows of W, added to their sums.  The matrix cores cut off where floats
+// round: the large products, exact where one is alone, are added as floats, and the small ones, 2^-8 of them, stay on the matrix cores, in a
+// sum of their own.  The blocks alternate: a product is done when the next one that adds to it begins.
+// more: W has more parts than the first.  One body for both (as two branches the sums of each had registers of their own).
 template <int TN>
-__device__ __forceinline__ void chunk_one_part(const u32x4 (&w0)[TN], const u32x4 (&x)[PARTS], f32x4 (&t)[TN]) {
+__device__ __forceinline__ void add_chunk(const u32x4 (&w)[TN][PARTS], const u32x4 (&x)[PARTS], bool more, f32x4 (&total)[TN], f32x4 (&small)[TN]) {
+    constexpr int MORE = 5, ORDER[MORE][2] = {{2, 1}, {1, 2}, {2, 0}, {1, 1}, {1, 0}};      // parts of W and X
+    f32x4 large[TN];
 #pragma unroll
-    for (int p = PARTS - 1; p >= 0; --p)
+    for (int j = 0; j < TN; ++j) large[j] = product(w[j][0], x[0], f32x4{0.f, 0.f, 0.f, 0.f});
+    if (more)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) t[j] = product(w0[j], x[p], p == PARTS - 1 ? f32x4{0.f, 0.f, 0.f, 0.f} : t[j]);
-}
-
-template <int TN>
-__device__ __forceinline__ void chunk_of_parts(const u32x4 (&w)[TN][PARTS], const u32x4 (&x)[PARTS], f32x4 (&t)[TN]) {
-    constexpr int ORDER[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};      // parts of W and X, small products first
+        for (int o = 0; o < MORE; ++o)
 #pragma unroll
-    for (int o = 0; o < 6; ++o)
+            for (int j = 0; j < TN; ++j) small[j] = product(w[j][ORDER[o][0]], x[ORDER[o][1]], small[j]);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) t[j] = product(w[j][ORDER[o][0]], x[ORDER[o][1]], o == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : t[j]);
+    for (int p = PARTS - 1; p > 0; --p)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) small[j] = product(w[j][0], x[p], small[j]);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) total[j] += large[j];
 }
 
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) <= 3.402823466e38f; }
@@ -183,11 +188,11 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
     const int begin = slice_begin(chunks, slice, SLICES);
     const int steps = n0 < N ? slice_begin(chunks, slice + 1, SLICES) - begin : 0;      // chunks of this wave
 
-    f32x4 total[MB][NB];
+    f32x4 total[MB][NB], small[MB][NB];
 #pragma unroll
     for (int b = 0; b < MB; ++b)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) total[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NB; ++j) total[b][j] = small[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     uint32_t rest_x[MB], rest_w[NB];      // of the rows r (a branch at every split: 17 rows x 2,048 x 8,192 22.8 us, 22.0 so)
 #pragma unroll
     for (int b = 0; b < MB; ++b) rest_x[b] = 0;
@@ -212,46 +217,21 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
 #pragma unroll
             for (int j = 0; j < NB; ++j) bits |= or_of(wa[u][j], wb[u][j]);
         }
-        if (!__any((bits & 0xffffu) != 0)) {
-            f32x4 t[U][MB][NB];
+        const bool more = __any((bits & 0xffffu) != 0);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                u32x4 w0[NB];
+        for (int u = 0; u < U; ++u) {
+            u32x4 w[NB][PARTS];
 #pragma unroll
-                for (int j = 0; j < NB; ++j) w0[j] = upper_halves(wa[u][j], wb[u][j]);
-#pragma unroll
-                for (int b = 0; b < MB; ++b) {
-                    u32x4 x[PARTS];
-                    rest_x[b] |= split8(xa[u][b], xb[u][b], x);
-                    chunk_one_part(w0, x, t[u][b]);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int b = 0; b < MB; ++b)
-#pragma unroll
-                    for (int j = 0; j < NB; ++j) total[b][j] += t[u][b][j];
-        } else {
-            f32x4 t[U][MB][NB];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                u32x4 w[NB][PARTS];
+            for (int j = 0; j < NB; ++j) w[j][0] = upper_halves(wa[u][j], wb[u][j]);
+            if (more)
 #pragma unroll
                 for (int j = 0; j < NB; ++j) rest_w[j] |= split8(wa[u][j], wb[u][j], w[j]);
 #pragma unroll
-                for (int b = 0; b < MB; ++b) {
-                    u32x4 x[PARTS];
-                    rest_x[b] |= split8(xa[u][b], xb[u][b], x);
-                    chunk_of_parts(w, x, t[u][b]);
-                }
+            for (int b = 0; b < MB; ++b) {
+                u32x4 x[PARTS];
+                rest_x[b] |= split8(xa[u][b], xb[u][b], x);
+                add_chunk(w, x, more, total[b], small[b]);
             }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int b = 0; b < MB; ++b)
-#pragma unroll
-                    for (int j = 0; j < NB; ++j) total[b][j] += t[u][b][j];
         }
     };
     u32x4 wa[U][NB], wb[U][NB], xa[U][MB], xb[U][MB];
@@ -322,6 +302,10 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
             multiply(s, wa, wb, xa, xb);
         }
     }
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) total[b][j] += small[b][j];
     uint32_t rest = 0;
 #pragma unroll
     for (int b = 0; b < MB; ++b) rest |= rest_x[b];
@@ -406,19 +390,19 @@ static void launch_few_rows(const float* X, const float* W, float* Y, int M, int
         hipLaunchKernelGGL((gemm_f32_few_rows_kernel<1, 8, MB, NB, XI, U, SLOTS, DIRECT>), columns(8), dim3(512), 0, stream, X, W, Y, M, N, K);
 }
 
-// The shape of the few-row kernel: blocks of X's and W's rows, and at what rate its workgroups fetch (MB a us).  More blocks share what is read
-// and split of the other operand, where enough workgroups are left.
+// The shape of the few-row kernel: blocks of X's and W's rows, and what it costs: a launch (us), and at what rate its workgroups fetch
+// (MB a us).  More blocks share what is read and split of the other operand, where enough workgroups are left.
 struct FewRows {
     int mb, nb;
-    double rate;
+    double launch, rate;
 };
 static FewRows few_rows_shape(int M, int N, int K) {
-    if (M <= 8 && N > 32 * 1024 && K % CHUNK == 0) return {1, 4, 12};      // rows of whole cache lines
-    if (M <= 16 || K <= 4 * CHUNK) return {1, 1, 16};
-    if (N < 8 * 1024) return {2, 1, 16};
-    if (M > 32 && N > 12 * 1024) return {4, 2, 10};
-    if (N <= 32 * 1024) return {2, 2, 12};
-    return K % CHUNK == 0 ? FewRows{2, 4, 12} : FewRows{2, 2, 7};
+    if (M <= 8 && N > 32 * 1024 && K % CHUNK == 0) return {1, 4, 2.5, 12};      // rows of whole cache lines
+    if (M <= 16 || K <= 4 * CHUNK) return {1, 1, 4, 16};
+    if (N < 8 * 1024) return {2, 1, 4, 13.6};
+    if (M > 32 && N > 12 * 1024) return {4, 2, 2.5, 10};
+    if (N <= 32 * 1024) return {2, 2, 2.5, 10.8};
+    return K % CHUNK == 0 ? FewRows{2, 4, 2.5, 9} : FewRows{2, 2, 2.5, 7};
 }
 
 static void few_rows(const float* X, const float* W, float* Y, int M, int N, int K, bool direct, hipStream_t stream) {
@@ -540,12 +524,12 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
 #pragma unroll
         for (int l = 0; l < LW; ++l) load_to_lds(w_from[l] + min((begin + s) * CHUNK + piece[l], Kt - 4), to + l * LL_TILE);
     };
-    f32x4 total[TM][TN], sum[SLICED ? TM : 1][SLICED ? TN : 1];      // of the slice, of the slices before it
+    f32x4 total[TM][TN], small[TM][TN], sum[SLICED ? TM : 1][SLICED ? TN : 1];      // of the slice, of the slices before it
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            total[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
             if constexpr (SLICED) sum[i][j] = total[i][j];
         }
     // total[i][j]: row 16 i + r of the wave's tile, columns 16 j + 4 g .. + 3
@@ -553,15 +537,17 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
     float* const to = apart ? slices + (size_t)slice * M * Ns : Y;
     bool odd = false;
     auto store = [&](bool more) {      // more: Y has the slices before
+        int first = m_first;
+        asm volatile("" : "+v"(first));      // addresses made here, not in front of the loop and kept through it
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            const int m = m_first + i * 16;
+            const int m = first + i * 16;
             if (m >= M) continue;
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int n = n_first + j * 16;
                 float* at = to + (size_t)m * stride + n;
-                f32x4 v = total[i][j];
+                f32x4 v = total[i][j] + small[i][j];
                 if constexpr (SLICED) v = sum[i][j] + v;
                 if (four || apart) {
                     if (n >= N) continue;
@@ -593,56 +579,55 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
         if (s + D < steps) request(s + D, slot == 0 ? D : slot - 1);
         const char* stage = lds + slot * STAGE;
         slot = slot == D ? 0 : slot + 1;
-        u32x4 a[TN], b[TN];
-        uint32_t bits = 0;
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            a[j] = *(const u32x4*)(stage + w_at + j * 2 * LL_TILE + place[0]);
-            b[j] = *(const u32x4*)(stage + w_at + j * 2 * LL_TILE + place[1]);
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) bits |= or_of(a[j], b[j]);
+        auto read_w = [&](int j, u32x4& a, u32x4& b) {
+            const char* at = stage + w_at + j * 2 * LL_TILE;
+            a = *(const u32x4*)(at + place[0]), b = *(const u32x4*)(at + place[1]);
+        };
         auto read_x = [&](int i, u32x4 (&x)[PARTS]) {
 #pragma unroll
             for (int e = 0; e < PARTS; ++e) x[e] = *(const u32x4*)(stage + x_at + (i * PARTS + e) * LL_TILE);
         };
-        if (!__any((bits & 0xffffu) != 0)) {
-            u32x4 w0[TN];
+        u32x4 w[TN][PARTS];
+        uint32_t bits = 0;
 #pragma unroll
-            for (int j = 0; j < TN; ++j) w0[j] = upper_halves(a[j], b[j]);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                u32x4 x[PARTS];
-                f32x4 t[TN];
-                read_x(i, x);
-                chunk_one_part(w0, x, t);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) total[i][j] += t[j];
-            }
-        } else {
-            u32x4 w[TN][PARTS];
+        for (int j = 0; j < TN; ++j) {
+            u32x4 a, b;
+            read_w(j, a, b);
+            bits |= or_of(a, b);
+            w[j][0] = upper_halves(a, b);
+        }
+        const bool more_parts = __any((bits & 0xffffu) != 0);
+        if (more_parts) {
             uint32_t rest = 0;
+            asm volatile("" ::: "memory");      // W is read again, here and below: kept, it would take the registers of the sums
 #pragma unroll
-            for (int j = 0; j < TN; ++j) rest |= split8(a[j], b[j], w[j]);
-            if (any_rest(rest))
-#pragma unroll
-                for (int j = 0; j < TN; ++j) mark_rests(a[j], b[j], w[j][PARTS - 1]);
-#pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                u32x4 x[PARTS];
-                f32x4 t[TN];
-                read_x(i, x);
-                chunk_of_parts(w, x, t);
-#pragma unroll
-                for (int j = 0; j < TN; ++j) total[i][j] += t[j];
+            for (int j = 0; j < TN; ++j) {
+                u32x4 a, b;
+                read_w(j, a, b);
+                rest |= split8(a, b, w[j]);
             }
+            if (any_rest(rest)) {
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    u32x4 a, b;
+                    read_w(j, a, b);
+                    mark_rests(a, b, w[j][PARTS - 1]);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            u32x4 x[PARTS];
+            read_x(i, x);
+            add_chunk(w, x, more_parts, total[i], small[i]);
         }
         if (s + 1 == end && s + 1 < steps) {
             if constexpr (SLICED) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) sum[i][j] += total[i][j];
+                    for (int j = 0; j < TN; ++j) sum[i][j] += total[i][j] + small[i][j];
             } else {
                 store(more);
                 more = true;
@@ -650,7 +635,7 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int j = 0; j < TN; ++j) total[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
             while (end == s + 1) end = slice_begin(chunks, ++ended, n_slices);
         }
     }
@@ -706,19 +691,24 @@ __global__ __launch_bounds__(256) void sum_slices_f32_kernel(const float* __rest
 // which kernel
 // ---------------------------------------------------------------------------------------------------------
 
-// The shapes, how many workgroups of each a compute unit holds at a time, and what a product costs in microseconds, by least squares
-// over 1,100 timings (512 to 128,256 columns, k of 2,048 to 14,336, 17 to 1,024 rows; a shape's median error 3 %, the choice 2.7 % above
-// the best of eleven shapes on average): a launch, a round of workgroups over the device, a chunk of a round, slices apart, a MB of
-// their sums written and read, a MB of W.
+// The shapes, how many workgroups of each a compute unit holds at a time, and what a product costs in microseconds, with all of K a
+// workgroup or its slices apart: a launch, a round of workgroups over the device, a chunk of a round, what each workgroup on a unit
+// adds to that, a MB of the slices' sums written and read (through Y, for tiles of 256 columns).  By least squares over the geometric mean
+// of weights of 8 and 24 bits, 2,900 products of 256 to 128,256 columns, k of 256 to 8,192, 17 to 1,024 rows:  median error 2 to 4 %; the choice
+// is 2.2 % above the best of seven shapes on average, 11 % in one of twenty.
+struct F32Cost {
+    double launch, round, step, more, sums;
+};
 struct F32Shape {
     int bm, bn, at_a_time;
-    double launch, round, step, apart, sums, weights;
+    F32Cost whole, apart;
 };
-static const F32Shape F32_SHAPES[] = {{128, 256, 1, 3.7, 6.8, 1.33, 1.5, 0.145, 0.030},
-                                      {96, 256, 1, 5.7, 2.6, 1.15, 2.4, 0.170, 0.015},
-                                      {64, 128, 2, 23.4, -9.0, 0.894, -8.7, 0.359, 0.087},
-                                      {64, 128, 2, 6.9, -1.4, 1.18, 2.4, 0.287, 0.026},
-                                      {32, 64, 3, 14.3, -3.8, 0.624, -2.8, 0.384, 0.066}};
+constexpr F32Cost NEVER = {1e30, 0, 0, 0, 0};
+static const F32Shape F32_SHAPES[] = {{96, 256, 1, {22.6, 13.1, 1.68, 0, 0.109}, {13.3, -2.4, 1.78, 0, 0.287}},
+                                      {64, 128, 2, {5.0, 3.2, 0.657, 0.372, 0}, {13.6, -3.9, 0.742, 0.319, 0.305}},
+                                      {64, 128, 1, {4.4, 3.2, 0.859, 0, 0}, {11.0, -1.7, 0.891, 0, 0.346}},
+                                      {32, 64, 3, {6.8, -0.5, 0.428, 0.127, 0}, NEVER},
+                                      {128, 128, 1, {-0.6, 10.1, 1.241, 0, 0}, {12.6, -2.8, 1.282, 0, 0.338}}};
 constexpr int N_F32_SHAPES = sizeof(F32_SHAPES) / sizeof(F32_SHAPES[0]);
 
 struct F32Plan {
@@ -738,20 +728,19 @@ static F32Plan f32_plan(int M, int N, int K, bool direct) {
     const FewRows few = few_rows_shape(M, N, K);
     const int rows_w = few.nb * 16, rows_x = few.mb * 16;
     const double fetched = (double)((M + rows_x - 1) / rows_x) * ((N + rows_w - 1) / rows_w) * (rows_w + rows_x) * K * 4e-6;
-    // the tiles take half as long again for weights of 24 bits, the few-row kernel a tenth: a line between the two
-    double least = (2.5 + fmax(fetched / few.rate, (double)N * K * 4e-6 / 5.4)) * (direct ? 1 : 3) / 1.15;
+    double least = (few.launch + fmax(fetched / few.rate, (double)N * K * 4e-6 / 5.4)) * (direct ? 1 : 3);
     for (int i = 0; i < N_F32_SHAPES; ++i) {
-        const F32Shape t = F32_SHAPES[i];
+        const F32Shape& t = F32_SHAPES[i];
         const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int apart = 0; apart <= (n_slices > 1); ++apart) {
+            const F32Cost& c = apart ? t.apart : t.whole;
             const long long workgroups = tiles * (apart ? n_slices : 1), room = (long long)cus * t.at_a_time;
             if (workgroups > 1 << 30 || (apart && (long long)n_slices * M * N > 1LL << 27)) continue;
             const int steps = apart ? (chunks + n_slices - 1) / n_slices : chunks;
-            // workgroups that share a unit: a last round that fills a part of them is as much shorter
-            const double rounds = (double)(workgroups / room) + (double)((workgroups % room + cus - 1) / cus) / t.at_a_time;
-            double us = (direct ? 0 : 4) + t.launch + t.weights * N * K * 4e-6 + rounds * (t.round + t.step * steps);
-            if (apart) us += t.apart + t.sums * n_slices * M * N * 8e-6;
-            if (!apart && t.bn == 256) us += t.sums * (n_slices - 1) * M * N * 8e-6;      // in Y
+            const double full = (double)(workgroups / room), last = (double)((workgroups % room + cus - 1) / cus);      // of `last` workgroups a unit
+            double us = (direct ? 0 : 4) + c.launch + (full + (last > 0)) * (c.round + c.step * steps) + (full * t.at_a_time + last) * c.more * steps;
+            if (apart) us += c.sums * n_slices * M * N * 8e-6;
+            else us += c.sums * (n_slices - 1) * M * N * 8e-6;
             if (us >= least) continue;
             least = us;
             best.shape = i, best.apart = apart;
@@ -827,11 +816,11 @@ SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* work
     int status = SIA_BAD_ARGUMENT;
 #define SHAPE(I, ...) \
     if (plan.shape == I) status = launch_f32_tiles<__VA_ARGS__>(X, W, Wt, Y, parts, slices, M, N, K, Kt, apart, four, stream)
-    SHAPE(0, 128, 256, 2, 4, 1);
-    SHAPE(1, 96, 256, 2, 4, 2);
-    SHAPE(2, 64, 128, 2, 2, 1);
-    SHAPE(3, 64, 128, 2, 4, 2);
-    SHAPE(4, 32, 64, 2, 2, 2);
+    SHAPE(0, 96, 256, 2, 4, 2);
+    SHAPE(1, 64, 128, 2, 2, 1);
+    SHAPE(2, 64, 128, 2, 4, 2);
+    SHAPE(3, 32, 64, 2, 2, 2);
+    SHAPE(4, 128, 128, 2, 4, 2);
 #undef SHAPE
     if (status == 0 && apart)
         hipLaunchKernelGGL(sum_slices_f32_kernel, dim3((M + 15) / 16, (N + 63) / 64), dim3(256), 0, stream, slices, X, W, Y, M, N, K, Ns,

@@ -634,6 +634,19 @@ def test_float32_products_of_small_numbers(hip, M, N, K):
     assert bool(((hip.linear(x, w).double() - want).abs() <= 4 * 2.0 ** -24 * size).all())
 
 
+@pytest.mark.parametrize("bits", [8, 24])
+@pytest.mark.parametrize("M, N, K", [(8, 2050, 1), (303, 2048, 2048), (100, 300, 70), (40, 40000, 64), (300, 16388, 512)])
+def test_float32_results_of_one_product_are_rounded_once(hip, M, N, K, bits):
+    """One product a result, among zeros: the rounding to float (2^-24), and what the products of the smallest parts leave (2^-31)."""
+    x, w = torch.zeros(M, K, device=DEV), rnd(N, K, seed=2)
+    if bits == 8:
+        w = w.bfloat16().float()
+    x[:, K // 3] = rnd(M, seed=1)
+    want = x[:, K // 3:K // 3 + 1].double() @ w[:, K // 3:K // 3 + 1].double().T
+    error = ((hip.linear(x, w).double() - want).abs() / want.abs()).max()
+    assert float(error) <= 2.0 ** -24 + 2.0 ** -31, float(error) * 2.0 ** 24
+
+
 def test_float32_product_has_no_reduced_precision(hip):
     """An operand bit below bfloat16 (8 bits) and tf32 (10 bits) resolution must reach the product."""
     K = 8
