@@ -155,6 +155,22 @@ __device__ __forceinline__ f32x4 float_sums(const float* __restrict__ x, const f
     return (sum[0] + sum[1]) + (sum[2] + sum[3]);
 }
 
+// A KiB of 8 rows of a chunk into LDS by loads of 16 bytes a lane (WIDE: rows at multiples of 16 bytes, K a multiple of 4), or by four loads of a float
+// a lane, of two rows each, for rows that begin anywhere; the places are the same (`turn`).  (Loaded into registers float by float, or copied to
+// rows of 16 bytes first, us:  32 rows x 2,048 x 2,049 32.6 -> 12.0, 17 x 16,384 x 2,049 78 -> 37, 303 x 40,000 x 2,049 2,873 -> 294, 303 x 1,000 x 333 18.4 -> 10.6;
+// slower 600 x 2,048 x 2,049 with weights of 24 bits, 70 -> 90.)  Lane's row of load q, and its k of a chunk:
+template <bool WIDE> __device__ __forceinline__ int row_of_load(int q, int lane) { return WIDE ? lane / 8 : 2 * q + lane / 32; }
+template <bool WIDE> __device__ __forceinline__ int k_of_load(int row, int lane) {      // row: of 16
+    return WIDE ? ((lane & 7) ^ turn(row)) * 4 : (((lane % 32 / 4) ^ turn(row)) * 4 + lane % 4);
+}
+template <bool WIDE> __device__ __forceinline__ void load_chunk(const float* row, int k, int K, char* to, int q) {      // behind the last k: the last
+    if constexpr (WIDE)
+        load_to_lds(row + min(k, K - 4), to);
+    else
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(row + min(k, K - 1)),
+                                         (__attribute__((address_space(3))) void*)(to + q * (LL_TILE / 4)), 4, 0, 0);
+}
+
 // Slices of K, in chunks: from N and K alone.  Few rows of W beside a long K are too little for the chip without; an output head
 // is enough, and its tiles then need no second sum.
 __host__ __device__ static inline int slices_of(int N, int K) { return N > 32 * 1024 || K <= 4 * CHUNK ? 1 : N > 12 * 1024 ? 2 : 8; }
@@ -168,15 +184,15 @@ __device__ __forceinline__ int slice_begin(int chunks, int slice, int slices) { 
 // A wave's step is U chunks, whose sums do not depend on one another.  W's and X's rows come to LDS directly as they are, 128 bytes of eight
 // rows an instruction, into a ring of SLOTS steps that the wave has for itself, and are split where they are read.  (Loaded into registers,
 // an instruction touches 16 lines in pieces of 16 bytes: see gemm_skinny.hip.)  XI: tiles of 8 rows of X, 2 MB or 1.
-// DIRECT: rows begin at multiples of 16 bytes and K is a multiple of 4.  Else operands are read float by float, into registers.
-template <int SLICES, int WAVES, int MB, int NB, int XI, int U, int SLOTS, bool DIRECT>
+// WIDE: see load_chunk.
+template <int SLICES, int WAVES, int MB, int NB, int XI, int U, int SLOTS, bool WIDE>
 __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(const float* __restrict__ X, const float* __restrict__ W,
                                                                             float* __restrict__ Y, int M, int N, int K) {
     static_assert(WAVES % SLICES == 0, "a wave a slice");
     constexpr int GROUPS = WAVES / SLICES;
     static_assert(XI == 2 * MB || (MB == 1 && XI == 1), "tiles of 8 rows");
-    constexpr int CHUNK_LOADS = 2 * NB + XI, LOADS = U * CHUNK_LOADS;
-    constexpr int RING = DIRECT ? WAVES * SLOTS * LOADS * LL_TILE : 0, SUMS = SLICES > 1 ? WAVES * MB * NB * 256 * 4 : 0;
+    constexpr int TILES = 2 * NB + XI, EACH = WIDE ? 1 : 4, LOADS = U * TILES * EACH;      // KiB of a chunk, loads of each
+    constexpr int RING = WAVES * SLOTS * U * TILES * LL_TILE, SUMS = SLICES > 1 ? WAVES * MB * NB * 256 * 4 : 0;
     constexpr int LDS = RING > SUMS ? RING : SUMS > 0 ? SUMS : 16;
     static_assert(LDS <= LL_LDS, "a workgroup's LDS");
     __shared__ __attribute__((aligned(1024))) char lds[LDS];
@@ -211,8 +227,11 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
             if (s + u >= steps || (begin + s + u + 1) * CHUNK > K)
 #pragma unroll
                 for (int b = 0; b < MB; ++b) {      // behind the last k too (W has there what was read instead)
-                    if (s + u >= steps || k >= K) xa[u][b] = none;
-                    if (s + u >= steps || k + 4 >= K) xb[u][b] = none;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {      // (wide: K is a multiple of 4)
+                        if (s + u >= steps || k + (WIDE ? 0 : e) >= K) xa[u][b][e] = 0;
+                        if (s + u >= steps || k + 4 + (WIDE ? 0 : e) >= K) xb[u][b][e] = 0;
+                    }
                 }
 #pragma unroll
             for (int j = 0; j < NB; ++j) bits |= or_of(wa[u][j], wb[u][j]);
@@ -235,72 +254,54 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
         }
     };
     u32x4 wa[U][NB], wb[U][NB], xa[U][MB], xb[U][MB];
-    if constexpr (DIRECT) {
-        // rows that do not exist are read as the last one and not stored
-        const float* from[CHUNK_LOADS];
-        int piece[CHUNK_LOADS];
+    // rows that do not exist are read as the last one and not stored
+    const float* from[TILES * EACH];
+    int piece[TILES * EACH];
 #pragma unroll
-        for (int l = 0; l < CHUNK_LOADS; ++l) {
-            const int row = (l < 2 * NB ? l : l - 2 * NB) * 8 + lane / 8;
-            from[l] = l < 2 * NB ? W + (size_t)min(n0 + row, N - 1) * K : X + (size_t)min(m0 + row, M - 1) * K;
-            piece[l] = begin * CHUNK + ((lane & 7) ^ turn(row & 15)) * 4;
+    for (int l = 0; l < TILES; ++l)
+#pragma unroll
+        for (int q = 0; q < EACH; ++q) {
+            const int row = (l < 2 * NB ? l : l - 2 * NB) * 8 + row_of_load<WIDE>(q, lane);
+            from[l * EACH + q] = l < 2 * NB ? W + (size_t)min(n0 + row, N - 1) * K : X + (size_t)min(m0 + row, M - 1) * K;
+            piece[l * EACH + q] = begin * CHUNK + k_of_load<WIDE>(row & 15, lane);
         }
-        char* const ring = lds + wave * (SLOTS * LOADS * LL_TILE);
-        // steps of U chunks; the last one's chunks behind the end are loaded again, so that the waits count the same
-        auto request = [&](int s, int slot) {
+    char* const ring = lds + wave * (SLOTS * U * TILES * LL_TILE);
+    // steps of U chunks; the last one's chunks behind the end are loaded again, so that the waits count the same
+    auto request = [&](int s, int slot) {
 #pragma unroll
-            for (int u = 0; u < U; ++u)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int l = 0; l < CHUNK_LOADS; ++l)
-                    load_to_lds(from[l] + min(min(s + u, steps - 1) * CHUNK + piece[l], K - 4), ring + ((slot * U + u) * CHUNK_LOADS + l) * LL_TILE);
-        };
+            for (int l = 0; l < TILES; ++l)
 #pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-            if (s * U < steps) request(s * U, s);
-        const int at[2] = {r * 128 + ((2 * g) ^ turn(r)) * 16, r * 128 + ((2 * g + 1) ^ turn(r)) * 16};
-        const int xr = XI == 1 ? r & 7 : r;
-        const int x_at[2] = {xr * 128 + ((2 * g) ^ turn(xr)) * 16, xr * 128 + ((2 * g + 1) ^ turn(xr)) * 16};
-        int slot = 0;
-        for (int s = 0; s < steps; s += U) {
-            wait_step<LOADS, SLOTS - 1>((steps - 1) / U - s / U);
+                for (int q = 0; q < EACH; ++q)
+                    load_chunk<WIDE>(from[l * EACH + q], min(s + u, steps - 1) * CHUNK + piece[l * EACH + q], K,
+                                     ring + ((slot * U + u) * TILES + l) * LL_TILE, q);
+    };
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const char* in = ring + (slot * U + u) * CHUNK_LOADS * LL_TILE;
+    for (int s = 0; s < SLOTS; ++s)
+        if (s * U < steps) request(s * U, s);
+    const int at[2] = {r * 128 + ((2 * g) ^ turn(r)) * 16, r * 128 + ((2 * g + 1) ^ turn(r)) * 16};
+    const int xr = XI == 1 ? r & 7 : r;
+    const int x_at[2] = {xr * 128 + ((2 * g) ^ turn(xr)) * 16, xr * 128 + ((2 * g + 1) ^ turn(xr)) * 16};
+    int slot = 0;
+    for (int s = 0; s < steps; s += U) {
+        wait_step<LOADS, SLOTS - 1>((steps - 1) / U - s / U);
 #pragma unroll
-                for (int j = 0; j < NB; ++j)
-                    wa[u][j] = *(const u32x4*)(in + 2 * j * LL_TILE + at[0]), wb[u][j] = *(const u32x4*)(in + 2 * j * LL_TILE + at[1]);
+        for (int u = 0; u < U; ++u) {
+            const char* in = ring + (slot * U + u) * TILES * LL_TILE;
 #pragma unroll
-                for (int b = 0; b < MB; ++b) {
-                    const char* in_x = in + (2 * NB + 2 * b) * LL_TILE;
-                    xa[u][b] = *(const u32x4*)(in_x + x_at[0]), xb[u][b] = *(const u32x4*)(in_x + x_at[1]);
-                }
+            for (int j = 0; j < NB; ++j)
+                wa[u][j] = *(const u32x4*)(in + 2 * j * LL_TILE + at[0]), wb[u][j] = *(const u32x4*)(in + 2 * j * LL_TILE + at[1]);
+#pragma unroll
+            for (int b = 0; b < MB; ++b) {
+                const char* in_x = in + (2 * NB + 2 * b) * LL_TILE;
+                xa[u][b] = *(const u32x4*)(in_x + x_at[0]), xb[u][b] = *(const u32x4*)(in_x + x_at[1]);
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the slot has been read: it may be filled again
-            if (s + SLOTS * U < steps) request(s + SLOTS * U, slot);
-            slot = slot + 1 < SLOTS ? slot + 1 : 0;
-            multiply(s, wa, wb, xa, xb);
         }
-    } else {
-        const uint32_t *w_row[NB], *x_row[MB];
-#pragma unroll
-        for (int j = 0; j < NB; ++j) w_row[j] = (const uint32_t*)W + (size_t)min(n0 + j * 16 + r, N - 1) * K;
-#pragma unroll
-        for (int b = 0; b < MB; ++b) x_row[b] = (const uint32_t*)X + (size_t)min(m0 + b * 16 + r, M - 1) * K;
-        for (int s = 0; s < steps; s += U) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int k = (begin + min(s + u, steps - 1)) * CHUNK + 8 * g;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-#pragma unroll
-                    for (int j = 0; j < NB; ++j) wa[u][j][e] = w_row[j][min(k + e, K - 1)], wb[u][j][e] = w_row[j][min(k + 4 + e, K - 1)];
-#pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        xa[u][b][e] = k + e < K ? x_row[b][k + e] : 0, xb[u][b][e] = k + 4 + e < K ? x_row[b][k + 4 + e] : 0;
-                }
-            }
-            multiply(s, wa, wb, xa, xb);
-        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // the slot has been read: it may be filled again
+        if (s + SLOTS * U < steps) request(s + SLOTS * U, slot);
+        slot = slot + 1 < SLOTS ? slot + 1 : 0;
+        multiply(s, wa, wb, xa, xb);
     }
 #pragma unroll
     for (int b = 0; b < MB; ++b)
@@ -374,20 +375,20 @@ __global__ __launch_bounds__(WAVES* SIA_WAVE) void gemm_f32_few_rows_kernel(cons
 
 // Small rings, and more workgroups on a unit, are faster than deep ones (us for one row and weights of 8 bits, 8 waves, the best two of
 // each:  2,048 x 2,048 6.4 with one step of two chunks, 6.8 with three;  28,672 x 4,096 78 and 86).
-template <int MB, int NB, int XI, bool DIRECT>
+template <int MB, int NB, int XI, bool WIDE>
 static void launch_few_rows(const float* X, const float* W, float* Y, int M, int N, int K, hipStream_t stream) {
     const int slices = slices_of(N, K), y = (M + MB * 16 - 1) / (MB * 16);
     auto columns = [&](int groups) { return dim3((N + groups * NB * 16 - 1) / (groups * NB * 16), y); };
     constexpr int EACH = 2 * NB + XI, U = MB * NB == 1 ? 2 : 1;
     constexpr int SLOTS2 = EACH <= 3 ? 3 : EACH <= 8 ? 2 : 1, SLOTS = EACH <= 9 && MB * NB <= 4 ? 2 : 1;
     if (slices == 8)
-        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<8, 8, MB, NB, XI, U, 1, DIRECT>), columns(1), dim3(512), 0, stream, X, W, Y, M, N, K);
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<8, 8, MB, NB, XI, U, 1, WIDE>), columns(1), dim3(512), 0, stream, X, W, Y, M, N, K);
     else if (slices == 2)
-        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<2, 4, MB, NB, XI, U, SLOTS2, DIRECT>), columns(2), dim3(256), 0, stream, X, W, Y, M, N, K);
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<2, 4, MB, NB, XI, U, SLOTS2, WIDE>), columns(2), dim3(256), 0, stream, X, W, Y, M, N, K);
     else if (N <= 32 * 1024)
-        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<1, 4, MB, NB, XI, U, 1, DIRECT>), columns(4), dim3(256), 0, stream, X, W, Y, M, N, K);
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<1, 4, MB, NB, XI, U, 1, WIDE>), columns(4), dim3(256), 0, stream, X, W, Y, M, N, K);
     else
-        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<1, 8, MB, NB, XI, U, SLOTS, DIRECT>), columns(8), dim3(512), 0, stream, X, W, Y, M, N, K);
+        hipLaunchKernelGGL((gemm_f32_few_rows_kernel<1, 8, MB, NB, XI, U, SLOTS, WIDE>), columns(8), dim3(512), 0, stream, X, W, Y, M, N, K);
 }
 
 // The shape of the few-row kernel: blocks of X's and W's rows, and what it costs: a launch (us), and at what rate its workgroups fetch
@@ -405,12 +406,17 @@ static FewRows few_rows_shape(int M, int N, int K) {
     return K % CHUNK == 0 ? FewRows{2, 4, 2.5, 9} : FewRows{2, 2, 2.5, 7};
 }
 
-static void few_rows(const float* X, const float* W, float* Y, int M, int N, int K, bool direct, hipStream_t stream) {
+// wide: both operands' rows lie so.
+static void few_rows(const float* X, const float* W, float* Y, int M, int N, int K, bool wide, hipStream_t stream) {
     const FewRows few = few_rows_shape(M, N, K);
-    if (!direct && M <= 16)
+    if (!wide && M <= 8)
+        launch_few_rows<1, 1, 1, false>(X, W, Y, M, N, K, stream);
+    else if (!wide && M <= 16)
         launch_few_rows<1, 1, 2, false>(X, W, Y, M, N, K, stream);
-    else if (!direct)
+    else if (!wide && few.nb == 1)
         launch_few_rows<2, 1, 4, false>(X, W, Y, M, N, K, stream);
+    else if (!wide)
+        launch_few_rows<2, 2, 4, false>(X, W, Y, M, N, K, stream);
     else if (few.mb == 4)
         launch_few_rows<4, 2, 8, true>(X, W, Y, M, N, K, stream);
     else if (few.mb == 2 && few.nb == 4)
@@ -455,32 +461,20 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
     for (int e = 0; e < PARTS; ++e) at[e * SIA_WAVE] = p[e];
 }
 
-// Rows of K floats that begin anywhere, copied to rows of `stride` (K up to a multiple of 4, zeros behind).  Four elements a thread.
-__global__ __launch_bounds__(256) void align_rows_kernel(const float* __restrict__ W, f32x4* __restrict__ out, int K, int stride, size_t pieces) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= pieces) return;
-    const size_t row = i / (stride / 4);
-    const int k = (int)(i % (stride / 4)) * 4;
-    f32x4 v;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? W[row * K + k + e] : 0.f;
-    out[i] = v;
-}
-
 // A tile of BM rows of W, taken by WM x WN waves.  A ring of D + 1 chunks of both in LDS, asked for D ahead; one
 // barrier a chunk: what is read next has come, what was read last may be overwritten.
 // apart: a workgroup has one slice of K, whose sums go to `slices` ([slice][M][Ns]) for sum_slices_f32_kernel.  Else it has all of K, and
 // adds up the slices, SLICED: in registers, else in Y.
-// Wt: W's rows as they are read, from multiples of 16 bytes, Kt floats apart (a multiple of 4).
-template <int BM, int BN, int WM, int WN, int D, bool SLICED>
+// WIDE: how W is read, see load_chunk.
+template <int BM, int BN, int WM, int WN, int D, bool SLICED, bool WIDE>
 __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
-    const u32x4* __restrict__ parts, const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ Wt,
-    float* __restrict__ Y, float* __restrict__ slices, int M, int N, int K, int Kt, int Ns, int n_slices, bool apart, bool four,
+    const u32x4* __restrict__ parts, const float* __restrict__ X, const float* __restrict__ W,
+    float* __restrict__ Y, float* __restrict__ slices, int M, int N, int K, int Ns, int n_slices, bool apart, bool four,
     int tiles_m, int n_tiles, int per_die) {
     constexpr int WAVES = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
     constexpr int XT = BM / 16 * PARTS, WT = BN / 8;                 // KiB of a chunk
     constexpr int LX = (XT + WAVES - 1) / WAVES, LW = WT / WAVES;    // loads of a wave
-    constexpr int STAGE = (XT + WT) * LL_TILE, LOADS = LX + LW;
+    constexpr int EACH = WIDE ? 1 : 4, STAGE = (XT + WT) * LL_TILE, LOADS = LX + LW * EACH;
     static_assert(TM * WM * 16 == BM && TN * WN * 16 == BN && LW * WAVES == WT && (D + 1) * STAGE <= LL_LDS, "tiles");
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     // Workgroups go to the dies in turn: a die gets consecutive tiles, row tiles of X innermost, so that the rows of W
@@ -500,14 +494,17 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
         x_kib[l] = min(wave * LX + l, XT - 1);
         x_from[l] = min(x_kib[l], (blocks - m0 / 16) * PARTS - 1) * SIA_WAVE + lane;
     }
-    const float* w_from[LW];
-    int piece[LW];
+    const float* const w_tile = W + (size_t)n0 * K;
+    unsigned w_from[LW * EACH];      // (f32_plan: K is below 2^22 where the tiles take W)
+    int piece[LW * EACH];
 #pragma unroll
-    for (int l = 0; l < LW; ++l) {      // rows that do not exist are read as the last one and not stored
-        const int row = (wave * LW + l) * 8 + lane / 8;
-        w_from[l] = Wt + (size_t)min(n0 + row, N - 1) * Kt;
-        piece[l] = ((lane & 7) ^ turn(row & 15)) * 4;
-    }
+    for (int l = 0; l < LW; ++l)
+#pragma unroll
+        for (int q = 0; q < EACH; ++q) {      // rows that do not exist are read as the last one and not stored
+            const int row = (wave * LW + l) * 8 + row_of_load<WIDE>(q, lane);
+            w_from[l * EACH + q] = (unsigned)(min(n0 + row, N - 1) - n0) * (unsigned)K;
+            piece[l * EACH + q] = k_of_load<WIDE>(row & 15, lane);
+        }
     const int x_at = wm * TM * PARTS * LL_TILE + lane * 16, w_at = XT * LL_TILE + (wn * (BN / WN) + r) * 128;
     const int place[2] = {((2 * g) ^ turn(r)) * 16, ((2 * g + 1) ^ turn(r)) * 16};
 
@@ -520,9 +517,11 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
 #pragma unroll
         for (int l = 0; l < LX; ++l) load_to_lds(from + x_from[l], to + x_kib[l] * LL_TILE);
         to += XT * LL_TILE + wave * LW * LL_TILE;
-        // behind the last k: the row's last four (X's parts are zero there)
 #pragma unroll
-        for (int l = 0; l < LW; ++l) load_to_lds(w_from[l] + min((begin + s) * CHUNK + piece[l], Kt - 4), to + l * LL_TILE);
+        for (int l = 0; l < LW; ++l)      // (X's parts are zero behind the last k)
+#pragma unroll
+            for (int q = 0; q < EACH; ++q)
+                load_chunk<WIDE>(w_tile + w_from[l * EACH + q], (begin + s) * CHUNK + piece[l * EACH + q], K, to + l * LL_TILE, q);
     };
     f32x4 total[TM][TN], small[TM][TN], sum[SLICED ? TM : 1][SLICED ? TN : 1];      // of the slice, of the slices before it
 #pragma unroll
@@ -714,23 +713,25 @@ constexpr int N_F32_SHAPES = sizeof(F32_SHAPES) / sizeof(F32_SHAPES[0]);
 struct F32Plan {
     int shape;      // -1: the few-row kernel
     bool apart;
-    long long parts, copied, slices;      // bytes of the workspace
+    long long parts, slices;      // bytes of the workspace
 };
 
-// direct: both operands' rows begin at multiples of 16 bytes.
-static F32Plan f32_plan(int M, int N, int K, bool direct) {
-    F32Plan best{-1, false, 0, 0, 0};
-    const int cus = compute_units(), n_slices = slices_of(N, K), chunks = (K + CHUNK - 1) / CHUNK, stride = (K + 3) / 4 * 4;
-    const long long copied = direct ? 0 : (long long)N * stride * 4;
-    if (M <= 16 || copied > 1LL << 28) return best;
-    // the few-row kernel: what its workgroups fetch (their rows of W and X, from L2 for the most part), or W from memory; float by float it
-    // takes twice as long
+static bool wide_rows(const float* rows, int K) { return K % 4 == 0 && ((uintptr_t)rows & 15) == 0; }
+
+// wide_x, wide_w: wide_rows of either.
+static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w) {
+    F32Plan best{-1, false, 0, 0};
+    const int cus = compute_units(), n_slices = slices_of(N, K), chunks = (K + CHUNK - 1) / CHUNK;
+    if (M <= 16 || K >= 1 << 22) return best;
+    // the few-row kernel: what its workgroups fetch (their rows of W and X, from L2 for the most part), or W from memory.
+    // Float by float 1.2 to 2 times as long.
     const FewRows few = few_rows_shape(M, N, K);
     const int rows_w = few.nb * 16, rows_x = few.mb * 16;
     const double fetched = (double)((M + rows_x - 1) / rows_x) * ((N + rows_w - 1) / rows_w) * (rows_w + rows_x) * K * 4e-6;
-    double least = (few.launch + fmax(fetched / few.rate, (double)N * K * 4e-6 / 5.4)) * (direct ? 1 : 3);
+    double least = (few.launch + fmax(fetched / few.rate, (double)N * K * 4e-6 / 5.4)) * (wide_x && wide_w ? 1 : 1.6);
     for (int i = 0; i < N_F32_SHAPES; ++i) {
         const F32Shape& t = F32_SHAPES[i];
+        if (t.bn == 256 && !wide_w) continue;      // four times the loads' addresses would spill
         const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int apart = 0; apart <= (n_slices > 1); ++apart) {
             const F32Cost& c = apart ? t.apart : t.whole;
@@ -738,7 +739,7 @@ static F32Plan f32_plan(int M, int N, int K, bool direct) {
             if (workgroups > 1 << 30 || (apart && (long long)n_slices * M * N > 1LL << 27)) continue;
             const int steps = apart ? (chunks + n_slices - 1) / n_slices : chunks;
             const double full = (double)(workgroups / room), last = (double)((workgroups % room + cus - 1) / cus);      // of `last` workgroups a unit
-            double us = (direct ? 0 : 4) + c.launch + (full + (last > 0)) * (c.round + c.step * steps) + (full * t.at_a_time + last) * c.more * steps;
+            double us = c.launch + (full + (last > 0)) * (c.round + c.step * steps) + (full * t.at_a_time + last) * c.more * steps;
             if (apart) us += c.sums * n_slices * M * N * 8e-6;
             else us += c.sums * (n_slices - 1) * M * N * 8e-6;
             if (us >= least) continue;
@@ -748,18 +749,17 @@ static F32Plan f32_plan(int M, int N, int K, bool direct) {
     }
     if (best.shape < 0) return best;
     best.parts = (long long)((M + 15) / 16) * chunks * PART_BLOCK * 16;
-    best.copied = copied;
     best.slices = best.apart ? (long long)n_slices * M * ((N + 3) / 4 * 4) * 4 : 0;
     return best;
 }
 
-template <int BM, int BN, int WM, int WN, int D, bool SLICED>
-static int launch_f32_shape(const float* X, const float* W, const float* Wt, float* Y, u32x4* parts, float* slices, int M, int N, int K, int Kt,
+template <int BM, int BN, int WM, int WN, int D, bool SLICED, bool WIDE>
+static int launch_f32_shape(const float* X, const float* W, float* Y, u32x4* parts, float* slices, int M, int N, int K,
                             bool apart, bool four, hipStream_t stream) {
     constexpr int bytes = (D + 1) * (BM / 16 * PARTS + BN / 8) * LL_TILE;
     const int n_slices = slices_of(N, K), tiles_m = (M + BM - 1) / BM;
     const int n_tiles = tiles_m * ((N + BN - 1) / BN) * (apart ? n_slices : 1), per_die = (n_tiles + 7) / 8;
-    const auto kernel = gemm_f32_tile_kernel<BM, BN, WM, WN, D, SLICED>;
+    const auto kernel = gemm_f32_tile_kernel<BM, BN, WM, WN, D, SLICED, WIDE>;
     static bool set[64];      // more LDS than a kernel gets unasked, allowed once per device
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return (int)hipGetLastError();
@@ -768,24 +768,24 @@ static int launch_f32_shape(const float* X, const float* W, const float* Wt, flo
         if (e != hipSuccess) return (int)e;
         if (device >= 0 && device < 64) set[device] = true;
     }
-    hipLaunchKernelGGL(kernel, dim3(8 * per_die), dim3(WM * WN * SIA_WAVE), bytes, stream, parts, X, W, Wt, Y, slices, M, N, K, Kt, (N + 3) / 4 * 4,
+    hipLaunchKernelGGL(kernel, dim3(8 * per_die), dim3(WM * WN * SIA_WAVE), bytes, stream, parts, X, W, Y, slices, M, N, K, (N + 3) / 4 * 4,
                        n_slices, apart, four, tiles_m, n_tiles, per_die);
     return SIA_LAUNCH_CHECK();
 }
 
-template <int BM, int BN, int WM, int WN, int D>
-static int launch_f32_tiles(const float* X, const float* W, const float* Wt, float* Y, u32x4* parts, float* slices, int M, int N, int K, int Kt,
-                            bool apart, bool four, hipStream_t stream) {
+template <int BM, int BN, int WM, int WN, int D, bool WIDE>
+static int launch_f32_tiles(const float* X, const float* W, float* Y, u32x4* parts, float* slices, int M, int N, int K, bool apart, bool four,
+                            hipStream_t stream) {
     if (apart || slices_of(N, K) == 1 || BN == 256)      // (registers of the large ones are full)
-        return launch_f32_shape<BM, BN, WM, WN, D, false>(X, W, Wt, Y, parts, slices, M, N, K, Kt, apart, four, stream);
-    return launch_f32_shape<BM, BN, WM, WN, D, BN != 256>(X, W, Wt, Y, parts, slices, M, N, K, Kt, false, four, stream);
+        return launch_f32_shape<BM, BN, WM, WN, D, false, WIDE>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
+    return launch_f32_shape<BM, BN, WM, WN, D, BN != 256, WIDE>(X, W, Y, parts, slices, M, N, K, false, four, stream);
 }
 
-// Bytes of workspace that a product of this size wants (0: none).  direct: K is a multiple of 4 and X and W are on 16 bytes.
-SIA_EXPORT long long sia_gemm_f32_workspace(int M, int N, int K, int direct) {
+// Bytes of workspace that this product wants (0: none).
+SIA_EXPORT long long sia_gemm_f32_workspace(const float* X, const float* W, int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
-    const F32Plan plan = f32_plan(M, N, K, direct);
-    return plan.shape < 0 ? 0 : plan.parts + plan.copied + plan.slices;
+    const F32Plan plan = f32_plan(M, N, K, wide_rows(X, K), wide_rows(W, K));
+    return plan.shape < 0 ? 0 : plan.parts + plan.slices;
 }
 
 // With `workspace` (of sia_gemm_f32_workspace bytes, on 16) the tiles where they are the faster way; without, the few-row kernel, whatever M
@@ -793,30 +793,26 @@ SIA_EXPORT long long sia_gemm_f32_workspace(int M, int N, int K, int direct) {
 SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* workspace, int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K <= 0 || ((uintptr_t)workspace & 15)) return SIA_BAD_ARGUMENT;
-    const bool direct = K % 4 == 0 && aligned16(X, W), four = N % 4 == 0 && ((uintptr_t)Y & 15) == 0;
-    const F32Plan plan = workspace ? f32_plan(M, N, K, direct) : F32Plan{-1, false, 0, 0, 0};
+    const bool wide_x = wide_rows(X, K), wide_w = wide_rows(W, K), four = N % 4 == 0 && ((uintptr_t)Y & 15) == 0;
+    const F32Plan plan = workspace ? f32_plan(M, N, K, wide_x, wide_w) : F32Plan{-1, false, 0, 0};
     if (plan.shape < 0) {
         constexpr int MOST = 65535 * 16;      // rows of a launch
-        for (; M > MOST; M -= MOST, X += (size_t)MOST * K, Y += (size_t)MOST * N) few_rows(X, W, Y, MOST, N, K, direct, stream);
-        few_rows(X, W, Y, M, N, K, direct, stream);
+        for (; M > MOST; M -= MOST, X += (size_t)MOST * K, Y += (size_t)MOST * N) few_rows(X, W, Y, MOST, N, K, wide_x && wide_w, stream);
+        few_rows(X, W, Y, M, N, K, wide_x && wide_w, stream);
         return SIA_LAUNCH_CHECK();
     }
     u32x4* const parts = (u32x4*)workspace;
-    f32x4* const copy = (f32x4*)((char*)workspace + plan.parts);
-    float* const slices = (float*)((char*)workspace + plan.parts + plan.copied);
-    const int blocks = (M + 15) / 16, chunks = (K + CHUNK - 1) / CHUNK, Kt = (K + 3) / 4 * 4, Ns = (N + 3) / 4 * 4;
+    float* const slices = (float*)((char*)workspace + plan.parts);
+    const int blocks = (M + 15) / 16, chunks = (K + CHUNK - 1) / CHUNK, Ns = (N + 3) / 4 * 4;
     hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)(((long long)blocks * chunks + 3) / 4)), dim3(256), 0, stream, X, parts, M, K, blocks, chunks,
-                       direct);
-    if (!direct) {
-        const size_t pieces = (size_t)N * (Kt / 4);
-        hipLaunchKernelGGL(align_rows_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, W, copy, K, Kt, pieces);
-    }
-    const float* const Wt = direct ? W : (const float*)copy;
+                       wide_x);
     const bool apart = plan.apart;
     int status = SIA_BAD_ARGUMENT;
-#define SHAPE(I, ...) \
-    if (plan.shape == I) status = launch_f32_tiles<__VA_ARGS__>(X, W, Wt, Y, parts, slices, M, N, K, Kt, apart, four, stream)
-    SHAPE(0, 96, 256, 2, 4, 2);
+#define SHAPE(I, ...)         \
+    if (plan.shape == I)     \
+    status = wide_w ? launch_f32_tiles<__VA_ARGS__, true>(X, W, Y, parts, slices, M, N, K, apart, four, stream)      \
+                    : launch_f32_tiles<__VA_ARGS__, false>(X, W, Y, parts, slices, M, N, K, apart, four, stream)
+    if (plan.shape == 0) status = launch_f32_tiles<96, 256, 2, 4, 2, true>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
     SHAPE(1, 64, 128, 2, 2, 1);
     SHAPE(2, 64, 128, 2, 4, 2);
     SHAPE(3, 32, 64, 2, 2, 2);

@@ -111,7 +111,7 @@ _SIGNATURES = {
     "sia_attention_generic_max_head_dim": [],
     "sia_gemm_generic": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_f32": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
-    "sia_gemm_f32_workspace": [_c_int, _c_int, _c_int, _c_int],
+    "sia_gemm_f32_workspace": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int],
     "sia_prenorm_block": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_prenorm_mixer": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
     "sia_sample": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
@@ -1024,7 +1024,7 @@ class HipKernels:
         """``y = x @ w^T`` in float32 (csrc/gemm_f32.hip); the rows' parts and the slices of k lie in a workspace."""
         M, K = x.shape
         N = w.shape[0]
-        size = self.core.sia_gemm_f32_workspace(M, N, K, int(K % 4 == 0 and _in_pieces(x, w)))
+        size = self.core.sia_gemm_f32_workspace(_ptr(x), _ptr(w), M, N, K)
         workspace = torch.empty(size, dtype=torch.uint8, device=x.device) if size else None
         self._check(self.core.sia_gemm_f32(_ptr(x), _ptr(w), _ptr(y), _ptr(workspace), M, N, K, self._stream()), "gemm_f32")
 

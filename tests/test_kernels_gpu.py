@@ -562,6 +562,26 @@ def test_float32_products_of_parts(hip, N, K, bits):
         assert torch.equal(hip.linear(x[:M].contiguous(), flat[1:].view(N, K)), all_rows[:M]), M
 
 
+@pytest.mark.parametrize("N, K", [(7, 1), (130, 35), (2050, 1056), (1000, 334), (16388, 2047), (33000, 258)])
+def test_float32_products_of_rows_that_begin_anywhere(hip, N, K):
+    """Either operand, or both, one to three floats behind a multiple of 16 bytes, rows of any length: the bits of operands that are not, and a
+    last k whose neighbours in W are not finite.  Nothing is copied for it: W does not count in the workspace, whatever its size."""
+    x, w = rnd(303, K, seed=1), rnd(N, K, seed=2)
+    want = x.double() @ w.double().T
+    want32 = hip.linear(x, w)
+    assert bool(((want32.double() - want).abs() <= (24 + K / 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-30).all())
+
+    def shifted(t, by):
+        flat = torch.full((t.numel() + 8,), float("nan"), device=DEV)
+        flat[by:by + t.numel()] = t.flatten()
+        return flat[by:by + t.numel()].view(t.shape)
+
+    for M in (1, 8, 9, 17, 40, 130, 303):
+        for bx, bw in ((1, 0), (0, 2), (3, 1), (2, 2)):
+            assert torch.equal(hip.linear(shifted(x[:M], bx), shifted(w, bw)), want32[:M]), (M, bx, bw)
+    assert 0 < hip.core.sia_gemm_f32_workspace(x.data_ptr(), w.data_ptr() + 4, 303, 40000, 2049) < 40000 * 2049
+
+
 @pytest.mark.parametrize("M, N, K", [(3, 96, 64), (40, 520, 333), (100, 2048, 512), (70, 40000, 64), (40, 12800, 256)])
 def test_float32_products_that_are_not_finite(hip, M, N, K):
     """Infinities, NaN, products of an infinity with zero and the largest finite numbers give what floats give."""
