@@ -1593,6 +1593,9 @@ class HipKernels:
         N = w.shape[0]
         out_dtype = torch.float32 if (out_float32 or x.dtype == torch.float32) else x.dtype
         y = torch.empty((M, N), dtype=out_dtype, device=x.device)
+        if x.dtype == torch.float32:
+            self._float_product(x, w, y)
+            return y
         self._check(self.core.sia_gemm_generic(_ptr(x), _ptr(w), _ptr(y), M, N, K, _DT[x.dtype],
                                                int(out_dtype == torch.float32), self._stream()), "gemm_generic")
         return y

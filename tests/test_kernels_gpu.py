@@ -135,6 +135,16 @@ def test_gemm_generic(hip, dtype, shape):
         torch.testing.assert_close(out.double(), ref, **tol(dtype))
 
 
+def test_gemm_generic_in_float32_has_the_tiles_workspace(hip):
+    x, w, seen, real = rnd(303, 512, seed=1), rnd(4096, 512, seed=2), [], hip.core.sia_gemm_f32
+    hip.core.sia_gemm_f32 = lambda *a: seen.append(a[3]) or real(*a)
+    try:
+        assert torch.equal(hip.gemm_generic(x, w), hip.linear(x, w))
+    finally:
+        hip.core.sia_gemm_f32 = real
+    assert len(seen) == 2 and all(seen)
+
+
 @pytest.mark.parametrize("shape", [(1, 48, 64), (8, 5120, 3072), (16, 3072, 8192), (3, 16, 320), (11, 1008, 1024),
                                    (7, 203, 192), (2, 1, 64), (9, 4099, 128), (16, 16384, 576)])
 def test_gemm_skinny(hip, shape):
