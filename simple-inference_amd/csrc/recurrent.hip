@@ -682,6 +682,9 @@ __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __re
 // block of channels takes the channels 4 g + i.  S and A are multiplied as floats (v_mfma_f32_16x16x4_f32); k R goes into the state's
 // product as the three bfloat16 numbers that it is the sum of, values as they are (v_mfma_f32_16x16x16_bf16, float sums).
 // All but the values is staged in LDS a block at a time, requested a block ahead.
+// A run or segment with a number of more than 2^32 among its q, k and v, or one that is not finite, is then taken again, token by token on
+// the vector units (one NaN among 2,048 tokens of 24 heads of 128 x 128 127 -> 630 us, beside 63 tokens in a run of 449 458 -> 600): a product by zero carries such a number to the tokens of its block in front of it, and k / P or q k
+// may leave the range of floats where the recurrence does not.
 // Segments behind one another: with OUT false only what a segment adds to the state (all but a sequence's last), and the product of its
 // decays; block_states_kernel makes the states in front of the segments; with OUT true the outputs, from there.
 // What bounds it: the barriers between staging, A and products, LDS (a wave reads 13 KiB a block) and the float products (36 of 32
@@ -693,6 +696,8 @@ __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __re
 // D up to BLOCK_D and a multiple of 16.  KF, q_share, state_stride, BEFORE and the segments as in the walk above.
 constexpr int BLOCK_TOKENS = 16, BLOCK_COLUMN = BLOCK_TOKENS + 4;
 constexpr float BLOCK_LEAST = 9.094947e-13f;      // 2^-40
+constexpr float BLOCK_MOST = 4294967296.f;        // 2^32
+constexpr int BLOCK_MOST_V = 0x4f80;              // the same in bfloat16
 typedef short segshort4 __attribute__((ext_vector_type(4)));
 template <int BLOCK_D, bool OUT, bool KF, bool BEFORE>
 __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
@@ -708,6 +713,7 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
     __shared__ __attribute__((aligned(16))) float end_s[BLOCK_D];                     // P of the block's last token
     __shared__ __attribute__((aligned(16))) float a_s[OUT ? BLOCK_WAVES * T * BLOCK_COLUMN : 4];      // [wave's channels][t][s]
     __shared__ int by_pairs[2];      // of 64 channels each
+    __shared__ int any_odd;
     const int n_slices = (Dv + BLOCK_D - 1) / BLOCK_D;
     const int seq = blockIdx.x, head = blockIdx.y, slice = blockIdx.z % n_slices, seg = blockIdx.z / n_slices;
     const int begin = cu_q[seq], first = begin + seg * cut.len, end = cu_q[seq + 1];
@@ -756,6 +762,8 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
     };
     request(first);
     float seg_product = 1.f;
+    if (tid == 0) any_odd = 0;
+    bool odd = false;
     for (int t0 = first; t0 < last; t0 += T) {
         const int nt = min(T, last - t0);
         if (nt < T || !has_ch)
@@ -763,6 +771,12 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
             for (int t = 0; t < T; ++t)
                 if (!has_ch || t >= nt) x[t] = 0.f, al[t] = 1.f;
         const segshort4 v = {(short)v_next[0], (short)v_next[1], (short)v_next[2], (short)v_next[3]};      // of no weight behind the last token: k is zero there
+        if (stages) {
+            float most[2] = {0.f, 0.f};      // NaN and infinities stay
+#pragma unroll
+            for (int t = 0; t < T; ++t) most[t & 1] += fabsf(x[t]);
+            odd |= !(most[0] + most[1] <= BLOCK_MOST);
+        }
         if (role == 1) {
             float p = 1.f;
 #pragma unroll
@@ -772,6 +786,7 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
             }
             end_s[ch] = p;
             seg_product *= p;
+            odd |= !(p <= BLOCK_MOST);      // (decays are at most one)
 #pragma unroll
             for (int e = 0; e < PARTS; ++e)
 #pragma unroll
@@ -840,6 +855,8 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
             __syncthreads();
         }
         if (has_j) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) odd |= (v[i] & 0x7fff) > BLOCK_MOST_V;
             if (OUT) {
                 segf32x4 o[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
                 float4 a4 = make_float4(0.f, 0.f, 0.f, 0.f);      // A_ts of t = r, s = 4 g .. 4 g + 3
@@ -881,9 +898,63 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
         }
         __syncthreads();
     }
+    if (odd) any_odd = 1;
+    __syncthreads();
     if (!OUT && role == 1 && has_ch && slice == 0)
         seg_decay[((size_t)segment_place(first, end, seq, cut) * n_heads + head) * D + ch] = seg_product;
-    if (has_j && (!OUT || last == end))
+    if (!has_j) return;
+    if (any_odd) {
+        const size_t per_token = (size_t)n_heads * D;
+        const int shared = head / q_share * D + 4 * g, own_at = head * D + 4 * g;
+        float s[TILES][4];      // (S itself, in the registers of the products, would spill)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // what is written again has been written
+#pragma unroll
+        for (int b = 0; b < TILES; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[b][i] = OUT && 16 * b < D ? (is_cut ? segment : own)[(16 * b + i) * Dv + from] : 0.f;
+#pragma clang loop unroll(disable)
+        for (int n = first; n < last; ++n) {
+            const bf16_t* row = proj + (size_t)n * row_stride;
+            const float vj = bf16_to_float(row[v_at]);
+            float o = 0.f;
+#pragma unroll
+            for (int b = 0; b < TILES; ++b)
+                if (16 * b < D) {
+                    const float4 a = *reinterpret_cast<const float4*>(alpha + n * per_token + own_at + 16 * b);
+                    float4 k, q;
+                    if constexpr (KF)
+                        k = *reinterpret_cast<const float4*>(k_f32 + n * per_token + own_at + 16 * b);
+                    else {
+                        const ushort4 u = *reinterpret_cast<const ushort4*>(row + k_col + shared + 16 * b);
+                        k = make_float4(bf16_to_float(u.x), bf16_to_float(u.y), bf16_to_float(u.z), bf16_to_float(u.w));
+                    }
+                    if constexpr (OUT) {
+                        const ushort4 u = *reinterpret_cast<const ushort4*>(row + q_col + shared + 16 * b);
+                        q = make_float4(bf16_to_float(u.x), bf16_to_float(u.y), bf16_to_float(u.z), bf16_to_float(u.w));
+                    }
+                    const float ai[4] = {a.x, a.y, a.z, a.w}, ki[4] = {k.x, k.y, k.z, k.w}, qi[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float moved = fmaf(ki[i], vj, ai[i] * s[b][i]);
+                        if constexpr (OUT) o = fmaf(qi[i] * q_scale, BEFORE ? s[b][i] : moved, o);
+                        s[b][i] = moved;
+                    }
+                }
+            if constexpr (OUT) {
+                o += __shfl_xor(o, 16, SIA_WAVE);
+                o += __shfl_xor(o, 32, SIA_WAVE);
+                if (g == 0) raw_out[((size_t)n * n_heads + head) * Dv + j] = o;
+            }
+        }
+        if (!OUT || last == end)
+#pragma unroll
+            for (int b = 0; b < TILES; ++b)
+                if (16 * b < D)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) (OUT ? own : segment)[(16 * b + i) * Dv + from] = s[b][i];
+        return;
+    }
+    if (!OUT || last == end)
 #pragma unroll
         for (int b = 0; b < TILES; ++b)
             if (16 * b < D)      // a multiple of 16

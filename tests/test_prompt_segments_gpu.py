@@ -127,6 +127,33 @@ def test_runs_by_blocks_against_64_bits(H, D, Dv, lengths, decay):
     assert bool(((y - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.std()).all()), float((y - ref).abs().max())
 
 
+@pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
+@pytest.mark.parametrize("H,D,Dv,lengths", [(2, 128, 128, [70, 41]), (2, 64, 64, [300, 64]), (1, 128, 64, [200, 100])])
+def test_numbers_without_bounds_reach_no_earlier_token(op, H, D, Dv, lengths):
+    """Infinities, NaN and numbers whose products leave the range of floats, in the columns of queries, keys and values: blocks of tokens
+    give what the tokens one after the other give, NaN in the same places, and finite results in front of them.  (At 2^127 whether a sum of
+    128 such products overflows on its way is a matter of its order; 2^110 leaves it 2^17.  An infinite state is NaN behind a whole segment whose decays' product is zero.)"""
+    from simple_inference_amd.kernels import HipKernels
+
+    if op == "bonus":
+        Dv = D
+    k, n = HipKernels(), sum(lengths)
+    clean = projected(torch.Generator().manual_seed(D), n, H, D, Dv)
+    for at, column in ((21, 3), (37, H * D + 5), (46, 2 * H * D + 9), (lengths[0] + 20, H * D + 8)):
+        for value in (float("inf"), float("-inf"), float("nan"), 2.0 ** 100, -2.0 ** 110):
+            rows = clean.clone()
+            rows[at, column] = value
+            whole, state, _ = run(op, k, rows, H, D, Dv, lengths, 10 ** 6)
+            tokens, want, _ = run(op, k, rows, H, D, Dv, lengths, 16)
+            first = 0 if at < lengths[0] else lengths[0]
+            assert bool(whole[first:at].isfinite().all()), (at, column, value)
+            assert torch.equal(whole.isnan(), tokens.isnan()) and torch.equal(state.isfinite(), want.isfinite()), (at, column, value)
+            spread = 1e-3 * float(tokens[tokens.isfinite()].std())
+            assert bool(((whole - tokens).abs() <= 2.0 ** -7 * tokens.abs() + spread)[tokens.isfinite()].all()), (at, column, value)
+            same = want.isfinite()
+            assert float((state - want)[same].abs().max()) <= 2e-5 * float(want[same].abs().max()), (at, column, value)
+
+
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("H,Dv,n", [(1, 8, 3), (3, 24, 33), (5, 64, 51), (2, 136, 40), (3, 256, 7), (2, 512, 129), (3, 20, 33)])
 def test_norm_and_gate_behind_a_prompt_s_recurrence(H, Dv, n, shift):
