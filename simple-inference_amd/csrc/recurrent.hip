@@ -697,6 +697,7 @@ __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __re
 constexpr int BLOCK_TOKENS = 16, BLOCK_COLUMN = BLOCK_TOKENS + 4;
 constexpr float BLOCK_LEAST = 9.094947e-13f;      // 2^-40
 constexpr float BLOCK_MOST = 4294967296.f;        // 2^32
+constexpr float BLOCK_SCALE = 1099511627776.f;    // 2^40: k R, which may be as small as floats get, goes into its parts that much larger
 constexpr int BLOCK_MOST_V = 0x4f80;              // the same in bfloat16
 typedef short segshort4 __attribute__((ext_vector_type(4)));
 template <int BLOCK_D, bool OUT, bool KF, bool BEFORE>
@@ -778,12 +779,13 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
             odd |= !(most[0] + most[1] <= BLOCK_MOST);
         }
         if (role == 1) {
-            float p = 1.f;
+            float p = BLOCK_SCALE;
 #pragma unroll
             for (int t = T - 1; t >= 0; --t) {
                 x[t] *= p;
                 p *= al[t];
             }
+            p *= 1.f / BLOCK_SCALE;
             end_s[ch] = p;
             seg_product *= p;
             odd |= !(p <= BLOCK_MOST);      // (decays are at most one)
@@ -891,6 +893,7 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
 #pragma unroll
                 for (int e = PARTS - 1; e >= 0; --e)
                     added = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(segshort4, kr_s[e][16 * b + r][g]), v, added, 0, 0, 0);
+                added *= 1.f / BLOCK_SCALE;
                 S[b][0] = fmaf(S[b][0], p.x, added[0]), S[b][1] = fmaf(S[b][1], p.y, added[1]);
                 S[b][2] = fmaf(S[b][2], p.z, added[2]), S[b][3] = fmaf(S[b][3], p.w, added[3]);
                 if (b % 2) __builtin_amdgcn_sched_barrier(0);

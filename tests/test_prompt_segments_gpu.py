@@ -127,6 +127,32 @@ def test_runs_by_blocks_against_64_bits(H, D, Dv, lengths, decay):
     assert bool(((y - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * ref.std()).all()), float((y - ref).abs().max())
 
 
+@pytest.mark.parametrize("H,D,Dv,lengths", [(2, 64, 64, [40, 16]), (1, 128, 128, [300])])
+def test_small_keys_keep_their_bits_in_runs_by_blocks(H, D, Dv, lengths):
+    """Keys around 2^-122, whose last bits times a decay lie below what bfloat16 numbers hold: a state's error is as for others (four units
+    in the last place a token for the decays, some 100 sums)."""
+    from simple_inference_amd.kernels import HipKernels
+
+    k, n, qk, v = HipKernels(), sum(lengths), H * D, H * Dv
+    g = torch.Generator().manual_seed(D)
+    cols = (0, qk, 2 * qk, 2 * qk + v, 2 * qk + 2 * v)
+    rows = rnd(g, n, cols[4] + 32)
+    rows[:, qk:2 * qk] *= 2.0 ** -122
+    rows = rows.to(torch.bfloat16).to(DEV)
+    a2, bias = rnd(g, qk, 32, std=0.1).to(torch.bfloat16).to(DEV), rnd(g, qk, std=0.1).float().to(DEV)
+    state = torch.zeros(len(lengths), H, D, Dv, device=DEV)
+    want, size, x, t = state.double(), state.double(), rows.double(), 0
+    alpha = torch.exp(torch.nn.functional.logsigmoid(x[:, cols[4]:] @ a2.double().T + bias.double()) / 4).view(n, H, D, 1)
+    for s, length in enumerate(lengths):
+        for _ in range(length):
+            added = x[t, qk:2 * qk].view(H, D, 1) * x[t, 2 * qk:cols[3]].view(H, 1, Dv)
+            want[s], size[s] = alpha[t] * want[s] + added, alpha[t] * size[s] + added.abs()
+            t += 1
+    k.gla_recurrent(rows, cols, a2, bias, torch.ones(Dv, device=DEV), H, D, Dv, 4.0, D ** -0.5, 1e-5,
+                    context(DEV, lengths, list(range(len(lengths)))), LayerCache(state=state))
+    assert bool(((state.double() - want).abs() <= (4 * max(lengths) + 100) * 2.0 ** -24 * size + n * 2.0 ** -149).all()), float(((state.double() - want).abs() / size).max())
+
+
 @pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
 @pytest.mark.parametrize("H,D,Dv,lengths", [(2, 128, 128, [70, 41]), (2, 64, 64, [300, 64]), (1, 128, 64, [200, 100])])
 def test_numbers_without_bounds_reach_no_earlier_token(op, H, D, Dv, lengths):
