@@ -745,17 +745,16 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
     uint16_t v_next[4];
     const unsigned x_at = (unsigned)((role == 0 ? q_col : k_col) + at), f_at = (unsigned)at_f, v_at = (unsigned)(v_col + head * Dv + j);
     auto request = [&](int t0) {      // tokens behind the last repeat it
+        auto row = [&](int t) { return (size_t)__builtin_amdgcn_readfirstlane(min(t0 + t, last - 1)); };      // it begins at a scalar
         if (stages) {
+            if (KF && role != 0)      // one branch, nothing converted in it: a conversion waits for its load
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
-                const size_t n = __builtin_amdgcn_readfirstlane(min(t0 + t, last - 1));      // a row begins at a scalar
-                const float* floats = alpha + n * n_heads * D;
-                if (KF && role != 0)
-                    x[t] = (k_f32 + n * n_heads * D)[f_at];
-                else
-                    x[t] = bf16_to_float((proj + n * row_stride)[x_at]);
-                al[t] = floats[f_at];
-            }
+                for (int t = 0; t < T; ++t) x[t] = (k_f32 + row(t) * n_heads * D)[f_at];
+            else
+#pragma unroll
+                for (int t = 0; t < T; ++t) x[t] = __uint_as_float((uint32_t)(proj + row(t) * row_stride)[x_at]);
+#pragma unroll
+            for (int t = 0; t < T; ++t) al[t] = (alpha + row(t) * n_heads * D)[f_at];
         }
         if (has_j)
 #pragma unroll
@@ -767,6 +766,9 @@ __global__ __launch_bounds__(BLOCK_D / 16 * SIA_WAVE, 4) void gla_blocks_kernel(
     bool odd = false;
     for (int t0 = first; t0 < last; t0 += T) {
         const int nt = min(T, last - t0);
+        if (stages && (!KF || role == 0))
+#pragma unroll
+            for (int t = 0; t < T; ++t) x[t] = __uint_as_float(__float_as_uint(x[t]) << 16);
         if (nt < T || !has_ch)
 #pragma unroll
             for (int t = 0; t < T; ++t)
