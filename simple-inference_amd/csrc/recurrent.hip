@@ -1211,7 +1211,10 @@ static bool gla_slices(int n_seqs, int max_q_len, int n_heads) {
 #define WALK_MIN_RUN 128
 
 // Whether runs go by blocks on the matrix cores, from BLOCKS_MIN_RUN tokens on (two blocks: even with the walk, 29 us for 24 heads of
-// 128 x 128; one block of 20 tokens 25 / 24).  States that leave more than half of a workgroup's channels or columns empty are walked.
+// 128 x 128; one block of 20 tokens 25 / 24).
+// A workgroup has room for 64 channels and columns where the state has 64 channels, else for 128: with 128, half of the products
+// of 64 channels multiplied nothing (us, walk, 128, 64:  16 of 64 x 128, 449 tokens beside 63 254, 295, 225, 16 runs of 200 123, 88, 69;  8 of 64 x 144,
+// 449 beside 63 197, 259, 165).  80 to 112 channels fill 128 by halves and more, and are faster so than walked (8 of 80 x 192, 2,048 tokens 128 -> 87).
 #define BLOCKS_MIN_RUN 32
 static bool by_blocks(int D, int Dv) { return D % 16 == 0 && D >= 64 && D <= 128 && Dv % 16 == 0 && Dv >= 64; }
 
@@ -1368,7 +1371,7 @@ static int launch_recurrence(const void* proj, int row_stride, int q_col, int k_
         float* seg_state = raw_space + (size_t)n_tokens * n_heads * Dv;
         if (blocks && long_runs) {
             float* seg_decay = raw;      // behind the states nobody reads them, and the outputs come after
-            const int width = D <= 64 && Dv <= 64 ? 64 : 128;
+            const int width = D <= 64 ? 64 : 128;
             const dim3 bgrid(n_seqs, n_heads, (Dv + width - 1) / width * n_segs), bblock(width / 16 * SIA_WAVE);
 #define BLOCKS_AS(WIDTH, OUT, KF, BEFORE)                                                                                    \
     hipLaunchKernelGGL((gla_blocks_kernel<WIDTH, OUT, KF, BEFORE>), bgrid, bblock, 0, stream, (const bf16_t*)proj, row_stride,   \

@@ -90,7 +90,7 @@ def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, len
 @pytest.mark.parametrize("decay", ["usual", "strong", "mixed"])
 @pytest.mark.parametrize("H,D,Dv,lengths", [
     (2, 64, 64, [32, 1, 15, 16, 17]), (3, 128, 128, [33, 47, 2]), (2, 80, 192, [100, 31, 1]), (1, 112, 80, [48] * 5), (2, 64, 144, [200, 3]),
-    (2, 128, 64, [513]), (1, 128, 128, [177, 300])])
+    (2, 128, 64, [513]), (1, 128, 128, [177, 300]), (1, 64, 272, [65, 50]), (2, 64, 128, [300, 17])])
 def test_runs_by_blocks_against_64_bits(H, D, Dv, lengths, decay):
     """Whole and cut runs, last blocks of one to 16 tokens, widths that leave waves or channels idle; decays as trained, decays that
     leave nothing within a block (which go pair by pair), and those in some channels only.  A state's error is that of its decays
