@@ -1210,12 +1210,13 @@ static bool gla_slices(int n_seqs, int max_q_len, int n_heads) {
 #define SEG_MIN 64
 #define WALK_MIN_RUN 128
 
-// Whether runs go by blocks on the matrix cores, from BLOCKS_MIN_RUN tokens on (two blocks: even with the walk, 29 us for 24 heads of
-// 128 x 128; one block of 20 tokens 25 / 24).
+// Whether runs go by blocks on the matrix cores, from BLOCKS_MIN_RUN tokens on.  us for one run, by the walk, by blocks, by blocks whose decays make
+// them go pair by pair:  24 heads of 128 x 128 with a bonus, 33 tokens 29, 28, 33;  48 33.6, 28.3, 33.5;  64 38.7, 32.7, 39.8;  128 62, 52, 66;  200 82,
+// 57, 63;  24 of 64 x 64 22.7, 21.2, 26.3;  25.5, 21.3, 26.7;  28.6, 24, 31;  45, 37, 51;  56, 39, 46.
 // A workgroup has room for 64 channels and columns where the state has 64 channels, else for 128: with 128, half of the products
 // of 64 channels multiplied nothing (us, walk, 128, 64:  16 of 64 x 128, 449 tokens beside 63 254, 295, 225, 16 runs of 200 123, 88, 69;  8 of 64 x 144,
 // 449 beside 63 197, 259, 165).  80 to 112 channels fill 128 by halves and more, and are faster so than walked (8 of 80 x 192, 2,048 tokens 128 -> 87).
-#define BLOCKS_MIN_RUN 32
+#define BLOCKS_MIN_RUN 48
 static bool by_blocks(int D, int Dv) { return D % 16 == 0 && D >= 64 && D <= 128 && Dv % 16 == 0 && Dv >= 64; }
 
 static long long segment_places(int n_tokens, int n_seqs, Segments cut) {
