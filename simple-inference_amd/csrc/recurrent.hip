@@ -688,11 +688,11 @@ __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __re
 // Segments behind one another: with OUT false only what a segment adds to the state (all but a sequence's last), and the product of its
 // decays; block_states_kernel makes the states in front of the segments; with OUT true the outputs, from there.
 // What bounds it: the barriers between staging, A and products, LDS (a wave reads 13 KiB a block) and the float products (36 of 32
-// cycles), about in equal parts; 124 registers leave two workgroups a unit.
+// cycles), by reading the code, about in equal parts; 128 registers leave two workgroups a unit.
 // us, a layer's recurrence with its decays and the finishing kernel, by the walk (with two or four columns a lane group) -> by blocks:  24 heads
-// of 128 x 128, one run of 33 tokens 29 -> 29, 64 39 -> 33, 128 60 -> 50, 200 85 -> 55, 512 104 -> 66, 2,048 214 -> 142 (the walk, its decays'
-// products, states and outputs 124 + 11 + 13 + 30 -> what segments add, states, outputs 29 + 13 + 64), 4,096 390 -> 244;  16 runs of 64 127 -> 66,
-// of 200 242 -> 157, one run of 449 beside 63 tokens 752 -> 449;  24 of 64 x 64, 2,048 115 -> 89;  8 of 128 x 64, 2,048 109 -> 72.
+// of 128 x 128, one run of 64 tokens 38 -> 31, 128 60 -> 49, 200 83 -> 52, 512 103 -> 62, 2,048 222 -> 131;  8 runs of 64 84 -> 42, 16 of 200 259 -> 135,
+// one run of 449 beside 63 tokens 740 -> 466;  24 of 64 x 64, 2,048 117 -> 70, 16 of 200 132 -> 72;  8 of 128 x 64, 2,048 109 -> 65.  With decays that go
+// pair by pair, lower-bounded gates, keys as floats:  24 of 128 x 128, 128 57 -> 60, 2,048 210 -> 147, 16 of 200 241 -> 168.
 // D up to BLOCK_D and a multiple of 16.  KF, q_share, state_stride, BEFORE and the segments as in the walk above.
 constexpr int BLOCK_TOKENS = 16, BLOCK_COLUMN = BLOCK_TOKENS + 4;
 constexpr float BLOCK_LEAST = 9.094947e-13f;      // 2^-40
@@ -1140,8 +1140,10 @@ __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_kernel
 
 // The same in bfloat16 for Dv a multiple of 8 and rows aligned to 16 bytes: a lane has eight neighbouring elements, 2^group_log lanes
 // (Dv / 8 or the next power of two; the lanes behind Dv add zeros) share a pair, so that a wave has up to 64 pairs and all of a lane's loads,
-// 16 bytes each, are on their way before the sum.  Bound by memory: 2,048 tokens of 24 heads of 128 move 50 MB.
-// FINISH_FIGURES
+// 16 bytes each, are on their way before the sum.  Bound by memory: 2,048 tokens of 24 heads of 128 move 50 MB, at 4.5 TB/s.
+// us, the kernel above -> this one:  24 heads of 128, 33 tokens 3.9 -> 3.9, 64 4.3 -> 4.6, 128 4.7 -> 4.1, 512 6.4 -> 4.9, 1,024 10.2 -> 7.2, 2,048 17.6 -> 11.2, 4,096
+// 34.4 -> 18.8;  24 of 64, 33 3.9 -> 4.0, 1,024 9.4 -> 5.0, 4,096 28.2 -> 11.0;  16 of 256, 64 4.6 -> 4.6, 2,048 19.0 -> 13.6;  4 of 512, 512 5.6 -> 4.0;  80 of
+// 16, 2,048 41.7 -> 6.6.
 __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_vec_kernel(
     const float* __restrict__ raw, const bf16_t* __restrict__ proj, int row_stride, int g_col, const float* __restrict__ norm_w,
     bf16_t* __restrict__ out, int n_pairs, int n_heads, int Dv, int group_log, float eps) {
@@ -1170,9 +1172,10 @@ __global__ __launch_bounds__(GLA_FINISH_WAVES * SIA_WAVE) void gla_finish_vec_ke
     y.store(out + (size_t)pair * Dv + c);
 }
 
-// The form with eight elements a lane where bfloat16 rows allow it (the 32-bit path keeps one order of sums whatever the step's addresses
-// are).  Else four pairs a wave where there are many narrow ones; a layer's recurrence, one and four, us:  24 heads of 128, 32 tokens 23.7 and
-// 25.8, 512: 75.1 and 75.9, 1,024: 91.5 and 91.2, 2,048: 138.9 and 137.7;  16 of 256, 32 tokens 24.9 and 27.7, 2,048: 149.0 and 151.6.
+// The form with eight elements a lane where bfloat16 rows allow it, from the smallest step on (figures there; the 32-bit path keeps one order
+// of sums whatever the step's addresses are).  Else four pairs a wave where there are many narrow ones, as the 32-bit path and rows that
+// begin anywhere have them;  one and four, a layer's recurrence as it was walked in bfloat16, us:  24 heads of 128, 512 tokens 75.1 and 75.9,
+// 1,024 91.5 and 91.2, 2,048 138.9 and 137.7;  16 of 256, 2,048 149.0 and 151.6.
 template <typename T>
 static void launch_finish(const float* raw, const void* proj, int row_stride, int g_col, const float* norm_w, void* out, int n_tokens,
                           int n_heads, int Dv, float eps, hipStream_t stream) {
@@ -1226,7 +1229,8 @@ static long long segment_places(int n_tokens, int n_seqs, Segments cut) {
 }
 
 // Whether runs that are not cut are walked with four columns a lane group (a longer chain a token, but LDS serves twice
-// the columns) or two: where the workgroups are many, and where two would not fit into LDS.  Four against two, us:
+// the columns) or two: where the workgroups are many, and where two would not fit into LDS.  Four against two, us (128 x 128 and 64 x 64 from
+// before they went by blocks):
 //   24 heads of 128 x 128, 128 tokens:  one run 83 against 62, 4 runs 96 against 88, 8 runs 118 against 133; one run beside 63
 //   single tokens 268 against 405;   24 of 64 x 64, 16 runs 82 against 80, one beside 63 104 against 120;   80 of 64 x 128, 4
 //   runs 120 against 135;   16 of 256 x 256, one run of 128 133 against 205 by the kernel that takes every size.
@@ -1241,10 +1245,14 @@ static bool four_columns(int n_seqs, int n_heads, int D, int Dv) {
 // segments 177 with two columns a lane group, 121 with four (LDS serves twice the columns, 140 registers), and 53 for
 // the decays' products, the states and the outputs behind it (100 MB of states and outputs).
 // A cut costs three kernels and the more traffic the more heads and rows; a run saves its chain: `shortest` follows where
-// both are even, in tokens of the longest run (measured with one run, 4, 8 and 16):  24 heads of 128 x 128 at 190, 210, -, -;  4 of them at
+// both are even, in tokens of the longest run (walked; measured with one run, 4, 8 and 16):  24 heads of 128 x 128 at 190, 210, -, -;  4 of them at
 // 172, 175, 192, 200;  24 of 64 x 64 at 165, 180, 200, 300;  8 of 128 x 64 at 172, 185, 190, 210;  32 of 16 x 64 at 148, 160,
 // 150, -.  States of more than 128 rows (no walk with two columns):  16 of 256 x 256 one run of 128 122 us against 133, 4
 // runs of 128 152 against 148 and of 256 257 against 257, 8 runs of 192 323 against 261;  4 of 256 x 128 are cut from 128 on with up to 16.
+// The same rule for states that go by blocks, whose cut costs two kernels and less traffic: us, whole and cut,  24 heads of 128 x 128, one run of 136 53
+// and 49, of 168 62 and 49, of 200 72 and 52, of 2,048 573 and 130;  4 runs of 168 74 and 73, of 2,048 637 and 412;  16 runs of 320 205 and 288 (not cut);
+// 24 of 64 x 64, one run of 168 42 and 34, 4 of 200 54 and 48;  8 of 128 x 64, 16 of 256 82 and 69.  (Both are even earlier than the rule
+// cuts, at 120 tokens for one run, and shorter segments would be faster there: 32 tokens, one run of 136, 40.)
 static Segments segments_of(int n_tokens, int n_seqs, int max_q_len, int n_heads, int D, int Dv, int dtype) {
     const Segments none{0, false};
     const int slices = (Dv + 63) / 64;

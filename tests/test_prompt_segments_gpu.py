@@ -61,8 +61,8 @@ def projected(g, n, H, D, Dv):
 
 # the shortest prompt that is cut and the one just beside it, remainders of a segment from one token on, one token beside
 # them; states of more than 128 rows; enough heads for the long segments; sequences enough for the sparse places of
-# segments; runs that are walked whole with four columns a lane group; tokens enough for decays on the matrix cores and for
-# the finishing kernel's four pairs a wave (its portions are below both); value widths that the cut does not take
+# segments; runs that are walked whole with four columns a lane group; tokens enough for decays on the matrix cores (its
+# portions are below); value widths that the cut does not take
 @pytest.mark.parametrize("op", ["gla", "hgrn", "ssd", "decay", "bonus"])
 @pytest.mark.parametrize("H,D,Dv,lengths,cut", [
     (2, 128, 128, [300, 1, 129, 64, 127], True), (2, 128, 128, [177], True), (2, 128, 128, [176], False),
@@ -87,14 +87,15 @@ def test_a_prompt_cut_into_segments_is_the_prompt_walked_along(op, H, D, Dv, len
     assert float(state[len(lengths):].abs().max()) == 0.0        # nobody else's slot was touched
 
 
-@pytest.mark.parametrize("decay", ["usual", "strong", "mixed"])
+@pytest.mark.parametrize("decay", ["usual", "strong", "mixed", "above", "around"])
 @pytest.mark.parametrize("H,D,Dv,lengths", [
     (2, 64, 64, [32, 1, 15, 16, 17]), (3, 128, 128, [33, 47, 2]), (2, 80, 192, [100, 31, 1]), (1, 112, 80, [48] * 5), (2, 64, 144, [200, 3]),
     (2, 128, 64, [513]), (1, 128, 128, [177, 300]), (1, 64, 272, [65, 50]), (2, 64, 128, [300, 17]),
     (2, 64, 64, [48, 1, 15, 16, 17]), (3, 128, 128, [49, 63, 2])])
 def test_runs_by_blocks_against_64_bits(H, D, Dv, lengths, decay):
     """Whole and cut runs, last blocks of one to 16 tokens, widths that leave waves or channels idle; decays as trained, decays that
-    leave nothing within a block (which go pair by pair), and those in some channels only.  A state's error is that of its decays
+    leave nothing within a block (which go pair by pair), and those in some channels only.  Decays that leave a little more than 2^-40 of a
+    block (the largest k / P there is), or about that, go one way and the other.  A state's error is that of its decays
     (four units in the last place a token) and of some 100 sums, of what the same recurrence gives with absolute values."""
     from simple_inference_amd.kernels import HipKernels
 
@@ -103,7 +104,9 @@ def test_runs_by_blocks_against_64_bits(H, D, Dv, lengths, decay):
     cols = (0, H * D, 2 * H * D, 2 * H * D + H * Dv, 2 * H * (D + Dv))
     rows = rnd(g, n, cols[4] + rank).to(torch.bfloat16).to(DEV)
     a2, bias = rnd(g, H * D, rank, std=0.1).to(torch.bfloat16).to(DEV), rnd(g, H * D, std=0.1).to(DEV)
-    if decay != "usual":
+    if decay in ("above", "around"):      # sixteen sixteenths of log sigmoid: 2^-39 and 2^-40
+        bias = bias * 0.3 - (39 if decay == "above" else 40) * 0.6931
+    elif decay != "usual":
         bias -= 2000.0
     if decay == "mixed":
         bias.view(H, D)[:, :D // 2] += 2000.0
@@ -182,10 +185,10 @@ def test_numbers_without_bounds_reach_no_earlier_token(op, H, D, Dv, lengths):
 
 
 @pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("H,Dv,n", [(1, 8, 3), (3, 24, 33), (5, 64, 51), (2, 136, 40), (3, 256, 7), (2, 512, 129), (3, 20, 33)])
+@pytest.mark.parametrize("H,Dv,n", [(1, 8, 3), (3, 24, 33), (5, 64, 51), (2, 136, 40), (3, 256, 7), (2, 512, 129), (3, 20, 33), (20, 20, 1010)])
 def test_norm_and_gate_behind_a_prompt_s_recurrence(H, Dv, n, shift):
     """Groups of one to 64 lanes a (token, head), lanes without elements, a last workgroup in part, and rows that do not begin at 16
-    bytes (the general form).  With decays and keys that leave the outputs q k v of one channel, each is known to a few
+    bytes or divide into eights (the general form: a (token, head) a wave, and four where there are many).  With decays and keys that leave the outputs q k v of one channel, each is known to a few
     roundings of float; the result is rounded once to bfloat16 (2^-9)."""
     from simple_inference_amd.kernels import HipKernels
 
