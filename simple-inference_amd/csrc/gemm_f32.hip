@@ -781,6 +781,13 @@ static int launch_f32_tiles(const float* X, const float* W, float* Y, u32x4* par
     return launch_f32_shape<BM, BN, WM, WN, D, BN != 256, WIDE>(X, W, Y, parts, slices, M, N, K, false, four, stream);
 }
 
+// The way that this product goes, for tests to tell which they reach: 2 * shape + apart of F32_SHAPES, or -(10 mb + nb) of the few-row kernel.
+SIA_EXPORT int sia_gemm_f32_way(const float* X, const float* W, int M, int N, int K) {
+    const F32Plan plan = f32_plan(M, N, K, wide_rows(X, K), wide_rows(W, K));
+    const FewRows few = few_rows_shape(M, N, K);
+    return plan.shape < 0 ? -(10 * few.mb + few.nb) : 2 * plan.shape + plan.apart;
+}
+
 // Bytes of workspace that this product wants (0: none).
 SIA_EXPORT long long sia_gemm_f32_workspace(const float* X, const float* W, int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;

@@ -549,10 +549,10 @@ def test_library_product_with_candidates_tried_out(hip, shape):
 @pytest.mark.parametrize("bits", [8, 24])
 @pytest.mark.parametrize("N, K", [(1, 4), (15, 31), (97, 129), (1000, 333), (520, 1056), (3072, 260), (8200, 2048), (12290, 192), (33000, 40)])
 def test_float32_products_of_parts(hip, N, K, bits):
-    """Every way the product goes (few rows, tiles, whole k and slices, empty slices too, short last chunks, tiles and columns, rows on 16 bytes or
-    not) against 64 bits, weights of one part and of three, one row of three parts among others of one; a row has the same bits whatever
+    """Few rows and tiles, whole k and slices, empty slices too, short last chunks, tiles and columns, rows on 16 bytes or not, against 64 bits,
+    weights of one part and of three, one row of three parts among others of one; a row has the same bits whatever
     rows are beside it.  A chunk's sum is at most 192 roundings of 2^-24 of sums below sum |x w|, the chunks' and slices' sums
-    K / 32 + 8 more, and what is left out of the parts' products 2^-24 of each."""
+    K / 32 + 8 more, and what is left out of the parts' products 2^-32 of each.  (Far from what the products give; the next test's bound is near.)"""
     w = rnd(N, K, seed=2)
     if bits == 8:
         w = w.bfloat16().float()
@@ -570,6 +570,53 @@ def test_float32_products_of_parts(hip, N, K, bits):
     flat[1:] = w.flatten()
     for M in (5, 40, 303):
         assert torch.equal(hip.linear(x[:M].contiguous(), flat[1:].view(N, K)), all_rows[:M]), M
+
+
+# (rows, columns, k, way):  2 * shape of the tiles + 1 where slices of k are apart, or blocks of rows and columns of the few-row kernel.  Each way of
+# the tiles with one slice, two and eight where there are some, k that is a multiple of four and not; last tiles and chunks in part.
+FLOAT_WAYS = [
+    (65, 32770, 2052, 0), (259, 20002, 2052, 0), (65, 20002, 1028, 1), (259, 2050, 2052, 1),
+    (303, 32770, 260, 2), (40, 32770, 1027, 2), (259, 12290, 260, 2), (193, 14337, 131, 2), (385, 8195, 260, 2), (385, 8195, 131, 2),
+    (303, 16385, 2052, 3), (40, 16385, 2049, 3), (193, 3074, 2052, 3), (65, 4100, 1027, 3),
+    (97, 14337, 1028, 4), (97, 12290, 261, 4), (385, 4100, 260, 4), (385, 4100, 131, 4), (33, 12290, 1027, 5), (40, 3074, 2049, 5),
+    (193, 12290, 64, 6), (17, 12290, 63, 6), (65, 14337, 516, 6), (700, 2050, 260, 6), (259, 2050, 131, 6),
+    (193, 14337, 516, 8), (97, 16385, 517, 8), (513, 4100, 516, 8), (513, 4100, 517, 8), (65, 12290, 2052, 9), (65, 2050, 2049, 9),
+    (8, 32800, 256, -14), (12, 32800, 256, -11), (12, 14337, 131, -11), (5, 130, 260, -11), (20, 32800, 256, -24), (40, 14337, 132, -42),
+    (17, 12290, 132, -22), (17, 12290, 131, -22), (33, 8195, 132, -22), (40, 130, 260, -21), (40, 130, 261, -21)]
+
+
+def test_the_ways_of_float32_products_are_all_tested():
+    """Way 7 is never taken: tiles of 32 x 64 have no slices apart."""
+    assert {way for *_, way in FLOAT_WAYS} == set(range(10)) - {7} | {-11, -14, -21, -22, -24, -42}
+
+
+@pytest.mark.parametrize("M, N, K, way", FLOAT_WAYS)
+def test_float32_products_every_way(hip, M, N, K, way):
+    """The bits of the few-row kernel without a workspace, with weights of one part, of three and of both; a 2-norm error against 64 bits of at most
+    2e-7 (measured up to 9e-8; any of the products above 2^-24 of the whole left out gives 1e-6 and more); rows and columns that
+    are not finite or have no three parts made again like the floats' product, in the last rows and columns too."""
+    assert hip.core.sia_gemm_f32_way(None, None, M, N, K) == way
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    few = torch.empty(M, N, device=DEV)
+
+    def same_as_few(x, w):
+        y = hip.linear(x, w)
+        assert hip.core.sia_gemm_f32(x.data_ptr(), w.data_ptr(), few.data_ptr(), None, M, N, K, hip._stream()) == 0
+        assert torch.equal(torch.nan_to_num(y, nan=1.5), torch.nan_to_num(few, nan=1.5))
+        return y
+
+    for mixed in (False, True):
+        if mixed:
+            w[N // 3:] = w[N // 3:].bfloat16().float()
+        y, want = same_as_few(x, w), x.double() @ w.double().T
+        assert float((y.double() - want).norm() / want.norm()) <= 2e-7
+    x[M - 1, 0], x[M // 2] = float("nan"), x[M // 2] * 2.0 ** -125
+    w[N - 1, K - 1], w[N // 2, 0], w[N // 4] = float("inf"), 3.3999e38, w[N // 4] * 2.0 ** -120
+    y, want = same_as_few(x, w), x.double() @ w.double().T
+    assert torch.equal(y.isnan(), want.isnan()) and bool(y[:M - 1, N - 1].isinf().all())
+    there = want.abs() < 1e38
+    size = torch.nan_to_num(x.double(), nan=0.0).abs() @ torch.nan_to_num(w.double(), posinf=0.0).abs().T
+    assert bool(((y.double() - want).abs() <= (24 + K / 4) * 2.0 ** -24 * size + K * 2.0 ** -149)[there].all())
 
 
 @pytest.mark.parametrize("N, K", [(7, 1), (130, 35), (2050, 1056), (1000, 334), (16388, 2047), (33000, 258)])
@@ -689,15 +736,14 @@ def test_float32_product_has_no_reduced_precision(hip):
     assert y[0, 1].item() - 8.0 == 2.0 ** -12
 
 
-# edges of the tiles (16, 32, 64, 128 columns; 16, 32, 64 rows), of a step of 64 k and of a piece of 16; the one of 50 rows is
-# misaligned.  By the rule's rounds: 16 rows and fewer stream, 17 to 50 and (64, 63) take 32 x 16, (300, 16500) and (129, 8320)
-# 64 x 128, (303, 3070) and (64, 16383) 64 x 64, (40, 4100) 32 x 32
+# edges of blocks of 16 rows and columns, of tiles and of chunks of 32 k; the one of 50 rows is misaligned.  Most go to the few-row
+# kernel, (300, 16500), (129, 8320) and (303, 3070) to tiles; test_float32_products_every_way reaches all of either
 @pytest.mark.parametrize("shape", [(1, 1, 1), (16, 17, 4), (17, 16, 60), (33, 33, 64), (64, 63, 68), (65, 130, 130), (40, 4100, 80),
                                    (129, 8320, 192), (300, 16500, 76), (50, 257, 128), (303, 3070, 76), (64, 16383, 66)])
 def test_float32_product(hip, shape):
-    """Against float64: a result is the sum of four chains of about K / 4 float products, each rounded once or twice, so
-    it errs by at most (K / 4 + 8) times 2^-24 of the sum of the products' sizes; and whichever kernel a number of
-    rows goes to, a row's bits are the same."""
+    """Against float64: a result is the sum of K / 32 chunks, each cut by the matrix cores (2^-23 of it) and rounded when it is added, and of small
+    products with a sum of their own, 2^-8 of that, so it errs by less than (K / 4 + 8) times 2^-24 of the sum of the products' sizes; and
+    whichever kernel a number of rows goes to, a row's bits are the same."""
     M, N, K = shape
     x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
     if shape[0] == 50:
