@@ -1,6 +1,7 @@
 // Y[M, N] = X[M, K] * W[N, K]^T in float: the product of the 32-bit path, on the bfloat16 matrix cores.
 //
-// A float of 24 bits is the sum of three bfloat16 numbers, exactly: x0 = x rounded, x1 = (x - x0) rounded, x2 = x - x0 - x1.
+// A float of 24 bits is the sum of three bfloat16 numbers, exactly (Henry, Tang, Heinecke, "Leveraging the bfloat16 artificial intelligence
+// datatype for higher-precision computations", 2019): x0 = x rounded, x1 = (x - x0) rounded, x2 = x - x0 - x1.
 // (A number under 2^-110 may have a rest below 2^-133, which no bfloat16 number holds: its results are made as those that are not finite,
 // below.)  A product of two parts is exact in float, and all but x2 w2, under 2^-32 of the whole, are summed.  The matrix cores multiply
 // bfloat16 sixteen times as fast as float, so eight products are twice as fast, and weights that are bfloat16 numbers kept in 32
@@ -24,11 +25,12 @@
 // * More rows: X is split into its parts ahead, once, in the order in which the matrix cores read it; tiles of Y, X's parts and W as it
 //   is staged through LDS by loads that pass no registers, W split where it is read.  Two sums a result
 //   are what its registers hold: 128 x 256 outputs, which one sum allowed (303 x 128,256 x 2,048 664 us), would spill.
-// us, v_mfma_f32_16x16x4_f32 -> now, weights of 8 bits and of 24:  303 rows x 128,256 x 2,048 1,464 -> 710 and 1,352, x 16,384 x 2,048 204 -> 110
-// and 191, x 2,048 x 8,192 135 -> 70 and 102, x 3,072 x 2,048 42 -> 37 and 50;  one row x 2,048 x 2,048 8.7 -> 5.9 and 7.4, x 2,048 x 8,192 23.6 -> 14.4
-// and 19.2, x 14,336 x 4,096 51 -> 40 and 42;  64 rows x 2,048 x 2,048 11.9 -> 9 and 11.  Slower: 200 to 1,024 rows of 1,000 x 1,000 (512: 16.6 -> 19.5
-// and 20.6), and with weights of 24 bits 17 to 64 rows of 14,336 to 16,384 columns (17 x 16,384 x 2,048 29.1 -> 30.6, 32 x 14,336 x 4,096 50.7 -> 57.9) and
-// 130 to 1,024 rows of 2,048 to 3,072 (512 x 2,048 x 2,048 42.9 -> 54.5, 303 x 3,072 x 2,048 42.7 -> 49.7).
+// Workspace: the parts, 6 bytes an element of X; where slices are apart their sums, a float a result and slice, 512 MiB at most.
+// us, v_mfma_f32_16x16x4_f32 -> now, weights of 8 bits and of 24:  303 rows x 128,256 x 2,048 1,461 -> 701 and 1,310, x 16,384 x 2,048 203 -> 110
+// and 191, x 2,048 x 8,192 136 -> 64 and 101, x 3,072 x 2,048 42.5 -> 36.9 and 50;  one row x 2,048 x 2,048 8.7 -> 6.1 and 7.3, x 2,048 x 8,192 23.4 -> 15.3
+// and 19.9, x 14,336 x 4,096 50 -> 42 and 42;  64 rows x 2,048 x 2,048 11.6 -> 8.9 and 10.9.  Slower: 200 to 1,024 rows of 1,000 x 1,000 (512: 16.5 -> 19.5
+// and 20.5, 1,024: 25 -> 28 and 41), one row x 128,256 x 2,048 (192 -> 198), and with weights of 24 bits 1 to 96 rows of 14,336 to 16,384 columns (17 x 16,384 x
+// 2,048 28.8 -> 30.8, 32 x 14,336 x 4,096 50.5 -> 57.9) and 130 to 1,024 rows of 2,048 to 3,072 (512 x 2,048 x 2,048 42.7 -> 52.9, 303 x 3,072 x 2,048 42.6 -> 50).
 #include "lds_load.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));

@@ -672,7 +672,8 @@ __global__ __launch_bounds__(256) void segment_outputs_kernel(const bf16_t* __re
         }
 }
 
-// The recurrence by blocks of 16 tokens on the matrix cores, for runs of a prompt in bfloat16.
+// The recurrence by blocks of 16 tokens on the matrix cores, for runs of a prompt in bfloat16: the chunked form of Yang and others, "Gated linear
+// attention transformers with hardware-efficient training" (2023).
 // With P_t the products of a block's decays up to token t, R_s those behind token s and S the state in front of the block:
 //   o_t = (q_t * P_t)^T S + sum_(s <= t) A_ts v_s,   A_ts = sum_d q_td k_sd prod_(s < r <= t) alpha_rd,   S <- diag(P_15) S + sum_s (k_s * R_s) v_s^T
 // A = (q P) (k / P)^T where no channel of 64 has decayed to 2^-40 within the block; else its part of A is made pair by pair on the vector units,
