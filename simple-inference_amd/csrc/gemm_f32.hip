@@ -463,6 +463,27 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
     for (int e = 0; e < PARTS; ++e) at[e * SIA_WAVE] = p[e];
 }
 
+// The results that are not finite of a wave's tile, which its lanes have stored themselves, made again.
+template <int TM, int TN>
+__device__ __forceinline__ void make_again(const float* __restrict__ X, const float* __restrict__ W, float* __restrict__ Y, int M, int N, int K,
+                                           int m_first, int n_first) {
+    const int lane = threadIdx.x % SIA_WAVE, r = lane % 16, g = lane / 16;
+#pragma clang loop unroll(disable)
+    for (int i = 0; i < TM * TN; ++i) {
+        const int m = m_first + i / TN * 16, n = n_first + i % TN * 16;
+        float* at = Y + (size_t)m * N + n;
+        unsigned again = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (m < M && n + e < N && !finite(*(volatile float*)(at + e))) again |= 1u << e;
+        if (!__any(again != 0)) continue;
+        const f32x4 v = float_sums(X + (size_t)min(m, M - 1) * K, W + (size_t)min(n - 4 * g + r, N - 1) * K, K);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (again >> e & 1) at[e] = v[e];
+    }
+}
+
 // A tile of BM rows of W, taken by WM x WN waves.  A ring of D + 1 chunks of both in LDS, asked for D ahead; one
 // barrier a chunk: what is read next has come, what was read last may be overwritten.
 // apart: a workgroup has one slice of K, whose sums go to `slices` ([slice][M][Ns]) for sum_slices_f32_kernel.  Else it has all of K, and
@@ -642,20 +663,178 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
     }
     store(more);
     if (apart || !__any(odd)) return;
-#pragma clang loop unroll(disable)
-    for (int i = 0; i < TM * TN; ++i) {      // a lane's results are what it has stored
-        const int m = m_first + i / TN * 16, n = n_first + i % TN * 16;
-        float* at = Y + (size_t)m * N + n;
-        unsigned again = 0;
+    make_again<TM, TN>(X, W, Y, M, N, K, m_first, n_first);
+}
+
+// Tiles of BM rows of X by BN of W for whole chunks (K a multiple of CHUNK) of rows on 16 bytes: the sums of 160 x 128 and 160 x 192 results, two each,
+// fit, because the parts of W beyond the first are never held for more than 16 rows.  Chunks go by with one part of W until the first that has more; from it on
+// X's parts are read again for every 16 rows of W (the eight products of a block need the time anyway).  Half of the waves bring X, half W,
+// each with a ring of its own, DX and DW chunks ahead: a wave's loads end in order, and X, which L2 holds, would wait for W behind it.
+// Bound by what a compute unit fetches and then reads from LDS, which the matrix cores wait for in part: cycles of a chunk of 160 x 128, each alone: loads
+// 1,800, reads 930, products and sums 1,350, all together 2,560 (1.1 us).  Wider tiles fetch less for a result: 303 rows x 128,256 x 2,048, weights of 8 bits,
+// 677 us in tiles of 64 x 128, 600 in 160 x 128, 573 in 160 x 192 (160 x 256 spills: 830);  x 16,384 x 2,048 117 -> 95 (160 x 128), x 3,072 x 2,048 36 -> 30.6 (160 x 192),
+// x 2,048 x 8,192 65 -> 54, x 2,048 x 2,048 29 -> 26 (160 x 128);  weights of 24 bits 1,270 -> 1,130, 184 -> 160, 48 -> 43, 107 -> 87, 38 -> 34.
+// With the next chunk's first reads in front of the last products of this one nothing changed (600 and 587 us), with four waves of twice the rows and
+// 512 registers 660.
+template <int BM, int BN, int WM, int WN, int DX, int DW>
+__global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tall_kernel(
+    const u32x4* __restrict__ parts, const float* __restrict__ X, const float* __restrict__ W,
+    float* __restrict__ Y, float* __restrict__ slices, int M, int N, int K, int Ns, int n_slices, bool apart, bool four,
+    int tiles_m, int n_tiles, int per_die) {
+    constexpr int WAVES = WM * WN, LOADERS = WAVES / 2, TM = BM / WM / 16, TN = BN / WN / 16;
+    constexpr int XT = BM / 16 * PARTS, WT = BN / 8;                   // KiB of a chunk
+    constexpr int LX = (XT + LOADERS - 1) / LOADERS, LW = WT / LOADERS, LOADS = LX > LW ? LX : LW;      // loads of a wave
+    static_assert(TM * WM * 16 == BM && TN * WN * 16 == BN && LW * LOADERS == WT, "tiles");
+    static_assert(((DX + 1) * XT + (DW + 1) * WT) * LL_TILE <= LL_LDS && (DX - 1) * LX < 64 && (DW - 1) * LW < 64, "LDS, loads on their way");
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    char* const x_ring = lds;
+    char* const w_ring = lds + (DX + 1) * XT * LL_TILE;
+    const int tile = (blockIdx.x % 8) * per_die + blockIdx.x / 8;      // as in gemm_f32_tile_kernel
+    if (tile >= n_tiles) return;
+    const int slice = apart ? (tile / tiles_m) % n_slices : 0;
+    const int m0 = (tile % tiles_m) * BM, n0 = tile / tiles_m / (apart ? n_slices : 1) * BN;
+    const int chunks = K / CHUNK, blocks = (M + 15) / 16;
+    const int lane = threadIdx.x % SIA_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / SIA_WAVE);
+    const int wm = wave % WM, wn = wave / WM, r = lane % 16, g = lane / 16;
+    const int begin = apart ? slice_begin(chunks, slice, n_slices) : 0;
+    const int steps = (apart ? slice_begin(chunks, slice + 1, n_slices) : chunks) - begin;
+
+    const bool brings_x = wave < LOADERS;
+    const int loader = brings_x ? wave : wave - LOADERS;
+    const char* const from = brings_x ? (const char*)(parts + ((size_t)begin * blocks + m0 / 16) * PART_BLOCK)
+                                      : (const char*)(W + (size_t)n0 * K + begin * CHUNK);
+    const size_t step_bytes = brings_x ? (size_t)blocks * (PART_BLOCK * 16) : (size_t)CHUNK * 4;
+    unsigned offset[LOADS];      // KiB of X beyond the tile or the last block repeat the last one, rows of W beyond the last that one (K is below 2^22)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (m < M && n + e < N && !finite(*(volatile float*)(at + e))) again |= 1u << e;
-        if (!__any(again != 0)) continue;
-        const f32x4 v = float_sums(X + (size_t)min(m, M - 1) * K, W + (size_t)min(n - 4 * g + r, N - 1) * K, K);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (again >> e & 1) at[e] = v[e];
+    for (int l = 0; l < LOADS; ++l) {
+        const int kib = min(loader * LX + l, min(XT, (blocks - m0 / 16) * PARTS) - 1), row = (loader * LW + min(l, LW - 1)) * 8 + lane / 8;
+        offset[l] = brings_x ? (unsigned)(kib * SIA_WAVE + lane) * 16
+                             : ((unsigned)(min(n0 + row, N - 1) - n0) * (unsigned)K + ((lane & 7) ^ turn(row & 15)) * 4) * 4;
     }
+    auto request = [&](int s, int slot) {
+        const char* at = from + s * step_bytes;
+        if (brings_x) {
+#pragma unroll
+            for (int l = 0; l < LX; ++l) load_to_lds(at + offset[l], x_ring + (slot * XT + min(loader * LX + l, XT - 1)) * LL_TILE);
+        } else {
+#pragma unroll
+            for (int l = 0; l < LW; ++l) load_to_lds(at + offset[l], w_ring + (slot * WT + loader * LW + l) * LL_TILE);
+        }
+    };
+    f32x4 total[TM][TN], small[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) total[i][j] = small[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < (brings_x ? DX : DW); ++s)
+        if (s < steps) request(s, s);
+    const int x_at = wm * TM * PARTS * LL_TILE + lane * 16, w_at = (wn * (BN / WN) + r) * 128;
+    const int place[2] = {((2 * g) ^ turn(r)) * 16, ((2 * g + 1) ^ turn(r)) * 16};
+    int x_slot = 0, w_slot = 0, s = 0;
+    const char *xs, *ws;
+    // chunk s has come for all waves, and all have read chunk s - 1, whose places are filled again
+    auto arrive = [&]() {
+        if (brings_x)
+            wait_step<LX, DX - 1>(steps - 1 - s);
+        else
+            wait_step<LW, DW - 1>(steps - 1 - s);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (brings_x) {
+            if (s + DX < steps) request(s + DX, x_slot == 0 ? DX : x_slot - 1);
+        } else {
+            if (s + DW < steps) request(s + DW, w_slot == 0 ? DW : w_slot - 1);
+        }
+        xs = x_ring + x_slot * XT * LL_TILE + x_at, ws = w_ring + w_slot * WT * LL_TILE + w_at;
+        x_slot = x_slot == DX ? 0 : x_slot + 1;
+        w_slot = w_slot == DW ? 0 : w_slot + 1;
+    };
+    auto read_w = [&](int j, u32x4& a, u32x4& b) {
+        const char* at = ws + j * 2 * LL_TILE;
+        a = *(const u32x4*)(at + place[0]), b = *(const u32x4*)(at + place[1]);
+    };
+    auto read_x = [&](int i, u32x4 (&x)[PARTS]) {
+#pragma unroll
+        for (int e = 0; e < PARTS; ++e) x[e] = *(const u32x4*)(xs + (i * PARTS + e) * LL_TILE);
+    };
+    u32x4 w[TN], x[2][PARTS];
+    auto multiply = [&](int i, const u32x4 (&xi)[PARTS]) {      // (written out in the loop it spills)
+        f32x4 large[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) large[j] = product(w[j], xi[0], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+        for (int p = PARTS - 1; p > 0; --p)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) small[i][j] = product(w[j], xi[p], small[i][j]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) total[i][j] += large[j];
+    };
+    for (; s < steps; ++s) {      // while W has one part
+        arrive();
+        u32x4 wa[TN], wb[TN];
+        read_x(0, x[0]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) read_w(j, wa[j], wb[j]);
+        uint32_t bits = 0;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            bits |= or_of(wa[j], wb[j]);
+            w[j] = upper_halves(wa[j], wb[j]);
+        }
+        if (__any((bits & 0xffffu) != 0)) break;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            if (i + 1 < TM) read_x(i + 1, x[(i + 1) & 1]);
+            __builtin_amdgcn_sched_barrier(0);      // no more reads ahead than this: they would take the registers of the sums
+            multiply(i, x[i & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    while (s < steps) {      // chunk s has arrived
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            asm volatile("" ::: "memory");      // X's parts are read again, not kept
+            u32x4 a, b, part[1][PARTS];
+            read_w(j, a, b);
+            if (any_rest(split8(a, b, part[0]))) mark_rests(a, b, part[0][PARTS - 1]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                u32x4 xi[PARTS];
+                read_x(i, xi);
+                f32x4 t[1] = {total[i][j]}, q[1] = {small[i][j]};
+                add_chunk(part, xi, true, t, q);
+                total[i][j] = t[0], small[i][j] = q[0];
+            }
+        }
+        if (++s < steps) arrive();
+    }
+    // total[i][j]: row 16 i + r of the wave's tile, columns 16 j + 4 g .. + 3
+    int m_first = m0 + wm * (BM / WM) + r, n_first = n0 + wn * (BN / WN) + 4 * g;
+    asm volatile("" : "+v"(m_first), "+v"(n_first));      // addresses made here, not in front of the loop and kept through it
+    const int stride = apart ? Ns : N;
+    float* const to = apart ? slices + (size_t)slice * M * Ns : Y;
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int m = m_first + i * 16;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = n_first + j * 16;
+            float* at = to + (size_t)m * stride + n;
+            const f32x4 v = total[i][j] + small[i][j];
+            if (four || apart) {
+                if (n < N) *(f32x4*)at = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) at[e] = v[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) odd |= n + e < N && !finite(v[e]);
+        }
+    }
+    if (apart || !__any(odd)) return;
+    make_again<TM, TN>(X, W, Y, M, N, K, m_first, n_first);
 }
 
 // Y = the slices' sums added in order.  A wave has 16 rows and columns, as float_sums gives them, a workgroup 64 columns.
@@ -696,7 +875,9 @@ __global__ __launch_bounds__(256) void sum_slices_f32_kernel(const float* __rest
 // workgroup or its slices apart: a launch, a round of workgroups over the device, a chunk of a round, what each workgroup on a unit
 // adds to that, a MB of the slices' sums written and read (through Y, for tiles of 256 columns).  By least squares over the geometric mean
 // of weights of 8 and 24 bits, 2,900 products of 256 to 128,256 columns, k of 256 to 8,192, 17 to 1,024 rows:  median error 2 to 4 %; the choice
-// is 2.2 % above the best of seven shapes on average, 11 % in one of twenty.
+// is 2.2 % above the best of seven shapes on average, 11 % in one of twenty.  The tall ones (gemm_f32_tall_kernel) by 695 products of the same sizes and of
+// columns to 40,000 (median error 2 to 3 %, one of twenty 10 %): they are the fastest by more than 3 % in 134 of them, up to 1.47 times, from 65 rows on (fewer not
+// measured), and leave the others as they were.
 struct F32Cost {
     double launch, round, step, more, sums;
 };
@@ -709,8 +890,10 @@ static const F32Shape F32_SHAPES[] = {{96, 256, 1, {22.6, 13.1, 1.68, 0, 0.109},
                                       {64, 128, 2, {5.0, 3.2, 0.657, 0.372, 0}, {13.6, -3.9, 0.742, 0.319, 0.305}},
                                       {64, 128, 1, {4.4, 3.2, 0.859, 0, 0}, {11.0, -1.7, 0.891, 0, 0.346}},
                                       {32, 64, 3, {6.8, -0.5, 0.428, 0.127, 0}, NEVER},
-                                      {128, 128, 1, {-0.6, 10.1, 1.241, 0, 0}, {12.6, -2.8, 1.282, 0, 0.338}}};
-constexpr int N_F32_SHAPES = sizeof(F32_SHAPES) / sizeof(F32_SHAPES[0]);
+                                      {128, 128, 1, {-0.6, 10.1, 1.241, 0, 0}, {12.6, -2.8, 1.282, 0, 0.338}},
+                                      {160, 128, 1, {0.8, 5.7, 1.534, 0, 0}, {10.9, 0.8, 1.606, 0, 0.186}},
+                                      {160, 192, 1, {5.2, 6.4, 1.978, 0, 0}, {11.7, 1.0, 2.042, 0, 0.175}}};
+constexpr int N_F32_SHAPES = sizeof(F32_SHAPES) / sizeof(F32_SHAPES[0]), FIRST_TALL = 5;
 
 struct F32Plan {
     int shape;      // -1: the few-row kernel
@@ -733,9 +916,11 @@ static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w) {
     double least = (few.launch + fmax(fetched / few.rate, (double)N * K * 4e-6 / 5.4)) * (wide_x && wide_w ? 1 : 1.6);
     for (int i = 0; i < N_F32_SHAPES; ++i) {
         const F32Shape& t = F32_SHAPES[i];
+        const bool tall = i >= FIRST_TALL;
         if (t.bn == 256 && !wide_w) continue;      // four times the loads' addresses would spill
+        if (tall && (!wide_w || K % CHUNK || M <= 64)) continue;
         const long long tiles = (long long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-        for (int apart = 0; apart <= (n_slices > 1); ++apart) {
+        for (int apart = tall && n_slices > 1; apart <= (n_slices > 1); ++apart) {      // (a tall one has one slice)
             const F32Cost& c = apart ? t.apart : t.whole;
             const long long workgroups = tiles * (apart ? n_slices : 1), room = (long long)cus * t.at_a_time;
             if (workgroups > 1 << 30 || (apart && (long long)n_slices * M * N > 1LL << 27)) continue;
@@ -755,6 +940,16 @@ static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w) {
     return best;
 }
 
+// More LDS than a kernel gets unasked, allowed once per device.
+static int allow_lds(const void* kernel, int bytes, bool (&set)[64]) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return (int)hipGetLastError();
+    if (device >= 0 && device < 64 && set[device]) return 0;
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess && device >= 0 && device < 64) set[device] = true;
+    return (int)e;
+}
+
 template <int BM, int BN, int WM, int WN, int D, bool SLICED, bool WIDE>
 static int launch_f32_shape(const float* X, const float* W, float* Y, u32x4* parts, float* slices, int M, int N, int K,
                             bool apart, bool four, hipStream_t stream) {
@@ -762,14 +957,9 @@ static int launch_f32_shape(const float* X, const float* W, float* Y, u32x4* par
     const int n_slices = slices_of(N, K), tiles_m = (M + BM - 1) / BM;
     const int n_tiles = tiles_m * ((N + BN - 1) / BN) * (apart ? n_slices : 1), per_die = (n_tiles + 7) / 8;
     const auto kernel = gemm_f32_tile_kernel<BM, BN, WM, WN, D, SLICED, WIDE>;
-    static bool set[64];      // more LDS than a kernel gets unasked, allowed once per device
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) return (int)hipGetLastError();
-    if (device < 0 || device >= 64 || !set[device]) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-        if (e != hipSuccess) return (int)e;
-        if (device >= 0 && device < 64) set[device] = true;
-    }
+    static bool set[64];
+    const int status = allow_lds((const void*)kernel, bytes, set);
+    if (status) return status;
     hipLaunchKernelGGL(kernel, dim3(8 * per_die), dim3(WM * WN * SIA_WAVE), bytes, stream, parts, X, W, Y, slices, M, N, K, (N + 3) / 4 * 4,
                        n_slices, apart, four, tiles_m, n_tiles, per_die);
     return SIA_LAUNCH_CHECK();
@@ -781,6 +971,21 @@ static int launch_f32_tiles(const float* X, const float* W, float* Y, u32x4* par
     if (apart || slices_of(N, K) == 1 || BN == 256)      // (registers of the large ones are full)
         return launch_f32_shape<BM, BN, WM, WN, D, false, WIDE>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
     return launch_f32_shape<BM, BN, WM, WN, D, BN != 256, WIDE>(X, W, Y, parts, slices, M, N, K, false, four, stream);
+}
+
+template <int BM, int BN, int DX, int DW>
+static int launch_f32_tall(const float* X, const float* W, float* Y, u32x4* parts, float* slices, int M, int N, int K, bool apart, bool four,
+                           hipStream_t stream) {
+    constexpr int bytes = ((DX + 1) * (BM / 16 * PARTS) + (DW + 1) * (BN / 8)) * LL_TILE;
+    const int n_slices = slices_of(N, K), tiles_m = (M + BM - 1) / BM;
+    const int n_tiles = tiles_m * ((N + BN - 1) / BN) * (apart ? n_slices : 1), per_die = (n_tiles + 7) / 8;
+    const auto kernel = gemm_f32_tall_kernel<BM, BN, 2, 4, DX, DW>;
+    static bool set[64];
+    const int status = allow_lds((const void*)kernel, bytes, set);
+    if (status) return status;
+    hipLaunchKernelGGL(kernel, dim3(8 * per_die), dim3(8 * SIA_WAVE), bytes, stream, parts, X, W, Y, slices, M, N, K, (N + 3) / 4 * 4, n_slices, apart,
+                       four, tiles_m, n_tiles, per_die);
+    return SIA_LAUNCH_CHECK();
 }
 
 // The way that this product goes, for tests to tell which they reach: 2 * shape + apart of F32_SHAPES, or -(10 mb + nb) of the few-row kernel.
@@ -827,6 +1032,8 @@ SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* work
     SHAPE(3, 32, 64, 2, 2, 2);
     SHAPE(4, 128, 128, 2, 4, 2);
 #undef SHAPE
+    if (plan.shape == 5) status = launch_f32_tall<160, 128, 2, 3>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
+    if (plan.shape == 6) status = launch_f32_tall<160, 192, 1, 3>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
     if (status == 0 && apart)
         hipLaunchKernelGGL(sum_slices_f32_kernel, dim3((M + 15) / 16, (N + 63) / 64), dim3(256), 0, stream, slices, X, W, Y, M, N, K, Ns,
                            slices_of(N, K), four);

@@ -619,6 +619,17 @@ def test_float32_products_every_way(hip, M, N, K, way):
     assert bool(((y.double() - want).abs() <= (24 + K / 4) * 2.0 ** -24 * size + K * 2.0 ** -149)[there].all())
 
 
+# Tiles of 160 rows:  whole k and slices of 2 and 8, rows behind a tile and last tiles in part, columns that are no multiple of 4.
+TALL_FLOAT_WAYS = [(129, 50003, 192, 10), (160, 50003, 224, 10), (150, 3074, 2048, 11), (129, 12290, 1024, 11), (160, 14337, 1024, 11),
+                   (129, 32770, 224, 12), (97, 40961, 256, 12), (303, 2050, 2048, 13), (97, 5123, 2048, 13), (129, 16386, 1024, 13)]
+
+
+@pytest.mark.parametrize("M, N, K, way", TALL_FLOAT_WAYS)
+def test_float32_products_in_tall_tiles(hip, M, N, K, way):
+    """As every other way: the few-row kernel's bits, and its bound against 64 bits."""
+    test_float32_products_every_way(hip, M, N, K, way)
+
+
 @pytest.mark.parametrize("N, K", [(7, 1), (130, 35), (2050, 1056), (1000, 334), (16388, 2047), (33000, 258)])
 def test_float32_products_of_rows_that_begin_anywhere(hip, N, K):
     """Either operand, or both, one to three floats behind a multiple of 16 bytes, rows of any length: the bits of operands that are not, and a
