@@ -1,257 +1,291 @@
 // Attention of the 32-bit path over the paged cache, for head sizes up to 128: the arithmetic of the plain kernel
-// (attention_generic.hip), operation for operation, with keys and values that several rows share.
+// (attention_generic.hip), operation for operation, on the float matrix cores.
 //
-// What bounds the plain kernel is its loads: a wave per (token, head) reads every key alone, a lane a key row, and the
-// values 4 bytes in every 64.  Here a workgroup of four waves takes the heads of one key/value head (up to four at a
-// time) of eight consecutive tokens, and brings each chunk of 64 absolute positions into LDS once, 16 bytes a
-// lane in the order of the pages; the next chunk is on its way from memory meanwhile, its pages looked up a chunk
-// earlier.  A token that is its sequence's only one (decode) has a workgroup of its own, and so has every token of a step
-// that leaves the chip room for that.  Everything a row's result is made of (chunks, order of sums, exponentials) is as in the
-// plain kernel, so it depends on the row's own keys only, not on which of the forms it goes through.
-//   303 tokens (three decoded over 200 keys, a prompt of 300), 32 heads of 64 on 8: 240 -> 58 us;  one token over 16,000 keys 3,895 ->
-//   1,365, 64 over 2,048 810 -> 215.
+// v_mfma_f32_16x16x4_f32 adds its four products one after the other, each with one rounding (the bits of four fmaf in order, denormal
+// numbers among them: 640,000 results compared), so that a dot product by it has the plain kernel's bits if the elements come in
+// their order.  What came before gave a lane a key and read queries and weights from LDS for every key, which LDS could not keep up with.
+//
+// A workgroup of four waves takes 16 rows: the heads of one key/value head for some consecutive tokens.  Of a chunk of 64 absolute
+// positions a wave brings 16 keys, of which it makes the scores, and then the values' dimensions that are its own for all 64: nothing is
+// loaded twice, and only the rows' maxima and weights go through LDS, behind a barrier each.  (A wave for 16 rows and a whole chunk
+// needs no barriers, but has four times the chain, which is what a step of few hundred tokens waits for.)
+// A token that is its sequence's only one (decode) has a workgroup of its own.
+// What bounds it is the chain of a chunk: 16 dependent products of 32 cycles a wave each for scores and values (heads of 64), and two barriers, 5,000 cycles
+// in all; 600 and more tokens fill the chip with chains.  us, before (a lane a key) and now: 303 tokens (three decoded over 200 keys, a prompt of 300), 32 heads of 64 on 8
+// 58 -> 17.6, 24 of 128 on 8 107 -> 24;  a prompt of 2,048 960 -> 315 (55 TFLOP/s of 157), 2,160 -> 446;  one token over 16,000 keys 1,347 -> 540;
+// 64 over 2,048 209 -> 116 (537 MB: 4.6 TB/s).
+#include <algorithm>
+
 #include "common.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-#define CHUNK SIA_WAVE      // keys at a time, a lane each
+#define CHUNK SIA_WAVE      // keys at a time
 #define WAVES 4
-#define TOKENS 8            // tokens a workgroup; a wave takes every fourth
-#define TURNS (TOKENS / WAVES)
+#define ROWS 16             // (token, head) pairs of a workgroup
+#define P_ROW (CHUNK + 4)
 
-// DP: 64 or 128, the head sizes' upper bound.  HB: heads a wave takes together.
-// KEEP: with kept first positions; what tells them from the window costs the others 3 to 5 % (one token over 550 keys beside seven
-// more, 32 heads of 64 on 8: 64.8 us with, 61.1 without;  600 tokens 138.7 and 131.0).
-template <int DP, int HB, bool KEEP>
+// Lane (r, g) = 16 g + r holds elements 4 g .. 4 g + 3 of its row; afterwards element e of it is element 4 e + g of the row: the order in which
+// four steps of the matrix instruction take them.  And the other way round.
+__device__ __forceinline__ void across_groups(f32x4& x) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const u32x2 v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[e]), __float_as_uint(x[e + 2]), false, false);
+        x[e] = __uint_as_float(v[0]), x[e + 2] = __uint_as_float(v[1]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+        const u32x2 v = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[e]), __float_as_uint(x[e + 1]), false, false);
+        x[e] = __uint_as_float(v[0]), x[e + 1] = __uint_as_float(v[1]);
+    }
+}
+
+// x of this lane and x of the lane OFF away (16 or 32), one way round or the other
+template <int OFF>
+__device__ __forceinline__ u32x2 beside(float x) {
+    const unsigned u = __float_as_uint(x);
+    return OFF == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false) : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+}
+template <int OFF>
+__device__ __forceinline__ float max_beside(float x) {
+    const u32x2 v = beside<OFF>(x);
+    return fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1]));
+}
+template <int OFF>
+__device__ __forceinline__ float sum_beside(float x) {
+    const u32x2 v = beside<OFF>(x);
+    return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+
+__device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// all waves have come here, and what they have written to LDS is there; loads from memory stay on their way
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// DP: 64 or 128, the head sizes' upper bound.
+template <int DP>
 __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
     const float* __restrict__ q, int q_row_stride, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ seq_of_token,
     const int* __restrict__ positions, float* __restrict__ out, int n_tokens, int n_single, int n_heads, int n_kv,
     int head_dim, int value_dim, int page_size, float scale, int window, int chunk, const float* __restrict__ sinks,
     float cap, int keep_first) {
-    constexpr int K_ROW = DP + 4, V_ROW = CHUNK + 4;      // 16 bytes more than the data: rows begin in other banks
-    constexpr int K_LOADS = CHUNK * DP / 4 / (WAVES * SIA_WAVE), V_LOADS = K_LOADS;
-    extern __shared__ float lds[];
-    float* k_s = lds;                            // [CHUNK][K_ROW]
-    float* v_s = k_s + CHUNK * K_ROW;            // [DP][V_ROW]
-    float* q_s = v_s + DP * V_ROW;               // [TOKENS][HB][DP]
-    float* p_s = q_s + TOKENS * HB * DP;         // [WAVES][HB][CHUNK]
+    constexpr int PIECES = DP / 16, BLOCKS = DP / 64;      // a lane's fours of a row of keys; blocks of 16 dimensions of a wave's values
+    __shared__ float most[WAVES][ROWS];
+    __shared__ __attribute__((aligned(16))) float weight[ROWS * P_ROW];      // [row][position: 16 (j % 4) + j / 4]
 
-    const int tid = threadIdx.x, lane = tid % SIA_WAVE, wave = tid / SIA_WAVE;
-    const int h0 = blockIdx.y * HB, hk = h0 / (n_heads / n_kv);
-    const bool single = (int)blockIdx.x < n_single;
-    int t0 = single ? blockIdx.x : n_single + (blockIdx.x - n_single) * TOKENS;
-    const int t_end = single ? t0 + 1 : min(t0 + TOKENS, n_tokens);
-    const int d4 = head_dim / 4, in_page = page_size - 1, page_log2 = __ffs(page_size) - 1;
-    const int run4 = min(page_size, CHUNK) / 4;  // pieces of four positions that lie together in a page
-    float* p_w = p_s + wave * HB * CHUNK;
+    const int lane = threadIdx.x % SIA_WAVE, wave = threadIdx.x / SIA_WAVE, r = lane % 16, g = lane / 16;
+    const int group = n_heads / n_kv, hk = blockIdx.x % n_kv, page_log2 = __ffs(page_size) - 1, in_page = page_size - 1;
+    // The rows: token * group + head, those of a single token in tiles of their own, which come first; then the others' from the last on, whose
+    // tokens see the most keys.
+    const int tile = blockIdx.x / n_kv, per_single = (group + ROWS - 1) / ROWS, single_tiles = n_single * per_single;
+    long long row0, row_end;
+    if (tile < single_tiles) {
+        row0 = (long long)(tile / per_single) * group + tile % per_single * ROWS;
+        row_end = (long long)(tile / per_single + 1) * group;
+    } else {
+        row_end = (long long)n_tokens * group;
+        row0 = (long long)n_single * group + (long long)((int)(gridDim.x / n_kv) - 1 - tile) * ROWS;
+    }
+    const int n_rows = (int)min((long long)ROWS, row_end - row0);
+    const int token = (int)((row0 + min(r, n_rows - 1)) / group), head = hk * group + (int)((row0 + min(r, n_rows - 1)) % group);
+    const int my_seq = seq_of_token[token], my_pos = positions[token];
+    auto oldest = [&](int pos) {
+        int lo = window > 0 ? max(0, pos - window + 1) : 0;
+        return chunk > 0 ? max(lo, pos - pos % chunk) : lo;
+    };
+    const int my_lo = oldest(my_pos), my_keep = min(keep_first, my_lo);
 
-    // The pieces of four floats that this thread brings in: key and dimension, in the order of a key's row, and
-    // dimension and first position, in the order of a page.  -1: none.
-    int kj[K_LOADS], kd[K_LOADS], vj[V_LOADS], vd[V_LOADS];
+    f32x4 qf[PIECES];
 #pragma unroll
-    for (int i = 0; i < K_LOADS; ++i) {
-        const int at = tid + i * WAVES * SIA_WAVE;
-        kj[i] = at < CHUNK * d4 ? at / d4 : -1;
-        kd[i] = at % d4 * 4;
-        vj[i] = at < CHUNK / 4 * value_dim ? (at / (run4 * value_dim) * run4 + at % run4) * 4 : -1;
-        vd[i] = at / run4 % value_dim;
+    for (int i = 0; i < PIECES; ++i) {
+        const int d = 16 * i + 4 * g;
+        qf[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (d < head_dim) qf[i] = *(const f32x4*)(q + (size_t)token * q_row_stride + head * head_dim + d);
+        across_groups(qf[i]);
     }
 
-    while (t0 < t_end) {      // the tokens of one sequence after those of another
-        const int seq = seq_of_token[t0];
-        int n = 1;
-        while (t0 + n < t_end && seq_of_token[t0 + n] == seq) ++n;
+    float m = -INFINITY, l = 0.f;
+    f32x4 acc[BLOCKS];
+#pragma unroll
+    for (int a = 0; a < BLOCKS; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (int begin = 0; begin < n_rows;) {      // the rows of one sequence after those of another
+        const int seq = __builtin_amdgcn_readlane(my_seq, begin);
+        const unsigned same = (unsigned)(__ballot(r < n_rows && my_seq == seq) & 0xffff) >> begin;
+        const int end = begin + __builtin_ctz(~same);
+        const bool mine = r >= begin && r < end;
         const int* table = block_table + (size_t)seq * table_width;
-        int first = positions[t0], last = first;
-        for (int i = 1; i < n; ++i) {
-            first = min(first, positions[t0 + i]);
-            last = max(last, positions[t0 + i]);
+        int first = mine ? my_pos : 0x7fffffff, last = mine ? my_pos : -1;
+#pragma unroll
+        for (int off = 1; off < 16; off *= 2) {
+            first = min(first, __shfl_xor(first, off, SIA_WAVE));
+            last = max(last, __shfl_xor(last, off, SIA_WAVE));
         }
-        auto oldest = [&](int pos) {
-            int lo = window > 0 ? max(0, pos - window + 1) : 0;
-            return chunk > 0 ? max(lo, pos - pos % chunk) : lo;
-        };
+        first = __builtin_amdgcn_readfirstlane(first), last = __builtin_amdgcn_readfirstlane(last);
         // chunks that some row of the run may see, in order: those of the kept positions, then from the window's on
-        const int lo0 = oldest(first), keep0 = KEEP ? min(keep_first, oldest(last)) : 0, c_lo = lo0 / CHUNK * CHUNK;
-        auto next_chunk = [&](int c0) { return KEEP && c0 + CHUNK < keep0 ? c0 + CHUNK : max(c0 + CHUNK, c_lo); };
+        const int lo0 = oldest(first), lo_last = oldest(last), keep0 = min(keep_first, lo_last), c_lo = lo0 / CHUNK * CHUNK;
+        auto next_chunk = [&](int c0) { return c0 + CHUNK < keep0 ? c0 + CHUNK : max(c0 + CHUNK, c_lo); };
         auto page_of = [&](int c0) {
             const int j = c0 + lane;
             return j <= last && (j >> page_log2) < table_width ? table[j >> page_log2] : -1;
         };
-
-        for (int i = tid; i < n * HB * d4; i += WAVES * SIA_WAVE) {
-            const int row = i / d4, piece = i % d4;
-            *(f32x4*)(q_s + row * DP + piece * 4) =
-                *(const f32x4*)(q + (size_t)(t0 + row / HB) * q_row_stride + (h0 + row % HB) * head_dim + piece * 4);
-        }
-
-        f32x4 kr[K_LOADS], vr[V_LOADS];
-        auto fetch = [&](int c0, int page) {
+        // Keys 16 wave + r of the chunk, and dimensions of the values, four positions at a time.  Where there is no page, or no such
+        // dimension, what is read is not used.
+        f32x4 kr[PIECES], vr[BLOCKS][4];
+        auto fetch_keys = [&](int c0, int page) {
+            const int j = 16 * wave + r, pg = max(__shfl(page, j, SIA_WAVE), 0);
+            const float* at = k_pages + ((((size_t)pg * n_kv + hk) << page_log2) + ((c0 + j) & in_page)) * head_dim;
 #pragma unroll
-            for (int i = 0; i < K_LOADS; ++i) {
-                const int pg = __shfl(page, max(kj[i], 0), SIA_WAVE);
-                kr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (kj[i] >= 0 && pg >= 0)
-                    kr[i] = *(const f32x4*)(k_pages + ((((size_t)pg * n_kv + hk) << page_log2) + ((c0 + kj[i]) & in_page)) * head_dim + kd[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < V_LOADS; ++i) {
-                const int pg = __shfl(page, max(vj[i], 0), SIA_WAVE);
-                vr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (vj[i] >= 0 && pg >= 0)
-                    vr[i] = *(const f32x4*)(v_pages + ((((size_t)pg * n_kv + hk) * value_dim + vd[i]) << page_log2) + ((c0 + vj[i]) & in_page));
+            for (int i = 0; i < PIECES; ++i) {
+                const int d = 16 * i + 4 * g;
+                kr[i] = *(const f32x4*)(at + (d < head_dim ? d : 0));
             }
         };
-        auto put = [&]() {
+        auto fetch_values = [&](int c0, int page) {
 #pragma unroll
-            for (int i = 0; i < K_LOADS; ++i)
-                if (kj[i] >= 0) *(f32x4*)(k_s + kj[i] * K_ROW + kd[i]) = kr[i];
+            for (int b = 0; b < 4; ++b) {
+                const int j = 16 * b + 4 * g, pg = max(__shfl(page, j, SIA_WAVE), 0);
 #pragma unroll
-            for (int i = 0; i < V_LOADS; ++i)
-                if (vj[i] >= 0) *(f32x4*)(v_s + vd[i] * V_ROW + vj[i]) = vr[i];
+                for (int a = 0; a < BLOCKS; ++a) {
+                    const int d = (wave * BLOCKS + a) * 16 + r;
+                    vr[a][b] = *(const f32x4*)(v_pages + ((((size_t)pg * n_kv + hk) * value_dim + (d < value_dim ? d : 0)) << page_log2) +
+                                               ((c0 + j) & in_page));
+                }
+            }
         };
 
-        float m[TURNS][HB], l[TURNS][HB], acc[TURNS][HB][DP / SIA_WAVE];
-#pragma unroll
-        for (int t = 0; t < TURNS; ++t)
-#pragma unroll
-            for (int h = 0; h < HB; ++h) {
-                m[t][h] = -INFINITY;
-                l[t][h] = 0.f;
-#pragma unroll
-                for (int a = 0; a < DP / SIA_WAVE; ++a) acc[t][h][a] = 0.f;
-            }
-
-        int c0 = KEEP && keep0 > 0 ? 0 : c_lo;
+        int c0 = keep0 > 0 ? 0 : c_lo;
         int page = page_of(c0), page_next = page_of(next_chunk(c0));
-        fetch(c0, page);
+        fetch_keys(c0, page);
+        fetch_values(c0, page);
         while (c0 <= last) {
             const int c1 = next_chunk(c0);
-            const bool has_page = page >= 0;
-            __syncthreads();      // the readers of the chunk before are through
-            put();
-            __syncthreads();
-            page = page_next;
-            if (c1 <= last) fetch(c1, page);
-            page_next = page_of(next_chunk(c1));
+            f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};      // of keys 16 wave + 4 g + e, row r
 #pragma unroll
-            for (int t = 0; t < TURNS; ++t) {
-                const int i = wave + t * WAVES;
-                if (i >= n) continue;
-                const int pos = positions[t0 + i], lo = oldest(pos), keep = KEEP ? min(keep_first, lo) : 0;
-                if (c0 > pos || (c0 + CHUNK <= lo && !(KEEP && c0 < keep))) continue;      // no visible key in this chunk
-                const int j = c0 + lane;
-                const bool visible = (j >= lo || (KEEP && j < keep)) && j <= pos && has_page;
-                float s[HB];
+            for (int i = 0; i < PIECES; ++i) {
+                if (16 * i + 4 * g >= head_dim) kr[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                across_groups(kr[i]);
 #pragma unroll
-                for (int h = 0; h < HB; ++h) s[h] = 0.f;
-                const float* q_row = q_s + i * HB * DP;
-                for (int d = 0; d < head_dim; d += 4) {
-                    const f32x4 kk = *(const f32x4*)(k_s + lane * K_ROW + d);
+                for (int e = 0; e < 4; ++e) s = mfma(kr[i][e], qf[i][e], s);
+            }
+            if (c1 <= last) fetch_keys(c1, page_next);
+            const bool has_page = __shfl(page, 16 * wave + 4 * g, SIA_WAVE) >= 0;
+            const bool sees = mine && c0 <= my_pos && (c0 + CHUNK > my_lo || c0 < my_keep);      // a key of this chunk
+            bool visible[4];
+            float x[4];
 #pragma unroll
-                    for (int h = 0; h < HB; ++h) {
-                        const f32x4 qq = *(const f32x4*)(q_row + h * DP + d);
+            for (int e = 0; e < 4; ++e) {
+                const int j = c0 + 16 * wave + 4 * g + e;
+                visible[e] = mine && (j >= my_lo || j < my_keep) && j <= my_pos && has_page;
+                x[e] = s[e] * scale;
+                if (cap > 0.f) x[e] = cap * tanhf(x[e] / cap);
+                if (!visible[e]) x[e] = -INFINITY;
+            }
+            float top = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+            top = max_beside<32>(max_beside<16>(top));
+            if (g == 0) most[wave][r] = top;
+            lds_barrier();
+            const float m_new = fmaxf(m, fmaxf(fmaxf(most[0][r], most[1][r]), fmaxf(most[2][r], most[3][r])));
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) s[h] += qq[e] * kk[e];
-                    }
-                }
+            for (int e = 0; e < 4; ++e) weight[r * P_ROW + e * 16 + wave * 4 + g] = visible[e] ? expf(x[e] - m_new) : 0.f;
+            const float alpha = sees ? expf(m - m_new) : 1.f;
+            m = m_new;
+            lds_barrier();
+            f32x4 p[4];      // element e of p[b]: position 16 b + 4 e + g
 #pragma unroll
-                for (int h = 0; h < HB; ++h) {
-                    float x = s[h] * scale;
-                    if (cap > 0.f) x = cap * tanhf(x / cap);
-                    if (!visible) x = -INFINITY;
-                    const float m_new = fmaxf(m[t][h], wave_max(x));
-                    const float p = visible ? expf(x - m_new) : 0.f;
-                    const float alpha = expf(m[t][h] - m_new);
-                    l[t][h] = l[t][h] * alpha + wave_sum(p);
-                    m[t][h] = m_new;
+            for (int b = 0; b < 4; ++b) p[b] = *(const f32x4*)(weight + r * P_ROW + g * 16 + b * 4);
+            const f32x4 pair = (p[0] + p[2]) + (p[1] + p[3]);      // the order of a wave's sum over 64 positions
+            const float sum = sum_beside<16>(sum_beside<32>((pair[0] + pair[2]) + (pair[1] + pair[3])));
+            if (sees) l = l * alpha + sum;
 #pragma unroll
-                    for (int a = 0; a < DP / SIA_WAVE; ++a) acc[t][h][a] *= alpha;
-                    p_w[h * CHUNK + lane] = p;
-                }
-                __builtin_amdgcn_wave_barrier();      // the wave's LDS accesses run in order: no more than that is needed
-                // values of keys that the row does not see may be anything: they are left out, not weighted with 0.  In a
-                // chunk with kept positions the loop is run for those, and again for what the window holds of the chunk.
-                const int j_last = min(pos, c0 + CHUNK - 1) - c0;
-                const bool kept = KEEP && c0 < keep;
-                int j_from = kept ? 0 : max(lo, c0) - c0, j_to = kept ? min(keep, c0 + CHUNK) - 1 - c0 : j_last;
-                for (;;) {
-                    for (int jj = j_from & ~3; jj <= j_to; jj += 4) {
-                        const bool whole = jj >= j_from && jj + 3 <= j_to;
-                        f32x4 pp[HB];
+            for (int a = 0; a < BLOCKS; ++a) acc[a] *= alpha;
+            // Values of keys that a row does not see may be anything: where they are finite a weight of 0 leaves them out.  Those that no
+            // row of the run sees are replaced; if one of the others is not finite, every row gets its own values.
+            bool apart = false;
+            if (c0 + CHUNK - 1 > first || c0 < lo_last || end - begin < n_rows || __any(page < 0)) {
 #pragma unroll
-                        for (int h = 0; h < HB; ++h) pp[h] = *(const f32x4*)(p_w + h * CHUNK + jj);
+                for (int b = 0; b < 4; ++b) {
+                    const int j = c0 + 16 * b + 4 * g;
+                    const bool there = __shfl(page, 16 * b + 4 * g, SIA_WAVE) >= 0;
 #pragma unroll
-                        for (int a = 0; a < DP / SIA_WAVE; ++a) {
-                            f32x4 vv = *(const f32x4*)(v_s + (lane + a * SIA_WAVE) * V_ROW + jj);
-                            if (!whole)
+                    for (int e = 0; e < 4; ++e) {
+                        const bool seen = there && j + e <= last && (j + e >= lo0 || j + e < keep0);
 #pragma unroll
-                                for (int e = 0; e < 4; ++e)
-                                    if (jj + e < j_from || jj + e > j_to) vv[e] = 0.f;
-#pragma unroll
-                            for (int h = 0; h < HB; ++h)
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) acc[t][h][a] += pp[h][e] * vv[e];
+                        for (int a = 0; a < BLOCKS; ++a) {
+                            vr[a][b][e] = seen ? vr[a][b][e] : 0.f;
+                            apart |= !__builtin_isfinite(vr[a][b][e]);
                         }
                     }
-                    if (!KEEP || j_to >= j_last) break;
-                    j_from = max(lo - c0, j_to + 1);
-                    j_to = j_last;
+                }
+                apart = __any(apart);
+            }
+#pragma unroll
+            for (int a = 0; a < BLOCKS; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) across_groups(vr[a][b]);
+            if (!apart) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int a = 0; a < BLOCKS; ++a) acc[a] = mfma(vr[a][b][e], p[b][e], acc[a]);
+            } else {
+#pragma clang loop unroll(disable)
+                for (int row = begin; row < end; ++row) {
+                    const int pos = __builtin_amdgcn_readlane(my_pos, row), lo = __builtin_amdgcn_readlane(my_lo, row);
+                    const int keep = min(keep_first, lo);
+#pragma unroll
+                    for (int a = 0; a < BLOCKS; ++a) {
+                        f32x4 own = acc[a];
+#pragma unroll
+                        for (int b = 0; b < 4; ++b)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const int j = c0 + 16 * b + 4 * e + g;
+                                own = mfma(j <= pos && (j >= lo || j < keep) ? vr[a][b][e] : 0.f, p[b][e], own);
+                            }
+                        if (r == row) acc[a] = own;
+                    }
                 }
             }
+            page = page_next;
+            if (c1 <= last) fetch_values(c1, page);
+            page_next = page_of(next_chunk(c1));
             c0 = c1;
         }
+        begin = end;
+    }
+    if (r >= n_rows) return;
+    if (sinks) l += expf(sinks[head] - m);
+    const float inv = 1.f / l;
+    float* o = out + ((size_t)token * n_heads + head) * value_dim;
 #pragma unroll
-        for (int t = 0; t < TURNS; ++t) {
-            const int i = wave + t * WAVES;
-            if (i >= n) continue;
+    for (int a = 0; a < BLOCKS; ++a) {
+        const int d = (wave * BLOCKS + a) * 16 + 4 * g;
+        if (value_dim % 4 == 0) {
+            if (d < value_dim) *(f32x4*)(o + d) = acc[a] * inv;
+        } else {
 #pragma unroll
-            for (int h = 0; h < HB; ++h) {
-                float sum = l[t][h];
-                if (sinks) sum += expf(sinks[h0 + h] - m[t][h]);
-                const float inv = 1.f / sum;
-                float* o = out + ((size_t)(t0 + i) * n_heads + h0 + h) * value_dim;
-#pragma unroll
-                for (int a = 0; a < DP / SIA_WAVE; ++a)
-                    if (lane + a * SIA_WAVE < value_dim) o[lane + a * SIA_WAVE] = acc[t][h][a] * inv;
-            }
+            for (int e = 0; e < 4; ++e)
+                if (d + e < value_dim) o[d + e] = acc[a][e] * inv;
         }
-        __syncthreads();      // before the next sequence's queries
-        t0 += n;
     }
 }
 
-template <int DP, int HB>
+template <int DP>
 static int launch(const float* q, int q_row_stride, const float* k_pages, const float* v_pages, const int* block_table,
                   int table_width, const int* seq_of_token, const int* positions, float* out, int n_tokens, int n_single,
-                  int n_seqs, int max_kv, int max_run_kv, int n_heads, int n_kv, int head_dim, int value_dim, int page_size, float scale,
+                  int n_heads, int n_kv, int head_dim, int value_dim, int page_size, float scale,
                   int window, int chunk, const float* sinks, float cap, int keep_first, hipStream_t stream) {
-    constexpr int bytes = (CHUNK * (DP + 4) + DP * (CHUNK + 4) + TOKENS * HB * DP + WAVES * HB * CHUNK) * (int)sizeof(float);
-    // Eight tokens a workgroup share what is loaded, but follow one another in a wave, and their sequences one another in the
-    // workgroup: a token each where one round of two workgroups a unit (one, if LDS holds no more) takes them all, or, if an eight
-    // holds several sequences, three rounds for four of them.  32 heads of 64 on 8, us, the plain kernel, eight, one:  8 tokens over 72 keys
-    // 20, 25, 14.5;  16 over 216 53, 49, 27;  64 over 264 87, 59, 36;  128 over 328 182, 71, 80 (two rounds);  24 heads of
-    // 128 on 8, 16 sequences of 3 over 300 (two rounds) 164, 170, 90.  Where single tokens see more keys than the others do, the step
-    // takes as long as theirs, which a second workgroup on the unit makes longer: 45 tokens beside six over up to 145 keys 19.0 eight, 20.3 one;
-    // 60 beside three over up to 234 24.9 and 25.5;  with the others' keys more, 45 beside one over 30 15.2 and 9.6.
-    const long long many = n_tokens - n_single, runs = n_seqs - n_single;
-    const long long at_once = 256 * (n_single > 0 && max_run_kv < max_kv ? 1 : min(2, 160 * 1024 / bytes));
-    if (many > 0 && 4 * many * n_tokens * (n_heads / HB) <= at_once * max(4 * many, 3 * TOKENS * runs)) n_single = n_tokens;
-    const dim3 grid(n_single + (n_tokens - n_single + TOKENS - 1) / TOKENS, n_heads / HB);
-    const bool keeps = keep_first > 0;
-    auto kernel = keeps ? attention_f32_kernel<DP, HB, true> : attention_f32_kernel<DP, HB, false>;
-    static bool set[64][2] = {};      // more LDS than a kernel gets unasked, allowed once per device
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) return (int)hipGetLastError();
-    if (device < 0 || device >= 64 || !set[device][keeps]) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-        if (e != hipSuccess) return (int)e;
-        if (device >= 0 && device < 64) set[device][keeps] = true;
-    }
-    hipLaunchKernelGGL(kernel, grid, dim3(WAVES * SIA_WAVE), bytes, stream, q, q_row_stride, k_pages, v_pages, block_table,
-                       table_width, seq_of_token, positions, out, n_tokens, n_single, n_heads, n_kv, head_dim, value_dim,
-                       page_size, scale, window, chunk, sinks, cap, keep_first);
+    const long long group = n_heads / n_kv;
+    const long long tiles = n_single * ((group + ROWS - 1) / ROWS) + ((n_tokens - n_single) * group + ROWS - 1) / ROWS;
+    if (tiles * n_kv > 0x7fffffff) return SIA_BAD_ARGUMENT;
+    hipLaunchKernelGGL(attention_f32_kernel<DP>, dim3((unsigned)(tiles * n_kv)), dim3(WAVES * SIA_WAVE), 0, stream, q, q_row_stride, k_pages,
+                       v_pages, block_table, table_width, seq_of_token, positions, out, n_tokens, n_single, n_heads, n_kv, head_dim,
+                       value_dim, page_size, scale, window, chunk, sinks, cap, keep_first);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -259,13 +293,13 @@ extern "C" int sia_attention_generic(const void*, int, const void*, const void*,
                                      int, int, int, int, int, int, float, int, int, const float*, float, int, int, hipStream_t);
 
 // The arguments of the plain kernel, and n_single: that many tokens, the first ones, are their sequences' only ones; n_seqs;
-// max_kv: no sequence holds more keys, max_run_kv: nor does one of more than a token (max_kv if that is not known).
-// Rows of other sizes, and rows and pages that do not lie in sixteens of bytes, go to the plain kernel; so do steps whose sequences hold so few keys that bringing them into LDS first takes longer than a wave a row and head
-// does, as long as those waves find room:  32 heads of 64 on 8, plain against this, us:  one token over 4 keys 6.1 / 8.2, 16: 7.4 / 8.6, 40:
-// 12.1 / 9.4, 16 tokens over 16 7.4 / 14.5;  24 heads of 128 on 8:  4: 6.6 / 10.4, 16: 11.3 / 10.9, 64 sequences over 16 13.4 / 20.8.
+// max_kv: no sequence holds more keys.
+// Rows of other sizes, and rows and pages that do not lie in sixteens of bytes, go to the plain kernel; so do steps whose sequences hold so few keys
+// that one of its waves is through before this kernel's barriers are, as long as those waves find room:  32 heads of 64 on 8, plain against this, us:
+// one token over 4 keys 5.2 / 7.0, 17: 7.3 / 7.0, 45 tokens over 45 14.5 / 7.1;  24 heads of 128 on 8:  4: 6.5 / 8.9, 17: 11.6 / 8.9.
 SIA_EXPORT int sia_attention_f32(const float* q, int q_row_stride, const float* k_pages, const float* v_pages,
                                  const int* block_table, int table_width, const int* seq_of_token, const int* positions,
-                                 float* out, int n_tokens, int n_single, int n_seqs, int max_kv, int max_run_kv, int n_heads, int n_kv,
+                                 float* out, int n_tokens, int n_single, int n_seqs, int max_kv, int n_heads, int n_kv,
                                  int head_dim, int value_dim, int page_size, float scale, int window, int chunk, const float* sinks, float cap,
                                  int keep_first, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
@@ -279,15 +313,16 @@ SIA_EXPORT int sia_attention_f32(const float* q, int q_row_stride, const float* 
                                      n_tokens, n_heads, n_kv, head_dim, value_dim, page_size, scale, window, chunk, sinks,
                                      cap, keep_first, SIA_F32, stream);
     n_single = min(n_single, n_tokens);
-    const int group = n_heads / n_kv;
-    auto run = [&](auto narrow, auto wide) {
-        return (head_dim <= 64 && value_dim <= 64 ? narrow : wide)(
-            q, q_row_stride, k_pages, v_pages, block_table, table_width, seq_of_token, positions, out, n_tokens, n_single,
-            n_seqs, max_kv, max_run_kv, n_heads, n_kv, head_dim, value_dim, page_size, scale, window, chunk, sinks, cap, keep_first,
-            stream);
-    };
-    if (group % 4 == 0) return run(launch<64, 4>, launch<128, 4>);
-    if (group % 3 == 0) return run(launch<64, 3>, launch<128, 3>);
-    if (group % 2 == 0) return run(launch<64, 2>, launch<128, 2>);
-    return run(launch<64, 1>, launch<128, 1>);
+    // A workgroup whose 16 rows belong to several sequences takes one after the other: where runs are short, a workgroup for every token instead, if the
+    // chip has room (two or three workgroups a unit take little longer than one).  16 sequences of 3 tokens over 300 keys, us, together and a token each:
+    // 16 heads of 64 on 16 98 / 25.5, 32 on 8 33 / 19.8, 24 of 128 on 8 68 / 30.
+    const long long per_token = (n_heads / n_kv + ROWS - 1) / ROWS, many = n_tokens - n_single, runs = n_seqs - n_single;
+    if (runs > 1) {
+        const double spans = 1.0 + (double)(runs - 1) * ROWS / ((double)many * (n_heads / n_kv));
+        const double together = spans * std::max(640.0, (double)many * n_heads / ROWS), alone = std::max(640.0, (double)many * per_token * n_kv);
+        if (5 * alone <= 4 * together) n_single = n_tokens;
+    }
+    return (head_dim <= 64 && value_dim <= 64 ? launch<64> : launch<128>)(
+        q, q_row_stride, k_pages, v_pages, block_table, table_width, seq_of_token, positions, out, n_tokens, n_single, n_heads, n_kv,
+        head_dim, value_dim, page_size, scale, window, chunk, sinks, cap, keep_first, stream);
 }

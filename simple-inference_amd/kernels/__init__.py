@@ -105,7 +105,7 @@ _SIGNATURES = {
                               _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int, _c_ptr, _c_float,
                               _c_int, _c_int, _c_ptr],
     "sia_attention_f32": [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr,
-                          _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int,
+                          _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int,
                           _c_ptr, _c_float, _c_int, _c_ptr],
     "sia_attention_max_head_dim": [],
     "sia_attention_generic_max_head_dim": [],
@@ -1928,7 +1928,7 @@ class HipKernels:
             self._check(self.core.sia_attention_f32(
                 _ptr(qkv), width, _ptr(cache.k_pages), _ptr(cache.v_pages), _ptr(cache.block_table),
                 cache.block_table.shape[1], _ptr(ctx.seq_of_token), _ptr(ctx.positions), _ptr(out), n, ctx.n_decode_seqs,
-                ctx.n_seqs, max_kv, int(getattr(ctx, "max_run_kv_len", 0) or max_kv), n_heads, n_kv_heads, head_dim, value_dim, page,
+                ctx.n_seqs, max_kv, n_heads, n_kv_heads, head_dim, value_dim, page,
                 float(scale), int(window or 0), int(chunk or 0), _ptr(sinks), float(softcap or 0.0), int(keep_first), self._stream()),
                 "attention_f32")
             return out

@@ -1050,6 +1050,33 @@ def test_float32_attention_has_the_same_bits_whichever_way_it_goes(hip, n_heads,
     assert rc == 0 and torch.equal(out, plain)
 
 
+# 16 rows that are several sequences' (two, six and sixteen of them), a part of one token's heads, and tokens that have workgroups of their own
+@pytest.mark.parametrize("n_heads,n_kv,D,Dv", [(8, 8, 64, 64), (12, 4, 20, 36), (40, 2, 128, 100), (17, 1, 64, 64)])
+@pytest.mark.parametrize("q_lens", [[1, 1, 30, 2, 1, 1, 70], [2] * 40, [3] * 400])
+def test_float32_attention_keeps_sequences_apart(hip, n_heads, n_kv, D, Dv, q_lens):
+    """Sequences that share a workgroup's rows: a value that is not finite reaches its own sequence's later rows only."""
+    kv_lens, ps = [q + 64 * (i % 3) + i % 5 for i, q in enumerate(q_lens)], 16
+    ctx = Ctx(q_lens, kv_lens)
+    cache = Cache(sum(-(-kv // ps) for kv in kv_lens), n_kv, ps, D, torch.float32, kv_lens, seed=3)
+    cache.k_pages.copy_(rnd(*cache.k_pages.shape, seed=4))
+    cache.v_pages = rnd(cache.v_pages.shape[0], n_kv, Dv, ps, seed=5)
+    qkv = rnd(ctx.n_tokens, (n_heads + n_kv) * D, seed=6)
+    attend = lambda: hip.paged_attention(qkv, n_heads, n_kv, D, 0.3, None, ctx, cache, value_dim=Dv)
+    whole = attend()
+    plain = torch.empty_like(whole)
+    for seq in (None, 2):
+        if seq is not None:      # the first key that the sequence's last row alone sees
+            at, j = sum(q_lens[:seq + 1]) - 1, kv_lens[seq] - 1
+            cache.v_pages[cache.block_table[seq, j // ps], :, :, j % ps] = float("nan")
+        got = attend()
+        rc = hip.core.sia_attention_generic(
+            qkv.data_ptr(), qkv.shape[1], cache.k_pages.data_ptr(), cache.v_pages.data_ptr(), cache.block_table.data_ptr(),
+            cache.block_table.shape[1], ctx.seq_of_token.data_ptr(), ctx.positions.data_ptr(), plain.data_ptr(), ctx.n_tokens, n_heads,
+            n_kv, D, Dv, ps, 0.3, 0, 0, None, 0.0, 0, 0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and torch.equal(got.isnan(), plain.isnan()) and torch.equal(got.nan_to_num(7.0), plain.nan_to_num(7.0)), seq
+    assert bool(got[at].isnan().all()) and torch.equal(got[:at], whole[:at]) and torch.equal(got[at + 1:], whole[at + 1:])
+
+
 # kept positions that end inside a four, at its end, and in the second and third chunk of keys
 @pytest.mark.parametrize("keep", [3, 4, 61, 64, 130])
 def test_float32_attention_leaves_out_values_between_the_kept_positions_and_the_window(hip, keep):
