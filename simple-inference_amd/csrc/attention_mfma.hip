@@ -812,8 +812,11 @@ __device__ __forceinline__ void compute_from_lds(const bf16_t* __restrict__ k_ld
 // every KSPLIT-th tile of keys: ROWS = PF_NQ * 16 * PF_WAVES / KSPLIT tokens per workgroup.  KTILES tiles of keys
 // are staged per step (and barrier); with KSPLIT = 1 every wave takes them one after the other, which at 8 waves
 // of 16 tokens is 7 % faster with two tiles than with one (fewer barriers a key) and changes no bit.
+// At least two waves a SIMD, so 256 registers: left to itself the compiler gives the wide shape 316 of heads of 128, and a compute unit then
+// holds one of its workgroups of four waves and not two (4,096 tokens, 24 heads of 128: 245 us, now 133; 7,001, 32 of 64: 357, now 271).
+constexpr int PF_MIN_WAVES = HD <= 128 ? 2 : 1;
 template <int PF_NQ, int PF_WAVES, int KSPLIT, int KTILES>
-__global__ __launch_bounds__(PF_WAVES* SIA_WAVE) void attn_prefill_kernel(
+__global__ __launch_bounds__(PF_WAVES* SIA_WAVE, PF_MIN_WAVES) void attn_prefill_kernel(
     const bf16_t* __restrict__ q, int q_row_stride, const bf16_t* __restrict__ kp, const bf16_t* __restrict__ vp,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ cu_q,
     const int* __restrict__ kv_len, bf16_t* __restrict__ out, int n_heads, int n_kv, int ps_log2, float scale,
@@ -1247,12 +1250,15 @@ static int launch_prefill(int tiles, const void* q, int q_row_stride, const void
 enum PrefillShape { PF_SPLIT, PF_PAIRED, PF_WIDE, PF_LONG };
 static PrefillShape prefill_shape(int n_tiles, int n_tiles_split, int n_tiles_long, int n_heads, int q_bound,
                                   int kv_bound) {
-    // Measured at 24 heads of 128 on 256 compute units.  For a prompt from its start, whose row tiles see from few
+    // Measured on 256 compute units.  For a prompt from its start, whose row tiles see from few
     // keys to all, the fastest shape follows the number of workgroups per compute unit: the split shape while all
     // its workgroups are on the chip at once (up to 6/8 of a wide workgroup per compute unit: prompts up to about
-    // 1,000 tokens), the paired shape of 128 tokens (two tiles of keys a step, one for each set of waves) up to 15/8
-    // (about 2,500 tokens), the wide shape (one tile a step) beyond, and from 36/8 on (about 6,000 tokens) 8 waves
-    // of 32 tokens (256 tokens a workgroup, two tiles a step: a tile staged in LDS then serves twice as many tokens).
+    // 1,000 tokens of 24 heads), the paired shape of 128 tokens (two tiles of keys a step, one for each set of waves) up to 18/8
+    // (about 3,000 tokens), the wide shape (one tile a step, two workgroups a unit) beyond, and for heads of more than 64 from 30/8 on (about 5,000
+    // tokens) 8 waves of 32 tokens (256 tokens a workgroup, two tiles a step: a tile staged in LDS then serves twice as many tokens).
+    // us, paired, wide, long, by wide workgroups a unit:  heads of 128:  1.5 51 68 76;  2.0 60 70 77 and 76 95 93;  2.3 108 105 110;  2.6 102 99 96;
+    // 3.0 159 133 145;  3.1 134 112 111;  3.8 235 223 209;  4.0 195 184 162;  5.1 412 360 374, 310 276 280;  6.9 535 475 457.
+    // heads of 64:  2.0 43 48 55;  2.6 75 74 73;  3.1 98 74 80;  4.0 145 104 114;  5.1 237 166 202;  6.9 406 271 330.
     const long long wide_groups = (long long)n_tiles * n_heads, cus = compute_units();
     const bool split_fits = n_tiles_split > 0 && wide_groups * 8 <= cus * 6;
     // A portion over a past is another matter: every row tile sees about as many keys, so the launch lasts as many
@@ -1268,8 +1274,8 @@ static PrefillShape prefill_shape(int n_tiles, int n_tiles_split, int n_tiles_lo
         return lng <= wide && lng <= paired ? PF_LONG : wide <= paired ? PF_WIDE : PF_PAIRED;
     }
     if (split_fits) return PF_SPLIT;
-    if (wide_groups * 8 <= cus * 15) return PF_PAIRED;
-    if (n_tiles_long > 0 && wide_groups * 8 >= cus * 36) return PF_LONG;
+    if (wide_groups * 8 <= cus * 18) return PF_PAIRED;
+    if (HD > 64 && n_tiles_long > 0 && wide_groups * 8 >= cus * 30) return PF_LONG;
     return PF_WIDE;
 }
 
