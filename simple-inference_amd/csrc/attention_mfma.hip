@@ -603,11 +603,59 @@ __global__ __launch_bounds__(DEC_WAVES* SIA_WAVE) void attn_decode_kernel(
 
 // Combines what workgroups of their own left in the workspaces for each (sequence, head): the splits' merged states
 // (ws_acc [..][split][HD], ws_ml [..][split][2]), or with `runs` the states of all runs (ws_acc [..][run][HD + 2]).
-__global__ __launch_bounds__(SIA_WAVE) void attn_decode_combine_kernel(
+// A thread an element.  What bounds it is latency: the splits' states come from other dies, and every load that waits for another
+// costs a trip to memory, so all of them go out before the first is used.  (The maxima first, by a lane a split, then four
+// splits' states after four for two elements a thread, one after the other:  what the launch adds, us, 8 rows of 24 heads of
+// 128 with 4 splits 3.4 -> 2.0, 27 of 32 of 64, most with one, 2.6 -> 1.8, 3 of 32 of 128 with up to 32 8.0 -> 4.3.)
+constexpr int COMBINE_THREADS = (HD + SIA_WAVE - 1) / SIA_WAVE * SIA_WAVE;
+
+// The states of the first N splits, beyond `last` that one again.
+template <int N>
+__device__ __forceinline__ void load_states(int last, const float* __restrict__ acc_at, const float2* __restrict__ ml, float (&acc)[N],
+                                            float2 (&state)[N]) {
+#pragma unroll
+    for (int s = 0; s < N; ++s) acc[s] = acc_at[(size_t)min(s, last) * HD];
+#pragma unroll
+    for (int s = 0; s < N; ++s) state[s] = ml[min(s, last)];
+}
+
+// merge_splits for one element of up to N splits, with its order of sums.  What is held of splits beyond n_splits may be anything.
+template <int N>
+__device__ __forceinline__ float combine_states(int n_splits, const float (&acc)[N], const float2 (&state)[N], const float* __restrict__ sinks,
+                                                int head) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < N; ++s) mx = s < n_splits ? fmaxf(mx, state[s].x) : mx;
+    float o = 0.f, denom = sink_term(sinks, head, mx);
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+        const float w = fast_exp2(state[s].x - mx), d = __builtin_fmaf(w, state[s].y, denom), a = __builtin_fmaf(w, acc[s], o);
+        denom = s < n_splits ? d : denom;
+        o = s < n_splits ? a : o;
+    }
+    return o * (1.f / denom);
+}
+template <int N>
+__device__ __forceinline__ float combine_all(int n_splits, const float* __restrict__ acc_at, const float2* __restrict__ ml,
+                                             const float* __restrict__ sinks, int head) {
+    float acc[N];
+    float2 state[N];
+    load_states(n_splits - 1, acc_at, ml, acc, state);
+    return combine_states(n_splits, acc, state, sinks, head);
+}
+
+__global__ __launch_bounds__(COMBINE_THREADS) void attn_decode_combine_kernel(
     const float* __restrict__ ws_acc, const float* __restrict__ ws_ml, const int* __restrict__ cu_q,
     const int* __restrict__ kv_len, bf16_t* __restrict__ out, int n_heads, int max_splits, int window, int chunk,
     const float* __restrict__ sinks, int runs, int ps_log2, const Forms forms) {
-    const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x;
+    const int head = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x % SIA_WAVE, d = min((int)threadIdx.x, HD - 1);
+    const size_t base = ((size_t)seq * n_heads + head) * max_splits;
+    const float* const acc_at = ws_acc + base * HD + d;
+    const float2* const ml = reinterpret_cast<const float2*>(ws_ml) + base;
+    constexpr int FIRST = 4;
+    float acc[FIRST];
+    float2 state[FIRST];
+    if (!runs) load_states(min(FIRST, max_splits) - 1, acc_at, ml, acc, state);      // on their way while the number of splits is worked out
     const int last_pos = kv_len[seq] - 1, oldest = first_visible(last_pos, window, chunk);
     const Places places = places_of(oldest, forms.keep_first, ps_log2);
     const int pos = last_pos - places.gap;
@@ -620,7 +668,7 @@ __global__ __launch_bounds__(SIA_WAVE) void attn_decode_combine_kernel(
         float mx = -INFINITY;  // a lane a run: the loads go out together
         for (int run = lane; run < n_splits * DEC_WAVES; run += SIA_WAVE) mx = fmaxf(mx, mine[(size_t)run * ROW + HD]);
         mx = wave_max(mx);
-        for (int d = lane; d < HD; d += SIA_WAVE)
+        for (int d = threadIdx.x; d < HD; d += COMBINE_THREADS)
             dst[d] = float_to_bf16(merge_splits(n_splits, mx, sink_term(sinks, head, mx),
                                                 [&](int sp, float& acc, float& m, float& l) {
                 merge_waves([&](int w) { return mine + (size_t)(sp * DEC_WAVES + w) * ROW; }, d, acc, m, l);
@@ -628,17 +676,11 @@ __global__ __launch_bounds__(SIA_WAVE) void attn_decode_combine_kernel(
         return;
     }
     if (n_splits == 1) return;  // its one workgroup wrote the result itself
-    const size_t base = ((size_t)seq * n_heads + head) * max_splits;
-    float mx = -INFINITY;
-    for (int s = lane; s < n_splits; s += SIA_WAVE) mx = fmaxf(mx, ws_ml[(base + s) * 2]);
-    mx = wave_max(mx);
-    for (int d = lane; d < HD; d += SIA_WAVE)
-        dst[d] = float_to_bf16(merge_splits(n_splits, mx, sink_term(sinks, head, mx),
-                                            [&](int s, float& acc, float& m, float& l) {
-            acc = ws_acc[(base + s) * HD + d];
-            m = ws_ml[(base + s) * 2];
-            l = ws_ml[(base + s) * 2 + 1];
-        }));
+    const float o = n_splits <= FIRST ? combine_states(n_splits, acc, state, sinks, head)
+                    : n_splits <= 8   ? combine_all<8>(n_splits, acc_at, ml, sinks, head)
+                    : n_splits <= 16  ? combine_all<16>(n_splits, acc_at, ml, sinks, head)
+                                      : combine_all<DEC_MAX_SPLITS>(n_splits, acc_at, ml, sinks, head);
+    if (threadIdx.x < HD) dst[d] = float_to_bf16(o);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -1180,7 +1222,7 @@ SIA_EXPORT int sia_attn_decode_forms(const void* q, int q_row_stride, const void
                        ws_ml, (bf16_t*)out, n_heads, n_kv, ps_log2, scale, window, chunk, sinks, n_splits, (int)mode,
                        kv_share, forms);
     if (mode == DEC_SPREAD || (mode == DEC_PLAIN && n_splits > 1))
-        hipLaunchKernelGGL(attn_decode_combine_kernel, dim3(n_heads, n_seqs), dim3(SIA_WAVE), 0, stream, ws_acc,
+        hipLaunchKernelGGL(attn_decode_combine_kernel, dim3(n_heads, n_seqs), dim3(COMBINE_THREADS), 0, stream, ws_acc,
                            ws_ml, cu_q, kv_len, (bf16_t*)out, n_heads, n_splits, window, chunk, sinks,
                            mode == DEC_SPREAD ? 1 : 0, ps_log2, forms);
     return SIA_LAUNCH_CHECK();
