@@ -154,7 +154,7 @@ __global__ __launch_bounds__(512) void gla_recurrent_kernel(
 // exchanges and through LDS.  Dv a power of two from 16 to 256, D up to ROWS * G.
 // LOW_RANK: the decays exp(logsigmoid(a2 a + bias) / tau) are taken here, four lanes a channel, while the state is on
 // its way; else they come as floats.
-// 8 sequences of 24 heads of 128 x 128 (25 MB), rank 64: 15.5 us and 9.4 for the decays -> 10.9 for both.
+// 8 sequences of 24 heads of 128 x 128 (25 MB), rank 64: 15.5 us and 9.4 for the decays -> 10.9 for both; 10.4 with the gates and gains asked for first.
 struct LowRank {
     const bf16_t* a2;
     const float* bias;
@@ -194,10 +194,15 @@ __global__ __launch_bounds__(512) void state_decode_kernel(
     const uint2 v2 = *reinterpret_cast<const uint2*>(row + v_col + head * Dv + 4 * quad);
     const float v[4] = {__uint_as_float(v2.x << 16), __uint_as_float(v2.x & 0xffff0000u), __uint_as_float(v2.y << 16),
                         __uint_as_float(v2.y & 0xffff0000u)};
+    // what the end needs, asked for here: a trip to memory less behind the sums
+    const int column = min(tid, Dv - 1);
+    const float g = !raw_out && g_col >= 0 ? bf16_to_float(row[g_col + head * Dv + column]) : 0.f;
+    const float gain = !raw_out ? norm_w[(BONUS ? head * Dv : 0) + column] : 0.f;
     if (LOW_RANK) {
         const uint4* in = reinterpret_cast<const uint4*>(row + low.a_col);
         for (int c = tid / 4; c < D; c += 512 / 4) {      // four lanes a channel, pieces of eight in turn
             const uint4* w = reinterpret_cast<const uint4*>(low.a2 + (size_t)(head * D + c) * low.rank);
+            const float bias = low.bias ? low.bias[head * D + c] : 0.f;
             float z = 0.f;
             for (int m = tid % 4; m < low.rank / 8; m += 4) {
                 Vec8<bf16_t> x, y;
@@ -211,7 +216,7 @@ __global__ __launch_bounds__(512) void state_decode_kernel(
             }
             z += __shfl_xor(z, 1, SIA_WAVE);
             z += __shfl_xor(z, 2, SIA_WAVE);
-            if (tid % 4 == 0) decay[c] = sigmoid_power(z + (low.bias ? low.bias[head * D + c] : 0.f), low.tau_inv);
+            if (tid % 4 == 0) decay[c] = sigmoid_power(z + bias, low.tau_inv);
         }
         __syncthreads();
 #pragma unroll
@@ -254,9 +259,8 @@ __global__ __launch_bounds__(512) void state_decode_kernel(
     float total = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) total += squares[w];      // of threads beyond the columns: zeros
-    const float g = g_col >= 0 ? bf16_to_float(row[g_col + head * Dv + tid]) : 0.f;
     out[((size_t)n * n_heads + head) * Dv + tid] =
-        float_to_bf16(y * rsqrtf(total / (float)Dv + eps) * norm_w[(BONUS ? head * Dv : 0) + tid] * (g_col >= 0 ? g / (1.f + expf(-g)) : 1.f));
+        float_to_bf16(y * rsqrtf(total / (float)Dv + eps) * gain * (g_col >= 0 ? g / (1.f + expf(-g)) : 1.f));
 }
 
 // Sum over the 16 lanes of a row of a wave by lane exchanges inside the vector unit (no trip through LDS's crossbar):
