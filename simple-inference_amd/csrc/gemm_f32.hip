@@ -867,6 +867,61 @@ __global__ __launch_bounds__(256) void sum_slices_f32_kernel(const float* __rest
             if (n + e < N) at[e] = v[e];
 }
 
+// The activation between the two products of a feed-forward: the slices' sums of gate and up added in order, silu(gate) * up, and its parts for the
+// product that reads it.  A wave has the 16 rows and 32 columns of a block of parts; lane (r, g) eight columns of row r.  G: [slice][M][2 inter];
+// again: sums that are not finite are made from X and W (where no slices are apart, the product has done that).
+// Bound by its bytes: 303 rows of 8,192, two slices (40 MB in, 25 out) 12.8 us, where the sums took 11.4, the activation 7.0 and the parts 6.4, each
+// a launch behind the other (the float32 step of 303 tokens, four layers, 1,694 -> 1,596).
+__global__ __launch_bounds__(256) void sum_swiglu_split_kernel(const float* __restrict__ G, const float* __restrict__ X, const float* __restrict__ W,
+                                                               float* __restrict__ act, u32x4* __restrict__ parts, int M, int inter, int K,
+                                                               int n_slices, bool again, int blocks) {
+    const int chunks = inter / CHUNK;
+    const long long id = (long long)blockIdx.x * 4 + threadIdx.x / SIA_WAVE, b = id / chunks;
+    const int lane = threadIdx.x % SIA_WAVE, r = lane % 16, g = lane / 16, c = (int)(id % chunks);
+    if (b >= blocks) return;      // a wave leaves as a whole
+    const long long m = b * 16 + r;
+    const int k = c * CHUNK + 8 * g;
+    const bool live = m < M;
+    const size_t elements = (size_t)M * 2 * inter, at = (live ? m : 0) * 2 * inter + k;
+    f32x4 v[2][2];      // gate and up, four columns each
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i / 2][i % 2] = *(const f32x4*)(G + at + i / 2 * inter + i % 2 * 4);
+    for (int s = 1; s < n_slices; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i / 2][i % 2] += *(const f32x4*)(G + s * elements + at + i / 2 * inter + i % 2 * 4);
+    if (again) {
+        bool odd = false;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) odd |= live && !finite(v[i / 8][i / 4 % 2][i % 4]);
+        if (__any(odd)) {
+            const float* x = X + (size_t)(live ? m : M - 1) * K;
+#pragma clang loop unroll(disable)
+            for (int i = 0; i < 4; ++i) {      // place 4 g + e of float_sums is column 8 g + 4 (i % 2) + e
+                const f32x4 sums = float_sums(x, W + ((size_t)i / 2 * inter + c * CHUNK + 8 * (r / 4) + 4 * (i % 2) + r % 4) * K, K);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)      // (registers are not indexed)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (i == j && !finite(v[j / 2][j % 2][e])) v[j / 2][j % 2][e] = sums[e];
+            }
+        }
+    }
+    u32x4 a[2], p[PARTS];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float gate = v[0][e / 4][e % 4], up = v[1][e / 4][e % 4], y = gate / (1.f + expf(-gate)) * up;
+        a[e / 4][e % 4] = live ? __float_as_uint(y) : 0u;
+    }
+    if (live) {
+        u32x4* out = (u32x4*)(act + m * inter + k);
+        out[0] = a[0], out[1] = a[1];
+    }
+    if (split8(a[0], a[1], p) & 0xffffu) mark_rests(a[0], a[1], p[PARTS - 1]);
+    u32x4* to = parts + ((long long)c * blocks + b) * PART_BLOCK + lane;
+#pragma unroll
+    for (int e = 0; e < PARTS; ++e) to[e * SIA_WAVE] = p[e];
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // which kernel
 // ---------------------------------------------------------------------------------------------------------
@@ -988,6 +1043,37 @@ static int launch_f32_tall(const float* X, const float* W, float* Y, u32x4* part
     return SIA_LAUNCH_CHECK();
 }
 
+static void split_rows(const float* X, u32x4* parts, int M, int K, bool wide_x, hipStream_t stream) {
+    const int blocks = (M + 15) / 16, chunks = (K + CHUNK - 1) / CHUNK;
+    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)(((long long)blocks * chunks + 3) / 4)), dim3(256), 0, stream, X, parts, M, K, blocks, chunks,
+                       wide_x);
+}
+
+static void sum_slices(const float* slices, const float* X, const float* W, float* Y, int M, int N, int K, bool four, hipStream_t stream) {
+    hipLaunchKernelGGL(sum_slices_f32_kernel, dim3((M + 15) / 16, (N + 63) / 64), dim3(256), 0, stream, slices, X, W, Y, M, N, K, (N + 3) / 4 * 4,
+                       slices_of(N, K), four);
+}
+
+// A product's tiles, from the parts of X: Y, or with plan.apart the slices' sums.
+static int f32_tiles(const F32Plan& plan, const float* X, const float* W, float* Y, u32x4* parts, float* slices, int M, int N, int K, bool wide_w,
+                     bool four, hipStream_t stream) {
+    const bool apart = plan.apart;
+    int status = SIA_BAD_ARGUMENT;
+#define SHAPE(I, ...)         \
+    if (plan.shape == I)     \
+    status = wide_w ? launch_f32_tiles<__VA_ARGS__, true>(X, W, Y, parts, slices, M, N, K, apart, four, stream)      \
+                    : launch_f32_tiles<__VA_ARGS__, false>(X, W, Y, parts, slices, M, N, K, apart, four, stream)
+    if (plan.shape == 0) status = launch_f32_tiles<96, 256, 2, 4, 2, true>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
+    SHAPE(1, 64, 128, 2, 2, 1);
+    SHAPE(2, 64, 128, 2, 4, 2);
+    SHAPE(3, 32, 64, 2, 2, 2);
+    SHAPE(4, 128, 128, 2, 4, 2);
+#undef SHAPE
+    if (plan.shape == 5) status = launch_f32_tall<160, 128, 2, 3>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
+    if (plan.shape == 6) status = launch_f32_tall<160, 192, 1, 3>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
+    return status;
+}
+
 // The way that this product goes, for tests to tell which they reach: 2 * shape + apart of F32_SHAPES, or -(10 mb + nb) of the few-row kernel.
 SIA_EXPORT int sia_gemm_f32_way(const float* X, const float* W, int M, int N, int K) {
     const F32Plan plan = f32_plan(M, N, K, wide_rows(X, K), wide_rows(W, K));
@@ -1017,25 +1103,50 @@ SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* work
     }
     u32x4* const parts = (u32x4*)workspace;
     float* const slices = (float*)((char*)workspace + plan.parts);
-    const int blocks = (M + 15) / 16, chunks = (K + CHUNK - 1) / CHUNK, Ns = (N + 3) / 4 * 4;
-    hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)(((long long)blocks * chunks + 3) / 4)), dim3(256), 0, stream, X, parts, M, K, blocks, chunks,
-                       wide_x);
-    const bool apart = plan.apart;
-    int status = SIA_BAD_ARGUMENT;
-#define SHAPE(I, ...)         \
-    if (plan.shape == I)     \
-    status = wide_w ? launch_f32_tiles<__VA_ARGS__, true>(X, W, Y, parts, slices, M, N, K, apart, four, stream)      \
-                    : launch_f32_tiles<__VA_ARGS__, false>(X, W, Y, parts, slices, M, N, K, apart, four, stream)
-    if (plan.shape == 0) status = launch_f32_tiles<96, 256, 2, 4, 2, true>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
-    SHAPE(1, 64, 128, 2, 2, 1);
-    SHAPE(2, 64, 128, 2, 4, 2);
-    SHAPE(3, 32, 64, 2, 2, 2);
-    SHAPE(4, 128, 128, 2, 4, 2);
-#undef SHAPE
-    if (plan.shape == 5) status = launch_f32_tall<160, 128, 2, 3>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
-    if (plan.shape == 6) status = launch_f32_tall<160, 192, 1, 3>(X, W, Y, parts, slices, M, N, K, apart, four, stream);
-    if (status == 0 && apart)
-        hipLaunchKernelGGL(sum_slices_f32_kernel, dim3((M + 15) / 16, (N + 63) / 64), dim3(256), 0, stream, slices, X, W, Y, M, N, K, Ns,
-                           slices_of(N, K), four);
+    split_rows(X, parts, M, K, wide_x, stream);
+    const int status = f32_tiles(plan, X, W, Y, parts, slices, M, N, K, wide_w, four, stream);
+    if (status == 0 && plan.apart) sum_slices(slices, X, W, Y, M, N, K, four, stream);
+    return status ? status : SIA_LAUNCH_CHECK();
+}
+
+// Y[M, N] = (silu(X Wg^T) * (X Wu^T)) Wd^T, W = [Wg; Wu] of 2 inter rows of K, Wd [N, inter]: the same sums as the two products and the activation by
+// themselves, where both are the tiles'.  Bytes of workspace, or 0 where they are not, or operands do not lie so: then product by product.
+struct FeedForwardPlan {
+    F32Plan first, second;
+    long long between, act;      // bytes
+};
+static bool feed_forward_plan(const float* X, const float* W, const float* Wd, int M, int N, int K, int inter, FeedForwardPlan& plan) {
+    if (M <= 0 || N <= 0 || K <= 0 || inter <= 0 || inter % CHUNK || inter > 1 << 29 || !wide_rows(X, K) || !wide_rows(W, K) || !wide_rows(Wd, inter))
+        return false;
+    plan.first = f32_plan(M, 2 * inter, K, true, true);
+    plan.second = f32_plan(M, N, inter, true, true);
+    if (plan.first.shape < 0 || plan.second.shape < 0) return false;
+    plan.between = plan.first.apart ? plan.first.slices : (long long)M * 2 * inter * 4;
+    plan.act = (long long)M * inter * 4;
+    return true;
+}
+SIA_EXPORT long long sia_f32_feed_forward_workspace(const float* X, const float* W, const float* Wd, int M, int N, int K, int inter) {
+    FeedForwardPlan p;
+    return feed_forward_plan(X, W, Wd, M, N, K, inter, p) ? p.first.parts + p.between + p.act + p.second.parts + p.second.slices : 0;
+}
+SIA_EXPORT int sia_f32_feed_forward(const float* X, const float* W, const float* Wd, float* Y, void* workspace, int M, int N, int K, int inter,
+                                    hipStream_t stream) {
+    FeedForwardPlan p;
+    if (!feed_forward_plan(X, W, Wd, M, N, K, inter, p) || !workspace || ((uintptr_t)workspace & 15)) return SIA_BAD_ARGUMENT;
+    char* at = (char*)workspace;
+    u32x4* const parts = (u32x4*)at;
+    float* const between = (float*)(at += p.first.parts);
+    float* const act = (float*)(at += p.between);
+    u32x4* const act_parts = (u32x4*)(at += p.act);
+    float* const slices = (float*)(at += p.second.parts);
+    const bool four = N % 4 == 0 && ((uintptr_t)Y & 15) == 0;
+    split_rows(X, parts, M, K, true, stream);
+    int status = f32_tiles(p.first, X, W, between, parts, between, M, 2 * inter, K, true, true, stream);
+    if (status) return status;
+    const int blocks = (M + 15) / 16;
+    hipLaunchKernelGGL(sum_swiglu_split_kernel, dim3((unsigned)(((long long)blocks * (inter / CHUNK) + 3) / 4)), dim3(256), 0, stream, between, X, W, act,
+                       act_parts, M, inter, K, p.first.apart ? slices_of(2 * inter, K) : 1, p.first.apart, blocks);
+    status = f32_tiles(p.second, act, Wd, Y, act_parts, slices, M, N, inter, true, four, stream);
+    if (status == 0 && p.second.apart) sum_slices(slices, act, Wd, Y, M, N, inter, four, stream);
     return status ? status : SIA_LAUNCH_CHECK();
 }

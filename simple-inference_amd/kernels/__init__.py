@@ -112,6 +112,8 @@ _SIGNATURES = {
     "sia_gemm_generic": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_f32": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     "sia_gemm_f32_workspace": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int],
+    "sia_f32_feed_forward": [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
+    "sia_f32_feed_forward_workspace": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int],
     "sia_gemm_f32_way": [_c_ptr, _c_ptr, _c_int, _c_int, _c_int],
     "sia_prenorm_block": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr],
     "sia_prenorm_mixer": [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
@@ -313,6 +315,7 @@ class HipKernels:
         _bind(self.core, _SIGNATURES)
         self.core.sia_sample_workspace_bytes.restype = ctypes.c_longlong
         self.core.sia_gemm_f32_workspace.restype = ctypes.c_longlong
+        self.core.sia_f32_feed_forward_workspace.restype = ctypes.c_longlong
         self.core.sia_gla_workspace.restype = ctypes.c_longlong
         self.core.sia_moe_tiled_workspace.restype = ctypes.c_longlong
         self.core.sia_hgrn2_workspace.restype = ctypes.c_longlong
@@ -1504,6 +1507,26 @@ class HipKernels:
                         "gemm_tiles_swiglu")
             return y
         return self.swiglu(self.linear(x, w_gate_up))
+
+    def float_feed_forward(self, x, w_gate_up, w_down):
+        """``pending_linear(gated_linear(x, w_gate_up), w_down)`` of float32 rows in one call, with the same bits, where both products are
+        the tiles' (csrc/gemm_f32.hip): the activation makes the second one's parts.  Else None, with nothing done."""
+        if (not isinstance(x, torch.Tensor) or x.dtype != torch.float32 or w_gate_up.dtype != torch.float32 or w_down.dtype != torch.float32
+                or x.dim() != 2 or w_gate_up.dim() != 2 or w_down.dim() != 2 or w_gate_up.shape[1] != x.shape[1]
+                or w_gate_up.shape[0] != 2 * w_down.shape[1] or x.shape[0] > 65535):
+            return None
+        for t, what in ((x, "gated linear input"), (w_gate_up, "gate/up weight"), (w_down, "linear weight")):
+            self._want(t, what)
+        M, K = x.shape
+        N, inter = w_down.shape
+        size = self.core.sia_f32_feed_forward_workspace(_ptr(x), _ptr(w_gate_up), _ptr(w_down), M, N, K, inter)
+        if not size:
+            return None
+        y = torch.empty((M, N), dtype=torch.float32, device=x.device)
+        workspace = torch.empty(size, dtype=torch.uint8, device=x.device)
+        self._check(self.core.sia_f32_feed_forward(_ptr(x), _ptr(w_gate_up), _ptr(w_down), _ptr(y), _ptr(workspace), M, N, K, inter,
+                                                   self._stream()), "f32_feed_forward")
+        return y
 
     def sum_slices(self, slices, splits, out):
         """``out`` = the sum of a product's slices, rounded."""

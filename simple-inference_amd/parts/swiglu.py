@@ -68,6 +68,11 @@ class SwiGLU:
 
     def forward(self, h, ctx):
         k = self.env.kernels
+        if self.activation == "silu" and not self.bias:      # both products and what is between them, where a kernel has it
+            whole = getattr(k, "float_feed_forward", None)
+            y = whole(h, self.w_gate_up, self.w_down) if whole is not None else None
+            if y is not None:
+                return y
         if self.activation == "silu":
             a = k.gated_linear(h, self.w_gate_up)   # the activation is fused into the product where a kernel has it
         else:
