@@ -278,27 +278,32 @@ static_assert(SP_CLEAR_BYTES % (sizeof(uint4) * SP_CHUNKS) == 0 && sizeof(Sample
 
 // 1. maximum and its (lowest) index of each chunk, on the raw logits.  With `clear` each chunk's workgroup also
 // sets its share of the row's histograms to zero: the counting launches come after this one.
-__global__ __launch_bounds__(SP_THREADS) void sample_max_kernel(const float* __restrict__ logits, int vocab,
-                                                                SampleRow* __restrict__ ws, int clear) {
-    __shared__ float vals[SP_WAVES];
-    __shared__ int idxs[SP_WAVES];
+// Workgroups of four waves: with many rows a compute unit then has the loads of eight on their way while others reduce, where it had two of
+// 16 waves that did both in step.  us with the pick behind it, 16 waves -> 4:  rows of 128,256: one 7.0 -> 6.7, 64 14.0 -> 11.0, 303 42.7 -> 29.1
+// (155 MB: 6 TB/s while it reads);  300 of 32,000 33.7 -> 12.6;  64 of 512 9.7 -> 6.4.  (Four logits a load: the same.)
+#define SP_MAX_THREADS 256
+__global__ __launch_bounds__(SP_MAX_THREADS) void sample_max_kernel(const float* __restrict__ logits, int vocab,
+                                                                    SampleRow* __restrict__ ws, int clear) {
+    constexpr int WAVES = SP_MAX_THREADS / SIA_WAVE;
+    __shared__ float vals[WAVES];
+    __shared__ int idxs[WAVES];
     const int chunk = blockIdx.x, r = blockIdx.y;
     const float* row = logits + (size_t)r * vocab;
     int begin, end;
     chunk_range(chunk, vocab, begin, end);
     float bv = -INFINITY;
     int bi = vocab;
-    for (int i0 = begin + threadIdx.x; i0 < end; i0 += SP_AT_ONCE * SP_THREADS) {
+    for (int i0 = begin + threadIdx.x; i0 < end; i0 += SP_AT_ONCE * SP_MAX_THREADS) {
         float v[SP_AT_ONCE];
-        load_together(row, i0, SP_THREADS, end, v);
+        load_together(row, i0, SP_MAX_THREADS, end, v);
 #pragma unroll
         for (int u = 0; u < SP_AT_ONCE; ++u)
-            if (i0 + u * SP_THREADS < end) take_better(bv, bi, v[u], i0 + u * SP_THREADS);
+            if (i0 + u * SP_MAX_THREADS < end) take_better(bv, bi, v[u], i0 + u * SP_MAX_THREADS);
     }
     if (clear) {
         constexpr int share = (int)(SP_CLEAR_BYTES / sizeof(uint4) / SP_CHUNKS);
         uint4* mine = (uint4*)(ws + r) + chunk * share;
-        for (int i = threadIdx.x; i < share; i += SP_THREADS) mine[i] = make_uint4(0, 0, 0, 0);
+        for (int i = threadIdx.x; i < share; i += SP_MAX_THREADS) mine[i] = make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int off = SIA_WAVE / 2; off > 0; off >>= 1) {
@@ -309,7 +314,7 @@ __global__ __launch_bounds__(SP_THREADS) void sample_max_kernel(const float* __r
     if (threadIdx.x % SIA_WAVE == 0) { vals[threadIdx.x / SIA_WAVE] = bv; idxs[threadIdx.x / SIA_WAVE] = bi; }
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < SP_WAVES; ++w) take_better(bv, bi, vals[w], idxs[w]);
+        for (int w = 1; w < WAVES; ++w) take_better(bv, bi, vals[w], idxs[w]);
         ws[r].chunk_max[chunk] = bv;
         ws[r].chunk_arg[chunk] = bi;
     }
@@ -979,7 +984,7 @@ static int launch_sampling(const float* logits, const float* temperature, const 
         return SIA_LAUNCH_CHECK();
     }
     filters &= 7;
-    hipLaunchKernelGGL(sample_max_kernel, grid, block, 0, stream, logits, vocab, ws, (filters & 3) != 0);
+    hipLaunchKernelGGL(sample_max_kernel, grid, dim3(SP_MAX_THREADS), 0, stream, logits, vocab, ws, (filters & 3) != 0);
     if (filters & 1)
         for (int pass = 0; pass < SP_PASSES; ++pass)
             hipLaunchKernelGGL(sample_top_k_kernel, grid, block, 0, stream, logits, temperature, top_k, vocab, ws,
