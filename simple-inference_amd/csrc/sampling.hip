@@ -278,13 +278,14 @@ static_assert(SP_CLEAR_BYTES % (sizeof(uint4) * SP_CHUNKS) == 0 && sizeof(Sample
 
 // 1. maximum and its (lowest) index of each chunk, on the raw logits.  With `clear` each chunk's workgroup also
 // sets its share of the row's histograms to zero: the counting launches come after this one.
-// Workgroups of four waves: with many rows a compute unit then has the loads of eight on their way while others reduce, where it had two of
-// 16 waves that did both in step.  us with the pick behind it, 16 waves -> 4:  rows of 128,256: one 7.0 -> 6.7, 64 14.0 -> 11.0, 303 42.7 -> 29.1
-// (155 MB: 6 TB/s while it reads);  300 of 32,000 33.7 -> 12.6;  64 of 512 9.7 -> 6.4.  (Four logits a load: the same.)
-#define SP_MAX_THREADS 256
-__global__ __launch_bounds__(SP_MAX_THREADS) void sample_max_kernel(const float* __restrict__ logits, int vocab,
+// Of many rows by workgroups of four waves: a compute unit then has the loads of eight on their way while others reduce, where it had two of
+// 16 waves that did both in step.  us with the pick behind it, 16 waves and 4:  rows of 128,256: 64 14.0 and 10.8, 303 42.7 and 29.1
+// (155 MB: 6 TB/s while it reads);  300 of 32,000 33.7 and 12.6;  64 of 512 9.7 and 6.2.  Up to 16 rows, which a unit has one workgroup of, 16 waves, whose threads
+// ask for a chunk's logits at once: one row 7.3 and 7.8, 8 7.6 and 8.2.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void sample_max_kernel(const float* __restrict__ logits, int vocab,
                                                                     SampleRow* __restrict__ ws, int clear) {
-    constexpr int WAVES = SP_MAX_THREADS / SIA_WAVE;
+    constexpr int WAVES = THREADS / SIA_WAVE;
     __shared__ float vals[WAVES];
     __shared__ int idxs[WAVES];
     const int chunk = blockIdx.x, r = blockIdx.y;
@@ -293,17 +294,17 @@ __global__ __launch_bounds__(SP_MAX_THREADS) void sample_max_kernel(const float*
     chunk_range(chunk, vocab, begin, end);
     float bv = -INFINITY;
     int bi = vocab;
-    for (int i0 = begin + threadIdx.x; i0 < end; i0 += SP_AT_ONCE * SP_MAX_THREADS) {
+    for (int i0 = begin + threadIdx.x; i0 < end; i0 += SP_AT_ONCE * THREADS) {
         float v[SP_AT_ONCE];
-        load_together(row, i0, SP_MAX_THREADS, end, v);
+        load_together(row, i0, THREADS, end, v);
 #pragma unroll
         for (int u = 0; u < SP_AT_ONCE; ++u)
-            if (i0 + u * SP_MAX_THREADS < end) take_better(bv, bi, v[u], i0 + u * SP_MAX_THREADS);
+            if (i0 + u * THREADS < end) take_better(bv, bi, v[u], i0 + u * THREADS);
     }
     if (clear) {
         constexpr int share = (int)(SP_CLEAR_BYTES / sizeof(uint4) / SP_CHUNKS);
         uint4* mine = (uint4*)(ws + r) + chunk * share;
-        for (int i = threadIdx.x; i < share; i += SP_MAX_THREADS) mine[i] = make_uint4(0, 0, 0, 0);
+        for (int i = threadIdx.x; i < share; i += THREADS) mine[i] = make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int off = SIA_WAVE / 2; off > 0; off >>= 1) {
@@ -984,7 +985,9 @@ static int launch_sampling(const float* logits, const float* temperature, const 
         return SIA_LAUNCH_CHECK();
     }
     filters &= 7;
-    hipLaunchKernelGGL(sample_max_kernel, grid, dim3(SP_MAX_THREADS), 0, stream, logits, vocab, ws, (filters & 3) != 0);
+    const int max_threads = rows <= 16 ? SP_THREADS : 256;
+    hipLaunchKernelGGL(rows <= 16 ? sample_max_kernel<SP_THREADS> : sample_max_kernel<256>, grid, dim3(max_threads), 0, stream, logits, vocab, ws,
+                       (filters & 3) != 0);
     if (filters & 1)
         for (int pass = 0; pass < SP_PASSES; ++pass)
             hipLaunchKernelGGL(sample_top_k_kernel, grid, block, 0, stream, logits, temperature, top_k, vocab, ws,
