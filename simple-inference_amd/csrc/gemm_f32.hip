@@ -33,6 +33,8 @@
 // 2,048 28.8 -> 30.8, 32 x 14,336 x 4,096 50.5 -> 57.9) and 130 to 1,024 rows of 2,048 to 3,072 (512 x 2,048 x 2,048 42.7 -> 52.9, 303 x 3,072 x 2,048 42.6 -> 50).
 #include "lds_load.h"
 
+#include <algorithm>
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1110,7 +1112,9 @@ SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* work
 }
 
 // Y[M, N] = (silu(X Wg^T) * (X Wu^T)) Wd^T, W = [Wg; Wu] of 2 inter rows of K, Wd [N, inter]: the same sums as the two products and the activation by
-// themselves, where both are the tiles'.  Bytes of workspace, or 0 where they are not, or operands do not lie so: then product by product.
+// themselves.  Where both products are the tiles', with one kernel between them, which makes the second one's parts; else the three one after the
+// other, in one call too (the host takes longer for a step of few tokens than the GPU does).
+extern "C" int sia_swiglu(const void* gu, void* out, int n_tokens, int inter, int dtype, hipStream_t stream);
 struct FeedForwardPlan {
     F32Plan first, second;
     long long between, act;      // bytes
@@ -1125,15 +1129,28 @@ static bool feed_forward_plan(const float* X, const float* W, const float* Wd, i
     plan.act = (long long)M * inter * 4;
     return true;
 }
+static long long on16(long long bytes) { return (bytes + 15) / 16 * 16; }
 SIA_EXPORT long long sia_f32_feed_forward_workspace(const float* X, const float* W, const float* Wd, int M, int N, int K, int inter) {
+    if (M <= 0 || N <= 0 || K <= 0 || inter <= 0 || inter > 1 << 29) return 0;
     FeedForwardPlan p;
-    return feed_forward_plan(X, W, Wd, M, N, K, inter, p) ? p.first.parts + p.between + p.act + p.second.parts + p.second.slices : 0;
+    if (feed_forward_plan(X, W, Wd, M, N, K, inter, p)) return p.first.parts + p.between + p.act + p.second.parts + p.second.slices;
+    return on16((long long)M * 2 * inter * 4) + on16((long long)M * inter * 4) +
+           std::max(sia_gemm_f32_workspace(X, W, M, 2 * inter, K), sia_gemm_f32_workspace(nullptr, Wd, M, N, inter));
 }
 SIA_EXPORT int sia_f32_feed_forward(const float* X, const float* W, const float* Wd, float* Y, void* workspace, int M, int N, int K, int inter,
                                     hipStream_t stream) {
     FeedForwardPlan p;
-    if (!feed_forward_plan(X, W, Wd, M, N, K, inter, p) || !workspace || ((uintptr_t)workspace & 15)) return SIA_BAD_ARGUMENT;
+    if (M <= 0 || N <= 0 || K <= 0 || inter <= 0 || inter > 1 << 29 || !workspace || ((uintptr_t)workspace & 15)) return SIA_BAD_ARGUMENT;
     char* at = (char*)workspace;
+    if (!feed_forward_plan(X, W, Wd, M, N, K, inter, p)) {
+        float* const gate_up = (float*)at;
+        float* const act = (float*)(at += on16((long long)M * 2 * inter * 4));
+        at += on16((long long)M * inter * 4);
+        int status = sia_gemm_f32(X, W, gate_up, sia_gemm_f32_workspace(X, W, M, 2 * inter, K) ? at : nullptr, M, 2 * inter, K, stream);
+        if (!status) status = sia_swiglu(gate_up, act, M, inter, SIA_F32, stream);
+        if (!status) status = sia_gemm_f32(act, Wd, Y, sia_gemm_f32_workspace(act, Wd, M, N, inter) ? at : nullptr, M, N, inter, stream);
+        return status;
+    }
     u32x4* const parts = (u32x4*)at;
     float* const between = (float*)(at += p.first.parts);
     float* const act = (float*)(at += p.between);

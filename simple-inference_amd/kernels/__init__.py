@@ -1509,8 +1509,8 @@ class HipKernels:
         return self.swiglu(self.linear(x, w_gate_up))
 
     def float_feed_forward(self, x, w_gate_up, w_down):
-        """``pending_linear(gated_linear(x, w_gate_up), w_down)`` of float32 rows in one call, with the same bits, where both products are
-        the tiles' (csrc/gemm_f32.hip): the activation makes the second one's parts.  Else None, with nothing done."""
+        """``pending_linear(gated_linear(x, w_gate_up), w_down)`` of float32 rows in one call, with the same bits (csrc/gemm_f32.hip: where both
+        products are the tiles', the activation makes the second one's parts).  None, with nothing done, for other operands."""
         if (not isinstance(x, torch.Tensor) or x.dtype != torch.float32 or w_gate_up.dtype != torch.float32 or w_down.dtype != torch.float32
                 or x.dim() != 2 or w_gate_up.dim() != 2 or w_down.dim() != 2 or w_gate_up.shape[1] != x.shape[1]
                 or w_gate_up.shape[0] != 2 * w_down.shape[1] or x.shape[0] > 65535):

@@ -1050,25 +1050,25 @@ def test_float32_attention_has_the_same_bits_whichever_way_it_goes(hip, n_heads,
     assert rc == 0 and torch.equal(out, plain)
 
 
-# gate and up in slices and in one, the same of the second product, rows and columns that are no multiples of a tile; sizes that are not taken
-@pytest.mark.parametrize("K,inter,N,M,taken", [
-    (2048, 8192, 2048, 70, True), (2048, 8192, 2048, 303, True), (1024, 2816, 1000, 530, True), (4096, 1056, 4096, 303, True),
-    (4096, 1056, 4096, 530, True), (512, 4128, 1028, 303, True), (2048, 8192, 2048, 33, False), (1024, 2816, 1000, 303, False),
-    (512, 4128, 1028, 17, False)])
+# gate and up in slices and in one, the same of the second product, rows and columns that are no multiples of a tile; one product by tiles, and none
+@pytest.mark.parametrize("K,inter,N,M,tiles", [
+    (2048, 8192, 2048, 70, 2), (2048, 8192, 2048, 303, 2), (1024, 2816, 1000, 530, 2), (4096, 1056, 4096, 303, 2),
+    (4096, 1056, 4096, 530, 2), (512, 4128, 1028, 303, 2), (2048, 8192, 2048, 33, 1), (1024, 2816, 1000, 303, 1),
+    (512, 4128, 1028, 17, 0), (50, 37, 21, 3, 0), (50, 37, 21, 1, 0)])
 @pytest.mark.parametrize("whole_weights", [False, True])
-def test_float_feed_forward_in_one_call_has_the_bits_of_its_parts(hip, K, inter, N, M, taken, whole_weights):
+def test_float_feed_forward_in_one_call_has_the_bits_of_its_parts(hip, K, inter, N, M, tiles, whole_weights):
     """Both products and the activation between them, numbers that are not finite and numbers whose sums are made again among the rows'."""
     x, w, down = rnd(M, K, seed=1), rnd(2 * inter, K, seed=2, scale=K ** -0.5), rnd(N, inter, seed=3, scale=inter ** -0.5)
     if whole_weights:
         w, down = w.bfloat16().float(), down.bfloat16().float()
     for odd in (False, True):
         if odd:
-            x[3, 5], x[M - 1, K - 1], x[M // 2, 7], w[inter + 9, 3] = float("nan"), float("inf"), 3.39e38, 1e-39
+            x[M // 3, 5], x[M - 1, K - 1], x[M // 2, 7], w[inter + 9, 3] = float("nan"), float("inf"), 3.39e38, 1e-39
         want = hip.linear(hip.swiglu(hip.linear(x, w)), down)
         got = hip.float_feed_forward(x, w, down)
-        assert (got is not None) == taken
-        if taken:
-            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)), odd
+        way = lambda t, m, n, k: hip.core.sia_gemm_f32_way(t.data_ptr(), t.data_ptr(), m, n, k) >= 0
+        assert way(w, M, 2 * inter, K) + way(down, M, N, inter) == tiles
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)), odd
 
 
 # 16 rows that are several sequences' (two, six and sixteen of them), a part of one token's heads, and tokens that have workgroups of their own
