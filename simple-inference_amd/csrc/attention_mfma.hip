@@ -1288,19 +1288,25 @@ static int launch_prefill(int tiles, const void* q, int q_row_stride, const void
 
 // Which of the four workgroup shapes a launch takes.  n_tiles, n_tiles_split, n_tiles_long: its row tiles at 128, 64
 // and 256 tokens a workgroup; q_bound, kv_bound: the most tokens and the most keys of one of its sequences (0: not
-// known, taken as a prompt from its start).
+// known); span: the most keys that a query sees (0: all before it).
 enum PrefillShape { PF_SPLIT, PF_PAIRED, PF_WIDE, PF_LONG };
 static PrefillShape prefill_shape(int n_tiles, int n_tiles_split, int n_tiles_long, int n_heads, int q_bound,
-                                  int kv_bound) {
-    // Measured on 256 compute units.  For a prompt from its start, whose row tiles see from few
-    // keys to all, the fastest shape follows the number of workgroups per compute unit: the split shape while all
+                                  int kv_bound, int span) {
+    // Measured on 256 compute units.  The fastest shape follows the number of workgroups per compute unit: the split shape while all
     // its workgroups are on the chip at once (up to 6/8 of a wide workgroup per compute unit: prompts up to about
-    // 1,000 tokens of 24 heads), the paired shape of 128 tokens (two tiles of keys a step, one for each set of waves) up to 18/8
-    // (about 3,000 tokens), the wide shape (one tile a step, two workgroups a unit) beyond, and for heads of more than 64 from 30/8 on (about 5,000
+    // 1,000 tokens of 24 heads), the paired shape of 128 tokens (two tiles of keys a step, one for each set of waves) up to 15/8
+    // (about 2,500 tokens), the wide shape (one tile a step, two workgroups a unit) beyond, and for heads of more than 64 from 36/8 on (about 6,000
     // tokens) 8 waves of 32 tokens (256 tokens a workgroup, two tiles a step: a tile staged in LDS then serves twice as many tokens).
-    // us, paired, wide, long, by wide workgroups a unit:  heads of 128:  1.5 51 68 76;  2.0 60 70 77 and 76 95 93;  2.3 108 105 110;  2.6 102 99 96;
-    // 3.0 159 133 145;  3.1 134 112 111;  3.8 235 223 209;  4.0 195 184 162;  5.1 412 360 374, 310 276 280;  6.9 535 475 457.
-    // heads of 64:  2.0 43 48 55;  2.6 75 74 73;  3.1 98 74 80;  4.0 145 104 114;  5.1 237 166 202;  6.9 406 271 330.
+    // One prompt from its start (or one that is half of the launch or more), whose row tiles see from few keys to all, keeps the paired shape up
+    // to 36/16 (35/16 with heads of 80 to 112) and takes the long one from 30/8 on with heads of 128, if it is more than half:
+    // us, paired, wide, long, by wide workgroups a unit, 24 or 32 heads:
+    //   heads of 128:  2.0 59 70 79;  2.25 96 101 115 and 76 78 89;  2.4 111 109 125;  3.2 168 145 161;  3.75 222 199 188;  4.0 190 172 167;  4.5 315 279 275;
+    //   heads of 96:  2.0 54 60 69;  2.13 66 65 68;  2.25 92 87 103;  3.2 165 128 142;  3.75 219 176 178;  4.25 212 167 171;  4.5 314 245 257;
+    //   heads of 64:  2.0 44 51 57;  2.25 71 73 82;  2.4 82 79 89;  3.2 126 103 114;  4.0 141 99 116;  6.0 395 274 336.
+    // With a quarter as many earlier ones or through a window of 7/10 of the keys up to 32/16, and from 30/8 to 32/8:  2.0, over a quarter, 128 79 86 98, 64 59 62 70;
+    // through 3/4, 128 56 60 71;  3.75, over a quarter, 128 332 334 303.
+    // Others, whose row tiles see more alike, at 2.25:  3,067 tokens of 24 heads of 128 through a window of 1,024 64 53 58, over 1,536 earlier ones 183 157
+    // 169;  of 64 46 38 39, 138 108 120;  three prompts of 700, 32 heads of 64 30 23 24;  and at 4.0 through a window of 256, 24 heads of 128 69 52 59.
     const long long wide_groups = (long long)n_tiles * n_heads, cus = compute_units();
     const bool split_fits = n_tiles_split > 0 && wide_groups * 8 <= cus * 6;
     // A portion over a past is another matter: every row tile sees about as many keys, so the launch lasts as many
@@ -1315,10 +1321,25 @@ static PrefillShape prefill_shape(int n_tiles, int n_tiles_split, int n_tiles_lo
         const long long lng = n_tiles_long > 0 ? ((long long)n_tiles_long * n_heads + cus - 1) / cus * 222 : paired + wide;
         return lng <= wide && lng <= paired ? PF_LONG : wide <= paired ? PF_WIDE : PF_PAIRED;
     }
+    const long long longest = (q_bound + PF_ROWS - 1) / PF_ROWS;      // row tiles of the longest
+    const bool from_start = q_bound > 0 && kv_bound <= q_bound && (span <= 0 || span >= kv_bound) && 2 * longest >= n_tiles;
+    const bool nearly = q_bound > 0 && 4LL * kv_bound <= 5LL * q_bound && (span <= 0 || 10LL * span >= 7LL * kv_bound) && 2 * longest >= n_tiles;
     if (split_fits) return PF_SPLIT;
-    if (wide_groups * 8 <= cus * 18) return PF_PAIRED;
-    if (HD > 64 && n_tiles_long > 0 && wide_groups * 8 >= cus * 30) return PF_LONG;
+    if (wide_groups * 16 <= cus * (from_start ? HD > 64 && HD < 128 ? 35 : 36 : nearly ? 32 : 30)) return PF_PAIRED;
+    if (HD > 64 && n_tiles_long > 0 && wide_groups * 8 >= cus * 36) return PF_LONG;
+    if (HD == 128 && n_tiles_long > 0 && 2 * longest > n_tiles && wide_groups * 8 >= cus * 30 && (from_start || (nearly && wide_groups <= cus * 4)))
+        return PF_LONG;
     return PF_WIDE;
+}
+
+// The most keys that a query sees through a window, in its block of chunk positions, or both (0: all before it).
+static int prefill_span(int window, int chunk) { return window > 0 && chunk > 0 ? (window < chunk ? window : chunk) : window > 0 ? window : chunk; }
+
+// The shape that such a launch takes (0 split, 1 paired, 2 wide, 3 long; -1: head sizes that have one only), for tests to tell which they reach.
+SIA_EXPORT int sia_attn_prefill_shape(int n_tiles, int n_tiles_split, int n_tiles_long, int q_bound, int kv_bound, int n_heads, int window,
+                                      int chunk) {
+    if (HD > 128 || !PF_USE_LDS) return -1;
+    return prefill_shape(n_tiles, n_tiles_split, n_tiles_long, n_heads, q_bound, kv_bound, prefill_span(window, chunk));
 }
 
 SIA_EXPORT int sia_attn_prefill_forms(const void* q, int q_row_stride, const void* k_pages, const void* v_pages,
@@ -1338,7 +1359,7 @@ SIA_EXPORT int sia_attn_prefill_forms(const void* q, int q_row_stride, const voi
     if constexpr (HD > 128 || !PF_USE_LDS) {
         return HD > 128 ? launch_prefill<1, PF_ROWS / 16, 1>(n_tiles, ARGS) : launch_prefill<2, PF_ROWS / 32, 1>(n_tiles, ARGS);
     } else {
-        switch (prefill_shape(n_tiles, n_tiles_split, n_tiles_long, n_heads, q_bound, kv_bound)) {
+        switch (prefill_shape(n_tiles, n_tiles_split, n_tiles_long, n_heads, q_bound, kv_bound, prefill_span(window, chunk))) {
             case PF_SPLIT: return launch_prefill<1, 2 * PF_ROWS_SPLIT / 16, 2>(n_tiles_split, ARGS);
             case PF_PAIRED: return launch_prefill<2, 2 * PF_ROWS / 32, 2, 2>(n_tiles, ARGS);
             case PF_LONG: return launch_prefill<2, PF_ROWS_LONG / 32, 1, 2>(n_tiles_long, ARGS);

@@ -208,6 +208,7 @@ _ATTN_SIGNATURES = {
     "sia_attn_decode_max_splits": [_c_int, _c_int],
     "sia_attn_decode_workspace": [_c_int, _c_int, _c_int, _c_int, _c_int],
     "sia_attn_decode_mode": [_c_int, _c_int, _c_int, _c_int],
+    "sia_attn_prefill_shape": [_c_int] * 8,
     "sia_attn_prefill_rows": [],
     "sia_attn_prefill_rows_split": [],
     "sia_attn_prefill_rows_long": [],

@@ -1253,6 +1253,35 @@ def test_the_product_into_the_residual_reads_the_weight_as_it_is(hip, N, K):
         w.mul_(2.0)
 
 
+SPLIT, PAIRED, WIDE, LONG = range(4)      # of sia_attn_prefill_shape
+
+
+def prefill_shape(hip, D, n_heads, q_lens, kv_lens, window=None, chunk=None, forms=False):
+    """The workgroup shape that a step of these portions takes, decoded tokens apart."""
+    lib = hip._attn_lib(D, forms=forms)
+    tiles = [sum(-(-q // rows()) for q in q_lens)
+             for rows in (lib.sia_attn_prefill_rows, lib.sia_attn_prefill_rows_split, lib.sia_attn_prefill_rows_long)]
+    return lib.sia_attn_prefill_shape(*tiles, max(q_lens), max(kv_lens), n_heads, window or 0, chunk or 0)
+
+
+# One prompt from its start, of 15/8 to 18/8 and of 30/8 to 36/8 workgroups of 128 tokens a compute unit, and what is none: through a window, in
+# blocks, over earlier tokens, several.
+@pytest.mark.parametrize("D, n_heads, q_lens, past, window, chunk, shape", [
+    (64, 24, [3067], 0, None, None, PAIRED), (64, 24, [3067], 0, 1024, None, WIDE), (64, 24, [3067], 0, None, 1024, WIDE),
+    (64, 24, [3067], 0, 4096, 8192, PAIRED), (64, 24, [3067], 1536, None, None, WIDE), (64, 32, [700] * 3, 0, None, None, WIDE),
+    (64, 32, [1100] * 2, 0, None, None, PAIRED), (64, 32, [2043], 510, None, None, PAIRED), (64, 32, [2043], 0, 1600, None, PAIRED),
+    (64, 32, [2171], 500, None, None, WIDE), (64, 24, [3000], 8192, None, None, WIDE), (32, 32, [2299], 0, 256, None, WIDE),
+    (128, 24, [3067], 0, None, None, PAIRED), (128, 24, [3067], 0, 1024, None, WIDE), (128, 24, [3067], 1536, None, None, WIDE),
+    (80, 24, [2939], 0, None, None, PAIRED), (80, 24, [3067], 0, None, None, WIDE), (112, 24, [3067], 0, None, None, WIDE),
+    (128, 32, [4091], 0, None, None, LONG), (128, 32, [4091], 0, 256, None, WIDE), (128, 32, [4091], 0, None, 300, WIDE),
+    (128, 32, [4091], 1000, None, None, LONG), (128, 32, [4347], 1000, None, None, WIDE), (128, 32, [2043] * 2, 0, None, None, WIDE),
+    (64, 32, [4091], 0, None, None, WIDE), (80, 32, [4091], 0, None, None, WIDE), (112, 32, [4091], 0, None, None, WIDE),
+    (80, 32, [4603], 0, None, None, LONG), (80, 32, [4603], 0, 256, None, LONG), (64, 32, [7001], 0, None, None, WIDE)])
+def test_prefill_shapes_follow_what_the_row_tiles_see(hip, D, n_heads, q_lens, past, window, chunk, shape):
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    assert prefill_shape(hip, D, n_heads, q_lens, [q + past for q in q_lens], window, chunk) == shape
+
+
 @pytest.mark.parametrize("q_len, kv_len, window", [(130, 130, None), (900, 1000, None), (1900, 1900, None),
                                                   (1900, 2100, 300)])
 def test_matrix_core_prefill_in_each_workgroup_shape(hip, q_len, kv_len, window):
