@@ -854,11 +854,8 @@ __device__ __forceinline__ void compute_from_lds(const bf16_t* __restrict__ k_ld
 // every KSPLIT-th tile of keys: ROWS = PF_NQ * 16 * PF_WAVES / KSPLIT tokens per workgroup.  KTILES tiles of keys
 // are staged per step (and barrier); with KSPLIT = 1 every wave takes them one after the other, which at 8 waves
 // of 16 tokens is 7 % faster with two tiles than with one (fewer barriers a key) and changes no bit.
-// At least two waves a SIMD, so 256 registers: left to itself the compiler gives the wide shape 316 of heads of 128, and a compute unit then
-// holds one of its workgroups of four waves and not two (4,096 tokens, 24 heads of 128: 245 us, now 133; 7,001, 32 of 64: 357, now 271).
-constexpr int PF_MIN_WAVES = HD <= 128 ? 2 : 1;
 template <int PF_NQ, int PF_WAVES, int KSPLIT, int KTILES>
-__global__ __launch_bounds__(PF_WAVES* SIA_WAVE, PF_MIN_WAVES) void attn_prefill_kernel(
+__global__ __launch_bounds__(PF_WAVES* SIA_WAVE) void attn_prefill_kernel(
     const bf16_t* __restrict__ q, int q_row_stride, const bf16_t* __restrict__ kp, const bf16_t* __restrict__ vp,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ cu_q,
     const int* __restrict__ kv_len, bf16_t* __restrict__ out, int n_heads, int n_kv, int ps_log2, float scale,
