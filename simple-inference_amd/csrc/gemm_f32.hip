@@ -933,8 +933,8 @@ __global__ __launch_bounds__(256) void sum_swiglu_split_kernel(const float* __re
 // adds to that, a MB of the slices' sums written and read (through Y, for tiles of 256 columns).  By least squares over the geometric mean
 // of weights of 8 and 24 bits, 2,900 products of 256 to 128,256 columns, k of 256 to 8,192, 17 to 1,024 rows:  median error 2 to 4 %; the choice
 // is 2.2 % above the best of seven shapes on average, 11 % in one of twenty.  The tall ones (gemm_f32_tall_kernel) by 695 products of the same sizes and of
-// columns to 40,000 (median error 2 to 3 %, one of twenty 10 %): they are the fastest by more than 3 % in 134 of them, up to 1.47 times, from 65 rows on (fewer not
-// measured), and leave the others as they were.
+// columns to 40,000 (median error 2 to 3 %, one of twenty 10 %; for them only where they are clearly the shorter, see f32_plan), from 65 rows on (fewer not
+// measured).
 struct F32Cost {
     double launch, round, step, more, sums;
 };
@@ -971,6 +971,8 @@ static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w) {
     const int rows_w = few.nb * 16, rows_x = few.mb * 16;
     const double fetched = (double)((M + rows_x - 1) / rows_x) * ((N + rows_w - 1) / rows_w) * (rows_w + rows_x) * K * 4e-6;
     double least = (few.launch + fmax(fetched / few.rate, (double)N * K * 4e-6 / 5.4)) * (wide_x && wide_w ? 1 : 1.6);
+    double others = least;      // the estimate without the tall shapes
+    bool two_a_unit = false;
     for (int i = 0; i < N_F32_SHAPES; ++i) {
         const F32Shape& t = F32_SHAPES[i];
         const bool tall = i >= FIRST_TALL;
@@ -986,8 +988,13 @@ static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w) {
             double us = c.launch + (full + (last > 0)) * (c.round + c.step * steps) + (full * t.at_a_time + last) * c.more * steps;
             if (apart) us += c.sums * n_slices * M * N * 8e-6;
             else us += c.sums * (n_slices - 1) * M * N * 8e-6;
+            // A tall shape's estimate has to be less than others' by what these err: 9 % where two workgroups of 64 x 128 share a unit, else 4 %; it takes
+            // no product from the few-row kernel.  (Of 1,560 products of 65 to 4,096 rows that it was estimated the shorter for, 246 took more
+            // than 3 % longer with it, up to 24 %;  so it takes 1,247, of which 41 do, and leaves 42 that it has 3 % and more to give.)
+            if (tall && (best.shape < 0 || us >= (two_a_unit ? 0.91 : 0.96) * others)) continue;
             if (us >= least) continue;
             least = us;
+            if (!tall) others = us, two_a_unit = i == 1 && !apart;
             best.shape = i, best.apart = apart;
         }
     }

@@ -620,8 +620,20 @@ def test_float32_products_every_way(hip, M, N, K, way):
 
 
 # Tiles of 160 rows:  whole k and slices of 2 and 8, rows behind a tile and last tiles in part, columns that are no multiple of 4.
-TALL_FLOAT_WAYS = [(129, 50003, 192, 10), (160, 50003, 224, 10), (150, 3074, 2048, 11), (129, 12290, 1024, 11), (160, 14337, 1024, 11),
-                   (129, 32770, 224, 12), (97, 40961, 256, 12), (303, 2050, 2048, 13), (97, 5123, 2048, 13), (129, 16386, 1024, 13)]
+TALL_FLOAT_WAYS = [(129, 28674, 128, 10), (160, 50003, 224, 10), (259, 14337, 128, 10), (145, 14337, 768, 11), (129, 12290, 1024, 11), (160, 14337, 1024, 11),
+                   (129, 32770, 224, 12), (150, 40961, 160, 12), (311, 2050, 2048, 13), (129, 5123, 1536, 13), (606, 16386, 1536, 13)]
+
+
+# The tall tiles take products of a float32 model's steps, and none that the smaller tiles or the few-row kernel take as long or less for:  us, theirs and the
+# tall ones', weights of 8 bits:  768 x 12,288 x 3,072 263 and 327;  1,280 x 8,192 x 4,096 366 and 446;  640 x 1,024 x 1,536 21.4 and 26.1;  160 x 3,072 x
+# 2,048 24.3 and 26.1;  303 x 128,256 x 2,048 691 and 594.
+@pytest.mark.parametrize("M, N, K, way", [
+    (303, 128256, 2048, 12), (303, 16384, 2048, 11), (303, 3072, 2048, 13), (303, 2048, 8192, 11), (303, 2048, 2048, 11),
+    (768, 12288, 3072, 2), (1280, 8192, 4096, 2), (640, 1024, 1536, -21), (129, 3072, 2048, -21), (160, 3072, 2048, -21),
+    (1024, 6144, 4096, 2), (256, 2048, 2048, 3)])
+def test_tall_tiles_take_the_float32_products_that_they_are_the_faster_for(hip, M, N, K, way):
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    assert hip.core.sia_gemm_f32_way(None, None, M, N, K) == way
 
 
 @pytest.mark.parametrize("M, N, K, way", TALL_FLOAT_WAYS)
