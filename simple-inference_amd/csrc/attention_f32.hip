@@ -12,9 +12,10 @@
 // A token that is its sequence's only one (decode) has a workgroup of its own.
 // What bounds it is the chain of a chunk: 16 dependent products of 32 cycles a wave each for scores and values (heads of 64), and two barriers, 5,000 cycles
 // in all; 600 and more tokens fill the chip with chains.  us, before (a lane a key) and now: 303 tokens (three decoded over 200 keys, a prompt of 300), 32 heads of 64 on 8
-// 58 -> 17.6, 24 of 128 on 8 107 -> 24;  a prompt of 2,048 960 -> 315 (55 TFLOP/s of 157), 2,160 -> 446;  one token over 16,000 keys 1,347 -> 540;
-// 64 over 2,048 209 -> 116 (537 MB: 4.6 TB/s).
+// 57 -> 16.2, 24 of 128 on 8 101 -> 22.8;  a prompt of 2,048 956 -> 308 (56 TFLOP/s of 157), 2,160 -> 443;  one token over 16,000 keys 1,358 -> 535;
+// 64 over 2,048 211 -> 115 (537 MB: 4.7 TB/s);  256 over 17 with a query head for each of 16 key/value heads of 64 33 -> 23 (by the plain kernel).
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 
@@ -63,22 +64,23 @@ __device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c) { return __buil
 // all waves have come here, and what they have written to LDS is there; loads from memory stay on their way
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// DP: 64 or 128, the head sizes' upper bound.
+// DP: 32, 64 or 128, the head sizes' upper bound.  (Of 32 dimensions two of the waves have the values.)
 template <int DP>
 __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
     const float* __restrict__ q, int q_row_stride, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ seq_of_token,
     const int* __restrict__ positions, float* __restrict__ out, int n_tokens, int n_single, int n_heads, int n_kv,
     int head_dim, int value_dim, int page_size, float scale, int window, int chunk, const float* __restrict__ sinks,
-    float cap, int keep_first) {
-    constexpr int PIECES = DP / 16, BLOCKS = DP / 64;      // a lane's fours of a row of keys; blocks of 16 dimensions of a wave's values
+    float cap, int keep_first, int tile_rows) {
+    constexpr int PIECES = DP / 16, BLOCKS = DP < 64 ? 1 : DP / 64;      // a lane's fours of a row of keys; blocks of 16 dimensions of a wave's values
     __shared__ float most[WAVES][ROWS];
     __shared__ __attribute__((aligned(16))) float weight[ROWS * P_ROW];      // [row][position: 16 (j % 4) + j / 4]
 
     const int lane = threadIdx.x % SIA_WAVE, wave = threadIdx.x / SIA_WAVE, r = lane % 16, g = lane / 16;
+    const bool has_values = DP >= 64 || wave < DP / 16;
     const int group = n_heads / n_kv, hk = blockIdx.x % n_kv, page_log2 = __ffs(page_size) - 1, in_page = page_size - 1;
-    // The rows: token * group + head, those of a single token in tiles of their own, which come first; then the others' from the last on, whose
-    // tokens see the most keys.
+    // The rows: token * group + head, those of a single token in tiles of their own, which come first; then the others', tile_rows a tile, from the
+    // last on, whose tokens see the most keys.
     const int tile = blockIdx.x / n_kv, per_single = (group + ROWS - 1) / ROWS, single_tiles = n_single * per_single;
     long long row0, row_end;
     if (tile < single_tiles) {
@@ -86,9 +88,9 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
         row_end = (long long)(tile / per_single + 1) * group;
     } else {
         row_end = (long long)n_tokens * group;
-        row0 = (long long)n_single * group + (long long)((int)(gridDim.x / n_kv) - 1 - tile) * ROWS;
+        row0 = (long long)n_single * group + (long long)((int)(gridDim.x / n_kv) - 1 - tile) * tile_rows;
     }
-    const int n_rows = (int)min((long long)ROWS, row_end - row0);
+    const int n_rows = (int)min((long long)(tile < single_tiles ? ROWS : tile_rows), row_end - row0);
     const int token = (int)((row0 + min(r, n_rows - 1)) / group), head = hk * group + (int)((row0 + min(r, n_rows - 1)) % group);
     const int my_seq = seq_of_token[token], my_pos = positions[token];
     auto oldest = [&](int pos) {
@@ -131,12 +133,13 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
             const int j = c0 + lane;
             return j <= last && (j >> page_log2) < table_width ? table[j >> page_log2] : -1;
         };
-        // Keys 16 wave + r of the chunk, and dimensions of the values, four positions at a time.  Where there is no page, or no such
-        // dimension, what is read is not used.
+        // Keys 16 wave + r of the chunk, and dimensions of the values, four positions at a time.  Where there is no page (nor is there behind the
+        // last position), or no such dimension, something near is read and not used:  a branch instead of that makes every chunk wait for its
+        // loads (one token over 16,000 keys, 32 heads of 64 on 8: 543 us, 695 so).
         f32x4 kr[PIECES], vr[BLOCKS][4];
         auto fetch_keys = [&](int c0, int page) {
-            const int j = 16 * wave + r, pg = max(__shfl(page, j, SIA_WAVE), 0);
-            const float* at = k_pages + ((((size_t)pg * n_kv + hk) << page_log2) + ((c0 + j) & in_page)) * head_dim;
+            const int j = 16 * wave + r, pg0 = __shfl(page, j, SIA_WAVE), pg = max(pg0, 0), in = pg0 < 0 ? 0 : (c0 + j) & in_page;
+            const float* at = k_pages + ((((size_t)pg * n_kv + hk) << page_log2) + in) * head_dim;
 #pragma unroll
             for (int i = 0; i < PIECES; ++i) {
                 const int d = 16 * i + 4 * g;
@@ -144,14 +147,14 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
             }
         };
         auto fetch_values = [&](int c0, int page) {
+            if (!has_values) return;
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                const int j = 16 * b + 4 * g, pg = max(__shfl(page, j, SIA_WAVE), 0);
+                const int j = 16 * b + 4 * g, pg0 = __shfl(page, j, SIA_WAVE), pg = max(pg0, 0), in = pg0 < 0 ? 0 : (c0 + j) & in_page;
 #pragma unroll
                 for (int a = 0; a < BLOCKS; ++a) {
                     const int d = (wave * BLOCKS + a) * 16 + r;
-                    vr[a][b] = *(const f32x4*)(v_pages + ((((size_t)pg * n_kv + hk) * value_dim + (d < value_dim ? d : 0)) << page_log2) +
-                                               ((c0 + j) & in_page));
+                    vr[a][b] = *(const f32x4*)(v_pages + ((((size_t)pg * n_kv + hk) * value_dim + (d < value_dim ? d : 0)) << page_log2) + in);
                 }
             }
         };
@@ -201,53 +204,59 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
             if (sees) l = l * alpha + sum;
 #pragma unroll
             for (int a = 0; a < BLOCKS; ++a) acc[a] *= alpha;
-            // Values of keys that a row does not see may be anything: where they are finite a weight of 0 leaves them out.  Those that no
-            // row of the run sees are replaced; if one of the others is not finite, every row gets its own values.
-            bool apart = false;
-            if (c0 + CHUNK - 1 > first || c0 < lo_last || end - begin < n_rows || __any(page < 0)) {
+            if (has_values) {
+                // Values of keys that a row does not see may be anything: where they are finite a weight of 0 leaves them out.  Those that no
+                // row of the run sees are replaced; if one of the others is not finite, and rows differ in what they see, every row gets its own values.
+                bool apart = false;
+                if (c0 + CHUNK - 1 > first || c0 < lo_last || end - begin < n_rows || __any(page < 0)) {
+                    const int j = c0 + lane;
+                    const unsigned long long seen = __ballot(page >= 0 && (j >= lo0 || j < keep0)) >> (4 * g);      // bit 16 b + e
+                    const unsigned half[2] = {(unsigned)seen, (unsigned)(seen >> 32)};
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const int j = c0 + 16 * b + 4 * g;
-                    const bool there = __shfl(page, 16 * b + 4 * g, SIA_WAVE) >= 0;
+                    for (int b = 0; b < 4; ++b)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const bool seen = there && j + e <= last && (j + e >= lo0 || j + e < keep0);
+                        for (int e = 0; e < 4; ++e)
 #pragma unroll
-                        for (int a = 0; a < BLOCKS; ++a) {
-                            vr[a][b][e] = seen ? vr[a][b][e] : 0.f;
-                            apart |= !__builtin_isfinite(vr[a][b][e]);
-                        }
-                    }
-                }
-                apart = __any(apart);
-            }
-#pragma unroll
-            for (int a = 0; a < BLOCKS; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) across_groups(vr[a][b]);
-            if (!apart) {
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-#pragma unroll
-                        for (int a = 0; a < BLOCKS; ++a) acc[a] = mfma(vr[a][b][e], p[b][e], acc[a]);
-            } else {
-#pragma clang loop unroll(disable)
-                for (int row = begin; row < end; ++row) {
-                    const int pos = __builtin_amdgcn_readlane(my_pos, row), lo = __builtin_amdgcn_readlane(my_lo, row);
-                    const int keep = min(keep_first, lo);
-#pragma unroll
-                    for (int a = 0; a < BLOCKS; ++a) {
-                        f32x4 own = acc[a];
+                            for (int a = 0; a < BLOCKS; ++a) vr[a][b][e] = half[b / 2] >> (16 * (b % 2) + e) & 1 ? vr[a][b][e] : 0.f;
+                    if (first < last || end - begin < n_rows) {
+                        float odd = 0.f;
 #pragma unroll
                         for (int b = 0; b < 4; ++b)
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const int j = c0 + 16 * b + 4 * e + g;
-                                own = mfma(j <= pos && (j >= lo || j < keep) ? vr[a][b][e] : 0.f, p[b][e], own);
-                            }
-                        if (r == row) acc[a] = own;
+                            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                                for (int a = 0; a < BLOCKS; ++a) odd = fmaf(vr[a][b][e], 0.f, odd);
+                        apart = __any(!(odd == 0.f));
+                    }
+                }
+#pragma unroll
+                for (int a = 0; a < BLOCKS; ++a)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) across_groups(vr[a][b]);
+                if (!apart) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+#pragma unroll
+                            for (int a = 0; a < BLOCKS; ++a) acc[a] = mfma(vr[a][b][e], p[b][e], acc[a]);
+                } else {
+#pragma clang loop unroll(disable)
+                    for (int row = begin; row < end; ++row) {
+                        const int pos = __builtin_amdgcn_readlane(my_pos, row), lo = __builtin_amdgcn_readlane(my_lo, row);
+                        const int keep = min(keep_first, lo);
+#pragma unroll
+                        for (int a = 0; a < BLOCKS; ++a) {
+                            f32x4 own = acc[a];
+#pragma unroll
+                            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    const int j = c0 + 16 * b + 4 * e + g;
+                                    own = mfma(j <= pos && (j >= lo || j < keep) ? vr[a][b][e] : 0.f, p[b][e], own);
+                                }
+                            if (r == row) acc[a] = own;
+                        }
                     }
                 }
             }
@@ -275,17 +284,20 @@ __global__ __launch_bounds__(WAVES * SIA_WAVE) void attention_f32_kernel(
     }
 }
 
+static long long tiles_of(long long n_tokens, long long n_single, long long group, int tile_rows) {
+    return n_single * ((group + ROWS - 1) / ROWS) + ((n_tokens - n_single) * group + tile_rows - 1) / tile_rows;
+}
+
 template <int DP>
 static int launch(const float* q, int q_row_stride, const float* k_pages, const float* v_pages, const int* block_table,
                   int table_width, const int* seq_of_token, const int* positions, float* out, int n_tokens, int n_single,
                   int n_heads, int n_kv, int head_dim, int value_dim, int page_size, float scale,
-                  int window, int chunk, const float* sinks, float cap, int keep_first, hipStream_t stream) {
-    const long long group = n_heads / n_kv;
-    const long long tiles = n_single * ((group + ROWS - 1) / ROWS) + ((n_tokens - n_single) * group + ROWS - 1) / ROWS;
+                  int window, int chunk, const float* sinks, float cap, int keep_first, int tile_rows, hipStream_t stream) {
+    const long long tiles = tiles_of(n_tokens, n_single, n_heads / n_kv, tile_rows);
     if (tiles * n_kv > 0x7fffffff) return SIA_BAD_ARGUMENT;
     hipLaunchKernelGGL(attention_f32_kernel<DP>, dim3((unsigned)(tiles * n_kv)), dim3(WAVES * SIA_WAVE), 0, stream, q, q_row_stride, k_pages,
                        v_pages, block_table, table_width, seq_of_token, positions, out, n_tokens, n_single, n_heads, n_kv, head_dim,
-                       value_dim, page_size, scale, window, chunk, sinks, cap, keep_first);
+                       value_dim, page_size, scale, window, chunk, sinks, cap, keep_first, tile_rows);
     return SIA_LAUNCH_CHECK();
 }
 
@@ -295,8 +307,11 @@ extern "C" int sia_attention_generic(const void*, int, const void*, const void*,
 // The arguments of the plain kernel, and n_single: that many tokens, the first ones, are their sequences' only ones; n_seqs;
 // max_kv: no sequence holds more keys.
 // Rows of other sizes, and rows and pages that do not lie in sixteens of bytes, go to the plain kernel; so do steps whose sequences hold so few keys
-// that one of its waves is through before this kernel's barriers are, as long as those waves find room:  32 heads of 64 on 8, plain against this, us:
-// one token over 4 keys 5.2 / 7.0, 17: 7.3 / 7.0, 45 tokens over 45 14.5 / 7.1;  24 heads of 128 on 8:  4: 6.5 / 8.9, 17: 11.6 / 8.9.
+// that one of its waves is through before this kernel's barriers are, as long as those waves find room:  32 heads of 64 on 8, one token, us, plain:  over 4 keys
+// 5.2, 17: 7.3, here 5.5 (7.0 when the border of 16 was set);  45 tokens over 45 14.5 and 5.8;  24 heads of 128 on 8:  4: 6.5, 17: 11.6, here 7.2.  And so
+// do those whose workgroups here would have one row of 16 each (a query head for every key/value head) in more than a round over the chip, with keys that
+// fill no chunk:  256 tokens over 17 and 33 keys, plain and here, 16 heads of 64 on 16 22.9 / 38.9 and 28.5 / 39.8 (64 keys: 58 / 40), 40 of 96 on 40 70 / 161
+// and 152 / 185;  64 tokens, 16 of 64 7.7 / 11.5 and 11.3 / 11.7.
 SIA_EXPORT int sia_attention_f32(const float* q, int q_row_stride, const float* k_pages, const float* v_pages,
                                  const int* block_table, int table_width, const int* seq_of_token, const int* positions,
                                  float* out, int n_tokens, int n_single, int n_seqs, int max_kv, int n_heads, int n_kv,
@@ -308,21 +323,35 @@ SIA_EXPORT int sia_attention_f32(const float* q, int q_row_stride, const float* 
                        n_heads % n_kv == 0 && n_heads <= 65535 && cap >= 0.f && keep_first >= 0 && n_single >= 0 && n_seqs >= 0 &&
                        !(max_kv <= 16 && (long long)n_tokens * n_heads <= 4096) &&
                        ((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0;
-    if (!takes)
+    auto plain = [&]() {
         return sia_attention_generic(q, q_row_stride, k_pages, v_pages, block_table, table_width, seq_of_token, positions, out,
                                      n_tokens, n_heads, n_kv, head_dim, value_dim, page_size, scale, window, chunk, sinks,
                                      cap, keep_first, SIA_F32, stream);
+    };
+    if (!takes) return plain();
     n_single = min(n_single, n_tokens);
     // A workgroup whose 16 rows belong to several sequences takes one after the other: where runs are short, a workgroup for every token instead, if the
-    // chip has room (two or three workgroups a unit take little longer than one).  16 sequences of 3 tokens over 300 keys, us, together and a token each:
-    // 16 heads of 64 on 16 98 / 25.5, 32 on 8 33 / 19.8, 24 of 128 on 8 68 / 30.
-    const long long per_token = (n_heads / n_kv + ROWS - 1) / ROWS, many = n_tokens - n_single, runs = n_seqs - n_single;
-    if (runs > 1) {
-        const double spans = 1.0 + (double)(runs - 1) * ROWS / ((double)many * (n_heads / n_kv));
-        const double together = spans * std::max(640.0, (double)many * n_heads / ROWS), alone = std::max(640.0, (double)many * per_token * n_kv);
-        if (5 * alone <= 4 * together) n_single = n_tokens;
+    // chip has room (two or three workgroups a unit, 640 in all, take little longer than one), or 8 or 4 rows a workgroup.  16 sequences of 3 tokens over
+    // 300 keys, us, together and a token each:  16 heads of 64 on 16 98 / 24, 32 on 8 33 / 18.5, 24 of 128 on 8 68 / 29;  200 of 4 over 64, 6 heads of 32
+    // on 6, 16 and 8 rows:  21 / 13 (10.7 with the kernel for heads of 32).
+    const double room = 640, group = n_heads / n_kv, many = n_tokens - n_single, runs = n_seqs - n_single;
+    const long long per_token = (n_heads / n_kv + ROWS - 1) / ROWS;
+    int tile_rows = ROWS;
+    if (runs > 1 && many > 0) {
+        const double together = (1.0 + (runs - 1) * ROWS / (many * group)) * std::max(room, many * n_heads / ROWS);
+        auto most = [&](int rows) {      // with the sequences that a workgroup's rows may be of
+            return (1.0 + std::ceil((rows - 1) * runs / (many * group))) * std::max(room, many * n_heads / rows);
+        };
+        if (5 * std::max(room, many * per_token * n_kv) <= 4 * together)
+            n_single = n_tokens;
+        else
+            for (int rows = ROWS / 2; rows >= 4; rows /= 2)
+                if (5 * most(rows) <= 4 * most(tile_rows)) tile_rows = rows;
     }
-    return (head_dim <= 64 && value_dim <= 64 ? launch<64> : launch<128>)(
+    const long long workgroups = tiles_of(n_tokens, n_single, n_heads / n_kv, tile_rows) * n_kv;
+    if (max_kv <= (workgroups >= 1536 ? 40 : 20) && workgroups >= 768 && 2LL * n_tokens * n_heads < 3 * workgroups) return plain();
+    const int widest = max(head_dim, value_dim);
+    return (widest <= 32 ? launch<32> : widest <= 64 ? launch<64> : launch<128>)(
         q, q_row_stride, k_pages, v_pages, block_table, table_width, seq_of_token, positions, out, n_tokens, n_single, n_heads, n_kv,
-        head_dim, value_dim, page_size, scale, window, chunk, sinks, cap, keep_first, stream);
+        head_dim, value_dim, page_size, scale, window, chunk, sinks, cap, keep_first, tile_rows, stream);
 }

@@ -1062,6 +1062,69 @@ def test_float32_attention_has_the_same_bits_whichever_way_it_goes(hip, n_heads,
     assert rc == 0 and torch.equal(out, plain)
 
 
+def plain_float_attention(hip, qkv, n_heads, n_kv, D, ctx, cache, window=0):
+    out = torch.empty(ctx.n_tokens, n_heads * D, device=DEV)
+    assert hip.core.sia_attention_generic(
+        qkv.data_ptr(), qkv.shape[1], cache.k_pages.data_ptr(), cache.v_pages.data_ptr(), cache.block_table.data_ptr(),
+        cache.block_table.shape[1], ctx.seq_of_token.data_ptr(), ctx.positions.data_ptr(), out.data_ptr(), ctx.n_tokens, n_heads, n_kv, D, D,
+        cache.page_size, 0.3, window, 0, None, 0.0, 0, 0, hip._stream()) == 0
+    return out
+
+
+def float_attention_step(n_heads, n_kv, D, q_lens, kv_lens):
+    ctx, ps = Ctx(q_lens, kv_lens), 16
+    cache = Cache(sum(-(-kv // ps) for kv in kv_lens), n_kv, ps, D, torch.float32, kv_lens, seed=3)
+    cache.k_pages.copy_(rnd(*cache.k_pages.shape, seed=4))
+    cache.v_pages.copy_(rnd(*cache.v_pages.shape, seed=5))
+    return ctx, cache, rnd(ctx.n_tokens, (n_heads + 2 * n_kv) * D, seed=6)
+
+
+# Rows of one query head a key/value head: a workgroup's 16 rows hold one of a decoded token, or those of several short runs, 16, 8 or 4 of them;
+# with few keys the plain kernel's.  Heads of up to 32, 64 and 128 have kernels of their own.
+@pytest.mark.parametrize("n_heads,n_kv,D", [(6, 6, 32), (16, 16, 64), (5, 5, 100), (8, 4, 24)])
+@pytest.mark.parametrize("n,q,kv", [(256, 1, 17), (256, 1, 41), (100, 1, 65), (200, 4, 64), (90, 3, 130), (64, 2, 40), (17, 9, 70)])
+@pytest.mark.parametrize("window", [0, 30])
+def test_float32_attention_of_a_query_head_a_key_head_has_the_plain_kernels_bits(hip, n_heads, n_kv, D, n, q, kv, window):
+    """Whatever lies in a page behind the last position, or in front of a window, reaches no row; a value that is not finite reaches the rows that see it."""
+    ctx, cache, qkv = float_attention_step(n_heads, n_kv, D, [q] * n, [kv - i % 3 for i in range(n)])
+    attend = lambda: hip.paged_attention(qkv, n_heads, n_kv, D, 0.3, window or None, ctx, cache)
+    whole = attend()
+    assert torch.equal(whole, plain_float_attention(hip, qkv, n_heads, n_kv, D, ctx, cache, window))
+    page, ps = cache.block_table[1, (kv - 2) // 16], 16      # of the second sequence's last position, kv - 2
+    cache.v_pages[page, :, :, (kv - 2) % ps + 1:] = float("nan")
+    cache.v_pages[cache.block_table[1, 0], :, :, 0] = float("nan") if window else 1.0
+    unseen = attend()
+    if window and kv - 1 - q >= window:
+        assert torch.equal(unseen, whole)
+    cache.v_pages[page, :, :, (kv - 2) % ps] = float("inf")
+    got, want = attend(), plain_float_attention(hip, qkv, n_heads, n_kv, D, ctx, cache, window)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+    assert not bool(got[2 * q - 1].isfinite().any()) and bool(got[2 * q:].isfinite().all())
+
+
+@pytest.mark.parametrize("n_heads,D", [(40, 96), (16, 128)])
+def test_float32_attention_over_few_keys_takes_no_longer_than_the_plain_kernel(hip, n_heads, D):
+    """256 decoded tokens over 17 keys, a query head for each key/value head: 70 and 32 us by the plain kernel, 161 and 70 with a row of 16 a workgroup."""
+    ctx, cache, qkv = float_attention_step(n_heads, n_heads, D, [1] * 256, [17] * 256)
+
+    def us(f):
+        best = math.inf
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            f()
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(40):
+                f()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) * 25)
+        return best
+
+    got = us(lambda: hip.paged_attention(qkv, n_heads, n_heads, D, 0.3, None, ctx, cache))
+    assert got <= 1.4 * us(lambda: plain_float_attention(hip, qkv, n_heads, n_heads, D, ctx, cache)) + 5
+
+
 # gate and up in slices and in one, the same of the second product, rows and columns that are no multiples of a tile; one product by tiles, and none
 @pytest.mark.parametrize("K,inter,N,M,tiles", [
     (2048, 8192, 2048, 70, 2), (2048, 8192, 2048, 303, 2), (1024, 2816, 1000, 530, 2), (4096, 1056, 4096, 303, 2),
