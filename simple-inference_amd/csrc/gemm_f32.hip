@@ -960,8 +960,8 @@ struct F32Plan {
 
 static bool wide_rows(const float* rows, int K) { return K % 4 == 0 && ((uintptr_t)rows & 15) == 0; }
 
-// wide_x, wide_w: wide_rows of either.
-static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w) {
+// wide_x, wide_w: wide_rows of either.  has_parts: the tiles find X's parts made.
+static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w, bool has_parts = false) {
     F32Plan best{-1, false, 0, 0};
     const int cus = compute_units(), n_slices = slices_of(N, K), chunks = (K + CHUNK - 1) / CHUNK;
     if (M <= 16 || K >= 1 << 22) return best;
@@ -991,7 +991,7 @@ static F32Plan f32_plan(int M, int N, int K, bool wide_x, bool wide_w) {
             // A tall shape's estimate has to be less than others' by what these err: 9 % where two workgroups of 64 x 128 share a unit, else 4 %; it takes
             // no product from the few-row kernel.  (Of 1,560 products of 65 to 4,096 rows that it was estimated the shorter for, 246 took more
             // than 3 % longer with it, up to 24 %;  so it takes 1,247, of which 41 do, and leaves 42 that it has 3 % and more to give.)
-            if (tall && (best.shape < 0 || us >= (two_a_unit ? 0.91 : 0.96) * others)) continue;
+            if (tall && ((best.shape < 0 && !has_parts) || us >= (two_a_unit ? 0.91 : 0.96) * others)) continue;
             if (us >= least) continue;
             least = us;
             if (!tall) others = us, two_a_unit = i == 1 && !apart;
@@ -1121,48 +1121,65 @@ SIA_EXPORT int sia_gemm_f32(const float* X, const float* W, float* Y, void* work
 // Y[M, N] = (silu(X Wg^T) * (X Wu^T)) Wd^T, W = [Wg; Wu] of 2 inter rows of K, Wd [N, inter]: the same sums as the two products and the activation by
 // themselves.  Where both products are the tiles', with one kernel between them, which makes the second one's parts; else the three one after the
 // other, in one call too (the host takes longer for a step of few tokens than the GPU does).
+// The workspace has two places, which the fused form uses twice each: `front` has X's parts, then the activation and its parts, `back` the first
+// product's result or slices, then the second's slices.  In the other form they hold what a product needs and the activation, the first's result and what
+// the second needs, beside one another.
 extern "C" int sia_swiglu(const void* gu, void* out, int n_tokens, int inter, int dtype, hipStream_t stream);
 struct FeedForwardPlan {
     F32Plan first, second;
-    long long between, act;      // bytes
+    bool fused;
+    long long act, front, back;      // bytes
 };
-static bool feed_forward_plan(const float* X, const float* W, const float* Wd, int M, int N, int K, int inter, FeedForwardPlan& plan) {
-    if (M <= 0 || N <= 0 || K <= 0 || inter <= 0 || inter % CHUNK || inter > 1 << 29 || !wide_rows(X, K) || !wide_rows(W, K) || !wide_rows(Wd, inter))
-        return false;
-    plan.first = f32_plan(M, 2 * inter, K, true, true);
-    plan.second = f32_plan(M, N, inter, true, true);
-    if (plan.first.shape < 0 || plan.second.shape < 0) return false;
-    plan.between = plan.first.apart ? plan.first.slices : (long long)M * 2 * inter * 4;
-    plan.act = (long long)M * inter * 4;
-    return true;
+static long long on_line(long long bytes) { return (bytes + 255) / 256 * 256; }
+static FeedForwardPlan feed_forward_plan(const float* X, const float* W, const float* Wd, int M, int N, int K, int inter) {
+    FeedForwardPlan p;
+    const bool wide_x = wide_rows(X, K), wide_w = wide_rows(W, K), wide_d = wide_rows(Wd, inter), wide_act = inter % 4 == 0;
+    p.first = f32_plan(M, 2 * inter, K, wide_x, wide_w);
+    p.fused = p.first.shape >= 0 && inter % CHUNK == 0 && wide_x && wide_w && wide_d;
+    p.second = f32_plan(M, N, inter, wide_act, wide_d, p.fused);
+    if (p.fused && p.second.shape < 0) p.fused = false, p.second = f32_plan(M, N, inter, wide_act, wide_d);
+    const long long gate_up = on_line((long long)M * 2 * inter * 4), first = on_line(p.first.parts + p.first.slices);
+    const long long second = on_line(p.second.parts + p.second.slices);
+    p.act = on_line((long long)M * inter * 4);
+    if (p.fused) {
+        p.front = std::max(on_line(p.first.parts), p.act + on_line(p.second.parts));
+        p.back = std::max(p.first.apart ? on_line(p.first.slices) : gate_up, on_line(p.second.slices));
+    } else {
+        p.front = first + p.act;
+        p.back = gate_up + second;
+    }
+    return p;
 }
-static long long on16(long long bytes) { return (bytes + 15) / 16 * 16; }
+// Bytes of workspace; 0 where the three by themselves are to be called: with it and Y there would be 64 MiB more in use at a time than they have (from about
+// 1,000 rows of 14,336 or 2,000 of 8,192 on, where the activation by itself is up to 7 % of the time:  4,096 rows of 8,192 1,774 us, in one 1,656, and 637 MB
+// for 403).
 SIA_EXPORT long long sia_f32_feed_forward_workspace(const float* X, const float* W, const float* Wd, int M, int N, int K, int inter) {
     if (M <= 0 || N <= 0 || K <= 0 || inter <= 0 || inter > 1 << 29) return 0;
-    FeedForwardPlan p;
-    if (feed_forward_plan(X, W, Wd, M, N, K, inter, p)) return p.first.parts + p.between + p.act + p.second.parts + p.second.slices;
-    return on16((long long)M * 2 * inter * 4) + on16((long long)M * inter * 4) +
-           std::max(sia_gemm_f32_workspace(X, W, M, 2 * inter, K), sia_gemm_f32_workspace(nullptr, Wd, M, N, inter));
+    const FeedForwardPlan p = feed_forward_plan(X, W, Wd, M, N, K, inter);
+    const long long y = (long long)M * N * 4, gate_up = (long long)M * 2 * inter * 4, act = gate_up / 2;
+    const long long apart = std::max({p.first.parts + p.first.slices + gate_up, gate_up + act, act + p.second.parts + p.second.slices + y});
+    return p.front + p.back + y > apart + (64LL << 20) ? 0 : p.front + p.back;
 }
 SIA_EXPORT int sia_f32_feed_forward(const float* X, const float* W, const float* Wd, float* Y, void* workspace, int M, int N, int K, int inter,
                                     hipStream_t stream) {
-    FeedForwardPlan p;
     if (M <= 0 || N <= 0 || K <= 0 || inter <= 0 || inter > 1 << 29 || !workspace || ((uintptr_t)workspace & 15)) return SIA_BAD_ARGUMENT;
-    char* at = (char*)workspace;
-    if (!feed_forward_plan(X, W, Wd, M, N, K, inter, p)) {
-        float* const gate_up = (float*)at;
-        float* const act = (float*)(at += on16((long long)M * 2 * inter * 4));
-        at += on16((long long)M * inter * 4);
-        int status = sia_gemm_f32(X, W, gate_up, sia_gemm_f32_workspace(X, W, M, 2 * inter, K) ? at : nullptr, M, 2 * inter, K, stream);
+    const FeedForwardPlan p = feed_forward_plan(X, W, Wd, M, N, K, inter);
+    char* const front = (char*)workspace;
+    char* const back = front + p.front;
+    if (!p.fused) {
+        float* const gate_up = (float*)back;
+        float* const act = (float*)(front + p.front - p.act);
+        char* const rest = back + on_line((long long)M * 2 * inter * 4);
+        int status = sia_gemm_f32(X, W, gate_up, p.first.shape >= 0 ? front : nullptr, M, 2 * inter, K, stream);
         if (!status) status = sia_swiglu(gate_up, act, M, inter, SIA_F32, stream);
-        if (!status) status = sia_gemm_f32(act, Wd, Y, sia_gemm_f32_workspace(act, Wd, M, N, inter) ? at : nullptr, M, N, inter, stream);
+        if (!status) status = sia_gemm_f32(act, Wd, Y, p.second.shape >= 0 ? rest : nullptr, M, N, inter, stream);
         return status;
     }
-    u32x4* const parts = (u32x4*)at;
-    float* const between = (float*)(at += p.first.parts);
-    float* const act = (float*)(at += p.between);
-    u32x4* const act_parts = (u32x4*)(at += p.act);
-    float* const slices = (float*)(at += p.second.parts);
+    float* const act = (float*)front;
+    u32x4* const parts = (u32x4*)front;
+    float* const between = (float*)back;
+    u32x4* const act_parts = (u32x4*)(front + p.act);
+    float* const slices = (float*)back;
     const bool four = N % 4 == 0 && ((uintptr_t)Y & 15) == 0;
     split_rows(X, parts, M, K, true, stream);
     int status = f32_tiles(p.first, X, W, between, parts, between, M, 2 * inter, K, true, true, stream);

@@ -1146,6 +1146,30 @@ def test_float_feed_forward_in_one_call_has_the_bits_of_its_parts(hip, K, inter,
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)), odd
 
 
+@pytest.mark.parametrize("M,K,inter", [(40000, 256, 1056), (3000, 1024, 8192), (300, 512, 4128), (2500, 512, 4100), (64, 2048, 8192)])
+def test_a_float_feed_forward_holds_no_more_memory_than_its_parts(hip, M, K, inter):
+    """At most 64 MiB beside what the products and the activation by themselves have in use at a time, in steps of any number of rows.  (The first two, fused
+    whatever they need: 200 to 270 MB more.)"""
+    from types import SimpleNamespace
+
+    from simple_inference_amd.parts.swiglu import SwiGLU
+    part = SwiGLU({"hidden_size": K, "intermediate_size": inter}, SimpleNamespace(kernels=hip))
+    x = rnd(M, K, seed=1)
+    gate, up, down = (rnd(*shape, seed=i, scale=K ** -0.5) for i, shape in enumerate(((inter, K), (inter, K), (K, inter))))
+    part.bind({"gate": gate, "up": up, "down": down})
+
+    def peak(f):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        y = f()
+        return torch.cuda.max_memory_allocated() - before, y
+
+    apart, want = peak(lambda: hip.pending_linear(hip.gated_linear(x, part.w_gate_up), part.w_down))
+    whole, got = peak(lambda: part.forward(x, None))
+    assert torch.equal(got, want) and whole <= apart + (64 << 20) + (1 << 20), (whole, apart)
+
+
 # 16 rows that are several sequences' (two, six and sixteen of them), a part of one token's heads, and tokens that have workgroups of their own
 @pytest.mark.parametrize("n_heads,n_kv,D,Dv", [(8, 8, 64, 64), (12, 4, 20, 36), (40, 2, 128, 100), (17, 1, 64, 64)])
 @pytest.mark.parametrize("q_lens", [[1, 1, 30, 2, 1, 1, 70], [2] * 40, [3] * 400])
