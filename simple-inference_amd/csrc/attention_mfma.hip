@@ -1170,7 +1170,7 @@ SIA_EXPORT long long sia_attn_decode_workspace(int n_seqs, int n_heads, int n_kv
 
 // Sequences 0 .. n_seqs-1 of the step, each with exactly one new token, which is row s of q (cu_q[s] = s), and
 // none longer than kv_bound.  max_splits = sia_attn_decode_max_splits(kv_bound, window); ws_acc and ws_ml hold
-// sia_attn_decode_workspace(.., 0) and (.., 1) floats (neither is read before it is written).
+// sia_attn_decode_workspace(.., 0) and (.., 1) floats, whatever they contain: the states of splits that a sequence does not have are read and not used.
 // chunk > 0: a query sees only its own block of chunk positions (max_splits then from min(window, chunk), whichever
 // are given); sinks: one float per query head that joins its softmax's denominator, or null.
 // kv_share > 1: the pages hold n_kv / kv_share key/value heads, and each is read by kv_share of the launch's n_kv

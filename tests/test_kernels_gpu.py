@@ -1291,6 +1291,33 @@ def test_decode_attention_of_a_sequence_does_not_depend_on_its_batch(hip, geom):
     assert torch.equal(pair[3], together[3]) and torch.equal(pair[9], together[9])
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("sinks", [False, True])
+def test_decode_attention_takes_nothing_from_splits_that_a_sequence_does_not_have(hip, D, sinks):
+    """Sequences of 1 to 32 splits in one launch with a second that combines them: whatever the workspaces held before, the bits are the same.
+    (The states of up to all splits are asked for before it is known how many there are.)"""
+    n_heads, n_kv, ps = 16, 8, 16
+    kv_lens = [40, 20000, 700, 1100, 2100, 1600, 5000, 9000]
+    ctx = Ctx([1] * len(kv_lens), kv_lens)
+    cache = Cache(sum(-(-kv // ps) for kv in kv_lens), n_kv, ps, D, torch.bfloat16, kv_lens, seed=8)
+    cache.k_pages.copy_(rnd(*cache.k_pages.shape, dtype=torch.bfloat16, seed=9))
+    cache.v_pages.copy_(rnd(*cache.v_pages.shape, dtype=torch.bfloat16, seed=10))
+    qkv = rnd(len(kv_lens), (n_heads + 2 * n_kv) * D, dtype=torch.bfloat16, seed=11)
+    sink = rnd(n_heads, seed=12) if sinks else None
+    attend = lambda: hip.paged_attention(qkv, n_heads, n_kv, D, D ** -0.5, None, ctx, cache, sinks=sink)
+    attend()
+    (_, max_splits, ws_acc, ws_ml, _, _), = ctx.attention_plans.values()
+    assert max_splits == 32 and hip._attn_lib(D).sia_attn_decode_mode(len(kv_lens), n_heads, n_kv, max_splits) == 0
+    results = []
+    for value in (0.0, float("nan"), float("inf"), -3e38):
+        ws_acc.fill_(value)
+        ws_ml.fill_(value)
+        results.append(attend())
+    assert bool(results[0].isfinite().all()) and all(torch.equal(r, results[0]) for r in results)
+    ref = twin.paged_attention(qkv, n_heads, n_kv, D, D ** -0.5, None, ctx, cache, sinks=sink)
+    torch.testing.assert_close(results[0].float(), ref.float(), **tol(torch.bfloat16))
+
+
 def test_few_row_products_do_not_depend_on_the_number_of_rows(hip):
     """Up to 16 rows every product (plain, gated, into the residual, with the norm's row scale, with rotation and
     cache write) sums k in an order that K alone fixes: a row's result is the same bit for bit whether it runs
