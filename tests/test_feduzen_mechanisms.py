@@ -406,12 +406,13 @@ def test_sinks_and_blocks_where_decode_attention_splits_the_keys(n_seqs, mode, c
 @pytest.mark.gpu
 @pytest.mark.parametrize("first,n", [(0, 2048), (0, 4096), (0, 9216), (7000, 1024), (100, 700)])
 @pytest.mark.parametrize("chunk", [None, 1500])
-def test_sinks_and_blocks_in_every_shape_of_prefill_workgroup(first, n, chunk):
+@pytest.mark.parametrize("dim", [64, 80])
+def test_sinks_and_blocks_in_every_shape_of_prefill_workgroup(first, n, chunk, dim):
     """Long prompts and portions over a long past in bfloat16: the prefill kernel takes another shape of workgroup
     by the number of row tiles (two sets of waves that share each pair of key tiles and merge at the end, or every
     wave all tiles); the sink joins the denominator after that merge, and a block's first key bounds every tile
-    range.  The plain computation runs in float64 on the GPU."""
-    prefill_case(first, n, chunk, 16, 4, 64)
+    range.  The shape of 256 tokens is for heads of more than 64.  The plain computation runs in float64 on the GPU."""
+    prefill_case(first, n, chunk, 16, 4, dim)
 
 
 @pytest.mark.gpu

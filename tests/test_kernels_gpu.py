@@ -1408,15 +1408,16 @@ def test_prefill_shapes_follow_what_the_row_tiles_see(hip, D, n_heads, q_lens, p
     assert prefill_shape(hip, D, n_heads, q_lens, [q + past for q in q_lens], window, chunk) == shape
 
 
-@pytest.mark.parametrize("q_len, kv_len, window", [(130, 130, None), (900, 1000, None), (1900, 1900, None),
-                                                  (1900, 2100, 300)])
-def test_matrix_core_prefill_in_each_workgroup_shape(hip, q_len, kv_len, window):
-    """The prefill kernel picks one of three workgroup shapes by the number of workgroups: with 34 heads, 130
+@pytest.mark.parametrize("q_len, kv_len, window, shape", [(130, 130, None, SPLIT), (900, 1000, None, PAIRED), (1900, 1900, None, PAIRED),
+                                                         (1900, 2100, 300, WIDE), (2900, 2900, None, WIDE)])
+def test_matrix_core_prefill_in_each_workgroup_shape(hip, q_len, kv_len, window, shape):
+    """The prefill kernel picks one of four workgroup shapes, three for heads of 16: with 34 heads, 130
     tokens take the split shape (64 tokens, even and odd key tiles on two sets of waves, merged at the end),
-    900 the 8-wave shape and 1,900 the wide one.  Lengths are no multiples of a tile."""
+    900 and 1,900 the paired one of 8 waves, and 1,900 through a window and 2,900 the wide one.  Lengths are no multiples of a tile."""
     n_heads, n_kv, D, ps = 34, 2, 16, 16
     dtype = torch.bfloat16
     ctx = Ctx([q_len, 3], [kv_len, 40])
+    assert prefill_shape(hip, D, n_heads, [q_len, 3], [kv_len, 40], window) == shape
     cache = Cache(-(-kv_len // ps) + 8, n_kv, ps, D, dtype, [kv_len, 40], seed=31)
     cache.k_pages.copy_(rnd(*cache.k_pages.shape, dtype=dtype, seed=32))
     cache.v_pages.copy_(rnd(*cache.v_pages.shape, dtype=dtype, seed=33))
@@ -1427,9 +1428,9 @@ def test_matrix_core_prefill_in_each_workgroup_shape(hip, q_len, kv_len, window)
 
 
 def test_matrix_core_prefill_in_workgroups_of_256_tokens(hip):
-    """Very many workgroups (128 heads, 2,500 tokens) take the shape of 8 waves of 32 tokens; a second and a third
+    """Very many workgroups (128 heads of 80, 2,500 tokens) take the shape of 8 waves of 32 tokens; a second and a third
     run in the same launch, shorter than a workgroup and a little longer than one, and a window."""
-    n_heads, n_kv, D, ps = 128, 8, 16, 16
+    n_heads, n_kv, D, ps = 128, 8, 80, 16
     dtype = torch.bfloat16
     q_lens, kv_lens = [2500, 40, 300], [2700, 40, 555]
     ctx = Ctx(q_lens, kv_lens)
@@ -1437,13 +1438,32 @@ def test_matrix_core_prefill_in_workgroups_of_256_tokens(hip):
     cache.k_pages.copy_(rnd(*cache.k_pages.shape, dtype=dtype, seed=42))
     cache.v_pages.copy_(rnd(*cache.v_pages.shape, dtype=dtype, seed=43))
     qkv = rnd(ctx.n_tokens, (n_heads + 2 * n_kv) * D, dtype=dtype, seed=44, scale=2.0)
-    lib = hip._attn_lib(D)
-    assert lib.sia_attn_prefill_rows_long() == 256
-    assert sum(-(-q // lib.sia_attn_prefill_rows()) for q in q_lens) * n_heads >= 2400   # the launch takes that shape
+    assert hip._attn_lib(D).sia_attn_prefill_rows_long() == 256
     for window in (None, 700):
+        assert prefill_shape(hip, D, n_heads, q_lens, kv_lens, window) == LONG
         out = hip.paged_attention(qkv, n_heads, n_kv, D, 1 / math.sqrt(D), window, ctx, cache)
         ref = twin.paged_attention(qkv, n_heads, n_kv, D, 1 / math.sqrt(D), window, ctx, cache)
         torch.testing.assert_close(out.float(), ref.float(), **tol(dtype))
+
+
+# Every shape of workgroup with every form of mask and score.  Lengths are no multiples of a tile.
+@pytest.mark.parametrize("q_len, shape", [(130, SPLIT), (900, PAIRED), (2600, WIDE), (4300, LONG)])
+@pytest.mark.parametrize("form", [{}, {"window": 333}, {"chunk": 500}, {"sinks": True}, {"softcap": 2.0}, {"window": 333, "keep_first": 75}])
+def test_matrix_core_prefill_shapes_in_every_form(hip, q_len, shape, form):
+    n_heads, n_kv, D, ps, dtype = 34, 2, 80, 16, torch.bfloat16
+    q_lens, kv_lens = [q_len, 3], [q_len + 50, 40]
+    forms = "softcap" in form or "keep_first" in form
+    assert prefill_shape(hip, D, n_heads, q_lens, kv_lens, form.get("window"), form.get("chunk"), forms) == shape
+    ctx = Ctx(q_lens, kv_lens)
+    cache = Cache(-(-kv_lens[0] // ps) + 8, n_kv, ps, D, dtype, kv_lens, seed=31)
+    cache.k_pages.copy_(rnd(*cache.k_pages.shape, dtype=dtype, seed=32))
+    cache.v_pages.copy_(rnd(*cache.v_pages.shape, dtype=dtype, seed=33))
+    qkv = rnd(ctx.n_tokens, (n_heads + 2 * n_kv) * D, dtype=dtype, seed=34, scale=2.0)
+    more = {k: v for k, v in form.items() if k != "window"}
+    if "sinks" in more:
+        more["sinks"] = rnd(n_heads, seed=35) + 1.0
+    args = (qkv, n_heads, n_kv, D, 1 / math.sqrt(D), form.get("window"), ctx, cache)
+    torch.testing.assert_close(hip.paged_attention(*args, **more).float(), twin.paged_attention(*args, **more).float(), **tol(dtype))
 
 
 def test_matrix_core_attention_runs_longer_than_a_block_table_window(hip, monkeypatch):
