@@ -624,6 +624,27 @@ TALL_FLOAT_WAYS = [(129, 28674, 128, 10), (160, 50003, 224, 10), (259, 14337, 12
                    (129, 32770, 224, 12), (150, 40961, 160, 12), (311, 2050, 2048, 13), (129, 5123, 1536, 13), (606, 16386, 1536, 13)]
 
 
+@pytest.mark.parametrize("M, N, K, way", [(303, 14337, 1536, 11), (150, 40961, 160, 12), (311, 2050, 2048, 13)])
+def test_tall_tiles_whose_waves_find_weights_of_24_bits_at_different_chunks(hip, M, N, K, way):
+    """Weights are bfloat16 numbers but for some from a chunk on, another for each of some rows: waves of a workgroup go on with all parts of the weights from
+    different chunks, with their sums and places in the rings.  A value under 2^-110 in a late chunk among them.  The few-row kernel's bits."""
+    assert hip.core.sia_gemm_f32_way(None, None, M, N, K) == way
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2).bfloat16().float()
+    whole = rnd(N, K, seed=3)
+    chunks = K // 32
+    for row, chunk in ((0, 0), (17, 1), (40, chunks // 2), (50, chunks // 2 + 1), (100, chunks - 1), (131, 3), (N // 2, chunks // 3), (N - 1, chunks - 1)):
+        w[row, 32 * chunk:] = whole[row, 32 * chunk:]
+    few = torch.empty(M, N, device=DEV)
+    for small in (False, True):
+        if small:
+            w[70, K - 5], w[N // 3, K - 33] = 2.0 ** -120 * 1.2345678, 2.0 ** -115 * 1.2345678
+        y = hip.linear(x, w)
+        assert hip.core.sia_gemm_f32(x.data_ptr(), w.data_ptr(), few.data_ptr(), None, M, N, K, hip._stream()) == 0
+        assert torch.equal(y, few)
+        want = x.double() @ w.double().T
+        assert float((y.double() - want).norm() / want.norm()) <= 2e-7
+
+
 # The tall tiles take products of a float32 model's steps, and none that the smaller tiles or the few-row kernel take as long or less for:  us, theirs and the
 # tall ones', weights of 8 bits:  768 x 12,288 x 3,072 263 and 327;  1,280 x 8,192 x 4,096 366 and 446;  640 x 1,024 x 1,536 21.4 and 26.1;  160 x 3,072 x
 # 2,048 24.3 and 26.1;  303 x 128,256 x 2,048 691 and 594.
@@ -1045,10 +1066,8 @@ def test_float32_attention_is_the_plain_kernels(hip, geom, more):
 @pytest.mark.parametrize("q_lens,kv_lens", [([16], [16]), ([17], [17]), ([1, 1, 3], [16, 2, 16]), ([3] * 16, [300] * 16), ([2] * 70, [40] * 70),
                                             ([1, 40], [70, 40]), ([1, 40], [30, 40]), ([64], [264]), ([65], [265])])
 def test_float32_attention_has_the_same_bits_whichever_way_it_goes(hip, n_heads, n_kv, D, q_lens, kv_lens):
-    """Few keys (the plain kernel), few tokens or short runs (a workgroup a token), more (eight tokens a workgroup): each
-    sequence's rows are those that it has alone."""
+    """Few keys (the plain kernel), short runs (a workgroup a token), more (16 rows a workgroup): the plain kernel's bits."""
     ctx, ps = Ctx(q_lens, kv_lens), 16
-    ctx.max_run_kv_len = max([kv for q, kv in zip(q_lens, kv_lens) if q > 1], default=0)
     cache = Cache(sum(-(-kv // ps) for kv in kv_lens), n_kv, ps, D, torch.float32, kv_lens, seed=3)
     cache.k_pages.copy_(rnd(*cache.k_pages.shape, seed=4))
     cache.v_pages.copy_(rnd(*cache.v_pages.shape, seed=5))
@@ -1144,6 +1163,28 @@ def test_float_feed_forward_in_one_call_has_the_bits_of_its_parts(hip, K, inter,
         way = lambda t, m, n, k: hip.core.sia_gemm_f32_way(t.data_ptr(), t.data_ptr(), m, n, k) >= 0
         assert way(w, M, 2 * inter, K) + way(down, M, N, inter) == tiles
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0)), odd
+
+
+# both by tiles and rows of the activation that are no chunks (in fours, and not);  the activation between, and a result whose rows are no fours
+@pytest.mark.parametrize("K,inter,N,M", [(512, 4132, 1028, 303), (512, 4131, 1029, 303), (512, 4128, 1029, 303), (2048, 8192, 2047, 303)])
+def test_float_feed_forward_of_odd_sizes_in_one_call(hip, K, inter, N, M):
+    test_float_feed_forward_in_one_call_has_the_bits_of_its_parts(hip, K, inter, N, M, 2, False)
+
+
+@pytest.mark.parametrize("which", ["input", "gate/up", "down"])
+def test_float_feed_forward_of_operands_that_begin_anywhere(hip, which):
+    """A float behind a multiple of 16 bytes: the same bits, by the products' general forms."""
+    K, inter, N, M = 512, 4128, 1028, 303
+    x, w, down = rnd(M, K, seed=1), rnd(2 * inter, K, seed=2, scale=K ** -0.5), rnd(N, inter, seed=3, scale=inter ** -0.5)
+    want = hip.float_feed_forward(x, w, down)
+
+    def shifted(t):
+        flat = torch.full((t.numel() + 8,), float("nan"), device=DEV)
+        flat[1:1 + t.numel()] = t.flatten()
+        return flat[1:1 + t.numel()].view(t.shape)
+
+    got = hip.float_feed_forward(shifted(x) if which == "input" else x, shifted(w) if which == "gate/up" else w, shifted(down) if which == "down" else down)
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("M,K,inter", [(40000, 256, 1056), (3000, 1024, 8192), (300, 512, 4128), (2500, 512, 4100), (64, 2048, 8192)])
