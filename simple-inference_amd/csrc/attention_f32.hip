@@ -12,7 +12,7 @@
 // A token that is its sequence's only one (decode) has a workgroup of its own.
 // What bounds it is the chain of a chunk: 16 dependent products of 32 cycles a wave each for scores and values (heads of 64), and two barriers, 5,000 cycles
 // in all; 600 and more tokens fill the chip with chains.  us, before (a lane a key) and now: 303 tokens (three decoded over 200 keys, a prompt of 300), 32 heads of 64 on 8
-// 57 -> 16.2, 24 of 128 on 8 101 -> 22.8;  a prompt of 2,048 956 -> 308 (56 TFLOP/s of 157), 2,160 -> 443;  one token over 16,000 keys 1,358 -> 535;
+// 57 -> 16.2 (19.4 in a step), 24 of 128 on 8 101 -> 22.8;  a prompt of 2,048 956 -> 308 (56 TFLOP/s of 157), 2,160 -> 443;  one token over 16,000 keys 1,358 -> 535;
 // 64 over 2,048 211 -> 115 (537 MB: 4.7 TB/s);  256 over 17 with a query head for each of 16 key/value heads of 64 33 -> 23 (by the plain kernel).
 #include <algorithm>
 #include <cmath>

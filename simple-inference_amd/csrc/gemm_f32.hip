@@ -26,11 +26,11 @@
 //   is staged through LDS by loads that pass no registers, W split where it is read.  Two sums a result
 //   are what its registers hold: 128 x 256 outputs, which one sum allowed (303 x 128,256 x 2,048 664 us), would spill.
 // Workspace: the parts, 6 bytes an element of X; where slices are apart their sums, a float a result and slice, 512 MiB at most.
-// us, v_mfma_f32_16x16x4_f32 -> now, weights of 8 bits and of 24:  303 rows x 128,256 x 2,048 1,461 -> 701 and 1,310, x 16,384 x 2,048 203 -> 110
-// and 191, x 2,048 x 8,192 136 -> 64 and 101, x 3,072 x 2,048 42.5 -> 36.9 and 50;  one row x 2,048 x 2,048 8.7 -> 6.1 and 7.3, x 2,048 x 8,192 23.4 -> 15.3
+// us, v_mfma_f32_16x16x4_f32 -> now, weights of 8 bits and of 24:  303 rows x 128,256 x 2,048 1,461 -> 594 and 1,204, x 16,384 x 2,048 203 -> 99
+// and 168, x 2,048 x 8,192 136 -> 55 and 90, x 3,072 x 2,048 42.5 -> 31.6 and 45;  one row x 2,048 x 2,048 8.7 -> 6.1 and 7.3, x 2,048 x 8,192 23.4 -> 15.3
 // and 19.9, x 14,336 x 4,096 50 -> 42 and 42;  64 rows x 2,048 x 2,048 11.6 -> 8.9 and 10.9.  Slower: 200 to 1,024 rows of 1,000 x 1,000 (512: 16.5 -> 19.5
 // and 20.5, 1,024: 25 -> 28 and 41), one row x 128,256 x 2,048 (192 -> 198), and with weights of 24 bits 1 to 96 rows of 14,336 to 16,384 columns (17 x 16,384 x
-// 2,048 28.8 -> 30.8, 32 x 14,336 x 4,096 50.5 -> 57.9) and 130 to 1,024 rows of 2,048 to 3,072 (512 x 2,048 x 2,048 42.7 -> 52.9, 303 x 3,072 x 2,048 42.6 -> 50).
+// 2,048 28.8 -> 30.8, 32 x 14,336 x 4,096 50.5 -> 57.9) and 130 to 1,024 rows of 2,048 to 3,072 (512 x 2,048 x 2,048 42.7 -> 52.9, 303 x 3,072 x 2,048 42.6 -> 45).
 #include "lds_load.h"
 
 #include <algorithm>
@@ -674,7 +674,7 @@ __global__ __launch_bounds__(WM* WN* SIA_WAVE) void gemm_f32_tile_kernel(
 // each with a ring of its own, DX and DW chunks ahead: a wave's loads end in order, and X, which L2 holds, would wait for W behind it.
 // Bound by what a compute unit fetches and then reads from LDS, which the matrix cores wait for in part: cycles of a chunk of 160 x 128, each alone: loads
 // 1,800, reads 930, products and sums 1,350, all together 2,560 (1.1 us).  Wider tiles fetch less for a result: 303 rows x 128,256 x 2,048, weights of 8 bits,
-// 677 us in tiles of 64 x 128, 600 in 160 x 128, 573 in 160 x 192 (160 x 256 spills: 830);  x 16,384 x 2,048 117 -> 95 (160 x 128), x 3,072 x 2,048 36 -> 30.6 (160 x 192),
+// 677 us in tiles of 64 x 128, 600 in 160 x 128, 573 in 160 x 192 (650 in a step; 160 x 256 spills: 830);  x 16,384 x 2,048 117 -> 95 (160 x 128), x 3,072 x 2,048 36 -> 30.6 (160 x 192),
 // x 2,048 x 8,192 65 -> 54, x 2,048 x 2,048 29 -> 26 (160 x 128);  weights of 24 bits 1,270 -> 1,130, 184 -> 160, 48 -> 43, 107 -> 87, 38 -> 34.
 // With the next chunk's first reads in front of the last products of this one nothing changed (600 and 587 us), with four waves of twice the rows and
 // 512 registers 660.

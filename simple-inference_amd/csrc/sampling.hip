@@ -280,8 +280,8 @@ static_assert(SP_CLEAR_BYTES % (sizeof(uint4) * SP_CHUNKS) == 0 && sizeof(Sample
 // sets its share of the row's histograms to zero: the counting launches come after this one.
 // Of many rows by workgroups of four waves: a compute unit then has the loads of eight on their way while others reduce, where it had two of
 // 16 waves that did both in step.  us with the pick behind it, 16 waves and 4:  rows of 128,256: 64 14.0 and 10.8, 303 42.7 and 29.1
-// (155 MB: 6 TB/s while it reads);  300 of 32,000 33.7 and 12.6;  64 of 512 9.7 and 6.2.  Up to 16 rows, which a unit has one workgroup of, 16 waves, whose threads
-// ask for a chunk's logits at once: one row 7.3 and 7.8, 8 7.6 and 8.2.
+// (155 MB: 6 TB/s while it reads);  17 8.4 and 8.1, 32 8.9 and 8.4;  rows of 512:  17 6.9 and 5.7, 64 9.7 and 6.1;  300 of 32,000 33 and 12.7.  Up to 16 rows,
+// whose chunks (SP_CHUNKS each) are a workgroup a unit, 16 waves, whose threads ask for a chunk's logits at once: one row of 128,256 7.3 and 7.8, 8 7.6 and 8.2.
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void sample_max_kernel(const float* __restrict__ logits, int vocab,
                                                                     SampleRow* __restrict__ ws, int clear) {
